@@ -30,7 +30,7 @@ int32_t tsv_write_logits(tsv_ctx* ctx, const uint16_t* logits, int32_t m, int64_
 /* One quantized small-M matmul through the same kernels the forward uses:
  * y[m][r] = sum_k W[r][k] x[m][k]; x is m x cols fp32 (rounded to fp16 on entry), y is
  * m x rows fp32.  W host tensor in GGUF layout (re-tiled per call).  `splits` <= 0 picks
- * the engine's own split-K factor. */
+ * the engine's own split-K factor.  More than TSV_MAX_ROWS rows (2048 at most) go through the prompt passes' kernel. */
 int32_t tsv_matmul(const tsv_tensor* w, const float* x, int32_t m, float* y, int32_t splits);
 
 /* Host arithmetic only: how many launches of the walk kernel a sampled tree round of this shape is given -- the most
@@ -75,6 +75,7 @@ int32_t tsv_copy_time(int64_t bytes, int32_t iters, float* avg_us);
  * slot base+i and sees [0, base) plus the slots of its root path (parent NULL: chain).
  * window > 0 keeps the last `window` positions of each row's sequence; sinks (nullable): one f32
  * logit per q head (crates/compute/src/attention.rs:29-137).
+ * More than TSV_MAX_ROWS rows (2048 at most, chains only) go through the prompt passes' kernel.
  * out: m x nq x hd fp16.  (The per-kernel parity hook of crates/gpu/tests/attention_tree_parity.rs.) */
 int32_t tsv_attention(const uint16_t* q, const uint16_t* k, const uint16_t* v, int32_t m, int32_t nq,
                       int32_t nkv, int32_t hd, int64_t base, const int32_t* parent, float scale,

@@ -1,0 +1,80 @@
+"""The kernels of a prompt pass at the edges of their tiles: the matmul over 17 and more rows for every storage type, attention
+over consecutive rows, and whole prompts at lengths around the passes' limits."""
+import numpy as np
+import pytest
+
+from oracle import binding as ob
+from tests import gpu_common as gc
+from tests.test_oracle_quant import lcg_weights
+
+pytestmark = pytest.mark.gpu
+
+
+# rows and columns around the 128-column tiles and the 256-, 128- and 64-wide chunks; m around the 64-, 128- and 256-row tiles
+@pytest.mark.parametrize("dtype,rows,cols", [(12, 64, 512), (12, 200, 768), (13, 64, 512), (13, 200, 768), (14, 130, 512), (14, 64, 1024),
+                                             (8, 64, 128), (8, 200, 1408), (30, 64, 64), (30, 130, 2880), (39, 64, 256), (39, 200, 2880)])
+@pytest.mark.parametrize("m", [17, 64, 65, 128, 129, 257])
+def test_the_prompt_matmul_is_the_dequantized_product(dtype, rows, cols, m):
+    from turbospark_amd import ffi
+    w = lcg_weights(rows * cols, 5).reshape(rows, cols) * 0.05
+    w[::7] *= 1e-3                                     # rows and blocks of very different scale
+    w[3, :cols // 2] *= 1e-2
+    w[5, :32] = w[9] = 0.0                             # a zero block, a zero row
+    entry = ffi.quantize(dtype, w)
+    x = lcg_weights(m * cols, 6).reshape(m, cols)
+    deq = ob.dequantize(dtype, entry[1], cols).astype(np.float64)
+    want = x.astype(np.float16).astype(np.float64) @ deq.T
+    # fp32 sums of exact products: rounding of about sqrt(K) terms of the row's size (the bound of the 16-row kernels' test)
+    scale = np.abs(want).max(0)
+    for splits in (0, 1):
+        got = ffi.matmul(entry, x, splits)
+        assert (np.abs(got - want) <= 2e-4 * scale + 1e-9).all(), (splits, np.abs(got - want).max() / scale.max())
+
+
+@pytest.mark.parametrize("nq,nkv,hd", [(8, 8, 64), (32, 8, 128), (16, 2, 64), (6, 2, 128)])
+@pytest.mark.parametrize("m,base,window,sinks", [(17, 0, 0, False), (33, 15, 0, True), (64, 200, 24, False), (130, 1000, 128, True),
+                                                 (70, 3001, 0, True), (300, 5, 40, False)])
+def test_prompt_attention_matches_the_oracle(nq, nkv, hd, m, base, window, sinks):
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(m + base)
+    r16 = lambda *s: rng.standard_normal(s).astype(np.float16).astype(np.float32)
+    q, k, v = r16(m, nq, hd), r16(base + m, nkv, hd), r16(base + m, nkv, hd)
+    sk = rng.standard_normal(nq).astype(np.float32) if sinks else None
+    got = ffi.attention(q, k, v, base, window=window, sinks=sk)
+    rows = sorted({0, 1, 15, 16, m // 2, m - 2, m - 1})
+    for i in rows:
+        want = ob.causal_attention(q[i], k, v, hd, nq, nkv, base + i + 1, window, 0.0, sk).reshape(nq, hd)
+        assert np.abs(got[i] - want).max() <= 5e-3 * max(1.0, np.abs(want).max()), i   # the bound of the verify passes' test
+
+
+@pytest.mark.parametrize("name,n,start", [("small_q4_k", 65, 0), ("xcd_q8_0", 257, 3), ("small_q5_k_m", 300, 31), ("xcd_q4_k", 2049, 0)])
+def test_prompts_around_the_limits_of_a_pass(name, n, start):
+    """Logits of the last token, what a verify pass after the prompt sees, and the rows left for tsv_accept, against passes of
+    sixteen rows."""
+    import os
+    import turbospark_amd as ts
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS[name], max_context=start + n + 32)
+    w = synth.make_weights(cfg, seed=3)
+    fast = ts.HipVerifier(cfg, w)
+    os.environ["TSV_WIDE_PREFILL"] = "0"
+    try:
+        slow = ts.HipVerifier(cfg, w)
+    finally:
+        del os.environ["TSV_WIDE_PREFILL"]
+    rng = np.random.default_rng(n)
+    prompt = rng.integers(0, cfg["vocab"], start + n).astype(np.int32)
+    feed = rng.integers(0, cfg["vocab"], 5).astype(np.int32)
+    out = []
+    for eng in (fast, slow):
+        if start:
+            eng.prefill(prompt[:start], 0, want_logits=False)
+        last = eng.prefill(prompt[start:], start)
+        m = (n - 1) % 16 + 1
+        acc = eng.accept(prompt[start + n - m:], start + n - m, ts.shaping(0.0))
+        eng.reset()
+        eng.prefill(prompt, 0, want_logits=False)
+        out.append((last, eng.verify(feed, start + n), acc))
+    assert gc.logit_error(out[0][0].reshape(1, -1), out[1][0].reshape(1, -1)) <= 2e-3
+    assert gc.logit_error(out[0][1], out[1][1]) <= 2e-3
+    assert (out[0][2].accepted, out[0][2].kv_position) == (out[1][2].accepted, out[1][2].kv_position)

@@ -96,6 +96,22 @@ struct tsv_ctx {
         size_t frag_e_sub = 0;
         float* moe_out = nullptr;
     } wide;
+    // prompt passes (prefill.hip): buffers for `rows` rows, allocated at the first pass and grown to the largest one asked
+    // for (PROMPT_ROWS at most); freed with the handle
+    struct Prompt {
+        bool ok = false;
+        int rows = 0;
+        float* x = nullptr;                 // residual rows
+        uint8_t *a_h = nullptr, *a_q = nullptr, *a_f = nullptr;  // activations: K = hidden, q width, ffn
+        uint8_t *s_h = nullptr, *s_q = nullptr, *s_f = nullptr;  // their sub-block sums
+        float* partial = nullptr;
+        size_t partial_floats = 0;
+        uint16_t* q16 = nullptr;
+        float2* cs = nullptr;
+        int32_t* ids = nullptr;
+        float *part_o = nullptr, *part_ml = nullptr;
+        std::vector<void*> allocs;
+    } prompt;
     bool route_forced_set = false;  // tsv_force_route holds selections: prompt passes stay at sixteen rows
     uint16_t* q16 = nullptr;
     float *part_o = nullptr, *part_ml = nullptr;
@@ -212,6 +228,13 @@ int check_matrix(const tsv_tensor& t, int64_t rows, int64_t cols, const char* wh
 int make_tiled(tsv_ctx* c, Stager& st, const tsv_tensor* const* parts, int n_parts, bool interleave, TiledW* out, int pair_parts = 0);
 int check_shaping(const tsv_shaping& s, bool sampled_supported_only);
 int fill_params(VerifyParams& vp, const int32_t* feed, const int32_t* parent, int m, int64_t base, int vocab);
+int stage_params(tsv_ctx* c, const VerifyParams* vp, int n, VerifyParams* dev);
+// Prompt passes (prefill.hip): whether the handle's layers can go that way, and one pass of n rows (PROMPT_MIN_ROWS ..
+// PROMPT_ROWS) at the cursor.  finish: the rows' last residual add as well, left in prompt.x and, the last (n - 1) % 16 + 1
+// rows, in x; logits: those rows' logits too.
+bool prompt_supported(const tsv_ctx* c);
+int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits);
+void prompt_free(tsv_ctx* c);
 // One verify pass: everything enqueued on the handle's stream, no synchronisation; then the optional copy of the rows' logits.
 int enqueue_verify(tsv_ctx* c, const int32_t* feed, const int32_t* parent, int m, int64_t base);
 int finish_verify(tsv_ctx* c, int m, uint16_t* logits_out);

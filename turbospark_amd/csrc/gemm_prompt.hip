@@ -1,0 +1,639 @@
+// The matmuls of a prompt pass (crates/runtime/src/families/llama/prefill.rs): Y[row][n] = sum_k W[n][k] X[row][k] over
+// hundreds of rows, straight from the quantized row tiles the verify passes read.
+//
+// One workgroup of four waves makes a BM x 128 tile of Y on v_mfma_f32_32x32x16_f16 (BM = 256, 128 or 64 rows; a wave
+// always has 64 rows and 128, 64 or 32 columns).  The workgroup walks K in stages of 64 or 128: each stage's 128 weight rows
+// are unpacked ONCE, by all four waves, into fp16 B operands in LDS (two buffers, one barrier per stage); the activations
+// arrive as ready A operands (prompt.h) and go from the L2 straight to the registers of the one wave that needs them, so
+// LDS carries the weights only: 4 KiB read per wave and 16-K step against 8 matrix instructions of 32 cycles.  Two workgroups
+// share a compute unit: while one waits at its barrier or unpacks, the other multiplies.
+//
+// No operand is rounded.  What is multiplied are
+//   Q4_K / Q5_K   sc_j * q, an integer below 2048.  The superblock's d is the unit its sums are counted in: the accumulator is
+//                 multiplied by (unit before) / d when the walk enters a chunk.  At the chunk's end the unit becomes -dmin and
+//                 one more matrix instruction adds the sub-block sums times the integers m_j: two multiplies per element and
+//                 256 K in all, and no second accumulator
+//   Q6_K          (level - 32) * 16 (sc >> 4) and (level - 32) * (sc & 15), two exact integer operands; units as above
+//   Q8_0          q * d split into an fp16 and what it leaves over, both exact
+//   bf16, MXFP4   the value itself, times the power of two that brings the row's largest value to the top of fp16's range
+// (the last three: row_scale; a value 2^35 below its row's largest would begin to lose bits, where fp32 sums keep 24).
+//
+// Bound by the matrix pipes: the gate/up product of 2048 rows (28672 x 4096 Q4_K, silu epilogue included) takes 489 us = 983
+// TFLOP/s on an MI355X, where a library product of 8192^3 fp16 values reaches 1164; 64 rows at a time (k_gemm_wide) the same
+// rows took 32 x 40.7 us.
+//
+// Workgroups are numbered so that an XCD works on every eighth block of columns with all row blocks side by side: the
+// weights of a block come into that XCD's L2 once, and the activations are shared by the blocks in flight.
+#include <algorithm>
+
+#include "prompt.h"
+
+namespace tsv {
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ float half_lo(uint32_t v) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(v & 0xFFFF)); }
+__device__ __forceinline__ float half_hi(uint32_t v) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(v >> 16)); }
+__device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+__device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ half2v pair_of(float v) { return half2v{(_Float16)v, (_Float16)v}; }
+
+// Constants that v_and_or_b32 takes from registers (the instruction has room for one literal)
+struct Bits {
+    uint32_t k6400, k5400;
+};
+
+// LDS of one stage: B operands [virtual 16-K step][4 column blocks of 32][64 lanes][16 B]; lane n % 32 + 32 * (k % 16 / 8).
+constexpr int STEP_BYTES = 4096;
+constexpr int MIN_BYTES = 4096;                    // min operands of a chunk, [4][64 lanes][16 B]
+constexpr int COEF_BYTES = 128 * 8;                // the rescale factors of the tile's 128 columns: into the chunk, into its min term
+constexpr int CHUNK_BYTES = MIN_BYTES + COEF_BYTES;  // two of them: a chunk's are used up to its end, the next one's written before
+__device__ __forceinline__ void put_piece(uint8_t* buf, int step, int half, int t64, int lane, u32x4 v) {
+    *(u32x4*)(buf + ((step * 4 + 2 * t64 + (lane >> 5)) * 64 + half * 32 + (lane & 31)) * 16) = v;
+}
+
+// The unit a row's sums are counted in, followed chunk by chunk by the lane that unpacks the row.
+struct Unit {
+    float u = 1.0f;
+    bool first = true;
+    // enters a chunk with scale d; returns what the accumulator has to be multiplied by.  d == 0 keeps the unit (the chunk's
+    // integers are then cleared by the caller)
+    __device__ __forceinline__ float enter(float d) {
+        const float nu = d == 0.0f ? u : d;
+        const float ratio = first ? 1.0f : u / nu;
+        first = false;
+        u = nu;
+        return ratio;
+    }
+    __device__ __forceinline__ float enter_mins(float dmin) {
+        const float nu = dmin == 0.0f ? u : -dmin;
+        const float ratio = u / nu;
+        u = nu;
+        return ratio;
+    }
+};
+
+// ---- storage types ------------------------------------------------------------------------------------------------------
+// STAGE_K real K per stage, TERMS operands per weight, SPC stages per tile chunk.  A wave's share of a stage is one half of
+// its K (`part`) of one 64-row tile: load() asks for the bytes of lane's row, unpack() leaves the operands in LDS.
+template <bool Q5>
+struct PromptQ45 {
+    static constexpr int TILE_BYTES = Q5 ? 11264 : 9216, STAGE_K = 128, TERMS = 1, SPC = 2;
+    static constexpr bool UNITS = true, MINS = true;
+    struct Regs {
+        u32x4 q[2], h, f[Q5 ? 2 : 1];
+    };
+    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
+        const u32x4* p = (const u32x4*)tile + lane;
+        const int u = 4 * sub + 2 * part;
+        r.q[0] = p[u * 64];
+        r.q[1] = p[(u + 1) * 64];
+        r.h = p[512];
+        if (Q5) {
+            r.f[0] = p[576];
+            r.f[1] = p[640];
+        }
+    }
+    // 64 K of the row: sub-blocks 2 p (low nibbles) and 2 p + 1 (high), p = 2 sub + part; unit i of the pair holds elements
+    // 16 i .. 16 i + 15 of both
+    static __device__ __forceinline__ void unpack(const Regs& r, const Bits& k, Unit& unit, float, uint8_t* buf, uint8_t* mins, float2* coef, int sub,
+                                                  int part, int t64, int lane) {
+        const float d = half_lo(r.h.x), dmin = half_hi(r.h.x);
+        uint32_t sl = r.h.y & 0x3F3F3F3Fu, sh = (r.h.w & 0x0F0F0F0Fu) | ((r.h.y >> 2) & 0x30303030u);
+        if (d == 0.0f) sl = sh = 0;
+        if (sub == 0) {
+            const float into = unit.enter(d), into_mins = unit.enter_mins(dmin);
+            if (part == 0) {
+                coef[t64 * 64 + lane] = float2{into, into_mins};
+            } else {
+                uint32_t ml = r.h.z & 0x3F3F3F3Fu, mh = ((r.h.w >> 4) & 0x0F0F0F0Fu) | ((r.h.z >> 2) & 0x30303030u);
+                if (dmin == 0.0f) ml = mh = 0;
+                u32x4 hi, lo;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t m2 = (i < 2 ? ml : mh) >> (16 * (i & 1));
+                    const half2v m = as_h2(k.k6400 | (m2 & 0xFF) | ((m2 & 0xFF00) << 8)) + pair_of(-1024.0f);
+                    hi[i] = as_u32(m * pair_of(1.0f / PROMPT_SUM_SCALE));
+                    lo[i] = as_u32(m * pair_of(1.0f / (PROMPT_SUM_SCALE * PROMPT_SUM_LEFT)));
+                }
+                put_piece(mins, 0, 0, t64, lane, hi);
+                put_piece(mins, 0, 1, t64, lane, lo);
+            }
+        }
+        const uint32_t s2 = (sub == 0 ? sl : sh) >> (16 * part);
+        const half2v sc_lo = as_h2(k.k6400 | (s2 & 0xFF) | ((s2 & 0xFF) << 16)) + pair_of(-1024.0f);
+        const half2v sc_hi = as_h2(k.k6400 | ((s2 >> 8) & 0xFF) | (((s2 >> 8) & 0xFF) << 16)) + pair_of(-1024.0f);
+        const half2v off_lo = sc_lo * pair_of(-1024.0f), off_hi = sc_hi * pair_of(-64.0f);
+        const int p = 2 * sub + part;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                u32x4 lo, hi;
+#pragma unroll
+                for (int w = 0; w < 2; w++) {
+                    const uint32_t v = r.q[i][2 * h + w];
+#pragma unroll
+                    for (int o = 0; o < 2; o++) {
+                        const uint32_t x = o ? v >> 8 : v;
+                        uint32_t lb = (x & 0x000F000Fu) | k.k6400, hb = (x & 0x00F000F0u) | k.k5400;  // 1024 + q, 64 + q
+                        if (Q5) {  // the fifth bit: bit 2 p (low) / 2 p + 1 (high) of the element's byte
+                            const uint32_t y = (o ? r.f[Q5 ? i : 0][2 * h + w] >> 8 : r.f[Q5 ? i : 0][2 * h + w]) >> (2 * p);
+                            lb |= (y & 0x00010001u) << 4;
+                            hb |= (y & 0x00020002u) << 7;
+                        }
+                        lo[2 * w + o] = as_u32(__builtin_elementwise_fma(as_h2(lb), sc_lo, off_lo));
+                        hi[2 * w + o] = as_u32(__builtin_elementwise_fma(as_h2(hb), sc_hi, off_hi));
+                    }
+                }
+                put_piece(buf, 4 * part + i, h, t64, lane, lo);
+                put_piece(buf, 4 * part + 2 + i, h, t64, lane, hi);
+            }
+    }
+};
+
+// Q6_K: the stage is one 64-K pair; part h holds K 32 h .. 32 h + 31 = words 0..3 of unit 3 p + h and words 2 h, 2 h + 1 of
+// unit 3 p + 2 (the order of the nibbles and bit pairs is k_repack_q6k's)
+struct PromptQ6 {
+    static constexpr int TILE_BYTES = 13568, STAGE_K = 64, TERMS = 2, SPC = 4;
+    static constexpr bool UNITS = true, MINS = false;
+    struct Regs {
+        u32x4 n;
+        u32x2 hb;
+        uint32_t sc, d;
+    };
+    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
+        r.n = ((const u32x4*)tile)[(3 * sub + part) * 64 + lane];
+        r.hb = *(const u32x2*)(tile + ((3 * sub + 2) * 64 + lane) * 16 + 8 * part);
+        r.sc = *(const uint32_t*)(tile + 12288 + lane * 16 + 4 * sub);
+        r.d = *(const uint32_t*)(tile + 13312 + lane * 4);
+    }
+    static __device__ __forceinline__ void unpack(const Regs& r, const Bits& k, Unit& unit, float, uint8_t* buf, uint8_t*, float2* coef, int sub, int part,
+                                                  int t64, int lane) {
+        const float d = half_lo(r.d);
+        if (sub == 0) {
+            const float ratio = unit.enter(d);
+            if (part == 0) coef[t64 * 64 + lane] = float2{ratio, 0.0f};
+        }
+        const uint32_t sc2 = d == 0.0f ? 0u : r.sc >> (16 * part);
+#pragma unroll
+        for (int q = 0; q < 2; q++) {  // 16 K with one scale each
+            const int s8 = (int)(sc2 << (24 - 8 * q)) >> 24;
+            const half2v fa = pair_of((float)(s8 & ~15)), fb = pair_of((float)(s8 & 15));
+            const uint32_t H = r.hb[q];
+            u32x4 a[2], b[2];
+#pragma unroll
+            for (int s = 0; s < 4; s++)  // 4-K steps
+#pragma unroll
+                for (int ab = 0; ab < 2; ab++) {
+                    const int e = 2 * s + ab;
+                    const uint32_t lo = ((r.n[2 * q + (s >> 1)] >> ((s & 1) * 8 + 4 * ab)) & 0x000F000Fu) | k.k6400;
+                    const uint32_t v = lo | (((H >> (2 * e)) & 0x00030003u) << 4);
+                    const half2v lv = as_h2(v) + pair_of(-1056.0f);
+                    a[s >> 1][(s & 1) * 2 + ab] = as_u32(lv * fa);
+                    b[s >> 1][(s & 1) * 2 + ab] = as_u32(lv * fb);
+                }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                put_piece(buf, 2 * part + q, h, t64, lane, a[h]);
+                put_piece(buf, 4 + 2 * part + q, h, t64, lane, b[h]);
+            }
+        }
+    }
+};
+
+// Q8_0: 64 K = blocks 2 sub, 2 sub + 1 of the tile chunk, part = block
+struct PromptQ8 {
+    static constexpr int TILE_BYTES = 8704, STAGE_K = 64, TERMS = 2, SPC = 2;
+    static constexpr bool UNITS = false, MINS = false;
+    struct Regs {
+        u32x4 q[2];
+        uint32_t d;
+    };
+    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
+        const u32x4* p = (const u32x4*)tile + lane;
+        const int u = 4 * sub + 2 * part;
+        r.q[0] = p[u * 64];
+        r.q[1] = p[(u + 1) * 64];
+        r.d = *(const uint16_t*)(tile + 8192 + lane * 8 + 2 * (2 * sub + part));
+    }
+    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float rs, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
+                                                  int lane) {
+        const float d = half_lo(r.d) * rs;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                u32x4 hi, lo;
+#pragma unroll
+                for (int w = 0; w < 2; w++) {
+                    const uint32_t v = r.q[i][2 * h + w];
+                    float f[4];
+#pragma unroll
+                    for (int b = 0; b < 4; b++) f[b] = (float)((int)(v << (24 - 8 * b)) >> 24) * d;
+#pragma unroll
+                    for (int o = 0; o < 2; o++) {  // (0, 2) then (1, 3)
+                        const half2v t = {(_Float16)f[o], (_Float16)f[o + 2]};
+                        hi[2 * w + o] = as_u32(t);
+                        lo[2 * w + o] = as_u32(half2v{(_Float16)(f[o] - (float)t.x), (_Float16)(f[o + 2] - (float)t.y)});
+                    }
+                }
+                put_piece(buf, 2 * part + i, h, t64, lane, hi);
+                put_piece(buf, 4 + 2 * part + i, h, t64, lane, lo);
+            }
+    }
+};
+
+// MXFP4: sub-blocks 4 sub + 2 part, + 1 of the chunk; word w of a unit is eight K in operand order
+struct PromptMx {
+    static constexpr int TILE_BYTES = 8704, STAGE_K = 128, TERMS = 1, SPC = 2;
+    static constexpr bool UNITS = false, MINS = false;
+    struct Regs {
+        u32x4 q[2];
+        uint32_t e;
+    };
+    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
+        const u32x4* p = (const u32x4*)tile + lane;
+        const int u = 4 * sub + 2 * part;
+        r.q[0] = p[u * 64];
+        r.q[1] = p[(u + 1) * 64];
+        r.e = *(const uint16_t*)(tile + 8192 + lane * 8 + u);
+    }
+    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float rs, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
+                                                  int lane) {
+        const int shift = (int)(__float_as_uint(rs) >> 23) - 127;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int field = (int)((r.e >> (8 * i)) & 0xFF) + shift;  // 2^(e - 127) times the row's factor
+            const float sc = __uint_as_float((uint32_t)min(max(field, 1), 254) << 23);
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const uint32_t v = r.q[i][w];
+                const u32x4 o = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 0)),
+                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 1)),
+                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 2)),
+                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 3))};
+                put_piece(buf, 4 * part + 2 * i + (w >> 1), w & 1, t64, lane, o);
+            }
+        }
+    }
+};
+
+// bf16: a stage is one tile chunk of 64 K; part holds units 4 part .. 4 part + 3, eight K each in operand order
+struct PromptBf {
+    static constexpr int TILE_BYTES = 8192, STAGE_K = 64, TERMS = 1, SPC = 1;
+    static constexpr bool UNITS = false, MINS = false;
+    struct Regs {
+        u32x4 q[4];
+    };
+    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int, int part, int lane) {
+        const u32x4* p = (const u32x4*)tile + lane;
+#pragma unroll
+        for (int i = 0; i < 4; i++) r.q[i] = p[(4 * part + i) * 64];
+    }
+    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float rs, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
+                                                  int lane) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            u32x4 o;
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const uint32_t v = r.q[i][w];
+                o[w] = as_u32(half2v{(_Float16)(__uint_as_float(v << 16) * rs), (_Float16)(__uint_as_float(v & 0xFFFF0000u) * rs)});
+            }
+            put_piece(buf, 2 * part + (i >> 1), i & 1, t64, lane, o);
+        }
+    }
+};
+
+__device__ __forceinline__ float silu_prompt(float x) { return x / (1.0f + __expf(-x)); }
+
+template <class F>
+constexpr int stage_bytes() {
+    return F::STAGE_K / 16 * F::TERMS * STEP_BYTES;
+}
+template <class F>
+constexpr int lds_bytes() {
+    return (2 * stage_bytes<F>() < 65536 ? 65536 : 2 * stage_bytes<F>()) + 2 * CHUNK_BYTES;
+}
+
+template <class F, int WN, int EPI>
+__global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
+    constexpr int NT = 4 / WN, BM = 64 * (4 / WN), KS = F::STAGE_K / 16, GROUPS = KS / 2, STAGE = stage_bytes<F>();
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    uint8_t* const side = lds + lds_bytes<F>() - 2 * CHUNK_BYTES;  // [chunk % 2][min operands, coefficients]
+    auto mins_of = [&](int c) { return side + (c & 1) * CHUNK_BYTES; };
+    auto coef_of = [&](int c) { return (float2*)(side + (c & 1) * CHUNK_BYTES + MIN_BYTES); };
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave / WN, wn = wave % WN, t64 = wave >> 1, part = wave & 1;
+    // which tile: XCD x takes the column blocks x, x + 8, ..., all row blocks of one before the next
+    const int per_split = (g.nt + 7) / 8 * 8 * g.mt, split = blockIdx.x / per_split, id = blockIdx.x - split * per_split;
+    const int slot = id >> 3, nb = slot / g.mt * 8 + (id & 7), mb = slot % g.mt;
+    if (nb >= g.nt) return;
+    const int c0 = split * g.chunks_per_split, c1 = min(c0 + g.chunks_per_split, g.kchunks);
+    const int s0 = c0 * F::SPC, s1 = c1 * F::SPC;
+    const int tile = min(2 * nb + t64, g.n_tiles - 1);  // (an odd count: the last block's second half repeats the last tile)
+    const uint8_t* const wt = g.w + (size_t)tile * g.kchunks * F::TILE_BYTES;
+    const size_t rbs = (size_t)g.a_k16 * 1024;
+    const int rb0 = mb * (BM / 32) + wm * 2;
+    const uint8_t* const ap = g.a + (size_t)rb0 * rbs + lane * 16;
+    const float rs = F::UNITS ? 1.0f : g.rs[tile * 64 + lane];
+    Bits bits{0x64006400u, 0x54005400u};
+    asm volatile("" : "+v"(bits.k6400), "+v"(bits.k5400));
+
+    float16v acc[2][NT];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[t][j][i] = 0.f;
+    Unit unit;
+    typename F::Regs w;
+    u32x4 a[2][2][2];  // [ring][16-K step of the group][row block]
+    auto load_w = [&](int s, int sub) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int c = min(s, s1 - 1) / F::SPC;
+        F::load(w, wt + (size_t)c * F::TILE_BYTES, sub, part, lane);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_a = [&](int ring, int s, int grp) {
+        const uint8_t* p = ap + (size_t)(min(s, s1 - 1) * KS + 2 * grp) * 1024;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) a[ring][q][t] = *(const u32x4*)(p + t * rbs + q * 1024);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load_w(s0, 0);
+    load_a(0, s0, 0);
+    F::unpack(w, bits, unit, rs, lds, mins_of(c0), coef_of(c0), 0, part, t64, lane);
+    load_w(s0 + 1, 1 % F::SPC);
+    __syncthreads();
+    int buf = 0;
+    for (int s = s0; s < s1; s += F::SPC) {
+#pragma unroll
+        for (int sub = 0; sub < F::SPC; sub++) {
+            uint8_t* const cur = lds + buf * STAGE;
+            const bool last = s + sub + 1 >= s1;
+            const int c = s / F::SPC;
+            u32x4 sm[2];
+            if (F::UNITS && sub == 0) {
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const float into = coef_of(c)[(wn * NT + j) * 32 + (lane & 31)].x;
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++) acc[t][j][i] *= into;
+                }
+            }
+            if (F::MINS && sub == F::SPC - 1) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) sm[t] = *(const u32x4*)(g.asum + ((size_t)(rb0 + t) * (g.a_k16 >> 4) + c) * 1024 + lane * 16);
+            }
+            if (!last) {
+                F::unpack(w, bits, unit, rs, lds + (buf ^ 1) * STAGE, mins_of((s + sub + 1) / F::SPC), coef_of((s + sub + 1) / F::SPC), (sub + 1) % F::SPC, part, t64, lane);
+                load_w(s + sub + 2, (sub + 2) % F::SPC);
+            }
+#pragma unroll
+            for (int grp = 0; grp < GROUPS; grp++) {
+                constexpr int one = 1;
+                if (grp + 1 < GROUPS) load_a((grp + one) & 1, s + sub, grp + 1);
+                else load_a((grp + one) & 1, s + sub + 1, 0);
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+#pragma unroll
+                    for (int term = 0; term < F::TERMS; term++) {
+                        u32x4 b[NT];
+#pragma unroll
+                        for (int j = 0; j < NT; j++) b[j] = *(const u32x4*)(cur + (((term * KS + 2 * grp + q) * 4 + wn * NT + j) * 64 + lane) * 16);
+#pragma unroll
+                        for (int j = 0; j < NT; j++)
+#pragma unroll
+                            for (int t = 0; t < 2; t++)
+                                acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a[grp & 1][q][t]),
+                                                                                   __builtin_bit_cast(half8, b[j]), acc[t][j], 0, 0, 0);
+                    }
+            }
+            if (F::MINS && sub == F::SPC - 1) {
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const float into = coef_of(c)[(wn * NT + j) * 32 + (lane & 31)].y;
+                    const u32x4 mn = *(const u32x4*)(mins_of(c) + ((wn * NT + j) * 64 + lane) * 16);
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+#pragma unroll
+                        for (int i = 0; i < 16; i++) acc[t][j][i] *= into;
+                        acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, sm[t]), __builtin_bit_cast(half8, mn), acc[t][j], 0, 0, 0);
+                    }
+                }
+            }
+            __syncthreads();
+            buf ^= 1;
+        }
+    }
+    // the columns' units (or the rows' power-of-two factors taken back out)
+    float* const fin = (float*)side;
+    if (part == 0) fin[t64 * 64 + lane] = F::UNITS ? unit.u : 1.0f / rs;
+    __syncthreads();
+    float un[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) un[j] = fin[(wn * NT + j) * 32 + (lane & 31)];
+    // register i of a 32 x 32 block is row 8 (i / 4) + 4 (lane / 32) + i % 4, column lane % 32
+    if (EPI == EPI_PARTIAL) {
+        float* const out = (float*)g.out;
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            const int col = nb * 128 + (wn * NT + j) * 32 + (lane & 31);
+            if (col >= g.n_valid) continue;
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int row = (rb0 + t) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                    if (row < g.m) out[(((size_t)(row >> 4) * g.splits + split) * 16 + (row & 15)) * g.ldo + col] = acc[t][j][i] * un[j];
+                }
+        }
+        return;
+    }
+    // silu(gate) * up: column block 2 q of the tile is 32 gate rows, 2 q + 1 the matching up rows.  The products go through LDS
+    // into the order of the next matmul's activations
+    _Float16* const act = (_Float16*)lds;
+    auto put_act = [&](int q, int t, int i, float gate, float up) {
+        const int c = q * 32 + (lane & 31), row = (wm * 2 + t) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+        act[((((row >> 5) * 4 + (c >> 4)) * 2 + ((c >> 3) & 1)) * 32 + (row & 31)) * 8 + (c & 4) + (((c & 1) << 1) | ((c >> 1) & 1))] =
+            (_Float16)(silu_prompt(gate) * up);
+    };
+    if (NT >= 2) {
+#pragma unroll
+        for (int jq = 0; jq < NT / 2; jq++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    put_act((wn * NT) / 2 + jq, t, i, acc[t][2 * jq][i] * un[2 * jq], acc[t][(2 * jq + 1) % NT][i] * un[(2 * jq + 1) % NT]);
+    } else {
+        // a wave holds one column block: gate and up meet in LDS (behind the activations' area), wave (q, t) finishes row block t
+        float* const swap = (float*)(lds + 32768);
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) swap[((wn * 2 + t) * 16 + i) * 64 + lane] = acc[t][0][i] * un[0];
+        __syncthreads();
+        const int q = wave >> 1, t = wave & 1;
+#pragma unroll
+        for (int i = 0; i < 16; i++) put_act(q, t, i, swap[((2 * q * 2 + t) * 16 + i) * 64 + lane], swap[(((2 * q + 1) * 2 + t) * 16 + i) * 64 + lane]);
+    }
+    __syncthreads();
+    const int kvalid = g.n_valid;  // K of the next matmul
+    for (int p = threadIdx.x; p < BM * 8; p += 256) {
+        const int rb = p >> 8, k16 = nb * 4 + ((p >> 6) & 3);
+        if (k16 * 16 < kvalid)
+            *(u32x4*)((uint8_t*)g.out + (((size_t)(mb * (BM / 32) + rb) * g.out_k16 + k16) * 64 + (p & 63)) * 16) = ((const u32x4*)lds)[p];
+    }
+    if (g.out_sum) {
+        for (int p = threadIdx.x; p < BM * 2; p += 256) {
+            const int row = p >> 1, sub = p & 1, gs = nb * 2 + sub;
+            if (gs * 32 >= kvalid) continue;
+            float sum = 0.f;
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const half8 v = __builtin_bit_cast(half8, ((const u32x4*)lds)[((row >> 5) * 4 + 2 * sub + (x >> 1)) * 64 + (x & 1) * 32 + (row & 31)]);
+#pragma unroll
+                for (int e = 0; e < 8; e++) sum += (float)v[e];
+            }
+            sum *= PROMPT_SUM_SCALE;
+            const _Float16 hi = (_Float16)sum, lo = (_Float16)((sum - (float)hi) * PROMPT_SUM_LEFT);
+            _Float16* o = (_Float16*)(g.out_sum + ((size_t)(mb * (BM / 32) + (row >> 5)) * (g.out_k16 >> 4) + (gs >> 3)) * 1024) + (row & 31) * 8 + (gs & 7);
+            o[0] = hi;
+            o[256] = lo;
+        }
+    }
+}
+
+// ---- row factors ----------------------------------------------------------------------------------------------------------
+// The power of two that brings the largest magnitude of a row near the top of fp16's range: 2^7 for a Q8_0 scale (its product
+// with a code stays below 2^15), 2^12 for an MXFP4 block scale (times 6), 2^14 for a bf16 value.  One wave per tile.
+__global__ __launch_bounds__(64) void k_row_scale(const uint8_t* __restrict__ tiles, int fmt, int kchunks, float* __restrict__ rs) {
+    const int lane = threadIdx.x, tile = blockIdx.x;
+    const int tb = fmt == FMT_BF16 ? 8192 : 8704;
+    const uint8_t* t = tiles + (size_t)tile * kchunks * tb;
+    int e = -1000;  // exponent of the largest magnitude
+    for (int c = 0; c < kchunks; c++, t += tb) {
+        if (fmt == FMT_Q80) {
+            for (int j = 0; j < 4; j++) {
+                const float d = fabsf((float)*(const _Float16*)(t + 8192 + lane * 8 + 2 * j));
+                if (d > 0.f && d < INFINITY) e = max(e, ilogbf(d));
+            }
+        } else if (fmt == FMT_MX4) {
+            for (int j = 0; j < 8; j++) {
+                const int b = t[8192 + lane * 8 + j];
+                if (b < 255) e = max(e, b - 127);
+            }
+        } else {
+            for (int u = 0; u < 8; u++) {
+                const u32x4 q = ((const u32x4*)t)[u * 64 + lane];
+                for (int w = 0; w < 4; w++) {
+                    const int lo = (int)((q[w] >> 7) & 0xFF), hi = (int)((q[w] >> 23) & 0xFF);  // bf16 exponents
+                    if (lo && lo < 255) e = max(e, lo - 127);
+                    if (hi && hi < 255) e = max(e, hi - 127);
+                }
+            }
+        }
+    }
+    const int top = fmt == FMT_Q80 ? 7 : fmt == FMT_MX4 ? 12 : 14;
+    const int s = e == -1000 ? 0 : min(max(top - e, -126), 126);
+    rs[tile * 64 + lane] = __uint_as_float((uint32_t)(s + 127) << 23);
+}
+
+template <class F, int WN, int EPI>
+int launch_p(hipStream_t s, const PromptGemmArgs& g) {
+    static bool raised = false;  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
+    if (!raised) {
+        TSV_HIP(hipFuncSetAttribute((const void*)k_prompt_gemm<F, WN, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<F>()));
+        raised = true;
+    }
+    const int blocks = (g.nt + 7) / 8 * 8 * g.mt * g.splits;
+    hipLaunchKernelGGL((k_prompt_gemm<F, WN, EPI>), dim3(blocks), dim3(256), lds_bytes<F>(), s, g);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+template <class F>
+int launch_f(hipStream_t s, PromptGemmArgs& g, int epi, int bm) {
+    g.mt = (g.m + bm - 1) / bm;
+    if (epi == EPI_SILU) return bm == 256 ? launch_p<F, 1, EPI_SILU>(s, g) : bm == 128 ? launch_p<F, 2, EPI_SILU>(s, g) : launch_p<F, 4, EPI_SILU>(s, g);
+    return bm == 256 ? launch_p<F, 1, EPI_PARTIAL>(s, g) : bm == 128 ? launch_p<F, 2, EPI_PARTIAL>(s, g) : launch_p<F, 4, EPI_PARTIAL>(s, g);
+}
+
+int row_block(int m) {
+    static const int forced = [] {
+        const char* e = getenv("TSV_PROMPT_BM");
+        return e ? atoi(e) : 0;
+    }();
+    return forced ? forced : m > 128 ? 256 : m > 64 ? 128 : 64;
+}
+
+}  // namespace
+
+bool prompt_fmt_has_sums(int fmt) { return fmt == FMT_Q4K || fmt == FMT_Q5K; }
+
+int launch_row_scale(hipStream_t s, const TiledW& w, float* rs) {
+    hipLaunchKernelGGL(k_row_scale, dim3(w.n_tiles), dim3(64), 0, s, w.tiles, w.fmt, w.kchunks, rs);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int prompt_splits(const TiledW& w, int m) {
+    const int bm = row_block(m), tiles = (m + bm - 1) / bm * ((w.n_tiles + 1) / 2);
+    int sp = std::min(std::min(8, w.kchunks), std::max(1, 512 / std::max(1, tiles)));
+    const int per = (w.kchunks + sp - 1) / sp;
+    return (w.kchunks + per - 1) / per;
+}
+
+int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int m, int splits, int epi,
+                       int ldo, int n_valid) {
+    if (m < 1 || (epi != EPI_PARTIAL && epi != EPI_SILU) || (epi == EPI_SILU && w.n_rows % 64) || splits < 1 || splits > 8 ||
+        (epi == EPI_SILU && splits != 1) || (prompt_fmt_has_sums(w.fmt) && !asum) ||
+        (!w.row_scale && (w.fmt == FMT_Q80 || w.fmt == FMT_BF16 || w.fmt == FMT_MX4))) {
+        set_error("prompt matmul: bad argument");
+        return TSV_ERR_INVALID;
+    }
+    PromptGemmArgs g{};
+    g.w = w.tiles;
+    g.a = (const uint8_t*)a;
+    g.asum = (const uint8_t*)asum;
+    g.rs = w.row_scale;
+    g.out = out;
+    g.out_sum = (uint8_t*)out_sum;
+    g.m = m;
+    g.n_tiles = w.n_tiles;
+    g.kchunks = w.kchunks;
+    g.chunks_per_split = (w.kchunks + splits - 1) / splits;
+    g.splits = (w.kchunks + g.chunks_per_split - 1) / g.chunks_per_split;
+    if (g.splits != splits) {
+        set_error("prompt matmul: split count leaves an empty K slice");
+        return TSV_ERR_INVALID;
+    }
+    g.ldo = ldo;
+    g.a_k16 = prompt_k16(w.k);
+    g.nt = (w.n_tiles + 1) / 2;
+    g.n_valid = epi == EPI_SILU ? w.n_rows / 2 : n_valid;
+    g.out_k16 = prompt_k16(w.n_rows / 2);
+    const int bm = row_block(m);
+    return w.fmt == FMT_Q4K    ? launch_f<PromptQ45<false>>(s, g, epi, bm)
+           : w.fmt == FMT_Q5K  ? launch_f<PromptQ45<true>>(s, g, epi, bm)
+           : w.fmt == FMT_Q6K  ? launch_f<PromptQ6>(s, g, epi, bm)
+           : w.fmt == FMT_Q80  ? launch_f<PromptQ8>(s, g, epi, bm)
+           : w.fmt == FMT_BF16 ? launch_f<PromptBf>(s, g, epi, bm)
+                               : launch_f<PromptMx>(s, g, epi, bm);
+}
+
+}  // namespace tsv

@@ -1,0 +1,212 @@
+// Prompt passes: the launch sequence of hundreds of consecutive rows through the decoder (crates/runtime/src/producer.rs:122-150,
+// the chunked prefill runner; families/llama/prefill.rs).  A pass takes up to PROMPT_ROWS rows, so that a matmul reads its
+// weights once for all of them and is bound by the matrix pipes; everything between the matmuls runs over all rows at once
+// (prompt.hip).  Rows are cached before any of them attends, as in the reference's batched prefill.
+#include "ctx.h"
+#include "prompt.h"
+
+namespace tsv {
+
+bool prompt_supported(const tsv_ctx* c) {
+    if (c->mtp.on) return false;
+    for (const LayerW& L : c->layers)
+        if (L.n_experts || L.cap < c->ctx_alloc || L.tq.k_bits) return false;
+    return true;
+}
+
+void prompt_free(tsv_ctx* c) {
+    for (void* p : c->prompt.allocs) (void)hipFree(p);
+    c->prompt.allocs.clear();
+    c->prompt.rows = 0;
+}
+
+namespace {
+
+template <class T>
+int prompt_alloc(tsv_ctx* c, T** p, size_t bytes, bool zero) {
+    void* q = nullptr;
+    TSV_HIP(hipMalloc(&q, bytes));
+    c->prompt.allocs.push_back(q);
+    if (zero) TSV_HIP(hipMemsetAsync(q, 0, bytes, c->stream));
+    *p = (T*)q;
+    return TSV_OK;
+}
+
+// Buffers for n rows.  The activations are cleared once: the K padding behind a width that is not whole 256s has to stay zero,
+// and rows past the last one have to hold finite values.
+int prompt_reserve(tsv_ctx* c, int n) {
+    tsv_ctx::Prompt& w = c->prompt;
+    if (n <= w.rows) return TSV_OK;
+    const int rows = n <= 256 ? 256 : n <= 1024 ? 1024 : PROMPT_ROWS;
+    if (w.rows) {
+        TSV_HIP(hipStreamSynchronize(c->stream));
+        prompt_free(c);
+    }
+    const int qd = c->nq * c->hd;
+    size_t width = (size_t)qd + 2 * c->nkv * c->hd;
+    for (const LayerW& L : c->layers)
+        for (const TiledW* t : {&L.wo, &L.down}) width = std::max(width, (size_t)t->n_rows);
+    // one partial sum per row and column, or as many as fill the chip: at most 512 tiles of 256 x 128 (prompt_splits), by half more
+    // where q and k are split by themselves and the value columns come on top
+    w.partial_floats = std::max((size_t)rows * width, std::min((size_t)8 * rows * width, (size_t)512 * 256 * 128 * 3 / 2));
+    int rc;
+    if ((rc = prompt_alloc(c, &w.x, (size_t)rows * c->hidden * 4, false)) || (rc = prompt_alloc(c, &w.a_h, prompt_a_bytes(rows, c->hidden), true)) ||
+        (rc = prompt_alloc(c, &w.s_h, prompt_sum_bytes(rows, c->hidden), true)) || (rc = prompt_alloc(c, &w.a_q, prompt_a_bytes(rows, qd), true)) ||
+        (rc = prompt_alloc(c, &w.s_q, prompt_sum_bytes(rows, qd), true)) || (rc = prompt_alloc(c, &w.a_f, prompt_a_bytes(rows, c->ffn), true)) ||
+        (rc = prompt_alloc(c, &w.s_f, prompt_sum_bytes(rows, c->ffn), true)) || (rc = prompt_alloc(c, &w.partial, w.partial_floats * 4, false)) ||
+        (rc = prompt_alloc(c, &w.q16, (size_t)rows * qd * 2, false)) || (rc = prompt_alloc(c, &w.cs, (size_t)rows * (c->hd / 2) * sizeof(float2), false)) ||
+        (rc = prompt_alloc(c, &w.ids, (size_t)rows * 4, false)) || (rc = prompt_alloc(c, &w.part_o, (size_t)512 * 128 * c->hd * 4, false)) ||
+        (rc = prompt_alloc(c, &w.part_ml, (size_t)512 * 128 * 2 * 4, false)))
+        return rc;
+    w.rows = rows;
+    return TSV_OK;
+}
+
+// one split count for a projection whose value part has a storage type of its own
+int common_splits(const TiledW& a, const TiledW& b, int n) {
+    auto fits = [](const TiledW& t, int k) {
+        const int per = (t.kchunks + k - 1) / k;
+        return (t.kchunks + per - 1) / per == k;
+    };
+    int sp = prompt_splits(a, n);
+    while (sp > 1 && !(fits(a, sp) && fits(b, sp))) sp--;
+    return sp;
+}
+
+int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits) {
+    hipStream_t s = c->stream;
+    tsv_ctx::Prompt& w = c->prompt;
+    const int H = c->hidden, qd = c->nq * c->hd, qkv_n = (c->nq + 2 * c->nkv) * c->hd;
+    int rc = launch_prompt_embed(s, c->embed_raw, c->embed_dtype, H, w.x, w.ids, n, (int)base, c->freqs, c->rope_mscale, c->hd / 2, w.cs);
+    if (rc) return rc;
+    PromptNormArgs na{};
+    na.x = w.x;
+    na.partial = w.partial;
+    na.n = n;
+    na.hidden = na.ldp = H;
+    na.eps = c->eps;
+    na.a = w.a_h;
+    auto norm = [&](const float* weight, int splits, const float* bias, const TiledW& next) {
+        na.w = weight;
+        na.splits = na.slots = splits;
+        na.bias = bias;
+        na.asum = prompt_fmt_has_sums(next.fmt) ? w.s_h : nullptr;
+        return launch_prompt_norm(s, na);
+    };
+    int sp = 0;
+    for (int l = 0; l < c->n_layers; l++) {
+        LayerW& L = c->layers[l];
+        if ((rc = norm(L.attn_norm, sp, nullptr, prompt_fmt_has_sums(L.qkv.fmt) || !L.v_only.tiles ? L.qkv : L.v_only))) return rc;
+        sp = L.v_only.tiles ? common_splits(L.qkv, L.v_only, n) : prompt_splits(L.qkv, n);
+        if ((rc = launch_prompt_gemm(s, L.qkv, w.a_h, w.s_h, w.partial, nullptr, n, sp, EPI_PARTIAL, qkv_n, L.qkv.n_rows))) return rc;
+        if (L.v_only.tiles &&
+            (rc = launch_prompt_gemm(s, L.v_only, w.a_h, w.s_h, w.partial + L.qkv.n_rows, nullptr, n, sp, EPI_PARTIAL, qkv_n, L.v_only.n_rows)))
+            return rc;
+        PromptRopeArgs ra{};
+        ra.qkv = w.partial;
+        ra.splits = sp;
+        ra.ldq = qkv_n;
+        ra.n = n;
+        ra.base = (int)base;
+        ra.cs = w.cs;
+        ra.bias = L.bqkv;
+        ra.q_norm = L.q_norm;
+        ra.k_norm = L.k_norm;
+        ra.eps = c->eps;
+        ra.q16 = w.q16;
+        ra.kc = L.kc;
+        ra.vc = L.vc;
+        ra.nq = c->nq;
+        ra.nkv = c->nkv;
+        ra.hd = c->hd;
+        ra.cap = L.kv_slots;
+        ra.paired = L.rope_fused && c->hd == 128;
+        if ((rc = launch_prompt_rope(s, ra))) return rc;
+        PromptAttnArgs aa{};
+        aa.q16 = w.q16;
+        aa.kc = L.kc;
+        aa.vc = L.vc;
+        aa.n = n;
+        aa.base = (int)base;
+        aa.nq = c->nq;
+        aa.nkv = c->nkv;
+        aa.hd = c->hd;
+        aa.cap = L.cap;
+        aa.window = L.window;
+        aa.scale = c->attn_scale;
+        aa.sinks = L.sinks;
+        aa.a = w.a_q;
+        aa.asum = prompt_fmt_has_sums(L.wo.fmt) ? w.s_q : nullptr;
+        aa.part_o = w.part_o;
+        aa.part_ml = w.part_ml;
+        aa.nch = prompt_attn_chunks(n, (int)base, c->nq, c->nkv, L.window);
+        if ((rc = launch_prompt_attention(s, aa))) return rc;
+        sp = prompt_splits(L.wo, n);
+        if ((rc = launch_prompt_gemm(s, L.wo, w.a_q, w.s_q, w.partial, nullptr, n, sp, EPI_PARTIAL, H, H)) ||
+            (rc = norm(L.ffn_norm, sp, L.bo, L.gate_up)) ||
+            (rc = launch_prompt_gemm(s, L.gate_up, w.a_h, w.s_h, w.a_f, prompt_fmt_has_sums(L.down.fmt) ? w.s_f : nullptr, n, 1, EPI_SILU, 0, 0)))
+            return rc;
+        sp = prompt_splits(L.down, n);
+        if ((rc = launch_prompt_gemm(s, L.down, w.a_f, w.s_f, w.partial, nullptr, n, sp, EPI_PARTIAL, H, H))) return rc;
+    }
+    (void)qd;
+    if (!finish && !logits) return TSV_OK;
+    const int m = (n - 1) % 16 + 1, t0 = n - m;
+    int tail_splits = sp;
+    if (finish) {  // the rows as a drafter head reads them
+        na.a = nullptr;
+        na.w = na.bias = nullptr;
+        na.splits = na.slots = sp;
+        if ((rc = launch_prompt_norm(s, na))) return rc;
+        tail_splits = 0;
+    }
+    TSV_HIP(hipMemcpyAsync(c->x, w.x + (size_t)t0 * H, (size_t)m * H * 4, hipMemcpyDeviceToDevice, s));
+    if ((rc = launch_addnorm(s, c->x, w.partial + (size_t)(t0 / 16) * sp * 16 * H, tail_splits, H, c->final_norm, c->eps, H, c->xf_a, m))) return rc;
+    if (!logits) return TSV_OK;
+    return launch_gemm(s, c->head, c->xf_a, c->logits, c->vp_dev, m, 1, EPI_LOGITS, c->vocab, c->vocab);
+}
+
+}  // namespace
+
+int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits) {
+    if (base != c->position) {
+        set_error("prefill: start position does not match the KV cursor");
+        return TSV_ERR_INVALID;
+    }
+    if (base + n > c->max_context) {
+        set_error("prefill: block would write past the KV capacity");
+        return TSV_ERR_INVALID;
+    }
+    if (n < PROMPT_MIN_ROWS || n > PROMPT_ROWS) {
+        set_error("prefill: rows of a prompt pass");
+        return TSV_ERR_INVALID;
+    }
+    for (int i = 0; i < n; i++)
+        if (ids[i] < 0 || ids[i] >= c->vocab) {
+            set_error("verify: token id outside the vocabulary");
+            return TSV_ERR_INVALID;
+        }
+    int rc = prompt_reserve(c, n);
+    if (rc) return rc;
+    // (from the caller's pageable memory: the runtime has taken its copy when this returns)
+    TSV_HIP(hipMemcpyAsync(c->prompt.ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
+    const int m = (n - 1) % 16 + 1;
+    VerifyParams vp;
+    if (logits) {  // the last rows are left as a verify pass of their own would leave them
+        if ((rc = fill_params(vp, ids + n - m, nullptr, m, base + n - m, c->vocab))) return rc;
+        *c->vp_host = vp;
+        if ((rc = stage_params(c, &vp, 1, c->vp_dev))) return rc;
+    }
+    if ((rc = launch_prompt_pass(c, n, base, finish, logits))) return rc;
+    c->position = base + n;
+    c->high_water = std::max(c->high_water, c->position);
+    c->last_m = logits ? m : 0;
+    c->last_base = base + n - m;
+    if (logits) c->last_shape_known = true;
+    c->x_base = base + n - m;
+    c->x_rows = finish || logits ? m : 0;
+    if (c->mtp_head) c->mtp_head->mtp.own_valid = false;
+    return TSV_OK;
+}
+
+}  // namespace tsv

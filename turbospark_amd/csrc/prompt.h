@@ -1,0 +1,94 @@
+// What the prompt passes share (producer.rs:122-150, the chunked prefill runner; families/llama/prefill.rs): a pass of up to
+// PROMPT_ROWS consecutive positions whose matmuls are real contractions (gemm_prompt.hip), with embedding, norms, rotation
+// and attention over all of its rows at once (prompt.hip).
+//
+// Activations of a matmul are kept as ready A operands of v_mfma_f32_32x32x16_f16: blocks of 32 rows, each
+// [K / 16][64 lanes][8 halfs], lane (row % 32) + 32 * (k % 16 / 8) holding its row's eight values of the step, in the
+// order 0 2 1 3 inside every four (what the nibble unpack of the weights produces).  K is padded to whole 256s with zeros.
+// Formats with a min term (Q4_K, Q5_K) need the sums of every 32 values as well; they are kept as an A operand of the same
+// instruction, one per 256 K: [K / 256][64 lanes][8 halfs], lane row % 32 the eight sub-block sums / 64 rounded to fp16, lane
+// 32 + row % 32 what that rounding left over, times 2048 -- 22 bits of the sum between them.
+#pragma once
+#include "tsv_internal.h"
+
+namespace tsv {
+
+constexpr int PROMPT_ROWS = 2048;     // most rows of one pass
+constexpr int PROMPT_MIN_ROWS = 64;   // fewer go in verify-sized passes
+constexpr float PROMPT_SUM_SCALE = 1.0f / 64.0f, PROMPT_SUM_LEFT = 2048.0f;
+
+__host__ __device__ inline int prompt_k16(int k) { return (k + 255) / 256 * 16; }
+__host__ __device__ inline int prompt_chunks(int k) { return (k + 255) / 256; }
+// halfs from the start of the activations to element (row, k) of a K-wide input
+__host__ __device__ inline size_t prompt_a_index(int row, int k, int k16) {
+    return (((size_t)(row >> 5) * k16 + (k >> 4)) * 64 + ((k >> 3) & 1) * 32 + (row & 31)) * 8 + (k & 4) + (((k & 1) << 1) | ((k >> 1) & 1));
+}
+__host__ __device__ inline size_t prompt_a_bytes(int rows, int k) { return (size_t)((rows + 31) / 32) * prompt_k16(k) * 1024; }
+__host__ __device__ inline size_t prompt_sum_bytes(int rows, int k) { return (size_t)((rows + 31) / 32) * prompt_chunks(k) * 1024; }
+
+// Rows are padded to whole 256-row tiles in every activation buffer: the padding is read (its products are never stored)
+inline int prompt_padded(int rows) { return (rows + 255) / 256 * 256; }
+
+struct PromptGemmArgs {
+    const uint8_t* w;     // row tiles (TiledW)
+    const uint8_t* a;     // activations
+    const uint8_t* asum;  // their sums (formats with a min term)
+    const float* rs;      // power-of-two factor of every tiled row (formats without a scale per chunk), see row_scale
+    void* out;            // EPI_PARTIAL: float [m / 16][splits][16][ldo]; EPI_SILU: the next matmul's activations
+    uint8_t* out_sum;     // EPI_SILU, nullable: their sums
+    int m, n_tiles, kchunks, chunks_per_split, splits, ldo, n_valid;
+    int a_k16;            // 16-K steps per row of the activations
+    int out_k16;
+    int mt, nt;           // tiles of the grid: rows, 128 columns
+};
+
+int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int m, int splits, int epi,
+                       int ldo, int n_valid);
+int prompt_splits(const TiledW& w, int m);
+// the power-of-two factors of a tiled matrix's rows, n_tiles * 64 floats (Q8_0, bf16, MXFP4)
+int launch_row_scale(hipStream_t s, const TiledW& w, float* rs);
+bool prompt_fmt_has_sums(int fmt);
+
+// residual rows x [n][hidden] += the partial sums of the matmul before (PromptGemmArgs::out); then, with w, their RMSNorm, as
+// the next matmul's activations (w NULL and a non-NULL: the rows themselves; a NULL: the residual add alone)
+struct PromptNormArgs {
+    float* x;
+    const float* partial;   // [n / 16][splits][16][ldp]; routed: [n / 16][8 slots][16][hidden] with `weights`
+    const float* weights;   // nullable: [n][8] factors of the slots
+    const float* bias;      // nullable, added after the partial sums
+    const float* w;
+    uint8_t *a, *asum;      // asum nullable
+    int n, hidden, splits, ldp, slots;  // slots: distance of the partials in rows of sixteen (splits, or 8)
+    float eps;
+};
+int launch_prompt_norm(hipStream_t s, const PromptNormArgs& a);
+// embedding rows of ids[0, n), and the rotation table of positions base ..
+int launch_prompt_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float* x, const int32_t* ids, int n, int base, const float* freqs,
+                        float mscale, int half, float2* cs);
+
+// bias, per-head norm, rotation; q as fp16 rows, K and V into the cache
+struct PromptRopeArgs {
+    const float* qkv;  // [n / 16][splits][16][ldq]
+    int splits, ldq, n, base;
+    const float2* cs;  // [n][hd / 2]
+    const float *bias, *q_norm, *k_norm;
+    float eps;
+    uint16_t *q16, *kc, *vc;
+    int nq, nkv, hd, cap;  // cap: positions of the cache, position p in slot p % cap
+    int paired;            // as in RopeKvArgs
+};
+int launch_prompt_rope(hipStream_t s, const PromptRopeArgs& a);
+
+struct PromptAttnArgs {
+    const uint16_t *q16, *kc, *vc;
+    int n, base, nq, nkv, hd, cap, window;
+    float scale;
+    const float* sinks;
+    uint8_t *a, *asum;      // the output projection's activations (K index = head * hd + d) and sums
+    float *part_o, *part_ml;  // nch > 1: [nch][nkv][n * G][hd] and [nch][nkv][n * G][2]
+    int nch;
+};
+int prompt_attn_chunks(int n, int base, int nq, int nkv, int window);
+int launch_prompt_attention(hipStream_t s, const PromptAttnArgs& a);
+
+}  // namespace tsv

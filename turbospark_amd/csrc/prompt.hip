@@ -1,0 +1,540 @@
+// What a prompt pass does between its matmuls, over all of its rows at once: embedding, residual add + RMSNorm, rotation and
+// cache stores, attention (crates/runtime/src/families/llama/{prefill,attn}.rs).  The verify passes' kernels (misc.hip,
+// attn.hip) take sixteen rows and read tree shapes from device memory; here rows are consecutive positions, so a row's number
+// says everything about it.
+#include <algorithm>
+#include <type_traits>
+
+#include "embed_row.h"
+#include "prompt.h"
+
+namespace tsv {
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// ---- embedding --------------------------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_prompt_embed(const uint8_t* __restrict__ raw, int dtype, int hidden, float* __restrict__ x,
+                                                      const int32_t* __restrict__ ids, int base, const float* __restrict__ freqs, float mscale,
+                                                      int half, float2* __restrict__ cs) {
+    const int row = blockIdx.x;
+    const long tok = ids[row];
+    for (int e = threadIdx.x; e < hidden; e += 256) x[(size_t)row * hidden + e] = embed_elem(raw, dtype, hidden, tok, e);
+    const float pos = (float)(base + row);
+    for (int i = threadIdx.x; i < half; i += 256) {
+        float sn, c;
+        sincosf(pos * freqs[i], &sn, &c);
+        cs[(size_t)row * half + i] = float2{c * mscale, sn * mscale};
+    }
+}
+
+// ---- residual add + RMSNorm -------------------------------------------------------------------------------------------------
+// Eight values (consecutive K) of a row as activations, and the sum of its 32-value sub-block, whose other values sit in the
+// three neighbouring lanes.  The halves are pinned in registers between the store and the sum: the sum has to be that of the
+// stored bits (pinned_half).
+__device__ __forceinline__ void put_activations(uint8_t* a, uint8_t* asum, int row, int k, int k16, const float (&v)[8], bool live) {
+    half8 h = {(_Float16)v[0], (_Float16)v[2], (_Float16)v[1], (_Float16)v[3], (_Float16)v[4], (_Float16)v[6], (_Float16)v[5], (_Float16)v[7]};
+    u32x4 b = __builtin_bit_cast(u32x4, h);
+    asm volatile("" : "+v"(b.x), "+v"(b.y), "+v"(b.z), "+v"(b.w));
+    if (live) *(u32x4*)(a + (((size_t)(row >> 5) * k16 + (k >> 4)) * 64 + ((k >> 3) & 1) * 32 + (row & 31)) * 16) = b;
+    if (asum) {
+        h = __builtin_bit_cast(half8, b);
+        float s = (((float)h[0] + (float)h[1]) + ((float)h[2] + (float)h[3])) + (((float)h[4] + (float)h[5]) + ((float)h[6] + (float)h[7]));
+        s += __shfl_xor(s, 1);
+        s += __shfl_xor(s, 2);
+        if (live && (k & 31) == 0) {
+            s *= PROMPT_SUM_SCALE;
+            const _Float16 hi = (_Float16)s, lo = (_Float16)((s - (float)hi) * PROMPT_SUM_LEFT);
+            _Float16* o = (_Float16*)(asum + ((size_t)(row >> 5) * (k16 >> 4) + (k >> 8)) * 1024) + (row & 31) * 8 + ((k >> 5) & 7);
+            o[0] = hi;
+            o[256] = lo;
+        }
+    }
+}
+
+// One wave per row, the row in registers (NV x 512 values); eight rows to a workgroup, so that the sixteen-byte pieces its
+// waves write side by side fill cache lines.  The partial sums are added in order, every split's loads in flight together.
+template <int NV, bool ROUTED>
+__global__ __launch_bounds__(512) void k_prompt_norm(PromptNormArgs p) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 8 + (threadIdx.x >> 6);
+    if (row >= p.n) return;
+    float* const xr = p.x + (size_t)row * p.hidden;
+    float v[NV][8];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int k = i * 512 + lane * 8;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 t = k < p.hidden ? *(const float4*)(xr + k + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
+            v[i][4 * h] = t.x, v[i][4 * h + 1] = t.y, v[i][4 * h + 2] = t.z, v[i][4 * h + 3] = t.w;
+        }
+    }
+    float r[ROUTED ? NV : 1][8];
+    if (ROUTED) {
+#pragma unroll
+        for (int i = 0; i < NV; i++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) r[i][e] = 0.f;
+    }
+    for (int s = 0; s < p.splits; s++) {
+        const float* pr = p.partial + (((size_t)(row >> 4) * p.slots + s) * 16 + (row & 15)) * p.ldp;
+        const float ws = ROUTED ? p.weights[(size_t)row * 8 + s] : 1.0f;
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int k = i * 512 + lane * 8;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const float4 t = k < p.hidden ? *(const float4*)(pr + k + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
+                const float f[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    // routed experts (families/llama/moe.rs:193-198): the slots' outputs are weighted and summed in rank order
+                    // from zero, then added to the stream; product and sum rounded apart
+                    if (ROUTED) r[i][4 * h + e] = __fadd_rn(r[i][4 * h + e], __fmul_rn(ws, f[e]));
+                    else v[i][4 * h + e] = __fadd_rn(v[i][4 * h + e], f[e]);
+                }
+            }
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int k = i * 512 + lane * 8;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            if (ROUTED) v[i][e] = __fadd_rn(v[i][e], r[i][e]);
+            if (p.bias && k < p.hidden) v[i][e] += p.bias[k + e];
+            ss += v[i][e] * v[i][e];
+        }
+        if (p.splits && k < p.hidden) {
+            *(float4*)(xr + k) = float4{v[i][0], v[i][1], v[i][2], v[i][3]};
+            *(float4*)(xr + k + 4) = float4{v[i][4], v[i][5], v[i][6], v[i][7]};
+        }
+    }
+    if (!p.a) return;
+    float inv = 1.0f;
+    if (p.w) {
+        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        inv = 1.0f / sqrtf(ss / (float)p.hidden + p.eps);
+    }
+    const int k16 = prompt_k16(p.hidden);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int k = i * 512 + lane * 8;
+        const bool live = k < p.hidden;
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = p.w ? v[i][e] * (live ? p.w[k + e] : 0.f) * inv : v[i][e];
+        put_activations(p.a, p.asum, row, k, k16, o, live);
+    }
+}
+
+// The same for rows wider than a wave's registers hold: the row is read again after its sum of squares.
+template <bool ROUTED>
+__global__ __launch_bounds__(512) void k_prompt_norm_long(PromptNormArgs p) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 8 + (threadIdx.x >> 6);
+    if (row >= p.n) return;
+    float* const xr = p.x + (size_t)row * p.hidden;
+    float ss = 0.f;
+    for (int k = lane * 8; k < p.hidden; k += 512) {
+        float v[8], r[8] = {};
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = xr[k + e];
+        for (int s = 0; s < p.splits; s++) {
+            const float* pr = p.partial + (((size_t)(row >> 4) * p.slots + s) * 16 + (row & 15)) * p.ldp + k;
+            const float ws = ROUTED ? p.weights[(size_t)row * 8 + s] : 1.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if (ROUTED) r[e] = __fadd_rn(r[e], __fmul_rn(ws, pr[e]));
+                else v[e] = __fadd_rn(v[e], pr[e]);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            if (ROUTED) v[e] = __fadd_rn(v[e], r[e]);
+            if (p.bias) v[e] += p.bias[k + e];
+            ss += v[e] * v[e];
+            if (p.splits) xr[k + e] = v[e];
+        }
+    }
+    if (!p.a) return;
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    const float inv = p.w ? 1.0f / sqrtf(ss / (float)p.hidden + p.eps) : 1.0f;
+    const int k16 = prompt_k16(p.hidden);
+    for (int k0 = 0; k0 < p.hidden; k0 += 512) {  // (whole waves: the sub-block sums cross lanes)
+        const int k = k0 + lane * 8;
+        const bool live = k < p.hidden;
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = live ? (p.w ? xr[k + e] * p.w[k + e] * inv : xr[k + e]) : 0.f;
+        put_activations(p.a, p.asum, row, k, k16, o, live);
+    }
+}
+
+// ---- rotation + cache stores --------------------------------------------------------------------------------------------------
+// One workgroup per (block of sixteen cache positions, head): a K or V block of the head is one contiguous run of the cache
+// (kcache_index / vcache_index), put together in LDS and written sixteen bytes at a time.  Element by element from one wave per
+// (row, head), as the verify passes do it, a pass of 2048 rows is 98 000 waves of two-byte stores.
+template <int HD>
+__global__ __launch_bounds__(256) void k_prompt_rope(PromptRopeArgs p) {
+    constexpr int HALF = HD / 2, LANES = HALF, RPI = 256 / LANES;  // rows per iteration
+    __shared__ _Float16 sh[16][HD + 8];
+    const int head = blockIdx.y, pb = (p.base >> 4) + blockIdx.x;
+    const int kind = head < p.nq ? 0 : head < p.nq + p.nkv ? 1 : 2;
+    const int h = kind == 0 ? head : kind == 1 ? head - p.nq : head - p.nq - p.nkv;
+    const int i = threadIdx.x % LANES, col = head * HD;
+    const bool paired = p.paired && kind != 2;
+    const int c0 = paired ? (i >> 5) * 64 + (i & 31) : i, c1 = paired ? c0 + 32 : i + HALF;
+    const float b0 = p.bias ? p.bias[col + i] : 0.f, b1 = p.bias ? p.bias[col + i + HALF] : 0.f;
+    const float* nw = kind == 0 ? p.q_norm : kind == 1 ? p.k_norm : nullptr;
+#pragma unroll
+    for (int it = 0; it < 16 / RPI; it++) {
+        const int slot = it * RPI + threadIdx.x / LANES, row = pb * 16 + slot - p.base;
+        const bool live = row >= 0 && row < p.n;
+        float x0 = 0.f, x1 = 0.f;
+        if (live) {
+            const float* q = p.qkv + ((size_t)(row >> 4) * p.splits * 16 + (row & 15)) * p.ldq + col;
+            for (int s = 0; s < p.splits; s++, q += (size_t)16 * p.ldq) {
+                x0 += q[c0];
+                x1 += q[c1];
+            }
+            if (p.bias) {  // before the rotation (families/gptoss/attn.rs:88-101)
+                x0 += b0;
+                x1 += b1;
+            }
+        }
+        if (nw) {  // RMSNorm over the head (families/llama/state.rs:344-347)
+            float ss = x0 * x0 + x1 * x1;
+            for (int o = LANES / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+            const float inv = 1.0f / sqrtf(ss / (float)HD + p.eps);
+            x0 = x0 * nw[i] * inv;
+            x1 = x1 * nw[i + HALF] * inv;
+        }
+        if (kind != 2 && live) {  // NeoX pairs (i, i + hd / 2) (crates/compute/src/rope.rs:208-256)
+            const float2 cs = p.cs[(size_t)row * HALF + i];
+            const float r0 = x0 * cs.x - x1 * cs.y, r1 = x0 * cs.y + x1 * cs.x;
+            x0 = r0;
+            x1 = r1;
+        }
+        sh[slot][i] = (_Float16)x0;
+        sh[slot][i + HALF] = (_Float16)x1;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t >= 16 * HD / 8) return;
+    if (kind == 0) {
+        const int slot = t / (HD / 8), d = t % (HD / 8) * 8, row = pb * 16 + slot - p.base;
+        if (row >= 0 && row < p.n) *(u32x4*)((_Float16*)p.q16 + ((size_t)row * p.nq + h) * HD + d) = *(const u32x4*)&sh[slot][d];
+        return;
+    }
+    const long blk = ((long)h * (p.cap >> 4) + pb % (p.cap >> 4)) * (16 * HD);
+    if (kind == 1) {  // piece t: dims 32 (t / 64) + 8 (t % 64 / 16) .. of position t % 16
+        const int slot = t & 15, d = (t >> 6) * 32 + ((t >> 4) & 3) * 8, row = pb * 16 + slot - p.base;
+        if (row >= 0 && row < p.n) *(u32x4*)((_Float16*)p.kc + blk + t * 8) = *(const u32x4*)&sh[slot][d];
+        return;
+    }
+    // piece t: positions 4 q .. 4 q + 3 (q = t % 64 / 16) of dims d and d + 16, d = 32 (t / 64) + t % 16
+    const int q4 = ((t >> 4) & 3) * 4, d = (t >> 6) * 32 + (t & 15), row = pb * 16 + q4 - p.base;
+    _Float16* o = (_Float16*)p.vc + blk + t * 8;
+    half8 v;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        v[e] = sh[q4 + e][d];
+        v[4 + e] = sh[q4 + e][d + 16];
+    }
+    if (row >= 0 && row + 3 < p.n) {
+        *(half8*)o = v;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (row + e >= 0 && row + e < p.n) {
+                o[e] = v[e];
+                o[4 + e] = v[4 + e];
+            }
+    }
+}
+
+// ---- attention ------------------------------------------------------------------------------------------------------------------
+// A wave holds 32 (row, q head of the group) pairs as the columns of v_mfma_f32_32x32x16_f16 and walks the cache 32 positions at
+// a time: S^T = K Q^T, weights, O^T += V^T P^T.  A lane's sixteen scores are of ONE pair, so the softmax crosses lanes once
+// (lane ^ 32), and they come out as the B operand of the second product in an order of positions that V is simply read in; K and
+// V are operands as the cache keeps them.  The four waves of a workgroup (128 pairs) walk the same blocks, so the L1 serves all
+// but the first.  2048 rows of the 8B shape: 101 us a layer (rotation and cache stores 16 us), where the verify passes' kernels,
+// 64 rows at a time, took 32 x (9.7 + 4.8 merge) us (and 32 x 4.8).  Rows see [0, position] (window: the last `window` positions); only blocks that straddle an edge look.
+__device__ __forceinline__ float other_half_max(float v) {
+    float w = v;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_max_f32 %0, %0, %1" : "+v"(v), "+v"(w));
+    return v;
+}
+constexpr float LOG2E = 1.44269504088896340736f, REF_SLACK = 8.0f;
+
+template <int HD, bool PART>
+__global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
+    constexpr int KS = HD / 16, VT = HD / 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int G = p.nq / p.nkv, cols = p.n * G, kvh = blockIdx.y;
+    // the longest rows first
+    const int wg = gridDim.x - 1 - blockIdx.x, c_first = (wg * 4 + wave) * 32;
+    if (c_first >= cols) return;
+    const int hl = lane >> 5, c = min(c_first + (lane & 31), cols - 1), row = c / G, hq = kvh * G + (c - row * G);
+    const int row_lo = c_first / G, row_hi = min(c_first + 31, cols - 1) / G;
+    const int pos = p.base + row;
+    int b0 = p.window > 0 ? max(p.base + row_lo + 1 - p.window, 0) >> 5 : 0, b1 = (p.base + row_hi) / 32 + 1;
+    if (PART) {
+        const int per = (b1 - b0 + p.nch - 1) / p.nch;
+        b0 += blockIdx.z * per;
+        b1 = min(b1, b0 + per);
+    }
+    const _Float16* qp = (const _Float16*)p.q16 + ((size_t)row * p.nq + hq) * HD + 8 * hl;
+    u32x4 q[KS];
+#pragma unroll
+    for (int t = 0; t < KS; t++) q[t] = *(const u32x4*)(qp + 16 * t);
+    const uint32_t head_bytes = (uint32_t)p.cap * HD * 2;  // (bounds the reads: blocks past the cache come back as zeros)
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)p.kc + (size_t)kvh * head_bytes), 0, head_bytes, 0x00027000);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)p.vc + (size_t)kvh * head_bytes), 0, head_bytes, 0x00027000);
+    const uint32_t koff = ((lane >> 4) & 1) * (HD * 32) + hl * 256 + (lane & 15) * 16;
+    const uint32_t voff = hl * 256 + (lane & 15) * 16 + ((lane >> 4) & 1) * 8;
+    float16v O[VT];
+#pragma unroll
+    for (int u = 0; u < VT; u++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) O[u][i] = 0.f;
+    float mrun = -INFINITY, lrun = 0.f;
+    const float c2 = p.scale * LOG2E;
+    u32x4 kf[KS];
+    auto load_k = [&](int b) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < KS; t++)
+            kf[t] = __builtin_amdgcn_raw_buffer_load_b128(krs, koff + (uint32_t)b * (HD * 64) + (t >> 1) * 1024 + (t & 1) * 512, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // (a block's V is asked for before its scores are made, the next block's K right after: both have the softmax and a product
+    // to arrive in, and one set of registers each)
+    auto step = [&](int b) {
+        u32x2 vf[2][VT][2];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int u = 0; u < VT; u++)
+#pragma unroll
+                for (int x = 0; x < 2; x++)
+                    vf[t][u][x] = __builtin_amdgcn_raw_buffer_load_b64(vrs, voff + (uint32_t)(2 * b + t) * (HD * 32) + u * 1024 + x * 512, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        float16v S;
+#pragma unroll
+        for (int i = 0; i < 16; i++) S[i] = 0.f;
+#pragma unroll
+        for (int t = 0; t < KS; t++)
+            S = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, kf[t]), __builtin_bit_cast(half8, q[t]), S, 0, 0, 0);
+        load_k(min(b + 1, b1 - 1));
+        // register i: position 32 b + 8 (i / 4) + 4 hl + i % 4
+        const int p0 = 32 * b;
+        if (p0 + 31 > p.base + row_lo || (p.window > 0 && p0 <= p.base + row_hi - p.window)) {  // (wave-uniform)
+            const int lo = p.window > 0 ? pos - p.window : -1;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int at = p0 + 8 * (i >> 2) + 4 * hl + (i & 3);
+                S[i] = at <= pos && at > lo ? S[i] : -INFINITY;
+            }
+        }
+        float mb = S[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) mb = fmaxf(mb, S[i]);
+        mb = other_half_max(mb) * c2;
+        // the reference follows the maximum lazily (attn_core.h): a weight never exceeds 2^REF_SLACK
+        const bool grow = mb > mrun + REF_SLACK;
+        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+            const float mnew = grow ? mb : mrun;
+            const float alpha = __builtin_amdgcn_exp2f(mrun - fmaxf(mnew, -3.0e38f));
+            lrun *= alpha;
+#pragma unroll
+            for (int u = 0; u < VT; u++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) O[u][i] *= alpha;
+            mrun = mnew;
+        }
+        const float nref = -fmaxf(mrun, -3.0e38f);
+        half8 P[2];
+        float ps = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(S[i], c2, nref));
+            ps += w;
+            P[i >> 3][i & 7] = (_Float16)w;
+        }
+        lrun += ps;
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int u = 0; u < VT; u++) {
+                const u32x4 va = {vf[t][u][0].x, vf[t][u][0].y, vf[t][u][1].x, vf[t][u][1].y};
+                O[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, va), P[t], O[u], 0, 0, 0);
+            }
+    };
+    if (b0 < b1) {
+        load_k(b0);
+        for (int b = b0; b < b1; b++) step(b);
+    }
+    float l = lrun + __shfl_xor(lrun, 32);
+    const bool live = c_first + (lane & 31) < cols;
+    if (PART) {
+        const size_t at = ((size_t)blockIdx.z * p.nkv + kvh) * cols + c;
+        if (!live) return;
+        if (hl == 0) {
+            p.part_ml[at * 2] = mrun;
+            p.part_ml[at * 2 + 1] = l;
+        }
+#pragma unroll
+        for (int u = 0; u < VT; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                *(float4*)(p.part_o + at * HD + 32 * u + 8 * i + 4 * hl) = float4{O[u][4 * i], O[u][4 * i + 1], O[u][4 * i + 2], O[u][4 * i + 3]};
+        return;
+    }
+    float scale = 1.0f;
+    if (p.sinks) {  // joins maximum and denominator only (crates/compute/src/attention.rs:94-105)
+        const float sink = p.sinks[hq] * LOG2E, m = fmaxf(mrun, sink);
+        scale = __builtin_amdgcn_exp2f(mrun - m);
+        l = l * scale + __builtin_amdgcn_exp2f(sink - m);
+    }
+    scale /= l;
+    const int k16 = prompt_k16(p.nq * HD);
+#pragma unroll
+    for (int u = 0; u < VT; u++) {
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int k = hq * HD + 32 * u + 8 * i + 4 * hl;
+            half4 o = {(_Float16)(O[u][4 * i] * scale), (_Float16)(O[u][4 * i + 2] * scale), (_Float16)(O[u][4 * i + 1] * scale),
+                       (_Float16)(O[u][4 * i + 3] * scale)};
+            u32x2 bits = __builtin_bit_cast(u32x2, o);
+            asm volatile("" : "+v"(bits.x), "+v"(bits.y));
+            o = __builtin_bit_cast(half4, bits);
+            sum += ((float)o[0] + (float)o[1]) + ((float)o[2] + (float)o[3]);
+            if (live) *(u32x2*)((_Float16*)p.a + prompt_a_index(row, k, k16)) = bits;
+        }
+        if (p.asum) {
+            sum += __shfl_xor(sum, 32);
+            if (live && hl == 0) {
+                sum *= PROMPT_SUM_SCALE;
+                const int k = hq * HD + 32 * u;
+                const _Float16 hi = (_Float16)sum, lo = (_Float16)((sum - (float)hi) * PROMPT_SUM_LEFT);
+                _Float16* o = (_Float16*)(p.asum + ((size_t)(row >> 5) * (k16 >> 4) + (k >> 8)) * 1024) + (row & 31) * 8 + ((k >> 5) & 7);
+                o[0] = hi;
+                o[256] = lo;
+            }
+        }
+    }
+}
+
+// The chunks' partial results of one (row, q head) merged, one thread per eight dims; HD / 8 threads to a pair
+template <int HD>
+__global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
+    constexpr int TPP = HD / 8;
+    const int G = p.nq / p.nkv, cols = p.n * G;
+    const int id = blockIdx.x * 256 + threadIdx.x, pair = id / TPP, d = id % TPP * 8;
+    // consecutive threads: dims, then rows of one head, so that the pieces written side by side are neighbours
+    const int row = pair % p.n, hq = min(pair / p.n, p.nq - 1), kvh = hq / G;
+    const bool live = pair < p.n * p.nq;
+    const size_t c = (size_t)row * G + (hq - kvh * G);
+    const float sink = p.sinks ? p.sinks[hq] * LOG2E : -INFINITY;
+    float m = sink;
+    for (int ch = 0; ch < p.nch; ch++) m = fmaxf(m, p.part_ml[(((size_t)ch * p.nkv + kvh) * cols + c) * 2]);
+    float l = p.sinks ? __builtin_amdgcn_exp2f(sink - m) : 0.f, o[8] = {};
+    for (int ch = 0; ch < p.nch; ch++) {
+        const size_t at = ((size_t)ch * p.nkv + kvh) * cols + c;
+        const float w = __builtin_amdgcn_exp2f(p.part_ml[at * 2] - m);
+        l = __builtin_fmaf(p.part_ml[at * 2 + 1], w, l);
+        const float4 a = *(const float4*)(p.part_o + at * HD + d), b = *(const float4*)(p.part_o + at * HD + d + 4);
+        const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = __builtin_fmaf(f[e], w, o[e]);
+    }
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[e] *= inv;
+    put_activations(p.a, p.asum, row, hq * HD + d, prompt_k16(p.nq * HD), o, live);
+}
+
+}  // namespace
+
+int launch_prompt_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float* x, const int32_t* ids, int n, int base, const float* freqs,
+                        float mscale, int half, float2* cs) {
+    hipLaunchKernelGGL(k_prompt_embed, dim3(n), dim3(256), 0, s, raw, dtype, hidden, x, ids, base, freqs, mscale, half, cs);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+template <int NV>
+static void launch_norm(hipStream_t s, const PromptNormArgs& a) {
+    const dim3 grid((a.n + 7) / 8), block(512);
+    if (a.weights) hipLaunchKernelGGL((k_prompt_norm<NV, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_prompt_norm<NV, false>), grid, block, 0, s, a);
+}
+
+int launch_prompt_norm(hipStream_t s, const PromptNormArgs& a) {
+    if (a.hidden % 32 || a.splits < 0 || a.splits > 8 || a.n < 1) {
+        set_error("prompt pass: bad norm arguments");
+        return TSV_ERR_UNSUPPORTED;
+    }
+    const int nv = (a.hidden + 511) / 512;
+    if (nv > 8) {
+        const dim3 grid((a.n + 7) / 8), block(512);
+        if (a.weights) hipLaunchKernelGGL(k_prompt_norm_long<true>, grid, block, 0, s, a);
+        else hipLaunchKernelGGL(k_prompt_norm_long<false>, grid, block, 0, s, a);
+    } else {
+        nv <= 2 ? launch_norm<2>(s, a) : nv <= 4 ? launch_norm<4>(s, a) : nv <= 6 ? launch_norm<6>(s, a) : launch_norm<8>(s, a);
+    }
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int launch_prompt_rope(hipStream_t s, const PromptRopeArgs& a) {
+    if (a.splits < 1 || a.splits > 8 || (a.hd != 64 && a.hd != 128) || a.cap % 16 || a.n > a.cap) {
+        set_error("prompt pass: bad rotation arguments");
+        return TSV_ERR_INVALID;
+    }
+    const dim3 grid((a.base + a.n - 1) / 16 - a.base / 16 + 1, a.nq + 2 * a.nkv);
+    if (a.hd == 128) hipLaunchKernelGGL(k_prompt_rope<128>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_prompt_rope<64>, grid, dim3(256), 0, s, a);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+// Chunks of the context per pair: a wave walks its positions alone, so where the pairs do not fill the chip (about two
+// workgroups per compute unit) the context is cut, as long as a chunk keeps sixteen blocks of 32.
+int prompt_attn_chunks(int n, int base, int nq, int nkv, int window) {
+    const int wgs = (n * (nq / nkv) + 127) / 128 * nkv, blocks = (window > 0 ? std::min(base + n, window + n) : base + n) / 32 + 1;
+    return std::max(1, std::min(std::min(512 / std::max(1, wgs), blocks / 16), 16));
+}
+
+template <int HD>
+static int launch_attn(hipStream_t s, const PromptAttnArgs& a) {
+    const int cols = a.n * (a.nq / a.nkv);
+    const dim3 grid((cols + 127) / 128, a.nkv, a.nch);
+    if (a.nch > 1) {
+        hipLaunchKernelGGL((k_prompt_attn<HD, true>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL(k_prompt_attn_merge<HD>, dim3(((size_t)a.n * a.nq * (HD / 8) + 255) / 256), dim3(256), 0, s, a);
+    } else {
+        hipLaunchKernelGGL((k_prompt_attn<HD, false>), grid, dim3(256), 0, s, a);
+    }
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int launch_prompt_attention(hipStream_t s, const PromptAttnArgs& a) {
+    if ((a.hd != 64 && a.hd != 128) || a.nch < 1 || a.cap % 16 || a.base + a.n > a.cap || (int64_t)a.cap * a.hd * 2 > 0x7FFFFFFF) {
+        set_error("prompt pass: bad attention arguments");
+        return TSV_ERR_INVALID;
+    }
+    return a.hd == 128 ? launch_attn<128>(s, a) : launch_attn<64>(s, a);
+}
+
+}  // namespace tsv

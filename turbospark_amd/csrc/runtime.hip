@@ -7,6 +7,7 @@
 // stream and all intermediates are fp32; fp16 appears where the engine's storage dtype is
 // fixed (KV cache, logits) and as the MFMA operand type of the matmuls.
 #include "ctx.h"
+#include "prompt.h"
 
 using namespace tsv;
 
@@ -145,6 +146,9 @@ int make_tiled(tsv_ctx* c, Stager& st, const tsv_tensor* const* parts, int n_par
         if (rc) return rc;
         TSV_HIP(hipStreamSynchronize(c->stream));  // the stager is reused by the next part
         row_off += rows;
+    }
+    if (fmt == FMT_Q80 || fmt == FMT_BF16 || fmt == FMT_MX4) {  // what the prompt matmuls scale the rows by
+        if ((rc = dev_alloc(c, &out->row_scale, (size_t)out->n_tiles * TILE_ROWS * 4)) || (rc = launch_row_scale(c->stream, *out, out->row_scale))) return rc;
     }
     return TSV_OK;
 }
@@ -1371,6 +1375,7 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
     if (const char* e = getenv("TSV_WIDE_PREFILL")) c->wide.ok = c->wide.ok && e[0] != '0';
     if (const char* e = getenv("TSV_WIDE_ROPE_FUSED")) c->wide.keep_epilogue = e[0] == '1';
     if (share) c->wide.ok = false;  // the head's rows come sixteen at a time
+    c->prompt.ok = c->wide.ok && prompt_supported(c);
     *out = c;
     return TSV_OK;
 }
@@ -1381,6 +1386,7 @@ extern "C" void tsv_close(tsv_ctx* c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
+    prompt_free(c);
     if (c->hist_dev) (void)hipFree(c->hist_dev);
     if (c->vp_host) (void)hipHostFree(c->vp_host);
     if (c->ring.host) (void)hipHostFree(c->ring.host);
@@ -1526,7 +1532,33 @@ extern "C" int32_t tsv_produce(tsv_ctx* c, int32_t token, int64_t position, uint
 // (mtp_prime_rows_batched, families/qwen/mtp.rs:146-400); next_token: the token after ids[n - 1], or -1.
 int tsv::prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0, uint16_t* logits, tsv_ctx* head, int32_t next_token) {
     const int wide_rows = 16 * WIDE_B;
+    // A call of fewer than 64 tokens keeps verify-sized passes, whose rows have the bits of one-row passes whatever their
+    // number: what a caller gets by feeding a few tokens one by one and at once is the same.
+    const bool by_prompt_pass = c->prompt.ok && !c->profile && !c->route_forced_set && (n > PROMPT_MIN_ROWS || (n == PROMPT_MIN_ROWS && !logits && !head));
     for (int64_t i = 0; i < n;) {
+        if (by_prompt_pass) {
+            // passes of equal length, a multiple of sixteen but for the last
+            const int64_t left = n - i, passes = (left + PROMPT_ROWS - 1) / PROMPT_ROWS;
+            const int rows = (int)std::min(left, ((left + passes - 1) / passes + 15) / 16 * 16);
+            const bool last = i + rows >= n;
+            if (int rc = enqueue_prompt_pass(c, ids + i, rows, pos0 + i, head != nullptr, last && logits)) return rc;
+            if (last && logits)
+                TSV_HIP(hipMemcpyAsync(logits, c->logits + (size_t)((rows - 1) % 16) * c->vocab, (size_t)c->vocab * 2, hipMemcpyDeviceToHost, c->stream));
+            for (int b = 0; head && b < rows; b += TSV_MAX_ROWS) {
+                int32_t nt[TSV_MAX_ROWS];
+                int m = 0;
+                for (; m < TSV_MAX_ROWS && b + m < rows; m++) {
+                    const int64_t j = i + b + m + 1;
+                    if (j < n) nt[m] = ids[j];
+                    else if (next_token >= 0) nt[m] = next_token;
+                    else break;
+                }
+                if (!m) break;
+                if (int rc = mtp_pass(head, nt, m, pos0 + i + b, c->prompt.x + (size_t)b * c->hidden, false)) return rc;
+            }
+            i += rows;
+            continue;
+        }
         // 64 rows at a time while that many remain and nobody wants their logits
         // (with a drafter head the last pass is a sixteen-row one: the first draft step reads its rows)
         if (c->wide.ok && !c->profile && !c->route_forced_set && n - i >= wide_rows && (i + wide_rows < n || (!logits && !head))) {

@@ -1,6 +1,7 @@
 // Test and measurement hooks of include/tsverify_testing.h: cache and logits I/O, the kernels one at a time, routing
 // read-back and forcing, per-class timing, the timing loops.  Nothing a producer needs.
 #include "ctx.h"
+#include "prompt.h"
 
 using namespace tsv;
 
@@ -212,7 +213,64 @@ extern "C" int32_t tsv_write_kv(tsv_ctx* c, int32_t layer, int64_t pos0, int64_t
     return rc;
 }
 
+// the same product through the prompt passes' kernel
+static int prompt_matmul(const tsv_tensor* w, const float* x, int32_t m, float* y, int32_t splits) {
+    tsv_ctx tmp;
+    tsv_ctx* c = &tmp;
+    TSV_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    Stager st;
+    TiledW tw;
+    const tsv_tensor* parts[1] = {w};
+    const int k = (int)w->cols, n = (int)w->rows, rows = prompt_padded(m), m16 = (m + 15) / 16;
+    float *xd = nullptr, *pd = nullptr;
+    uint8_t *a = nullptr, *asum = nullptr;
+    std::vector<float> part;
+    int sp = 1;
+    int rc = make_tiled(c, st, parts, 1, false, &tw);
+    if (!rc) {
+        sp = splits > 0 ? std::min(splits, tw.kchunks) : prompt_splits(tw, m);
+        const int per = (tw.kchunks + sp - 1) / sp;
+        sp = (tw.kchunks + per - 1) / per;
+    }
+    if (!rc) rc = dev_alloc(c, &xd, (size_t)m * k * 4);
+    if (!rc) rc = dev_alloc(c, &a, prompt_a_bytes(rows, k), true);
+    if (!rc) rc = dev_alloc(c, &asum, prompt_sum_bytes(rows, k), true);
+    if (!rc) rc = dev_alloc(c, &pd, (size_t)m16 * sp * 16 * n * 4, true);
+    if (!rc && hipMemcpyAsync(xd, x, (size_t)m * k * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess) rc = TSV_ERR_DEVICE;
+    PromptNormArgs na{};
+    na.x = xd;
+    na.n = m;
+    na.hidden = k;
+    na.a = a;
+    na.asum = asum;
+    if (!rc) rc = launch_prompt_norm(c->stream, na);
+    if (!rc) rc = launch_prompt_gemm(c->stream, tw, a, asum, pd, nullptr, m, sp, EPI_PARTIAL, n, n);
+    if (!rc) {
+        part.resize((size_t)m16 * sp * 16 * n);
+        if (hipMemcpyAsync(part.data(), pd, part.size() * 4, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+            hipStreamSynchronize(c->stream) != hipSuccess) {
+            set_error("matmul: device execution failed");
+            rc = TSV_ERR_DEVICE;
+        }
+    }
+    for (int b = 0; !rc && b < m; b++)
+        for (int j = 0; j < n; j++) {
+            float acc = 0.f;
+            for (int s = 0; s < sp; s++) acc += part[(((size_t)(b >> 4) * sp + s) * 16 + (b & 15)) * n + j];
+            y[(size_t)b * n + j] = acc;
+        }
+    if (st.dev) (void)hipFree(st.dev);
+    (void)hipStreamSynchronize(c->stream);
+    for (void* p : c->allocs) (void)hipFree(p);
+    (void)hipStreamDestroy(c->stream);
+    return rc;
+}
+
 extern "C" int32_t tsv_matmul(const tsv_tensor* w, const float* x, int32_t m, float* y, int32_t splits) {
+    if (w && x && y && m > TSV_MAX_ROWS && m <= PROMPT_ROWS && splits <= 8) {
+        const int rc = check_matrix(*w, w->rows, w->cols, "matmul weight");
+        return rc ? rc : prompt_matmul(w, x, m, y, splits);
+    }
     if (!w || !x || !y || m < 1 || m > TSV_MAX_ROWS) {
         set_error("matmul: bad argument");
         return TSV_ERR_INVALID;
@@ -273,7 +331,8 @@ extern "C" int32_t tsv_matmul(const tsv_tensor* w, const float* x, int32_t m, fl
 extern "C" int32_t tsv_attention(const uint16_t* q, const uint16_t* k, const uint16_t* v, int32_t m, int32_t nq,
                                  int32_t nkv, int32_t hd, int64_t base, const int32_t* parent, float scale,
                                  int32_t window, const float* sinks, uint16_t* out) {
-    if (!q || !k || !v || !out || m < 1 || m > TSV_MAX_ROWS || nq % nkv || nq / nkv > 8 || base < 0 || window < 0 ||
+    const bool prompt = m > TSV_MAX_ROWS && m <= PROMPT_ROWS && !parent;  // a prompt pass: consecutive positions, any number of rows
+    if (!q || !k || !v || !out || m < 1 || (m > TSV_MAX_ROWS && !prompt) || nq % nkv || nq / nkv > 8 || base < 0 || window < 0 ||
         (window > 0 && window <= TSV_MAX_ROWS)) {
         set_error("attention: bad argument");
         return TSV_ERR_INVALID;
@@ -282,14 +341,15 @@ extern "C" int32_t tsv_attention(const uint16_t* q, const uint16_t* k, const uin
     tsv_ctx* c = &tmp;
     TSV_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     VerifyParams vp;
-    int rc = fill_params(vp, nullptr, parent, m, base, 0);
+    int rc = prompt ? TSV_OK : fill_params(vp, nullptr, parent, m, base, 0);
     const int seq = (int)base + m, ctx = (seq + 15) / 16 * 16, nch = attn_chunks(nkv), G = nq / nkv;
     const size_t kvb = (size_t)nkv * ctx * hd * 2, inb = (size_t)seq * nkv * hd * 2, qb = (size_t)m * nq * hd * 2;
     uint16_t *kc = nullptr, *vc = nullptr, *kin = nullptr, *vin = nullptr, *q16 = nullptr;
     float *po = nullptr, *pml = nullptr, *sinks_dev = nullptr;
     uint4* xf = nullptr;
     VerifyParams* vpd = nullptr;
-    const size_t xfb = xfrag_bytes(nq * hd);
+    const int pch = prompt ? prompt_attn_chunks(m, (int)base, nq, nkv, window) : 0, k16 = prompt_k16(nq * hd);
+    const size_t xfb = prompt ? prompt_a_bytes(m, nq * hd) : xfrag_bytes(nq * hd);
     if (!rc && sinks) {
         rc = dev_alloc(c, &sinks_dev, (size_t)nq * 4);
         if (!rc && hipMemcpyAsync(sinks_dev, sinks, (size_t)nq * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess)
@@ -300,8 +360,8 @@ extern "C" int32_t tsv_attention(const uint16_t* q, const uint16_t* k, const uin
     if (!rc) rc = dev_alloc(c, &kin, inb);
     if (!rc) rc = dev_alloc(c, &vin, inb);
     if (!rc) rc = dev_alloc(c, &q16, qb);
-    if (!rc) rc = dev_alloc(c, &po, (size_t)nkv * nch * m * G * hd * 4, true);
-    if (!rc) rc = dev_alloc(c, &pml, (size_t)nkv * nch * m * G * 2 * 4, true);
+    if (!rc) rc = dev_alloc(c, &po, (size_t)nkv * std::max(nch, pch) * m * G * hd * 4, true);
+    if (!rc) rc = dev_alloc(c, &pml, (size_t)nkv * std::max(nch, pch) * m * G * 2 * 4, true);
     if (!rc) rc = dev_alloc(c, &xf, xfb, true);
     if (!rc) rc = dev_alloc(c, &vpd, sizeof vp);
     if (!rc && (hipMemcpyAsync(kin, k, inb, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
@@ -310,7 +370,26 @@ extern "C" int32_t tsv_attention(const uint16_t* q, const uint16_t* k, const uin
                 hipMemcpyAsync(vpd, &vp, sizeof vp, hipMemcpyHostToDevice, c->stream) != hipSuccess))
         rc = TSV_ERR_DEVICE;
     if (!rc) rc = launch_kv_fill(c->stream, kc, vc, nkv, hd, ctx, 0, seq, kin, vin);
-    if (!rc) {
+    if (!rc && prompt) {
+        PromptAttnArgs pa{};
+        pa.q16 = q16;
+        pa.kc = kc;
+        pa.vc = vc;
+        pa.n = m;
+        pa.base = (int)base;
+        pa.nq = nq;
+        pa.nkv = nkv;
+        pa.hd = hd;
+        pa.cap = ctx;
+        pa.window = window;
+        pa.scale = scale > 0.f ? scale : 1.0f / std::sqrt((float)hd);
+        pa.sinks = sinks_dev;
+        pa.a = (uint8_t*)xf;
+        pa.part_o = po;
+        pa.part_ml = pml;
+        pa.nch = pch;
+        rc = launch_prompt_attention(c->stream, pa);
+    } else if (!rc) {
         AttnArgs aa{};
         aa.q16 = q16;
         aa.kc = kc;
@@ -339,7 +418,8 @@ extern "C" int32_t tsv_attention(const uint16_t* q, const uint16_t* k, const uin
     }
     if (!rc)
         for (int b = 0; b < m; b++)
-            for (int kk = 0; kk < nq * hd; kk++) out[(size_t)b * nq * hd + kk] = frag[(size_t)frag_index(kk, b)];
+            for (int kk = 0; kk < nq * hd; kk++)
+                out[(size_t)b * nq * hd + kk] = frag[prompt ? prompt_a_index(b, kk, k16) : (size_t)frag_index(kk, b)];
     (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
     (void)hipStreamDestroy(c->stream);
