@@ -110,6 +110,14 @@ struct tsv_ctx {
         float2* cs = nullptr;
         int32_t* ids = nullptr;
         float *part_o = nullptr, *part_ml = nullptr;
+        // routed layers: factors and selections of the rows, the sorted pairs and their tiles, the normed rows as plain rows,
+        // the pairs' activations before and after gate / up with their sums, the down outputs by slot
+        float* route_w = nullptr;
+        int32_t *route_sel = nullptr, *pair = nullptr, *n_tiles = nullptr;
+        void* tiles = nullptr;
+        uint16_t* rows16 = nullptr;
+        uint8_t *a_s = nullptr, *a_e = nullptr, *s_e = nullptr, *s_s = nullptr;
+        float* moe_out = nullptr;
         std::vector<void*> allocs;
     } prompt;
     bool route_forced_set = false;  // tsv_force_route holds selections: prompt passes stay at sixteen rows

@@ -336,12 +336,20 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     const int per_split = (g.nt + 7) / 8 * 8 * g.mt, split = blockIdx.x / per_split, id = blockIdx.x - split * per_split;
     const int slot = id >> 3, nb = slot / g.mt * 8 + (id & 7), mb = slot % g.mt;
     if (nb >= g.nt) return;
+    int row0 = mb * BM, rows = g.m - row0, expert = 0;  // the tile's first row and how many of its rows exist
+    if (g.tiles) {
+        if (mb >= *g.tile_count) return;
+        const PromptTile t = g.tiles[mb];
+        row0 = t.first;
+        rows = t.cnt;
+        expert = t.expert;
+    }
     const int c0 = split * g.chunks_per_split, c1 = min(c0 + g.chunks_per_split, g.kchunks);
     const int s0 = c0 * F::SPC, s1 = c1 * F::SPC;
-    const int tile = min(2 * nb + t64, g.n_tiles - 1);  // (an odd count: the last block's second half repeats the last tile)
+    const int tile = expert * g.n_tiles + min(2 * nb + t64, g.n_tiles - 1);  // (an odd count: the last block's second half repeats the last tile)
     const uint8_t* const wt = g.w + (size_t)tile * g.kchunks * F::TILE_BYTES;
     const size_t rbs = (size_t)g.a_k16 * 1024;
-    const int rb0 = mb * (BM / 32) + wm * 2;
+    const int rb0 = (row0 >> 5) + wm * 2;
     const uint8_t* const ap = g.a + (size_t)rb0 * rbs + lane * 16;
     const float rs = F::UNITS ? 1.0f : g.rs[tile * 64 + lane];
     Bits bits{0x64006400u, 0x54005400u};
@@ -454,12 +462,20 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
         for (int j = 0; j < NT; j++) {
             const int col = nb * 128 + (wn * NT + j) * 32 + (lane & 31);
             if (col >= g.n_valid) continue;
+            const float bias = g.bias ? g.bias[(size_t)expert * g.n_valid + col] : 0.f;
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    const int row = (rb0 + t) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-                    if (row < g.m) out[(((size_t)(row >> 4) * g.splits + split) * 16 + (row & 15)) * g.ldo + col] = acc[t][j][i] * un[j];
+                    const int local = (wm * 2 + t) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                    if (local >= rows) continue;
+                    if (g.tiles) {  // into the row's slot
+                        const int pr = g.pair[row0 + local], row = pr >> 3;
+                        out[((size_t)(row >> 4) * 128 + (pr & 7) * 16 + (row & 15)) * g.ldo + col] = acc[t][j][i] * un[j] + bias;
+                    } else {
+                        const int row = row0 + local;
+                        out[(((size_t)(row >> 4) * g.splits + split) * 16 + (row & 15)) * g.ldo + col] = acc[t][j][i] * un[j];
+                    }
                 }
         }
         return;
@@ -467,19 +483,36 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     // silu(gate) * up: column block 2 q of the tile is 32 gate rows, 2 q + 1 the matching up rows.  The products go through LDS
     // into the order of the next matmul's activations
     _Float16* const act = (_Float16*)lds;
-    auto put_act = [&](int q, int t, int i, float gate, float up) {
+    auto put_act = [&](int q, int t, int i, float gate, float up, float bg, float bu) {
         const int c = q * 32 + (lane & 31), row = (wm * 2 + t) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-        act[((((row >> 5) * 4 + (c >> 4)) * 2 + ((c >> 3) & 1)) * 32 + (row & 31)) * 8 + (c & 4) + (((c & 1) << 1) | ((c >> 1) & 1))] =
-            (_Float16)(silu_prompt(gate) * up);
+        float v;
+        if (g.tiles) {  // (biases before the activation, where the clamp reads them too: moe_gguf.metal:585-600)
+            gate += bg;
+            up += bu;
+        }
+        if (g.alpha > 0.0f) {
+            const float x = fminf(gate, g.limit), y = fminf(fmaxf(up, -g.limit), g.limit);
+            v = (x / (1.0f + __expf(-g.alpha * x))) * (y + 1.0f);
+        } else {
+            v = silu_prompt(gate) * up;
+        }
+        act[((((row >> 5) * 4 + (c >> 4)) * 2 + ((c >> 3) & 1)) * 32 + (row & 31)) * 8 + (c & 4) + (((c & 1) << 1) | ((c >> 1) & 1))] = (_Float16)v;
+    };
+    auto bias_of = [&](const float* b, int q) {
+        const int col = nb * 64 + q * 32 + (lane & 31);
+        return b && col < g.n_valid ? b[(size_t)expert * g.n_valid + col] : 0.f;
     };
     if (NT >= 2) {
 #pragma unroll
-        for (int jq = 0; jq < NT / 2; jq++)
+        for (int jq = 0; jq < NT / 2; jq++) {
+            const int q = (wn * NT) / 2 + jq;
+            const float bg = bias_of(g.bias, q), bu = bias_of(g.bias2, q);
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
                 for (int i = 0; i < 16; i++)
-                    put_act((wn * NT) / 2 + jq, t, i, acc[t][2 * jq][i] * un[2 * jq], acc[t][(2 * jq + 1) % NT][i] * un[(2 * jq + 1) % NT]);
+                    put_act(q, t, i, acc[t][2 * jq][i] * un[2 * jq], acc[t][(2 * jq + 1) % NT][i] * un[(2 * jq + 1) % NT], bg, bu);
+        }
     } else {
         // a wave holds one column block: gate and up meet in LDS (behind the activations' area), wave (q, t) finishes row block t
         float* const swap = (float*)(lds + 32768);
@@ -489,20 +522,22 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
             for (int i = 0; i < 16; i++) swap[((wn * 2 + t) * 16 + i) * 64 + lane] = acc[t][0][i] * un[0];
         __syncthreads();
         const int q = wave >> 1, t = wave & 1;
+        const float bg = bias_of(g.bias, q), bu = bias_of(g.bias2, q);
 #pragma unroll
-        for (int i = 0; i < 16; i++) put_act(q, t, i, swap[((2 * q * 2 + t) * 16 + i) * 64 + lane], swap[(((2 * q + 1) * 2 + t) * 16 + i) * 64 + lane]);
+        for (int i = 0; i < 16; i++)
+            put_act(q, t, i, swap[((2 * q * 2 + t) * 16 + i) * 64 + lane], swap[(((2 * q + 1) * 2 + t) * 16 + i) * 64 + lane], bg, bu);
     }
     __syncthreads();
     const int kvalid = g.n_valid;  // K of the next matmul
     for (int p = threadIdx.x; p < BM * 8; p += 256) {
         const int rb = p >> 8, k16 = nb * 4 + ((p >> 6) & 3);
-        if (k16 * 16 < kvalid)
-            *(u32x4*)((uint8_t*)g.out + (((size_t)(mb * (BM / 32) + rb) * g.out_k16 + k16) * 64 + (p & 63)) * 16) = ((const u32x4*)lds)[p];
+        if (k16 * 16 < kvalid && rb * 32 < rows)  // (a 32-row block belongs to one tile)
+            *(u32x4*)((uint8_t*)g.out + (((size_t)((row0 >> 5) + rb) * g.out_k16 + k16) * 64 + (p & 63)) * 16) = ((const u32x4*)lds)[p];
     }
     if (g.out_sum) {
         for (int p = threadIdx.x; p < BM * 2; p += 256) {
             const int row = p >> 1, sub = p & 1, gs = nb * 2 + sub;
-            if (gs * 32 >= kvalid) continue;
+            if (gs * 32 >= kvalid || (row & ~31) >= rows) continue;
             float sum = 0.f;
 #pragma unroll
             for (int x = 0; x < 4; x++) {
@@ -512,7 +547,7 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
             }
             sum *= PROMPT_SUM_SCALE;
             const _Float16 hi = (_Float16)sum, lo = (_Float16)((sum - (float)hi) * PROMPT_SUM_LEFT);
-            _Float16* o = (_Float16*)(g.out_sum + ((size_t)(mb * (BM / 32) + (row >> 5)) * (g.out_k16 >> 4) + (gs >> 3)) * 1024) + (row & 31) * 8 + (gs & 7);
+            _Float16* o = (_Float16*)(g.out_sum + ((size_t)((row0 >> 5) + (row >> 5)) * (g.out_k16 >> 4) + (gs >> 3)) * 1024) + (row & 31) * 8 + (gs & 7);
             o[0] = hi;
             o[256] = lo;
         }
@@ -568,7 +603,7 @@ int launch_p(hipStream_t s, const PromptGemmArgs& g) {
 }
 template <class F>
 int launch_f(hipStream_t s, PromptGemmArgs& g, int epi, int bm) {
-    g.mt = (g.m + bm - 1) / bm;
+    if (!g.tiles) g.mt = (g.m + bm - 1) / bm;
     if (epi == EPI_SILU) return bm == 256 ? launch_p<F, 1, EPI_SILU>(s, g) : bm == 128 ? launch_p<F, 2, EPI_SILU>(s, g) : launch_p<F, 4, EPI_SILU>(s, g);
     return bm == 256 ? launch_p<F, 1, EPI_PARTIAL>(s, g) : bm == 128 ? launch_p<F, 2, EPI_PARTIAL>(s, g) : launch_p<F, 4, EPI_PARTIAL>(s, g);
 }
@@ -596,6 +631,15 @@ int prompt_splits(const TiledW& w, int m) {
     int sp = std::min(std::min(8, w.kchunks), std::max(1, 512 / std::max(1, tiles)));
     const int per = (w.kchunks + sp - 1) / sp;
     return (w.kchunks + per - 1) / per;
+}
+
+static int launch_any(hipStream_t s, int fmt, PromptGemmArgs& g, int epi, int bm) {
+    return fmt == FMT_Q4K    ? launch_f<PromptQ45<false>>(s, g, epi, bm)
+           : fmt == FMT_Q5K  ? launch_f<PromptQ45<true>>(s, g, epi, bm)
+           : fmt == FMT_Q6K  ? launch_f<PromptQ6>(s, g, epi, bm)
+           : fmt == FMT_Q80  ? launch_f<PromptQ8>(s, g, epi, bm)
+           : fmt == FMT_BF16 ? launch_f<PromptBf>(s, g, epi, bm)
+                             : launch_f<PromptMx>(s, g, epi, bm);
 }
 
 int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int m, int splits, int epi,
@@ -627,13 +671,41 @@ int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void
     g.nt = (w.n_tiles + 1) / 2;
     g.n_valid = epi == EPI_SILU ? w.n_rows / 2 : n_valid;
     g.out_k16 = prompt_k16(w.n_rows / 2);
-    const int bm = row_block(m);
-    return w.fmt == FMT_Q4K    ? launch_f<PromptQ45<false>>(s, g, epi, bm)
-           : w.fmt == FMT_Q5K  ? launch_f<PromptQ45<true>>(s, g, epi, bm)
-           : w.fmt == FMT_Q6K  ? launch_f<PromptQ6>(s, g, epi, bm)
-           : w.fmt == FMT_Q80  ? launch_f<PromptQ8>(s, g, epi, bm)
-           : w.fmt == FMT_BF16 ? launch_f<PromptBf>(s, g, epi, bm)
-                               : launch_f<PromptMx>(s, g, epi, bm);
+    return launch_any(s, w.fmt, g, epi, row_block(m));
+}
+
+int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int epi, int ldo,
+                          const PromptExperts& x) {
+    if ((epi != EPI_PARTIAL && epi != EPI_SILU) || x.n_experts < 1 || w.n_tiles % x.n_experts || (prompt_fmt_has_sums(w.fmt) && !asum) ||
+        (!w.row_scale && (w.fmt == FMT_Q80 || w.fmt == FMT_BF16 || w.fmt == FMT_MX4)) || (x.bm != 64 && x.bm != 128 && x.bm != 256)) {
+        set_error("prompt experts: bad argument");
+        return TSV_ERR_INVALID;
+    }
+    PromptGemmArgs g{};
+    g.w = w.tiles;
+    g.a = (const uint8_t*)a;
+    g.asum = (const uint8_t*)asum;
+    g.rs = w.row_scale;
+    g.out = out;
+    g.out_sum = (uint8_t*)out_sum;
+    g.n_tiles = w.n_tiles / x.n_experts;
+    g.kchunks = g.chunks_per_split = w.kchunks;
+    g.splits = 1;
+    g.ldo = ldo;
+    g.a_k16 = prompt_k16(w.k);
+    g.nt = (g.n_tiles + 1) / 2;
+    const int cols = w.n_rows / x.n_experts;
+    g.n_valid = epi == EPI_SILU ? cols / 2 : cols;
+    g.out_k16 = prompt_k16(cols / 2);
+    g.mt = x.max_tiles;
+    g.tiles = x.routes.tiles;
+    g.tile_count = x.routes.n_tiles;
+    g.pair = x.routes.pair;
+    g.bias = x.bias;
+    g.bias2 = x.bias2;
+    g.alpha = epi == EPI_SILU ? x.alpha : 0.f;
+    g.limit = x.limit;
+    return launch_any(s, w.fmt, g, epi, x.bm);
 }
 
 }  // namespace tsv

@@ -10,7 +10,7 @@ namespace tsv {
 bool prompt_supported(const tsv_ctx* c) {
     if (c->mtp.on) return false;
     for (const LayerW& L : c->layers)
-        if (L.n_experts || L.cap < c->ctx_alloc || L.tq.k_bits) return false;
+        if (L.cap < c->ctx_alloc || L.tq.k_bits || (L.n_experts && c->moe_fp4_terms)) return false;
     return true;
 }
 
@@ -45,7 +45,7 @@ int prompt_reserve(tsv_ctx* c, int n) {
     const int qd = c->nq * c->hd;
     size_t width = (size_t)qd + 2 * c->nkv * c->hd;
     for (const LayerW& L : c->layers)
-        for (const TiledW* t : {&L.wo, &L.down}) width = std::max(width, (size_t)t->n_rows);
+        width = std::max(width, (size_t)(L.n_experts ? std::max(c->hidden, L.n_experts) : c->hidden));
     // one partial sum per row and column, or as many as fill the chip: at most 512 tiles of 256 x 128 (prompt_splits), by half more
     // where q and k are split by themselves and the value columns come on top
     w.partial_floats = std::max((size_t)rows * width, std::min((size_t)8 * rows * width, (size_t)512 * 256 * 128 * 3 / 2));
@@ -57,6 +57,22 @@ int prompt_reserve(tsv_ctx* c, int n) {
         (rc = prompt_alloc(c, &w.q16, (size_t)rows * qd * 2, false)) || (rc = prompt_alloc(c, &w.cs, (size_t)rows * (c->hd / 2) * sizeof(float2), false)) ||
         (rc = prompt_alloc(c, &w.ids, (size_t)rows * 4, false)) || (rc = prompt_alloc(c, &w.part_o, (size_t)512 * 128 * c->hd * 4, false)) ||
         (rc = prompt_alloc(c, &w.part_ml, (size_t)512 * 128 * 2 * 4, false)))
+        return rc;
+    int sorted = 0, tiles = 0;
+    for (const LayerW& L : c->layers)
+        if (L.n_experts) {
+            sorted = std::max(sorted, prompt_padded(prompt_sorted_rows(rows, L.top_k, L.n_experts)) + 256);  // (a tile may reach past its run)
+            tiles = std::max(tiles, prompt_max_tiles(rows, L.top_k, L.n_experts, 64));
+        }
+    if (sorted &&
+        ((rc = prompt_alloc(c, &w.route_w, (size_t)rows * 8 * 4, true)) || (rc = prompt_alloc(c, &w.route_sel, (size_t)rows * 8 * 4, true)) ||
+         (rc = prompt_alloc(c, &w.pair, (size_t)sorted * 4, false)) || (rc = prompt_alloc(c, &w.n_tiles, 4, false)) ||
+         (rc = prompt_alloc(c, &w.tiles, (size_t)tiles * sizeof(PromptTile), false)) ||
+         (rc = prompt_alloc(c, &w.rows16, (size_t)rows * prompt_k16(c->hidden) * 32, true)) ||
+         (rc = prompt_alloc(c, &w.a_s, prompt_a_bytes(sorted, c->hidden), true)) ||
+         (rc = prompt_alloc(c, &w.s_s, prompt_sum_bytes(sorted, c->hidden), true)) || (rc = prompt_alloc(c, &w.a_e, prompt_a_bytes(sorted, c->ffn), true)) ||
+         (rc = prompt_alloc(c, &w.s_e, prompt_sum_bytes(sorted, c->ffn), true)) ||
+         (rc = prompt_alloc(c, &w.moe_out, (size_t)rows * 8 * c->hidden * 4, false))))
         return rc;
     w.rows = rows;
     return TSV_OK;
@@ -76,7 +92,7 @@ int common_splits(const TiledW& a, const TiledW& b, int n) {
 int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits) {
     hipStream_t s = c->stream;
     tsv_ctx::Prompt& w = c->prompt;
-    const int H = c->hidden, qd = c->nq * c->hd, qkv_n = (c->nq + 2 * c->nkv) * c->hd;
+    const int H = c->hidden, qkv_n = (c->nq + 2 * c->nkv) * c->hd;
     int rc = launch_prompt_embed(s, c->embed_raw, c->embed_dtype, H, w.x, w.ids, n, (int)base, c->freqs, c->rope_mscale, c->hd / 2, w.cs);
     if (rc) return rc;
     PromptNormArgs na{};
@@ -88,15 +104,54 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
     na.a = w.a_h;
     auto norm = [&](const float* weight, int splits, const float* bias, const TiledW& next) {
         na.w = weight;
-        na.splits = na.slots = splits;
+        na.splits = splits;
+        na.slots = na.weights ? 8 : splits;
         na.bias = bias;
         na.asum = prompt_fmt_has_sums(next.fmt) ? w.s_h : nullptr;
         return launch_prompt_norm(s, na);
     };
+    // router, ranking, the pairs sorted by expert, then every expert's matrices against the rows that chose it
+    auto routed_ffn = [&](const LayerW& L) {
+        const int rsp = prompt_splits(L.router, n);
+        int rc = launch_prompt_gemm(s, L.router, w.a_h, w.s_h, w.partial, nullptr, n, rsp, EPI_PARTIAL, L.n_experts, L.n_experts);
+        if (rc) return rc;
+        MoeRouteArgs ra{};
+        ra.logits = w.partial;
+        ra.splits = rsp;
+        ra.ld = L.n_experts;
+        ra.n_experts = L.n_experts;
+        ra.top_k = L.top_k;
+        ra.m = 16;
+        ra.weights = w.route_w;
+        ra.selected = w.route_sel;
+        ra.bias = L.router_bias;
+        ra.blocks = (n + 15) / 16;
+        ra.logits_block_stride = (long)rsp * 16 * L.n_experts;
+        PromptExperts x{};
+        x.routes = PromptRoutes{w.pair, (PromptTile*)w.tiles, w.n_tiles};
+        x.n_experts = L.n_experts;
+        x.bm = prompt_expert_rows(n, L.top_k, L.n_experts);
+        x.max_tiles = prompt_max_tiles(n, L.top_k, L.n_experts, x.bm);
+        x.bias = L.be_gate;
+        x.bias2 = L.be_up;
+        x.alpha = c->act_alpha;
+        x.limit = c->act_limit;
+        if ((rc = launch_route(s, ra)) || (rc = launch_prompt_groups(s, w.route_sel, n, L.top_k, L.n_experts, x.bm, x.routes)) ||
+            (rc = launch_prompt_gather(s, w.rows16, w.s_h, H, x.routes, n, L.top_k, L.n_experts, w.a_s,
+                                       prompt_fmt_has_sums(L.gate_up.fmt) ? w.s_s : nullptr)) ||
+            (rc = launch_prompt_experts(s, L.gate_up, w.a_s, w.s_s, w.a_e, prompt_fmt_has_sums(L.down.fmt) ? w.s_e : nullptr, EPI_SILU, 0, x)))
+            return rc;
+        x.bias = L.be_down;
+        x.bias2 = nullptr;
+        return launch_prompt_experts(s, L.down, w.a_e, w.s_e, w.moe_out, nullptr, EPI_PARTIAL, H, x);
+    };
     int sp = 0;
     for (int l = 0; l < c->n_layers; l++) {
         LayerW& L = c->layers[l];
+        na.rows16 = nullptr;
         if ((rc = norm(L.attn_norm, sp, nullptr, prompt_fmt_has_sums(L.qkv.fmt) || !L.v_only.tiles ? L.qkv : L.v_only))) return rc;
+        na.partial = w.partial;
+        na.weights = nullptr;
         sp = L.v_only.tiles ? common_splits(L.qkv, L.v_only, n) : prompt_splits(L.qkv, n);
         if ((rc = launch_prompt_gemm(s, L.qkv, w.a_h, w.s_h, w.partial, nullptr, n, sp, EPI_PARTIAL, qkv_n, L.qkv.n_rows))) return rc;
         if (L.v_only.tiles &&
@@ -142,26 +197,36 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
         aa.nch = prompt_attn_chunks(n, (int)base, c->nq, c->nkv, L.window);
         if ((rc = launch_prompt_attention(s, aa))) return rc;
         sp = prompt_splits(L.wo, n);
-        if ((rc = launch_prompt_gemm(s, L.wo, w.a_q, w.s_q, w.partial, nullptr, n, sp, EPI_PARTIAL, H, H)) ||
-            (rc = norm(L.ffn_norm, sp, L.bo, L.gate_up)) ||
+        if ((rc = launch_prompt_gemm(s, L.wo, w.a_q, w.s_q, w.partial, nullptr, n, sp, EPI_PARTIAL, H, H))) return rc;
+        if (L.n_experts) {
+            na.rows16 = w.rows16;
+            if ((rc = norm(L.ffn_norm, sp, L.bo, prompt_fmt_has_sums(L.gate_up.fmt) ? L.gate_up : L.router)) || (rc = routed_ffn(L))) return rc;
+            na.partial = w.moe_out;
+            na.weights = w.route_w;
+            sp = L.top_k;
+            continue;
+        }
+        if ((rc = norm(L.ffn_norm, sp, L.bo, L.gate_up)) ||
             (rc = launch_prompt_gemm(s, L.gate_up, w.a_h, w.s_h, w.a_f, prompt_fmt_has_sums(L.down.fmt) ? w.s_f : nullptr, n, 1, EPI_SILU, 0, 0)))
             return rc;
         sp = prompt_splits(L.down, n);
         if ((rc = launch_prompt_gemm(s, L.down, w.a_f, w.s_f, w.partial, nullptr, n, sp, EPI_PARTIAL, H, H))) return rc;
     }
-    (void)qd;
     if (!finish && !logits) return TSV_OK;
     const int m = (n - 1) % 16 + 1, t0 = n - m;
     int tail_splits = sp;
     if (finish) {  // the rows as a drafter head reads them
         na.a = nullptr;
         na.w = na.bias = nullptr;
-        na.splits = na.slots = sp;
+        na.splits = sp;
+        na.slots = na.weights ? 8 : sp;
         if ((rc = launch_prompt_norm(s, na))) return rc;
         tail_splits = 0;
     }
     TSV_HIP(hipMemcpyAsync(c->x, w.x + (size_t)t0 * H, (size_t)m * H * 4, hipMemcpyDeviceToDevice, s));
-    if ((rc = launch_addnorm(s, c->x, w.partial + (size_t)(t0 / 16) * sp * 16 * H, tail_splits, H, c->final_norm, c->eps, H, c->xf_a, m))) return rc;
+    const float* tail = na.weights ? w.moe_out + (size_t)t0 * 8 * H : w.partial + (size_t)(t0 / 16) * sp * 16 * H;
+    if ((rc = launch_addnorm(s, c->x, tail, tail_splits, H, c->final_norm, c->eps, H, c->xf_a, m, na.weights && tail_splits ? na.weights + (size_t)t0 * 8 : nullptr)))
+        return rc;
     if (!logits) return TSV_OK;
     return launch_gemm(s, c->head, c->xf_a, c->logits, c->vp_dev, m, 1, EPI_LOGITS, c->vocab, c->vocab);
 }

@@ -29,6 +29,30 @@ __host__ __device__ inline size_t prompt_sum_bytes(int rows, int k) { return (si
 // Rows are padded to whole 256-row tiles in every activation buffer: the padding is read (its products are never stored)
 inline int prompt_padded(int rows) { return (rows + 255) / 256 * 256; }
 
+// Routed experts: the (row, slot) pairs of a pass sorted by expert, every expert's run padded to whole 32-row blocks, and the
+// row tiles the expert matmuls work on, all of one expert side by side.
+struct PromptTile {
+    int32_t expert, first, cnt, pad;  // pairs [first, first + cnt) in sorted order
+};
+struct PromptRoutes {
+    int32_t* pair;       // sorted position -> row * 8 + slot
+    PromptTile* tiles;
+    int32_t* n_tiles;    // device count
+};
+__host__ __device__ inline int prompt_sorted_rows(int n, int top_k, int n_experts) { return n * top_k + 31 * n_experts; }
+// rows of an expert tile: the average expert fills one, or half of one
+inline int prompt_expert_rows(int n, int top_k, int n_experts) {
+    const int avg = n * top_k / n_experts;
+    return avg <= 96 ? 64 : avg <= 192 ? 128 : 256;
+}
+inline int prompt_max_tiles(int n, int top_k, int n_experts, int bm) { return n * top_k / bm + n_experts; }
+// selected: [n][8], rank order
+int launch_prompt_groups(hipStream_t s, const int32_t* selected, int n, int top_k, int n_experts, int bm, const PromptRoutes& r);
+// rows [n][k_pad] (fp16, four in the order 0 2 1 3) -> activations of the sorted pairs; asum (nullable): their sums too, out of
+// the rows' own
+int launch_prompt_gather(hipStream_t s, const uint16_t* rows, const uint8_t* row_sums, int k, const PromptRoutes& r, int n, int top_k, int n_experts,
+                         uint8_t* a, uint8_t* asum);
+
 struct PromptGemmArgs {
     const uint8_t* w;     // row tiles (TiledW)
     const uint8_t* a;     // activations
@@ -40,10 +64,26 @@ struct PromptGemmArgs {
     int a_k16;            // 16-K steps per row of the activations
     int out_k16;
     int mt, nt;           // tiles of the grid: rows, 128 columns
+    // routed experts: the row tiles, expert e owning n_tiles row tiles of w from e * n_tiles on; biases [expert][columns];
+    // alpha > 0: the clamped SwiGLU (moe_gguf.metal:528-556).  EPI_PARTIAL then writes float [row / 16][8 slots][16][ldo]
+    const PromptTile* tiles;
+    const int32_t* tile_count;
+    const int32_t* pair;
+    const float *bias, *bias2;
+    float alpha, limit;
+};
+struct PromptExperts {
+    PromptRoutes routes;
+    int n_experts, max_tiles, bm;
+    const float *bias, *bias2;
+    float alpha, limit;
 };
 
 int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int m, int splits, int epi,
                        int ldo, int n_valid);
+// a: the sorted pairs' activations; EPI_SILU or EPI_PARTIAL; w holds every expert's tiles one after the other
+int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int epi, int ldo,
+                          const PromptExperts& x);
 int prompt_splits(const TiledW& w, int m);
 // the power-of-two factors of a tiled matrix's rows, n_tiles * 64 floats (Q8_0, bf16, MXFP4)
 int launch_row_scale(hipStream_t s, const TiledW& w, float* rs);
@@ -58,6 +98,7 @@ struct PromptNormArgs {
     const float* bias;      // nullable, added after the partial sums
     const float* w;
     uint8_t *a, *asum;      // asum nullable
+    uint16_t* rows16;       // nullable: the same values as plain rows [n][prompt_k16 * 16], for the experts' gather
     int n, hidden, splits, ldp, slots;  // slots: distance of the partials in rows of sixteen (splits, or 8)
     float eps;
 };

@@ -37,11 +37,13 @@ __global__ __launch_bounds__(256) void k_prompt_embed(const uint8_t* __restrict_
 // Eight values (consecutive K) of a row as activations, and the sum of its 32-value sub-block, whose other values sit in the
 // three neighbouring lanes.  The halves are pinned in registers between the store and the sum: the sum has to be that of the
 // stored bits (pinned_half).
-__device__ __forceinline__ void put_activations(uint8_t* a, uint8_t* asum, int row, int k, int k16, const float (&v)[8], bool live) {
+__device__ __forceinline__ void put_activations(uint8_t* a, uint8_t* asum, int row, int k, int k16, const float (&v)[8], bool live,
+                                                uint16_t* rows16 = nullptr) {
     half8 h = {(_Float16)v[0], (_Float16)v[2], (_Float16)v[1], (_Float16)v[3], (_Float16)v[4], (_Float16)v[6], (_Float16)v[5], (_Float16)v[7]};
     u32x4 b = __builtin_bit_cast(u32x4, h);
     asm volatile("" : "+v"(b.x), "+v"(b.y), "+v"(b.z), "+v"(b.w));
     if (live) *(u32x4*)(a + (((size_t)(row >> 5) * k16 + (k >> 4)) * 64 + ((k >> 3) & 1) * 32 + (row & 31)) * 16) = b;
+    if (live && rows16) *(u32x4*)(rows16 + (size_t)row * (k16 * 16) + k) = b;
     if (asum) {
         h = __builtin_bit_cast(half8, b);
         float s = (((float)h[0] + (float)h[1]) + ((float)h[2] + (float)h[3])) + (((float)h[4] + (float)h[5]) + ((float)h[6] + (float)h[7]));
@@ -130,7 +132,7 @@ __global__ __launch_bounds__(512) void k_prompt_norm(PromptNormArgs p) {
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) o[e] = p.w ? v[i][e] * (live ? p.w[k + e] : 0.f) * inv : v[i][e];
-        put_activations(p.a, p.asum, row, k, k16, o, live);
+        put_activations(p.a, p.asum, row, k, k16, o, live, p.rows16);
     }
 }
 
@@ -172,7 +174,7 @@ __global__ __launch_bounds__(512) void k_prompt_norm_long(PromptNormArgs p) {
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) o[e] = live ? (p.w ? xr[k + e] * p.w[k + e] * inv : xr[k + e]) : 0.f;
-        put_activations(p.a, p.asum, row, k, k16, o, live);
+        put_activations(p.a, p.asum, row, k, k16, o, live, p.rows16);
     }
 }
 
@@ -463,6 +465,77 @@ __global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
     put_activations(p.a, p.asum, row, hq * HD + d, prompt_k16(p.nq * HD), o, live);
 }
 
+// ---- routed experts: pairs sorted by expert -------------------------------------------------------------------------------
+// One workgroup: counts, runs and tiles of all experts, then every pair's place.  (Where a pair lands inside its expert's run
+// depends on the order of the atomics; no value does: a row of a product does not see its neighbours.)
+constexpr int MAX_EXPERTS = 256;
+__global__ __launch_bounds__(1024) void k_prompt_groups(const int32_t* __restrict__ selected, int n, int top_k, int ne, int bm, PromptRoutes r) {
+    __shared__ int cnt[MAX_EXPERTS], at[MAX_EXPERTS], scan[2][MAX_EXPERTS];
+    const int tid = threadIdx.x;
+    if (tid < MAX_EXPERTS) cnt[tid] = 0;
+    __syncthreads();
+    const int np = n * top_k;
+    for (int p = tid; p < np; p += 1024) {
+        const int row = p / top_k, e = min(max(selected[row * 8 + p - row * top_k], 0), ne - 1);
+        atomicAdd(&cnt[e], 1);
+    }
+    __syncthreads();
+    // exclusive sums over the experts: rows of the padded runs, then tiles
+    int padded = 0, tiles = 0;
+    if (tid < MAX_EXPERTS) {
+        padded = (cnt[tid] + 31) & ~31;
+        tiles = (cnt[tid] + bm - 1) / bm;
+        scan[0][tid] = padded;
+        scan[1][tid] = tiles;
+    }
+    __syncthreads();
+    for (int o = 1; o < MAX_EXPERTS; o <<= 1) {
+        int a = 0, b = 0;
+        if (tid >= o && tid < MAX_EXPERTS) {
+            a = scan[0][tid - o];
+            b = scan[1][tid - o];
+        }
+        __syncthreads();
+        if (tid < MAX_EXPERTS) {
+            scan[0][tid] += a;
+            scan[1][tid] += b;
+        }
+        __syncthreads();
+    }
+    if (tid < ne) {
+        const int first = scan[0][tid] - padded, t0 = scan[1][tid] - tiles;
+        at[tid] = first;
+        for (int t = 0; t < tiles; t++) r.tiles[t0 + t] = PromptTile{tid, first + t * bm, min(bm, cnt[tid] - t * bm), 0};
+        if (tid == ne - 1) *r.n_tiles = scan[1][tid];
+        for (int q = cnt[tid]; q < padded; q++) r.pair[first + q] = -1;
+    }
+    if (tid == 0)
+        for (int q = scan[0][ne - 1]; q < prompt_sorted_rows(n, top_k, ne); q += 32) r.pair[q] = -2;  // a block past the last run
+    __syncthreads();
+    for (int p = tid; p < np; p += 1024) {
+        const int row = p / top_k, slot = p - row * top_k, e = min(max(selected[row * 8 + slot], 0), ne - 1);
+        r.pair[atomicAdd(&at[e], 1)] = row * 8 + slot;
+    }
+}
+
+// One workgroup per 32 sorted pairs: lane = pair, so the stores are whole lines of the operand layout; the sixteen-byte loads of
+// a row's line come from the eight half waves side by side
+__global__ __launch_bounds__(256) void k_prompt_gather(const uint16_t* __restrict__ rows, const uint8_t* __restrict__ row_sums, int k16,
+                                                       const int32_t* __restrict__ pair, int n_sorted, uint8_t* __restrict__ a, uint8_t* __restrict__ asum) {
+    const int p = blockIdx.x * 32 + (threadIdx.x & 31);
+    if (pair[blockIdx.x * 32] == -2 || p >= n_sorted) return;
+    const int pr = pair[p];
+    if (pr < 0) return;
+    const u32x4* src = (const u32x4*)(rows + (size_t)(pr >> 3) * (k16 * 16));
+    u32x4* dst = (u32x4*)(a + (size_t)blockIdx.x * k16 * 1024) + (threadIdx.x & 31);
+    for (int k8 = threadIdx.x >> 5; k8 < 2 * k16; k8 += 8) dst[k8 * 32] = src[k8];
+    if (!asum) return;
+    const int row = pr >> 3, kc = k16 >> 4;
+    for (int c = threadIdx.x >> 5; c < 2 * kc; c += 8)  // (both halves of the sums of every 256 K)
+        *(u32x4*)(asum + ((size_t)blockIdx.x * 2 * kc + c) * 512 + (threadIdx.x & 31) * 16) =
+            *(const u32x4*)(row_sums + ((size_t)(row >> 5) * 2 * kc + c) * 512 + (row & 31) * 16);
+}
+
 }  // namespace
 
 int launch_prompt_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float* x, const int32_t* ids, int n, int base, const float* freqs,
@@ -492,6 +565,24 @@ int launch_prompt_norm(hipStream_t s, const PromptNormArgs& a) {
     } else {
         nv <= 2 ? launch_norm<2>(s, a) : nv <= 4 ? launch_norm<4>(s, a) : nv <= 6 ? launch_norm<6>(s, a) : launch_norm<8>(s, a);
     }
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int launch_prompt_groups(hipStream_t s, const int32_t* selected, int n, int top_k, int n_experts, int bm, const PromptRoutes& r) {
+    if (n < 1 || n_experts < 1 || n_experts > MAX_EXPERTS || top_k < 1 || top_k > 8) {
+        set_error("moe: at most 256 experts and top-k 8 in a prompt pass");
+        return TSV_ERR_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL(k_prompt_groups, dim3(1), dim3(1024), 0, s, selected, n, top_k, n_experts, bm, r);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int launch_prompt_gather(hipStream_t s, const uint16_t* rows, const uint8_t* row_sums, int k, const PromptRoutes& r, int n, int top_k, int n_experts,
+                         uint8_t* a, uint8_t* asum) {
+    const int sorted = prompt_sorted_rows(n, top_k, n_experts);
+    hipLaunchKernelGGL(k_prompt_gather, dim3((sorted + 31) / 32), dim3(256), 0, s, rows, row_sums, prompt_k16(k), r.pair, sorted, a, asum);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }

@@ -1375,7 +1375,8 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
     if (const char* e = getenv("TSV_WIDE_PREFILL")) c->wide.ok = c->wide.ok && e[0] != '0';
     if (const char* e = getenv("TSV_WIDE_ROPE_FUSED")) c->wide.keep_epilogue = e[0] == '1';
     if (share) c->wide.ok = false;  // the head's rows come sixteen at a time
-    c->prompt.ok = c->wide.ok && prompt_supported(c);
+    const char* wide_env = getenv("TSV_WIDE_PREFILL");
+    c->prompt.ok = !share && !(wide_env && wide_env[0] == '0') && prompt_supported(c);
     *out = c;
     return TSV_OK;
 }
