@@ -59,20 +59,24 @@ __device__ __forceinline__ void put_activations(uint8_t* a, uint8_t* asum, int r
     }
 }
 
-// One wave per row, the row in registers (NV x 512 values); eight rows to a workgroup, so that the sixteen-byte pieces its
-// waves write side by side fill cache lines.  The partial sums are added in order, every split's loads in flight together.
-template <int NV, bool ROUTED>
+// The row in the registers of W waves (NV x 512 values each), 8 / W rows to a workgroup.  Bound by what one compute unit draws
+// from L2 (a row is up to nine of its length: the stream and every split), so a pass has to spread over all of them: W is the
+// smallest that gives every compute unit a workgroup (norm_waves).  Where rows suffice W = 1: the sixteen-byte pieces that eight
+// rows' waves write side by side fill cache lines.  The partial sums are added in order, every split's loads in flight together.
+template <int NV, int W, bool ROUTED>
 __global__ __launch_bounds__(512) void k_prompt_norm(PromptNormArgs p) {
-    const int lane = threadIdx.x & 63, row = blockIdx.x * 8 + (threadIdx.x >> 6);
-    if (row >= p.n) return;
+    __shared__ float sums[8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = blockIdx.x * (8 / W) + wave / W, k0 = wave % W * (NV * 512) + lane * 8;
+    const bool here = row < p.n;
+    if (W == 1 && !here) return;  // (with more waves to a row every wave reaches the barrier)
     float* const xr = p.x + (size_t)row * p.hidden;
     float v[NV][8];
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int k = i * 512 + lane * 8;
+        const int k = k0 + i * 512;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const float4 t = k < p.hidden ? *(const float4*)(xr + k + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
+            const float4 t = here && k < p.hidden ? *(const float4*)(xr + k + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
             v[i][4 * h] = t.x, v[i][4 * h + 1] = t.y, v[i][4 * h + 2] = t.z, v[i][4 * h + 3] = t.w;
         }
     }
@@ -85,13 +89,13 @@ __global__ __launch_bounds__(512) void k_prompt_norm(PromptNormArgs p) {
     }
     for (int s = 0; s < p.splits; s++) {
         const float* pr = p.partial + (((size_t)(row >> 4) * p.slots + s) * 16 + (row & 15)) * p.ldp;
-        const float ws = ROUTED ? p.weights[(size_t)row * 8 + s] : 1.0f;
+        const float ws = ROUTED && here ? p.weights[(size_t)row * 8 + s] : 1.0f;
 #pragma unroll
         for (int i = 0; i < NV; i++) {
-            const int k = i * 512 + lane * 8;
+            const int k = k0 + i * 512;
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const float4 t = k < p.hidden ? *(const float4*)(pr + k + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
+                const float4 t = here && k < p.hidden ? *(const float4*)(pr + k + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
                 const float f[4] = {t.x, t.y, t.z, t.w};
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
@@ -106,14 +110,14 @@ __global__ __launch_bounds__(512) void k_prompt_norm(PromptNormArgs p) {
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int k = i * 512 + lane * 8;
+        const int k = k0 + i * 512;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             if (ROUTED) v[i][e] = __fadd_rn(v[i][e], r[i][e]);
             if (p.bias && k < p.hidden) v[i][e] += p.bias[k + e];
             ss += v[i][e] * v[i][e];
         }
-        if (p.splits && k < p.hidden) {
+        if (p.splits && here && k < p.hidden) {
             *(float4*)(xr + k) = float4{v[i][0], v[i][1], v[i][2], v[i][3]};
             *(float4*)(xr + k + 4) = float4{v[i][4], v[i][5], v[i][6], v[i][7]};
         }
@@ -122,13 +126,20 @@ __global__ __launch_bounds__(512) void k_prompt_norm(PromptNormArgs p) {
     float inv = 1.0f;
     if (p.w) {
         for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        if (W > 1) {
+            if (lane == 0) sums[wave] = ss;
+            __syncthreads();
+            ss = 0.f;
+#pragma unroll
+            for (int u = 0; u < W; u++) ss += sums[wave / W * W + u];
+        }
         inv = 1.0f / sqrtf(ss / (float)p.hidden + p.eps);
     }
     const int k16 = prompt_k16(p.hidden);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int k = i * 512 + lane * 8;
-        const bool live = k < p.hidden;
+        const int k = k0 + i * 512;
+        const bool live = here && k < p.hidden;
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) o[e] = p.w ? v[i][e] * (live ? p.w[k + e] : 0.f) * inv : v[i][e];
@@ -545,11 +556,18 @@ int launch_prompt_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden
     return TSV_OK;
 }
 
-template <int NV>
+template <int NV, int W>
 static void launch_norm(hipStream_t s, const PromptNormArgs& a) {
-    const dim3 grid((a.n + 7) / 8), block(512);
-    if (a.weights) hipLaunchKernelGGL((k_prompt_norm<NV, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_prompt_norm<NV, false>), grid, block, 0, s, a);
+    const dim3 grid((a.n + 8 / W - 1) / (8 / W)), block(512);
+    if (a.weights) hipLaunchKernelGGL((k_prompt_norm<NV, W, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_prompt_norm<NV, W, false>), grid, block, 0, s, a);
+}
+
+// Waves to a row: as many as it takes for a workgroup per compute unit, as long as each keeps 512 values
+static int norm_waves(int n, int nv) {
+    int w = 1;
+    while (w < 8 && w < nv && (n * w + 7) / 8 < 256) w *= 2;
+    return w;
 }
 
 int launch_prompt_norm(hipStream_t s, const PromptNormArgs& a) {
@@ -563,7 +581,11 @@ int launch_prompt_norm(hipStream_t s, const PromptNormArgs& a) {
         if (a.weights) hipLaunchKernelGGL(k_prompt_norm_long<true>, grid, block, 0, s, a);
         else hipLaunchKernelGGL(k_prompt_norm_long<false>, grid, block, 0, s, a);
     } else {
-        nv <= 2 ? launch_norm<2>(s, a) : nv <= 4 ? launch_norm<4>(s, a) : nv <= 6 ? launch_norm<6>(s, a) : launch_norm<8>(s, a);
+        const int w = norm_waves(a.n, nv), per = (nv + w - 1) / w;
+        if (w == 8) launch_norm<1, 8>(s, a);
+        else if (w == 4) per == 1 ? launch_norm<1, 4>(s, a) : launch_norm<2, 4>(s, a);
+        else if (w == 2) per == 1 ? launch_norm<1, 2>(s, a) : per == 2 ? launch_norm<2, 2>(s, a) : per == 3 ? launch_norm<3, 2>(s, a) : launch_norm<4, 2>(s, a);
+        else nv <= 2 ? launch_norm<2, 1>(s, a) : nv <= 4 ? launch_norm<4, 1>(s, a) : nv <= 6 ? launch_norm<6, 1>(s, a) : launch_norm<8, 1>(s, a);
     }
     TSV_HIP(hipGetLastError());
     return TSV_OK;
