@@ -25,6 +25,7 @@
 // Workgroups are numbered so that an XCD works on every eighth block of columns with all row blocks side by side: the
 // weights of a block come into that XCD's L2 once, and the activations are shared by the blocks in flight.
 #include <algorithm>
+#include <atomic>
 
 #include "prompt.h"
 
@@ -313,6 +314,14 @@ struct PromptBf {
 };
 
 __device__ __forceinline__ float silu_prompt(float x) { return x / (1.0f + __expf(-x)); }
+// silu(gate) * up, or with alpha > 0 the clamped form (moe_gguf.metal:528-556)
+__device__ __forceinline__ float gated(float gate, float up, float alpha, float limit) {
+    if (alpha > 0.0f) {
+        const float x = fminf(gate, limit), y = fminf(fmaxf(up, -limit), limit);
+        return (x / (1.0f + __expf(-alpha * x))) * (y + 1.0f);
+    }
+    return silu_prompt(gate) * up;
+}
 
 template <class F>
 constexpr int stage_bytes() {
@@ -485,17 +494,11 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     _Float16* const act = (_Float16*)lds;
     auto put_act = [&](int q, int t, int i, float gate, float up, float bg, float bu) {
         const int c = q * 32 + (lane & 31), row = (wm * 2 + t) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-        float v;
         if (g.tiles) {  // (biases before the activation, where the clamp reads them too: moe_gguf.metal:585-600)
             gate += bg;
             up += bu;
         }
-        if (g.alpha > 0.0f) {
-            const float x = fminf(gate, g.limit), y = fminf(fmaxf(up, -g.limit), g.limit);
-            v = (x / (1.0f + __expf(-g.alpha * x))) * (y + 1.0f);
-        } else {
-            v = silu_prompt(gate) * up;
-        }
+        const float v = gated(gate, up, g.alpha, g.limit);
         act[((((row >> 5) * 4 + (c >> 4)) * 2 + ((c >> 3) & 1)) * 32 + (row & 31)) * 8 + (c & 4) + (((c & 1) << 1) | ((c >> 1) & 1))] = (_Float16)v;
     };
     auto bias_of = [&](const float* b, int q) {
@@ -554,6 +557,163 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     }
 }
 
+// ---- experts with few rows, MXFP4 -----------------------------------------------------------------------------------------
+// The tile of the kernel above at 64 rows is bound by the L1 and the LDS, not by the matrix pipes (each wave draws all 64 rows'
+// activations, and every unpacked weight crosses the LDS for 64 rows only), and a stage ahead is too little in flight for a
+// stream of weights.  Here a workgroup makes the 64 columns of ONE row tile, its waves each a quarter of K: a lane unpacks the
+// weights of its own row and one v_permlane32_swap per register turns two eight-K pieces of 64 rows into the B operands of two
+// 32-column blocks, so nothing goes through LDS before the four partial sums meet there, no barrier stands in the loop, and
+// operands are asked for `RING - 1` units of 32 K ahead (activations and weights alike: loads return in order, the nearer
+// distance is the one that counts).  32-row blocks past the expert's last row are not multiplied.
+// A workgroup's neighbours on its XCD are the other tiles of the same expert: the activations stay in that L2, weights pass once.
+// Taken where the average expert has at most 96 rows (prompt_expert_rows) and the storage type needs no sums.  Measured, gate/up
+// and down of one layer: 1500 rows, 128 experts, top 4, 2880 x 2880: 577 + 339 us in tiles of the kernel above, 454 + 247 here
+// (2.5 TB/s of weights; between 32 and 64 rows the unpack and the products take the same time, below the unpack bounds it);
+// 1000 rows, 128 experts, top 8, 768 x 2048: 144 each, 114 + 93 here.
+constexpr int NARROW_ROWS = 64;
+template <int RB, int RING>
+__device__ __forceinline__ void narrow_products(const uint8_t* w, const uint8_t* a, size_t rbs, int units, int unit0, int shift, int lane,
+                                                float16v (&acc)[2][2]) {
+    struct Piece {
+        u32x4 q, a[2][RB];
+        uint32_t e;
+    } r[RING];
+    const int last = unit0 + units - 1;
+    auto load = [&](Piece& p, int u) {
+        u = min(u, last);
+        const uint8_t* t = w + (size_t)(u >> 3) * PromptMx::TILE_BYTES;
+        const uint8_t* x = a + (size_t)u * 2048;
+        __builtin_amdgcn_sched_barrier(0);
+        p.q = *(const u32x4*)(t + ((u & 7) * 64 + lane) * 16);
+        p.e = t[8192 + lane * 8 + (u & 7)];
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int b = 0; b < RB; b++) p.a[q][b] = *(const u32x4*)(x + b * rbs + q * 1024);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const Piece& p) {
+        const float sc = __uint_as_float((uint32_t)min(max((int)p.e + shift, 1), 254) << 23);
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            u32x4 b[2];
+            const uint32_t lo = p.q[2 * q], hi = p.q[2 * q + 1];
+            auto put = [&](int i, auto l, auto h) {
+                const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, l), __builtin_bit_cast(uint32_t, h), false, false);
+                b[0][i] = t[0];
+                b[1][i] = t[1];
+            };
+            put(0, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 0));
+            put(1, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 1), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 1));
+            put(2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 2), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 2));
+            put(3, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 3), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 3));
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int t = 0; t < RB; t++)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, p.a[q][t]), __builtin_bit_cast(half8, b[j]), acc[t][j], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < RING - 1; i++) load(r[i], unit0 + i);
+    for (int u = unit0; u <= last; u += RING) {
+#pragma unroll
+        for (int i = 0; i < RING; i++) {
+            load(r[(i + RING - 1) % RING], u + i + RING - 1);
+            if (i == 0 || u + i <= last) multiply(r[i]);
+        }
+    }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256, 3) void k_prompt_experts_narrow(PromptGemmArgs g) {
+    __shared__ __attribute__((aligned(16))) float meet[4 * 3 * 16 * 64];  // [reader][the other waves][values][lanes]
+    __shared__ float factor[64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // XCD x takes the row tiles x, x + 8, ..., all columns of one before the next
+    const int slot = blockIdx.x >> 3, mb = slot / g.n_tiles * 8 + (blockIdx.x & 7), nb = slot % g.n_tiles;
+    if (mb >= *g.tile_count) return;
+    const PromptTile t = g.tiles[mb];
+    const int tile = t.expert * g.n_tiles + nb;
+    const float rs = g.rs[tile * 64 + lane];
+    if (wave == 0) factor[lane] = 1.0f / rs;
+    float16v acc[2][2];
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[b][j][i] = 0.f;
+    const uint8_t* const w = g.w + (size_t)tile * g.kchunks * PromptMx::TILE_BYTES;
+    const size_t rbs = (size_t)g.a_k16 * 1024;
+    const uint8_t* const a = g.a + (size_t)(t.first >> 5) * rbs + lane * 16;
+    const int units = 2 * g.kchunks, shift = (int)(__float_as_uint(rs) >> 23) - 127;
+    if (t.cnt > 32) narrow_products<2, 3>(w, a, rbs, units, wave * units, shift, lane, acc);
+    else narrow_products<1, 5>(w, a, rbs, units, wave * units, shift, lane, acc);
+    // wave d ends with registers 4 d .. 4 d + 3 of all four blocks: rows 8 d + 4 (lane / 32) + i of both row blocks, column lane % 32
+    // of both column blocks.  Summed in the order of K.
+    float mine[16];
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        if (wave == d) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) mine[v] = acc[v >> 3][(v >> 2) & 1][4 * d + (v & 3)];
+        } else {
+            float* o = meet + (size_t)(d * 3 + (wave < d ? wave : wave - 1)) * 1024 + lane;
+#pragma unroll
+            for (int v = 0; v < 16; v++) o[v * 64] = acc[v >> 3][(v >> 2) & 1][4 * d + (v & 3)];
+        }
+    }
+    __syncthreads();
+    const float* in = meet + (size_t)wave * 3 * 1024 + lane;
+    const float f0 = factor[lane & 31], f1 = factor[32 + (lane & 31)];
+    float sum[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        float x = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) x += k == wave ? mine[v] : in[((k < wave ? k : k == wave ? 0 : k - 1) * 16 + v) * 64];
+        sum[v] = x * ((v >> 2) & 1 ? f1 : f0);
+    }
+    if (EPI == EPI_PARTIAL) {
+        float* const out = (float*)g.out;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int col = nb * 64 + 32 * j + (lane & 31);
+            if (col >= g.n_valid) continue;
+            const float bias = g.bias ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int local = 32 * b + 8 * wave + 4 * (lane >> 5) + i;
+                    if (local >= t.cnt) continue;
+                    const int pr = g.pair[t.first + local], row = pr >> 3;
+                    out[((size_t)(row >> 4) * 128 + (pr & 7) * 16 + (row & 15)) * g.ldo + col] = sum[b * 8 + j * 4 + i] + bias;
+                }
+        }
+        return;
+    }
+    // 32 gate columns and the matching up columns; the products go through LDS into the order of the next matmul's activations
+    __syncthreads();
+    _Float16* const act = (_Float16*)meet;
+    const int c = lane & 31, col = nb * 32 + c;
+    const float bg = g.bias && col < g.n_valid ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
+    const float bu = g.bias2 && col < g.n_valid ? g.bias2[(size_t)t.expert * g.n_valid + col] : 0.f;
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 8 * wave + 4 * (lane >> 5) + i;
+            act[(((b * 2 + (c >> 4)) * 2 + ((c >> 3) & 1)) * 32 + row) * 8 + (c & 4) + (((c & 1) << 1) | ((c >> 1) & 1))] =
+                (_Float16)gated(sum[b * 8 + i] + bg, sum[b * 8 + 4 + i] + bu, g.alpha, g.limit);
+        }
+    __syncthreads();
+    const int p = threadIdx.x, b = p >> 7, k16 = nb * 2 + ((p >> 6) & 1);
+    if (k16 * 16 < g.n_valid && b * 32 < t.cnt)
+        *(u32x4*)((uint8_t*)g.out + (((size_t)((t.first >> 5) + b) * g.out_k16 + k16) * 64 + (p & 63)) * 16) = ((const u32x4*)meet)[p];
+}
+
 // ---- row factors ----------------------------------------------------------------------------------------------------------
 // The power of two that brings the largest magnitude of a row near the top of fp16's range: 2^7 for a Q8_0 scale (its product
 // with a code stays below 2^15), 2^12 for an MXFP4 block scale (times 6), 2^14 for a bf16 value.  One wave per tile.
@@ -591,10 +751,14 @@ __global__ __launch_bounds__(64) void k_row_scale(const uint8_t* __restrict__ ti
 
 template <class F, int WN, int EPI>
 int launch_p(hipStream_t s, const PromptGemmArgs& g) {
-    static bool raised = false;  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
-    if (!raised) {
+    // more than 64 KiB of dynamic LDS has to be allowed once per kernel and device
+    static std::atomic<uint64_t> allowed{0};
+    int dev = 0;
+    TSV_HIP(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (!(allowed.load(std::memory_order_acquire) & bit)) {
         TSV_HIP(hipFuncSetAttribute((const void*)k_prompt_gemm<F, WN, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<F>()));
-        raised = true;
+        allowed.fetch_or(bit, std::memory_order_release);
     }
     const int blocks = (g.nt + 7) / 8 * 8 * g.mt * g.splits;
     hipLaunchKernelGGL((k_prompt_gemm<F, WN, EPI>), dim3(blocks), dim3(256), lds_bytes<F>(), s, g);
@@ -706,6 +870,13 @@ int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const v
     g.bias2 = x.bias2;
     g.alpha = epi == EPI_SILU ? x.alpha : 0.f;
     g.limit = x.limit;
+    if (w.fmt == FMT_MX4 && x.bm == NARROW_ROWS && !out_sum) {
+        const dim3 grid((x.max_tiles + 7) / 8 * 8 * g.n_tiles);
+        if (epi == EPI_SILU) hipLaunchKernelGGL(k_prompt_experts_narrow<EPI_SILU>, grid, dim3(256), 0, s, g);
+        else hipLaunchKernelGGL(k_prompt_experts_narrow<EPI_PARTIAL>, grid, dim3(256), 0, s, g);
+        TSV_HIP(hipGetLastError());
+        return TSV_OK;
+    }
     return launch_any(s, w.fmt, g, epi, x.bm);
 }
 
