@@ -143,6 +143,16 @@ __device__ __forceinline__ double prob_of(uint16_t bits, int v, const RowStat& s
 // largest fp16 value not above it, so bins stay ordered; inside a bin the candidates with a score
 // above the bin's own value come first (score descending, index ascending: the few "side"
 // candidates), then the candidates exactly on the value in index order.
+__device__ __forceinline__ float penalised(const AcceptParams& ap, float w, bool seen, uint32_t gen) {
+    if (ap.pen_has_rep && seen) {
+        const float a = w > 0.0f ? __fdiv_rn(w, ap.pen_rep) : __fmul_rn(w, ap.pen_rep);
+        w = fminf(fmaxf(a, -3.40282347e+38f), 3.40282347e+38f);
+    }
+    if (ap.pen_has_pf && gen != 0)
+        w = __fsub_rn(w, (float)__dadd_rn(ap.pen_presence, __dmul_rn(ap.pen_frequency, (double)gen)));
+    return w;
+}
+
 template <bool PEN>
 __device__ __forceinline__ float score_of(const AcceptParams& ap, int row, int v, uint16_t bits) {
     float w = h2f(bits);
@@ -156,12 +166,7 @@ __device__ __forceinline__ float score_of(const AcceptParams& ap, int row, int v
                 seen = true;
                 gen += 1;
             }
-        if (ap.pen_has_rep && seen) {
-            const float a = w > 0.0f ? __fdiv_rn(w, ap.pen_rep) : __fmul_rn(w, ap.pen_rep);
-            w = fminf(fmaxf(a, -3.40282347e+38f), 3.40282347e+38f);
-        }
-        if (ap.pen_has_pf && gen != 0)
-            w = __fsub_rn(w, (float)__dadd_rn(ap.pen_presence, __dmul_rn(ap.pen_frequency, (double)gen)));
+        w = penalised(ap, w, seen, gen);
     }
     return w;
 }
@@ -617,8 +622,111 @@ __device__ __forceinline__ uint32_t key_bits(int key) {
     return (asc & 0x8000u) ? (asc & 0x7FFFu) : (~asc & 0xFFFFu);
 }
 
-// The candidates of rank bin `bin` that sit exactly on the bin's value, in index order over
-// [v0, v1).  Without penalties they are found by their fp16 bits.
+// Calls fn(v) for the tokens of a row's root path without the root (the ones its penalties count besides the history), from
+// as many lanes, a repeated token once.
+template <class Fn>
+__device__ __forceinline__ void on_path_tokens(const AcceptParams& ap, int row, Fn&& fn) {
+    if (row >= ap.m || threadIdx.x >= TSV_MAX_ROWS) return;
+    int at = row;
+    for (int i = threadIdx.x; i > 0 && at > 0; i--) at = ap.parent[at];
+    if (at <= 0) return;
+    const int v = ap.feed[at];
+    for (int s = row; s != at; s = ap.parent[s])
+        if (ap.feed[s] == v) return;
+    fn(v);
+}
+
+// The candidates of rank bin `bin` that sit exactly on the bin's value, found by a workgroup of 1024 threads: the row (and with
+// penalties the history's table) is read ONCE, coalesced -- neighbouring lanes take neighbouring groups of eight entries, where
+// a lane reading its own contiguous chunk touches 64 cache lines per load -- and leaves one bit per entry in LDS; each thread
+// then walks the bits of its own contiguous chunk of `groups` bytes, in the index order the sums are defined in.
+// Penalised: an entry that no penalty touches is found by its fp16 bits like any other; the few touched ones are noted in
+// registers and scored afterwards, each lane its own (scoring inside the sweep would have every wave do it for every group).
+// 128 256 entries, 2000 tokens of history: k_pick 192 -> 43 us; k_trunc_cut, seven rows, 281 -> 46 us (with sum_bins): they read
+// entry by entry and walked the root path for each.
+constexpr int PICK_MASK_GROUPS = 32;  // groups of eight entries per thread the match mask holds: vocabularies to 262 144
+__device__ __forceinline__ int mask_groups(int vocab) { return ((vocab + 1023) / 1024 + 7) >> 3; }
+template <bool PEN>
+__device__ __forceinline__ void build_mask(const AcceptParams& ap, int row, const uint16_t* lp, int bin, uint8_t* mask8) {
+    const int tid = threadIdx.x, vocab = ap.vocab, groups = mask_groups(vocab);
+    const uint32_t want = key_bits(bin);
+    const bool zero_bin = want == 0;
+    const float g16 = h2f((uint16_t)want);
+    const int whole = vocab >> 3;  // groups of eight entries that lie wholly inside the row
+    constexpr int B = PEN ? 8 : 16;  // loads of the row in flight per lane; a group past the last whole one reads group 0 and is discarded
+    for (int g0 = 0; g0 < groups; g0 += B) {
+        uint4 q[B], c[PEN ? 2 * B : 1];
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const int g = (g0 + j) * 1024 + tid;
+            const long at = g0 + j < groups && g < whole ? (long)g * 8 : 0;
+            q[j] = *(const uint4*)(lp + at);
+            if constexpr (PEN) {
+                c[2 * j] = *(const uint4*)(ap.pen_cnt + at);
+                c[2 * j + 1] = *(const uint4*)(ap.pen_cnt + at + 4);
+            }
+        }
+        uint32_t touched[PEN ? B / 4 : 1] = {};
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const int g = (g0 + j) * 1024 + tid;
+            const uint32_t t[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+            uint32_t m = 0;
+#pragma unroll
+            for (int h = 0; h < 8; h++) {
+                const uint32_t bits = (t[h >> 1] >> (16 * (h & 1))) & 0xFFFFu;
+                m |= (uint32_t)(bits == want || (zero_bin && bits == 0x8000u)) << h;
+            }
+            if constexpr (PEN) {
+                const uint4 a = c[2 * j], b = c[2 * j + 1];
+                const uint32_t cc[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+                uint32_t pen = 0;
+#pragma unroll
+                for (int h = 0; h < 8; h++) pen |= (uint32_t)(cc[h] != 0) << h;
+                m &= ~pen;
+                if (g0 + j < groups && g < whole) touched[j >> 2] |= pen << (8 * (j & 3));
+            }
+            if (g0 + j < groups) mask8[g] = g < whole ? (uint8_t)m : (uint8_t)0;
+        }
+        if constexpr (PEN) {
+#pragma unroll
+            for (int w = 0; w < B / 4; w++)
+                for (uint32_t left = touched[w]; left; left &= left - 1) {
+                    const int at = __ffs(left) - 1, g = (g0 + 4 * w + (at >> 3)) * 1024 + tid, v = g * 8 + (at & 7);
+                    const uint32_t cnt = ap.pen_cnt[v];
+                    if (penalised(ap, h2f(lp[v]), (cnt >> 31) != 0, cnt & 0x7FFFFFFFu) == g16) mask8[g] |= (uint8_t)(1u << (at & 7));
+                }
+        }
+    }
+    if ((vocab & 7) && whole < groups * 1024 && tid == (whole & 1023)) {  // the row's last, partial group
+        uint32_t m = 0;
+        for (int h = 0; h < (vocab & 7); h++) {
+            const int v = whole * 8 + h;
+            bool on = lp[v] == want || (zero_bin && lp[v] == 0x8000u);
+            if constexpr (PEN) on = score_of<true>(ap, row, v, lp[v]) == g16;
+            m |= (uint32_t)on << h;
+        }
+        mask8[whole] = (uint8_t)m;
+    }
+    __syncthreads();
+    if constexpr (PEN) {
+        on_path_tokens(ap, row, [&](int v) {  // their penalties count more than the table says
+            uint32_t* const word = (uint32_t*)mask8 + (v >> 5);
+            if (score_of<true>(ap, row, v, lp[v]) == g16) atomicOr(word, 1u << (v & 31));
+            else atomicAnd(word, ~(1u << (v & 31)));
+        });
+        __syncthreads();
+    }
+}
+// the entries of thread tid's chunk whose bit is set, ascending
+template <class Fn>
+__device__ __forceinline__ void walk_mask(const uint8_t* mask8, int groups, Fn&& on_match) {
+    const uint8_t* mine = mask8 + threadIdx.x * groups;
+    for (int k = 0; k < groups; k++)
+        for (uint32_t m = mine[k]; m; m &= m - 1) on_match((threadIdx.x * groups + k) * 8 + (__ffs(m) - 1));
+}
+
+// The same candidates over [v0, v1) without a mask, for rows that are not 16-byte aligned or longer than it holds.
 template <bool PEN, class Fn>
 __device__ __forceinline__ void scan_on(const AcceptParams& ap, int row, const uint16_t* lp, int v0, int v1, int bin,
                                         bool vec, Fn&& on_match) {
@@ -640,23 +748,52 @@ struct SideEnt {
     float w;
     int32_t v;
 };
-__device__ int collect_side(const AcceptParams& ap, int row, const uint16_t* lp, int bin, SideEnt* raw,
+__device__ __forceinline__ int collect_side(const AcceptParams& ap, int row, const uint16_t* lp, int bin, SideEnt* raw,
                             SideEnt* sorted, int* counter, int32_t* err) {
     const int tid = threadIdx.x;
     const float g = h2f((uint16_t)key_bits(bin));
     __syncthreads();
     if (tid == 0) *counter = 0;
     __syncthreads();
-    for (int v = tid; v < ap.vocab; v += 1024) {
-        bool flagged = ap.pen_cnt[v] != 0;
-        for (int s = row < ap.m ? row : 0; s > 0; s = ap.parent[s]) flagged |= ap.feed[s] == v;
-        if (!flagged) continue;  // an untouched score is an fp16 value: on its bin's value
-        const float w = score_of<true>(ap, row, v, lp[v]);
+    // (an untouched score is an fp16 value: on its bin's value)
+    auto look = [&](int v, float w) {
         if (w != g && (int)rank_key(floor16(w)) == bin) {
             const int i = atomicAdd(counter, 1);
             if (i < SIDE_CAP) raw[i] = SideEnt{w, v};
         }
+    };
+    // the history's table in fours, eight loads in flight; the touched entries are scored afterwards, each lane its own, and
+    // the tokens of the row's path once more by themselves
+    auto on_path = [&](int v) {
+        for (int s = row < ap.m ? row : 0; s > 0; s = ap.parent[s])
+            if (ap.feed[s] == v) return true;
+        return false;
+    };
+    auto from_table = [&](int v) {
+        const uint32_t c = ap.pen_cnt[v];
+        const float w = penalised(ap, h2f(lp[v]), (c >> 31) != 0, c & 0x7FFFFFFFu);
+        if (!on_path(v)) look(v, w);
+    };
+    const int fours = ap.vocab >> 2;
+    for (int g0 = 0; g0 < fours; g0 += 8 * 1024) {
+        uint4 c[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int f = g0 + j * 1024 + tid;
+            c[j] = *(const uint4*)(ap.pen_cnt + (f < fours ? (long)f * 4 : 0));
+        }
+        uint32_t touched = 0;
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (g0 + j * 1024 + tid < fours)
+                touched |= ((uint32_t)(c[j].x != 0) | (uint32_t)(c[j].y != 0) << 1 | (uint32_t)(c[j].z != 0) << 2 | (uint32_t)(c[j].w != 0) << 3) << (4 * j);
+        for (; touched; touched &= touched - 1) {
+            const int at = __ffs(touched) - 1;
+            from_table((g0 + (at >> 2) * 1024 + tid) * 4 + (at & 3));
+        }
     }
+    if (tid < (ap.vocab & 3) && ap.pen_cnt[fours * 4 + tid] != 0) from_table(fours * 4 + tid);
+    on_path_tokens(ap, row, [&](int v) { look(v, score_of<true>(ap, row, v, lp[v])); });
     __syncthreads();
     int n = *counter;
     if (n > SIDE_CAP) {  // refused: more penalised candidates between two neighbouring fp16 values than the list holds
@@ -695,6 +832,47 @@ __device__ unsigned long long block_scan_u64(unsigned long long loc, unsigned lo
     return wbase + inc - loc;
 }
 
+// The 64 rank bins of one thread (64 words apart, see bin_addr): their sum, in four runs of sixteen, and the first bin at which
+// the running sum from *c on reaches `target` (c < target <= c + sum); *c becomes the sum before it.  Only the run that holds it
+// is fetched again, all of it at once: a loop that stops at the hit waits out one memory round trip per bin.
+template <class T>
+__device__ __forceinline__ unsigned long long sum_bins(const T* mine, unsigned long long (&quarter)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        T v[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = mine[(q * 16 + i) * 64];
+        quarter[q] = 0;
+#pragma unroll
+        for (int i = 0; i < 16; i++) quarter[q] += v[i];
+    }
+    return quarter[0] + quarter[1] + quarter[2] + quarter[3];
+}
+template <class T>
+__device__ __forceinline__ int bin_reaching(const T* mine, const unsigned long long (&quarter)[4], unsigned long long target, unsigned long long* c) {
+    int b = 0;
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+        if (b == q && *c + quarter[q] < target) {
+            *c += quarter[q];
+            b = q + 1;
+        }
+    T v[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = mine[(b * 16 + i) * 64];
+    unsigned long long at = *c;
+    int hit = -1;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        if (hit < 0 && target <= at + v[i]) {
+            hit = b * 16 + i;
+            *c = at;
+        }
+        at += v[i];
+    }
+    return hit;
+}
+
 // One workgroup per distribution row.
 template <bool PEN>
 __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, const uint16_t* draft,
@@ -702,6 +880,7 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
                                                     const unsigned long long* tmass, const uint32_t* tcount,
                                                     AcceptResult* res, int32_t* err) {
     __shared__ SideEnt s_raw[PEN ? SIDE_CAP : 1], s_sorted[PEN ? SIDE_CAP : 1];
+    __shared__ uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // build_mask
     __shared__ int s_nside;
     __shared__ unsigned long long wsum[16];
     __shared__ unsigned long long s_before_p;
@@ -723,43 +902,29 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
     __syncthreads();
     unsigned long long total, total_p = 0;
     if (ap.top_k > 0) {
-        unsigned long long loc = 0;
-#pragma unroll 16
-        for (int i = 0; i < 64; i++) loc += cmine[i * 64];
+        unsigned long long quarter[4];
+        const unsigned long long loc = sum_bins(cmine, quarter);
         const unsigned long long excl = block_scan_u64(loc, wsum, &total);
         const unsigned long long K = (unsigned long long)ap.top_k;
         if (excl < K && K <= excl + loc) {
             unsigned long long c = excl;
-            for (int i = 0; i < 64; i++) {
-                const unsigned long long cv = cmine[i * 64];
-                if (K <= c + cv) {
-                    s_bin_k = tid * 64 + i;
-                    s_j_k = (int)(K - c);
-                    break;
-                }
-                c += cv;
-            }
+            const int i = bin_reaching(cmine, quarter, K, &c);
+            s_bin_k = tid * 64 + i;
+            s_j_k = (int)(K - c);
         }
     }
     if (ap.has_top_p) {
-        unsigned long long loc = 0;
-#pragma unroll 16
-        for (int i = 0; i < 64; i++) loc += mmine[i * 64];
+        unsigned long long quarter[4];
+        const unsigned long long loc = sum_bins(mmine, quarter);
         const unsigned long long excl = block_scan_u64(loc, wsum, &total);
         total_p = total;
         const unsigned long long tgt = (unsigned long long)(ap.top_p * FIX);
         if (excl < tgt && tgt <= excl + loc) {
             unsigned long long c = excl;
-            for (int i = 0; i < 64; i++) {
-                const unsigned long long mv = mmine[i * 64];
-                if (mv > 0 && tgt <= c + mv) {
-                    s_bin_p = tid * 64 + i;
-                    s_before_p = c;
-                    s_cnt_p = (int)cmine[i * 64];
-                    break;
-                }
-                c += mv;
-            }
+            const int i = bin_reaching(mmine, quarter, tgt, &c);
+            s_bin_p = tid * 64 + i;
+            s_before_p = c;
+            s_cnt_p = (int)cmine[i * 64];
         }
     }
     if (!PEN && ap.has_min_p) {  // (penalised rounds test e >= min_p per candidate instead)
@@ -847,14 +1012,19 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
         }
         if (on_value) {
             // the j-th candidate on the bin's value in index order
-            const int per = ((vocab + 1023) / 1024 + 7) & ~7, v0 = min(tid * per, vocab), v1 = min(v0 + per, vocab);
-            const bool vec = ((uintptr_t)lp & 15) == 0;
+            const int groups = mask_groups(vocab), v0 = min(tid * groups * 8, vocab), v1 = min(v0 + groups * 8, vocab);
+            const bool vec = ((uintptr_t)lp & 15) == 0, masked = vec && groups <= PICK_MASK_GROUPS;
+            if (masked) build_mask<PEN>(ap, row, lp, bin, (uint8_t*)s_mask);
+            auto for_matches = [&](auto&& on_match) {
+                if (masked) walk_mask((const uint8_t*)s_mask, groups, on_match);
+                else scan_on<PEN>(ap, row, lp, v0, v1, bin, vec, on_match);
+            };
             int n = 0;
-            scan_on<PEN>(ap, row, lp, v0, v1, bin, vec, [&](int) { n++; });
+            for_matches([&](int) { n++; });
             const unsigned long long excl = block_scan_u64((unsigned long long)n, wsum, &total);
             if ((int)excl < j && j <= (int)excl + n) {
                 int c = (int)excl;
-                scan_on<PEN>(ap, row, lp, v0, v1, bin, vec, [&](int v) {
+                for_matches([&](int v) {
                     c++;
                     if (c == j) s_idx = v;
                 });
@@ -875,7 +1045,6 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
 // One workgroup per job.  Finds the rank bin in which the cumulative mass first exceeds the
 // uniform (exact integer prefix over the fixed-point bins, which the round's first kernel zeroed), then
 // walks that bin's candidates in index order in f64.
-constexpr int PICK_MASK_GROUPS = 32;  // groups of eight entries per thread the match mask holds: vocabularies to 262 144
 template <bool PEN>
 __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uint16_t* draft,
                                                const AcceptParams* app, double* scratch, const double* work,
@@ -883,7 +1052,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
                                                AcceptResult* res, int32_t* tokens_out, int32_t* err,
                                                int kind) {
     __shared__ SideEnt s_raw[PEN ? SIDE_CAP : 1], s_sorted[PEN ? SIDE_CAP : 1];
-    __shared__ uint32_t s_mask[PEN ? 1 : 1024 * PICK_MASK_GROUPS / 4];  // one bit per vocabulary entry: on the bin's value
+    __shared__ uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // one bit per vocabulary entry: on the bin's value
     __shared__ int s_nside, s_side_last;
     __shared__ double s_side_sum;
     __shared__ unsigned long long wsum[16];
@@ -1038,64 +1207,13 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
             side_sum = s_side_sum;
         }
         // walk the bin in index order: contiguous index chunk per thread
-        const int per = ((vocab + 1023) / 1024 + 7) & ~7, v0 = min(tid * per, vocab), v1 = min(v0 + per, vocab);
-        const bool vec = ((uintptr_t)lp & 15) == 0;
-        // Without penalties a candidate of the bin is found by its fp16 bits.  The row is read ONCE, coalesced --
-        // neighbouring lanes take neighbouring groups of eight entries, where a lane reading its own contiguous chunk
-        // touches 64 cache lines per load -- and leaves one bit per entry in LDS; each thread then walks the bits of
-        // its own chunk, here and again in the walk below, in the index order the sums are defined in.
-        const int groups = per >> 3;
-        const bool masked = !PEN && vec && groups <= PICK_MASK_GROUPS;
-        if constexpr (!PEN) {
-            if (masked) {
-                uint8_t* mask8 = (uint8_t*)s_mask;
-                const uint32_t want = key_bits(bin);
-                const bool zero_bin = want == 0;
-                // sixteen loads in flight per lane: a group past the row's last whole one reads group 0 and is discarded
-                const int whole = vocab >> 3;  // groups of eight entries that lie wholly inside the row
-                for (int g0 = 0; g0 < groups; g0 += 16) {
-                    uint4 q[16];
-#pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        const int g = (g0 + j) * 1024 + tid;
-                        q[j] = *(const uint4*)(lp + (g0 + j < groups && g < whole ? (long)g * 8 : 0));
-                    }
-#pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        if (g0 + j >= groups) break;
-                        const int g = (g0 + j) * 1024 + tid;
-                        const uint32_t t[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
-                        uint32_t m = 0;
-#pragma unroll
-                        for (int h = 0; h < 8; h++) {
-                            const uint32_t bits = (t[h >> 1] >> (16 * (h & 1))) & 0xFFFFu;
-                            m |= (uint32_t)(bits == want || (zero_bin && bits == 0x8000u)) << h;
-                        }
-                        mask8[g] = g < whole ? (uint8_t)m : (uint8_t)0;
-                    }
-                }
-                if ((vocab & 7) && whole < groups * 1024 && tid == (whole & 1023)) {  // the row's last, partial group
-                    uint32_t m = 0;
-                    for (int h = 0; h < (vocab & 7); h++) {
-                        const uint32_t bits = lp[(long)whole * 8 + h];
-                        m |= (uint32_t)(bits == want || (zero_bin && bits == 0x8000u)) << h;
-                    }
-                    mask8[whole] = (uint8_t)m;
-                }
-                __syncthreads();
-            }
-        }
+        const int groups = mask_groups(vocab), v0 = min(tid * groups * 8, vocab), v1 = min(v0 + groups * 8, vocab);
+        const bool vec = ((uintptr_t)lp & 15) == 0, masked = vec && groups <= PICK_MASK_GROUPS;
+        if (masked) build_mask<PEN>(ap, dec.job.row_p, lp, bin, (uint8_t*)s_mask);
         // on_match(v) for the candidates of this thread's chunk that sit on the bin's value, ascending
         auto for_matches = [&](auto&& on_match) {
-            if constexpr (!PEN) {
-                if (masked) {
-                    const uint8_t* mine = (const uint8_t*)s_mask + tid * groups;
-                    for (int k = 0; k < groups; k++)
-                        for (uint32_t m = mine[k]; m; m &= m - 1) on_match(v0 + 8 * k + (__ffs(m) - 1));
-                    return;
-                }
-            }
-            scan_on<PEN>(ap, dec.job.row_p, lp, v0, v1, bin, vec, on_match);
+            if (masked) walk_mask((const uint8_t*)s_mask, groups, on_match);
+            else scan_on<PEN>(ap, dec.job.row_p, lp, v0, v1, bin, vec, on_match);
         };
         double lsum = 0.0;
         int lastv = -1;
