@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # rows and columns around the 128-column tiles and the 256-, 128- and 64-wide chunks; m around the 64-, 128- and 256-row tiles
 @pytest.mark.parametrize("dtype,rows,cols", [(12, 64, 512), (12, 200, 768), (13, 64, 512), (13, 200, 768), (14, 130, 512), (14, 64, 1024),
                                              (8, 64, 128), (8, 200, 1408), (30, 64, 64), (30, 130, 2880), (39, 64, 256), (39, 200, 2880)])
-@pytest.mark.parametrize("m", [17, 64, 65, 128, 129, 257])
+@pytest.mark.parametrize("m", [17, 64, 65, 128, 129, 257, 321])
 def test_the_prompt_matmul_is_the_dequantized_product(dtype, rows, cols, m):
     from turbospark_amd import ffi
     w = lcg_weights(rows * cols, 5).reshape(rows, cols) * 0.05

@@ -332,27 +332,15 @@ constexpr int lds_bytes() {
     return (2 * stage_bytes<F>() < 65536 ? 65536 : 2 * stage_bytes<F>()) + 2 * CHUNK_BYTES;
 }
 
+// One tile: BM = 64 * 4 / WN rows from row0 on, of which `rows` exist.
 template <class F, int WN, int EPI>
-__global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
+__device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* lds, int split, int nb, int row0, int rows, int expert) {
     constexpr int NT = 4 / WN, BM = 64 * (4 / WN), KS = F::STAGE_K / 16, GROUPS = KS / 2, STAGE = stage_bytes<F>();
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint8_t* const side = lds + lds_bytes<F>() - 2 * CHUNK_BYTES;  // [chunk % 2][min operands, coefficients]
     auto mins_of = [&](int c) { return side + (c & 1) * CHUNK_BYTES; };
     auto coef_of = [&](int c) { return (float2*)(side + (c & 1) * CHUNK_BYTES + MIN_BYTES); };
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WN, wn = wave % WN, t64 = wave >> 1, part = wave & 1;
-    // which tile: XCD x takes the column blocks x, x + 8, ..., all row blocks of one before the next
-    const int per_split = (g.nt + 7) / 8 * 8 * g.mt, split = blockIdx.x / per_split, id = blockIdx.x - split * per_split;
-    const int slot = id >> 3, nb = slot / g.mt * 8 + (id & 7), mb = slot % g.mt;
-    if (nb >= g.nt) return;
-    int row0 = mb * BM, rows = g.m - row0, expert = 0;  // the tile's first row and how many of its rows exist
-    if (g.tiles) {
-        if (mb >= *g.tile_count) return;
-        const PromptTile t = g.tiles[mb];
-        row0 = t.first;
-        rows = t.cnt;
-        expert = t.expert;
-    }
     const int c0 = split * g.chunks_per_split, c1 = min(c0 + g.chunks_per_split, g.kchunks);
     const int s0 = c0 * F::SPC, s1 = c1 * F::SPC;
     const int tile = expert * g.n_tiles + min(2 * nb + t64, g.n_tiles - 1);  // (an odd count: the last block's second half repeats the last tile)
@@ -557,6 +545,29 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     }
 }
 
+// The grid's tiles are g.bm rows; a tile that holds fewer takes the smallest form that covers them.  Short last tiles cost what
+// their rows cost then: 299 rows in tiles of 256 were multiplied as 512, in tiles of 128 as 384 (and came out at 1.3 workgroups
+// per place on the chip).
+template <class F, int EPI>
+__global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    // which tile: XCD x takes the column blocks x, x + 8, ..., all row blocks of one before the next
+    const int per_split = (g.nt + 7) / 8 * 8 * g.mt, split = blockIdx.x / per_split, id = blockIdx.x - split * per_split;
+    const int slot = id >> 3, nb = slot / g.mt * 8 + (id & 7), mb = slot % g.mt;
+    if (nb >= g.nt) return;
+    int row0 = mb * g.bm, rows = min(g.m - row0, g.bm), expert = 0;  // the tile's first row and how many of its rows exist
+    if (g.tiles) {
+        if (mb >= *g.tile_count) return;
+        const PromptTile t = g.tiles[mb];
+        row0 = t.first;
+        rows = t.cnt;
+        expert = t.expert;
+    }
+    if (rows > 128) prompt_tile<F, 1, EPI>(g, lds, split, nb, row0, rows, expert);
+    else if (rows > 64) prompt_tile<F, 2, EPI>(g, lds, split, nb, row0, rows, expert);
+    else prompt_tile<F, 4, EPI>(g, lds, split, nb, row0, rows, expert);
+}
+
 // ---- experts with few rows, MXFP4 -----------------------------------------------------------------------------------------
 // The tile of the kernel above at 64 rows is bound by the L1 and the LDS, not by the matrix pipes (each wave draws all 64 rows'
 // activations, and every unpacked weight crosses the LDS for 64 rows only), and a stage ahead is too little in flight for a
@@ -749,7 +760,7 @@ __global__ __launch_bounds__(64) void k_row_scale(const uint8_t* __restrict__ ti
     rs[tile * 64 + lane] = __uint_as_float((uint32_t)(s + 127) << 23);
 }
 
-template <class F, int WN, int EPI>
+template <class F, int EPI>
 int launch_p(hipStream_t s, const PromptGemmArgs& g) {
     // more than 64 KiB of dynamic LDS has to be allowed once per kernel and device
     static std::atomic<uint64_t> allowed{0};
@@ -757,29 +768,21 @@ int launch_p(hipStream_t s, const PromptGemmArgs& g) {
     TSV_HIP(hipGetDevice(&dev));
     const uint64_t bit = 1ull << (dev & 63);
     if (!(allowed.load(std::memory_order_acquire) & bit)) {
-        TSV_HIP(hipFuncSetAttribute((const void*)k_prompt_gemm<F, WN, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<F>()));
+        TSV_HIP(hipFuncSetAttribute((const void*)k_prompt_gemm<F, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<F>()));
         allowed.fetch_or(bit, std::memory_order_release);
     }
     const int blocks = (g.nt + 7) / 8 * 8 * g.mt * g.splits;
-    hipLaunchKernelGGL((k_prompt_gemm<F, WN, EPI>), dim3(blocks), dim3(256), lds_bytes<F>(), s, g);
+    hipLaunchKernelGGL((k_prompt_gemm<F, EPI>), dim3(blocks), dim3(256), lds_bytes<F>(), s, g);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }
 template <class F>
-int launch_f(hipStream_t s, PromptGemmArgs& g, int epi, int bm) {
-    if (!g.tiles) g.mt = (g.m + bm - 1) / bm;
-    if (epi == EPI_SILU) return bm == 256 ? launch_p<F, 1, EPI_SILU>(s, g) : bm == 128 ? launch_p<F, 2, EPI_SILU>(s, g) : launch_p<F, 4, EPI_SILU>(s, g);
-    return bm == 256 ? launch_p<F, 1, EPI_PARTIAL>(s, g) : bm == 128 ? launch_p<F, 2, EPI_PARTIAL>(s, g) : launch_p<F, 4, EPI_PARTIAL>(s, g);
+int launch_f(hipStream_t s, PromptGemmArgs& g, int epi) {
+    if (!g.tiles) g.mt = (g.m + g.bm - 1) / g.bm;
+    return epi == EPI_SILU ? launch_p<F, EPI_SILU>(s, g) : launch_p<F, EPI_PARTIAL>(s, g);
 }
 
-// Rows of a tile: 256, where the weights are unpacked for the most rows; 128 where that saves a twelfth of the padded rows.
-// (299 rows behind 3001, 16 layers of the 8B shape in the Q5_K_M mix: 7.06 ms in tiles of 256, 6.66 of 128, 7.48 of 64;
-// 1500 rows, the same padding either way: 5.16 against 5.28 in the gpt-oss shape.)
-int row_block(int m) {
-    if (m <= 64) return 64;
-    const int p128 = (m + 127) / 128 * 128, p256 = (m + 255) / 256 * 256;
-    return p256 * 12 > p128 * 13 ? 128 : 256;
-}
+int row_block(int m) { return m > 128 ? 256 : m > 64 ? 128 : 64; }
 
 }  // namespace
 
@@ -798,13 +801,13 @@ int prompt_splits(const TiledW& w, int m) {
     return (w.kchunks + per - 1) / per;
 }
 
-static int launch_any(hipStream_t s, int fmt, PromptGemmArgs& g, int epi, int bm) {
-    return fmt == FMT_Q4K    ? launch_f<PromptQ45<false>>(s, g, epi, bm)
-           : fmt == FMT_Q5K  ? launch_f<PromptQ45<true>>(s, g, epi, bm)
-           : fmt == FMT_Q6K  ? launch_f<PromptQ6>(s, g, epi, bm)
-           : fmt == FMT_Q80  ? launch_f<PromptQ8>(s, g, epi, bm)
-           : fmt == FMT_BF16 ? launch_f<PromptBf>(s, g, epi, bm)
-                             : launch_f<PromptMx>(s, g, epi, bm);
+static int launch_any(hipStream_t s, int fmt, PromptGemmArgs& g, int epi) {
+    return fmt == FMT_Q4K    ? launch_f<PromptQ45<false>>(s, g, epi)
+           : fmt == FMT_Q5K  ? launch_f<PromptQ45<true>>(s, g, epi)
+           : fmt == FMT_Q6K  ? launch_f<PromptQ6>(s, g, epi)
+           : fmt == FMT_Q80  ? launch_f<PromptQ8>(s, g, epi)
+           : fmt == FMT_BF16 ? launch_f<PromptBf>(s, g, epi)
+                             : launch_f<PromptMx>(s, g, epi);
 }
 
 int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int m, int splits, int epi,
@@ -836,7 +839,8 @@ int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void
     g.nt = (w.n_tiles + 1) / 2;
     g.n_valid = epi == EPI_SILU ? w.n_rows / 2 : n_valid;
     g.out_k16 = prompt_k16(w.n_rows / 2);
-    return launch_any(s, w.fmt, g, epi, row_block(m));
+    g.bm = row_block(m);
+    return launch_any(s, w.fmt, g, epi);
 }
 
 int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int epi, int ldo,
@@ -877,7 +881,8 @@ int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const v
         TSV_HIP(hipGetLastError());
         return TSV_OK;
     }
-    return launch_any(s, w.fmt, g, epi, x.bm);
+    g.bm = x.bm;
+    return launch_any(s, w.fmt, g, epi);
 }
 
 }  // namespace tsv

@@ -63,7 +63,7 @@ struct PromptGemmArgs {
     int m, n_tiles, kchunks, chunks_per_split, splits, ldo, n_valid;
     int a_k16;            // 16-K steps per row of the activations
     int out_k16;
-    int mt, nt;           // tiles of the grid: rows, 128 columns
+    int mt, nt, bm;       // tiles of the grid: row tiles of bm = 256, 128 or 64 rows, 128 columns
     // routed experts: the row tiles, expert e owning n_tiles row tiles of w from e * n_tiles on; biases [expert][columns];
     // alpha > 0: the clamped SwiGLU (moe_gguf.metal:528-556).  EPI_PARTIAL then writes float [row / 16][8 slots][16][ldo]
     const PromptTile* tiles;
