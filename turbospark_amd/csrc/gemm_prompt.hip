@@ -406,13 +406,15 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
             }
             if (!last) {
                 F::unpack(w, bits, unit, rs, lds + (buf ^ 1) * STAGE, mins_of((s + sub + 1) / F::SPC), coef_of((s + sub + 1) / F::SPC), (sub + 1) % F::SPC, part, t64, lane);
-                load_w(s + sub + 2, (sub + 2) % F::SPC);
             }
 #pragma unroll
             for (int grp = 0; grp < GROUPS; grp++) {
                 constexpr int one = 1;
                 if (grp + 1 < GROUPS) load_a((grp + one) & 1, s + sub, grp + 1);
                 else load_a((grp + one) & 1, s + sub + 1, 0);
+                // loads return in order: asked for before the activations of group 1, the weights (from memory, where the
+                // activations are in the L2) would have to be there before that group; now they have two groups' products
+                if (grp == 0) load_w(s + sub + 2, (sub + 2) % F::SPC);
 #pragma unroll
                 for (int q = 0; q < 2; q++)
 #pragma unroll
