@@ -106,3 +106,26 @@ def test_routed_prompts_give_every_row_its_experts(name, n):
         # 8 units in the last place of an fp16 value of the row's largest size: fp32 sums in another order, rounded to fp16 activations
         far = np.abs(got - want).max(1) > 8 * 2.0 ** -11 * np.abs(want).max(1)
         assert far.sum() <= max(1, n // 50), np.flatnonzero(far)
+
+
+@pytest.mark.parametrize("name,n,limit", [("small_q4_k", 300, 0), ("moe_small", 130, 1 << 20), ("small_q4_k", 64, 3 << 20)])
+def test_a_device_without_room_for_prompt_buffers_takes_the_64_row_passes(name, n, limit):
+    """The buffers refused at the first and at a later allocation: the same call succeeds, in the passes the handle has buffers
+    for, and takes the large passes again once there is room."""
+    import turbospark_amd as ts
+    from turbospark_amd import ffi, synth
+    cfg = dict(synth.CONFIGS[name], max_context=n + 32)
+    eng = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=9))
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
+    kv = []
+    for bytes_ in (limit, limit, 1 << 40):
+        eng.reset()
+        ffi.check(ffi.lib().tsv_limit_prompt_buffers(eng._h, bytes_))
+        eng.prefill(prompt, 0, want_logits=False)
+        assert eng.position == n
+        kv.append(eng.read_kv(0, 0, n))
+    for (a, b, c) in zip(*kv):          # the first layer's rows: sums of the same products
+        a, b, c = (t.astype(np.float32) for t in (a, b, c))
+        assert (a == b).all()
+        # each side rounds an fp32 sum of about sqrt(K) roundings to fp16: two units in the last place of the largest value
+        assert np.abs(a - c).max() <= 2 * 2.0 ** -11 * np.abs(a).max()

@@ -119,6 +119,8 @@ struct tsv_ctx {
         uint8_t *a_s = nullptr, *a_e = nullptr, *s_e = nullptr, *s_s = nullptr;
         float* moe_out = nullptr;
         std::vector<void*> allocs;
+        size_t held = 0;
+        size_t limit = SIZE_MAX;  // test hook (tsv_limit_prompt_buffers): most bytes the buffers may take
     } prompt;
     bool route_forced_set = false;  // tsv_force_route holds selections: prompt passes stay at sixteen rows
     uint16_t* q16 = nullptr;
@@ -241,6 +243,8 @@ int stage_params(tsv_ctx* c, const VerifyParams* vp, int n, VerifyParams* dev);
 // PROMPT_ROWS) at the cursor.  finish: the rows' last residual add as well, left in prompt.x and, the last (n - 1) % 16 + 1
 // rows, in x; logits: those rows' logits too.
 bool prompt_supported(const tsv_ctx* c);
+// prompt_reserve: buffers for passes of n rows, or none at all where the device has no room for them.
+int prompt_reserve(tsv_ctx* c, int n);
 int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits);
 void prompt_free(tsv_ctx* c);
 // One verify pass: everything enqueued on the handle's stream, no synchronisation; then the optional copy of the rows' logits.

@@ -18,6 +18,7 @@ void prompt_free(tsv_ctx* c) {
     for (void* p : c->prompt.allocs) (void)hipFree(p);
     c->prompt.allocs.clear();
     c->prompt.rows = 0;
+    c->prompt.held = 0;
 }
 
 namespace {
@@ -25,8 +26,13 @@ namespace {
 template <class T>
 int prompt_alloc(tsv_ctx* c, T** p, size_t bytes, bool zero) {
     void* q = nullptr;
+    if (c->prompt.held + bytes > c->prompt.limit) {
+        set_error("prefill: buffers of a prompt pass past the limit of tsv_limit_prompt_buffers");
+        return TSV_ERR_DEVICE;
+    }
     TSV_HIP(hipMalloc(&q, bytes));
     c->prompt.allocs.push_back(q);
+    c->prompt.held += bytes;
     if (zero) TSV_HIP(hipMemsetAsync(q, 0, bytes, c->stream));
     *p = (T*)q;
     return TSV_OK;
@@ -34,9 +40,8 @@ int prompt_alloc(tsv_ctx* c, T** p, size_t bytes, bool zero) {
 
 // Buffers for n rows.  The activations are cleared once: the K padding behind a width that is not whole 256s has to stay zero,
 // and rows past the last one have to hold finite values.
-int prompt_reserve(tsv_ctx* c, int n) {
+int reserve_rows(tsv_ctx* c, int n) {
     tsv_ctx::Prompt& w = c->prompt;
-    if (n <= w.rows) return TSV_OK;
     const int rows = n <= 256 ? 256 : n <= 1024 ? 1024 : PROMPT_ROWS;
     if (w.rows) {
         TSV_HIP(hipStreamSynchronize(c->stream));
@@ -232,6 +237,17 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
 }
 
 }  // namespace
+
+int prompt_reserve(tsv_ctx* c, int n) {
+    if (n <= c->prompt.rows) return TSV_OK;
+    const int rc = reserve_rows(c, n);
+    if (rc) {
+        (void)hipStreamSynchronize(c->stream);  // buffers that were given may still be cleared
+        prompt_free(c);
+        (void)hipGetLastError();  // a refused allocation is not the next launch's error
+    }
+    return rc;
+}
 
 int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits) {
     if (base != c->position) {

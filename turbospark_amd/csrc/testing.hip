@@ -137,6 +137,12 @@ extern "C" int32_t tsv_force_route(tsv_ctx* c, const int32_t* sel, int32_t n_lay
     return TSV_OK;
 }
 
+extern "C" int32_t tsv_limit_prompt_buffers(tsv_ctx* c, int64_t bytes) {
+    TSV_NEED(c && bytes >= 0, "limit_prompt_buffers: bad argument");
+    c->prompt.limit = (size_t)bytes;
+    return TSV_OK;
+}
+
 extern "C" int32_t tsv_write_logits(tsv_ctx* c, const uint16_t* logits, int32_t m, int64_t base) {
     if (!c || !logits || m < 1 || m > TSV_MAX_ROWS || base < 0) {
         set_error("write_logits: bad argument");
