@@ -426,6 +426,8 @@ def main():
         dt = time.perf_counter() - t0
         wide = cfg["dtype"] in (ts.ffi.Q4_K, ts.ffi.Q5_K, ts.ffi.Q8_0, ts.ffi.BF16) and not (cfg.get("n_experts") and os.environ.get("TSV_MOE_FP4"))
         rows = 64 if wide and os.environ.get("TSV_WIDE_PREFILL") != "0" else 16
+        if rows == 64 and n > 64 and args.kv_bits == "off":      # equal passes of up to 2048 rows, whole sixteens
+            rows = min(n, -(-(-(-n // -(-n // 2048))) // 16) * 16)
         print(json.dumps({"metric": "prefill tokens/s", "value": round(n / dt, 1), "unit": "tokens/s", "n_gpus": 1,
                           "higher_is_better": True, "dtype": "f16", "data": "synthetic", "seconds": round(dt, 4),
                           "config": {"workload": args.workload, "weights": args.weights_dtype or "as the workload names",
