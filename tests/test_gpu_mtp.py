@@ -97,6 +97,23 @@ def test_priming_by_the_prefill_equals_priming_token_by_token(name, n):
     assert gc.logit_error(head_a.step(11, n - 1), head_b.step(11, n - 1)) <= 5e-4
 
 
+@pytest.mark.parametrize("name,n", [("xcd_q4_k", 70), ("xcd_q8_0", 100), ("moe_small", 128)])
+def test_a_prompt_without_logits_leaves_its_last_rows_for_an_attached_head(name, n, monkeypatch):
+    """tsv_prefill on a target with a head keeps the last pass's residual rows (tsv_mtp_open), logits or not: the head
+    steps from the last one, as after sixteen-row passes."""
+    cfg, gpu_a, head_a = _build(name, ctx=200, oracle=False)
+    monkeypatch.setenv("TSV_WIDE_PREFILL", "0")
+    _, gpu_b, head_b = _build(name, ctx=200, oracle=False)
+    prompt = np.random.default_rng(12).integers(0, cfg["vocab"], n).astype(np.int32)
+    steps = []
+    for gpu, head in ((gpu_a, head_a), (gpu_b, head_b)):
+        head.prefill_chunk(prompt, 0)              # the head's cache over [0, n - 1)
+        gpu.reset()
+        gpu.prefill(prompt, 0, want_logits=False)
+        steps.append(head.step(11, n - 1))
+    assert gc.logit_error(*steps) <= 5e-4          # the bound of the priming test
+
+
 @pytest.mark.parametrize("block", [1, 4, 15])
 def test_a_block_draft_is_the_chain_of_single_steps(block):
     cfg, gpu, head = _build("small_q4_k", oracle=False)

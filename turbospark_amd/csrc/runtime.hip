@@ -1545,7 +1545,8 @@ int tsv::prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0,
             const int64_t left = n - i, passes = (left + PROMPT_ROWS - 1) / PROMPT_ROWS;
             const int rows = (int)std::min(left, ((left + passes - 1) / passes + 15) / 16 * 16);
             const bool last = i + rows >= n;
-            if (int rc = enqueue_prompt_pass(c, ids + i, rows, pos0 + i, head != nullptr, last && logits)) return rc;
+            // (an attached head's next step reads the pass's last rows, whoever asked for the pass)
+            if (int rc = enqueue_prompt_pass(c, ids + i, rows, pos0 + i, c->mtp_head != nullptr, last && logits)) return rc;
             if (last && logits)
                 TSV_HIP(hipMemcpyAsync(logits, c->logits + (size_t)((rows - 1) % 16) * c->vocab, (size_t)c->vocab * 2, hipMemcpyDeviceToHost, c->stream));
             for (int b = 0; head && b < rows; b += TSV_MAX_ROWS) {
