@@ -47,6 +47,29 @@ def test_prompt_attention_matches_the_oracle(nq, nkv, hd, m, base, window, sinks
         assert np.abs(got[i] - want).max() <= 5e-3 * max(1.0, np.abs(want).max()), i   # the bound of the verify passes' test
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(8, 2, 128), (4, 2, 64)])
+@pytest.mark.parametrize("m,base,spread", [(320, 0, 1.0), (320, 0, 2.5), (96, 2000, 1.0), (96, 2000, 2.5)])
+def test_prompt_attention_is_the_exact_result_rounded(nq, nkv, hd, m, base, spread):
+    """Against softmax and product in 64 bits: the distance is that of the exact result rounded to fp16.  Weights of 21 bits and
+    fp32 sums add a part in 2^-9 of that rounding and less; one per cent covers what is left of it by chance, 1e-5 the scores'
+    own fp32 sums (128 products of a few units: 2^-24 of about 50, seen through exp)."""
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(m + base)
+    r16 = lambda *s: rng.standard_normal(s).astype(np.float16).astype(np.float32)
+    q = (r16(m, nq, hd) * spread).astype(np.float16).astype(np.float32)
+    k, v = r16(base + m, nkv, hd), r16(base + m, nkv, hd)
+    want = np.empty((m, nq, hd))
+    hidden = np.arange(base + m)[None] > base + np.arange(m)[:, None]
+    for h in range(nq):
+        s = q[:, h].astype(np.float64) @ k[:, h * nkv // nq].astype(np.float64).T / np.sqrt(hd)
+        s[hidden] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        want[:, h] = (p / p.sum(1, keepdims=True)) @ v[:, h * nkv // nq].astype(np.float64)
+    got = np.asarray(ffi.attention(q, k, v, base)).reshape(m, nq, hd)
+    off = lambda t: np.linalg.norm(t - want) / np.linalg.norm(want)
+    assert off(got) <= 1.01 * off(want.astype(np.float16).astype(np.float64)) + 1e-5
+
+
 @pytest.mark.parametrize("name,n,start", [("small_q4_k", 65, 0), ("xcd_q8_0", 257, 3), ("small_q5_k_m", 300, 31), ("xcd_q4_k", 2049, 0)])
 def test_prompts_around_the_limits_of_a_pass(name, n, start):
     """Logits of the last token, what a verify pass after the prompt sees, and the rows left for tsv_accept, against passes of
