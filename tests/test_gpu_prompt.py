@@ -31,6 +31,125 @@ def test_the_prompt_matmul_is_the_dequantized_product(dtype, rows, cols, m):
         assert (np.abs(got - want) <= 2e-4 * scale + 1e-9).all(), (splits, np.abs(got - want).max() / scale.max())
 
 
+def _off(entry, values, x, splits=0, column=slice(None)):
+    """Distance of the prompt matmul (or one output column) from the exact product, relative to its norm."""
+    from turbospark_amd import ffi
+    want = (x.astype(np.float16).astype(np.float64) @ values.astype(np.float64).T)[:, column]
+    return np.linalg.norm(ffi.matmul(entry, x, splits)[:, column] - want) / np.linalg.norm(want)
+
+
+# Exact products summed in fp32: a sum of K = 512 values takes 32 roundings of 2^-24 of its running size, twice that where a
+# weight goes in as two terms: 64^0.5 * 2^-24 = 5e-7, and one more factor of two for rows smaller than their running sums.
+SUMS_OF_512 = 1e-6
+
+
+@pytest.mark.parametrize("m", [17, 65, 129, 257])
+@pytest.mark.parametrize("rows,at,big", [(64, 0, 2.0 ** 12), (64, 17, 2.0 ** 31), (130, 129, 2.0 ** 36), (200, 70, 2.0 ** 90), (256, 255, 3e38)])
+def test_bf16_rows_of_any_span_keep_their_bits(rows, at, big, m):
+    """One value far above the rest of a row, against an activation of zero: what is left are the products of the small values,
+    multiplied as bf16 where they are no normal fp16 beside that one (2^29 below it), in the tiles it concerns."""
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(rows + m)
+    w, x = (rng.standard_normal((rows, 512)) * 0.02).astype(np.float32), rng.standard_normal((m, 512)).astype(np.float32)
+    w[at, 7] = big
+    w[rows // 2, 100] = 1e-39                          # and one with a subnormal value
+    x[:, 7] = 0.0
+    entry = ffi.quantize(ffi.BF16, w)
+    values = (np.asarray(entry[1]).reshape(rows, -1).view(np.uint16).astype(np.uint32) << 16).view(np.float32)
+    for splits in (0, 1):
+        assert _off(entry, values, x, splits) <= SUMS_OF_512
+        assert _off(entry, values, x, splits, at) <= SUMS_OF_512
+
+
+@pytest.mark.parametrize("dtype,scale", [(39, 127), (39, 170), (39, 254), (8, 1.0), (8, 65504.0)])
+def test_a_zero_block_of_any_scale_is_zero(dtype, scale):
+    """Blocks whose codes are all zero do not set the power of two that their row is multiplied in."""
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(3)
+    entry = ffi.quantize(dtype, (rng.standard_normal((64, 512)) * 0.02).astype(np.float32))
+    head = 1 if dtype == 39 else 2
+    b = np.array(entry[1]).reshape(64, 16, -1)
+    b[:, 0] = 0
+    values = ob.dequantize(dtype, np.ascontiguousarray(b.reshape(64, -1)), 512)
+    b[:, 0, :head] = np.frombuffer(np.uint8(scale).tobytes() if dtype == 39 else np.float16(scale).tobytes(), np.uint8)
+    entry = (dtype, np.ascontiguousarray(b.reshape(64, -1)), 64, 512)
+    assert _off(entry, values, rng.standard_normal((65, 512)).astype(np.float32)) <= SUMS_OF_512
+
+
+@pytest.mark.parametrize("scale,rest,held", [(0.125, 2.0 ** -24, True), (0.25, 2.0 ** -24, False), (0.25, 1.99 * 2.0 ** -23, True),
+                                             (65504.0, 2.0 ** -6, True), (65504.0, 2.0 ** -7, False), (np.inf, 1.0, False)])
+def test_q8_0_scales_keep_their_bits_or_the_product_is_refused(scale, rest, held):
+    """Scales down to 2^21 below the row's largest; a row with a smaller one is not multiplied in fp16."""
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(4)
+    b = np.array(ffi.quantize(8, (rng.standard_normal((64, 512)) * 0.02).astype(np.float32))[1]).reshape(64, 16, 34)
+    b[:, 0, :2] = np.frombuffer(np.float16(scale).tobytes(), np.uint8)
+    b[:, 1:, :2] = np.frombuffer(np.float16(rest).tobytes(), np.uint8)
+    entry = (8, np.ascontiguousarray(b.reshape(64, -1)), 64, 512)
+    x = rng.standard_normal((65, 512)).astype(np.float32)
+    x[:, :32] = 0.0
+    if held:
+        assert _off(entry, ob.dequantize(8, entry[1], 512), x) <= SUMS_OF_512
+    else:
+        with pytest.raises(ffi.TsvError):
+            ffi.matmul(entry, x)
+
+
+@pytest.mark.parametrize("low,held", [(127 - 25, True), (127 - 26, False), (255, False)])
+def test_mxfp4_blocks_keep_their_bits_or_the_product_is_refused(low, held):
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(5)
+    b = np.array(ffi.quantize(39, rng.standard_normal((64, 512)).astype(np.float32))[1]).reshape(64, 16, 17)
+    b[:, 0, 0], b[:, 1:, 0] = 127, low
+    entry = (39, np.ascontiguousarray(b.reshape(64, -1)), 64, 512)
+    x = rng.standard_normal((65, 512)).astype(np.float32)
+    x[:, :32] = 0.0
+    if held:
+        assert _off(entry, ob.dequantize(39, entry[1], 512), x) <= SUMS_OF_512
+    else:
+        with pytest.raises(ffi.TsvError):
+            ffi.matmul(entry, x)
+
+
+@pytest.mark.parametrize("name", ["tiny_q8_0", "gptoss_small"])
+def test_a_model_of_rows_that_fp16_cannot_hold_prompts_as_before(name):
+    """The first 32 columns of the query, key and value projections hold weights 2^30 above the others (behind a norm weight of
+    zero): a Q8_0 model takes the smaller passes, a bf16 one multiplies those tiles as bf16."""
+    import os
+    import turbospark_amd as ts
+    from turbospark_amd import ffi, synth
+    n = 100
+    cfg = dict(synth.CONFIGS[name], max_context=n + 32)
+    w = synth.make_weights(cfg, seed=8)
+    for lw in w["layers"]:
+        _, v, r, c = lw["attn_norm"]
+        v = np.array(v)
+        v.view(np.float32)[0, :32] = 0.0
+        lw["attn_norm"] = (ffi.F32, v, r, c)
+        for key in ("wq", "wk", "wv"):
+            dt, v, r, c = lw[key]
+            v = np.array(v)
+            if dt == ffi.Q8_0:
+                b = v.reshape(r, -1, 34)
+                b[:, 0, :2], b[:, 0, 2:] = np.frombuffer(np.float16(2.0 ** 15).tobytes(), np.uint8), 1
+            else:
+                v.reshape(r, -1).view(np.uint16)[:, :32] = np.float32(2.0 ** 30).view(np.uint32) >> 16
+            lw[key] = (dt, v, r, c)
+    fast = ts.HipVerifier(cfg, w)
+    os.environ["TSV_WIDE_PREFILL"] = "0"
+    try:
+        slow = ts.HipVerifier(cfg, w)
+    finally:
+        del os.environ["TSV_WIDE_PREFILL"]
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
+    for eng in (fast, slow):
+        eng.prefill(prompt, 0, want_logits=False)
+    for got, want in zip(fast.read_kv(0, 0, n), slow.read_kv(0, 0, n)):
+        got, want = got.astype(np.float32), want.astype(np.float32)
+        # each side rounds an fp32 sum to fp16: two units in the last place of the largest value
+        assert np.abs(got - want).max() <= 2 * 2.0 ** -11 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("nq,nkv,hd", [(8, 8, 64), (32, 8, 128), (16, 2, 64), (6, 2, 128)])
 @pytest.mark.parametrize("m,base,window,sinks", [(17, 0, 0, False), (33, 15, 0, True), (64, 200, 24, False), (130, 1000, 128, True),
                                                  (70, 3001, 0, True), (300, 5, 40, False)])

@@ -8,15 +8,21 @@
 // LDS carries the weights only: 4 KiB read per wave and 16-K step against 8 matrix instructions of 32 cycles.  Two workgroups
 // share a compute unit: while one waits at its barrier or unpacks, the other multiplies.
 //
-// No operand is rounded.  What is multiplied are
+// What is multiplied are the stored values themselves, in operands that hold all of their bits:
 //   Q4_K / Q5_K   sc_j * q, an integer below 2048.  The superblock's d is the unit its sums are counted in: the accumulator is
 //                 multiplied by (unit before) / d when the walk enters a chunk.  At the chunk's end the unit becomes -dmin and
 //                 one more matrix instruction adds the sub-block sums times the integers m_j: two multiplies per element and
 //                 256 K in all, and no second accumulator
 //   Q6_K          (level - 32) * 16 (sc >> 4) and (level - 32) * (sc & 15), two exact integer operands; units as above
-//   Q8_0          q * d split into an fp16 and what it leaves over, both exact
-//   bf16, MXFP4   the value itself, times the power of two that brings the row's largest value to the top of fp16's range
-// (the last three: row_scale; a value 2^35 below its row's largest would begin to lose bits, where fp32 sums keep 24).
+//   Q8_0          q * d split into an fp16 and what it leaves over
+//   bf16, MXFP4   the value, in fp16
+// the last three times the power of two that brings the row's largest value to the top of fp16's range.  That is taken while
+// every value of the row is a normal fp16 then (below, bits fall off, and before that the matrix instructions' sums grow coarser:
+// they align products by the exponent fields): Q8_0 scales within 2^21 of the row's largest (smaller ones than 2^-24 there are
+// not, so a row of weights below 16 always is), MXFP4 block scales within 2^25, bf16 values within 2^29.  k_row_scale looks at
+// every row.  Tiles with another row of bf16 are multiplied as bf16 by activations split into two bf16 terms, at half the rate (of
+// rows of 4096 normally distributed values one in about 80 000); a model with one in Q8_0 or MXFP4 takes the 16- and 64-row
+// passes (prompt_supported).
 //
 // Bound by the matrix pipes: the gate/up product of 2048 rows (28672 x 4096 Q4_K, silu epilogue included) takes 489 us = 983
 // TFLOP/s on an MI355X, where a library product of 8192^3 fp16 values reaches 1164; 64 rows at a time (k_gemm_wide) the same
@@ -26,6 +32,7 @@
 // weights of a block come into that XCD's L2 once, and the activations are shared by the blocks in flight.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "prompt.h"
 
@@ -35,6 +42,7 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -313,6 +321,29 @@ struct PromptBf {
     }
 };
 
+// ... and as it is stored, for tiles with a row that fp16 cannot hold
+struct PromptBfStored : PromptBf {
+    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
+                                                  int lane) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) put_piece(buf, 2 * part + (i >> 1), i & 1, t64, lane, r.q[i]);
+    }
+};
+// what a launch over a bf16 matrix with such tiles is compiled for: each workgroup takes the form its two tiles allow
+struct PromptBfEither : PromptBf {};
+
+// Eight fp16 values as two bf16 terms, both exact: the upper eight bits and the rest
+__device__ __forceinline__ void split_bf16(u32x4 v, u32x4& hi, u32x4& lo) {
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const float f0 = half_lo(v[w]), f1 = half_hi(v[w]);
+        const uint32_t b0 = __float_as_uint(f0) & 0xFFFF0000u, b1 = __float_as_uint(f1) & 0xFFFF0000u;
+        const uint32_t r0 = __float_as_uint(f0 - __uint_as_float(b0)), r1 = __float_as_uint(f1 - __uint_as_float(b1));
+        hi[w] = (b0 >> 16) | b1;
+        lo[w] = (r0 >> 16) | (r1 & 0xFFFF0000u);
+    }
+}
+
 __device__ __forceinline__ float silu_prompt(float x) { return x / (1.0f + __expf(-x)); }
 // silu(gate) * up, or with alpha > 0 the clamped form (moe_gguf.metal:528-556)
 __device__ __forceinline__ float gated(float gate, float up, float alpha, float limit) {
@@ -348,7 +379,8 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
     const size_t rbs = (size_t)g.a_k16 * 1024;
     const int rb0 = (row0 >> 5) + wm * 2;
     const uint8_t* const ap = g.a + (size_t)rb0 * rbs + lane * 16;
-    const float rs = F::UNITS ? 1.0f : g.rs[tile * 64 + lane];
+    constexpr bool STORED = std::is_same<F, PromptBfStored>::value;
+    const float rs = F::UNITS || STORED ? 1.0f : g.rs[tile * 64 + lane];
     Bits bits{0x64006400u, 0x54005400u};
     asm volatile("" : "+v"(bits.k6400), "+v"(bits.k5400));
 
@@ -422,6 +454,19 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
                         u32x4 b[NT];
 #pragma unroll
                         for (int j = 0; j < NT; j++) b[j] = *(const u32x4*)(cur + (((term * KS + 2 * grp + q) * 4 + wn * NT + j) * 64 + lane) * 16);
+                        if constexpr (STORED) {
+#pragma unroll
+                            for (int t = 0; t < 2; t++) {
+                                u32x4 hi, lo;
+                                split_bf16(a[grp & 1][q][t], hi, lo);
+#pragma unroll
+                                for (int j = 0; j < NT; j++) {
+                                    acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, b[j]), acc[t][j], 0, 0, 0);
+                                    acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, lo), __builtin_bit_cast(bf16x8, b[j]), acc[t][j], 0, 0, 0);
+                                }
+                            }
+                            continue;
+                        }
 #pragma unroll
                         for (int j = 0; j < NT; j++)
 #pragma unroll
@@ -564,6 +609,16 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
         row0 = t.first;
         rows = t.cnt;
         expert = t.expert;
+    }
+    if constexpr (std::is_same<F, PromptBfEither>::value) {
+        const float* const rs = g.rs + (size_t)expert * g.n_tiles * 64 + (threadIdx.x & 63);
+        const bool unfit = rs[2 * nb * 64] == 0.0f || rs[min(2 * nb + 1, g.n_tiles - 1) * 64] == 0.0f;
+        if (__builtin_amdgcn_ballot_w64(unfit) != 0) {  // (the same for all four waves)
+            if (rows > 128) prompt_tile<PromptBfStored, 1, EPI>(g, lds, split, nb, row0, rows, expert);
+            else if (rows > 64) prompt_tile<PromptBfStored, 2, EPI>(g, lds, split, nb, row0, rows, expert);
+            else prompt_tile<PromptBfStored, 4, EPI>(g, lds, split, nb, row0, rows, expert);
+            return;
+        }
     }
     if (rows > 128) prompt_tile<F, 1, EPI>(g, lds, split, nb, row0, rows, expert);
     else if (rows > 64) prompt_tile<F, 2, EPI>(g, lds, split, nb, row0, rows, expert);
@@ -729,37 +784,57 @@ __global__ __launch_bounds__(256, 3) void k_prompt_experts_narrow(PromptGemmArgs
 
 // ---- row factors ----------------------------------------------------------------------------------------------------------
 // The power of two that brings the largest magnitude of a row near the top of fp16's range: 2^7 for a Q8_0 scale (its product
-// with a code stays below 2^15), 2^12 for an MXFP4 block scale (times 6), 2^14 for a bf16 value.  One wave per tile.
-__global__ __launch_bounds__(64) void k_row_scale(const uint8_t* __restrict__ tiles, int fmt, int kchunks, float* __restrict__ rs) {
+// with a code stays below 2^15), 2^12 for an MXFP4 block scale (times 6), 2^15 for a bf16 value (65280 at most).  Blocks whose
+// codes are all zero say nothing, whatever their scale.  0 for a row with a non-zero value (Q8_0: scale) that is below the normal
+// fp16 range then, or an infinity or a NaN; `unfit` counts those.  One wave per tile.
+__global__ __launch_bounds__(64) void k_row_scale(const uint8_t* __restrict__ tiles, int fmt, int kchunks, float* __restrict__ rs, int32_t* unfit) {
     const int lane = threadIdx.x, tile = blockIdx.x;
     const int tb = fmt == FMT_BF16 ? 8192 : 8704;
     const uint8_t* t = tiles + (size_t)tile * kchunks * tb;
-    int e = -1000;  // exponent of the largest magnitude
+    int e = -1000, low = 1000;  // exponents of the largest and the smallest magnitude
+    bool finite = true;
     for (int c = 0; c < kchunks; c++, t += tb) {
+        u32x4 q[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) q[u] = ((const u32x4*)t)[u * 64 + lane];
         if (fmt == FMT_Q80) {
+#pragma unroll
             for (int j = 0; j < 4; j++) {
+                const u32x4 any = q[2 * j] | q[2 * j + 1];
                 const float d = fabsf((float)*(const _Float16*)(t + 8192 + lane * 8 + 2 * j));
-                if (d > 0.f && d < INFINITY) e = max(e, ilogbf(d));
+                finite &= d < INFINITY;
+                if (d == 0.f || !(d < INFINITY) || (any.x | any.y | any.z | any.w) == 0) continue;
+                e = max(e, ilogbf(d));
+                low = min(low, ilogbf(d));
             }
         } else if (fmt == FMT_MX4) {
+#pragma unroll
             for (int j = 0; j < 8; j++) {
                 const int b = t[8192 + lane * 8 + j];
-                if (b < 255) e = max(e, b - 127);
+                finite &= b < 255;
+                if (((q[j].x | q[j].y | q[j].z | q[j].w) & 0x77777777u) == 0) continue;
+                e = max(e, b - 127);
+                low = min(low, b - 128);  // (half a scale)
             }
         } else {
-            for (int u = 0; u < 8; u++) {
-                const u32x4 q = ((const u32x4*)t)[u * 64 + lane];
-                for (int w = 0; w < 4; w++) {
-                    const int lo = (int)((q[w] >> 7) & 0xFF), hi = (int)((q[w] >> 23) & 0xFF);  // bf16 exponents
-                    if (lo && lo < 255) e = max(e, lo - 127);
-                    if (hi && hi < 255) e = max(e, hi - 127);
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int w = 0; w < 8; w++) {
+                    const int v = (int)(q[u][w >> 1] >> (16 * (w & 1))) & 0x7FFF, exponent = v >> 7;
+                    if (v == 0) continue;
+                    finite &= exponent < 255;
+                    const int at = exponent ? exponent - 127 : -102 - __clz(v);  // (subnormals: v * 2^-133)
+                    e = max(e, at);
+                    low = min(low, at);
                 }
-            }
         }
     }
-    const int top = fmt == FMT_Q80 ? 7 : fmt == FMT_MX4 ? 12 : 14;
+    const int top = fmt == FMT_Q80 ? 7 : fmt == FMT_MX4 ? 12 : 15;
     const int s = e == -1000 ? 0 : min(max(top - e, -126), 126);
-    rs[tile * 64 + lane] = __uint_as_float((uint32_t)(s + 127) << 23);
+    const bool fits = finite && low + s >= -14;
+    rs[tile * 64 + lane] = fits ? __uint_as_float((uint32_t)(s + 127) << 23) : 0.0f;
+    if (!fits) atomicAdd(unfit, 1);
 }
 
 template <class F, int EPI>
@@ -790,11 +865,20 @@ int row_block(int m) { return m > 128 ? 256 : m > 64 ? 128 : 64; }
 
 bool prompt_fmt_has_sums(int fmt) { return fmt == FMT_Q4K || fmt == FMT_Q5K; }
 
-int launch_row_scale(hipStream_t s, const TiledW& w, float* rs) {
-    hipLaunchKernelGGL(k_row_scale, dim3(w.n_tiles), dim3(64), 0, s, w.tiles, w.fmt, w.kchunks, rs);
+int make_row_scale(hipStream_t s, TiledW& w) {
+    const size_t n = (size_t)w.n_tiles * TILE_ROWS;
+    int32_t* const unfit = (int32_t*)(w.row_scale + n);
+    int32_t count = 0;
+    TSV_HIP(hipMemsetAsync(unfit, 0, 4, s));
+    hipLaunchKernelGGL(k_row_scale, dim3(w.n_tiles), dim3(64), 0, s, w.tiles, w.fmt, w.kchunks, w.row_scale, unfit);
     TSV_HIP(hipGetLastError());
+    TSV_HIP(hipMemcpyAsync(&count, unfit, 4, hipMemcpyDeviceToHost, s));
+    TSV_HIP(hipStreamSynchronize(s));
+    w.rows_unfit = count;
     return TSV_OK;
 }
+
+bool prompt_holds(const TiledW& w) { return !w.rows_unfit || w.fmt == FMT_BF16; }
 
 int prompt_splits(const TiledW& w, int m) {
     const int bm = row_block(m), tiles = (m + bm - 1) / bm * ((w.n_tiles + 1) / 2);
@@ -803,21 +887,24 @@ int prompt_splits(const TiledW& w, int m) {
     return (w.kchunks + per - 1) / per;
 }
 
-static int launch_any(hipStream_t s, int fmt, PromptGemmArgs& g, int epi) {
+static int launch_any(hipStream_t s, const TiledW& w, PromptGemmArgs& g, int epi) {
+    const int fmt = w.fmt;
     return fmt == FMT_Q4K    ? launch_f<PromptQ45<false>>(s, g, epi)
            : fmt == FMT_Q5K  ? launch_f<PromptQ45<true>>(s, g, epi)
            : fmt == FMT_Q6K  ? launch_f<PromptQ6>(s, g, epi)
            : fmt == FMT_Q80  ? launch_f<PromptQ8>(s, g, epi)
-           : fmt == FMT_BF16 ? launch_f<PromptBf>(s, g, epi)
-                             : launch_f<PromptMx>(s, g, epi);
+           : fmt == FMT_MX4  ? launch_f<PromptMx>(s, g, epi)
+           : w.rows_unfit    ? launch_f<PromptBfEither>(s, g, epi)
+                             : launch_f<PromptBf>(s, g, epi);
 }
 
 int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int m, int splits, int epi,
                        int ldo, int n_valid) {
     if (m < 1 || (epi != EPI_PARTIAL && epi != EPI_SILU) || (epi == EPI_SILU && w.n_rows % 64) || splits < 1 || splits > 8 ||
         (epi == EPI_SILU && splits != 1) || (prompt_fmt_has_sums(w.fmt) && !asum) ||
+        !prompt_holds(w) ||
         (!w.row_scale && (w.fmt == FMT_Q80 || w.fmt == FMT_BF16 || w.fmt == FMT_MX4))) {
-        set_error("prompt matmul: bad argument");
+        set_error("prompt matmul: bad argument, or a weight row that spans more than fp16 operands hold");
         return TSV_ERR_INVALID;
     }
     PromptGemmArgs g{};
@@ -842,14 +929,15 @@ int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void
     g.n_valid = epi == EPI_SILU ? w.n_rows / 2 : n_valid;
     g.out_k16 = prompt_k16(w.n_rows / 2);
     g.bm = row_block(m);
-    return launch_any(s, w.fmt, g, epi);
+    return launch_any(s, w, g, epi);
 }
 
 int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int epi, int ldo,
                           const PromptExperts& x) {
     if ((epi != EPI_PARTIAL && epi != EPI_SILU) || x.n_experts < 1 || w.n_tiles % x.n_experts || (prompt_fmt_has_sums(w.fmt) && !asum) ||
+        !prompt_holds(w) ||
         (!w.row_scale && (w.fmt == FMT_Q80 || w.fmt == FMT_BF16 || w.fmt == FMT_MX4)) || (x.bm != 64 && x.bm != 128 && x.bm != 256)) {
-        set_error("prompt experts: bad argument");
+        set_error("prompt experts: bad argument, or a weight row that spans more than fp16 operands hold");
         return TSV_ERR_INVALID;
     }
     PromptGemmArgs g{};
@@ -884,7 +972,7 @@ int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const v
         return TSV_OK;
     }
     g.bm = x.bm;
-    return launch_any(s, w.fmt, g, epi);
+    return launch_any(s, w, g, epi);
 }
 
 }  // namespace tsv

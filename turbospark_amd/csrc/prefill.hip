@@ -10,7 +10,9 @@ namespace tsv {
 bool prompt_supported(const tsv_ctx* c) {
     if (c->mtp.on) return false;
     for (const LayerW& L : c->layers)
-        if (L.cap < c->ctx_alloc || L.tq.k_bits || (L.n_experts && c->moe_fp4_terms)) return false;
+        if (L.cap < c->ctx_alloc || L.tq.k_bits || (L.n_experts && c->moe_fp4_terms) || !prompt_holds(L.qkv) || !prompt_holds(L.v_only) ||
+            !prompt_holds(L.wo) || !prompt_holds(L.gate_up) || !prompt_holds(L.down) || !prompt_holds(L.router))
+            return false;
     return true;
 }
 

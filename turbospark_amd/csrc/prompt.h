@@ -85,8 +85,12 @@ int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void
 int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int epi, int ldo,
                           const PromptExperts& x);
 int prompt_splits(const TiledW& w, int m);
-// the power-of-two factors of a tiled matrix's rows, n_tiles * 64 floats (Q8_0, bf16, MXFP4)
-int launch_row_scale(hipStream_t s, const TiledW& w, float* rs);
+// Q8_0, bf16, MXFP4: fills w.row_scale (prompt_row_scales floats), the power-of-two factors of the matrix's rows, and w.rows_unfit;
+// waits for the stream
+inline size_t prompt_row_scales(const TiledW& w) { return (size_t)w.n_tiles * TILE_ROWS + 1; }
+int make_row_scale(hipStream_t s, TiledW& w);
+// whether the prompt matmuls have operands for all bits of the matrix
+bool prompt_holds(const TiledW& w);
 bool prompt_fmt_has_sums(int fmt);
 
 // residual rows x [n][hidden] += the partial sums of the matmul before (PromptGemmArgs::out); then, with w, their RMSNorm, as

@@ -148,7 +148,7 @@ int make_tiled(tsv_ctx* c, Stager& st, const tsv_tensor* const* parts, int n_par
         row_off += rows;
     }
     if (fmt == FMT_Q80 || fmt == FMT_BF16 || fmt == FMT_MX4) {  // what the prompt matmuls scale the rows by
-        if ((rc = dev_alloc(c, &out->row_scale, (size_t)out->n_tiles * TILE_ROWS * 4)) || (rc = launch_row_scale(c->stream, *out, out->row_scale))) return rc;
+        if ((rc = dev_alloc(c, &out->row_scale, prompt_row_scales(*out) * 4)) || (rc = make_row_scale(c->stream, *out))) return rc;
     }
     return TSV_OK;
 }

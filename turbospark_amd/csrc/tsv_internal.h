@@ -76,6 +76,7 @@ struct TiledW {
     int k = 0;
     size_t bytes = 0;
     float* row_scale = nullptr;  // device, n_tiles * 64: what the prompt matmuls multiply a row by (gemm_prompt.hip); Q8_0, bf16, MXFP4
+    int rows_unfit = 0;          // rows of those that fp16 operands cannot hold exactly (factor 0)
 };
 
 inline int fmt_chunk_elems(int fmt) { return fmt == FMT_Q80 ? 128 : fmt == FMT_BF16 ? 64 : 256; }
