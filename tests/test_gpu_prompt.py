@@ -144,6 +144,7 @@ def test_a_model_of_rows_that_fp16_cannot_hold_prompts_as_before(name):
     prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
     for eng in (fast, slow):
         eng.prefill(prompt, 0, want_logits=False)
+    assert _buffers(fast)[2] == (0 if name == "tiny_q8_0" else 1) and _buffers(slow)[2] == 0
     for got, want in zip(fast.read_kv(0, 0, n), slow.read_kv(0, 0, n)):
         got, want = got.astype(np.float32), want.astype(np.float32)
         # each side rounds an fp32 sum to fp16: two units in the last place of the largest value
@@ -250,24 +251,61 @@ def test_routed_prompts_give_every_row_its_experts(name, n):
         assert far.sum() <= max(1, n // 50), np.flatnonzero(far)
 
 
-@pytest.mark.parametrize("name,n,limit", [("small_q4_k", 300, 0), ("moe_small", 130, 1 << 20), ("small_q4_k", 64, 3 << 20)])
-def test_a_device_without_room_for_prompt_buffers_takes_the_64_row_passes(name, n, limit):
-    """The buffers refused at the first and at a later allocation: the same call succeeds, in the passes the handle has buffers
-    for, and takes the large passes again once there is room."""
+def _buffers(eng):
+    """(rows of the longest prompt pass, bytes held, prompt passes so far)"""
+    import ctypes as C
+    from turbospark_amd import ffi
+    rows, bytes_, passes = C.c_int32(), C.c_int64(), C.c_int64()
+    ffi.check(ffi.lib().tsv_prompt_buffers(eng._h, C.byref(rows), C.byref(bytes_), C.byref(passes)))
+    return rows.value, bytes_.value, passes.value
+
+
+# the limits leave no prompt pass at all, or one of 256 rows where the context asks for 512
+@pytest.mark.parametrize("name,n,limit,most,passes", [("small_q4_k", 300, 0, 0, 0), ("moe_small", 130, 1 << 20, 0, 0), ("small_q4_k", 64, 3 << 20, 0, 0),
+                                                      ("small_q4_k", 300, "half", 256, 2), ("moe_small", 300, "half", 256, 2)])
+def test_a_device_without_room_for_prompt_buffers_takes_smaller_passes(name, n, limit, most, passes):
+    """The same call succeeds, in the passes the handle has buffers for, and takes the large passes again once there is room."""
     import turbospark_amd as ts
     from turbospark_amd import ffi, synth
     cfg = dict(synth.CONFIGS[name], max_context=n + 32)
     eng = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=9))
+    whole, held, _ = _buffers(eng)
+    assert whole == -(-(n + 32) // 256) * 256 and held > 0
     prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
     kv = []
-    for bytes_ in (limit, limit, 1 << 40):
+    for bytes_, rows, count in ((limit, most, passes), (limit, most, passes), (1 << 40, whole, 1)):
         eng.reset()
-        ffi.check(ffi.lib().tsv_limit_prompt_buffers(eng._h, bytes_))
+        ffi.check(ffi.lib().tsv_limit_prompt_buffers(eng._h, held - 1 if bytes_ == "half" else bytes_))
+        before = _buffers(eng)
         eng.prefill(prompt, 0, want_logits=False)
-        assert eng.position == n
+        after = _buffers(eng)
+        assert eng.position == n and after[:2] == (rows, held) and after[2] - before[2] == count
         kv.append(eng.read_kv(0, 0, n))
     for (a, b, c) in zip(*kv):          # the first layer's rows: sums of the same products
         a, b, c = (t.astype(np.float32) for t in (a, b, c))
         assert (a == b).all()
         # each side rounds an fp32 sum of about sqrt(K) roundings to fp16: two units in the last place of the largest value
         assert np.abs(a - c).max() <= 2 * 2.0 ** -11 * np.abs(a).max()
+
+
+@pytest.mark.parametrize("name", ["small_q4_k", "moe_small"])
+def test_prompts_of_any_length_allocate_nothing(name):
+    """A handle's buffers come with it: the device's free memory is the same before and after prompts that grow."""
+    import ctypes as C
+    import turbospark_amd as ts
+    from turbospark_amd import hip, synth
+
+    def room():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.rt().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    cfg = dict(synth.CONFIGS[name], max_context=2300)
+    eng = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=9))
+    assert _buffers(eng)[0] == 2048
+    eng.prefill(np.zeros(20, np.int32), 0, want_logits=False)     # code objects, the runtime's own first use
+    free = room()
+    for n in (100, 700, 2200):
+        eng.reset()
+        eng.prefill(np.zeros(n, np.int32), 0, want_logits=False)
+        assert room() == free, n

@@ -12,6 +12,8 @@
 
 namespace tsv {
 
+struct PromptTile;  // prompt.h
+
 struct LayerW {
     // the fused q/k/v projection; when the value projection has a format of its own (Q4_K_M files
     // keep attn_v in Q6_K) `qkv` holds q and k only and `v_only` the rest, written to the same
@@ -96,16 +98,17 @@ struct tsv_ctx {
         size_t frag_e_sub = 0;
         float* moe_out = nullptr;
     } wide;
-    // prompt passes (prefill.hip): buffers for `rows` rows, allocated at the first pass and grown to the largest one asked
-    // for (PROMPT_ROWS at most); freed with the handle
+    // prompt passes (prefill.hip): buffers for `rows` rows, one allocation made at open and freed with the handle
     struct Prompt {
         bool ok = false;
-        int rows = 0;
+        int rows = 0, most = 0;             // what the buffers hold; rows of the longest pass taken (tsv_limit_prompt_buffers)
+        uint8_t* arena = nullptr;
+        size_t bytes = 0;
+        int64_t passes = 0;                 // run so far
         float* x = nullptr;                 // residual rows
         uint8_t *a_h = nullptr, *a_q = nullptr, *a_f = nullptr;  // activations: K = hidden, q width, ffn
         uint8_t *s_h = nullptr, *s_q = nullptr, *s_f = nullptr;  // their sub-block sums
         float* partial = nullptr;
-        size_t partial_floats = 0;
         uint16_t* q16 = nullptr;
         float2* cs = nullptr;
         int32_t* ids = nullptr;
@@ -114,13 +117,10 @@ struct tsv_ctx {
         // the pairs' activations before and after gate / up with their sums, the down outputs by slot
         float* route_w = nullptr;
         int32_t *route_sel = nullptr, *pair = nullptr, *n_tiles = nullptr;
-        void* tiles = nullptr;
+        PromptTile* tiles = nullptr;
         uint16_t* rows16 = nullptr;
         uint8_t *a_s = nullptr, *a_e = nullptr, *s_e = nullptr, *s_s = nullptr;
         float* moe_out = nullptr;
-        std::vector<void*> allocs;
-        size_t held = 0;
-        size_t limit = SIZE_MAX;  // test hook (tsv_limit_prompt_buffers): most bytes the buffers may take
     } prompt;
     bool route_forced_set = false;  // tsv_force_route holds selections: prompt passes stay at sixteen rows
     uint16_t* q16 = nullptr;
@@ -243,10 +243,10 @@ int stage_params(tsv_ctx* c, const VerifyParams* vp, int n, VerifyParams* dev);
 // PROMPT_ROWS) at the cursor.  finish: the rows' last residual add as well, left in prompt.x and, the last (n - 1) % 16 + 1
 // rows, in x; logits: those rows' logits too.
 bool prompt_supported(const tsv_ctx* c);
-// prompt_reserve: buffers for passes of n rows, or none at all where the device has no room for them.
-int prompt_reserve(tsv_ctx* c, int n);
+// prompt_open: the handle's buffers.  prompt_limit: passes of at most the rows whose buffers fit in `bytes`, 0: no such passes.
+int prompt_open(tsv_ctx* c);
+void prompt_limit(tsv_ctx* c, size_t bytes);
 int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits);
-void prompt_free(tsv_ctx* c);
 // One verify pass: everything enqueued on the handle's stream, no synchronisation; then the optional copy of the rows' logits.
 int enqueue_verify(tsv_ctx* c, const int32_t* feed, const int32_t* parent, int m, int64_t base);
 int finish_verify(tsv_ctx* c, int m, uint16_t* logits_out);

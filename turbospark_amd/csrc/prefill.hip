@@ -2,6 +2,8 @@
 // the chunked prefill runner; families/llama/prefill.rs).  A pass takes up to PROMPT_ROWS rows, so that a matmul reads its
 // weights once for all of them and is bound by the matrix pipes; everything between the matmuls runs over all rows at once
 // (prompt.hip).  Rows are cached before any of them attends, as in the reference's batched prefill.
+#include <type_traits>
+
 #include "ctx.h"
 #include "prompt.h"
 
@@ -16,74 +18,95 @@ bool prompt_supported(const tsv_ctx* c) {
     return true;
 }
 
-void prompt_free(tsv_ctx* c) {
-    for (void* p : c->prompt.allocs) (void)hipFree(p);
-    c->prompt.allocs.clear();
-    c->prompt.rows = 0;
-    c->prompt.held = 0;
-}
-
 namespace {
 
-template <class T>
-int prompt_alloc(tsv_ctx* c, T** p, size_t bytes, bool zero) {
-    void* q = nullptr;
-    if (c->prompt.held + bytes > c->prompt.limit) {
-        set_error("prefill: buffers of a prompt pass past the limit of tsv_limit_prompt_buffers");
-        return TSV_ERR_DEVICE;
-    }
-    TSV_HIP(hipMalloc(&q, bytes));
-    c->prompt.allocs.push_back(q);
-    c->prompt.held += bytes;
-    if (zero) TSV_HIP(hipMemsetAsync(q, 0, bytes, c->stream));
-    *p = (T*)q;
-    return TSV_OK;
-}
-
-// Buffers for n rows.  The activations are cleared once: the K padding behind a width that is not whole 256s has to stay zero,
-// and rows past the last one have to hold finite values.
-int reserve_rows(tsv_ctx* c, int n) {
+// The buffers of passes of up to `rows` rows (a multiple of 256) one after the other from `at` on: sets the handle's pointers,
+// or with `at` null counts only.  Returns the bytes in all.
+size_t lay_out(tsv_ctx* c, int rows, uint8_t* at) {
     tsv_ctx::Prompt& w = c->prompt;
-    const int rows = n <= 256 ? 256 : n <= 1024 ? 1024 : PROMPT_ROWS;
-    if (w.rows) {
-        TSV_HIP(hipStreamSynchronize(c->stream));
-        prompt_free(c);
-    }
+    size_t used = 0;
+    auto put = [&](auto*& p, size_t bytes) {
+        if (at) p = (std::remove_reference_t<decltype(p)>)(at + used);
+        used += (bytes + 255) & ~(size_t)255;
+    };
     const int qd = c->nq * c->hd;
     size_t width = (size_t)qd + 2 * c->nkv * c->hd;
     for (const LayerW& L : c->layers)
         width = std::max(width, (size_t)(L.n_experts ? std::max(c->hidden, L.n_experts) : c->hidden));
     // one partial sum per row and column, or as many as fill the chip: at most 512 tiles of 256 x 128 (prompt_splits), by half more
     // where q and k are split by themselves and the value columns come on top
-    w.partial_floats = std::max((size_t)rows * width, std::min((size_t)8 * rows * width, (size_t)512 * 256 * 128 * 3 / 2));
-    int rc;
-    if ((rc = prompt_alloc(c, &w.x, (size_t)rows * c->hidden * 4, false)) || (rc = prompt_alloc(c, &w.a_h, prompt_a_bytes(rows, c->hidden), true)) ||
-        (rc = prompt_alloc(c, &w.s_h, prompt_sum_bytes(rows, c->hidden), true)) || (rc = prompt_alloc(c, &w.a_q, prompt_a_bytes(rows, qd), true)) ||
-        (rc = prompt_alloc(c, &w.s_q, prompt_sum_bytes(rows, qd), true)) || (rc = prompt_alloc(c, &w.a_f, prompt_a_bytes(rows, c->ffn), true)) ||
-        (rc = prompt_alloc(c, &w.s_f, prompt_sum_bytes(rows, c->ffn), true)) || (rc = prompt_alloc(c, &w.partial, w.partial_floats * 4, false)) ||
-        (rc = prompt_alloc(c, &w.q16, (size_t)rows * qd * 2, false)) || (rc = prompt_alloc(c, &w.cs, (size_t)rows * (c->hd / 2) * sizeof(float2), false)) ||
-        (rc = prompt_alloc(c, &w.ids, (size_t)rows * 4, false)) || (rc = prompt_alloc(c, &w.part_o, (size_t)512 * 128 * c->hd * 4, false)) ||
-        (rc = prompt_alloc(c, &w.part_ml, (size_t)512 * 128 * 2 * 4, false)))
-        return rc;
+    const size_t partial_floats = std::max((size_t)rows * width, std::min((size_t)8 * rows * width, (size_t)512 * 256 * 128 * 3 / 2));
+    put(w.x, (size_t)rows * c->hidden * 4);
+    put(w.a_h, prompt_a_bytes(rows, c->hidden));
+    put(w.s_h, prompt_sum_bytes(rows, c->hidden));
+    put(w.a_q, prompt_a_bytes(rows, qd));
+    put(w.s_q, prompt_sum_bytes(rows, qd));
+    put(w.a_f, prompt_a_bytes(rows, c->ffn));
+    put(w.s_f, prompt_sum_bytes(rows, c->ffn));
+    put(w.partial, partial_floats * 4);
+    put(w.q16, (size_t)rows * qd * 2);
+    put(w.cs, (size_t)rows * (c->hd / 2) * sizeof(float2));
+    put(w.ids, (size_t)rows * 4);
+    put(w.part_o, (size_t)512 * 128 * c->hd * 4);
+    put(w.part_ml, (size_t)512 * 128 * 2 * 4);
     int sorted = 0, tiles = 0;
     for (const LayerW& L : c->layers)
         if (L.n_experts) {
             sorted = std::max(sorted, prompt_padded(prompt_sorted_rows(rows, L.top_k, L.n_experts)) + 256);  // (a tile may reach past its run)
             tiles = std::max(tiles, prompt_max_tiles(rows, L.top_k, L.n_experts, 64));
         }
-    if (sorted &&
-        ((rc = prompt_alloc(c, &w.route_w, (size_t)rows * 8 * 4, true)) || (rc = prompt_alloc(c, &w.route_sel, (size_t)rows * 8 * 4, true)) ||
-         (rc = prompt_alloc(c, &w.pair, (size_t)sorted * 4, false)) || (rc = prompt_alloc(c, &w.n_tiles, 4, false)) ||
-         (rc = prompt_alloc(c, &w.tiles, (size_t)tiles * sizeof(PromptTile), false)) ||
-         (rc = prompt_alloc(c, &w.rows16, (size_t)rows * prompt_k16(c->hidden) * 32, true)) ||
-         (rc = prompt_alloc(c, &w.a_s, prompt_a_bytes(sorted, c->hidden), true)) ||
-         (rc = prompt_alloc(c, &w.s_s, prompt_sum_bytes(sorted, c->hidden), true)) || (rc = prompt_alloc(c, &w.a_e, prompt_a_bytes(sorted, c->ffn), true)) ||
-         (rc = prompt_alloc(c, &w.s_e, prompt_sum_bytes(sorted, c->ffn), true)) ||
-         (rc = prompt_alloc(c, &w.moe_out, (size_t)rows * 8 * c->hidden * 4, false))))
-        return rc;
-    w.rows = rows;
+    if (sorted) {
+        put(w.route_w, (size_t)rows * 8 * 4);
+        put(w.route_sel, (size_t)rows * 8 * 4);
+        put(w.pair, (size_t)sorted * 4);
+        put(w.n_tiles, 4);
+        put(w.tiles, (size_t)tiles * sizeof(PromptTile));
+        put(w.rows16, (size_t)rows * prompt_k16(c->hidden) * 32);
+        put(w.a_s, prompt_a_bytes(sorted, c->hidden));
+        put(w.s_s, prompt_sum_bytes(sorted, c->hidden));
+        put(w.a_e, prompt_a_bytes(sorted, c->ffn));
+        put(w.s_e, prompt_sum_bytes(sorted, c->ffn));
+        put(w.moe_out, (size_t)rows * 8 * c->hidden * 4);
+    }
+    return used;
+}
+
+int fewer(int rows) { return rows > 256 ? (rows / 2 + 255) / 256 * 256 : 0; }
+
+}  // namespace
+
+// One allocation with the handle, for the longest pass its context allows; where the device has no room for it, for half the
+// rows, and so on down to 256.  A prompt takes as many passes as that makes (64-row ones if there was no room at all), and none
+// of them allocates: an allocation in a call would stop the whole device, other handles' streams and captures with it, and takes
+// longer than a short prompt's pass (a handle's first 1500 tokens over four gpt-oss layers: 8.2 ms with allocations, 4.7 without).
+int prompt_open(tsv_ctx* c) {
+    tsv_ctx::Prompt& w = c->prompt;
+    if (c->max_context < PROMPT_MIN_ROWS) return TSV_OK;
+    for (int rows = prompt_padded(std::min(c->max_context, PROMPT_ROWS)); rows; rows = fewer(rows)) {
+        const size_t bytes = lay_out(c, rows, nullptr);
+        if (hipMalloc((void**)&w.arena, bytes) != hipSuccess) {
+            w.arena = nullptr;
+            (void)hipGetLastError();  // a refused allocation is not the next launch's error
+            continue;
+        }
+        // Cleared once: the K padding behind a width that is not whole 256s has to stay zero, and rows past a pass's last one hold
+        // finite values
+        TSV_HIP(hipMemsetAsync(w.arena, 0, bytes, c->stream));
+        TSV_HIP(hipStreamSynchronize(c->stream));
+        lay_out(c, rows, w.arena);
+        w.rows = w.most = rows;
+        w.bytes = bytes;
+        break;
+    }
     return TSV_OK;
 }
+
+void prompt_limit(tsv_ctx* c, size_t bytes) {
+    c->prompt.most = c->prompt.rows;
+    while (c->prompt.most && lay_out(c, c->prompt.most, nullptr) > bytes) c->prompt.most = fewer(c->prompt.most);
+}
+
+namespace {
 
 // one split count for a projection whose value part has a storage type of its own
 int common_splits(const TiledW& a, const TiledW& b, int n) {
@@ -135,7 +158,7 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
         ra.blocks = (n + 15) / 16;
         ra.logits_block_stride = (long)rsp * 16 * L.n_experts;
         PromptExperts x{};
-        x.routes = PromptRoutes{w.pair, (PromptTile*)w.tiles, w.n_tiles};
+        x.routes = PromptRoutes{w.pair, w.tiles, w.n_tiles};
         x.n_experts = L.n_experts;
         x.bm = prompt_expert_rows(n, L.top_k, L.n_experts);
         x.max_tiles = prompt_max_tiles(n, L.top_k, L.n_experts, x.bm);
@@ -240,17 +263,6 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
 
 }  // namespace
 
-int prompt_reserve(tsv_ctx* c, int n) {
-    if (n <= c->prompt.rows) return TSV_OK;
-    const int rc = reserve_rows(c, n);
-    if (rc) {
-        (void)hipStreamSynchronize(c->stream);  // buffers that were given may still be cleared
-        prompt_free(c);
-        (void)hipGetLastError();  // a refused allocation is not the next launch's error
-    }
-    return rc;
-}
-
 int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits) {
     if (base != c->position) {
         set_error("prefill: start position does not match the KV cursor");
@@ -260,7 +272,7 @@ int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, boo
         set_error("prefill: block would write past the KV capacity");
         return TSV_ERR_INVALID;
     }
-    if (n < PROMPT_MIN_ROWS || n > PROMPT_ROWS) {
+    if (n < PROMPT_MIN_ROWS || n > c->prompt.most) {
         set_error("prefill: rows of a prompt pass");
         return TSV_ERR_INVALID;
     }
@@ -269,8 +281,7 @@ int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, boo
             set_error("verify: token id outside the vocabulary");
             return TSV_ERR_INVALID;
         }
-    int rc = prompt_reserve(c, n);
-    if (rc) return rc;
+    int rc;
     // (from the caller's pageable memory: the runtime has taken its copy when this returns)
     TSV_HIP(hipMemcpyAsync(c->prompt.ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
     const int m = (n - 1) % 16 + 1;
@@ -281,6 +292,7 @@ int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, boo
         if ((rc = stage_params(c, &vp, 1, c->vp_dev))) return rc;
     }
     if ((rc = launch_prompt_pass(c, n, base, finish, logits))) return rc;
+    c->prompt.passes++;
     c->position = base + n;
     c->high_water = std::max(c->high_water, c->position);
     c->last_m = logits ? m : 0;

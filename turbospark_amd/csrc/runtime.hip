@@ -1377,6 +1377,7 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
     if (share) c->wide.ok = false;  // the head's rows come sixteen at a time
     const char* wide_env = getenv("TSV_WIDE_PREFILL");
     c->prompt.ok = !share && !(wide_env && wide_env[0] == '0') && prompt_supported(c);
+    if (c->prompt.ok && (rc = prompt_open(c))) return fail(rc);
     *out = c;
     return TSV_OK;
 }
@@ -1387,7 +1388,7 @@ extern "C" void tsv_close(tsv_ctx* c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
-    prompt_free(c);
+    if (c->prompt.arena) (void)hipFree(c->prompt.arena);
     if (c->hist_dev) (void)hipFree(c->hist_dev);
     if (c->vp_host) (void)hipHostFree(c->vp_host);
     if (c->ring.host) (void)hipHostFree(c->ring.host);
@@ -1535,14 +1536,12 @@ int tsv::prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0,
     const int wide_rows = 16 * WIDE_B;
     // A call of fewer than 64 tokens keeps verify-sized passes, whose rows have the bits of one-row passes whatever their
     // number: what a caller gets by feeding a few tokens one by one and at once is the same.
-    // Where the weights and the cache leave no room for a prompt pass's buffers (0.3 GB at the 8B shape) the 64-row passes do
-    // it, whose buffers came with the handle.
-    const bool by_prompt_pass = c->prompt.ok && !c->profile && !c->route_forced_set && (n > PROMPT_MIN_ROWS || (n == PROMPT_MIN_ROWS && !logits && !head)) &&
-                                prompt_reserve(c, (int)std::min<int64_t>(n, PROMPT_ROWS)) == TSV_OK;
+    const bool by_prompt_pass = c->prompt.ok && c->prompt.most && !c->profile && !c->route_forced_set &&
+                                (n > PROMPT_MIN_ROWS || (n == PROMPT_MIN_ROWS && !logits && !head));
     for (int64_t i = 0; i < n;) {
         if (by_prompt_pass) {
             // passes of equal length, a multiple of sixteen but for the last
-            const int64_t left = n - i, passes = (left + PROMPT_ROWS - 1) / PROMPT_ROWS;
+            const int64_t left = n - i, passes = (left + c->prompt.most - 1) / c->prompt.most;
             const int rows = (int)std::min(left, ((left + passes - 1) / passes + 15) / 16 * 16);
             const bool last = i + rows >= n;
             // (an attached head's next step reads the pass's last rows, whoever asked for the pass)

@@ -139,7 +139,15 @@ extern "C" int32_t tsv_force_route(tsv_ctx* c, const int32_t* sel, int32_t n_lay
 
 extern "C" int32_t tsv_limit_prompt_buffers(tsv_ctx* c, int64_t bytes) {
     TSV_NEED(c && bytes >= 0, "limit_prompt_buffers: bad argument");
-    c->prompt.limit = (size_t)bytes;
+    prompt_limit(c, (size_t)bytes);
+    return TSV_OK;
+}
+
+extern "C" int32_t tsv_prompt_buffers(const tsv_ctx* c, int32_t* rows, int64_t* bytes, int64_t* passes) {
+    TSV_NEED(c && rows && bytes && passes, "prompt_buffers: null argument");
+    *rows = c->prompt.most;
+    *bytes = (int64_t)c->prompt.bytes;
+    *passes = c->prompt.passes;
     return TSV_OK;
 }
 
