@@ -125,7 +125,8 @@ int32_t tsv_force_route(tsv_ctx* ctx, const int32_t* sel, int32_t n_layers);
 /* Prompt passes take at most the rows whose buffers fit in `bytes`, as on a device that had no more room when the
  * handle was opened (0: the prompt goes in 64-row passes); a larger value gives the rows back. */
 int32_t tsv_limit_prompt_buffers(tsv_ctx* ctx, int64_t bytes);
-/* Rows of the longest prompt pass the handle takes (0: none), the bytes its buffers hold, and the prompt passes run so far. */
+/* Rows of the longest prompt pass the handle takes (0: none), the bytes its buffers hold, and how many prompt passes
+ * (passes[0]) and 64-row passes (passes[1]) it has run so far. */
 int32_t tsv_prompt_buffers(const tsv_ctx* ctx, int32_t* rows, int64_t* bytes, int64_t* passes);
 
 #ifdef __cplusplus

@@ -445,14 +445,7 @@ def test_prompt_passes_of_64_rows_over_quantized_rows(name, kv_bits, n_prompt):
     cfg = dict(synth.CONFIGS[name], max_context=n_prompt + 48, n_layers=3)
     w = synth.make_weights(cfg, seed=11)
 
-    def engine(wide):
-        os.environ["TSV_WIDE_PREFILL"] = "1" if wide else "0"
-        try:
-            return ts.HipVerifier(cfg, w, kv_bits=kv_bits)
-        finally:
-            del os.environ["TSV_WIDE_PREFILL"]
-
-    wide, narrow = engine(True), engine(False)
+    wide, narrow = gc.engine(cfg, w, "prompt", kv_bits=kv_bits), gc.engine(cfg, w, "16", kv_bits=kv_bits)   # (quantized rows: 64 at most)
     cpu = ob.Model(cfg, w, round_kv_f16=True, threads=16, kv_bits=kv_bits)
     rng = np.random.default_rng(2)
     prompt = rng.integers(0, cfg["vocab"], n_prompt).astype(np.int32)
@@ -461,6 +454,7 @@ def test_prompt_passes_of_64_rows_over_quantized_rows(name, kv_bits, n_prompt):
     narrow.prefill(prompt, 0, want_logits=False)
     for i in range(0, n_prompt, 16):
         cpu.verify(prompt[i:i + 16], i)
+    assert gc.took(wide, "64") and gc.took(narrow, "16")
     assert wide.position == narrow.position == n_prompt
     same = []
     for layer in (0, 1):

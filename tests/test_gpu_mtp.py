@@ -72,17 +72,21 @@ def test_the_heads_logits_match_the_oracle_through_priming_steps_chained_steps_a
     assert max(errs) <= tol
 
 
-# the longer prompts go through 64-row passes, which prime the head too (Q8_0: the rotation as a kernel of its own
-# under TSV_ROPE_FUSED=0 elsewhere, here the epilogue; routed layers: the experts' members over 64 rows)
+# the longer prompts go through large passes, which prime the head too (Q8_0: the rotation as a kernel of its own
+# under TSV_ROPE_FUSED=0 elsewhere, here the epilogue; routed layers: every expert against the rows that chose it)
+@pytest.mark.parametrize("passes", ["64", "prompt"])
 @pytest.mark.parametrize("name,n", [("xcd_q4_k", 37), ("xcd_q4_k", 171), ("xcd_q8_0", 171), ("moe_small", 171)])
-def test_priming_by_the_prefill_equals_priming_token_by_token(name, n):
+def test_priming_by_the_prefill_equals_priming_token_by_token(name, n, passes):
     cfg, gpu_a, head_a = _build(name, ctx=200, oracle=False)
     _, gpu_b, head_b = _build(name, ctx=200, oracle=False)
+    if passes == "64":
+        ffi.check(ffi.lib().tsv_limit_prompt_buffers(gpu_a._h, 0))
     V = cfg["vocab"]
     prompt = np.random.default_rng(6).integers(0, V, n).astype(np.int32)
     la = head_a.prefill_chunk(prompt[:20], 0, next_token=int(prompt[20]))   # two chunks, the first names its next token
     assert head_a.position == 20
     la = head_a.prefill_chunk(prompt[20:], 20)
+    assert gc.took(gpu_a, passes if n > 100 else "16")
     for i in range(n):
         lb = gpu_b.produce(int(prompt[i]), i)
         if i + 1 < n:

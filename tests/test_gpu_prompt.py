@@ -29,6 +29,10 @@ def test_the_prompt_matmul_is_the_dequantized_product(dtype, rows, cols, m):
     for splits in (0, 1):
         got = ffi.matmul(entry, x, splits)
         assert (np.abs(got - want) <= 2e-4 * scale + 1e-9).all(), (splits, np.abs(got - want).max() / scale.max())
+        # and column by column: K / 16 sums in one chain, twice that for weights of two terms, each rounded to 2^-24 of the running
+        # size; four times that covers the min terms of Q4_K / Q5_K, larger than what they leave
+        norm = np.linalg.norm(want, axis=0)
+        assert (np.linalg.norm(got - want, axis=0) <= 4 * (cols / 16) ** 0.5 * 2.0 ** -24 * norm).all()
 
 
 def _off(entry, values, x, splits=0, column=slice(None)):
@@ -115,8 +119,6 @@ def test_mxfp4_blocks_keep_their_bits_or_the_product_is_refused(low, held):
 def test_a_model_of_rows_that_fp16_cannot_hold_prompts_as_before(name):
     """The first 32 columns of the query, key and value projections hold weights 2^30 above the others (behind a norm weight of
     zero): a Q8_0 model takes the smaller passes, a bf16 one multiplies those tiles as bf16."""
-    import os
-    import turbospark_amd as ts
     from turbospark_amd import ffi, synth
     n = 100
     cfg = dict(synth.CONFIGS[name], max_context=n + 32)
@@ -135,16 +137,11 @@ def test_a_model_of_rows_that_fp16_cannot_hold_prompts_as_before(name):
             else:
                 v.reshape(r, -1).view(np.uint16)[:, :32] = np.float32(2.0 ** 30).view(np.uint32) >> 16
             lw[key] = (dt, v, r, c)
-    fast = ts.HipVerifier(cfg, w)
-    os.environ["TSV_WIDE_PREFILL"] = "0"
-    try:
-        slow = ts.HipVerifier(cfg, w)
-    finally:
-        del os.environ["TSV_WIDE_PREFILL"]
+    fast, slow = gc.engine(cfg, w, "prompt"), gc.engine(cfg, w, "16")
     prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
     for eng in (fast, slow):
         eng.prefill(prompt, 0, want_logits=False)
-    assert _buffers(fast)[2] == (0 if name == "tiny_q8_0" else 1) and _buffers(slow)[2] == 0
+    assert gc.took(fast, "64" if name == "tiny_q8_0" else "prompt") and gc.took(slow, "16")
     for got, want in zip(fast.read_kv(0, 0, n), slow.read_kv(0, 0, n)):
         got, want = got.astype(np.float32), want.astype(np.float32)
         # each side rounds an fp32 sum to fp16: two units in the last place of the largest value
@@ -194,17 +191,11 @@ def test_prompt_attention_is_the_exact_result_rounded(nq, nkv, hd, m, base, spre
 def test_prompts_around_the_limits_of_a_pass(name, n, start):
     """Logits of the last token, what a verify pass after the prompt sees, and the rows left for tsv_accept, against passes of
     sixteen rows."""
-    import os
     import turbospark_amd as ts
     from turbospark_amd import synth
     cfg = dict(synth.CONFIGS[name], max_context=start + n + 32)
     w = synth.make_weights(cfg, seed=3)
-    fast = ts.HipVerifier(cfg, w)
-    os.environ["TSV_WIDE_PREFILL"] = "0"
-    try:
-        slow = ts.HipVerifier(cfg, w)
-    finally:
-        del os.environ["TSV_WIDE_PREFILL"]
+    fast, slow = gc.engine(cfg, w, "prompt"), gc.engine(cfg, w, "16")
     rng = np.random.default_rng(n)
     prompt = rng.integers(0, cfg["vocab"], start + n).astype(np.int32)
     feed = rng.integers(0, cfg["vocab"], 5).astype(np.int32)
@@ -218,6 +209,7 @@ def test_prompts_around_the_limits_of_a_pass(name, n, start):
         eng.reset()
         eng.prefill(prompt, 0, want_logits=False)
         out.append((last, eng.verify(feed, start + n), acc))
+    assert gc.took(fast, "prompt") and gc.took(slow, "16")
     assert gc.logit_error(out[0][0].reshape(1, -1), out[1][0].reshape(1, -1)) <= 2e-3
     assert gc.logit_error(out[0][1], out[1][1]) <= 2e-3
     assert (out[0][2].accepted, out[0][2].kv_position) == (out[1][2].accepted, out[1][2].kv_position)
@@ -230,20 +222,14 @@ def test_routed_prompts_give_every_row_its_experts(name, n):
     """The second layer's K and V rows, which the first layer's experts made, against passes of sixteen rows.  Single rows may
     differ where a last expert falls the other way (one decision in two hundred lies within the rounding of a tie); a wrong
     block edge would move a row of every expert, a tenth of all rows and more."""
-    import os
-    import turbospark_amd as ts
     from turbospark_amd import synth
     cfg = dict(synth.CONFIGS[name], max_context=n + 32)
     w = synth.make_weights(cfg, seed=5)
-    fast = ts.HipVerifier(cfg, w)
-    os.environ["TSV_WIDE_PREFILL"] = "0"
-    try:
-        slow = ts.HipVerifier(cfg, w)
-    finally:
-        del os.environ["TSV_WIDE_PREFILL"]
+    fast, slow = gc.engine(cfg, w, "prompt"), gc.engine(cfg, w, "16")
     prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
     for eng in (fast, slow):
         eng.prefill(prompt, 0, want_logits=False)
+    assert gc.took(fast, "prompt") and gc.took(slow, "16")
     for got, want in zip(fast.read_kv(1, 0, n), slow.read_kv(1, 0, n)):
         got, want = got.astype(np.float32).reshape(n, -1), want.astype(np.float32).reshape(n, -1)
         # 8 units in the last place of an fp16 value of the row's largest size: fp32 sums in another order, rounded to fp16 activations
@@ -251,13 +237,43 @@ def test_routed_prompts_give_every_row_its_experts(name, n):
         assert far.sum() <= max(1, n // 50), np.flatnonzero(far)
 
 
-def _buffers(eng):
-    """(rows of the longest prompt pass, bytes held, prompt passes so far)"""
-    import ctypes as C
-    from turbospark_amd import ffi
-    rows, bytes_, passes = C.c_int32(), C.c_int64(), C.c_int64()
-    ffi.check(ffi.lib().tsv_prompt_buffers(eng._h, C.byref(rows), C.byref(bytes_), C.byref(passes)))
-    return rows.value, bytes_.value, passes.value
+# experts in every storage type: with sums (Q4_K, Q5_K: of the gathered rows, and of what gate / up leave), without, and mixed;
+# 16 experts of which four are chosen, 18 to 94 members an expert (tiles of 64 rows) and 188 (128)
+@pytest.mark.parametrize("expert,down", [(12, 12), (13, 14), (14, 13), (8, 8), (30, 30), (12, 8), (39, 12)])
+@pytest.mark.parametrize("n", [72, 375, 750])
+def test_routed_prompts_in_every_storage_type(expert, down, n):
+    from turbospark_amd import ffi, synth
+    cfg = dict(synth.CONFIGS["moe_small"], max_context=n + 32, expert_dtype=expert)
+    w = synth.make_weights(cfg, seed=5)
+    for lw in w["layers"]:
+        lw["we_down"] = ffi.synth_tensor(down, 5, 900, 0.02, lw["we_down"][2], lw["we_down"][3])
+    fast, slow = gc.engine(cfg, w, "prompt"), gc.engine(cfg, w, "16")
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
+    for eng in (fast, slow):
+        eng.prefill(prompt, 0, want_logits=False)
+    assert gc.took(fast, "prompt") and gc.took(slow, "16")
+    for got, want in zip(fast.read_kv(1, 0, n), slow.read_kv(1, 0, n)):
+        got, want = got.astype(np.float32).reshape(n, -1), want.astype(np.float32).reshape(n, -1)
+        far = np.abs(got - want).max(1) > 8 * 2.0 ** -11 * np.abs(want).max(1)   # as above
+        assert far.sum() <= max(1, n // 50), np.flatnonzero(far)
+
+
+@pytest.mark.parametrize("dtype,n", [(12, 100), (8, 300)])
+def test_rows_wider_than_a_waves_registers(dtype, n):
+    """Hidden 4352: the norm reads such a row twice (shapes of 70B models are 8192 wide).  K and V rows of both layers against
+    passes of sixteen rows."""
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS["xcd_q4_k"], hidden=4352, n_q_heads=8, n_kv_heads=2, ffn=512, dtype=dtype, max_context=n + 32)
+    w = synth.make_weights(cfg, seed=6)
+    fast, slow = gc.engine(cfg, w, "prompt"), gc.engine(cfg, w, "16")
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
+    for eng in (fast, slow):
+        eng.prefill(prompt, 0, want_logits=False)
+    assert gc.took(fast, "prompt") and gc.took(slow, "16")
+    for layer in range(2):
+        for got, want in zip(fast.read_kv(layer, 0, n), slow.read_kv(layer, 0, n)):
+            got, want = got.astype(np.float32), want.astype(np.float32)
+            assert np.abs(got - want).max() <= 8 * 2.0 ** -11 * np.abs(want).max()   # the bound of the routed rows
 
 
 # the limits leave no prompt pass at all, or one of 256 rows where the context asks for 512
@@ -269,17 +285,18 @@ def test_a_device_without_room_for_prompt_buffers_takes_smaller_passes(name, n, 
     from turbospark_amd import ffi, synth
     cfg = dict(synth.CONFIGS[name], max_context=n + 32)
     eng = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=9))
-    whole, held, _ = _buffers(eng)
+    whole, held = gc.prompt_buffers(eng)[:2]
     assert whole == -(-(n + 32) // 256) * 256 and held > 0
     prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
     kv = []
     for bytes_, rows, count in ((limit, most, passes), (limit, most, passes), (1 << 40, whole, 1)):
         eng.reset()
         ffi.check(ffi.lib().tsv_limit_prompt_buffers(eng._h, held - 1 if bytes_ == "half" else bytes_))
-        before = _buffers(eng)
+        before = gc.prompt_buffers(eng)
         eng.prefill(prompt, 0, want_logits=False)
-        after = _buffers(eng)
+        after = gc.prompt_buffers(eng)
         assert eng.position == n and after[:2] == (rows, held) and after[2] - before[2] == count
+        assert (after[3] > before[3]) == (count == 0)
         kv.append(eng.read_kv(0, 0, n))
     for (a, b, c) in zip(*kv):          # the first layer's rows: sums of the same products
         a, b, c = (t.astype(np.float32) for t in (a, b, c))
@@ -302,7 +319,7 @@ def test_prompts_of_any_length_allocate_nothing(name):
 
     cfg = dict(synth.CONFIGS[name], max_context=2300)
     eng = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=9))
-    assert _buffers(eng)[0] == 2048
+    assert gc.prompt_buffers(eng)[0] == 2048
     eng.prefill(np.zeros(20, np.int32), 0, want_logits=False)     # code objects, the runtime's own first use
     free = room()
     for n in (100, 700, 2200):

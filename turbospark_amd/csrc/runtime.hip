@@ -898,6 +898,7 @@ int enqueue_wide_prefill(tsv_ctx* c, const int32_t* ids, int64_t base) {
     static_assert(WIDE_B <= tsv_ctx::ParamRing::PER_SLOT, "a staging slot holds a prompt pass's blocks");
     if ((rc = stage_params(c, vp, WIDE_B, c->wide.vp))) return rc;
     if ((rc = launch_wide_pass(c, base))) return rc;
+    c->wide.passes++;
     c->position = base + rows;
     c->high_water = std::max(c->high_water, c->position);
     c->last_m = 0;  // no logits on the device for tsv_accept to judge

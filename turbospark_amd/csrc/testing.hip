@@ -147,7 +147,8 @@ extern "C" int32_t tsv_prompt_buffers(const tsv_ctx* c, int32_t* rows, int64_t* 
     TSV_NEED(c && rows && bytes && passes, "prompt_buffers: null argument");
     *rows = c->prompt.most;
     *bytes = (int64_t)c->prompt.bytes;
-    *passes = c->prompt.passes;
+    passes[0] = c->prompt.passes;
+    passes[1] = c->wide.passes;
     return TSV_OK;
 }
 
