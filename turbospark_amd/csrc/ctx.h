@@ -103,6 +103,8 @@ struct tsv_ctx {
     struct Prompt {
         bool ok = false;
         int rows = 0, most = 0;             // what the buffers hold; rows of the longest pass taken (tsv_limit_prompt_buffers)
+        bool two_terms = false;             // most of the weights are Q8_0, whose prompt matmul makes two products of each
+        int full_experts = 0;               // rows that give every routed expert three on average
         uint8_t* arena = nullptr;
         size_t bytes = 0;
         int64_t passes = 0;                 // run so far
@@ -246,6 +248,9 @@ int stage_params(tsv_ctx* c, const VerifyParams* vp, int n, VerifyParams* dev);
 bool prompt_supported(const tsv_ctx* c);
 // prompt_open: the handle's buffers.  prompt_limit: passes of at most the rows whose buffers fit in `bytes`, 0: no such passes.
 int prompt_open(tsv_ctx* c);
+// prompt_pays: whether a call of n tokens at `base` is faster in prompt passes than in passes of 64 and 16 rows; tail: the last
+// rows have to come out of a pass of sixteen (their logits are wanted, or a drafter head is primed).
+bool prompt_pays(const tsv_ctx* c, int64_t n, int64_t base, bool tail);
 void prompt_limit(tsv_ctx* c, size_t bytes);
 int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits);
 // One verify pass: everything enqueued on the handle's stream, no synchronisation; then the optional copy of the rows' logits.

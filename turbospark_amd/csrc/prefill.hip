@@ -81,6 +81,15 @@ int fewer(int rows) { return rows > 256 ? (rows / 2 + 255) / 256 * 256 : 0; }
 // longer than a short prompt's pass (a handle's first 1500 tokens over four gpt-oss layers: 8.2 ms with allocations, 4.7 without).
 int prompt_open(tsv_ctx* c) {
     tsv_ctx::Prompt& w = c->prompt;
+    size_t q8 = 0, all = 0;
+    for (const LayerW& L : c->layers) {
+        if (L.n_experts) w.full_experts = std::max(w.full_experts, (3 * L.n_experts + L.top_k - 1) / L.top_k);
+        for (const TiledW* t : {&L.qkv, &L.v_only, &L.wo, &L.gate_up, &L.down}) {
+            all += t->bytes;
+            q8 += t->fmt == FMT_Q80 ? t->bytes : 0;
+        }
+    }
+    w.two_terms = 2 * q8 > all;
     if (c->max_context < PROMPT_MIN_ROWS) return TSV_OK;
     for (int rows = prompt_padded(std::min(c->max_context, PROMPT_ROWS)); rows; rows = fewer(rows)) {
         const size_t bytes = lay_out(c, rows, nullptr);
@@ -99,6 +108,26 @@ int prompt_open(tsv_ctx* c) {
         break;
     }
     return TSV_OK;
+}
+
+// Against three smaller passes and more a prompt pass is the faster one (81 rows of the 8B shape in Q4_K_M, six layers: 1118 us
+// against 1587; gpt-oss, three layers: 1470 against 1594), against a single one it is not (64 rows: 976 against 789, 1367 against
+// 962: its tiles have 128 columns, where 64 rows leave most of the chip idle).  Of two passes (65 to 80 rows, or 128 without a
+// tail) the 64-row pass and the sixteen rows behind it, or the second one, win
+//   for Q8_0 weights (8B shape, 65 / 80 / 128 rows at position 0: 799 / 882 / 1010 us, a prompt pass 945 / 948 / 974; with 16
+//   layers of 2048 486 / 530 / 612 against 580 / 583 / 613, and the further the longer the context);
+//   where routed experts have fewer than three rows on average, so that each is read for next to nothing whatever reads it
+//   (gpt-oss layers, 65 / 80 rows: 1151 / 1482 us against 1403 / 1524; the 128-expert shape of eight chosen at 65 rows, four each:
+//   788 against 743);
+//   far into a context: a prompt pass's attention takes its blocks in whole 128-pair workgroups.  Q4_K, 8B shape, 65 rows: 715
+//   against 695 us at 0, 750 / 765 at 4000, 780 / 846 at 8000; 80 rows: 799 / 701, 831 / 769, 861 / 856, and 564 / 588 (two
+//   layers) at 32 000.
+bool prompt_pays(const tsv_ctx* c, int64_t n, int64_t base, bool tail) {
+    if (n < PROMPT_MIN_ROWS || (n == PROMPT_MIN_ROWS && tail)) return false;  // (see prefill_passes)
+    if (!c->wide.ok) return true;
+    const int64_t blocks = n / 64 - (tail && n % 64 == 0), rest = n - 64 * blocks, smaller = blocks + (rest + 15) / 16;
+    if (smaller != 2) return smaller > 2;
+    return !c->prompt.two_terms && n >= c->prompt.full_experts && (n > 80 || base < 2048 * (n - 63));
 }
 
 void prompt_limit(tsv_ctx* c, size_t bytes) {

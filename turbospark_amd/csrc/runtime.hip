@@ -1537,8 +1537,7 @@ int tsv::prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0,
     const int wide_rows = 16 * WIDE_B;
     // A call of fewer than 64 tokens keeps verify-sized passes, whose rows have the bits of one-row passes whatever their
     // number: what a caller gets by feeding a few tokens one by one and at once is the same.
-    const bool by_prompt_pass = c->prompt.ok && c->prompt.most && !c->profile && !c->route_forced_set &&
-                                (n > PROMPT_MIN_ROWS || (n == PROMPT_MIN_ROWS && !logits && !head));
+    const bool by_prompt_pass = c->prompt.ok && c->prompt.most && !c->profile && !c->route_forced_set && prompt_pays(c, n, pos0, logits || head);
     for (int64_t i = 0; i < n;) {
         if (by_prompt_pass) {
             // passes of equal length, a multiple of sixteen but for the last
