@@ -47,6 +47,21 @@ def _off(entry, values, x, splits=0, column=slice(None)):
 SUMS_OF_512 = 1e-6
 
 
+@pytest.mark.parametrize("dtype", [12, 13])
+@pytest.mark.parametrize("spread", ["normal", "small", "wide"])
+def test_the_sums_behind_the_min_terms_keep_their_bits(dtype, spread):
+    """All codes zero leaves -dmin * m * (sum of 32 activations) alone.  Sums below 1/2 are exact as the two fp16 terms they are kept
+    in, larger ones to 2^-23; then two chains of two products each: 4 * 2^-24, and the same again for sums that cancel."""
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(6)
+    b = np.array(ffi.quantize(dtype, (rng.standard_normal((64, 512)) * 0.02).astype(np.float32))[1]).reshape(64, 2, -1)
+    b[:, :, 16:] = 0
+    entry = (dtype, np.ascontiguousarray(b.reshape(64, -1)), 64, 512)
+    x = rng.standard_normal((65, 512)).astype(np.float32)
+    x = x if spread == "normal" else x * 1e-3 if spread == "small" else np.sign(x) * 2.0 ** rng.uniform(-14, 4, x.shape).astype(np.float32)
+    assert _off(entry, ob.dequantize(dtype, entry[1], 512), x.astype(np.float32)) <= 8 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("m", [17, 65, 129, 257])
 @pytest.mark.parametrize("rows,at,big", [(64, 0, 2.0 ** 12), (64, 17, 2.0 ** 31), (130, 129, 2.0 ** 36), (200, 70, 2.0 ** 90), (256, 255, 3e38)])
 def test_bf16_rows_of_any_span_keep_their_bits(rows, at, big, m):

@@ -7,7 +7,10 @@
 // order 0 2 1 3 inside every four (what the nibble unpack of the weights produces).  K is padded to whole 256s with zeros.
 // Formats with a min term (Q4_K, Q5_K) need the sums of every 32 values as well; they are kept as an A operand of the same
 // instruction, one per 256 K: [K / 256][64 lanes][8 halfs], lane row % 32 the eight sub-block sums / 64 rounded to fp16, lane
-// 32 + row % 32 what that rounding left over, times 2048 -- 22 bits of the sum between them.
+// 32 + row % 32 what that rounding left over, times 2048.  A sum of fp16 values is a multiple of 2^-24: below 1/2 the two terms
+// are exact, above they are within 2^-23 of its size, where an fp32 is within 2^-24.  Products of 4096 values by Q4_K weights come out
+// 2.8e-7 of the exact result's norm off (weights whose codes are all zero, the min terms alone: 8e-8), by the verify passes'
+// kernels, which keep fp32 sums and take 1024 times them off again, 1.7e-5 (7e-6).
 #pragma once
 #include "tsv_internal.h"
 
