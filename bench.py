@@ -8,6 +8,7 @@ configuration the headline metric is quoted on.  Inputs (weights, KV cache, draf
 proposals) are resident in HBM before the timed region.  Prints one JSON line.
 """
 import argparse
+import ctypes as C
 import json
 import os
 import sys
@@ -424,10 +425,10 @@ def main():
         t0 = time.perf_counter()
         eng.prefill(prompt, 0, want_logits=False)     # returns after the stream has drained
         dt = time.perf_counter() - t0
-        wide = cfg["dtype"] in (ts.ffi.Q4_K, ts.ffi.Q5_K, ts.ffi.Q8_0, ts.ffi.BF16) and not (cfg.get("n_experts") and os.environ.get("TSV_MOE_FP4"))
-        rows = 64 if wide and os.environ.get("TSV_WIDE_PREFILL") != "0" else 16
-        if rows == 64 and n > 64 and args.kv_bits == "off":      # equal passes of up to 2048 rows, whole sixteens
-            rows = min(n, -(-(-(-n // -(-n // 2048))) // 16) * 16)
+        # what the handle's own count says of the two prompts: equal passes of whole sixteens, or blocks of 64, or of 16
+        passes = (C.c_int64 * 2)()
+        ts.ffi.check(ts.ffi.lib().tsv_prompt_buffers(eng._h, C.byref(C.c_int32()), C.byref(C.c_int64()), passes))
+        rows = min(n, -(-2 * n // (16 * passes[0])) * 16) if passes[0] else 64 if passes[1] else 16
         print(json.dumps({"metric": "prefill tokens/s", "value": round(n / dt, 1), "unit": "tokens/s", "n_gpus": 1,
                           "higher_is_better": True, "dtype": "f16", "data": "synthetic", "seconds": round(dt, 4),
                           "config": {"workload": args.workload, "weights": args.weights_dtype or "as the workload names",
