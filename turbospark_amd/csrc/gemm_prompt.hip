@@ -24,7 +24,7 @@
 // rows of 4096 normally distributed values one in about 80 000); a model with one in Q8_0 or MXFP4 takes the 16- and 64-row
 // passes (prompt_supported).
 //
-// Bound by the matrix pipes: the gate/up product of 2048 rows (28672 x 4096 Q4_K, silu epilogue included) takes 489 us = 983
+// Bound by the matrix pipes: the gate/up product of 2048 rows (28672 x 4096 Q4_K, silu epilogue included) takes 476 us = 1010
 // TFLOP/s on an MI355X, where a library product of 8192^3 fp16 values reaches 1164; 64 rows at a time (k_gemm_wide) the same
 // rows took 32 x 40.7 us.
 //
@@ -634,7 +634,7 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
 // operands are asked for `RING - 1` units of 32 K ahead (activations and weights alike: loads return in order, the nearer
 // distance is the one that counts).  32-row blocks past the expert's last row are not multiplied.
 // A workgroup's neighbours on its XCD are the other tiles of the same expert: the activations stay in that L2, weights pass once.
-// Taken where the average expert has at most 96 rows (prompt_expert_rows) and the storage type needs no sums.  Measured, gate/up
+// Taken for MXFP4 where the average expert has at most 96 rows (prompt_expert_rows).  Measured, gate/up
 // and down of one layer: 1500 rows, 128 experts, top 4, 2880 x 2880: 577 + 339 us in tiles of the kernel above, 454 + 247 here
 // (2.5 TB/s of weights; between 32 and 64 rows the unpack and the products take the same time, below the unpack bounds it);
 // 1000 rows, 128 experts, top 8, 768 x 2048: 144 each, 114 + 93 here.

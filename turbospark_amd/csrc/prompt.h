@@ -43,7 +43,16 @@ struct PromptRoutes {
     int32_t* n_tiles;    // device count
 };
 __host__ __device__ inline int prompt_sorted_rows(int n, int top_k, int n_experts) { return n * top_k + 31 * n_experts; }
-// rows of an expert tile: the average expert fills one, or half of one
+// Rows of an expert tile.  Two layers, whole prompts, us (n rows of them to the average expert):
+//   MXFP4, 128 experts of 768 x 2048          n = 62     96    128;  64 experts  192    256;  32 of 2880 x 2880  96    128    256
+//   64 rows in the narrow kernel                  927   1204   1544               1115   1427                    1023   1191   1938
+//   64 / 128 / 256 in k_prompt_gemm, 64          1128   1467   1855               1348   1722                    1342   1550   2549
+//                                   128          1051   1341   1689               1225   1531                    1139   1349   2115
+//                                   256          1070   1332   1669               1242   1531                    1210   1370   2215
+//   Q4_K, 128 experts of 768 x 2048, 19 / 62 / 96 / 128 rows: 64-row tiles 734 / 1190 / 1555 / 1945, 128 749 / 1119 / 1421 / 1747,
+//   256 769 / 1152 / 1471 / 1747
+// So the narrow kernel earns its 96 rows and would earn more; Q4_K takes 128 better from somewhere between 19 and 62 rows on; 256 against 128 is
+// within 5 % either way.
 inline int prompt_expert_rows(int n, int top_k, int n_experts) {
     const int avg = n * top_k / n_experts;
     return avg <= 96 ? 64 : avg <= 192 ? 128 : 256;

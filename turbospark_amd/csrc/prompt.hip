@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) void k_prompt_rope(PromptRopeArgs p) {
 // a time: S^T = K Q^T, weights, O^T += V^T P^T.  A lane's sixteen scores are of ONE pair, so the softmax crosses lanes once
 // (lane ^ 32), and they come out as the B operand of the second product in an order of positions that V is simply read in; K and
 // V are operands as the cache keeps them.  The four waves of a workgroup (128 pairs) walk the same blocks, so the L1 serves all
-// but the first.  2048 rows of the 8B shape: 101 us a layer (rotation and cache stores 16 us), where the verify passes' kernels,
+// but the first.  2048 rows of the 8B shape: 107 us a layer (rotation and cache stores 16 us), where the verify passes' kernels,
 // 64 rows at a time, took 32 x (9.7 + 4.8 merge) us (and 32 x 4.8).
 // The weights go in as two fp16 terms, 21 bits.  With one term a weight is exact only where it is its wave's largest, and here a
 // wave keeps one reference for all of a row's positions, where the verify passes' kernel has one for every few blocks: 1504 rows,
