@@ -101,11 +101,14 @@ def test_priming_by_the_prefill_equals_priming_token_by_token(name, n, passes):
     assert gc.logit_error(head_a.step(11, n - 1), head_b.step(11, n - 1)) <= 5e-4
 
 
-@pytest.mark.parametrize("name,n", [("xcd_q4_k", 70), ("xcd_q8_0", 100), ("moe_small", 128)])
-def test_a_prompt_without_logits_leaves_its_last_rows_for_an_attached_head(name, n, monkeypatch):
+@pytest.mark.parametrize("passes", ["64", "prompt"])
+@pytest.mark.parametrize("name,n", [("xcd_q4_k", 64), ("xcd_q4_k", 70), ("xcd_q8_0", 100), ("xcd_q8_0", 128), ("moe_small", 128)])
+def test_a_prompt_without_logits_leaves_its_last_rows_for_an_attached_head(name, n, passes, monkeypatch):
     """tsv_prefill on a target with a head keeps the last pass's residual rows (tsv_mtp_open), logits or not: the head
     steps from the last one, as after sixteen-row passes."""
     cfg, gpu_a, head_a = _build(name, ctx=200, oracle=False)
+    if passes == "64":
+        ffi.check(ffi.lib().tsv_limit_prompt_buffers(gpu_a._h, 0))
     monkeypatch.setenv("TSV_WIDE_PREFILL", "0")
     _, gpu_b, head_b = _build(name, ctx=200, oracle=False)
     prompt = np.random.default_rng(12).integers(0, cfg["vocab"], n).astype(np.int32)

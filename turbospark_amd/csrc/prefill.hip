@@ -125,6 +125,7 @@ int prompt_open(tsv_ctx* c) {
 bool prompt_pays(const tsv_ctx* c, int64_t n, int64_t base, bool tail) {
     if (n < PROMPT_MIN_ROWS || (n == PROMPT_MIN_ROWS && tail)) return false;  // (see prefill_passes)
     if (!c->wide.ok) return true;
+    tail |= c->mtp_head != nullptr;  // (the rows an attached head steps from)
     const int64_t blocks = n / 64 - (tail && n % 64 == 0), rest = n - 64 * blocks, smaller = blocks + (rest + 15) / 16;
     if (smaller != 2) return smaller > 2;
     return !c->prompt.two_terms && n >= c->prompt.full_experts && (n > 80 || base < 2048 * (n - 63));

@@ -1564,8 +1564,8 @@ int tsv::prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0,
             continue;
         }
         // 64 rows at a time while that many remain and nobody wants their logits
-        // (with a drafter head the last pass is a sixteen-row one: the first draft step reads its rows)
-        if (c->wide.ok && !c->profile && !c->route_forced_set && n - i >= wide_rows && (i + wide_rows < n || (!logits && !head))) {
+        // (with a drafter head, asking or attached, the last pass is a sixteen-row one: the next draft step reads its rows)
+        if (c->wide.ok && !c->profile && !c->route_forced_set && n - i >= wide_rows && (i + wide_rows < n || (!logits && !head && !c->mtp_head))) {
             if (int rc = enqueue_wide_prefill(c, ids + i, pos0 + i)) return rc;
             if (head) {
                 for (int b = 0; b < WIDE_B; b++) {
