@@ -6,7 +6,8 @@
 // are unpacked ONCE, by all four waves, into fp16 B operands in LDS (two buffers, one barrier per stage); the activations
 // arrive as ready A operands (prompt.h) and go from the L2 straight to the registers of the one wave that needs them, so
 // LDS carries the weights only: 4 KiB read per wave and 16-K step against 8 matrix instructions of 32 cycles.  Two workgroups
-// share a compute unit: while one waits at its barrier or unpacks, the other multiplies.
+// share a compute unit where there are enough; a wave by itself keeps the matrix pipe busy too, because the next stage is
+// unpacked between the products of this one (prompt_tile), a share behind each.
 //
 // What is multiplied are the stored values themselves, in operands that hold all of their bits:
 //   Q4_K / Q5_K   sc_j * q, an integer below 2048.  The superblock's d is the unit its sums are counted in: the accumulator is
@@ -24,9 +25,12 @@
 // rows of 4096 normally distributed values one in about 80 000); a model with one in Q8_0 or MXFP4 takes the 16- and 64-row
 // passes (prompt_supported).
 //
-// Bound by the matrix pipes: the gate/up product of 2048 rows (28672 x 4096 Q4_K, silu epilogue included) takes 476 us = 1010
-// TFLOP/s on an MI355X, where a library product of 8192^3 fp16 values reaches 1164; 64 rows at a time (k_gemm_wide) the same
-// rows took 32 x 40.7 us.
+// What bounds it, 28672 x 4096 Q4_K with the silu epilogue, operands of random bits on an MI355X.  At 2048 rows power: 523 us, 1042
+// TFLOP/s with the unpack left out and the activations in the L1, 2457 if the operands are all zero (a loop of products alone:
+// 1640 with random values); in a model 446 us = 1078 TFLOP/s (before 476), where a library product of 8192^3 normally distributed values
+// reaches 1164.  With few rows the instructions a wave has to issue and the round trips between them: 128 rows take 47.6 us
+// and 256 74.  With a stage unpacked ahead of its products, flat addresses for every load and the last registers of a load under
+// way given to something else (which then waits for it) these were 564, 62 and 90, 299 rows 119 (now 109; Q5_K 131 and 115).
 //
 // Workgroups are numbered so that an XCD works on every eighth block of columns with all row blocks side by side: the
 // weights of a block come into that XCD's L2 once, and the activations are shared by the blocks in flight.
@@ -52,6 +56,15 @@ __device__ __forceinline__ float half_hi(uint32_t v) { return (float)__builtin_b
 __device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
 __device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ half2v pair_of(float v) { return half2v{(_Float16)v, (_Float16)v}; }
+
+// Loads through a buffer descriptor: lane offset in a register, the walk's offset in a scalar one, so that no vector instruction
+// goes into addresses (a third of the loop's in the forms of few rows).  Past the end they return zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (uint32_t)bytes, 0x00027000);
+}
+__device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t b, uint32_t lane_at, uint32_t at) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, lane_at, at, 0));
+}
 
 // Constants that v_and_or_b32 takes from registers (the instruction has room for one literal)
 struct Bits {
@@ -90,243 +103,226 @@ struct Unit {
 
 // ---- storage types ------------------------------------------------------------------------------------------------------
 // STAGE_K real K per stage, TERMS operands per weight, SPC stages per tile chunk.  A wave's share of a stage is one half of
-// its K (`part`) of one 64-row tile: load() asks for the bytes of lane's row, unpack() leaves the operands in LDS.
+// its K (`part`) of one 64-row tile.  It is unpacked in PIECES, so that each can stand between the products of another step:
+// prepare() takes the scales (and, with the first stage of a chunk, leaves the chunk's rescale factors and min operands),
+// piece() leaves a run of operands in LDS.  The bytes come in PARTS: load() asks for one, which is free for the next stage's
+// once the piece last_piece(part) is through (-1: after prepare()).
 template <bool Q5>
 struct PromptQ45 {
-    static constexpr int TILE_BYTES = Q5 ? 11264 : 9216, STAGE_K = 128, TERMS = 1, SPC = 2;
+    static constexpr int TILE_BYTES = Q5 ? 11264 : 9216, STAGE_K = 128, TERMS = 1, SPC = 2, PIECES = 8, PARTS = 3;
     static constexpr bool UNITS = true, MINS = true;
     struct Regs {
         u32x4 q[2], h, f[Q5 ? 2 : 1];
+        half2v sc_lo, sc_hi, off_lo, off_hi;
     };
-    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
-        const u32x4* p = (const u32x4*)tile + lane;
+    static constexpr int last_piece(int part) { return 4 * part - 1; }
+    static __device__ __forceinline__ void load(Regs& r, int what, __amdgpu_buffer_rsrc_t w, uint32_t at, int sub, int part, int lane) {
         const int u = 4 * sub + 2 * part;
-        r.q[0] = p[u * 64];
-        r.q[1] = p[(u + 1) * 64];
-        r.h = p[512];
-        if (Q5) {
-            r.f[0] = p[576];
-            r.f[1] = p[640];
+        if (what == 0) {
+            if (sub == 0) r.h = load16(w, lane * 16, at + 8192);  // (the chunk's second stage has it from the first; every word of it is read there: a register of a
+            return;                      // load under way that nothing reads is given to something else, which then waits for the load)
         }
+        r.q[what - 1] = load16(w, lane * 16, at + (u + what - 1) * 1024);
+        if (Q5) r.f[Q5 ? what - 1 : 0] = load16(w, lane * 16, at + 9216 + 1024 * (what - 1));
     }
-    // 64 K of the row: sub-blocks 2 p (low nibbles) and 2 p + 1 (high), p = 2 sub + part; unit i of the pair holds elements
-    // 16 i .. 16 i + 15 of both
-    static __device__ __forceinline__ void unpack(const Regs& r, const Bits& k, Unit& unit, float, uint8_t* buf, uint8_t* mins, float2* coef, int sub,
-                                                  int part, int t64, int lane) {
+    static __device__ __forceinline__ void prepare(Regs& r, const Bits& k, Unit& unit, float, uint8_t* mins, float2* coef, int sub, int part, int t64,
+                                                   int lane) {
         const float d = half_lo(r.h.x), dmin = half_hi(r.h.x);
         uint32_t sl = r.h.y & 0x3F3F3F3Fu, sh = (r.h.w & 0x0F0F0F0Fu) | ((r.h.y >> 2) & 0x30303030u);
         if (d == 0.0f) sl = sh = 0;
-        if (sub == 0) {
+        if (sub == 0) {  // (the two waves of a tile's halves leave the same factors, and one term of the min operands each)
             const float into = unit.enter(d), into_mins = unit.enter_mins(dmin);
-            if (part == 0) {
-                coef[t64 * 64 + lane] = float2{into, into_mins};
-            } else {
-                uint32_t ml = r.h.z & 0x3F3F3F3Fu, mh = ((r.h.w >> 4) & 0x0F0F0F0Fu) | ((r.h.z >> 2) & 0x30303030u);
-                if (dmin == 0.0f) ml = mh = 0;
-                u32x4 hi, lo;
+            coef[t64 * 64 + lane] = float2{into, into_mins};
+            uint32_t ml = r.h.z & 0x3F3F3F3Fu, mh = ((r.h.w >> 4) & 0x0F0F0F0Fu) | ((r.h.z >> 2) & 0x30303030u);
+            if (dmin == 0.0f) ml = mh = 0;
+            const half2v by = pair_of(part ? 1.0f / (PROMPT_SUM_SCALE * PROMPT_SUM_LEFT) : 1.0f / PROMPT_SUM_SCALE);
+            u32x4 o;
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t m2 = (i < 2 ? ml : mh) >> (16 * (i & 1));
-                    const half2v m = as_h2(k.k6400 | (m2 & 0xFF) | ((m2 & 0xFF00) << 8)) + pair_of(-1024.0f);
-                    hi[i] = as_u32(m * pair_of(1.0f / PROMPT_SUM_SCALE));
-                    lo[i] = as_u32(m * pair_of(1.0f / (PROMPT_SUM_SCALE * PROMPT_SUM_LEFT)));
-                }
-                put_piece(mins, 0, 0, t64, lane, hi);
-                put_piece(mins, 0, 1, t64, lane, lo);
+            for (int i = 0; i < 4; i++) {
+                const uint32_t m2 = (i < 2 ? ml : mh) >> (16 * (i & 1));
+                o[i] = as_u32((as_h2(k.k6400 | (m2 & 0xFF) | ((m2 & 0xFF00) << 8)) + pair_of(-1024.0f)) * by);
             }
+            put_piece(mins, 0, part, t64, lane, o);
         }
         const uint32_t s2 = (sub == 0 ? sl : sh) >> (16 * part);
-        const half2v sc_lo = as_h2(k.k6400 | (s2 & 0xFF) | ((s2 & 0xFF) << 16)) + pair_of(-1024.0f);
-        const half2v sc_hi = as_h2(k.k6400 | ((s2 >> 8) & 0xFF) | (((s2 >> 8) & 0xFF) << 16)) + pair_of(-1024.0f);
-        const half2v off_lo = sc_lo * pair_of(-1024.0f), off_hi = sc_hi * pair_of(-64.0f);
-        const int p = 2 * sub + part;
+        r.sc_lo = as_h2(k.k6400 | (s2 & 0xFF) | ((s2 & 0xFF) << 16)) + pair_of(-1024.0f);
+        r.sc_hi = as_h2(k.k6400 | ((s2 >> 8) & 0xFF) | (((s2 >> 8) & 0xFF) << 16)) + pair_of(-1024.0f);
+        r.off_lo = r.sc_lo * pair_of(-1024.0f);
+        r.off_hi = r.sc_hi * pair_of(-64.0f);
+    }
+    // 64 K of the row: sub-blocks 2 p (low nibbles) and 2 p + 1 (high), p = 2 sub + part; unit i of the pair holds elements
+    // 16 i .. 16 i + 15 of both
+    static __device__ __forceinline__ void piece(const Regs& r, int n, const Bits& k, float, uint8_t* buf, int sub, int part, int t64, int lane) {
+        const int i = n >> 2, h = (n >> 1) & 1, high = n & 1, p = 2 * sub + part;
+        u32x4 out;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int w = 0; w < 2; w++) {
+            const uint32_t v = r.q[i][2 * h + w];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                u32x4 lo, hi;
-#pragma unroll
-                for (int w = 0; w < 2; w++) {
-                    const uint32_t v = r.q[i][2 * h + w];
-#pragma unroll
-                    for (int o = 0; o < 2; o++) {
-                        const uint32_t x = o ? v >> 8 : v;
-                        uint32_t lb = (x & 0x000F000Fu) | k.k6400, hb = (x & 0x00F000F0u) | k.k5400;  // 1024 + q, 64 + q
-                        if (Q5) {  // the fifth bit: bit 2 p (low) / 2 p + 1 (high) of the element's byte
-                            const uint32_t y = (o ? r.f[Q5 ? i : 0][2 * h + w] >> 8 : r.f[Q5 ? i : 0][2 * h + w]) >> (2 * p);
-                            lb |= (y & 0x00010001u) << 4;
-                            hb |= (y & 0x00020002u) << 7;
-                        }
-                        lo[2 * w + o] = as_u32(__builtin_elementwise_fma(as_h2(lb), sc_lo, off_lo));
-                        hi[2 * w + o] = as_u32(__builtin_elementwise_fma(as_h2(hb), sc_hi, off_hi));
-                    }
+            for (int o = 0; o < 2; o++) {
+                const uint32_t x = o ? v >> 8 : v;
+                uint32_t b = high ? (x & 0x00F000F0u) | k.k5400 : (x & 0x000F000Fu) | k.k6400;  // 64 + q, 1024 + q
+                if (Q5) {  // the fifth bit: bit 2 p (low) / 2 p + 1 (high) of the element's byte
+                    const uint32_t y = (o ? r.f[Q5 ? i : 0][2 * h + w] >> 8 : r.f[Q5 ? i : 0][2 * h + w]) >> (2 * p);
+                    b |= high ? (y & 0x00020002u) << 7 : (y & 0x00010001u) << 4;
                 }
-                put_piece(buf, 4 * part + i, h, t64, lane, lo);
-                put_piece(buf, 4 * part + 2 + i, h, t64, lane, hi);
+                out[2 * w + o] = as_u32(__builtin_elementwise_fma(as_h2(b), high ? r.sc_hi : r.sc_lo, high ? r.off_hi : r.off_lo));
             }
+        }
+        put_piece(buf, 4 * part + 2 * high + i, h, t64, lane, out);
     }
 };
 
 // Q6_K: the stage is one 64-K pair; part h holds K 32 h .. 32 h + 31 = words 0..3 of unit 3 p + h and words 2 h, 2 h + 1 of
 // unit 3 p + 2 (the order of the nibbles and bit pairs is k_repack_q6k's)
 struct PromptQ6 {
-    static constexpr int TILE_BYTES = 13568, STAGE_K = 64, TERMS = 2, SPC = 4;
+    static constexpr int TILE_BYTES = 13568, STAGE_K = 64, TERMS = 2, SPC = 4, PIECES = 4, PARTS = 2;
     static constexpr bool UNITS = true, MINS = false;
     struct Regs {
         u32x4 n;
         u32x2 hb;
         uint32_t sc, d;
+        half2v fa[2], fb[2];
     };
-    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
-        r.n = ((const u32x4*)tile)[(3 * sub + part) * 64 + lane];
-        r.hb = *(const u32x2*)(tile + ((3 * sub + 2) * 64 + lane) * 16 + 8 * part);
-        r.sc = *(const uint32_t*)(tile + 12288 + lane * 16 + 4 * sub);
-        r.d = *(const uint32_t*)(tile + 13312 + lane * 4);
-    }
-    static __device__ __forceinline__ void unpack(const Regs& r, const Bits& k, Unit& unit, float, uint8_t* buf, uint8_t*, float2* coef, int sub, int part,
-                                                  int t64, int lane) {
-        const float d = half_lo(r.d);
-        if (sub == 0) {
-            const float ratio = unit.enter(d);
-            if (part == 0) coef[t64 * 64 + lane] = float2{ratio, 0.0f};
+    static constexpr int last_piece(int part) { return part ? 3 : -1; }
+    static __device__ __forceinline__ void load(Regs& r, int what, __amdgpu_buffer_rsrc_t w, uint32_t at, int sub, int part, int lane) {
+        if (what == 0) {
+            r.sc = __builtin_amdgcn_raw_buffer_load_b32(w, lane * 16, at + 12288 + 4 * sub, 0);
+            if (sub == 0) r.d = __builtin_amdgcn_raw_buffer_load_b32(w, lane * 4, at + 13312, 0);
+            return;
         }
+        r.n = load16(w, lane * 16, at + (3 * sub + part) * 1024);
+        r.hb = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(w, lane * 16, at + (3 * sub + 2) * 1024 + 8 * part, 0));
+    }
+    static __device__ __forceinline__ void prepare(Regs& r, const Bits&, Unit& unit, float, uint8_t*, float2* coef, int sub, int part, int t64, int lane) {
+        const float d = half_lo(r.d);
+        if (sub == 0) coef[t64 * 64 + lane] = float2{unit.enter(d), 0.0f};
         const uint32_t sc2 = d == 0.0f ? 0u : r.sc >> (16 * part);
 #pragma unroll
         for (int q = 0; q < 2; q++) {  // 16 K with one scale each
             const int s8 = (int)(sc2 << (24 - 8 * q)) >> 24;
-            const half2v fa = pair_of((float)(s8 & ~15)), fb = pair_of((float)(s8 & 15));
-            const uint32_t H = r.hb[q];
-            u32x4 a[2], b[2];
-#pragma unroll
-            for (int s = 0; s < 4; s++)  // 4-K steps
-#pragma unroll
-                for (int ab = 0; ab < 2; ab++) {
-                    const int e = 2 * s + ab;
-                    const uint32_t lo = ((r.n[2 * q + (s >> 1)] >> ((s & 1) * 8 + 4 * ab)) & 0x000F000Fu) | k.k6400;
-                    const uint32_t v = lo | (((H >> (2 * e)) & 0x00030003u) << 4);
-                    const half2v lv = as_h2(v) + pair_of(-1056.0f);
-                    a[s >> 1][(s & 1) * 2 + ab] = as_u32(lv * fa);
-                    b[s >> 1][(s & 1) * 2 + ab] = as_u32(lv * fb);
-                }
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                put_piece(buf, 2 * part + q, h, t64, lane, a[h]);
-                put_piece(buf, 4 + 2 * part + q, h, t64, lane, b[h]);
-            }
+            r.fa[q] = pair_of((float)(s8 & ~15));
+            r.fb[q] = pair_of((float)(s8 & 15));
         }
+    }
+    static __device__ __forceinline__ void piece(const Regs& r, int n, const Bits& k, float, uint8_t* buf, int, int part, int t64, int lane) {
+        const int q = n >> 1, h = n & 1;
+        const uint32_t H = r.hb[q];
+        u32x4 a, b;
+#pragma unroll
+        for (int s = 0; s < 2; s++)  // 4-K steps
+#pragma unroll
+            for (int ab = 0; ab < 2; ab++) {
+                const int e = 2 * (2 * h + s) + ab;
+                const uint32_t lo = ((r.n[2 * q + h] >> (s * 8 + 4 * ab)) & 0x000F000Fu) | k.k6400;
+                const uint32_t v = lo | (((H >> (2 * e)) & 0x00030003u) << 4);
+                const half2v lv = as_h2(v) + pair_of(-1056.0f);
+                a[s * 2 + ab] = as_u32(lv * r.fa[q]);
+                b[s * 2 + ab] = as_u32(lv * r.fb[q]);
+            }
+        put_piece(buf, 2 * part + q, h, t64, lane, a);
+        put_piece(buf, 4 + 2 * part + q, h, t64, lane, b);
     }
 };
 
 // Q8_0: 64 K = blocks 2 sub, 2 sub + 1 of the tile chunk, part = block
 struct PromptQ8 {
-    static constexpr int TILE_BYTES = 8704, STAGE_K = 64, TERMS = 2, SPC = 2;
+    static constexpr int TILE_BYTES = 8704, STAGE_K = 64, TERMS = 2, SPC = 2, PIECES = 4, PARTS = 3;
     static constexpr bool UNITS = false, MINS = false;
     struct Regs {
         u32x4 q[2];
         uint32_t d;
+        float f;
     };
-    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
-        const u32x4* p = (const u32x4*)tile + lane;
-        const int u = 4 * sub + 2 * part;
-        r.q[0] = p[u * 64];
-        r.q[1] = p[(u + 1) * 64];
-        r.d = *(const uint16_t*)(tile + 8192 + lane * 8 + 2 * (2 * sub + part));
+    static constexpr int last_piece(int part) { return 2 * part - 1; }
+    static __device__ __forceinline__ void load(Regs& r, int what, __amdgpu_buffer_rsrc_t w, uint32_t at, int sub, int part, int lane) {
+        if (what == 0) r.d = __builtin_amdgcn_raw_buffer_load_b16(w, lane * 8, at + 8192 + 2 * (2 * sub + part), 0);
+        else r.q[what - 1] = load16(w, lane * 16, at + (4 * sub + 2 * part + what - 1) * 1024);
     }
-    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float rs, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
-                                                  int lane) {
-        const float d = half_lo(r.d) * rs;
+    static __device__ __forceinline__ void prepare(Regs& r, const Bits&, Unit&, float rs, uint8_t*, float2*, int, int, int, int) { r.f = half_lo(r.d) * rs; }
+    static __device__ __forceinline__ void piece(const Regs& r, int n, const Bits&, float, uint8_t* buf, int, int part, int t64, int lane) {
+        const int i = n >> 1, h = n & 1;
+        u32x4 hi, lo;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int w = 0; w < 2; w++) {
+            const uint32_t v = r.q[i][2 * h + w];
+            float f[4];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                u32x4 hi, lo;
+            for (int b = 0; b < 4; b++) f[b] = (float)((int)(v << (24 - 8 * b)) >> 24) * r.f;
 #pragma unroll
-                for (int w = 0; w < 2; w++) {
-                    const uint32_t v = r.q[i][2 * h + w];
-                    float f[4];
-#pragma unroll
-                    for (int b = 0; b < 4; b++) f[b] = (float)((int)(v << (24 - 8 * b)) >> 24) * d;
-#pragma unroll
-                    for (int o = 0; o < 2; o++) {  // (0, 2) then (1, 3)
-                        const half2v t = {(_Float16)f[o], (_Float16)f[o + 2]};
-                        hi[2 * w + o] = as_u32(t);
-                        lo[2 * w + o] = as_u32(half2v{(_Float16)(f[o] - (float)t.x), (_Float16)(f[o + 2] - (float)t.y)});
-                    }
-                }
-                put_piece(buf, 2 * part + i, h, t64, lane, hi);
-                put_piece(buf, 4 + 2 * part + i, h, t64, lane, lo);
+            for (int o = 0; o < 2; o++) {  // (0, 2) then (1, 3)
+                const half2v t = {(_Float16)f[o], (_Float16)f[o + 2]};
+                hi[2 * w + o] = as_u32(t);
+                lo[2 * w + o] = as_u32(half2v{(_Float16)(f[o] - (float)t.x), (_Float16)(f[o + 2] - (float)t.y)});
             }
+        }
+        put_piece(buf, 2 * part + i, h, t64, lane, hi);
+        put_piece(buf, 4 + 2 * part + i, h, t64, lane, lo);
     }
 };
 
 // MXFP4: sub-blocks 4 sub + 2 part, + 1 of the chunk; word w of a unit is eight K in operand order
 struct PromptMx {
-    static constexpr int TILE_BYTES = 8704, STAGE_K = 128, TERMS = 1, SPC = 2;
+    static constexpr int TILE_BYTES = 8704, STAGE_K = 128, TERMS = 1, SPC = 2, PIECES = 8, PARTS = 3;
     static constexpr bool UNITS = false, MINS = false;
     struct Regs {
         u32x4 q[2];
         uint32_t e;
+        float f[2];
     };
-    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int sub, int part, int lane) {
-        const u32x4* p = (const u32x4*)tile + lane;
+    static constexpr int last_piece(int part) { return 4 * part - 1; }
+    static __device__ __forceinline__ void load(Regs& r, int what, __amdgpu_buffer_rsrc_t w, uint32_t at, int sub, int part, int lane) {
         const int u = 4 * sub + 2 * part;
-        r.q[0] = p[u * 64];
-        r.q[1] = p[(u + 1) * 64];
-        r.e = *(const uint16_t*)(tile + 8192 + lane * 8 + u);
+        if (what == 0) r.e = __builtin_amdgcn_raw_buffer_load_b16(w, lane * 8, at + 8192 + u, 0);
+        else r.q[what - 1] = load16(w, lane * 16, at + (u + what - 1) * 1024);
     }
-    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float rs, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
-                                                  int lane) {
+    static __device__ __forceinline__ void prepare(Regs& r, const Bits&, Unit&, float rs, uint8_t*, float2*, int, int, int, int) {
         const int shift = (int)(__float_as_uint(rs) >> 23) - 127;
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int field = (int)((r.e >> (8 * i)) & 0xFF) + shift;  // 2^(e - 127) times the row's factor
-            const float sc = __uint_as_float((uint32_t)min(max(field, 1), 254) << 23);
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const uint32_t v = r.q[i][w];
-                const u32x4 o = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 0)),
-                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 1)),
-                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 2)),
-                                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 3))};
-                put_piece(buf, 4 * part + 2 * i + (w >> 1), w & 1, t64, lane, o);
-            }
+            r.f[i] = __uint_as_float((uint32_t)min(max(field, 1), 254) << 23);
         }
+    }
+    static __device__ __forceinline__ void piece(const Regs& r, int n, const Bits&, float, uint8_t* buf, int, int part, int t64, int lane) {
+        const int i = n >> 2, w = n & 3;
+        const uint32_t v = r.q[i][w];
+        const float sc = r.f[i];
+        const u32x4 o = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 0)),
+                         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 1)),
+                         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 2)),
+                         __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, sc, 3))};
+        put_piece(buf, 4 * part + 2 * i + (w >> 1), w & 1, t64, lane, o);
     }
 };
 
 // bf16: a stage is one tile chunk of 64 K; part holds units 4 part .. 4 part + 3, eight K each in operand order
 struct PromptBf {
-    static constexpr int TILE_BYTES = 8192, STAGE_K = 64, TERMS = 1, SPC = 1;
+    static constexpr int TILE_BYTES = 8192, STAGE_K = 64, TERMS = 1, SPC = 1, PIECES = 4, PARTS = 4;
     static constexpr bool UNITS = false, MINS = false;
     struct Regs {
         u32x4 q[4];
     };
-    static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int, int part, int lane) {
-        const u32x4* p = (const u32x4*)tile + lane;
-#pragma unroll
-        for (int i = 0; i < 4; i++) r.q[i] = p[(4 * part + i) * 64];
+    static constexpr int last_piece(int part) { return part; }
+    static __device__ __forceinline__ void load(Regs& r, int what, __amdgpu_buffer_rsrc_t w, uint32_t at, int, int part, int lane) {
+        r.q[what] = load16(w, lane * 16, at + (4 * part + what) * 1024);
     }
-    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float rs, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
-                                                  int lane) {
+    static __device__ __forceinline__ void prepare(Regs&, const Bits&, Unit&, float, uint8_t*, float2*, int, int, int, int) {}
+    static __device__ __forceinline__ void piece(const Regs& r, int i, const Bits&, float rs, uint8_t* buf, int, int part, int t64, int lane) {
+        u32x4 o;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            u32x4 o;
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const uint32_t v = r.q[i][w];
-                o[w] = as_u32(half2v{(_Float16)(__uint_as_float(v << 16) * rs), (_Float16)(__uint_as_float(v & 0xFFFF0000u) * rs)});
-            }
-            put_piece(buf, 2 * part + (i >> 1), i & 1, t64, lane, o);
+        for (int w = 0; w < 4; w++) {
+            const uint32_t v = r.q[i][w];
+            o[w] = as_u32(half2v{(_Float16)(__uint_as_float(v << 16) * rs), (_Float16)(__uint_as_float(v & 0xFFFF0000u) * rs)});
         }
+        put_piece(buf, 2 * part + (i >> 1), i & 1, t64, lane, o);
     }
 };
 
 // ... and as it is stored, for tiles with a row that fp16 cannot hold
 struct PromptBfStored : PromptBf {
-    static __device__ __forceinline__ void unpack(const Regs& r, const Bits&, Unit&, float, uint8_t* buf, uint8_t*, float2*, int, int part, int t64,
-                                                  int lane) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) put_piece(buf, 2 * part + (i >> 1), i & 1, t64, lane, r.q[i]);
+    static __device__ __forceinline__ void piece(const Regs& r, int i, const Bits&, float, uint8_t* buf, int, int part, int t64, int lane) {
+        put_piece(buf, 2 * part + (i >> 1), i & 1, t64, lane, r.q[i]);
     }
 };
 // what a launch over a bf16 matrix with such tiles is compiled for: each workgroup takes the form its two tiles allow
@@ -363,10 +359,37 @@ constexpr int lds_bytes() {
     return (2 * stage_bytes<F>() < 65536 ? 65536 : 2 * stage_bytes<F>()) + 2 * CHUNK_BYTES;
 }
 
+// The order of a slot's instructions: what others wait for first (activations, operands), then a share of the vector instructions
+// behind every product, which keeps the matrix pipe for 32 cycles and the issue port for four.
+template <int NT, bool STORED>
+__device__ __forceinline__ void slot_order(bool rescaled) {
+    if (STORED) return;
+    __builtin_amdgcn_sched_group_barrier(0x20, 4, 0);
+    if (NT < 4) __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT, 0);
+    if (rescaled) {
+#pragma unroll
+        for (int i = 0; i < 2 * NT; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x2, 24, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * NT; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 16 / NT, 0);
+        if (NT == 4 && (i & 1)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
+}
+
 // One tile: BM = 64 * 4 / WN rows from row0 on, of which `rows` exist.
 template <class F, int WN, int EPI>
 __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* lds, int split, int nb, int row0, int rows, int expert) {
-    constexpr int NT = 4 / WN, BM = 64 * (4 / WN), KS = F::STAGE_K / 16, GROUPS = KS / 2, STAGE = stage_bytes<F>();
+    constexpr int NT = 4 / WN, BM = 64 * (4 / WN), KS = F::STAGE_K / 16, SLOTS = KS * F::TERMS, STAGE = stage_bytes<F>();
+    constexpr int STEPS = F::SPC * KS, WANT = 16 / NT, RING = STEPS < WANT ? STEPS : WANT;  // activations: steps of 16 K in registers
+    constexpr int AHEAD = NT == 4 ? 1 : NT == 2 ? 2 : 3, BARRIER = SLOTS - AHEAD, SETS = NT == 4 ? 1 : 4;  // operands: slots ahead of their products
+    static_assert(STEPS % RING == 0 && (SETS == 1 || SLOTS % SETS == 0), "the place of a step's registers is known at compile time");
     uint8_t* const side = lds + lds_bytes<F>() - 2 * CHUNK_BYTES;  // [chunk % 2][min operands, coefficients]
     auto mins_of = [&](int c) { return side + (c & 1) * CHUNK_BYTES; };
     auto coef_of = [&](int c) { return (float2*)(side + (c & 1) * CHUNK_BYTES + MIN_BYTES); };
@@ -375,10 +398,11 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
     const int c0 = split * g.chunks_per_split, c1 = min(c0 + g.chunks_per_split, g.kchunks);
     const int s0 = c0 * F::SPC, s1 = c1 * F::SPC;
     const int tile = expert * g.n_tiles + min(2 * nb + t64, g.n_tiles - 1);  // (an odd count: the last block's second half repeats the last tile)
-    const uint8_t* const wt = g.w + (size_t)tile * g.kchunks * F::TILE_BYTES;
-    const size_t rbs = (size_t)g.a_k16 * 1024;
+    const size_t tile_bytes = (size_t)g.kchunks * F::TILE_BYTES, rbs = (size_t)g.a_k16 * 1024, sbs = (size_t)(g.a_k16 >> 4) * 1024;
     const int rb0 = (row0 >> 5) + wm * 2;
-    const uint8_t* const ap = g.a + (size_t)rb0 * rbs + lane * 16;
+    const __amdgpu_buffer_rsrc_t wsrc = buffer_of(g.w + tile * tile_bytes, tile_bytes), asrc = buffer_of(g.a + rb0 * rbs, 2 * rbs),
+                                 ssrc = buffer_of(F::MINS ? g.asum + rb0 * sbs : nullptr, 2 * sbs);
+    const uint32_t a_at[2] = {(uint32_t)lane * 16, (uint32_t)(lane * 16 + rbs)}, s_at[2] = {(uint32_t)lane * 16, (uint32_t)(lane * 16 + sbs)};
     constexpr bool STORED = std::is_same<F, PromptBfStored>::value;
     const float rs = F::UNITS || STORED ? 1.0f : g.rs[tile * 64 + lane];
     Bits bits{0x64006400u, 0x54005400u};
@@ -392,109 +416,148 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[t][j][i] = 0.f;
     Unit unit;
+    float left_in = 1.0f;  // the unit of the chunk being multiplied
     typename F::Regs w;
-    u32x4 a[2][2][2];  // [ring][16-K step of the group][row block]
-    auto load_w = [&](int s, int sub) {
-        __builtin_amdgcn_sched_barrier(0);
-        const int c = min(s, s1 - 1) / F::SPC;
-        F::load(w, wt + (size_t)c * F::TILE_BYTES, sub, part, lane);
-        __builtin_amdgcn_sched_barrier(0);
+    u32x4 a[RING][2], b[SETS][NT], sm[2], mn[NT];
+    float into[NT];
+    auto load_w = [&](int what, int s, int sub) {
+        F::load(w, what, wsrc, s / F::SPC * F::TILE_BYTES, sub, part, lane);
     };
-    auto load_a = [&](int ring, int s, int grp) {
-        const uint8_t* p = ap + (size_t)(min(s, s1 - 1) * KS + 2 * grp) * 1024;
-        __builtin_amdgcn_sched_barrier(0);
+    auto load_a = [&](int place, int step) {
 #pragma unroll
-        for (int q = 0; q < 2; q++)
-#pragma unroll
-            for (int t = 0; t < 2; t++) a[ring][q][t] = *(const u32x4*)(p + t * rbs + q * 1024);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int t = 0; t < 2; t++) a[place][t] = load16(asrc, a_at[t], step * 1024);
     };
-    load_w(s0, 0);
-    load_a(0, s0, 0);
-    F::unpack(w, bits, unit, rs, lds, mins_of(c0), coef_of(c0), 0, part, t64, lane);
-    load_w(s0 + 1, 1 % F::SPC);
+    // operand j of a stage's slot: 16-K step slot / TERMS, term slot % TERMS
+    auto load_b = [&](u32x4& to, const uint8_t* stage, int slot, int j) {
+        to = *(const u32x4*)(stage + (((slot % F::TERMS * KS + slot / F::TERMS) * 4 + wn * NT + j) * 64 + lane) * 16);
+    };
+    auto load_into = [&](int c) {
+        if (!F::UNITS) return;
+#pragma unroll
+        for (int j = 0; j < NT; j++) into[j] = coef_of(c)[(wn * NT + j) * 32 + (lane & 31)].x;
+    };
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < F::PARTS; i++) load_w(i, s0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    F::prepare(w, bits, unit, rs, mins_of(c0), coef_of(c0), 0, part, t64, lane);
+#pragma unroll
+    for (int i = 0; i < F::PIECES; i++) F::piece(w, i, bits, rs, lds, 0, part, t64, lane);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < F::PARTS; i++) load_w(i, s0 + 1, 1 % F::SPC);
+    // (the activations behind the weights, as in the loop: its first wait for weights is compiled for what either way into it leaves)
+#pragma unroll
+    for (int i = 0; i < RING - 1; i++) load_a(i, s0 * KS + i);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) load_b(b[i][j], lds, i, j);
+    load_into(c0);
     int buf = 0;
+    // A slot is one operand's products.  Around them stand, all for later: the operands of slot + AHEAD from LDS (with one or two
+    // products to a slot the LDS answers later than the next one starts), activations RING - 1 steps ahead, and a share of the
+    // next stage's unpacking.  The barrier stands AHEAD slots before a stage's end: everything unpacked is written by then, and
+    // every wave holds the stage's last operands in registers.
     for (int s = s0; s < s1; s += F::SPC) {
 #pragma unroll
         for (int sub = 0; sub < F::SPC; sub++) {
-            uint8_t* const cur = lds + buf * STAGE;
-            const bool last = s + sub + 1 >= s1;
-            const int c = s / F::SPC;
-            u32x4 sm[2];
-            if (F::UNITS && sub == 0) {
+            const uint8_t* const cur = lds + buf * STAGE;
+            uint8_t* const nxt = lds + (buf ^ 1) * STAGE;
+            const int c = s / F::SPC, sub_next = (sub + 1) % F::SPC, c_next = (s + sub + 1) / F::SPC;
 #pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    const float into = coef_of(c)[(wn * NT + j) * 32 + (lane & 31)].x;
-#pragma unroll
-                    for (int t = 0; t < 2; t++)
-#pragma unroll
-                        for (int i = 0; i < 16; i++) acc[t][j][i] *= into;
+            for (int slot = 0; slot < SLOTS; slot++) {
+                const int step = slot / F::TERMS, at = (sub * KS + step) % RING;
+                __builtin_amdgcn_sched_barrier(0);
+                if (slot == BARRIER) {
+                    __syncthreads();
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            }
-            if (F::MINS && sub == F::SPC - 1) {
+                if (slot % F::TERMS == 0) load_a((at + RING - 1) % RING, (s + sub) * KS + step + RING - 1);
+                if (F::MINS && sub == F::SPC - 1 && slot == 0) {
 #pragma unroll
-                for (int t = 0; t < 2; t++) sm[t] = *(const u32x4*)(g.asum + ((size_t)(rb0 + t) * (g.a_k16 >> 4) + c) * 1024 + lane * 16);
-            }
-            if (!last) {
-                F::unpack(w, bits, unit, rs, lds + (buf ^ 1) * STAGE, mins_of((s + sub + 1) / F::SPC), coef_of((s + sub + 1) / F::SPC), (sub + 1) % F::SPC, part, t64, lane);
-            }
+                    for (int t = 0; t < 2; t++) sm[t] = load16(ssrc, s_at[t], c * 1024);
+                }
+                const bool mins_next = F::MINS && sub == F::SPC - 1 && slot == SLOTS - 1;
+                auto next_b = [&](u32x4& to, int j) {
+                    if (slot + AHEAD < SLOTS) load_b(to, cur, slot + AHEAD, j);
+                    else if (NT == 4 && mins_next) to = *(const u32x4*)(mins_of(c) + ((wn * NT + j) * 64 + lane) * 16);
+                    else load_b(to, nxt, slot + AHEAD - SLOTS, j);
+                };
+                if (NT < 4) {
 #pragma unroll
-            for (int grp = 0; grp < GROUPS; grp++) {
-                constexpr int one = 1;
-                if (grp + 1 < GROUPS) load_a((grp + one) & 1, s + sub, grp + 1);
-                else load_a((grp + one) & 1, s + sub + 1, 0);
-                // loads return in order: asked for before the activations of group 1, the weights (from memory, where the
-                // activations are in the L2) would have to be there before that group; now they have two groups' products
-                if (grp == 0) load_w(s + sub + 2, (sub + 2) % F::SPC);
+                    for (int j = 0; j < NT; j++) next_b(b[(slot + AHEAD) % SETS][j], j);
+                    if (mins_next) {
 #pragma unroll
-                for (int q = 0; q < 2; q++)
-#pragma unroll
-                    for (int term = 0; term < F::TERMS; term++) {
-                        u32x4 b[NT];
-#pragma unroll
-                        for (int j = 0; j < NT; j++) b[j] = *(const u32x4*)(cur + (((term * KS + 2 * grp + q) * 4 + wn * NT + j) * 64 + lane) * 16);
-                        if constexpr (STORED) {
-#pragma unroll
-                            for (int t = 0; t < 2; t++) {
-                                u32x4 hi, lo;
-                                split_bf16(a[grp & 1][q][t], hi, lo);
-#pragma unroll
-                                for (int j = 0; j < NT; j++) {
-                                    acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, b[j]), acc[t][j], 0, 0, 0);
-                                    acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, lo), __builtin_bit_cast(bf16x8, b[j]), acc[t][j], 0, 0, 0);
-                                }
-                            }
-                            continue;
-                        }
-#pragma unroll
-                        for (int j = 0; j < NT; j++)
-#pragma unroll
-                            for (int t = 0; t < 2; t++)
-                                acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a[grp & 1][q][t]),
-                                                                                   __builtin_bit_cast(half8, b[j]), acc[t][j], 0, 0, 0);
+                        for (int j = 0; j < NT; j++) mn[j] = *(const u32x4*)(mins_of(c) + ((wn * NT + j) * 64 + lane) * 16);
                     }
-            }
-            if (F::MINS && sub == F::SPC - 1) {
+                }
+                // the share of the next stage's unpacking (past the last stage: of that stage again, into the buffer that nobody
+                // reads any more; the unit that the sums were left in is kept)
+                if (slot == 0) {
+                    if (sub_next == 0) left_in = unit.u;
+                    F::prepare(w, bits, unit, rs, mins_of(c_next), coef_of(c_next), sub_next, part, t64, lane);
+                }
+#pragma unroll
+                for (int p = 0; p < F::PIECES; p++)
+                    if (p * BARRIER / F::PIECES == slot) F::piece(w, p, bits, rs, nxt, sub_next, part, t64, lane);
+#pragma unroll
+                for (int i = 0; i < F::PARTS; i++)
+                    if ((F::last_piece(i) < 0 ? 0 : F::last_piece(i) * BARRIER / F::PIECES) == slot) load_w(i, s + sub + 2, (sub + 2) % F::SPC);
 #pragma unroll
                 for (int j = 0; j < NT; j++) {
-                    const float into = coef_of(c)[(wn * NT + j) * 32 + (lane & 31)].y;
-                    const u32x4 mn = *(const u32x4*)(mins_of(c) + ((wn * NT + j) * 64 + lane) * 16);
+                    const u32x4 bj = b[slot % SETS][j];
 #pragma unroll
                     for (int t = 0; t < 2; t++) {
+                        if (F::UNITS && sub == 0 && slot == 0) {
 #pragma unroll
-                        for (int i = 0; i < 16; i++) acc[t][j][i] *= into;
-                        acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, sm[t]), __builtin_bit_cast(half8, mn), acc[t][j], 0, 0, 0);
+                            for (int i = 0; i < 16; i++) acc[t][j][i] *= into[j];
+                        }
+                        if constexpr (STORED) {
+                            u32x4 hi, lo;
+                            split_bf16(a[at][t], hi, lo);
+                            acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, bj), acc[t][j], 0, 0, 0);
+                            acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, lo), __builtin_bit_cast(bf16x8, bj), acc[t][j], 0, 0, 0);
+                        } else {
+                            acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a[at][t]), __builtin_bit_cast(half8, bj), acc[t][j], 0, 0, 0);
+                        }
+                    }
+                    if (NT == 4) next_b(b[0][j], j);
+                }
+                slot_order<NT, STORED>(F::UNITS && sub == 0 && slot == 0);
+                if (mins_next) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    float by[NT];
+#pragma unroll
+                    for (int j = 0; j < NT; j++) by[j] = coef_of(c)[(wn * NT + j) * 32 + (lane & 31)].y;
+#pragma unroll
+                    for (int j = 0; j < NT; j++) {
+                        const u32x4 bj = NT == 4 ? b[0][j] : mn[j];
+#pragma unroll
+                        for (int t = 0; t < 2; t++) {
+#pragma unroll
+                            for (int i = 0; i < 16; i++) acc[t][j][i] *= by[j];
+                            acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, sm[t]), __builtin_bit_cast(half8, bj), acc[t][j], 0, 0, 0);
+                        }
+                        if (NT == 4) load_b(b[0][j], nxt, 0, j);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 2 * NT; i++) {
+                        __builtin_amdgcn_sched_group_barrier(0x2, 16, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
                     }
                 }
+                if (sub == F::SPC - 1 && slot == SLOTS - 1) load_into(c + 1);
             }
-            __syncthreads();
             buf ^= 1;
         }
     }
+    __syncthreads();
     // the columns' units (or the rows' power-of-two factors taken back out)
     float* const fin = (float*)side;
-    if (part == 0) fin[t64 * 64 + lane] = F::UNITS ? unit.u : 1.0f / rs;
+    if (part == 0) fin[t64 * 64 + lane] = F::UNITS ? left_in : 1.0f / rs;
     __syncthreads();
     float un[NT];
 #pragma unroll
