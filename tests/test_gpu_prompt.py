@@ -35,6 +35,24 @@ def test_the_prompt_matmul_is_the_dequantized_product(dtype, rows, cols, m):
         assert (np.linalg.norm(got - want, axis=0) <= 4 * (cols / 16) ** 0.5 * 2.0 ** -24 * norm).all()
 
 
+# Matrices wide enough for tiles of 128 and 256 rows, with a last tile in each of the shorter forms: 128 + 12, 128 + 100, 256 + 43,
+# 256 + 100 and 256 + 144 rows; an odd count of 64-row tiles, the last of them with 6 rows
+@pytest.mark.parametrize("dtype", [8, 12, 13, 14, 30, 39])
+@pytest.mark.parametrize("m", [140, 228, 299, 356, 400])
+def test_full_tiles_and_a_short_last_one(dtype, m):
+    from turbospark_amd import ffi
+    rows, cols = 16390, 512
+    rng = np.random.default_rng(m)
+    entry = ffi.quantize(dtype, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, cols)).astype(np.float32)
+    want = x.astype(np.float16).astype(np.float64) @ ob.dequantize(dtype, entry[1], cols).astype(np.float64).T
+    got = ffi.matmul(entry, x)
+    # K / 16 sums in one chain (see above), by row and by column
+    bound = 4 * (cols / 16) ** 0.5 * 2.0 ** -24
+    for axis in (0, 1):
+        assert (np.linalg.norm(got - want, axis=axis) <= bound * np.linalg.norm(want, axis=axis)).all()
+
+
 def _off(entry, values, x, splits=0, column=slice(None)):
     """Distance of the prompt matmul (or one output column) from the exact product, relative to its norm."""
     from turbospark_amd import ffi

@@ -655,15 +655,19 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
     }
 }
 
-// The grid's tiles are g.bm rows; a tile that holds fewer takes the smallest form that covers them.  Short last tiles cost what
-// their rows cost then: 299 rows in tiles of 256 were multiplied as 512, in tiles of 128 as 384 (and came out at 1.3 workgroups
-// per place on the chip).
+// The grid's tiles are g.bm rows; a tile that holds fewer takes the smallest form that covers them, and these come after all
+// full ones: they fill the places that the long ones leave free.  299 rows in tiles of 256 (28672 x 4096 Q4_K, 224 long tiles and
+// 224 short ones) took 111 us with a column block's two tiles side by side and take 91 so; the short tiles' weights come from
+// memory a second time, which is hidden.
 template <class F, int EPI>
 __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    // which tile: XCD x takes the column blocks x, x + 8, ..., all row blocks of one before the next
-    const int per_split = (g.nt + 7) / 8 * 8 * g.mt, split = blockIdx.x / per_split, id = blockIdx.x - split * per_split;
-    const int slot = id >> 3, nb = slot / g.mt * 8 + (id & 7), mb = slot % g.mt;
+    // which tile: XCD x takes the column blocks x, x + 8, ..., all full row blocks of one before the next; then the short ones
+    const int nt8 = (g.nt + 7) / 8 * 8, full = g.tiles || g.mt == 1 || g.m % g.bm == 0 ? g.mt : g.mt - 1, first_short = nt8 * full * g.splits;
+    const bool is_short = (int)blockIdx.x >= first_short;
+    const int across = is_short ? 1 : full, at = is_short ? blockIdx.x - first_short : blockIdx.x;
+    const int split = at / (nt8 * across), id = at - split * nt8 * across;
+    const int slot = id >> 3, nb = slot / across * 8 + (id & 7), mb = is_short ? full : slot % across;
     if (nb >= g.nt) return;
     int row0 = mb * g.bm, rows = min(g.m - row0, g.bm), expert = 0;  // the tile's first row and how many of its rows exist
     if (g.tiles) {
@@ -922,7 +926,34 @@ int launch_f(hipStream_t s, PromptGemmArgs& g, int epi) {
     return epi == EPI_SILU ? launch_p<F, EPI_SILU>(s, g) : launch_p<F, EPI_PARTIAL>(s, g);
 }
 
-int row_block(int m) { return m > 128 ? 256 : m > 64 ? 128 : 64; }
+// What a matmul of m rows in tiles of bm and `splits` parts of K takes, us (6 for the launch left out).  A tile of 256 / 128 / 64 rows
+// x 128 columns takes 3.95 / 2.52 / 1.52 us per 256 K by itself on a compute unit, and one of two that share it half of 6.9 / 4.14 /
+// 2.8 (Q4_K; 1.7 times that with two operands per weight); beside that 1.1 us a tile, and the partial sums' way through memory
+// (written here, read by the norm or the rotation).  Full tiles go out first, 256 at a time, and the short ones into what these
+// leave.  Fitted to 24 shapes of 90 to 1500 rows (Q4_K, Q5_K, Q6_K, Q8_0, bf16) measured in every tiling: the choice is within 2 %
+// of the best one on average, 13 % at worst.  Tiles of 256 in as many parts as fill 512 places were up to 1.9 times the best: 299
+// rows of 6144 x 4096 took 46 us so and 31 in (128, 2), of 4096 x 4096 31 and 21 in (128, 4), of 1024 x 4096 Q6_K 29 and 15 in
+// (64, 6).
+float tiling_time(const TiledW& w, int m, int bm, int splits) {
+    struct Cost {
+        float alone, shared;
+    };
+    auto cost = [](int rows) { return rows > 128 ? Cost{3.95f, 3.45f} : rows > 64 ? Cost{2.52f, 2.07f} : Cost{1.52f, 1.4f}; };
+    const int per = (w.kchunks + splits - 1) / splits, nt = (w.n_tiles + 1) / 2 * splits;
+    const int full = m / bm, rest = m % bm, n_long = nt * std::max(full, 1), n_short = full && rest ? nt : 0;
+    const Cost l = cost(full ? bm : rest), s = cost(rest);
+    const int deep = (n_long + 255) / 256;
+    float t = deep % 2 ? (deep - 1) * l.shared + l.alone : deep * l.shared;
+    if (n_short) t = std::max(t, (n_long * l.shared + n_short * s.shared) / 256 + 0.26f * s.shared);
+    const float k256 = per * fmt_chunk_elems(w.fmt) / 256.0f * (w.fmt == FMT_Q6K || w.fmt == FMT_Q80 ? 1.7f : 1.0f);
+    return k256 * t + (n_long + n_short) * (1.1f / 256) + (float)splits * m * w.n_rows * 1.7e-6f;
+}
+int row_block(const TiledW& w, int m, int splits) {
+    int best = 256;
+    for (int bm : {128, 64})
+        if (bm < 2 * m && tiling_time(w, m, bm, splits) < tiling_time(w, m, best, splits)) best = bm;
+    return best;
+}
 
 }  // namespace
 
@@ -943,11 +974,24 @@ int make_row_scale(hipStream_t s, TiledW& w) {
 
 bool prompt_holds(const TiledW& w) { return !w.rows_unfit || w.fmt == FMT_BF16; }
 
-int prompt_splits(const TiledW& w, int m) {
-    const int bm = row_block(m), tiles = (m + bm - 1) / bm * ((w.n_tiles + 1) / 2);
-    int sp = std::min(std::min(8, w.kchunks), std::max(1, 512 / std::max(1, tiles)));
-    const int per = (w.kchunks + sp - 1) / sp;
-    return (w.kchunks + per - 1) / per;
+int prompt_splits(const TiledW& w, int m, const TiledW* beside) {
+    auto fits = [](const TiledW& t, int k) {
+        const int per = (t.kchunks + k - 1) / k;
+        return (t.kchunks + per - 1) / per == k;
+    };
+    auto time = [&](const TiledW& t, int k) { return tiling_time(t, m, row_block(t, m, k), k); };
+    const int64_t sums = (int64_t)((m + 15) / 16 * 16) * (w.n_rows + (beside ? beside->n_rows : 0));
+    int best = 1;
+    float least = 0.f;
+    for (int k = 1; k <= 8 && (k == 1 || k * sums <= PROMPT_PARTIALS); k++) {
+        if (!fits(w, k) || (beside && !fits(*beside, k))) continue;
+        const float t = time(w, k) + (beside ? time(*beside, k) : 0.f);
+        if (k == 1 || t < least) {
+            best = k;
+            least = t;
+        }
+    }
+    return best;
 }
 
 static int launch_any(hipStream_t s, const TiledW& w, PromptGemmArgs& g, int epi) {
@@ -991,7 +1035,7 @@ int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void
     g.nt = (w.n_tiles + 1) / 2;
     g.n_valid = epi == EPI_SILU ? w.n_rows / 2 : n_valid;
     g.out_k16 = prompt_k16(w.n_rows / 2);
-    g.bm = row_block(m);
+    g.bm = row_block(w, m, splits);
     return launch_any(s, w, g, epi);
 }
 

@@ -33,9 +33,8 @@ size_t lay_out(tsv_ctx* c, int rows, uint8_t* at) {
     size_t width = (size_t)qd + 2 * c->nkv * c->hd;
     for (const LayerW& L : c->layers)
         width = std::max(width, (size_t)(L.n_experts ? std::max(c->hidden, L.n_experts) : c->hidden));
-    // one partial sum per row and column, or as many as fill the chip: at most 512 tiles of 256 x 128 (prompt_splits), by half more
-    // where q and k are split by themselves and the value columns come on top
-    const size_t partial_floats = std::max((size_t)rows * width, std::min((size_t)8 * rows * width, (size_t)512 * 256 * 128 * 3 / 2));
+    // one partial sum per row and column, or what prompt_splits makes of them
+    const size_t partial_floats = std::max((size_t)rows * width, std::min((size_t)8 * rows * width, (size_t)PROMPT_PARTIALS));
     put(w.x, (size_t)rows * c->hidden * 4);
     put(w.a_h, prompt_a_bytes(rows, c->hidden));
     put(w.s_h, prompt_sum_bytes(rows, c->hidden));
@@ -138,17 +137,6 @@ void prompt_limit(tsv_ctx* c, size_t bytes) {
 
 namespace {
 
-// one split count for a projection whose value part has a storage type of its own
-int common_splits(const TiledW& a, const TiledW& b, int n) {
-    auto fits = [](const TiledW& t, int k) {
-        const int per = (t.kchunks + k - 1) / k;
-        return (t.kchunks + per - 1) / per == k;
-    };
-    int sp = prompt_splits(a, n);
-    while (sp > 1 && !(fits(a, sp) && fits(b, sp))) sp--;
-    return sp;
-}
-
 int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits) {
     hipStream_t s = c->stream;
     tsv_ctx::Prompt& w = c->prompt;
@@ -212,7 +200,7 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
         if ((rc = norm(L.attn_norm, sp, nullptr, prompt_fmt_has_sums(L.qkv.fmt) || !L.v_only.tiles ? L.qkv : L.v_only))) return rc;
         na.partial = w.partial;
         na.weights = nullptr;
-        sp = L.v_only.tiles ? common_splits(L.qkv, L.v_only, n) : prompt_splits(L.qkv, n);
+        sp = prompt_splits(L.qkv, n, L.v_only.tiles ? &L.v_only : nullptr);
         if ((rc = launch_prompt_gemm(s, L.qkv, w.a_h, w.s_h, w.partial, nullptr, n, sp, EPI_PARTIAL, qkv_n, L.qkv.n_rows))) return rc;
         if (L.v_only.tiles &&
             (rc = launch_prompt_gemm(s, L.v_only, w.a_h, w.s_h, w.partial + L.qkv.n_rows, nullptr, n, sp, EPI_PARTIAL, qkv_n, L.v_only.n_rows)))

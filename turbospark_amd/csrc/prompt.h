@@ -96,7 +96,10 @@ int launch_prompt_gemm(hipStream_t s, const TiledW& w, const void* a, const void
 // a: the sorted pairs' activations; EPI_SILU or EPI_PARTIAL; w holds every expert's tiles one after the other
 int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const void* asum, void* out, void* out_sum, int epi, int ldo,
                           const PromptExperts& x);
-int prompt_splits(const TiledW& w, int m);
+// How many parts of K a matmul of m rows goes in, or one of the same rows by w and `beside` into the same sums: at most 8, and (more
+// than one) at most PROMPT_PARTIALS sums in all
+constexpr int64_t PROMPT_PARTIALS = (int64_t)512 * 256 * 128;
+int prompt_splits(const TiledW& w, int m, const TiledW* beside = nullptr);
 // Q8_0, bf16, MXFP4: fills w.row_scale (prompt_row_scales floats), the power-of-two factors of the matrix's rows, and w.rows_unfit;
 // waits for the stream
 inline size_t prompt_row_scales(const TiledW& w) { return (size_t)w.n_tiles * TILE_ROWS + 1; }
