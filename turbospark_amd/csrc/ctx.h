@@ -212,6 +212,7 @@ struct tsv_ctx {
         VerifyParams *vp_block = nullptr, *vp_block_host = nullptr;  // [16] the parameter blocks of a block draft's steps
         int32_t *chain = nullptr, *chain_host = nullptr;  // the tokens of a block draft and the error word
         AcceptParams *draw_dev = nullptr, *draw_host = nullptr;  // [16] the draw parameters of a sampled block's steps
+        uint8_t *prompt_a = nullptr, *prompt_s = nullptr;  // fc's input rows as a prompt matmul's activations and their sums; null: none
     } mtp;
     int64_t x_base = -1;  // rows [0, x_rows) of x are the finished residual rows of positions x_base ..
     int x_rows = 0;
@@ -253,6 +254,10 @@ int prompt_open(tsv_ctx* c);
 bool prompt_pays(const tsv_ctx* c, int64_t n, int64_t base, bool tail);
 void prompt_limit(tsv_ctx* c, size_t bytes);
 int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits);
+// A head's cache rows for n <= the target's rows of a prompt pass: row r pairs next[r] with row r of the target's prompt.x, which
+// is used up.  prompt_prime_open: its buffers, or none where the head's matrices or widths do not allow it.
+int prompt_prime_open(tsv_ctx* head);
+int prompt_prime(tsv_ctx* head, const int32_t* next, int n, int64_t position);
 // One verify pass: everything enqueued on the handle's stream, no synchronisation; then the optional copy of the rows' logits.
 int enqueue_verify(tsv_ctx* c, const int32_t* feed, const int32_t* parent, int m, int64_t base);
 int finish_verify(tsv_ctx* c, int m, uint16_t* logits_out);

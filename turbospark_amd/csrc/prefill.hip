@@ -281,6 +281,110 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
 
 }  // namespace
 
+// fc's columns pass through the target's buffers, and the head's K / V columns too
+int prompt_prime_open(tsv_ctx* h) {
+    const tsv_ctx* t = h->mtp.target;
+    const LayerW& L = h->layers[0];
+    if (!t->prompt.ok || !t->prompt.rows || !prompt_holds(h->mtp.fc) || !prompt_holds(L.qkv) || !prompt_holds(L.v_only) || h->nq * h->hd % 64 ||
+        h->hd > t->hd || 2 * h->nkv * h->hd > std::max(t->hidden, (t->nq + 2 * t->nkv) * t->hd))
+        return TSV_OK;
+    const size_t a = prompt_a_bytes(t->prompt.rows, 2 * h->hidden), s = prompt_fmt_has_sums(h->mtp.fc.fmt) ? prompt_sum_bytes(t->prompt.rows, 2 * h->hidden) : 0;
+    uint8_t* at = nullptr;
+    if (hipMalloc((void**)&at, a + s) != hipSuccess) {
+        (void)hipGetLastError();  // (no room: sixteen rows at a time)
+        return TSV_OK;
+    }
+    h->allocs.push_back(at);
+    TSV_HIP(hipMemsetAsync(at, 0, a + s, h->stream));  // (rows past a pass's last one hold finite values, K padding zeros)
+    h->mtp.prompt_a = at;
+    h->mtp.prompt_s = s ? at + a : nullptr;
+    return TSV_OK;
+}
+
+// A prompt leaves nothing in a head but its cache rows, so these are made and nothing behind them: fc, the layer's first norm, the
+// K and V columns of its projection, rotation.  In the buffers of the target's pass, on its stream.
+int prompt_prime(tsv_ctx* h, const int32_t* next, int n, int64_t position) {
+    tsv_ctx* t = h->mtp.target;
+    tsv_ctx::Prompt& w = t->prompt;
+    hipStream_t s = h->stream;
+    const LayerW& L = h->layers[0];
+    const int H = h->hidden, q_rows = h->nq * h->hd, kv_n = 2 * h->nkv * h->hd;
+    if (position != h->position || position + n > h->max_context) {
+        set_error(position != h->position ? "mtp: the rows to prime do not start where the head's cache ends" : "verify: block would write past the KV capacity");
+        return TSV_ERR_INVALID;
+    }
+    for (int i = 0; i < n; i++)
+        if (next[i] < 0 || next[i] >= h->vocab) {
+            set_error("verify: token id outside the vocabulary");
+            return TSV_ERR_INVALID;
+        }
+    int rc;
+    // (from the caller's pageable memory: the runtime has taken its copy when this returns)
+    TSV_HIP(hipMemcpyAsync(w.ids, next, (size_t)n * 4, hipMemcpyHostToDevice, s));
+    PromptMtpArgs ma{};
+    ma.raw = h->embed_raw;
+    ma.dtype = h->embed_dtype;
+    ma.hidden = H;
+    ma.n = n;
+    ma.base = (int)position;
+    ma.half = h->hd / 2;
+    ma.x = w.x;
+    ma.ids = w.ids;
+    ma.norm_e = h->mtp.norm_e;
+    ma.norm_t = t->final_norm;
+    ma.norm_h = h->mtp.norm_h;
+    ma.freqs = h->freqs;
+    ma.eps = h->eps;
+    ma.mscale = h->rope_mscale;
+    ma.cs = w.cs;
+    ma.a = h->mtp.prompt_a;
+    ma.asum = h->mtp.prompt_s;
+    if ((rc = launch_prompt_mtp_input(s, ma))) return rc;
+    int sp = prompt_splits(h->mtp.fc, n);
+    if ((rc = launch_prompt_gemm(s, h->mtp.fc, ma.a, ma.asum, w.partial, nullptr, n, sp, EPI_PARTIAL, H, H))) return rc;
+    PromptNormArgs na{};
+    na.x = w.x;
+    na.partial = w.partial;
+    na.w = L.attn_norm;
+    na.a = w.a_h;
+    na.asum = prompt_fmt_has_sums(L.qkv.fmt) || (L.v_only.tiles && prompt_fmt_has_sums(L.v_only.fmt)) ? w.s_h : nullptr;
+    na.n = n;
+    na.hidden = na.ldp = H;
+    na.splits = na.slots = sp;
+    na.eps = h->eps;
+    if ((rc = launch_prompt_norm(s, na))) return rc;
+    TiledW kv = L.qkv;  // the rows behind the q heads'
+    kv.tiles += (size_t)(q_rows / TILE_ROWS) * kv.kchunks * fmt_tile_bytes(kv.fmt);
+    kv.n_tiles -= q_rows / TILE_ROWS;
+    kv.n_rows -= q_rows;
+    if (kv.row_scale) kv.row_scale += q_rows;
+    sp = prompt_splits(kv, n, L.v_only.tiles ? &L.v_only : nullptr);
+    if ((rc = launch_prompt_gemm(s, kv, w.a_h, w.s_h, w.partial, nullptr, n, sp, EPI_PARTIAL, kv_n, kv.n_rows))) return rc;
+    if (L.v_only.tiles && (rc = launch_prompt_gemm(s, L.v_only, w.a_h, w.s_h, w.partial + kv.n_rows, nullptr, n, sp, EPI_PARTIAL, kv_n, L.v_only.n_rows)))
+        return rc;
+    PromptRopeArgs ra{};
+    ra.qkv = w.partial;
+    ra.splits = sp;
+    ra.ldq = kv_n;
+    ra.n = n;
+    ra.base = (int)position;
+    ra.cs = w.cs;
+    ra.bias = L.bqkv ? L.bqkv + q_rows : nullptr;
+    ra.k_norm = L.k_norm;
+    ra.eps = h->eps;
+    ra.kc = L.kc;
+    ra.vc = L.vc;
+    ra.nkv = h->nkv;
+    ra.hd = h->hd;
+    ra.cap = L.kv_slots;
+    ra.paired = L.rope_fused && h->hd == 128;
+    if ((rc = launch_prompt_rope(s, ra))) return rc;
+    h->position = position + n;
+    h->high_water = std::max(h->high_water, h->position);
+    h->mtp.own_valid = false;
+    return TSV_OK;
+}
+
 int enqueue_prompt_pass(tsv_ctx* c, const int32_t* ids, int n, int64_t base, bool finish, bool logits) {
     if (base != c->position) {
         set_error("prefill: start position does not match the KV cursor");

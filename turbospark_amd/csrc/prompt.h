@@ -126,6 +126,20 @@ int launch_prompt_norm(hipStream_t s, const PromptNormArgs& a);
 int launch_prompt_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float* x, const int32_t* ids, int n, int base, const float* freqs,
                         float mscale, int half, float2* cs);
 
+// A drafter head's input rows (k_mtp_input, misc.hip): [norm_e(embedding of ids[row]) ; norm_h(norm_t(x[row]))] as the fc matmul's
+// activations (K = 2 hidden) and sums (nullable), the rotation table of positions base .., and x cleared for the sums to come
+struct PromptMtpArgs {
+    const uint8_t* raw;
+    int dtype, hidden, n, base, half;
+    float* x;
+    const int32_t* ids;
+    const float *norm_e, *norm_t, *norm_h, *freqs;
+    float eps, mscale;
+    float2* cs;
+    uint8_t *a, *asum;
+};
+int launch_prompt_mtp_input(hipStream_t s, const PromptMtpArgs& a);
+
 // bias, per-head norm, rotation; q as fp16 rows, K and V into the cache
 struct PromptRopeArgs {
     const float* qkv;  // [n / 16][splits][16][ldq]
@@ -134,7 +148,7 @@ struct PromptRopeArgs {
     const float *bias, *q_norm, *k_norm;
     float eps;
     uint16_t *q16, *kc, *vc;
-    int nq, nkv, hd, cap;  // cap: positions of the cache, position p in slot p % cap
+    int nq, nkv, hd, cap;  // cap: positions of the cache, position p in slot p % cap; nq = 0: the columns are those of K and V alone
     int paired;            // as in RopeKvArgs
 };
 int launch_prompt_rope(hipStream_t s, const PromptRopeArgs& a);

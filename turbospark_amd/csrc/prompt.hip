@@ -33,7 +33,19 @@ __global__ __launch_bounds__(256) void k_prompt_embed(const uint8_t* __restrict_
     }
 }
 
-// ---- residual add + RMSNorm -------------------------------------------------------------------------------------------------
+// ---- a drafter head's input ----------------------------------------------------------------------------------------------------
+template <int WAVES>
+__device__ __forceinline__ float sum_of_waves(float v, float* red) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) v += red[w];
+    __syncthreads();
+    return v;
+}
+
 // Eight values (consecutive K) of a row as activations, and the sum of its 32-value sub-block, whose other values sit in the
 // three neighbouring lanes.  The halves are pinned in registers between the store and the sum: the sum has to be that of the
 // stored bits (pinned_half).
@@ -57,6 +69,75 @@ __device__ __forceinline__ void put_activations(uint8_t* a, uint8_t* asum, int r
             o[256] = lo;
         }
     }
+}
+
+// One workgroup per row.  The table's row is decoded value by value side by side (its bytes are) and passes through LDS to the
+// lanes, which hold eight consecutive values of it and of the state, NV times.  400 rows of 4096 take 26 us, most of it the decoding's
+// round trips; sixteen rows at a time (k_mtp_input) took 25 x 14.
+template <int NV>
+__global__ __launch_bounds__(512) void k_prompt_mtp_input(PromptMtpArgs p) {
+    __shared__ float red[8];
+    __shared__ __attribute__((aligned(16))) float emb[NV * 4096];
+    const int row = blockIdx.x;
+    const long tok = p.ids[row];
+    float* const xr = p.x + (size_t)row * p.hidden;
+    float hv[NV][8], ev[NV][8], se = 0.f, sh = 0.f;
+    auto for_each = [&](auto f) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int k = i * 4096 + threadIdx.x * 8;
+            f(i, k, k < p.hidden);
+        }
+    };
+    for_each([&](int i, int k, bool live) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 t = live ? *(const float4*)(xr + k + 4 * h) : float4{0.f, 0.f, 0.f, 0.f};
+            hv[i][4 * h] = t.x, hv[i][4 * h + 1] = t.y, hv[i][4 * h + 2] = t.z, hv[i][4 * h + 3] = t.w;
+        }
+    });
+#pragma unroll 8
+    for (int j = 0; j < NV * 8; j++) {
+        const int e = j * 512 + threadIdx.x;
+        emb[e] = e < p.hidden ? embed_elem(p.raw, p.dtype, p.hidden, tok, e) : 0.f;
+    }
+    const float pos = (float)(p.base + row);
+    for (int i = threadIdx.x; i < p.half; i += 512) {
+        float sn, c;
+        sincosf(pos * p.freqs[i], &sn, &c);
+        p.cs[(size_t)row * p.half + i] = float2{c * p.mscale, sn * p.mscale};
+    }
+    __syncthreads();
+    for_each([&](int i, int k, bool) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            ev[i][e] = emb[k + e];
+            se += ev[i][e] * ev[i][e];
+            sh += hv[i][e] * hv[i][e];
+        }
+    });
+    const float inv_e = 1.0f / sqrtf(sum_of_waves<8>(se, red) / (float)p.hidden + p.eps);
+    const float inv_h = 1.0f / sqrtf(sum_of_waves<8>(sh, red) / (float)p.hidden + p.eps);
+    float st = 0.f;
+    for_each([&](int i, int k, bool live) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            hv[i][e] = live ? hv[i][e] * p.norm_t[k + e] * inv_h : 0.f;
+            st += hv[i][e] * hv[i][e];
+        }
+    });
+    const float inv_t = 1.0f / sqrtf(sum_of_waves<8>(st, red) / (float)p.hidden + p.eps);
+    const int k16 = prompt_k16(2 * p.hidden);
+    for_each([&](int i, int k, bool live) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            ev[i][e] = live ? ev[i][e] * p.norm_e[k + e] * inv_e : 0.f;
+            hv[i][e] = live ? hv[i][e] * p.norm_h[k + e] * inv_t : 0.f;
+            if (live) xr[k + e] = 0.f;
+        }
+        put_activations(p.a, p.asum, row, k, k16, ev[i], live);
+        put_activations(p.a, p.asum, row, p.hidden + k, k16, hv[i], live);
+    });
 }
 
 // The row in the registers of W waves (NV x 512 values each), 8 / W rows to a workgroup.  Bound by what one compute unit draws
@@ -569,6 +650,17 @@ __global__ __launch_bounds__(256) void k_prompt_gather(const uint16_t* __restric
 int launch_prompt_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float* x, const int32_t* ids, int n, int base, const float* freqs,
                         float mscale, int half, float2* cs) {
     hipLaunchKernelGGL(k_prompt_embed, dim3(n), dim3(256), 0, s, raw, dtype, hidden, x, ids, base, freqs, mscale, half, cs);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int launch_prompt_mtp_input(hipStream_t s, const PromptMtpArgs& a) {
+    if (a.hidden > 8192 || a.hidden % 32 || a.n < 1) {
+        set_error("drafter head: hidden must be a multiple of 32, at most 8192");
+        return TSV_ERR_UNSUPPORTED;
+    }
+    if (a.hidden <= 4096) hipLaunchKernelGGL(k_prompt_mtp_input<1>, dim3(a.n), dim3(512), 0, s, a);
+    else hipLaunchKernelGGL(k_prompt_mtp_input<2>, dim3(a.n), dim3(512), 0, s, a);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }

@@ -412,6 +412,7 @@ int launch_pass(tsv_ctx* c, int m) {
             for (int rep = 0; rep < c->repeat[PC_ROPE] && !rc; rep++) rc = launch_rope_kv(s, ra, m);
         }
         if (rc) return rc;
+        if (c->mtp.on && c->headless) return TSV_OK;  // a head's primed rows leave nothing but the cache's
         if (L.tq.k_bits) {
             // the pass's K / V rows sit in the staging cache (crates/runtime/src/kv_write.rs:66-118): quantize them
             // into the layer's stores and rotate q -- attention then runs in the rotated space, over the stores
@@ -1379,6 +1380,7 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
     const char* wide_env = getenv("TSV_WIDE_PREFILL");
     c->prompt.ok = !share && !(wide_env && wide_env[0] == '0') && prompt_supported(c);
     if (c->prompt.ok && (rc = prompt_open(c))) return fail(rc);
+    if (share && (rc = prompt_prime_open(c))) return fail(rc);
     *out = c;
     return TSV_OK;
 }
@@ -1548,6 +1550,14 @@ int tsv::prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0,
             if (int rc = enqueue_prompt_pass(c, ids + i, rows, pos0 + i, c->mtp_head != nullptr, last && logits)) return rc;
             if (last && logits)
                 TSV_HIP(hipMemcpyAsync(logits, c->logits + (size_t)((rows - 1) % 16) * c->vocab, (size_t)c->vocab * 2, hipMemcpyDeviceToHost, c->stream));
+            const int primed = (int)std::min<int64_t>(rows, n - 1 - i + (next_token >= 0));  // (rows whose next token is known)
+            if (head && head->mtp.prompt_a && primed) {
+                std::vector<int32_t> nt(primed);
+                for (int r = 0; r < primed; r++) nt[r] = i + r + 1 < n ? ids[i + r + 1] : next_token;
+                if (int rc = prompt_prime(head, nt.data(), primed, pos0 + i)) return rc;
+                i += rows;
+                continue;
+            }
             for (int b = 0; head && b < rows; b += TSV_MAX_ROWS) {
                 int32_t nt[TSV_MAX_ROWS];
                 int m = 0;
