@@ -655,6 +655,11 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
     }
 }
 
+// Into scalar registers: a buffer descriptor made from vector registers is gone through lane by lane
+__device__ __forceinline__ PromptTile uniform_tile(PromptTile t) {
+    return {__builtin_amdgcn_readfirstlane(t.expert), __builtin_amdgcn_readfirstlane(t.first), __builtin_amdgcn_readfirstlane(t.cnt), 0};
+}
+
 // The grid's tiles are g.bm rows; a tile that holds fewer takes the smallest form that covers them, and these come after all
 // full ones: they fill the places that the long ones leave free.  299 rows in tiles of 256 (28672 x 4096 Q4_K, 224 long tiles and
 // 224 short ones) took 111 us with a column block's two tiles side by side and take 91 so; the short tiles' weights come from
@@ -672,7 +677,7 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     int row0 = mb * g.bm, rows = min(g.m - row0, g.bm), expert = 0;  // the tile's first row and how many of its rows exist
     if (g.tiles) {
         if (mb >= *g.tile_count) return;
-        const PromptTile t = g.tiles[mb];
+        const PromptTile t = uniform_tile(g.tiles[mb]);
         row0 = t.first;
         rows = t.cnt;
         expert = t.expert;
@@ -695,59 +700,64 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
 // ---- experts with few rows, MXFP4 -----------------------------------------------------------------------------------------
 // The tile of the kernel above at 64 rows is bound by the L1 and the LDS, not by the matrix pipes (each wave draws all 64 rows'
 // activations, and every unpacked weight crosses the LDS for 64 rows only), and a stage ahead is too little in flight for a
-// stream of weights.  Here a workgroup makes the 64 columns of ONE row tile, its waves each a quarter of K: a lane unpacks the
+// stream of weights.  Here a workgroup makes the 128 columns of TWO row tiles, its waves each a quarter of K: a lane unpacks the
 // weights of its own row and one v_permlane32_swap per register turns two eight-K pieces of 64 rows into the B operands of two
 // 32-column blocks, so nothing goes through LDS before the four partial sums meet there, no barrier stands in the loop, and
 // operands are asked for `RING - 1` units of 32 K ahead (activations and weights alike: loads return in order, the nearer
 // distance is the one that counts).  32-row blocks past the expert's last row are not multiplied.
 // A workgroup's neighbours on its XCD are the other tiles of the same expert: the activations stay in that L2, weights pass once.
-// Taken for MXFP4 where the average expert has at most 96 rows (prompt_expert_rows).  Measured, gate/up
-// and down of one layer: 1500 rows, 128 experts, top 4, 2880 x 2880: 577 + 339 us in tiles of the kernel above, 454 + 247 here
-// (2.5 TB/s of weights; between 32 and 64 rows the unpack and the products take the same time, below the unpack bounds it);
-// 1000 rows, 128 experts, top 8, 768 x 2048: 144 each, 114 + 93 here.
-constexpr int NARROW_ROWS = 64;
+// Measured, gate/up and down of one layer, 1500 rows, 128 experts, top 4, 2880 x 2880: 577 + 339 us in tiles of the kernel above,
+// 452 + 247 with one row tile to a workgroup (every activation drawn twice as often), 357 + 228 here (3.1 TB/s of weights); 1000
+// rows, 128 experts, top 8, 768 x 2048: 144 each, 114 + 93, 93 + 96.  Of the 357, 298 are left with the weights in the cache, 331
+// with the activations in the L1 and 334 without the unpack: no one thing bounds it, a workgroup's start and end are the rest.
+// Rings of 3 and 4 (1 and 2 units more ahead) are 2 and 4 % slower.
+constexpr int NARROW_ROWS = 64, NARROW_RING2 = 2, NARROW_RING1 = 4;
 template <int RB, int RING>
-__device__ __forceinline__ void narrow_products(const uint8_t* w, const uint8_t* a, size_t rbs, int units, int unit0, int shift, int lane,
-                                                float16v (&acc)[2][2]) {
+__device__ __forceinline__ void narrow_products(__amdgpu_buffer_rsrc_t w0, __amdgpu_buffer_rsrc_t w1, __amdgpu_buffer_rsrc_t a, uint32_t rbs, int units,
+                                                int unit0, const int (&shift)[2], int lane, float16v (&acc)[2][2][2]) {
     struct Piece {
-        u32x4 q, a[2][RB];
-        uint32_t e;
+        u32x4 q[2], a[2][RB];
+        uint32_t e[2];
     } r[RING];
     const int last = unit0 + units - 1;
     auto load = [&](Piece& p, int u) {
         u = min(u, last);
-        const uint8_t* t = w + (size_t)(u >> 3) * PromptMx::TILE_BYTES;
-        const uint8_t* x = a + (size_t)u * 2048;
+        const uint32_t t = (u >> 3) * PromptMx::TILE_BYTES, qa = t + (u & 7) * 1024, ea = t + 8192 + (u & 7);
         __builtin_amdgcn_sched_barrier(0);
-        p.q = *(const u32x4*)(t + ((u & 7) * 64 + lane) * 16);
-        p.e = t[8192 + lane * 8 + (u & 7)];
+        p.q[0] = load16(w0, lane * 16, qa);
+        p.q[1] = load16(w1, lane * 16, qa);
+        p.e[0] = __builtin_amdgcn_raw_buffer_load_b8(w0, lane * 8, ea, 0);
+        p.e[1] = __builtin_amdgcn_raw_buffer_load_b8(w1, lane * 8, ea, 0);
 #pragma unroll
         for (int q = 0; q < 2; q++)
 #pragma unroll
-            for (int b = 0; b < RB; b++) p.a[q][b] = *(const u32x4*)(x + b * rbs + q * 1024);
+            for (int b = 0; b < RB; b++) p.a[q][b] = load16(a, lane * 16 + b * rbs, u * 2048 + q * 1024);
         __builtin_amdgcn_sched_barrier(0);
     };
     auto multiply = [&](const Piece& p) {
-        const float sc = __uint_as_float((uint32_t)min(max((int)p.e + shift, 1), 254) << 23);
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            u32x4 b[2];
-            const uint32_t lo = p.q[2 * q], hi = p.q[2 * q + 1];
-            auto put = [&](int i, auto l, auto h) {
-                const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, l), __builtin_bit_cast(uint32_t, h), false, false);
-                b[0][i] = t[0];
-                b[1][i] = t[1];
-            };
-            put(0, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 0));
-            put(1, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 1), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 1));
-            put(2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 2), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 2));
-            put(3, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 3), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 3));
+        for (int q = 0; q < 2; q++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int c = 0; c < 2; c++) {
+                const float sc = __uint_as_float((uint32_t)min(max((int)p.e[c] + shift[c], 1), 254) << 23);
+                u32x4 b[2];
+                const uint32_t lo = p.q[c][2 * q], hi = p.q[c][2 * q + 1];
+                auto put = [&](int i, auto l, auto h) {
+                    const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, l), __builtin_bit_cast(uint32_t, h), false, false);
+                    b[0][i] = t[0];
+                    b[1][i] = t[1];
+                };
+                put(0, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 0));
+                put(1, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 1), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 1));
+                put(2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 2), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 2));
+                put(3, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(lo, sc, 3), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(hi, sc, 3));
 #pragma unroll
-                for (int t = 0; t < RB; t++)
-                    acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, p.a[q][t]), __builtin_bit_cast(half8, b[j]), acc[t][j], 0, 0, 0);
-        }
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int t = 0; t < RB; t++)
+                        acc[c][t][j] =
+                            __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, p.a[q][t]), __builtin_bit_cast(half8, b[j]), acc[c][t][j], 0, 0, 0);
+            }
     };
 #pragma unroll
     for (int i = 0; i < RING - 1; i++) load(r[i], unit0 + i);
@@ -761,92 +771,107 @@ __device__ __forceinline__ void narrow_products(const uint8_t* w, const uint8_t*
 }
 
 template <int EPI>
-__global__ __launch_bounds__(256, 3) void k_prompt_experts_narrow(PromptGemmArgs g) {
+__global__ __launch_bounds__(256, 2) void k_prompt_experts_narrow(PromptGemmArgs g) {
     __shared__ __attribute__((aligned(16))) float meet[4 * 3 * 16 * 64];  // [reader][the other waves][values][lanes]
-    __shared__ float factor[64];
+    __shared__ float factor[128];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // XCD x takes the row tiles x, x + 8, ..., all columns of one before the next
-    const int slot = blockIdx.x >> 3, mb = slot / g.n_tiles * 8 + (blockIdx.x & 7), nb = slot % g.n_tiles;
+    const int slot = blockIdx.x >> 3, mb = slot / g.nt * 8 + (blockIdx.x & 7), nb0 = slot % g.nt * 2;
     if (mb >= *g.tile_count) return;
-    const PromptTile t = g.tiles[mb];
-    const int tile = t.expert * g.n_tiles + nb;
-    const float rs = g.rs[tile * 64 + lane];
-    if (wave == 0) factor[lane] = 1.0f / rs;
-    float16v acc[2][2];
+    const PromptTile t = uniform_tile(g.tiles[mb]);
+    const int columns = min(2, g.n_tiles - nb0);  // (an odd count: the last workgroup's second half repeats the last tile, and leaves nothing)
+    int shift[2];
+    const size_t tile_bytes = (size_t)g.kchunks * PromptMx::TILE_BYTES;
+    const uint8_t* const w = g.w + ((size_t)t.expert * g.n_tiles + nb0) * tile_bytes;
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+    for (int c = 0; c < 2; c++) {
+        const float rs = g.rs[(t.expert * g.n_tiles + nb0 + min(c, columns - 1)) * 64 + lane];
+        if (wave == 0) factor[c * 64 + lane] = 1.0f / rs;
+        shift[c] = (int)(__float_as_uint(rs) >> 23) - 127;
+    }
+    float16v acc[2][2][2];
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+    for (int c = 0; c < 2; c++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[b][j][i] = 0.f;
-    const uint8_t* const w = g.w + (size_t)tile * g.kchunks * PromptMx::TILE_BYTES;
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[c][b][j][i] = 0.f;
     const size_t rbs = (size_t)g.a_k16 * 1024;
-    const uint8_t* const a = g.a + (size_t)(t.first >> 5) * rbs + lane * 16;
-    const int units = 2 * g.kchunks, shift = (int)(__float_as_uint(rs) >> 23) - 127;
-    if (t.cnt > 32) narrow_products<2, 3>(w, a, rbs, units, wave * units, shift, lane, acc);
-    else narrow_products<1, 5>(w, a, rbs, units, wave * units, shift, lane, acc);
-    // wave d ends with registers 4 d .. 4 d + 3 of all four blocks: rows 8 d + 4 (lane / 32) + i of both row blocks, column lane % 32
-    // of both column blocks.  Summed in the order of K.
-    float mine[16];
+    const __amdgpu_buffer_rsrc_t w0 = buffer_of(w, tile_bytes), w1 = buffer_of(w + (columns - 1) * tile_bytes, tile_bytes),
+                                 a = buffer_of(g.a + (size_t)(t.first >> 5) * rbs, (t.cnt > 32 ? 2 : 1) * rbs);
+    const int units = 2 * g.kchunks;
+    if (t.cnt > 32) narrow_products<2, NARROW_RING2>(w0, w1, a, rbs, units, wave * units, shift, lane, acc);
+    else narrow_products<1, NARROW_RING1>(w0, w1, a, rbs, units, wave * units, shift, lane, acc);
 #pragma unroll
-    for (int d = 0; d < 4; d++) {
-        if (wave == d) {
+    for (int c = 0; c < 2; c++) {
+        const int nb = nb0 + c;
+        if (c >= columns) break;
+        if (c) __syncthreads();  // (what the first tile left in `meet` has been read)
+        // wave d ends with registers 4 d .. 4 d + 3 of all four blocks: rows 8 d + 4 (lane / 32) + i of both row blocks, column lane % 32
+        // of both column blocks.  Summed in the order of K.
+        float mine[16];
 #pragma unroll
-            for (int v = 0; v < 16; v++) mine[v] = acc[v >> 3][(v >> 2) & 1][4 * d + (v & 3)];
-        } else {
-            float* o = meet + (size_t)(d * 3 + (wave < d ? wave : wave - 1)) * 1024 + lane;
+        for (int d = 0; d < 4; d++) {
+            if (wave == d) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) o[v * 64] = acc[v >> 3][(v >> 2) & 1][4 * d + (v & 3)];
+                for (int v = 0; v < 16; v++) mine[v] = acc[c][v >> 3][(v >> 2) & 1][4 * d + (v & 3)];
+            } else {
+                float* o = meet + (size_t)(d * 3 + (wave < d ? wave : wave - 1)) * 1024 + lane;
+#pragma unroll
+                for (int v = 0; v < 16; v++) o[v * 64] = acc[c][v >> 3][(v >> 2) & 1][4 * d + (v & 3)];
+            }
         }
-    }
-    __syncthreads();
-    const float* in = meet + (size_t)wave * 3 * 1024 + lane;
-    const float f0 = factor[lane & 31], f1 = factor[32 + (lane & 31)];
-    float sum[16];
+        __syncthreads();
+        const float* in = meet + (size_t)wave * 3 * 1024 + lane;
+        const float f0 = factor[c * 64 + (lane & 31)], f1 = factor[c * 64 + 32 + (lane & 31)];
+        float sum[16];
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        float x = 0.f;
+        for (int v = 0; v < 16; v++) {
+            float x = 0.f;
 #pragma unroll
-        for (int k = 0; k < 4; k++) x += k == wave ? mine[v] : in[((k < wave ? k : k == wave ? 0 : k - 1) * 16 + v) * 64];
-        sum[v] = x * ((v >> 2) & 1 ? f1 : f0);
-    }
-    if (EPI == EPI_PARTIAL) {
-        float* const out = (float*)g.out;
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int col = nb * 64 + 32 * j + (lane & 31);
-            if (col >= g.n_valid) continue;
-            const float bias = g.bias ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int local = 32 * b + 8 * wave + 4 * (lane >> 5) + i;
-                    if (local >= t.cnt) continue;
-                    const int pr = g.pair[t.first + local], row = pr >> 3;
-                    out[((size_t)(row >> 4) * 128 + (pr & 7) * 16 + (row & 15)) * g.ldo + col] = sum[b * 8 + j * 4 + i] + bias;
-                }
+            for (int k = 0; k < 4; k++) x += k == wave ? mine[v] : in[((k < wave ? k : k == wave ? 0 : k - 1) * 16 + v) * 64];
+            sum[v] = x * ((v >> 2) & 1 ? f1 : f0);
         }
-        return;
-    }
-    // 32 gate columns and the matching up columns; the products go through LDS into the order of the next matmul's activations
-    __syncthreads();
-    _Float16* const act = (_Float16*)meet;
-    const int c = lane & 31, col = nb * 32 + c;
-    const float bg = g.bias && col < g.n_valid ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
-    const float bu = g.bias2 && col < g.n_valid ? g.bias2[(size_t)t.expert * g.n_valid + col] : 0.f;
+        if (EPI == EPI_PARTIAL) {
+            float* const out = (float*)g.out;
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+            for (int j = 0; j < 2; j++) {
+                const int col = nb * 64 + 32 * j + (lane & 31);
+                if (col >= g.n_valid) continue;
+                const float bias = g.bias ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = 8 * wave + 4 * (lane >> 5) + i;
-            act[(((b * 2 + (c >> 4)) * 2 + ((c >> 3) & 1)) * 32 + row) * 8 + (c & 4) + (((c & 1) << 1) | ((c >> 1) & 1))] =
-                (_Float16)gated(sum[b * 8 + i] + bg, sum[b * 8 + 4 + i] + bu, g.alpha, g.limit);
+                for (int b = 0; b < 2; b++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int local = 32 * b + 8 * wave + 4 * (lane >> 5) + i;
+                        if (local >= t.cnt) continue;
+                        const int pr = g.pair[t.first + local], row = pr >> 3;
+                        out[((size_t)(row >> 4) * 128 + (pr & 7) * 16 + (row & 15)) * g.ldo + col] = sum[b * 8 + j * 4 + i] + bias;
+                    }
+            }
+            continue;
         }
-    __syncthreads();
-    const int p = threadIdx.x, b = p >> 7, k16 = nb * 2 + ((p >> 6) & 1);
-    if (k16 * 16 < g.n_valid && b * 32 < t.cnt)
-        *(u32x4*)((uint8_t*)g.out + (((size_t)((t.first >> 5) + b) * g.out_k16 + k16) * 64 + (p & 63)) * 16) = ((const u32x4*)meet)[p];
+        // 32 gate columns and the matching up columns; the products go through LDS into the order of the next matmul's activations
+        __syncthreads();
+        _Float16* const act = (_Float16*)meet;
+        const int cc = lane & 31, col = nb * 32 + cc;
+        const float bg = g.bias && col < g.n_valid ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
+        const float bu = g.bias2 && col < g.n_valid ? g.bias2[(size_t)t.expert * g.n_valid + col] : 0.f;
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int row = 8 * wave + 4 * (lane >> 5) + i;
+                act[(((b * 2 + (cc >> 4)) * 2 + ((cc >> 3) & 1)) * 32 + row) * 8 + (cc & 4) + (((cc & 1) << 1) | ((cc >> 1) & 1))] =
+                    (_Float16)gated(sum[b * 8 + i] + bg, sum[b * 8 + 4 + i] + bu, g.alpha, g.limit);
+            }
+        __syncthreads();
+        const int p = threadIdx.x, b = p >> 7, k16 = nb * 2 + ((p >> 6) & 1);
+        if (k16 * 16 < g.n_valid && b * 32 < t.cnt)
+            *(u32x4*)((uint8_t*)g.out + (((size_t)((t.first >> 5) + b) * g.out_k16 + k16) * 64 + (p & 63)) * 16) = ((const u32x4*)meet)[p];
+    }
 }
 
 // ---- row factors ----------------------------------------------------------------------------------------------------------
@@ -1072,7 +1097,7 @@ int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const v
     g.alpha = epi == EPI_SILU ? x.alpha : 0.f;
     g.limit = x.limit;
     if (w.fmt == FMT_MX4 && x.bm == NARROW_ROWS && !out_sum) {
-        const dim3 grid((x.max_tiles + 7) / 8 * 8 * g.n_tiles);
+        const dim3 grid((x.max_tiles + 7) / 8 * 8 * g.nt);
         if (epi == EPI_SILU) hipLaunchKernelGGL(k_prompt_experts_narrow<EPI_SILU>, grid, dim3(256), 0, s, g);
         else hipLaunchKernelGGL(k_prompt_experts_narrow<EPI_PARTIAL>, grid, dim3(256), 0, s, g);
         TSV_HIP(hipGetLastError());

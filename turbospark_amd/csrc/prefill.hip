@@ -178,7 +178,7 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
         PromptExperts x{};
         x.routes = PromptRoutes{w.pair, w.tiles, w.n_tiles};
         x.n_experts = L.n_experts;
-        x.bm = prompt_expert_rows(n, L.top_k, L.n_experts);
+        x.bm = prompt_expert_rows(n, L.top_k, L.n_experts, L.gate_up.fmt == FMT_MX4 && L.down.fmt == FMT_MX4);
         x.max_tiles = prompt_max_tiles(n, L.top_k, L.n_experts, x.bm);
         x.bias = L.be_gate;
         x.bias2 = L.be_up;

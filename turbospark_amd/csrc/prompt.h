@@ -43,19 +43,20 @@ struct PromptRoutes {
     int32_t* n_tiles;    // device count
 };
 __host__ __device__ inline int prompt_sorted_rows(int n, int top_k, int n_experts) { return n * top_k + 31 * n_experts; }
-// Rows of an expert tile.  Two layers, whole prompts, us (n rows of them to the average expert):
-//   MXFP4, 128 experts of 768 x 2048          n = 62     96    128;  64 experts  192    256;  32 of 2880 x 2880  96    128    256
-//   64 rows in the narrow kernel                  927   1204   1544               1115   1427                    1023   1191   1938
-//   64 / 128 / 256 in k_prompt_gemm, 64          1128   1467   1855               1348   1722                    1342   1550   2549
-//                                   128          1051   1341   1689               1225   1531                    1139   1349   2115
-//                                   256          1070   1332   1669               1242   1531                    1210   1370   2215
-//   Q4_K, 128 experts of 768 x 2048, 19 / 62 / 96 / 128 rows: 64-row tiles 734 / 1190 / 1555 / 1945, 128 749 / 1119 / 1421 / 1747,
-//   256 769 / 1152 / 1471 / 1747
-// So the narrow kernel earns its 96 rows and would earn more; Q4_K takes 128 better from somewhere between 19 and 62 rows on; 256 against 128 is
-// within 5 % either way.
-inline int prompt_expert_rows(int n, int top_k, int n_experts) {
+// Rows of an expert tile; narrow: both of the expert's matrices go through k_prompt_experts_narrow, which takes tiles of 64.  Two
+// layers, whole prompts, us (n rows of them to the average expert):
+//   MXFP4, 128 experts of 768 x 2048    n = 18     38     62     96    128;  64 experts  192    256
+//   64 rows in the narrow kernel           551    715    955   1302   1645              1254   1589
+//   128 in k_prompt_gemm                   709    816   1046   1349   1742              1290   1619
+//   256                                    693    821   1052   1364   1785              1274   1626
+//   Q4_K, 128 experts of 768 x 2048,  64:  723    872   1191   1625   2051
+//                                    128:  716    862   1156   1470   1879
+//                                    256:  734    872   1151   1523   1984
+// 256 is as far as a pass of 2048 rows gets with eight of 64 experts; beyond, and for other formats beyond 192, tiles of 256 save
+// unpacking.
+inline int prompt_expert_rows(int n, int top_k, int n_experts, bool narrow) {
     const int avg = n * top_k / n_experts;
-    return avg <= 96 ? 64 : avg <= 192 ? 128 : 256;
+    return narrow && avg <= 256 ? 64 : !narrow && avg <= 192 ? 128 : 256;
 }
 inline int prompt_max_tiles(int n, int top_k, int n_experts, int bm) { return n * top_k / bm + n_experts; }
 // selected: [n][8], rank order
