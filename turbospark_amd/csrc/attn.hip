@@ -37,7 +37,7 @@ int attn_chunks(int nkv) {
 // Eight waves per workgroup share a chunk of the context (attn_core.h).
 template <int HD, int RT, int STAGES>
 __global__ __launch_bounds__(512) void k_attn_partial(AttnArgs a, int G, int R) {
-    extern __shared__ float xch[];  // [4 slots][PER_LANE values][64 lanes]
+    extern __shared__ float xch[];  // [8 slots][PER_LANE values][64 lanes]
     if (a.xcd_groups) {  // several row groups of a verify pass: placed by die
         int chunk, kvh, grp;
         if (attn_grid_place(a, blockIdx.x, chunk, kvh, grp)) attn_partial_body<HD, RT, STAGES, false>(a, G, R, chunk, kvh, grp * RT, xch);
@@ -173,11 +173,10 @@ __global__ void k_attn_combine(AttnArgs a0, int G, int R) {
 template <int HD, int RT, int STAGES>
 static int launch_partial(hipStream_t s, const AttnArgs& a, int G, int R, int groups) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT;
-    const size_t lds = (size_t)4 * 64 * PER_LANE * 4;
+    constexpr size_t lds = (size_t)8 * 64 * PER_LANE * 4;
     static bool raised = false;  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
     if (lds > 65536 && !raised) {
-        TSV_HIP(hipFuncSetAttribute((const void*)k_attn_partial<HD, RT, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds));
+        TSV_HIP(hipFuncSetAttribute((const void*)k_attn_partial<HD, RT, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         raised = true;
     }
     const dim3 grid = a.xcd_groups ? dim3(attn_grid_size(a.nch * a.nkv, groups)) : dim3(a.nch, a.nkv, groups * std::max(a.blocks, 1));
@@ -188,8 +187,8 @@ static int launch_partial(hipStream_t s, const AttnArgs& a, int G, int R, int gr
 
 template <int HD, int RT, int STAGES, int TG>
 static int launch_partial_groups(hipStream_t s, const AttnArgs& a, int G, int R) {
-    constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT, NW = attn_phases(TG), SLOTS = NW < 4 ? NW : 4;
-    const size_t lds = (size_t)TG * SLOTS * 64 * PER_LANE * 4;
+    constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT, NW = attn_phases(TG);
+    const size_t lds = (size_t)TG * NW * 64 * PER_LANE * 4;
     static bool raised = false;  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
     if (lds > 65536 && !raised) {
         TSV_HIP(hipFuncSetAttribute((const void*)k_attn_partial_groups<HD, RT, STAGES, TG>,
@@ -208,7 +207,7 @@ static int launch_combine(hipStream_t s, const AttnArgs& a, int m, int G, int R)
 template <int HD, int RT, int KB, int VB>
 static int launch_partial_tq(hipStream_t s, const AttnArgs& a, int G, int R, int groups) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT;
-    const size_t lds = (size_t)4 * 64 * PER_LANE * 4;
+    const size_t lds = (size_t)8 * 64 * PER_LANE * 4;
     static bool raised = false;
     if (lds > 60000 && !raised) {  // with the pair tables beside it the exchange area passes 64 KiB
         TSV_HIP(hipFuncSetAttribute((const void*)k_attn_partial_tq<HD, RT, KB, VB>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -239,6 +238,17 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
     // about one workgroup per compute unit: the chunk count shrinks as the row groups multiply
     // (fewer, longer chunks also mean fewer partial results for the merge to read)
     AttnArgs a = a0;
+    // A short context in one workgroup per KV head and row group, up to DIRECT_BLOCKS / 8 blocks a wave, which finishes its rows itself:
+    // DIRECT_NOTE
+    // Layers of a short window always do (a window's blocks: its own, the pass's, one cut).  All row groups take the form of eight
+    // phases here, so that a row's sums run in one order whatever shares its pass.
+    const bool few = attn_short(a.kv_end) || (a.window > 0 && (a.window + TSV_MAX_ROWS + 14) / 16 + 1 <= ATTN_DIRECT_BLOCKS);
+    if (a.kv_end > 0 && a.blocks <= 1 && !a.tq.k_bits && !a.frag16 && few) {
+        a.direct = a.nch = 1;
+        a.xcd_groups = 0;
+        return trt <= 1 ? launch_partial<HD, 1, 3>(s, a, G, R, 1)
+                        : launch_partial<HD, 2, (HD == 128 ? TSV_ATTN_STAGES2_HD128 : TSV_ATTN_STAGES2_HD64)>(s, a, G, R, groups);
+    }
     a.nch = std::max(std::min(a0.nch, 8), std::min(a0.nch, 256 / (a0.nkv * groups * std::max(a0.blocks, 1))));
     // Several row groups of a verify pass read the same K / V: they are placed on one die.  A workgroup fills a
     // compute unit (eight waves at two per SIMD) and a die has 32 of them: no die may be handed more than 32

@@ -19,28 +19,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // left to itself the compiler contracts a * b + c * d one way in one template instantiation and the
 // other way in the next, and a row's bits would then depend on how many rows share its pass.
 //
-// One (m, l, O) running state merged into another (flash-decoding rescale).
-// (BASE2: the maxima are kept in units of log 2, the weights are powers of two)
-template <int RT, int VT, bool BASE2 = false>
-__device__ __forceinline__ void merge_state(float (&mrun)[RT], float (&lrun)[RT], float4v (&O)[RT][VT], const float* src) {
-    // `src` points at this lane's column of a [values][64 lanes] slot: consecutive lanes touch
-    // consecutive LDS banks
-#pragma unroll
-    for (int t = 0; t < RT; t++) {
-        const float m1 = src[64 * (2 * t)], l1 = src[64 * (2 * t + 1)];
-        const float mnew = fmaxf(mrun[t], m1);
-        if (mnew > -INFINITY) {
-            const float a0 = BASE2 ? __builtin_amdgcn_exp2f(mrun[t] - mnew) : __expf(mrun[t] - mnew);
-            const float a1 = BASE2 ? __builtin_amdgcn_exp2f(m1 - mnew) : __expf(m1 - mnew);
-            lrun[t] = fmaf(lrun[t], a0, l1 * a1);
-#pragma unroll
-            for (int d = 0; d < VT; d++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) O[t][d][i] = fmaf(O[t][d][i], a0, src[64 * (2 * RT + (t * VT + d) * 4 + i)] * a1);
-            mrun[t] = mnew;
-        }
-    }
-}
+// One wave's (m, l, O) running state into its slot of the LDS, [values][64 lanes]: consecutive lanes touch consecutive banks
 template <int RT, int VT>
 __device__ __forceinline__ void store_state(const float (&mrun)[RT], const float (&lrun)[RT], const float4v (&O)[RT][VT],
                                             float* dst) {
@@ -52,6 +31,77 @@ __device__ __forceinline__ void store_state(const float (&mrun)[RT], const float
         for (int d = 0; d < VT; d++)
 #pragma unroll
             for (int i = 0; i < 4; i++) dst[64 * (2 * RT + (t * VT + d) * 4 + i)] = O[t][d][i];
+    }
+}
+
+// The running (m, l, O) of the NW waves of a tile group put together, and the chunk's partial results or, of the only chunk, the finished
+// rows written.
+// Every wave of the group leaves its state in LDS and then puts 32 dims of one row tile together: one barrier and eight waves at
+// work, where folding the states into one wave's, four to a barrier, ended with that wave going through 64 values of each alone
+// (8B shape, a layer's pass at 60 positions, attention in one chunk: 68.9 -> 65.4 us with five rows, 82.7 -> 78.7 with sixteen).
+// (BASE2: the maxima are kept in units of log 2, the weights are powers of two.)  grp: the group's slots, from this lane's column on.
+template <int HD, int RT, int NW, bool BASE2>
+__device__ __forceinline__ void attn_finish(const AttnArgs& a, int G, int R, int chunk, int h, int rt0, int wave, int lane, float* grp,
+                                            const float (&mrun)[RT], const float (&lrun)[RT], const float4v (&O)[RT][HD / 16]) {
+    constexpr int VT = HD / 16, PER_LANE = RT * VT * 4 + 2 * RT;
+    const int j = lane & 15, kg = lane >> 4;
+    store_state<RT, VT>(mrun, lrun, O, grp + wave * 64 * PER_LANE);
+    __syncthreads();
+    for (int job = wave; job < RT * (VT / 2); job += NW) {
+        const int t = job / (VT / 2), u = job % (VT / 2);
+        const int r = (rt0 + t) * 16 + j;
+        float wgt[NW], l = 0.f, top = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < NW; k++) wgt[k] = grp[(k * PER_LANE + 2 * t) * 64];
+#pragma unroll
+        for (int k = 0; k < NW; k++) top = fmaxf(top, wgt[k]);
+        const float ref = fmaxf(top, -3.0e38f);  // (a chunk none of whose positions the row sees: weights of zero)
+#pragma unroll
+        for (int k = 0; k < NW; k++) {
+            wgt[k] = BASE2 ? __builtin_amdgcn_exp2f(wgt[k] - ref) : __expf(wgt[k] - ref);
+            l = fmaf(grp[(k * PER_LANE + 2 * t + 1) * 64], wgt[k], l);
+        }
+        float o[2][4];
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                o[e][i] = 0.f;
+#pragma unroll
+                for (int k = 0; k < NW; k++) o[e][i] = fmaf(grp[(k * PER_LANE + 2 * RT + (t * VT + 2 * u + e) * 4 + i) * 64], wgt[k], o[e][i]);
+            }
+        l += __shfl_xor(l, 16);
+        l += __shfl_xor(l, 32);
+        if (!a.direct) {
+            if (r >= R) continue;
+            const long slot = ((long)h * a.nch + chunk) * R + r;
+            if (kg == 0 && u == 0) {
+                a.part_ml[slot * 2] = BASE2 ? top * 0.69314718055994530942f : top;  // the merge works with natural logarithms
+                a.part_ml[slot * 2 + 1] = l;
+            }
+#pragma unroll
+            for (int e = 0; e < 2; e++) *(float4v*)(a.part_o + slot * HD + 16 * (2 * u + e) + 4 * kg) = float4v{o[e][0], o[e][1], o[e][2], o[e][3]};
+            continue;
+        }
+        // the only chunk: what the merge would make of it (attn.hip)
+        const int m = min(r, R - 1) / G, qh = h * G + min(r, R - 1) % G;
+        const float mx = BASE2 ? ref * 0.69314718055994530942f : ref, sink = a.sinks ? a.sinks[qh] : -INFINITY, over = fmaxf(mx, sink);
+        const float w = __expf(mx - over);
+        const float den = a.sinks ? fmaf(l, w, __expf(sink - over)) : l * w;
+        const float inv = w / den;
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            // (the sums have to be those of the stored bits: pinned_half)
+            const _Float16 h0 = pinned_half((_Float16)(o[e][0] * inv)), h1 = pinned_half((_Float16)(o[e][1] * inv)),
+                           h2 = pinned_half((_Float16)(o[e][2] * inv)), h3 = pinned_half((_Float16)(o[e][3] * inv));
+            const int kk = qh * HD + 16 * (2 * u + e) + 4 * kg;
+            if (r < R) *(half4*)((_Float16*)a.xfrag + frag_index(kk, m)) = half4{h0, h2, h1, h3};
+            sum += ((float)h0 + (float)h1) + ((float)h2 + (float)h3);
+        }
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if (r < R && kg == 0) ((float*)((char*)a.xfrag + xfrag_sum_offset(a.nq * HD)))[xsum_index((qh * HD >> 5) + u, m)] = sum;
     }
 }
 
@@ -81,7 +131,7 @@ __device__ __forceinline__ float max_over_position_groups(float v) {
 // once for all (row, q head) pairs of the pass.  (Legacy callers pass TG = 1 and their own rt0: eight waves, one group.)
 // COH: the query rows and the K / V blocks are read device-coherently (sc1), for a caller whose
 // other compute units wrote them earlier in the same kernel.
-// xch: [TG][min(NW, 4) slots][PER_LANE values][64 lanes] floats of LDS.
+// xch: [TG][NW slots][PER_LANE values][64 lanes] floats of LDS.
 __host__ __device__ constexpr int attn_phases(int tg) { return tg == 1 ? 8 : tg == 2 ? 4 : 2; }
 
 template <int HD, int RT, int STAGES, bool COH, int TG = 1>
@@ -298,35 +348,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
             if (i + s < nb) consume(st[s], i + s);
     }
 
-    // fold the group's running (m, l, O): with eight phases 4..7 into 0..3 first, then 1.. into 0
-    constexpr int SLOTS = NW < 4 ? NW : 4;
-    float* grp = xch + tg * SLOTS * 64 * PER_LANE + lane;
-    if (NW == 8) {
-        if (wave >= 4) store_state<RT, VT>(mrun, lrun, O, grp + (wave & 3) * 64 * PER_LANE);
-        __syncthreads();
-        if (wave < 4) merge_state<RT, VT, true>(mrun, lrun, O, grp + wave * 64 * PER_LANE);
-        __syncthreads();
-    }
-    if (wave >= 1 && wave < 4) store_state<RT, VT>(mrun, lrun, O, grp + wave * 64 * PER_LANE);
-    __syncthreads();
-    if (wave != 0) return;
-    for (int w = 1; w < SLOTS; w++) merge_state<RT, VT, true>(mrun, lrun, O, grp + w * 64 * PER_LANE);
-#pragma unroll
-    for (int t = 0; t < RT; t++) {
-        float l = lrun[t];
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
-        const int r = (rt0 + t) * 16 + j;
-        if (r >= R) continue;
-        const long slot = ((long)h * a.nch + chunk) * R + r;
-        if (kg == 0) {
-            a.part_ml[slot * 2] = mrun[t] * 0.69314718055994530942f;  // the merge works with natural logarithms
-            a.part_ml[slot * 2 + 1] = l;
-        }
-        float* o = a.part_o + slot * HD + 4 * kg;
-#pragma unroll
-        for (int d = 0; d < VT; d++) *(float4v*)(o + 16 * d) = O[t][d];
-    }
+    attn_finish<HD, RT, NW, true>(a, G, R, chunk, h, rt0, wave, lane, xch + tg * NW * 64 * PER_LANE + lane, mrun, lrun, O);
 }
 
 }  // namespace tsv

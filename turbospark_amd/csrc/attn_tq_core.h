@@ -35,7 +35,7 @@ __device__ __forceinline__ void tq_fill_pairs(uint32_t* table, const float* cb, 
     }
 }
 
-// xch: [4 slots][PER_LANE values][64 lanes] floats of LDS; kpair / vpair: the two pair tables
+// xch: [8 slots][PER_LANE values][64 lanes] floats of LDS; kpair / vpair: the two pair tables
 template <int HD, int RT, int STAGES, int KB, int VB>
 __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, int R, int chunk, int h, int rt0, float* xch,
                                                      const uint32_t* kpair, const uint32_t* vpair) {
@@ -225,32 +225,7 @@ __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, i
             if (i + s < nb) consume(st[s], i + s);
     }
 
-    // fold the eight waves' running (m, l, O): 4..7 into 0..3, then 1..3 into 0
-    float* mine = xch + (wave & 3) * 64 * PER_LANE + lane;
-    if (wave >= 4) store_state<RT, VT>(mrun, lrun, O, mine);
-    __syncthreads();
-    if (wave < 4) merge_state<RT, VT>(mrun, lrun, O, mine);
-    __syncthreads();
-    if (wave >= 1 && wave < 4) store_state<RT, VT>(mrun, lrun, O, mine);
-    __syncthreads();
-    if (wave != 0) return;
-    for (int w = 1; w < 4; w++) merge_state<RT, VT>(mrun, lrun, O, xch + w * 64 * PER_LANE + lane);
-#pragma unroll
-    for (int t = 0; t < RT; t++) {
-        float l = lrun[t];
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
-        const int r = (rt0 + t) * 16 + j;
-        if (r >= R) continue;
-        const long slot = ((long)h * a.nch + chunk) * R + r;
-        if (kg == 0) {
-            a.part_ml[slot * 2] = mrun[t];
-            a.part_ml[slot * 2 + 1] = l;
-        }
-        float* o = a.part_o + slot * HD + 4 * kg;
-#pragma unroll
-        for (int d = 0; d < VT; d++) *(float4v*)(o + 16 * d) = O[t][d];
-    }
+    attn_finish<HD, RT, 8, false>(a, G, R, chunk, h, rt0, wave, lane, xch + lane, mrun, lrun, O);
 }
 
 }  // namespace tsv

@@ -189,7 +189,7 @@ struct tsv_ctx {
     // the GPU-side cost of ~290 dependent kernels, not by host launch time, and replay measured
     // the same step time as plain stream launches.
     bool use_graph = false;
-    hipGraphExec_t pass_graph[TSV_MAX_ROWS + 1] = {};
+    hipGraphExec_t pass_graph[2][TSV_MAX_ROWS + 1] = {};  // [attn_short][rows]
     // per-kernel-class timing (tsv_set_profile): one event pair per launch
     bool profile = false;
     int repeat[TSV_PROFILE_CLASSES] = {1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1};  // tsv_set_repeat

@@ -457,6 +457,7 @@ int launch_pass(tsv_ctx* c, int m) {
         aa.vp = c->vp_dev;
         aa.m_hint = m;
         aa.base_hint = c->use_graph ? -1 : c->vp_host->base;  // a captured launch must read the position at replay
+        aa.kv_end = c->vp_host->base + m;
         {
             PROF(PC_ATTN);
             rc = 0;
@@ -910,7 +911,8 @@ int enqueue_wide_prefill(tsv_ctx* c, const int32_t* ids, int64_t base) {
 
 int run_pass(tsv_ctx* c, int m) {
     if (!c->use_graph || c->profile || c->headless || c->mtp.on) return launch_pass(c, m);
-    if (!c->pass_graph[m]) {
+    hipGraphExec_t& graph = c->pass_graph[attn_short(c->vp_host->base + m)][m];
+    if (!graph) {
         hipGraph_t g = nullptr;
         TSV_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         const int rc = launch_pass(c, m);
@@ -920,15 +922,15 @@ int run_pass(tsv_ctx* c, int m) {
             if (!rc) set_error(std::string("verify: graph capture failed: ") + hipGetErrorString(e));
             return rc ? rc : TSV_ERR_DEVICE;
         }
-        const hipError_t ei = hipGraphInstantiate(&c->pass_graph[m], g, nullptr, nullptr, 0);
+        const hipError_t ei = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (ei != hipSuccess) {
-            c->pass_graph[m] = nullptr;
+            graph = nullptr;
             set_error(std::string("verify: graph instantiation failed: ") + hipGetErrorString(ei));
             return TSV_ERR_DEVICE;
         }
     }
-    TSV_HIP(hipGraphLaunch(c->pass_graph[m], c->stream));
+    TSV_HIP(hipGraphLaunch(graph, c->stream));
     return TSV_OK;
 }
 
@@ -1404,8 +1406,9 @@ extern "C" void tsv_close(tsv_ctx* c) {
     if (c->mtp.draw_host) (void)hipHostFree(c->mtp.draw_host);
     if (c->mtp.vp_block_host) (void)hipHostFree(c->mtp.vp_block_host);
     if (c->mtp.on && c->mtp.target && c->mtp.target->mtp_head == c) c->mtp.target->mtp_head = nullptr;
-    for (hipGraphExec_t g : c->pass_graph)
-        if (g) (void)hipGraphExecDestroy(g);
+    for (auto& graphs : c->pass_graph)
+        for (hipGraphExec_t g : graphs)
+            if (g) (void)hipGraphExecDestroy(g);
     for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
     if (c->stream && c->owns_stream) (void)hipStreamDestroy(c->stream);
     delete c;

@@ -423,6 +423,7 @@ extern "C" int32_t tsv_attention(const uint16_t* q, const uint16_t* k, const uin
         aa.vp = vpd;
         aa.m_hint = m;
         aa.base_hint = (int)base;
+        aa.kv_end = (int)base + m;
         rc = launch_attention(c->stream, aa, m);
     }
     std::vector<uint16_t> frag(xfb / 2);

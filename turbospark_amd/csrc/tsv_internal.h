@@ -374,6 +374,7 @@ struct AttnArgs {
     float* part_ml;  // [nkv][nch][rows][2]
     uint4* xfrag;    // output, K index = qh*hd + d
     int nq, nkv, hd, max_ctx, nch;  // max_ctx: positions the layer's cache holds
+    int direct;          // set by the launcher: nch is 1 and the partial kernel writes the fragments itself, no merge follows
     int ring;            // non-zero: the cache is a ring, position p in slot p % max_ctx (a windowed layer)
     float scale;
     int window;          // 0: full; else a row sees the last `window` positions of its sequence
@@ -382,6 +383,9 @@ struct AttnArgs {
     // row count and base position by value when the launch knows them (saves the kernel one
     // dependent memory round trip before its first K/V load); base_hint < 0: read them from vp
     int m_hint, base_hint;
+    // base + m as the host knows it, also where the kernels read the base from vp (a captured pass: replayed only where attn_short is
+    // what it was at capture); 0: always by chunks
+    int kv_end;
     int frag16;  // write the output fragments in the prompt kernel's layout (frag16_index)
     // nullable: head_dim signs.  The values were summed in a rotated space (a quantized KV layer); the merge
     // applies the normalized Hadamard transform to each head's result and multiplies by these signs
@@ -462,6 +466,9 @@ size_t tq_kq_bytes(int nkv, int cap, int hd, int k_bits);
 size_t tq_vq_bytes(int nkv, int cap, int hd, int v_bits);
 int launch_attention_merge(hipStream_t s, const AttnArgs& a, int m);
 int attn_chunks(int nkv);
+// whether a pass that ends at position `kv_end` attends in one workgroup per KV head and row group (attn.hip)
+constexpr int ATTN_DIRECT_BLOCKS = 48;
+inline bool attn_short(int64_t kv_end) { return kv_end <= 16 * ATTN_DIRECT_BLOCKS; }
 
 int launch_kv_gather(hipStream_t s, uint16_t* const* caches_dev, const int32_t* caps_dev, int n_layers, int nkv, int hd,
                      const int32_t* path_dev, int n, int base);
