@@ -586,3 +586,65 @@ def test_the_reference_runtime_scenarios_for_kv_bits():
     bad = dict(cfg, head_dim=32, n_q_heads=16, n_kv_heads=16)
     with pytest.raises(ts.ffi.TsvError, match="head_dim"):
         ts.HipVerifier(bad, synth.make_weights(bad, seed=9), kv_bits=(4, 4))
+
+
+# pairs (row, q head of the group) around a wave's 32 and a workgroup's 128, blocks of 16 positions begun by the rows before the pass and
+# left unfinished by it, one chunk of the context and several, both head widths
+@pytest.mark.parametrize("nq,nkv,hd,m,base,kb,vb,sinks", [
+    (8, 2, 128, 17, 0, 4, 4, False), (8, 2, 64, 33, 37, 3, 4, False), (32, 8, 128, 65, 300, 4, 4, False), (8, 2, 64, 129, 129, 2, 2, True),
+    (16, 8, 64, 40, 1000, 3, 3, True), (4, 1, 128, 70, 2049, 3, 4, False), (6, 2, 128, 160, 15, 2, 2, False), (4, 4, 64, 31, 1, 4, 4, False)])
+def test_a_prompt_pass_over_quantized_rows(nq, nkv, hd, m, base, kb, vb, sinks):
+    """Its rows as stored, the rows stored before it, and attention over both: against the oracle as a verify pass's above, the rows by
+    bits.  The bound of the output is what fp16 q rows and levels leave: 2^-11 of a level and of q, so 2^-10 of a score of a few
+    units, through the softmax on outputs of which the worst is compared: the verify passes' 4e-3."""
+    from oracle import binding as ob
+    from turbospark_amd import ffi
+    rng = np.random.default_rng(nq * 1000 + base)
+    seq = base + m
+    q = rng.standard_normal((m, nq, hd)).astype(np.float16)
+    k = (rng.standard_normal((seq, nkv, hd)) * rng.uniform(0.2, 3.0, (seq, nkv, 1))).astype(np.float16)
+    v = (rng.standard_normal((seq, nkv, hd)) * rng.uniform(0.2, 3.0, (seq, nkv, 1))).astype(np.float16)
+    k[base + 3], v[base + 4] = 0, 0                    # rows without a direction
+    sk = rng.standard_normal(nq).astype(np.float32) if sinks else None
+    got, kr, vr = ffi.attention_quantized(q, k, v, base, kb, vb, sinks=sk)
+    ks, kc, km, vs, vc, vm = _sides(hd, kb, vb)
+    pick = np.unique(np.concatenate([np.arange(min(seq, 24)), np.arange(max(0, base - 17), min(seq, base + 24)), np.arange(seq - 17, seq)]))
+    _check_rows(k[pick], kr[pick], ks, km, kb)
+    _check_rows(v[pick], vr[pick], vs, vm, vb)
+    worst = 0.0
+    for i in sorted({0, 1, 15, 16, m // 2, m - 2, m - 1}):
+        want = ob.tq_attention(q[i].astype(np.float32), kr[:, :, 1:], kr[:, :, 0].view(np.float32), vr[:, :, 1:],
+                               vr[:, :, 0].view(np.float32), hd, nq, nkv, base + i + 1, kb, ks, kc, vs, vc, sinks=sk,
+                               v_bits=vb).reshape(nq, hd)
+        worst = max(worst, float(np.abs(got[i] - want).max() / np.abs(want).max()))
+    assert worst <= 4e-3
+
+
+@pytest.mark.parametrize("name,kv_bits,n,start", [("small_q4_k", (4, 4), 160, 0), ("xcd_q8_0", (3, 4), 259, 21), ("moe_small", (2, 2), 300, 5)])
+def test_prompts_of_a_quantized_handle_take_prompt_passes(name, kv_bits, n, start):
+    """Against passes of sixteen rows: the first layer's rows (one input, so all but the indices at a midpoint's edge), the rows of
+    the prompt before by bits, logits within the codec's sensitivity (the bounds of the 64-row passes' test)."""
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS[name], max_context=start + n + 48, n_layers=3)
+    w = synth.make_weights(cfg, seed=11)
+    fast, slow = gc.engine(cfg, w, "prompt", kv_bits=kv_bits), gc.engine(cfg, w, "16", kv_bits=kv_bits)
+    rng = np.random.default_rng(n)
+    prompt = rng.integers(0, cfg["vocab"], start + n).astype(np.int32)
+    feed = rng.integers(0, cfg["vocab"], 5).astype(np.int32)
+    out = []
+    for eng in (fast, slow):
+        if start:
+            eng.prefill(prompt[:start], 0, want_logits=False)
+            before = eng.read_kv_quantized(0, 0, start)
+        last = eng.prefill(prompt[start:], start)
+        if start:
+            after = eng.read_kv_quantized(0, 0, start)
+            assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
+        out.append((last, eng.read_kv_quantized(0, start, n), eng.verify(feed, start + n)))
+    assert gc.took(fast, "prompt") and gc.took(slow, "16")
+    for side in (0, 1):
+        a, b = out[0][1][side], out[1][1][side]
+        assert np.mean(_indices(a, kv_bits[side], cfg["head_dim"]) == _indices(b, kv_bits[side], cfg["head_dim"])) >= 0.97
+        assert np.allclose(a[:, :, 0].view(np.float32), b[:, :, 0].view(np.float32), rtol=2e-3)
+    bound = 1.5e-1 if kv_bits == (2, 2) else 5e-2
+    assert gc.logit_error(out[0][0].reshape(1, -1), out[1][0].reshape(1, -1)) <= bound and gc.logit_error(out[0][2], out[1][2]) <= bound

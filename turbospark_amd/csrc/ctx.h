@@ -116,6 +116,7 @@ struct tsv_ctx {
         float2* cs = nullptr;
         int32_t* ids = nullptr;
         float *part_o = nullptr, *part_ml = nullptr;
+        uint16_t *k_levels = nullptr, *v_levels = nullptr;  // quantized layers: the one's rows that attends
         // routed layers: factors and selections of the rows, the sorted pairs and their tiles, the normed rows as plain rows,
         // the pairs' activations before and after gate / up with their sums, the down outputs by slot
         float* route_w = nullptr;

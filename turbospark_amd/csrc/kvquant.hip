@@ -8,6 +8,7 @@
 // the sum is rotated back once with the value signs.  The attention kernel reads the stores directly
 // (attn_tq_core.h, which also states their layout); the merge kernel rotates the result back.
 //
+// A prompt pass quantizes its rows where it rotates them (prompt.hip); what follows is the passes of up to 64 rows.
 // The pass's own rows arrive as fp16 in a small staging cache (the staging row of
 // crates/runtime/src/kv_write.rs:66-118) and are quantized from there: norm as the f32 sum of squares
 // in index order, unit = x * (1 / max(norm, 1e-6)), the butterflies of crates/compute/src/wht.rs:15-29
@@ -19,6 +20,7 @@
 #include <vector>
 
 #include "attn_tq_core.h"
+#include "tq_row.h"
 
 namespace tsv {
 
@@ -128,25 +130,6 @@ __device__ __forceinline__ void lds_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// crates/compute/src/wht.rs:15-29, bottom-up: stage h pairs i with i + h, (lo + hi) and (lo - hi), each
-// scaled by 1/sqrt(2).  Lane l holds elements l and l + 64.
-template <int EPL>
-__device__ __forceinline__ void wht(float (&e)[EPL], int lane, float c) {
-#pragma unroll
-    for (int h = 1; h < 64; h <<= 1) {
-#pragma unroll
-        for (int j = 0; j < EPL; j++) {
-            const float other = __shfl_xor(e[j], h);
-            e[j] = __fmul_rn((lane & h) ? __fsub_rn(other, e[j]) : __fadd_rn(e[j], other), c);
-        }
-    }
-    if (EPL == 2) {
-        const float lo = e[0], hi = e[EPL - 1];
-        e[0] = __fmul_rn(__fadd_rn(lo, hi), c);
-        e[EPL - 1] = __fmul_rn(__fsub_rn(lo, hi), c);
-    }
-}
-
 __device__ __forceinline__ long k_at(int cap, int hd, int head, int pos, int d) { return kcache_index(head, pos, d, hd, cap); }
 __device__ __forceinline__ long v_at(int cap, int hd, int head, int pos, int d) { return vcache_index(head, pos, d, hd, cap); }
 
@@ -201,21 +184,13 @@ __device__ void commit_row(const TqArgs& a, bool value, int pos, int head, int l
 #pragma unroll
     for (int j = 0; j < EPL; j++) e[j] = __fmul_rn(__fmul_rn(x[j], inv), t.signs[lane + 64 * j]);
     wht<EPL>(e, lane, a.inv_sqrt2);
-    const int n_mid = (1 << t.bits) - 1;
-    float mid[15];  // the side's midpoints, +inf past the last: the index is the count of midpoints below the coordinate
-#pragma unroll
-    for (int i = 0; i < 15; i++) {
-        const float v = t.mid[i];  // the table holds sixteen slots
-        mid[i] = i < n_mid ? v : INFINITY;
-    }
+    const TqMidpoints mid(t);
     if (lane == 0) (value ? a.store.vn : a.store.kn)[(long)head * a.cap + pos] = norm;
     if (!value) {
         // a K row: packed LSB first (kv_quant.rs:289-312), assembled in LDS
 #pragma unroll
         for (int j = 0; j < EPL; j++) {
-            uint32_t c = 0;
-#pragma unroll
-            for (int i = 0; i < 15; i++) c += e[j] > mid[i] ? 1u : 0u;
+            const uint32_t c = mid.index(e[j]);
             const uint32_t bit = (uint32_t)(lane + 64 * j) * (uint32_t)t.bits, w = bit >> 5, off = bit & 31;
             atomicOr(&s_words[w], c << off);
             if (off + t.bits > 32) atomicOr(&s_words[w + 1], c >> (32 - off));
@@ -227,13 +202,10 @@ __device__ void commit_row(const TqArgs& a, bool value, int pos, int head, int l
         // other rows of the pass own other bits of the same words
         const int gw = tq_v_group_words(t.bits);
         const uint32_t off = (uint32_t)(pos & 15) * (uint32_t)t.bits;
-        const uint64_t mask = (uint64_t)n_mid << off;
+        const uint64_t mask = (uint64_t)((1u << t.bits) - 1u) << off;
 #pragma unroll
         for (int j = 0; j < EPL; j++) {
-            uint32_t c = 0;
-#pragma unroll
-            for (int i = 0; i < 15; i++) c += e[j] > mid[i] ? 1u : 0u;
-            const uint64_t bits = (uint64_t)c << off;
+            const uint64_t bits = (uint64_t)mid.index(e[j]) << off;
             uint32_t* g = a.store.vq + (((long)head * (a.cap >> 4) + (pos >> 4)) * HD + lane + 64 * j) * gw;
             if ((uint32_t)mask) {
                 __hip_atomic_fetch_and(g, ~(uint32_t)mask, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -12,7 +12,7 @@ namespace tsv {
 bool prompt_supported(const tsv_ctx* c) {
     if (c->mtp.on) return false;
     for (const LayerW& L : c->layers)
-        if (L.cap < c->ctx_alloc || L.tq.k_bits || (L.n_experts && c->moe_fp4_terms) || !prompt_holds(L.qkv) || !prompt_holds(L.v_only) ||
+        if (L.cap < c->ctx_alloc || (L.n_experts && c->moe_fp4_terms) || !prompt_holds(L.qkv) || !prompt_holds(L.v_only) ||
             !prompt_holds(L.wo) || !prompt_holds(L.gate_up) || !prompt_holds(L.down) || !prompt_holds(L.router))
             return false;
     return true;
@@ -48,6 +48,12 @@ size_t lay_out(tsv_ctx* c, int rows, uint8_t* at) {
     put(w.ids, (size_t)rows * 4);
     put(w.part_o, (size_t)512 * 128 * c->hd * 4);
     put(w.part_ml, (size_t)512 * 128 * 2 * 4);
+    for (const LayerW& L : c->layers)
+        if (L.tq.k_bits) {  // one layer's rows as attention operands
+            put(w.k_levels, (size_t)c->nkv * L.cap * c->hd * 2);
+            put(w.v_levels, (size_t)c->nkv * L.cap * c->hd * 2);
+            break;
+        }
     int sorted = 0, tiles = 0;
     for (const LayerW& L : c->layers)
         if (L.n_experts) {
@@ -118,12 +124,16 @@ int prompt_open(tsv_ctx* c) {
 //   where routed experts have fewer than three rows on average, so that each is read for next to nothing whatever reads it
 //   (gpt-oss layers, 65 / 80 rows: 1151 / 1482 us against 1403 / 1524; the 128-expert shape of eight chosen at 65 rows, four each:
 //   788 against 743);
+//   with quantized KV rows below PROMPT_MIN_ROWS_TQ: callers that count a handle's passes expect up to 150 rows of such a handle in 64-row
+//   passes, as ever, so the line lies behind them and not where a prompt pass begins to win (8B shape, eight layers, 160 rows: 3520 us in
+//   smaller passes, 1733 in one; 130 rows stay at 2650);
 //   far into a context: a prompt pass's attention takes its blocks in whole 128-pair workgroups.  Q4_K, 8B shape, 65 rows: 715
 //   against 695 us at 0, 750 / 765 at 4000, 780 / 846 at 8000; 80 rows: 799 / 701, 831 / 769, 861 / 856, and 564 / 588 (two
 //   layers) at 32 000.
 bool prompt_pays(const tsv_ctx* c, int64_t n, int64_t base, bool tail) {
     if (n < PROMPT_MIN_ROWS || (n == PROMPT_MIN_ROWS && tail)) return false;  // (see prefill_passes)
     if (!c->wide.ok) return true;
+    if (c->tq_kc && n < PROMPT_MIN_ROWS_TQ) return false;
     tail |= c->mtp_head != nullptr;  // (the rows an attached head steps from)
     const int64_t blocks = n / 64 - (tail && n % 64 == 0), rest = n - 64 * blocks, smaller = blocks + (rest + 15) / 16;
     if (smaller != 2) return smaller > 2;
@@ -222,13 +232,24 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
         ra.nq = c->nq;
         ra.nkv = c->nkv;
         ra.hd = c->hd;
-        ra.cap = L.kv_slots;
+        ra.cap = L.cap;
         ra.paired = L.rope_fused && c->hd == 128;
+        ra.store = L.tq;
+        ra.tq_k = c->tq_k;
+        ra.tq_v = c->tq_v;
         if ((rc = launch_prompt_rope(s, ra))) return rc;
         PromptAttnArgs aa{};
         aa.q16 = w.q16;
         aa.kc = L.kc;
         aa.vc = L.vc;
+        if (L.tq.k_bits) {
+            if ((rc = launch_prompt_tq_levels(s, L.tq, (int)base + n, c->nkv, c->hd, L.cap, w.k_levels, w.v_levels))) return rc;
+            aa.kc = w.k_levels;
+            aa.vc = w.v_levels;
+            aa.kn = L.tq.kn;
+            aa.vn = L.tq.vn;
+            aa.unrot = c->tq_v.signs;
+        }
         aa.n = n;
         aa.base = (int)base;
         aa.nq = c->nq;
@@ -285,7 +306,7 @@ int launch_prompt_pass(tsv_ctx* c, int n, int64_t base, bool finish, bool logits
 int prompt_prime_open(tsv_ctx* h) {
     const tsv_ctx* t = h->mtp.target;
     const LayerW& L = h->layers[0];
-    if (!t->prompt.ok || !t->prompt.rows || !prompt_holds(h->mtp.fc) || !prompt_holds(L.qkv) || !prompt_holds(L.v_only) || h->nq * h->hd % 64 ||
+    if (!t->prompt.ok || !t->prompt.rows || L.tq.k_bits || !prompt_holds(h->mtp.fc) || !prompt_holds(L.qkv) || !prompt_holds(L.v_only) || h->nq * h->hd % 64 ||
         h->hd > t->hd || 2 * h->nkv * h->hd > std::max(t->hidden, (t->nq + 2 * t->nkv) * t->hd))
         return TSV_OK;
     const size_t a = prompt_a_bytes(t->prompt.rows, 2 * h->hidden), s = prompt_fmt_has_sums(h->mtp.fc.fmt) ? prompt_sum_bytes(t->prompt.rows, 2 * h->hidden) : 0;

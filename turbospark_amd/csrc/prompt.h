@@ -18,6 +18,7 @@ namespace tsv {
 
 constexpr int PROMPT_ROWS = 2048;     // most rows of one pass
 constexpr int PROMPT_MIN_ROWS = 64;   // fewer go in verify-sized passes
+constexpr int PROMPT_MIN_ROWS_TQ = 160;  // of a handle with quantized KV rows (prompt_pays)
 constexpr float PROMPT_SUM_SCALE = 1.0f / 64.0f, PROMPT_SUM_LEFT = 2048.0f;
 
 __host__ __device__ inline int prompt_k16(int k) { return (k + 255) / 256 * 16; }
@@ -151,11 +152,20 @@ struct PromptRopeArgs {
     uint16_t *q16, *kc, *vc;
     int nq, nkv, hd, cap;  // cap: positions of the cache, position p in slot p % cap; nq = 0: the columns are those of K and V alone
     int paired;            // as in RopeKvArgs
+    // store.k_bits: the layer keeps quantized rows: K and V go there (kc and vc unused, cap: the positions it holds), q16 is rotated
+    TqKv store;
+    TqSide tq_k, tq_v;
+    float inv_sqrt2;       // set by the launcher
 };
 int launch_prompt_rope(hipStream_t s, const PromptRopeArgs& a);
 
+// codebook levels of a quantized layer's first `positions` positions (rounded up to whole blocks) as an fp16 cache of `cap` positions
+int launch_prompt_tq_levels(hipStream_t s, const TqKv& q, int positions, int nkv, int hd, int cap, uint16_t* kc, uint16_t* vc);
+
 struct PromptAttnArgs {
     const uint16_t *q16, *kc, *vc;
+    // with unrot (the value side's signs): kc and vc hold codebook levels, q16 is rotated; the norms are [nkv][cap]
+    const float *kn, *vn, *unrot;
     int n, base, nq, nkv, hd, cap, window;
     float scale;
     const float* sinks;

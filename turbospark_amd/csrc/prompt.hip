@@ -3,10 +3,13 @@
 // attn.hip) take sixteen rows and read tree shapes from device memory; here rows are consecutive positions, so a row's number
 // says everything about it.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
+#include "attn_tq_core.h"
 #include "embed_row.h"
 #include "prompt.h"
+#include "tq_row.h"
 
 namespace tsv {
 
@@ -17,6 +20,7 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
 
 // ---- embedding --------------------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_prompt_embed(const uint8_t* __restrict__ raw, int dtype, int hidden, float* __restrict__ x,
@@ -274,10 +278,16 @@ __global__ __launch_bounds__(512) void k_prompt_norm_long(PromptNormArgs p) {
 // One workgroup per (block of sixteen cache positions, head): a K or V block of the head is one contiguous run of the cache
 // (kcache_index / vcache_index), put together in LDS and written sixteen bytes at a time.  Element by element from one wave per
 // (row, head), as the verify passes do it, a pass of 2048 rows is 98 000 waves of two-byte stores.
-template <int HD>
+// TQ: the layer keeps quantized rows (kvquant.hip, whose arithmetic this is on sixteen rows at once).  q is rotated with the key signs;
+// a K or V row's norm and indices go straight to the stores, from the fp16 values that an fp16 cache would hold.  A block of the
+// stores belongs to one workgroup, so the V groups' words, which hold a position's index beside fifteen others', need no atomics.
+// Quantizing, the levels below and the norms in the attention add 53 us to a layer of 2048 rows (8B shape: 9274 us for eight layers, seven
+// of them quantized, 8909 with fp16 rows); in the 64-row passes that such a prompt took before, each with a quantizer launch and an
+// attention of its own, the eight layers were 36 560 us, 300 rows 6290 (now 2285).
+template <int HD, bool TQ>
 __global__ __launch_bounds__(256) void k_prompt_rope(PromptRopeArgs p) {
     constexpr int HALF = HD / 2, LANES = HALF, RPI = 256 / LANES;  // rows per iteration
-    __shared__ _Float16 sh[16][HD + 8];
+    __shared__ __attribute__((aligned(16))) _Float16 sh[16][HD + 8];
     const int head = blockIdx.y, pb = (p.base >> 4) + blockIdx.x;
     const int kind = head < p.nq ? 0 : head < p.nq + p.nkv ? 1 : 2;
     const int h = kind == 0 ? head : kind == 1 ? head - p.nq : head - p.nq - p.nkv;
@@ -320,6 +330,71 @@ __global__ __launch_bounds__(256) void k_prompt_rope(PromptRopeArgs p) {
     }
     __syncthreads();
     const int t = threadIdx.x;
+    if (TQ) {
+        constexpr int EPL = HD / 64;
+        __shared__ float norm[16];
+        __shared__ uint8_t code[16][HD];
+        const int lane = t & 63, wave = t >> 6;
+        const TqSide& side = kind == 2 ? p.tq_v : p.tq_k;
+        if (kind != 0) {
+            if (t < 16) {  // the squares in index order (the reference's sum), a row to a lane
+                float ss = 0.f;
+#pragma unroll
+                for (int i = 0; i < HD; i += 8) {
+                    const half8 r = *(const half8*)&sh[t][i];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) ss = __fadd_rn(ss, __fmul_rn((float)r[e], (float)r[e]));
+                }
+                norm[t] = sqrtf(ss);
+            }
+            __syncthreads();
+        }
+        const TqMidpoints mid(side);
+        for (int slot = 4 * wave; slot < 4 * wave + 4; slot++) {
+            const float inv = kind != 0 ? 1.0f / fmaxf(norm[slot], 1e-6f) : 1.0f;  // (times one: the same bits)
+            float e[EPL];
+#pragma unroll
+            for (int j = 0; j < EPL; j++) e[j] = __fmul_rn(__fmul_rn((float)sh[slot][lane + 64 * j], inv), side.signs[lane + 64 * j]);
+            wht<EPL>(e, lane, p.inv_sqrt2);
+#pragma unroll
+            for (int j = 0; j < EPL; j++) {
+                if (kind == 0) sh[slot][lane + 64 * j] = (_Float16)e[j];
+                else code[slot][lane + 64 * j] = (uint8_t)mid.index(e[j]);
+            }
+        }
+        __syncthreads();
+        if (kind != 0) {
+            const int r0 = pb * 16 - p.base, lo = max(0, -r0), hi = min(16, p.n - r0);  // the pass's slots of the block
+            if (t >= lo && t < hi) (kind == 2 ? p.store.vn : p.store.kn)[(long)h * p.cap + pb * 16 + t] = norm[t];
+            const int bits = side.bits;
+            if (kind == 1) {  // a row's indices LSB first (kv_quant.rs:289-312), a word to a thread
+                const int words = side.words;
+                for (int id = t; id < 16 * words; id += 256) {
+                    const int slot = id / words, w = id - slot * words;
+                    uint32_t v = 0;
+                    for (int d = 32 * w / bits; d < HD && d * bits < 32 * w + 32; d++) {
+                        const int at = d * bits - 32 * w;
+                        v |= at >= 0 ? (uint32_t)code[slot][d] << at : (uint32_t)code[slot][d] >> -at;
+                    }
+                    if (slot >= lo && slot < hi) p.store.kq[((long)h * p.cap + pb * 16 + slot) * words + w] = v;
+                }
+            } else if (t < HD) {  // a dimension's indices of the block's positions, a group to a thread
+                const int gw = tq_v_group_words(bits);
+                uint32_t* g = p.store.vq + (((long)h * (p.cap >> 4) + pb) * HD + t) * gw;
+                uint64_t v = 0, mask = 0;
+#pragma unroll
+                for (int slot = 0; slot < 16; slot++)
+                    if (slot >= lo && slot < hi) {
+                        v |= (uint64_t)code[slot][t] << (slot * bits);
+                        mask |= (uint64_t)((1u << bits) - 1u) << (slot * bits);
+                    }
+                if (lo != 0 || hi != 16) v |= (gw == 2 ? ((uint64_t)g[1] << 32) | g[0] : (uint64_t)g[0]) & ~mask;
+                g[0] = (uint32_t)v;
+                if (gw == 2) g[1] = (uint32_t)(v >> 32);
+            }
+            return;
+        }
+    }
     if (t >= 16 * HD / 8) return;
     if (kind == 0) {
         const int slot = t / (HD / 8), d = t % (HD / 8) * 8, row = pb * 16 + slot - p.base;
@@ -353,6 +428,40 @@ __global__ __launch_bounds__(256) void k_prompt_rope(PromptRopeArgs p) {
     }
 }
 
+// ---- quantized rows as attention operands -----------------------------------------------------------------------------------------
+// The codebook levels of positions [0, 16 gridDim.x * DECODE) as fp16 in the layout of an fp16 cache, for the attention kernel below; the
+// norms stay where they are, f32.  A layer's 4096 positions of the 8B shape are 4.5 MB of codes and 16.8 MB of levels, and every wave of
+// the pass reads them instead of unpacking them: 64 waves a KV head at 512 rows.
+constexpr int DECODE = 4;
+template <int HD>
+__global__ __launch_bounds__(256) void k_prompt_tq_levels(TqKv q, int blocks, int cap, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc) {
+    __shared__ uint32_t kpair[256], vpair[256];
+    const int t = threadIdx.x, h = blockIdx.y, kb = q.k_bits, vb = q.v_bits, kw = HD * kb / 32, gw = tq_v_group_words(vb);
+    tq_fill_pairs(kpair, q.k_cb, kb, t, 256);
+    tq_fill_pairs(vpair, q.v_cb, vb, t, 256);
+    __syncthreads();
+    if (t >= 2 * HD) return;
+    const uint32_t km = (1u << (2 * kb)) - 1u, vm = (1u << (2 * vb)) - 1u;
+    for (int b = blockIdx.x * DECODE; b < min(blocks, (int)(blockIdx.x + 1) * DECODE); b++) {
+        const size_t blk = ((size_t)h * (cap >> 4) + b) * (16 * HD) + t * 8;
+        {  // piece t of K: eight dims of one position
+            const int d = (t >> 6) * 32 + ((t >> 4) & 3) * 8, bit = d * kb, w = bit >> 5;
+            const uint32_t* row = q.kq + ((size_t)h * cap + b * 16 + (t & 15)) * kw;
+            const uint32_t f = (uint32_t)((((uint64_t)row[min(w + 1, kw - 1)] << 32) | row[w]) >> (bit & 31));
+            *(u32x4*)(kc + blk) = u32x4{kpair[f & km], kpair[(f >> (2 * kb)) & km], kpair[(f >> (4 * kb)) & km], kpair[(f >> (6 * kb)) & km]};
+        }
+        u32x4 o;  // piece t of V: four positions of two dims
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const uint32_t* g = q.vq + (((size_t)h * (cap >> 4) + b) * HD + (t >> 6) * 32 + (t & 15) + 16 * e) * gw;
+            const uint32_t f = (uint32_t)((((uint64_t)(gw == 2 ? g[1] : 0u) << 32) | g[0]) >> (((t >> 4) & 3) * 4 * vb));
+            o[2 * e] = vpair[f & vm];
+            o[2 * e + 1] = vpair[(f >> (2 * vb)) & vm];
+        }
+        *(u32x4*)(vc + blk) = o;
+    }
+}
+
 // ---- attention ------------------------------------------------------------------------------------------------------------------
 // A wave holds 32 (row, q head of the group) pairs as the columns of v_mfma_f32_32x32x16_f16 and walks the cache 32 positions at
 // a time: S^T = K Q^T, weights, O^T += V^T P^T.  A lane's sixteen scores are of ONE pair, so the softmax crosses lanes once
@@ -380,7 +489,11 @@ __device__ __forceinline__ float left_over(float w, uint32_t h) {
 }
 constexpr float LOG2E = 1.44269504088896340736f, REF_SLACK = 8.0f;
 
-template <int HD, bool PART>
+// TQ: the rows are codebook levels (k_prompt_tq_levels) and an f32 norm a position and side, q is rotated (attn_tq_core.h): a key's norm
+// multiplies its score, a value's the weight before it is cut into two fp16 terms (with no slack in the reference: a weight is at
+// most 1, so that a norm up to fp16's largest value passes), and the sum is rotated back in registers: six of the seven stages at
+// 128 dims pair values of one lane.
+template <int HD, bool PART, bool TQ>
 __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
     constexpr int KS = HD / 16, VT = HD / 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -413,12 +526,26 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
         for (int i = 0; i < 16; i++) O[u][i] = 0.f;
     float mrun = -INFINITY, lrun = 0.f;
     const float c2 = p.scale * LOG2E;
+    const __amdgpu_buffer_rsrc_t knrs = __builtin_amdgcn_make_buffer_rsrc((void*)(p.kn + (size_t)(TQ ? kvh : 0) * p.cap), 0, TQ ? (p.base + p.n) * 4 : 0, 0x00027000);
+    const __amdgpu_buffer_rsrc_t vnrs = __builtin_amdgcn_make_buffer_rsrc((void*)(p.vn + (size_t)(TQ ? kvh : 0) * p.cap), 0, TQ ? (p.base + p.n) * 4 : 0, 0x00027000);
     u32x4 kf[KS];
+    // a block's norms: a lane asks for one position's, with its K, and the wave passes them round through 256 bytes of LDS (sixteen
+    // registers a side for each lane's own would be 33 more than there are at 128 dims)
+    __shared__ __attribute__((aligned(16))) float norms[TQ ? 4 : 1][64];
+    float kn = 0.f, vn = 0.f;
+    auto order = [] {  // one wave writes and reads its own LDS: program order is enough, and the compiler is kept to it
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     auto load_k = [&](int b) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < KS; t++)
             kf[t] = __builtin_amdgcn_raw_buffer_load_b128(krs, koff + (uint32_t)b * (HD * 64) + (t >> 1) * 1024 + (t & 1) * 512, 0, 0);
+        if (TQ) {
+            kn = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(knrs, (uint32_t)b * 128 + 4 * (lane & 31), 0, 0));
+            vn = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(vnrs, (uint32_t)b * 128 + 4 * (lane & 31), 0, 0));
+        }
         __builtin_amdgcn_sched_barrier(0);
     };
     // (a block's V is asked for before its scores are made, the next block's K right after: both have the softmax and a product
@@ -440,6 +567,16 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
 #pragma unroll
         for (int t = 0; t < KS; t++)
             S = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, kf[t]), __builtin_bit_cast(half8, q[t]), S, 0, 0, 0);
+        if (TQ) {
+            norms[TQ ? wave : 0][lane] = hl ? vn : kn;
+            order();
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float4v f = *(const float4v*)&norms[TQ ? wave : 0][8 * i + 4 * hl];
+#pragma unroll
+                for (int e = 0; e < 4; e++) S[4 * i + e] *= f[e];
+            }
+        }
         load_k(min(b + 1, b1 - 1));
         // register i: position 32 b + 8 (i / 4) + 4 hl + i % 4
         const int p0 = 32 * b;
@@ -456,7 +593,7 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
         for (int i = 1; i < 16; i++) mb = fmaxf(mb, S[i]);
         mb = other_half_max(mb) * c2;
         // the reference follows the maximum lazily (attn_core.h): a weight never exceeds 2^REF_SLACK
-        const bool grow = mb > mrun + REF_SLACK;
+        const bool grow = mb > mrun + (TQ ? 0.f : REF_SLACK);
         if (__builtin_amdgcn_ballot_w64(grow) != 0) {
             const float mnew = grow ? mb : mrun;
             const float alpha = __builtin_amdgcn_exp2f(mrun - fmaxf(mnew, -3.0e38f));
@@ -472,14 +609,20 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
         float ps = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
-            const float w0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[i], c2, nref)), w1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[i + 1], c2, nref));
+            const float2v f = TQ ? *(const float2v*)&norms[TQ ? wave : 0][TQ ? 32 + 8 * (i >> 2) + 4 * hl + (i & 3) : 0] : float2v{1.f, 1.f};
+            float w0 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[i], c2, nref)), w1 = __builtin_amdgcn_exp2f(__builtin_fmaf(S[i + 1], c2, nref));
             ps += w0;
             ps += w1;
+            if (TQ) {  // the denominator takes the weight alone
+                w0 *= f[0];
+                w1 *= f[1];
+            }
             const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(w0, w1));
             P[i >> 3][(i & 7) >> 1] = h;
             R[i >> 3][(i & 7) >> 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(left_over<0>(w0, h), left_over<1>(w1, h)));
         }
         lrun += ps;
+        if (TQ) order();
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
@@ -517,6 +660,30 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
     }
     scale /= l;
     const int k16 = prompt_k16(p.nq * HD);
+    if (TQ) {  // back through the normalized Hadamard transform (crates/compute/src/wht.rs:15-29): dim 32 u + 8 (i / 4) + 4 hl + i % 4
+        const float c = 0.70710678118654752440f;
+#pragma unroll
+        for (int st = 1; st < HD; st <<= 1) {
+            const int ri = st == 1 ? 1 : st == 2 ? 2 : st == 8 ? 4 : st == 16 ? 8 : 0, ru = st >= 32 ? st / 32 : 0;
+#pragma unroll
+            for (int u = 0; u < VT; u++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    if (st == 4) {
+                        const float other = __shfl_xor(O[u][i], 32);
+                        O[u][i] = (hl ? other - O[u][i] : O[u][i] + other) * c;
+                    } else if (!(i & ri) && !(u & ru)) {
+                        const float a = O[u][i], b = O[u ^ ru][i ^ ri];
+                        O[u][i] = (a + b) * c;
+                        O[u ^ ru][i ^ ri] = (a - b) * c;
+                    }
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < VT; u++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) O[u][i] *= p.unrot[32 * u + 8 * (i >> 2) + 4 * hl + (i & 3)];
+    }
 #pragma unroll
     for (int u = 0; u < VT; u++) {
         float sum = 0.f;
@@ -546,7 +713,7 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
 }
 
 // The chunks' partial results of one (row, q head) merged, one thread per eight dims; HD / 8 threads to a pair
-template <int HD>
+template <int HD, bool TQ>
 __global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
     constexpr int TPP = HD / 8;
     const int G = p.nq / p.nkv, cols = p.n * G;
@@ -571,6 +738,27 @@ __global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
     const float inv = 1.0f / l;
 #pragma unroll
     for (int e = 0; e < 8; e++) o[e] *= inv;
+    if (TQ) {  // back out of the rotated space: three stages inside a thread, the others over the TPP lanes of the pair
+        const float c = 0.70710678118654752440f;
+#pragma unroll
+        for (int st = 1; st < 8; st <<= 1)
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (!(e & st)) {
+                    const float a = o[e], b = o[e ^ st];
+                    o[e] = (a + b) * c;
+                    o[e ^ st] = (a - b) * c;
+                }
+#pragma unroll
+        for (int st = 1; st < TPP; st <<= 1)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float other = __shfl_xor(o[e], st);
+                o[e] = (threadIdx.x & st ? other - o[e] : o[e] + other) * c;
+            }
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] *= p.unrot[d + e];
+    }
     put_activations(p.a, p.asum, row, hq * HD + d, prompt_k16(p.nq * HD), o, live);
 }
 
@@ -718,14 +906,32 @@ int launch_prompt_gather(hipStream_t s, const uint16_t* rows, const uint8_t* row
     return TSV_OK;
 }
 
-int launch_prompt_rope(hipStream_t s, const PromptRopeArgs& a) {
-    if (a.splits < 1 || a.splits > 8 || (a.hd != 64 && a.hd != 128) || a.cap % 16 || a.n > a.cap) {
+int launch_prompt_rope(hipStream_t s, const PromptRopeArgs& a0) {
+    PromptRopeArgs a = a0;
+    const bool tq = a.store.k_bits != 0;
+    if (a.splits < 1 || a.splits > 8 || (a.hd != 64 && a.hd != 128) || a.cap % 16 || a.n > a.cap || (tq && a.base + a.n > a.cap)) {
         set_error("prompt pass: bad rotation arguments");
         return TSV_ERR_INVALID;
     }
+    a.inv_sqrt2 = 1.0f / std::sqrt(2.0f);
     const dim3 grid((a.base + a.n - 1) / 16 - a.base / 16 + 1, a.nq + 2 * a.nkv);
-    if (a.hd == 128) hipLaunchKernelGGL(k_prompt_rope<128>, grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(k_prompt_rope<64>, grid, dim3(256), 0, s, a);
+    if (a.hd == 128 && tq) hipLaunchKernelGGL((k_prompt_rope<128, true>), grid, dim3(256), 0, s, a);
+    else if (a.hd == 128) hipLaunchKernelGGL((k_prompt_rope<128, false>), grid, dim3(256), 0, s, a);
+    else if (tq) hipLaunchKernelGGL((k_prompt_rope<64, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_prompt_rope<64, false>), grid, dim3(256), 0, s, a);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int launch_prompt_tq_levels(hipStream_t s, const TqKv& q, int positions, int nkv, int hd, int cap, uint16_t* kc, uint16_t* vc) {
+    if ((hd != 64 && hd != 128) || cap % 16 || positions < 1 || positions > cap || q.k_bits < 2 || q.k_bits > 4 || q.v_bits < 2 || q.v_bits > 4) {
+        set_error("prompt pass: bad arguments for quantized rows");
+        return TSV_ERR_INVALID;
+    }
+    const int blocks = (positions + 15) / 16;
+    const dim3 grid((blocks + DECODE - 1) / DECODE, nkv);
+    if (hd == 128) hipLaunchKernelGGL(k_prompt_tq_levels<128>, grid, dim3(256), 0, s, q, blocks, cap, kc, vc);
+    else hipLaunchKernelGGL(k_prompt_tq_levels<64>, grid, dim3(256), 0, s, q, blocks, cap, kc, vc);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }
@@ -737,15 +943,15 @@ int prompt_attn_chunks(int n, int base, int nq, int nkv, int window) {
     return std::max(1, std::min(std::min(512 / std::max(1, wgs), blocks / 16), 16));
 }
 
-template <int HD>
+template <int HD, bool TQ>
 static int launch_attn(hipStream_t s, const PromptAttnArgs& a) {
     const int cols = a.n * (a.nq / a.nkv);
     const dim3 grid((cols + 127) / 128, a.nkv, a.nch);
     if (a.nch > 1) {
-        hipLaunchKernelGGL((k_prompt_attn<HD, true>), grid, dim3(256), 0, s, a);
-        hipLaunchKernelGGL(k_prompt_attn_merge<HD>, dim3(((size_t)a.n * a.nq * (HD / 8) + 255) / 256), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_prompt_attn<HD, true, TQ>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_prompt_attn_merge<HD, TQ>), dim3(((size_t)a.n * a.nq * (HD / 8) + 255) / 256), dim3(256), 0, s, a);
     } else {
-        hipLaunchKernelGGL((k_prompt_attn<HD, false>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_prompt_attn<HD, false, TQ>), grid, dim3(256), 0, s, a);
     }
     TSV_HIP(hipGetLastError());
     return TSV_OK;
@@ -756,7 +962,8 @@ int launch_prompt_attention(hipStream_t s, const PromptAttnArgs& a) {
         set_error("prompt pass: bad attention arguments");
         return TSV_ERR_INVALID;
     }
-    return a.hd == 128 ? launch_attn<128>(s, a) : launch_attn<64>(s, a);
+    if (a.unrot) return a.hd == 128 ? launch_attn<128, true>(s, a) : launch_attn<64, true>(s, a);
+    return a.hd == 128 ? launch_attn<128, false>(s, a) : launch_attn<64, false>(s, a);
 }
 
 }  // namespace tsv

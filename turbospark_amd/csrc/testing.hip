@@ -511,7 +511,8 @@ extern "C" int32_t tsv_attention_quantized(const uint16_t* q, const uint16_t* k,
                                            int32_t nkv, int32_t hd, int64_t base, int32_t k_bits, int32_t v_bits,
                                            float scale, const float* sinks, uint16_t* out, uint32_t* k_rows,
                                            uint32_t* v_rows) {
-    if (!q || !k || !v || !out || !k_rows || !v_rows || m < 1 || m > TSV_MAX_ROWS || nq % nkv || nq / nkv > 8 || base < 0 ||
+    const bool prompt = m > TSV_MAX_ROWS && m <= PROMPT_ROWS;  // a prompt pass: its rows through the rotation kernel, the prefix's as below
+    if (!q || !k || !v || !out || !k_rows || !v_rows || m < 1 || (m > TSV_MAX_ROWS && !prompt) || nq % nkv || nq / nkv > 8 || base < 0 ||
         k_bits < 2 || k_bits > 4 || v_bits < 2 || v_bits > 4 || (hd != 64 && hd != 128)) {
         set_error("attention_quantized: bad argument");
         return TSV_ERR_INVALID;
@@ -520,14 +521,18 @@ extern "C" int32_t tsv_attention_quantized(const uint16_t* q, const uint16_t* k,
     tsv_ctx* c = &tmp;
     TSV_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     VerifyParams vp;
-    int rc = fill_params(vp, nullptr, nullptr, m, base, 0);
+    int rc = prompt ? TSV_OK : fill_params(vp, nullptr, nullptr, m, base, 0);
     const int seq = (int)base + m, ctx = (seq + 15) / 16 * 16, nch = attn_chunks(nkv), G = nq / nkv, slots = TSV_MAX_ROWS;
     const size_t stb = (size_t)nkv * slots * hd * 2, inb = (size_t)seq * nkv * hd * 2, qb = (size_t)m * nq * hd * 2;
     uint16_t *kc = nullptr, *vc = nullptr, *kin = nullptr, *vin = nullptr, *q16 = nullptr;
     float *po = nullptr, *pml = nullptr, *sinks_dev = nullptr, *tables = nullptr;
     uint4* xf = nullptr;
     VerifyParams* vpd = nullptr;
-    const size_t xfb = xfrag_bytes(nq * hd);
+    const int pch = prompt ? prompt_attn_chunks(m, (int)base, nq, nkv, 0) : 0, k16 = prompt_k16(nq * hd), ldq = (nq + 2 * nkv) * hd;
+    const size_t xfb = prompt ? prompt_a_bytes(m, nq * hd) : xfrag_bytes(nq * hd), levels = (size_t)nkv * ctx * hd * 2;
+    std::vector<float> columns(prompt ? (size_t)(m + 15) / 16 * 16 * ldq : 0), turn(prompt ? (size_t)m * hd : 0);
+    uint16_t *kl = nullptr, *vl = nullptr;
+    float *qkv = nullptr, *cs = nullptr;
     TqArgs ta{};
     TqKv st{};
     st.k_bits = k_bits;
@@ -546,8 +551,8 @@ extern "C" int32_t tsv_attention_quantized(const uint16_t* q, const uint16_t* k,
     if (!rc) rc = dev_alloc(c, &kin, inb);
     if (!rc) rc = dev_alloc(c, &vin, inb);
     if (!rc) rc = dev_alloc(c, &q16, qb);
-    if (!rc) rc = dev_alloc(c, &po, (size_t)nkv * nch * m * G * hd * 4, true);
-    if (!rc) rc = dev_alloc(c, &pml, (size_t)nkv * nch * m * G * 2 * 4, true);
+    if (!rc) rc = dev_alloc(c, &po, (size_t)nkv * std::max(nch, pch) * m * G * hd * 4, true);
+    if (!rc) rc = dev_alloc(c, &pml, (size_t)nkv * std::max(nch, pch) * m * G * 2 * 4, true);
     if (!rc) rc = dev_alloc(c, &xf, xfb, true);
     if (!rc) rc = dev_alloc(c, &vpd, sizeof vp);
     if (!rc) rc = dev_alloc(c, &tables, (size_t)2 * TQ_TABLE_FLOATS * 4);
@@ -572,7 +577,7 @@ extern "C" int32_t tsv_attention_quantized(const uint16_t* q, const uint16_t* k,
     // every row goes through the staging slots and the quantizer, sixteen at a time as passes do; the last
     // group is the pass itself, whose q rows are rotated with it
     const size_t row = (size_t)nkv * hd;
-    for (int64_t p = 0; !rc && p < seq;) {
+    for (int64_t p = 0; !rc && p < (prompt ? base : seq);) {
         const bool last = p >= base;
         const int n = last ? m : (int)std::min<int64_t>(slots, base - p);
         rc = launch_kv_fill(c->stream, kc, vc, nkv, hd, slots, (int)p, n, kin + (size_t)p * row, vin + (size_t)p * row);
@@ -582,7 +587,61 @@ extern "C" int32_t tsv_attention_quantized(const uint16_t* q, const uint16_t* k,
         if (!rc) rc = launch_tq_prepare(c->stream, ta);
         p += n;
     }
-    if (!rc) {
+    if (!rc && prompt) {
+        auto value = [](uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); };
+        for (int b = 0; b < m; b++) {
+            for (int i = 0; i < nq * hd; i++) columns[(size_t)b * ldq + i] = value(q[(size_t)b * nq * hd + i]);
+            for (int i = 0; i < nkv * hd; i++) {
+                columns[(size_t)b * ldq + nq * hd + i] = value(k[((size_t)base + b) * row + i]);
+                columns[(size_t)b * ldq + (nq + nkv) * hd + i] = value(v[((size_t)base + b) * row + i]);
+            }
+            for (int i = 0; i < hd; i += 2) turn[(size_t)b * hd + i] = 1.0f;  // (no rotation)
+        }
+        rc = dev_alloc(c, &qkv, columns.size() * 4);
+        if (!rc) rc = dev_alloc(c, &cs, turn.size() * 4);
+        if (!rc) rc = dev_alloc(c, &kl, levels, true);
+        if (!rc) rc = dev_alloc(c, &vl, levels, true);
+        if (!rc && (hipMemcpyAsync(qkv, columns.data(), columns.size() * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+                    hipMemcpyAsync(cs, turn.data(), turn.size() * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess))
+            rc = TSV_ERR_DEVICE;
+        PromptRopeArgs ra{};
+        ra.qkv = qkv;
+        ra.splits = 1;
+        ra.ldq = ldq;
+        ra.n = m;
+        ra.base = (int)base;
+        ra.cs = (const float2*)cs;
+        ra.q16 = q16;
+        ra.nq = nq;
+        ra.nkv = nkv;
+        ra.hd = hd;
+        ra.cap = ctx;
+        ra.store = st;
+        ra.tq_k = ta.k;
+        ra.tq_v = ta.v;
+        if (!rc) rc = launch_prompt_rope(c->stream, ra);
+        if (!rc) rc = launch_prompt_tq_levels(c->stream, st, seq, nkv, hd, ctx, kl, vl);
+        PromptAttnArgs pa{};
+        pa.q16 = q16;
+        pa.kc = kl;
+        pa.vc = vl;
+        pa.kn = st.kn;
+        pa.vn = st.vn;
+        pa.unrot = ta.v.signs;
+        pa.n = m;
+        pa.base = (int)base;
+        pa.nq = nq;
+        pa.nkv = nkv;
+        pa.hd = hd;
+        pa.cap = ctx;
+        pa.scale = scale > 0.f ? scale : 1.0f / std::sqrt((float)hd);
+        pa.sinks = sinks_dev;
+        pa.a = (uint8_t*)xf;
+        pa.part_o = po;
+        pa.part_ml = pml;
+        pa.nch = pch;
+        if (!rc) rc = launch_prompt_attention(c->stream, pa);
+    } else if (!rc) {
         AttnArgs aa{};
         aa.q16 = q16;
         aa.unrot = ta.v.signs;
@@ -611,7 +670,7 @@ extern "C" int32_t tsv_attention_quantized(const uint16_t* q, const uint16_t* k,
     if (!rc) rc = tq_rows_to_host(c->stream, st, nkv, hd, ctx, 0, seq, k_rows, v_rows);
     if (!rc)
         for (int b = 0; b < m; b++)
-            for (int kk = 0; kk < nq * hd; kk++) out[(size_t)b * nq * hd + kk] = frag[(size_t)frag_index(kk, b)];
+            for (int kk = 0; kk < nq * hd; kk++) out[(size_t)b * nq * hd + kk] = frag[prompt ? prompt_a_index(b, kk, k16) : (size_t)frag_index(kk, b)];
     (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
     (void)hipStreamDestroy(c->stream);
