@@ -497,9 +497,15 @@ template <int HD, bool PART, bool TQ>
 __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
     constexpr int KS = HD / 16, VT = HD / 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int G = p.nq / p.nkv, cols = p.n * G, kvh = blockIdx.y;
-    // the longest rows first
-    const int wg = gridDim.x - 1 - blockIdx.x, c_first = (wg * 4 + wave) * 32;
+    const int G = p.nq / p.nkv, cols = p.n * G;
+    // The longest rows first, head by head, so that with eight KV heads an XCD has one head's K and V in its L2; where everything
+    // is in flight at once and a compute unit gets two workgroups, the 256 behind the first 256 come in the opposite order, a short
+    // one beside a long one.  (With all rows of one head side by side the two were of one length, and the launch took as long as twice
+    // the longest: 8B shape, eight layers, us: 2048 rows 8594 -> 8335, 1300 rows 6150 -> 6022, 1500 behind 2000 7820 -> 7698; 64-wide
+    // heads, 2000 rows 3148 -> 3058; 1000 rows, one workgroup to a compute unit, 4638 -> 4634.)
+    int id = blockIdx.x;
+    if (!PART && gridDim.x > 256 && gridDim.x <= 512 && id >= 256) id = 256 + gridDim.x - 1 - id;
+    const int kvh = id % p.nkv, wg = gridDim.x / p.nkv - 1 - id / p.nkv, c_first = (wg * 4 + wave) * 32;
     if (c_first >= cols) return;
     const int hl = lane >> 5, c = min(c_first + (lane & 31), cols - 1), row = c / G, hq = kvh * G + (c - row * G);
     const int row_lo = c_first / G, row_hi = min(c_first + 31, cols - 1) / G;
@@ -946,7 +952,7 @@ int prompt_attn_chunks(int n, int base, int nq, int nkv, int window) {
 template <int HD, bool TQ>
 static int launch_attn(hipStream_t s, const PromptAttnArgs& a) {
     const int cols = a.n * (a.nq / a.nkv);
-    const dim3 grid((cols + 127) / 128, a.nkv, a.nch);
+    const dim3 grid((cols + 127) / 128 * a.nkv, 1, a.nch);
     if (a.nch > 1) {
         hipLaunchKernelGGL((k_prompt_attn<HD, true, TQ>), grid, dim3(256), 0, s, a);
         hipLaunchKernelGGL((k_prompt_attn_merge<HD, TQ>), dim3(((size_t)a.n * a.nq * (HD / 8) + 255) / 256), dim3(256), 0, s, a);
