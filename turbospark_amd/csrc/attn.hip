@@ -238,8 +238,10 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
     // about one workgroup per compute unit: the chunk count shrinks as the row groups multiply
     // (fewer, longer chunks also mean fewer partial results for the merge to read)
     AttnArgs a = a0;
-    // A short context in one workgroup per KV head and row group, up to DIRECT_BLOCKS / 8 blocks a wave, which finishes its rows itself:
-    // DIRECT_NOTE
+    // A short context in one workgroup per KV head and row group, up to ATTN_DIRECT_BLOCKS / 8 blocks a wave, which finishes its rows
+    // itself.  What that takes off a layer against chunks and a merge (8B shape, 1 / 5 / 16 rows, us): 2.0 / 1.5 / 4.9 at 250 positions,
+    // -0.1 / -0.6 / 2.0 at 700, and beyond the line, with the limit raised, -0.4 / -0.1 / 3.3 at 1000, -1.2 / -2.5 / 0.9 at 1500: a wave then
+    // walks too many blocks alone, and only sixteen rows, whose merge is the longest, would still gain.
     // Layers of a short window always do (a window's blocks: its own, the pass's, one cut).  All row groups take the form of eight
     // phases here, so that a row's sums run in one order whatever shares its pass.
     const bool few = attn_short(a.kv_end) || (a.window > 0 && (a.window + TSV_MAX_ROWS + 14) / 16 + 1 <= ATTN_DIRECT_BLOCKS);
