@@ -428,3 +428,22 @@ def test_a_vocabulary_that_is_not_a_multiple_of_anything_convenient():
         want = ob.chain_round(logits, draft, props, ocfg, history=list(prompt) + [7], draw_step=ds)
         _same(res, want, 33)
         gpu.rollback(point)
+
+
+# entries of a segment (vocabulary / 64) around the four folds' 64 and the chains' 256, and past the 2048 values that four workgroups to a
+# segment make at once; one to four rows take those, five the form of one workgroup
+@pytest.mark.parametrize("vocab,k", [(70, 1), (4097, 4), (16447, 2), (16448, 5), (131073, 1), (140001, 3), (140001, 5)])
+@pytest.mark.parametrize("temperature,kw", [(0.8, {}), (1.0, dict(top_k=50, top_p=0.95))])
+def test_draft_draws_of_any_vocabulary_match_the_oracle(vocab, k, temperature, kw):
+    """The same tokens: a draw differs from the oracle's only where a uniform lies within 1e-13 of a bin's edge (one draw in 1e9)."""
+    import turbospark_amd as ts
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS["tiny_q8_0"], vocab=vocab, n_layers=1, max_context=64)
+    gpu = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=3))
+    rng = np.random.default_rng(vocab + k)
+    gpu.prefill(rng.integers(0, vocab, 5).astype(np.int32), 0, want_logits=False)
+    for seed in range(6):
+        draft = (rng.standard_normal((k, vocab)) * (1 + 2 * (seed % 3))).astype(np.float16)
+        got = gpu.draft_chain(draft, ts.shaping(temperature, seed=seed, **kw), seed)
+        want = ob.draft_chain(draft, ob.shaping(temperature, seed=seed, **kw), [1, 2, 3], 0, seed)
+        assert list(got[0]) == list(want[0]) and got[1] == want[1], seed

@@ -33,14 +33,16 @@ constexpr int NSEG = 64;          // index segments per vocabulary row
 constexpr int MAX_DIST_ROWS = 32;  // target rows + drafter rows
 constexpr int MAX_JOBS = 16;
 constexpr int NSUB = 4;  // workgroups per segment in the mass / histogram pass
+// A round's rank histograms: [job][p, residual][65536] bins, and behind them the sums of every 64 consecutive ones, which is what the
+// draw's cumulative walk reads (8 KB instead of 512 by one workgroup: k_pick 21.0 -> 15.8 us a draw at 128 256 entries)
+constexpr int RANK_GROUPS = 65536 / 64;
 constexpr double FIX = 4611686018427387904.0;  // 2^62
 
 struct RowStat {
-    double mx, sum, total, top;
-    double minp;               // penalised rounds: candidates with e < minp are out (0: off)
     int32_t cut_key, cut_idx;  // last surviving candidate in rank order (truncation off: 65536, INT_MAX)
     float cut_w;               // its score (penalised rounds: a rank bin can hold several values)
 };
+__device__ __forceinline__ unsigned long long* rank_groups(unsigned long long* hist) { return hist + (size_t)MAX_JOBS * 2 * 65536; }
 struct Cut {
     int32_t key, idx;
     float w, pad;
@@ -51,8 +53,8 @@ struct Cut {
 //   pmax / psum / ptot partials follow, then the residual pieces and the decisions
 struct Layout {
     double* pmax;  // [rows][NSEG]
-    double* psum;
-    double* ptot;
+    double* psum;  // [rows][NSEG][4]
+    double* ptot;            // of the reweighted values, which k_row_total leaves in the work rows
     double* segtot;  // [jobs][NSEG * NSUB] residual mass per piece of a segment
     Cut* cut;        // [rows] truncation cut
 };
@@ -60,8 +62,8 @@ __host__ __device__ inline Layout layout(double* base) {
     Layout l;
     l.pmax = base + 4 * MAX_DIST_ROWS;
     l.psum = l.pmax + MAX_DIST_ROWS * NSEG;
-    l.ptot = l.psum + MAX_DIST_ROWS * NSEG;
-    l.segtot = l.ptot + MAX_DIST_ROWS * NSEG;
+    l.ptot = l.psum + MAX_DIST_ROWS * NSEG * 4;
+    l.segtot = l.ptot + MAX_DIST_ROWS * NSEG * 4;
     l.cut = (Cut*)base;
     return l;
 }
@@ -108,26 +110,10 @@ __device__ __forceinline__ uint32_t bin_addr(uint32_t key) {
     return (key & 0xF000u) | ((key & 63u) << 6) | ((key >> 6) & 63u);
 }
 
-// Whether candidate v (logit `bits`) is inside the row's truncated candidate set: the set is a
-// prefix of the rank order (logit descending, index ascending), so it is described by its last
-// member.
-__device__ __forceinline__ bool survives(uint16_t bits, int v, const RowStat& s) {
-    const int key = (int)rank_key(bits);
-    return key < s.cut_key || (key == s.cut_key && v <= s.cut_idx);
-}
-
 // (p / top)^(1/T), choose.rs:296-311.  At T = 1 the power is the identity -- the host library's pow returns its
 // argument exactly there -- and the device's software pow, the most expensive operation of these kernels, is skipped
 // (a branch every lane takes the same way).
 __device__ __forceinline__ double temper(double x, double inv_t) { return inv_t == 1.0 ? x : pow(x, inv_t); }
-
-// choose.rs:296-319 for one candidate of a row whose statistics are known
-__device__ __forceinline__ double prob_of(uint16_t bits, int v, const RowStat& s, double inv_t) {
-    if (!survives(bits, v, s)) return 0.0;
-    const double e = exp((double)h2f(bits) - s.mx);
-    const double p = e / s.sum;
-    return temper(p / s.top, inv_t) / s.total;
-}
 
 // ---- penalised scores -------------------------------------------------------------------------
 // crates/selection/src/penalty.rs:15-82 through choose.rs:138-154: the repetition penalty divides
@@ -193,23 +179,13 @@ __device__ __forceinline__ uint32_t key_of(float w, uint16_t bits) {
     return rank_key(bits);
 }
 
+// Whether candidate v is inside the row's truncated candidate set: the set is a prefix of the rank order (logit descending, index
+// ascending), so it is described by its last member.
 template <bool PEN>
 __device__ __forceinline__ bool survives_w(float w, int key, int v, const RowStat& s) {
     if constexpr (PEN)
         return key < s.cut_key || (key == s.cut_key && (w > s.cut_w || (w == s.cut_w && v <= s.cut_idx)));
     return key < s.cut_key || (key == s.cut_key && v <= s.cut_idx);
-}
-
-// choose.rs:296-319 for a candidate given by its score
-template <bool PEN>
-__device__ __forceinline__ double prob_of_w(float w, int key, int v, const RowStat& s, double inv_t) {
-    if (!survives_w<PEN>(w, key, v, s)) return 0.0;
-    const double e = exp((double)w - s.mx);
-    if constexpr (PEN) {
-        if (e < s.minp) return 0.0;
-    }
-    const double p = e / s.sum;
-    return temper(p / s.top, inv_t) / s.total;
 }
 
 template <typename T>
@@ -254,15 +230,19 @@ static_assert(NSEG == 64, "one lane per segment");
 template <bool PEN>
 __global__ __launch_bounds__(256) void k_row_max(const uint16_t* target, const uint16_t* draft, int m,
                                                  int vocab, double* scratch, int32_t* err,
-                                                 unsigned long long* hist, int hist_words,
+                                                 unsigned long long* hist, int jobs,
                                                  const AcceptParams* app) {
     __shared__ double red[4];
     const int row = blockIdx.y, seg = blockIdx.x;
     {
         // the rank histograms of this round's draws start from zero: every workgroup clears a slice
         const int nwg = gridDim.x * gridDim.y, wg = blockIdx.y * gridDim.x + blockIdx.x;
-        const int per = (hist_words + nwg - 1) / nwg, h0 = wg * per, h1 = min(h0 + per, hist_words);
-        for (int i = h0 + threadIdx.x; i < h1; i += 256) hist[i] = 0;
+        auto clear = [&](unsigned long long* at, int words) {
+            const int per = (words + nwg - 1) / nwg, h0 = wg * per, h1 = min(h0 + per, words);
+            for (int i = h0 + threadIdx.x; i < h1; i += 256) at[i] = 0;
+        };
+        clear(hist, jobs * 2 * 65536);
+        clear(rank_groups(hist), jobs * 2 * RANK_GROUPS);
     }
     const uint16_t* p = row_ptr(target, draft, m, vocab, row);
     const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
@@ -293,37 +273,70 @@ __global__ __launch_bounds__(256) void k_row_max(const uint16_t* target, const u
     }
 }
 
-template <bool PEN>
+// The sum of value(v) over a segment's [v0, v1): 256 chains, chain t every 256th value from v0 + t on, folded over the 64 lanes of a wave
+// and left as four numbers (fold_row adds them up).  A thread to a chain; or, SPLIT, the four folds are workgroups of their own
+// (blockIdx.z) whose four waves make the values of the chains (an exp, and a pow with it, in f64 each) a quarter each.  The same bits.
+// 64 segments of a single row, a draft step's, leave three quarters of the chip idle otherwise: k_row_total 10.6 -> 4.9 us at
+// 128 256 entries and T = 0.8.
+template <bool SPLIT, class Value>
+__device__ __forceinline__ void chained_sum(int v0, int v1, double* out, Value&& value) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fold = SPLIT ? blockIdx.z : wave;
+    double acc = 0.0;
+    if (SPLIT) {
+        __shared__ double vals[8][64];
+        for (int at = v0 + 64 * fold + lane; at - lane < v1; at += 8 * 256) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int v = at + (wave + 4 * i) * 256;
+                if (v < v1) vals[wave + 4 * i][lane] = value(v);
+            }
+            __syncthreads();
+            if (wave == 0)
+                for (int i = 0; i < 8 && at + i * 256 < v1; i++) acc += vals[i][lane];
+            __syncthreads();
+        }
+    } else {
+        for (int v = v0 + threadIdx.x; v < v1; v += 256) acc += value(v);
+    }
+    for (int o = 32; o > 0; o >>= 1) acc += shfl_xor_t(acc, o);
+    if (lane == 0 && (!SPLIT || wave == 0)) out[fold] = acc;
+}
+// Called by whole waves: the row's sum out of its segments' four folds each, identical in every lane
+__device__ __forceinline__ double fold_row(const double* folds, int row) {
+    const double* f = folds + ((size_t)row * NSEG + (threadIdx.x & 63)) * 4;
+    const double a = f[0], b = f[1], c = f[2], d = f[3];
+    return wave_sum_f64(((a + b) + c) + d);
+}
+
+template <bool PEN, bool SPLIT>
 __global__ __launch_bounds__(256) void k_row_sum(const uint16_t* target, const uint16_t* draft, int m,
                                                  int vocab, double* scratch, const AcceptParams* app) {
-    __shared__ double red[4];
     const int row = blockIdx.y, seg = blockIdx.x;
     Layout L = layout(scratch);
     const double mx = wave_max_f64(L.pmax[row * NSEG + (threadIdx.x & 63)]);
     const uint16_t* p = row_ptr(target, draft, m, vocab, row);
     const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
-    double acc = 0.0;
-    for (int v = v0 + threadIdx.x; v < v1; v += 256) {
+    chained_sum<SPLIT>(v0, v1, L.psum + ((size_t)row * NSEG + seg) * 4, [&](int v) {
         float w;
         if constexpr (PEN)
             w = score_of<true>(*app, row, v, p[v]);
         else
             w = h2f(p[v]);
-        acc += exp((double)w - mx);
-    }
-    acc = block_sum_f64(acc, red);
-    if (threadIdx.x == 0) L.psum[row * NSEG + seg] = acc;
+        return exp((double)w - mx);
+    });
 }
 
-template <bool PEN>
+// Also leaves the reweighted values (zero: not a candidate) in work row slot0 + row * slot_step: whoever needs a probability
+// divides one by the row's total.  (Every later kernel made them again, an exp and a pow in f64 each: k_mass_hist 13.0 -> 5.3 us; a
+// tree's rows took a kernel of their own for it, 17.9 us, for 4 that this one has become slower by with 32 rows.)
+template <bool PEN, bool SPLIT>
 __global__ __launch_bounds__(256) void k_row_total(const uint16_t* target, const uint16_t* draft, int m,
                                                    int vocab, double* scratch, double inv_t,
-                                                   const AcceptParams* app) {
-    __shared__ double red[4];
+                                                   const AcceptParams* app, double* work, int slot0, int slot_step) {
     const int row = blockIdx.y, seg = blockIdx.x;
     Layout L = layout(scratch);
     const double mx = wave_max_f64(L.pmax[row * NSEG + (threadIdx.x & 63)]);
-    const double sum = wave_sum_f64(L.psum[row * NSEG + (threadIdx.x & 63)]);
+    const double sum = fold_row(L.psum, row);
     const double top = 1.0 / sum;  // the arg-max candidate has e == exp(0) == 1
     const uint16_t* p = row_ptr(target, draft, m, vocab, row);
     const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
@@ -331,38 +344,24 @@ __global__ __launch_bounds__(256) void k_row_total(const uint16_t* target, const
     cs.cut_key = L.cut[row].key;
     cs.cut_idx = L.cut[row].idx;
     cs.cut_w = L.cut[row].w;
-    double acc = 0.0;
-    for (int v = v0 + threadIdx.x; v < v1; v += 256) {
+    double* out = work + (size_t)(slot0 + row * slot_step) * vocab;
+    chained_sum<SPLIT>(v0, v1, L.ptot + ((size_t)row * NSEG + seg) * 4, [&](int v) {
         const uint16_t b = p[v];
-        if constexpr (PEN) {
-            const float w = score_of<true>(*app, row, v, b);
-            if (!survives_w<true>(w, (int)key_of<true>(w, b), v, cs)) continue;
+        const float w = score_of<PEN>(*app, row, v, b);
+        double t = 0.0;
+        if (survives_w<PEN>(w, (int)key_of<PEN>(w, b), v, cs)) {
             const double e = exp((double)w - mx);
-            if (app->has_min_p && e < app->min_p) continue;
-            acc += temper((e / sum) / top, inv_t);
-        } else {
-            if (!survives(b, v, cs)) continue;
-            const double e = exp((double)h2f(b) - mx);
-            acc += temper((e / sum) / top, inv_t);
+            if (!PEN || !app->has_min_p || !(e < app->min_p)) t = temper((e / sum) / top, inv_t);
         }
-    }
-    acc = block_sum_f64(acc, red);
-    if (threadIdx.x == 0) L.ptot[row * NSEG + seg] = acc;
+        out[v] = t;
+        return t;
+    });
 }
 
-// Called by one whole wave: the finished statistics of `row`, identical in every lane.
-__device__ RowStat load_stat(const Layout& L, int row) {
-    const int lane = threadIdx.x & 63;
-    RowStat s;
-    s.mx = wave_max_f64(L.pmax[row * NSEG + lane]);
-    s.sum = wave_sum_f64(L.psum[row * NSEG + lane]);
-    s.top = 1.0 / s.sum;
-    s.total = wave_sum_f64(L.ptot[row * NSEG + lane]);
-    s.cut_key = L.cut[row].key;
-    s.cut_idx = L.cut[row].idx;
-    s.cut_w = L.cut[row].w;
-    s.minp = 0.0;
-    return s;
+// Called by whole waves: the total of `row`, identical in every lane (1 where there is no candidate: its values are zeros).
+__device__ __forceinline__ double row_total(const Layout& L, int row) {
+    const double t = fold_row(L.ptot, row);
+    return t > 0.0 ? t : 1.0;
 }
 
 __device__ __forceinline__ void fold_margin(double& margin, double a, double b) {
@@ -433,35 +432,34 @@ __global__ __launch_bounds__(256) void k_mass_hist(const uint16_t* target, const
                                                    unsigned long long* hist, Decision* dec_out, int kind) {
     __shared__ Decision dec;
     __shared__ double red[4];
-    __shared__ RowStat stats[MAX_DIST_ROWS];
-    __shared__ uint16_t s_tb[TSV_MAX_ROWS], s_db[TSV_MAX_ROWS];
+    __shared__ double totals[MAX_DIST_ROWS];
     __shared__ double s_px[TSV_MAX_ROWS], s_qx[TSV_MAX_ROWS];
+    __shared__ unsigned long long groups[2][RANK_GROUPS];
     const AcceptParams& ap = *app;
     const int seg = blockIdx.x, jobi = blockIdx.y, sub = blockIdx.z;
     Layout L = layout(scratch);
+    // the reweighted values (k_row_total): of a chain round in the work rows behind its draw's two, of draft draw j beside its own
+    auto weights = [&](int row) { return work + (size_t)(kind == 0 ? 2 + row : 2 * row + 1) * ap.vocab; };
     if (kind == 0 && (int)threadIdx.x < ap.k) {
         const int i = threadIdx.x;
         const int32_t x = ap.feed[i + 1];
-        s_tb[i] = target[(long)i * ap.vocab + x];
-        s_db[i] = draft[(long)i * ap.vocab + x];
+        s_px[i] = weights(i)[x];
+        s_qx[i] = weights(ap.m + i)[x];
     }
     {
-        // every row's statistics, one wave per row at a time
+        // every row's total, one wave per row at a time
         const int rows = kind == 0 ? ap.m + ap.k : ap.k;
         for (int r = threadIdx.x >> 6; r < rows; r += 4) {
-            RowStat st = load_stat(L, r);
-            if (PEN && ap.has_min_p) st.minp = ap.min_p;
-            if ((threadIdx.x & 63) == 0) stats[r] = st;
+            const double t = row_total(L, r);
+            if ((threadIdx.x & 63) == 0) totals[r] = t;
         }
     }
+    for (int i = threadIdx.x; i < RANK_GROUPS; i += 256) groups[0][i] = groups[1][i] = 0;
     __syncthreads();
     if (kind == 0 && (int)threadIdx.x < ap.k) {
         const int i = threadIdx.x;
-        const double it = 1.0 / ap.temperature;
-        const int32_t x = ap.feed[i + 1];
-        const float wt = score_of<PEN>(ap, i, x, s_tb[i]), wd = score_of<PEN>(ap, ap.m + i, x, s_db[i]);
-        s_px[i] = prob_of_w<PEN>(wt, (int)key_of<PEN>(wt, s_tb[i]), x, stats[i], it);
-        s_qx[i] = prob_of_w<PEN>(wd, (int)key_of<PEN>(wd, s_db[i]), x, stats[ap.m + i], it);
+        s_px[i] /= totals[i];
+        s_qx[i] /= totals[ap.m + i];
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -481,12 +479,10 @@ __global__ __launch_bounds__(256) void k_mass_hist(const uint16_t* target, const
     __syncthreads();
     const Job job = dec.job;
     if (job.mode == 0) return;
-    const int vocab = ap.vocab;
-    const double inv_t = 1.0 / ap.temperature;
-    const RowStat sp = stats[job.row_p];
-    const RowStat sq = stats[job.mode == 2 ? job.row_q : job.row_p];
+    const int vocab = ap.vocab, row_q = job.mode == 2 ? job.row_q : job.row_p;
+    const double total_p = totals[job.row_p], total_q = totals[row_q];
     const uint16_t* lp = row_ptr(target, draft, ap.m, vocab, job.row_p);
-    const uint16_t* lq = row_ptr(target, draft, ap.m, vocab, job.row_q);
+    const double *tp = weights(job.row_p), *tq = weights(row_q);
     double* wp = work + (long)jobi * 2 * vocab;
     double* wr = wp + vocab;
     unsigned long long* hp = hist + (long)jobi * 2 * 65536;
@@ -495,20 +491,29 @@ __global__ __launch_bounds__(256) void k_mass_hist(const uint16_t* target, const
     double racc = 0.0;
     for (int v = v0 + sub * 256 + threadIdx.x; v < v1; v += 256 * NSUB) {
         const uint16_t b = lp[v];
-        const float w = score_of<PEN>(ap, job.row_p, v, b);
-        const uint32_t rk = key_of<PEN>(w, b);
-        const double pv = prob_of_w<PEN>(w, (int)rk, v, sp, inv_t);
+        const uint32_t rk = key_of<PEN>(score_of<PEN>(ap, job.row_p, v, b), b);
+        const double pv = tp[v] / total_p;
         const uint32_t key = bin_addr(rk);
         wp[v] = pv;
-        if (pv > 0.0) atomicAdd(hp + key, (unsigned long long)(pv * FIX));
+        auto add = [&](unsigned long long* bins, unsigned long long* sums, double mass) {
+            const unsigned long long fixed = (unsigned long long)(mass * FIX);
+            if (!fixed) return;
+            atomicAdd(bins + key, fixed);
+            atomicAdd(sums + (rk >> 6), fixed);
+        };
+        add(hp, groups[0], pv);
         if (job.mode == 2) {
-            const uint16_t bq = lq[v];
-            const float wq = score_of<PEN>(ap, job.row_q, v, bq);
-            const double mv = fmax(pv - prob_of_w<PEN>(wq, (int)key_of<PEN>(wq, bq), v, sq, inv_t), 0.0);
+            const double mv = fmax(pv - tq[v] / total_q, 0.0);
             wr[v] = mv;
             racc += mv;
-            if (mv > 0.0) atomicAdd(hr + key, (unsigned long long)(mv * FIX));
+            add(hr, groups[1], mv);
         }
+    }
+    __syncthreads();
+    unsigned long long* gp = rank_groups(hist) + (long)jobi * 2 * RANK_GROUPS;
+    for (int i = threadIdx.x; i < 2 * RANK_GROUPS; i += 256) {
+        const unsigned long long s = groups[i / RANK_GROUPS][i % RANK_GROUPS];
+        if (s) atomicAdd(gp + i, s);
     }
     if (job.mode == 2) {
         racc = block_sum_f64(racc, red);
@@ -585,7 +590,7 @@ __global__ __launch_bounds__(256) void k_trunc_hist(const uint16_t* target, cons
     const int row = blockIdx.y, seg = blockIdx.x, lane = threadIdx.x & 63;
     Layout L = layout(scratch);
     const double mx = wave_max_f64(L.pmax[row * NSEG + lane]);
-    const double sum = wave_sum_f64(L.psum[row * NSEG + lane]);
+    const double sum = fold_row(L.psum, row);
     const uint16_t* p = row_ptr(target, draft, m, vocab, row);
     const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
     unsigned long long* hm = tmass + (size_t)row * 65536;
@@ -891,7 +896,7 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
     const int vocab = ap.vocab;
     Layout L = layout(scratch);
     const double mx = wave_max_f64(L.pmax[row * NSEG + lane]);
-    const double sum = wave_sum_f64(L.psum[row * NSEG + lane]);
+    const double sum = fold_row(L.psum, row);
     const uint32_t* cmine = tcount + (size_t)row * 65536 + (tid >> 6) * 4096 + (tid & 63);
     const unsigned long long* mmine = tmass + (size_t)row * 65536 + (tid >> 6) * 4096 + (tid & 63);
     if (tid == 0) {
@@ -1088,26 +1093,10 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
         const double* w = kind == 2 ? work + (long)dec.pad * vocab : work + (long)jobi * 2 * vocab + (mode == 2 ? vocab : 0);
         const uint16_t* lp = row_ptr(target, draft, ap.m, vocab, dec.job.row_p);
 
-        // 64 consecutive rank bins per thread (see bin_addr); integer sums are exact and order
+        // 64 consecutive rank bins per thread (see bin_addr), whose sum is there already; integer sums are exact and order
         // independent
         const unsigned long long* hmine = hsel + (tid >> 6) * 4096 + (tid & 63);
-        // (one workgroup reads the whole histogram: what bounds it is how many loads a wave keeps in flight, so the 64
-        // bins come as two rounds of 32 loads)
-        unsigned long long quarter[4], loc = 0;  // the bins' sum in four runs of sixteen: the rescan below needs one run
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            unsigned long long hv[32];
-#pragma unroll
-            for (int i = 0; i < 32; i++) hv[i] = hmine[(half * 32 + i) * 64];
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                unsigned long long q = 0;
-#pragma unroll
-                for (int i = 0; i < 16; i++) q += hv[b * 16 + i];
-                quarter[half * 2 + b] = q;
-                loc += q;
-            }
-        }
+        const unsigned long long loc = rank_groups(hist)[(jobi * 2 + (mode == 2)) * RANK_GROUPS + tid];
         unsigned long long inc = loc;
         for (int o = 1; o < 64; o <<= 1) {
             const uint32_t lo = __shfl_up((uint32_t)inc, o), hi = __shfl_up((uint32_t)(inc >> 32), o);
@@ -1132,29 +1121,23 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
         const unsigned long long tgt = (unsigned long long)(dec.job.u * (double)total);
         if (loc > 0) atomicMax(&s_last_bin, tid * 64 + 63);
         if (excl <= tgt && tgt < excl + loc) {
-            // the one thread whose 64 bins hold the target: first bin at which the running sum passes it.  Only the
-            // run of sixteen the target falls into is fetched again, all of it at once (a loop over the 64 bins that
-            // stops at the hit waits out one L2 round trip per bin)
-            unsigned long long c = excl;
-            int b = 0;
-#pragma unroll
-            for (int t = 0; t < 3; t++)
-                if (b == t && !(tgt < c + quarter[t])) {
-                    c += quarter[t];
-                    b = t + 1;
-                }
-            unsigned long long hv[16];
-#pragma unroll
-            for (int i = 0; i < 16; i++) hv[i] = hmine[(b * 16 + i) * 64];
-            unsigned long long before = c;
+            // the one thread whose 64 bins hold the target: first bin at which the running sum passes it, out of two rounds of
+            // 32 loads in flight (a loop that stops at the hit waits out one L2 round trip per bin)
+            unsigned long long c = excl, before = excl;
             int hit = -1;
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                if (hit < 0 && tgt < c + hv[i]) {
-                    hit = b * 16 + i;
-                    before = c;
+            for (int half = 0; half < 2; half++) {
+                unsigned long long hv[32];
+#pragma unroll
+                for (int i = 0; i < 32; i++) hv[i] = hmine[(half * 32 + i) * 64];
+#pragma unroll
+                for (int i = 0; i < 32; i++) {
+                    if (hit < 0 && tgt < c + hv[i]) {
+                        hit = half * 32 + i;
+                        before = c;
+                    }
+                    c += hv[i];
                 }
-                c += hv[i];
             }
             s_bin = tid * 64 + hit;
             s_before = before;
@@ -1303,8 +1286,8 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
 // p by normalise(max(p - q, 0)) (kept as is when that mass is below 1e-12) -- and when no child
 // survives the next token is drawn from the p that is left.  No stop / budget bookkeeping.
 //
-// First every node's p and q are written out as dense f64 rows by the whole chip (work slots
-// 0..m-1 and m..2m-1); then the tree is walked one child test per launch.  A test is two lookups;
+// The statistics leave every node's p and q as dense f64 rows (work slots 0..m-1 and m..2m-1) that are divided by their row's
+// total where they are read; then the tree is walked one child test per launch.  A test is two lookups;
 // only a rejection costs a pass over the vocabulary (slots 32 and 33 alternate as the residual,
 // whose normalising division is applied when it is read, so a pass reads two rows and writes one).
 constexpr int TREE_SCRATCH_SLOT = 2 * TSV_MAX_ROWS;  // two residual rows behind the 32 distribution rows
@@ -1325,52 +1308,28 @@ struct TreeWalk {
 static_assert(sizeof(TreeWalk) % 8 == 0 && sizeof(TreeWalk) <= 32 * 8, "fits its slot of the statistics block");
 
 // behind the decisions: two copies of the state (32 doubles each), then two sets of TREE_WGS partial sums
-constexpr int STATS_DOUBLES = 4 * MAX_DIST_ROWS + 3 * MAX_DIST_ROWS * NSEG + MAX_JOBS * NSEG * NSUB + MAX_JOBS * 16;
+constexpr int DECISIONS_AT = 4 * MAX_DIST_ROWS + 9 * MAX_DIST_ROWS * NSEG + MAX_JOBS * NSEG * NSUB;
+constexpr int STATS_DOUBLES = DECISIONS_AT + MAX_JOBS * 16;
 constexpr int TREE_STATE_DOUBLES = 2 * 32 + 2 * TREE_WGS;
 __device__ TreeWalk* tree_walk(double* scratch, int copy) { return (TreeWalk*)(scratch + STATS_DOUBLES + 32 * copy); }
 __device__ double* tree_partials(double* scratch, int copy) { return scratch + STATS_DOUBLES + 64 + TREE_WGS * copy; }
 
-template <bool PEN>
-__global__ __launch_bounds__(256) void k_tree_probs(const uint16_t* target, const uint16_t* draft,
-                                                    const AcceptParams* app, double* scratch, double* work) {
-    __shared__ RowStat st;
-    const AcceptParams& ap = *app;
-    const int seg = blockIdx.x, row = blockIdx.y, vocab = ap.vocab;
-    Layout L = layout(scratch);
-    if (threadIdx.x < 64) {
-        const RowStat s0 = load_stat(L, row);
-        if (threadIdx.x == 0) st = s0;
-    }
-    __syncthreads();
-    RowStat s0 = st;
-    if (PEN && ap.has_min_p) s0.minp = ap.min_p;
-    const double inv_t = 1.0 / ap.temperature;
-    const uint16_t* lp = row_ptr(target, draft, ap.m, vocab, row);
-    double* out = work + (long)row * vocab;
-    if (seg == 0 && row == 0 && threadIdx.x == 0) {  // the walk starts at the root
-        TreeWalk w;
+// The state launch k starts from: copy k & 1 with the previous launch's residual pass resolved
+// (its total decides whether the residual replaces the node's distribution: distribution.rs:96-126).
+__device__ TreeWalk tree_state(const AcceptParams& ap, double* scratch, int k, double* red) {
+    TreeWalk w;
+    if (k == 0) {  // the walk starts at the root
         w.at = 0;
         w.next_s = 1;
         w.plen = 1;
         w.which = w.done = w.pending = w.src_slot = w.pend_slot = w.pad = 0;
-        w.Z = 1.0;
+        w.Z = row_total(layout(scratch), 0);
         w.margin = 1.0;
         w.ds = ap.draw_step;
         w.path[0] = 0;
-        *tree_walk(scratch, 0) = w;
+        return w;
     }
-    const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
-    for (int v = v0 + threadIdx.x; v < v1; v += 256) {
-        const uint16_t b = lp[v];
-        const float w = score_of<PEN>(ap, row, v, b);
-        out[v] = prob_of_w<PEN>(w, (int)key_of<PEN>(w, b), v, s0, inv_t);
-    }
-}
-
-// The state launch k starts from: copy k & 1 with the previous launch's residual pass resolved
-// (its total decides whether the residual replaces the node's distribution: distribution.rs:96-126).
-__device__ TreeWalk tree_state(double* scratch, int k, double* red) {
-    TreeWalk w = *tree_walk(scratch, k & 1);
+    w = *tree_walk(scratch, k & 1);
     if (w.pending) {
         const double part = (int)threadIdx.x < TREE_WGS ? tree_partials(scratch, k & 1)[threadIdx.x] : 0.0;
         const double total = block_sum_f64(part, red);
@@ -1389,7 +1348,7 @@ __global__ __launch_bounds__(256) void k_tree_step(const AcceptParams* app, doub
     __shared__ double red[4];
     const AcceptParams& ap = *app;
     const int vocab = ap.vocab, m = ap.m;
-    TreeWalk w = tree_state(scratch, k, red);
+    TreeWalk w = tree_state(ap, scratch, k, red);
     TreeWalk* out = tree_walk(scratch, (k + 1) & 1);
     const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
     int s = -1;
@@ -1406,9 +1365,10 @@ __global__ __launch_bounds__(256) void k_tree_step(const AcceptParams* app, doub
     }
     const double* src = work + (long)w.src_slot * vocab;  // the node's p; its values are src[v] / Z
     const double* q = work + (long)(m + w.at) * vocab;
+    const double total_q = row_total(layout(scratch), m + w.at);
     const int32_t x = ap.feed[s];
     const double r = unit_draw(ap.seed, w.ds);
-    const double px = src[x] / w.Z, qx = q[x];
+    const double px = src[x] / w.Z, qx = q[x] / total_q;
     fold_margin(w.margin, r * qx, px);
     w.ds += 1;
     w.next_s = s + 1;
@@ -1417,7 +1377,7 @@ __global__ __launch_bounds__(256) void k_tree_step(const AcceptParams* app, doub
         w.plen += 1;
         w.at = s;
         w.src_slot = s;
-        w.Z = 1.0;
+        w.Z = row_total(layout(scratch), s);
         w.which = 0;
         if (writer) *out = w;
         return;
@@ -1427,7 +1387,7 @@ __global__ __launch_bounds__(256) void k_tree_step(const AcceptParams* app, doub
     const int per = (vocab + TREE_WGS - 1) / TREE_WGS, v0 = blockIdx.x * per, v1 = min(v0 + per, vocab);
     double acc = 0.0;
     for (int v = v0 + threadIdx.x; v < v1; v += 256) {
-        const double mv = fmax(src[v] / w.Z - q[v], 0.0);
+        const double mv = fmax(src[v] / w.Z - q[v] / total_q, 0.0);
         dst[v] = mv;
         acc += mv;
     }
@@ -1445,9 +1405,12 @@ __global__ __launch_bounds__(256) void k_tree_finish(const uint16_t* target, con
                                                      double* work, unsigned long long* hist, Decision* dec_out,
                                                      int32_t* path_out, int k) {
     __shared__ double red[4];
+    __shared__ unsigned long long groups[RANK_GROUPS];
+    for (int i = threadIdx.x; i < RANK_GROUPS; i += 256) groups[i] = 0;
+    __syncthreads();
     const AcceptParams& ap = *app;
     const int vocab = ap.vocab;
-    const TreeWalk w = tree_state(scratch, k, red);
+    const TreeWalk w = tree_state(ap, scratch, k, red);
     Layout L = layout(scratch);
     unsigned long long* hr = hist + 65536;
     const double* src = work + (long)w.src_slot * vocab;
@@ -1455,11 +1418,17 @@ __global__ __launch_bounds__(256) void k_tree_finish(const uint16_t* target, con
     const int per = (vocab + TREE_WGS - 1) / TREE_WGS, v0 = blockIdx.x * per, v1 = min(v0 + per, vocab);
     for (int v = v0 + threadIdx.x; v < v1; v += 256) {
         const double mv = src[v] / w.Z;
-        if (mv > 0.0) {
+        const unsigned long long fixed = (unsigned long long)(mv * FIX);
+        if (fixed) {
             const uint16_t b = lpk[v];
-            atomicAdd(hr + bin_addr(key_of<PEN>(score_of<PEN>(ap, w.at, v, b), b)), (unsigned long long)(mv * FIX));
+            const uint32_t rk = key_of<PEN>(score_of<PEN>(ap, w.at, v, b), b);
+            atomicAdd(hr + bin_addr(rk), fixed);
+            atomicAdd(&groups[rk >> 6], fixed);
         }
     }
+    __syncthreads();
+    for (int i = threadIdx.x; i < RANK_GROUPS; i += 256)
+        if (groups[i]) atomicAdd(rank_groups(hist) + RANK_GROUPS + i, groups[i]);
     if (blockIdx.x != 0) return;
     // the draw divides the stored values by the fold of these pieces: Z, exactly
     if (threadIdx.x < NSEG * NSUB) L.segtot[threadIdx.x] = threadIdx.x == 0 ? w.Z : 0.0;
@@ -1639,9 +1608,11 @@ __global__ void k_clear_result(AcceptResult* res, int32_t* err) {
 // arg-max partials (value, then index, per row and run); decisions live after the
 // statistics block; histograms and work arrays are separate allocations in AcceptScratch.
 size_t accept_stats_doubles() { return STATS_DOUBLES + TREE_STATE_DOUBLES; }
+size_t accept_hist_words() { return (size_t)MAX_JOBS * 2 * (65536 + RANK_GROUPS); }
+int accept_work_rows() { return 2 + MAX_DIST_ROWS; }
 
 static Decision* decisions(const AcceptScratch& sc) {
-    return (Decision*)(sc.stats + 4 * MAX_DIST_ROWS + 3 * MAX_DIST_ROWS * NSEG + MAX_JOBS * NSEG * NSUB);
+    return (Decision*)(sc.stats + DECISIONS_AT);
 }
 
 // Between the softmax sums and the reweighting totals: the truncation cut of every row.
@@ -1662,24 +1633,32 @@ static void launch_trunc(hipStream_t s, const uint16_t* target, const uint16_t* 
 }
 
 // The statistics of `rows` distribution rows, their truncation cuts and reweighting totals.
+// Up to SPLIT_ROWS rows the sums' folds are workgroups of their own: one to four rows are a draft block's draws (a loop of 48 tokens,
+// block 4, on a small decoder: 9640 -> 9300 us with this and the stored values).  Nine rows, a round of five, fill the chip without, and
+// everything a wave does besides is done once (the same loop with the folds of all rows apart: 9060 -> 9380; sixteen-row trees 517 -> 530).
+constexpr int SPLIT_ROWS = 4;
 template <bool PEN>
-static void launch_stats(hipStream_t s, const uint16_t* target, const uint16_t* draft, int m, int rows, int hist_words,
-                         const AcceptParams* ap_dev, const AcceptParams& ap, const AcceptScratch& sc) {
+static void launch_stats(hipStream_t s, const uint16_t* target, const uint16_t* draft, int m, int rows, int jobs,
+                         const AcceptParams* ap_dev, const AcceptParams& ap, const AcceptScratch& sc, int slot0, int slot_step) {
     int32_t* err = (int32_t*)sc.counters;
     const double inv_t = 1.0 / ap.temperature;
     hipLaunchKernelGGL(k_row_max<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, err,
-                       (unsigned long long*)sc.hist, hist_words, ap_dev);
-    hipLaunchKernelGGL(k_row_sum<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, ap_dev);
+                       (unsigned long long*)sc.hist, jobs, ap_dev);
+    const dim3 grid(NSEG, rows, rows <= SPLIT_ROWS ? 4 : 1), block(256);
+    if (grid.z > 1) hipLaunchKernelGGL((k_row_sum<PEN, true>), grid, block, 0, s, target, draft, m, ap.vocab, sc.stats, ap_dev);
+    else hipLaunchKernelGGL((k_row_sum<PEN, false>), grid, block, 0, s, target, draft, m, ap.vocab, sc.stats, ap_dev);
     launch_trunc<PEN>(s, target, draft, m, rows, ap_dev, ap, sc);
-    hipLaunchKernelGGL(k_row_total<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, inv_t,
-                       ap_dev);
+    if (grid.z > 1)
+        hipLaunchKernelGGL((k_row_total<PEN, true>), grid, block, 0, s, target, draft, m, ap.vocab, sc.stats, inv_t, ap_dev, sc.work, slot0, slot_step);
+    else
+        hipLaunchKernelGGL((k_row_total<PEN, false>), grid, block, 0, s, target, draft, m, ap.vocab, sc.stats, inv_t, ap_dev, sc.work, slot0, slot_step);
 }
 
 template <bool PEN>
 static void launch_chain_sampled(hipStream_t s, const uint16_t* target, const uint16_t* draft,
                                  const AcceptParams* ap_dev, const AcceptParams& ap, const AcceptScratch& sc) {
     int32_t* err = (int32_t*)sc.counters;
-    launch_stats<PEN>(s, target, draft, ap.m, ap.m + ap.k, 2 * 65536, ap_dev, ap, sc);
+    launch_stats<PEN>(s, target, draft, ap.m, ap.m + ap.k, 1, ap_dev, ap, sc, 2, 1);
     hipLaunchKernelGGL(k_mass_hist<PEN>, dim3(NSEG, 1, NSUB), dim3(256), 0, s, target, draft, ap_dev, sc.stats, sc.work,
                        (unsigned long long*)sc.hist, decisions(sc), 0);
     hipLaunchKernelGGL(k_pick<PEN>, dim3(1), dim3(1024), 0, s, target, draft, ap_dev, sc.stats, sc.work,
@@ -1711,8 +1690,7 @@ static void launch_tree_sampled(hipStream_t s, const uint16_t* target, const uin
     int32_t* err = (int32_t*)sc.counters;
     int32_t* path = (int32_t*)sc.counters + 32;
     // statistics of the m target rows and the m rows the children were drawn from
-    launch_stats<PEN>(s, target, draft, ap.m, 2 * ap.m, 2 * 65536, ap_dev, ap, sc);
-    hipLaunchKernelGGL(k_tree_probs<PEN>, dim3(NSEG, 2 * ap.m), dim3(256), 0, s, target, draft, ap_dev, sc.stats, sc.work);
+    launch_stats<PEN>(s, target, draft, ap.m, 2 * ap.m, 1, ap_dev, ap, sc, 0, 1);
     // one child test per launch: as many launches as the longest walk through this tree can take
     const int steps = tree_walk_bound(ap.parent, ap.m);
     for (int k = 0; k < steps; k++)
@@ -1727,7 +1705,7 @@ template <bool PEN>
 static void launch_draft_sampled(hipStream_t s, const uint16_t* draft, const AcceptParams* ap_dev,
                                  const AcceptParams& ap, const AcceptScratch& sc, int32_t* proposals_dev) {
     int32_t* err = (int32_t*)sc.counters;
-    launch_stats<PEN>(s, draft, draft, 0, ap.k, ap.k * 2 * 65536, ap_dev, ap, sc);
+    launch_stats<PEN>(s, draft, draft, 0, ap.k, ap.k, ap_dev, ap, sc, 1, 2);
     hipLaunchKernelGGL(k_mass_hist<PEN>, dim3(NSEG, ap.k, NSUB), dim3(256), 0, s, draft, draft, ap_dev, sc.stats, sc.work,
                        (unsigned long long*)sc.hist, decisions(sc), 1);
     hipLaunchKernelGGL(k_pick<PEN>, dim3(ap.k), dim3(1024), 0, s, draft, draft, ap_dev, sc.stats, sc.work,

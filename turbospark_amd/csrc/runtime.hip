@@ -1326,8 +1326,8 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         (rc = dev_alloc(c, &c->pen_cnt, (size_t)c->vocab * 4, true)) ||
         (rc = dev_alloc(c, &c->tok_dev, 64 * 4, true)) ||
         (rc = dev_alloc(c, &c->sc.stats, accept_stats_doubles() * 8, true)) ||
-        (rc = dev_alloc(c, &c->sc.work, (size_t)(16 * 2 + 2) * c->vocab * 8, true)) ||
-        (rc = dev_alloc(c, &c->sc.hist, (size_t)16 * 2 * 65536 * 8, true)) ||
+        (rc = dev_alloc(c, &c->sc.work, (size_t)accept_work_rows() * c->vocab * 8, true)) ||
+        (rc = dev_alloc(c, &c->sc.hist, accept_hist_words() * 8, true)) ||
         (rc = dev_alloc(c, &c->sc.counters, ACCEPT_COUNTER_WORDS * 4, true)) ||
         (rc = dev_alloc(c, &c->sc.tmass, (size_t)32 * 65536 * 8, true)) ||
         (rc = dev_alloc(c, &c->sc.tcount, (size_t)32 * 65536 * 4, true)) ||

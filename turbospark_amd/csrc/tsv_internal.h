@@ -509,15 +509,17 @@ struct AcceptResult {
 };
 struct AcceptScratch {
     double* stats;       // accept_stats_doubles() doubles: row statistics, partials, decisions
-    double* work;        // [16 jobs][2][vocab] candidate masses (p, residual) + two more rows (tree residuals)
-    uint64_t* hist;      // [16 jobs][2][65536] fixed-point mass per rank bin; a round clears what it uses first
+    double* work;        // accept_work_rows() rows of vocab: a draw's candidate masses (p, residual), the distributions' reweighted
+                         // values, a tree's residuals
+    uint64_t* hist;      // accept_hist_words(): fixed-point mass per rank bin and per 64 of them; a round clears what it uses first
     uint32_t* counters;  // ACCEPT_COUNTER_WORDS words: error flag, tree path, greedy arg-max partials
     uint64_t* tmass;     // [32 rows][65536] fixed-point softmax mass per rank bin (top-p cut)
     uint32_t* tcount;    // [32 rows][65536] candidates per rank bin (top-k / top-p cut)
     AcceptResult* result;  // device
 };
 constexpr int ACCEPT_COUNTER_WORDS = 1024;
-size_t accept_stats_doubles();
+size_t accept_stats_doubles(), accept_hist_words();
+int accept_work_rows();
 // launches of the walk kernel a sampled tree round of this shape needs (parent[s] in [0, s), m <= TSV_MAX_ROWS)
 int tree_walk_bound(const int32_t* parent, int m);
 int launch_accept(hipStream_t s, const uint16_t* target, const uint16_t* draft, const AcceptParams* ap_dev,
