@@ -169,3 +169,29 @@ def test_graph_replay_of_the_pass_equals_plain_launches():
     parent = [-1, 0, 0, 1, 1]
     feed = rng.integers(0, cfg["vocab"], 5).astype(np.int32)
     assert np.array_equal(plain.verify_tree(feed, parent, base), graph.verify_tree(feed, parent, base))
+
+
+@pytest.mark.parametrize("name,layer,over", [("small_q4_k_m", 0, {}), ("small_q5_k_m", 1, {}), ("small_q4_k_m", 0, dict(head_dim=64, n_q_heads=8, n_kv_heads=2)),
+                                             ("small_q4_k_m", 0, dict(hidden=2304, n_q_heads=6, n_kv_heads=2))])
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])
+def test_a_value_projection_of_its_own_type_goes_with_q_and_k(name, layer, over, m, monkeypatch):
+    """One launch that rotates and stores against the projections and the rotation apart: the rows they store differ by the order of
+    fp32 sums (2^-24 of the row's norm and its root of a thousand terms: 1e-5 of the largest value covers it), which moves an fp16 by
+    one unit in the last place at most, 2^-10 of the value."""
+    import turbospark_amd as ts
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS[name], max_context=96, **over)
+    w = synth.make_weights(cfg, seed=9)
+    one = ts.HipVerifier(cfg, w)
+    monkeypatch.setenv("TSV_ROPE_FUSED", "0")
+    apart = ts.HipVerifier(cfg, w)
+    tokens = np.random.default_rng(m).integers(0, cfg["vocab"], 21 + m).astype(np.int32)
+    out = []
+    for eng in (one, apart):
+        eng.prefill(tokens[:21], 0, want_logits=False)
+        out.append((eng.verify(tokens[21:], 21), eng.read_kv(layer, 21, m)))
+    assert gc.logit_error(out[0][0], out[1][0]) <= 2e-3
+    if layer == 0:
+        for a, b in zip(out[0][1], out[1][1]):
+            a, b = np.asarray(a).view(np.float16).astype(np.float64), np.asarray(b).view(np.float16).astype(np.float64)
+            assert (np.abs(a - b) <= 2.0 ** -10 * np.abs(b) + 1e-5 * np.abs(b).max()).all()

@@ -297,12 +297,11 @@ __device__ __forceinline__ void epilogue(const GemmArgs& a, int tile, int split,
 #define TSV_GEMM_STAGES 1
 #endif
 
+// out_tile: the tile's number in the output (a matrix whose rows follow another's)
 template <class F, int EPI, int NG>
-__global__ __launch_bounds__(512) void k_gemm(GemmArgs a) {
-    extern __shared__ float4v red[];
+__device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split, int out_tile, float4v* red) {
     constexpr int STAGES = TSV_GEMM_STAGES;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int split = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
     // this wave's run of chunks inside the workgroup's K slice
     const int s0 = split * a.kslice, s1 = min(s0 + a.kslice, a.kchunks);
     const int c0 = min(s0 + wave * a.per, s1);
@@ -353,7 +352,7 @@ __global__ __launch_bounds__(512) void k_gemm(GemmArgs a) {
 
     if (a.kparts == 1) {
 #pragma unroll
-        for (int g = 0; g < NG; g++) epilogue<EPI>(a, tile, split, g, acc[g], lane, M);
+        for (int g = 0; g < NG; g++) epilogue<EPI>(a, out_tile, split, g, acc[g], lane, M);
         return;
     }
     // fold the waves' accumulators in wave order; wave w finishes row groups w, w + kparts, ...
@@ -363,8 +362,15 @@ __global__ __launch_bounds__(512) void k_gemm(GemmArgs a) {
     for (int g = wave; g < NG; g += a.kparts) {
         float4v v = red[g * 64 + lane];
         for (int w = 1; w < a.kparts; w++) v += red[(w * NG + g) * 64 + lane];
-        epilogue<EPI>(a, tile, split, g, v, lane, M);
+        epilogue<EPI>(a, out_tile, split, g, v, lane, M);
     }
+}
+
+template <class F, int EPI, int NG>
+__global__ __launch_bounds__(512) void k_gemm(GemmArgs a) {
+    extern __shared__ float4v red[];
+    const int split = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
+    gemm_tile<F, EPI, NG>(a, tile, split, tile, red);
 }
 
 // ------------------------------------------------------------------------------- nine to sixteen rows
@@ -534,10 +540,8 @@ __device__ __forceinline__ void epilogue16(const GemmArgs& a, int tile, int spli
 }
 
 template <int EPI>
-__global__ __launch_bounds__(512) void k_gemm16(GemmArgs a) {
-    extern __shared__ float4v red[];
+__device__ __forceinline__ void gemm16_tile(const GemmArgs& a, int tile, int split, float4v* red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int split = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
     const int s0 = split * a.kslice, s1 = min(s0 + a.kslice, a.kchunks);
     const int c0 = min(s0 + wave * a.per, s1);
     const int nc = min(a.per, s1 - c0);
@@ -581,6 +585,27 @@ __global__ __launch_bounds__(512) void k_gemm16(GemmArgs a) {
             sums[xsum_index(tile, threadIdx.x)] = ssum[threadIdx.x] + ssum[16 + threadIdx.x];
         }
     }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(512) void k_gemm16(GemmArgs a) {
+    extern __shared__ float4v red[];
+    gemm16_tile<EPI>(a, blockIdx.x / a.splits, blockIdx.x % a.splits, red);
+}
+
+// The rotating q/k/v projection of files that keep the value projection in Q6_K (the *_K_M mixes): the workgroups behind those of the
+// q and k tiles take the V tiles, in one launch, and each finishes its own rows as k_gemm does with one storage type.
+// F: the q and k tiles' type; NG = 0: theirs go through the 16-row form.  Projection of q and k, projection of v and
+// rotation were three launches, of which the 16 V tiles' ran on 16 to 128 of 256 compute units: 7 us a layer less with one.  Q4_K_M, 8B
+// shape, 16 layers, four tokens one by one 4152 -> 4075 us (half of the layers have such a V); Q5_K_M, eight layers, 2561 -> 2484; rounds of
+// 5 / 12 rows, eight layers, 664 / 781 -> 652 / 768; 64-wide heads 458 / 510 -> 436 / 486.
+template <class F, int NG>
+__global__ __launch_bounds__(512) void k_gemm_qk_v(GemmArgs a, GemmArgs v) {
+    extern __shared__ float4v red[];
+    const int tile = blockIdx.x;
+    if (tile >= a.n_tiles) gemm_tile<Q6K, EPI_ROPE, NG ? NG : 4>(v, tile - a.n_tiles, 0, tile, red);
+    else if constexpr (NG == 0) gemm16_tile<EPI_ROPE>(a, tile, 0, red);
+    else gemm_tile<F, EPI_ROPE, NG>(a, tile, 0, tile, red);
 }
 
 // ------------------------------------------------------------------------------- prompt blocks of 64 rows
@@ -1219,7 +1244,9 @@ static int fill_gemm_args(GemmArgs& a, const TiledW& w, const uint4* xfrag, void
     a.ldo = ldo;
     a.n_valid = n_valid;
     if (epi == EPI_ROPE) {
-        if (!rope || (rope->hd != 64 && rope->hd != 128) || w.n_rows != (rope->nq + 2 * rope->nkv) * rope->hd) {
+        // (all of the projection, or what k_gemm_qk_v takes: q and k, or v)
+        const int heads = rope ? rope->nq + 2 * rope->nkv : 0, rows = rope ? w.n_rows / std::max(1, rope->hd) : 0;
+        if (!rope || (rope->hd != 64 && rope->hd != 128) || w.n_rows % rope->hd || (rows != heads && rows != heads - rope->nkv && rows != rope->nkv)) {
             set_error("matmul: the rotating epilogue needs the fused q/k/v projection of a 64- or 128-wide head");
             return TSV_ERR_INVALID;
         }
@@ -1250,6 +1277,40 @@ int launch_gemm(hipStream_t s, const TiledW& w, const uint4* xfrag, void* out, c
            : w.fmt == FMT_Q6K  ? launch_f<Q6K>(s, a, m, epi)
            : w.fmt == FMT_Q5K  ? launch_f<Q5K>(s, a, m, epi)
                                : launch_f<MX4>(s, a, m, epi);
+}
+
+bool gemm_qk_v_supported(const TiledW& qk, const TiledW& v) {
+    return (qk.fmt == FMT_Q4K || qk.fmt == FMT_Q5K) && v.fmt == FMT_Q6K && qk.k == v.k && qk.n_rows % TILE_ROWS == 0;
+}
+
+template <class F, int NG>
+static int launch_qk_v(hipStream_t s, const GemmArgs& a, const GemmArgs& v) {
+    const int kparts = std::max(a.kparts, v.kparts);
+    const size_t lds = std::max((size_t)kparts * (NG ? NG : 4) * 1024, (size_t)a.kparts * 4096 + 128);
+    hipLaunchKernelGGL((k_gemm_qk_v<F, NG>), dim3(a.n_tiles + v.n_tiles), dim3(64 * kparts), lds, s, a, v);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
+int launch_gemm_qk_v(hipStream_t s, const TiledW& qk, const TiledW& v, const uint4* xfrag, const VerifyParams* vp, int m, const RopeEpi& rope) {
+    if (m < 1 || m > TSV_MAX_ROWS || !gemm_qk_v_supported(qk, v) || qk.n_rows + v.n_rows != (rope.nq + 2 * rope.nkv) * rope.hd) {
+        set_error("matmul: no launch for this q/k and v projection");
+        return TSV_ERR_INVALID;
+    }
+    GemmArgs a, b;
+    if (int rc = fill_gemm_args(a, qk, xfrag, nullptr, vp, 1, EPI_ROPE, 0, qk.n_rows, &rope)) return rc;
+    if (int rc = fill_gemm_args(b, v, xfrag, nullptr, vp, 1, EPI_ROPE, 0, v.n_rows, &rope)) return rc;
+    // one workgroup shape for both: the same K in the same chunks, so as many waves as either takes serve the other's runs too
+    if (a.kparts != b.kparts) {
+        const GemmArgs& more = a.kparts > b.kparts ? a : b;
+        a.per = b.per = more.per;
+        a.kparts = b.kparts = more.kparts;
+    }
+    if (qk.fmt == FMT_Q4K) {
+        if (m >= gemm16_min_rows()) return launch_qk_v<Q4K, 0>(s, a, b);
+        return m <= 4 ? launch_qk_v<Q4K, 1>(s, a, b) : m <= 8 ? launch_qk_v<Q4K, 2>(s, a, b) : launch_qk_v<Q4K, 4>(s, a, b);
+    }
+    return m <= 4 ? launch_qk_v<Q5K, 1>(s, a, b) : m <= 8 ? launch_qk_v<Q5K, 2>(s, a, b) : launch_qk_v<Q5K, 4>(s, a, b);
 }
 
 int gemm_wide_rows() { return 16 * WIDE_BLOCKS; }

@@ -376,7 +376,8 @@ int launch_pass(tsv_ctx* c, int m) {
             PROF(PC_QKV);
             rc = 0;
             for (int rep = 0; rep < c->repeat[PC_QKV] && !rc; rep++)
-                rc = launch_gemm(s, L.qkv, c->xf_a, nullptr, c->vp_dev, m, 1, EPI_ROPE, qkv_n, L.qkv.n_rows, &re);
+                rc = L.v_only.tiles ? launch_gemm_qk_v(s, L.qkv, L.v_only, c->xf_a, c->vp_dev, m, re)
+                                    : launch_gemm(s, L.qkv, c->xf_a, nullptr, c->vp_dev, m, 1, EPI_ROPE, qkv_n, L.qkv.n_rows, &re);
         } else {
             PROF(PC_QKV);
             rc = 0;
@@ -684,7 +685,7 @@ int launch_wide_pass(tsv_ctx* c, int64_t base) {
         // The rotating epilogue needs whole sums, so its launch has one workgroup per tile (96 at the 8B shape, for 256
         // compute units: 29.7 us); split along K it fills the chip and the rotation kernel finishes all four blocks in
         // one launch.  TSV_WIDE_ROPE_FUSED=1 keeps the epilogue (not on ring layers: it stores all 64 rows at once).
-        const bool epilogue = L.rope_fused && w.keep_epilogue && !ring;
+        const bool epilogue = L.rope_fused && w.keep_epilogue && !ring && !L.v_only.tiles;
         int spq = 1;
         if (epilogue) {
             if ((rc = launch_gemm_wide(s, L.qkv, (const uint4*)w.xf_a, w.xfb, nullptr, 0, w.vp, 1, EPI_ROPE, qkv_n, L.qkv.n_rows, &re))) return rc;
@@ -1046,13 +1047,17 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         // it is taken while a tile's weights stay under 256 KiB (8B Q4_K: 147 KB per tile, a tie with the two
         // launches; gpt-oss-120B bf16: 369 KB, 15.3 us fused against 7.9 + 3.1 us apart).
         const bool light_tiles = 64 * row_bytes(s.wq.dtype, s.wq.cols) <= 256 * 1024;
-        L.rope_fused = c->rope_fused_ok && (light_tiles || c->rope_fused_force) && s.wv.dtype == s.wq.dtype &&
+        // (a Q6_K value projection beside Q4_K or Q5_K ones goes in the same launch: 215 KB a tile at 4096 columns)
+        const bool one_launch = s.wv.dtype == s.wq.dtype || ((s.wq.dtype == TSV_Q4_K || s.wq.dtype == TSV_Q5_K) && s.wv.dtype == TSV_Q6_K &&
+                                                             64 * row_bytes(TSV_Q6_K, s.wv.cols) <= 256 * 1024);
+        L.rope_fused = c->rope_fused_ok && (light_tiles || c->rope_fused_force) && one_launch &&
                        !s.q_norm.data && !s.k_norm.data && (c->hd == 64 || c->hd == 128);
         if (s.wv.dtype == s.wq.dtype) {
             if ((rc = make_tiled(c, st, qkv, 3, false, &L.qkv, L.rope_fused && c->hd == 128 ? 2 : 0))) return fail(rc);
         } else {
             const tsv_tensor* vonly[1] = {&s.wv};
-            if ((rc = make_tiled(c, st, qkv, 2, false, &L.qkv)) || (rc = make_tiled(c, st, vonly, 1, false, &L.v_only)))
+            if ((rc = make_tiled(c, st, qkv, 2, false, &L.qkv, L.rope_fused && c->hd == 128 ? 2 : 0)) ||
+                (rc = make_tiled(c, st, vonly, 1, false, &L.v_only)))
                 return fail(rc);
         }
         if ((rc = make_tiled(c, st, wo, 1, false, &L.wo))) return fail(rc);
