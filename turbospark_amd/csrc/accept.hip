@@ -1604,7 +1604,7 @@ __global__ void k_clear_result(AcceptResult* res, int32_t* err) {
 
 }  // namespace
 
-// scratch.counters (ACCEPT_COUNTER_WORDS words): [0] error flag, [32..49) tree path, [64..) the greedy
+// scratch.counters (ACCEPT_COUNTER_WORDS words): [0] error flag of an arg-max chain, [32..49) tree path, [64..) the greedy
 // arg-max partials (value, then index, per row and run); decisions live after the
 // statistics block; histograms and work arrays are separate allocations in AcceptScratch.
 size_t accept_stats_doubles() { return STATS_DOUBLES + TREE_STATE_DOUBLES; }
@@ -1629,7 +1629,7 @@ static void launch_trunc(hipStream_t s, const uint16_t* target, const uint16_t* 
                            sc.tcount, ap.has_top_p, ap_dev);
     }
     hipLaunchKernelGGL(k_trunc_cut<PEN>, dim3(rows), dim3(1024), 0, s, target, draft, ap_dev, m, sc.stats, tm, sc.tcount,
-                       sc.result, (int32_t*)sc.counters);
+                       sc.result, &sc.result->flag);
 }
 
 // The statistics of `rows` distribution rows, their truncation cuts and reweighting totals.
@@ -1640,7 +1640,7 @@ constexpr int SPLIT_ROWS = 4;
 template <bool PEN>
 static void launch_stats(hipStream_t s, const uint16_t* target, const uint16_t* draft, int m, int rows, int jobs,
                          const AcceptParams* ap_dev, const AcceptParams& ap, const AcceptScratch& sc, int slot0, int slot_step) {
-    int32_t* err = (int32_t*)sc.counters;
+    int32_t* err = &sc.result->flag;
     const double inv_t = 1.0 / ap.temperature;
     hipLaunchKernelGGL(k_row_max<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, err,
                        (unsigned long long*)sc.hist, jobs, ap_dev);
@@ -1657,7 +1657,7 @@ static void launch_stats(hipStream_t s, const uint16_t* target, const uint16_t* 
 template <bool PEN>
 static void launch_chain_sampled(hipStream_t s, const uint16_t* target, const uint16_t* draft,
                                  const AcceptParams* ap_dev, const AcceptParams& ap, const AcceptScratch& sc) {
-    int32_t* err = (int32_t*)sc.counters;
+    int32_t* err = &sc.result->flag;
     launch_stats<PEN>(s, target, draft, ap.m, ap.m + ap.k, 1, ap_dev, ap, sc, 2, 1);
     hipLaunchKernelGGL(k_mass_hist<PEN>, dim3(NSEG, 1, NSUB), dim3(256), 0, s, target, draft, ap_dev, sc.stats, sc.work,
                        (unsigned long long*)sc.hist, decisions(sc), 0);
@@ -1687,7 +1687,7 @@ int tree_walk_bound(const int32_t* parent, int m) {
 template <bool PEN>
 static void launch_tree_sampled(hipStream_t s, const uint16_t* target, const uint16_t* draft, const AcceptParams* ap_dev,
                                 const AcceptParams& ap, const AcceptScratch& sc) {
-    int32_t* err = (int32_t*)sc.counters;
+    int32_t* err = &sc.result->flag;
     int32_t* path = (int32_t*)sc.counters + 32;
     // statistics of the m target rows and the m rows the children were drawn from
     launch_stats<PEN>(s, target, draft, ap.m, 2 * ap.m, 1, ap_dev, ap, sc, 0, 1);
@@ -1704,7 +1704,7 @@ static void launch_tree_sampled(hipStream_t s, const uint16_t* target, const uin
 template <bool PEN>
 static void launch_draft_sampled(hipStream_t s, const uint16_t* draft, const AcceptParams* ap_dev,
                                  const AcceptParams& ap, const AcceptScratch& sc, int32_t* proposals_dev) {
-    int32_t* err = (int32_t*)sc.counters;
+    int32_t* err = &sc.result->flag;
     launch_stats<PEN>(s, draft, draft, 0, ap.k, ap.k, ap_dev, ap, sc, 1, 2);
     hipLaunchKernelGGL(k_mass_hist<PEN>, dim3(NSEG, ap.k, NSUB), dim3(256), 0, s, draft, draft, ap_dev, sc.stats, sc.work,
                        (unsigned long long*)sc.hist, decisions(sc), 1);
@@ -1714,10 +1714,9 @@ static void launch_draft_sampled(hipStream_t s, const uint16_t* draft, const Acc
 
 int launch_accept(hipStream_t s, const uint16_t* target, const uint16_t* draft, const AcceptParams* ap_dev,
                   const AcceptParams& ap, const AcceptScratch& sc) {
-    int32_t* err = (int32_t*)sc.counters;
+    int32_t* err = &sc.result->flag;
     float* pv = (float*)sc.counters + 64;
     int32_t* pi = (int32_t*)sc.counters + 64 + TSV_MAX_ROWS * ARGMAX_SEG;
-    hipLaunchKernelGGL(k_clear_result, dim3(1), dim3(64), 0, s, sc.result, err);
     if (!ap.sampled) {  // (the arg-max ignores penalties and truncation: choose.rs:84-88)
         hipLaunchKernelGGL(k_argmax_part, dim3(ARGMAX_SEG, ap.m), dim3(256), 0, s, target, ap.vocab, pv, pi, err);
         hipLaunchKernelGGL(k_walk_greedy, dim3(1), dim3(64), 0, s, ap_dev, pv, pi, sc.result, err);
@@ -1744,8 +1743,7 @@ int launch_accept(hipStream_t s, const uint16_t* target, const uint16_t* draft, 
 // or the arg-max at temperature 0.  ap_dev: m = 0, k = rows, draw_step = first position.
 int launch_draft_chain(hipStream_t s, const uint16_t* draft, const AcceptParams* ap_dev, const AcceptParams& ap,
                        const AcceptScratch& sc, int32_t* proposals_dev) {
-    int32_t* err = (int32_t*)sc.counters;
-    hipLaunchKernelGGL(k_clear_result, dim3(1), dim3(64), 0, s, sc.result, err);
+    int32_t* err = &sc.result->flag;
     if (!ap.sampled) {
         float* pv = (float*)sc.counters + 64;
         int32_t* pi = (int32_t*)sc.counters + 64 + TSV_MAX_ROWS * ARGMAX_SEG;

@@ -143,9 +143,11 @@ struct tsv_ctx {
         bool used[SLOTS] = {};
         int next = 0;
     } ring;
-    AcceptParams *ap_dev = nullptr, *ap_host = nullptr;
+    AcceptUpload *up_dev = nullptr, *up_host = nullptr;
+    // the stream may still be reading the pinned blocks that calls upload from (a call that failed between its copy and its wait)
+    bool uploading = false;
     uint16_t** kv_ptrs = nullptr;  // device: [2 * layer] = K buffer, [2 * layer + 1] = V buffer (tree compaction)
-    int32_t* hist_dev = nullptr;  // the token history of a penalised round (grows on demand)
+    int32_t *hist_dev = nullptr, *hist_host = nullptr;  // the token history of a penalised round (grows on demand), and its pinned copy
     size_t hist_cap = 0;
     uint32_t* pen_cnt = nullptr;  // [vocab] seen flag + generated-suffix count per token
     AcceptResult* res_host = nullptr;
@@ -210,9 +212,15 @@ struct tsv_ctx {
         bool own_valid = false;  // x row 0 is this head's own residual of the step at position - 1 (a chained step)
         const int32_t* feed_dev = nullptr;  // the pass in flight takes row 0's token from device memory
         bool params_staged = false;         // ... and finds its parameter block on the device already (vp_dev)
-        VerifyParams *vp_block = nullptr, *vp_block_host = nullptr;  // [16] the parameter blocks of a block draft's steps
-        int32_t *chain = nullptr, *chain_host = nullptr;  // the tokens of a block draft and the error word
-        AcceptParams *draw_dev = nullptr, *draw_host = nullptr;  // [16] the draw parameters of a sampled block's steps
+        // what a block draft's steps read, uploaded in one copy: the tokens (the anchor, then each step's pick), the steps' parameter
+        // blocks and, of a sampled block, their draws'
+        struct Block {
+            int32_t chain[32];
+            VerifyParams vp[TSV_MAX_ROWS];
+            AcceptUpload draw[TSV_MAX_ROWS];
+        };
+        Block *block = nullptr, *block_host = nullptr;
+        int32_t* chain_host = nullptr;  // the picks and the error word as they come back
         uint8_t *prompt_a = nullptr, *prompt_s = nullptr;  // fc's input rows as a prompt matmul's activations and their sums; null: none
     } mtp;
     int64_t x_base = -1;  // rows [0, x_rows) of x are the finished residual rows of positions x_base ..
@@ -270,6 +278,9 @@ int prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0, uint
                    int32_t next_token = -1);
 // one pass of a drafter head over m rows at position ..: row r pairs next_tokens[r] with row r of h_rows (mtp.hip)
 int mtp_pass(tsv_ctx* c, const int32_t* next_tokens, int m, int64_t position, const float* h_rows, bool want_logits);
+// before a pinned upload block is rewritten, and after the wait that ends a call
+int upload_begin(tsv_ctx* c);
+int upload_end(tsv_ctx* c);
 void fill_truncation(AcceptParams* ap, const tsv_shaping& sh);
 int setup_penalties(tsv_ctx* c, const tsv_shaping& sh, const int32_t* history, int64_t n, uint64_t generated, AcceptParams* ap);
 const char* accept_error_text(int bits);

@@ -106,14 +106,24 @@ extern "C" int32_t tsv_mtp_prefill_chunk(tsv_ctx* c, const int32_t* tokens, int6
     return rc;
 }
 
-// The parameter blocks of a block draft's steps (one row each at base - 1 + d, d = 0 .. block) to the device in ONE copy;
-// step d then runs with vp_dev naming its block and stages nothing.
-static int stage_block_params(tsv_ctx* c, int64_t base, int block) {
+// The anchor and the parameter blocks of a block draft's steps (one row each at base - 1 + d, d = 0 .. block), and with `ap` its draws'
+// parameters (draw d at position draw_step + d) and cleared results, to the device in ONE copy; step d then runs with vp_dev naming its
+// block and stages nothing.
+static int stage_block(tsv_ctx* c, int32_t anchor, int64_t base, int block, const AcceptParams* ap, uint64_t draw_step) {
     tsv_ctx::Mtp& h = c->mtp;
     const int32_t none = 0;
+    h.block_host->chain[0] = anchor;
     for (int d = 0; d <= block; d++)
-        if (int rc = fill_params(h.vp_block_host[d], &none, nullptr, 1, base - 1 + d, c->vocab)) return rc;
-    TSV_HIP(hipMemcpyAsync(h.vp_block, h.vp_block_host, (size_t)(block + 1) * sizeof(VerifyParams), hipMemcpyHostToDevice, c->stream));
+        if (int rc = fill_params(h.block_host->vp[d], &none, nullptr, 1, base - 1 + d, c->vocab)) return rc;
+    for (int d = 0; ap && d < block; d++) {
+        AcceptUpload& u = h.block_host->draw[d];
+        u.ap = *ap;
+        u.ap.draw_step = draw_step + (uint64_t)d;
+        u.clear_result();
+    }
+    const size_t bytes = ap ? offsetof(tsv_ctx::Mtp::Block, draw) + block * sizeof(AcceptUpload)
+                            : offsetof(tsv_ctx::Mtp::Block, vp) + (block + 1) * sizeof(VerifyParams);
+    TSV_HIP(hipMemcpyAsync(h.block, h.block_host, bytes, hipMemcpyHostToDevice, c->stream));
     return TSV_OK;
 }
 
@@ -131,30 +141,28 @@ extern "C" int32_t tsv_mtp_draft_block(tsv_ctx* c, int32_t anchor, int64_t base,
         return TSV_ERR_INVALID;
     }
     // every step takes its token from chain[d] on the device: the anchor is put there with the parameter blocks
-    h.chain_host[30] = anchor;
-    TSV_HIP(hipMemcpyAsync(h.chain, h.chain_host + 30, 4, hipMemcpyHostToDevice, c->stream));
-    if ((rc = stage_block_params(c, base, block))) return rc;
+    if ((rc = upload_begin(c)) || (rc = stage_block(c, anchor, base, block, nullptr, 0))) return rc;
     VerifyParams* const vp_own = c->vp_dev;
     for (int d = 0; d <= block; d++) {
         // step d pairs the state of base - 1 + d with the token at base + d: the anchor, then each pick of the
         // step before, read where the arg-max left it; the last step is the row-only one (speculative.rs:612-625)
         const float* src = nullptr;
         if ((rc = mtp_source(c, base - 1 + d, &src))) break;
-        h.feed_dev = h.chain + d;
+        h.feed_dev = h.block->chain + d;
         h.params_staged = true;
-        c->vp_dev = h.vp_block + d;
+        c->vp_dev = h.block->vp + d;
         rc = mtp_pass(c, &none, 1, base - 1 + d, src, d < block);
         c->vp_dev = vp_own;
         h.params_staged = false;
         h.feed_dev = nullptr;
         if (rc) return rc;
-        if (d < block && (rc = launch_argmax_rows(c->stream, c->logits, 1, c->vocab, c->sc, h.chain + d + 1, d == 0))) return rc;
+        if (d < block && (rc = launch_argmax_rows(c->stream, c->logits, 1, c->vocab, c->sc, h.block->chain + d + 1, d == 0))) return rc;
     }
     if (rc) return rc;
     h.own_valid = false;
-    TSV_HIP(hipMemcpyAsync(h.chain_host, h.chain + 1, (size_t)block * 4, hipMemcpyDeviceToHost, c->stream));
+    TSV_HIP(hipMemcpyAsync(h.chain_host, h.block->chain + 1, (size_t)block * 4, hipMemcpyDeviceToHost, c->stream));
     TSV_HIP(hipMemcpyAsync(h.chain_host + 31, c->sc.counters, 4, hipMemcpyDeviceToHost, c->stream));
-    TSV_HIP(hipStreamSynchronize(c->stream));
+    if ((rc = upload_end(c))) return rc;
     if (h.chain_host[31]) {
         set_error("mtp_draft_block: score vector must not contain a non-finite entry");
         return TSV_ERR_INVALID;
@@ -187,40 +195,38 @@ int tsv_mtp_draft_block_sampled(tsv_ctx* c, int32_t anchor, int64_t base, int32_
     ap.temperature = sh->temperature;
     ap.seed = sh->seed;
     fill_truncation(&ap, *sh);
-    if ((rc = setup_penalties(c, *sh, history, n_history, generated, &ap))) return rc;  // the same history for every step of a round
+    if ((rc = upload_begin(c)) || (rc = setup_penalties(c, *sh, history, n_history, generated, &ap))) return rc;  // the same history for every step of a round
     const int32_t none = 0;
     if (anchor < 0 || anchor >= c->vocab) {
         set_error("mtp_draft_block: token id outside the vocabulary");
         return TSV_ERR_INVALID;
     }
-    h.chain_host[30] = anchor;
-    TSV_HIP(hipMemcpyAsync(h.chain, h.chain_host + 30, 4, hipMemcpyHostToDevice, c->stream));
-    if ((rc = stage_block_params(c, base, block))) return rc;
+    if ((rc = stage_block(c, anchor, base, block, &ap, draw_step))) return rc;
     VerifyParams* const vp_own = c->vp_dev;
     for (int d = 0; d <= block; d++) {
         const float* src = nullptr;
         if ((rc = mtp_source(c, base - 1 + d, &src))) return rc;
-        h.feed_dev = h.chain + d;
+        h.feed_dev = h.block->chain + d;
         h.params_staged = true;
-        c->vp_dev = h.vp_block + d;
+        c->vp_dev = h.block->vp + d;
+        uint16_t *const row = rows + (size_t)d * c->vocab, *const own = c->logits;
+        if (d < block) c->logits = row;  // (the pass writes the row where it is kept)
         rc = mtp_pass(c, &none, 1, base - 1 + d, src, d < block);
+        c->logits = own;
         c->vp_dev = vp_own;
         h.params_staged = false;
         h.feed_dev = nullptr;
         if (rc) return rc;
         if (d == block) break;
-        uint16_t* row = rows + (size_t)d * c->vocab;
-        TSV_HIP(hipMemcpyAsync(row, c->logits, (size_t)c->vocab * 2, hipMemcpyDeviceToDevice, c->stream));
-        h.draw_host[d] = ap;
-        h.draw_host[d].draw_step = draw_step + (uint64_t)d;
-        TSV_HIP(hipMemcpyAsync(h.draw_dev + d, h.draw_host + d, sizeof(AcceptParams), hipMemcpyHostToDevice, c->stream));
-        if ((rc = launch_draft_chain(c->stream, row, h.draw_dev + d, h.draw_host[d], c->sc, h.chain + d + 1))) return rc;
+        AcceptScratch sc = c->sc;
+        sc.result = &h.block->draw[d].res;
+        if ((rc = launch_draft_chain(c->stream, row, &h.block->draw[d].ap, h.block_host->draw[d].ap, sc, h.block->chain + d + 1))) return rc;
     }
     h.own_valid = false;
-    TSV_HIP(hipMemcpyAsync(h.chain_host, h.chain + 1, (size_t)block * 4, hipMemcpyDeviceToHost, c->stream));
-    TSV_HIP(hipMemcpyAsync(c->res_host, c->sc.result, sizeof(AcceptResult), hipMemcpyDeviceToHost, c->stream));
-    TSV_HIP(hipStreamSynchronize(c->stream));
-    if (c->res_host->error) {  // (each step's draw clears the flag first: this is the last step's)
+    TSV_HIP(hipMemcpyAsync(h.chain_host, h.block->chain + 1, (size_t)block * 4, hipMemcpyDeviceToHost, c->stream));
+    TSV_HIP(hipMemcpyAsync(c->res_host, &h.block->draw[block - 1].res, sizeof(AcceptResult), hipMemcpyDeviceToHost, c->stream));
+    if ((rc = upload_end(c))) return rc;
+    if (c->res_host->error) {  // (every draw has a result of its own: this is the last step's)
         set_error(std::string("mtp_draft_block: ") + accept_error_text(c->res_host->error));
         return (c->res_host->error & 1) ? TSV_ERR_INVALID : TSV_ERR_UNSUPPORTED;
     }

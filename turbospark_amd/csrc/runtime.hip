@@ -1327,7 +1327,7 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         (rc = dev_alloc(c, &c->logits, (size_t)16 * c->vocab * 2, true)) ||
         (rc = dev_alloc(c, &c->draft_stage, (size_t)16 * c->vocab * 2, true)) ||
         (rc = dev_alloc(c, &c->vp_dev, sizeof(VerifyParams), true)) ||
-        (rc = dev_alloc(c, &c->ap_dev, sizeof(AcceptParams), true)) ||
+        (rc = dev_alloc(c, &c->up_dev, sizeof(AcceptUpload), true)) ||
         (rc = dev_alloc(c, &c->pen_cnt, (size_t)c->vocab * 4, true)) ||
         (rc = dev_alloc(c, &c->tok_dev, 64 * 4, true)) ||
         (rc = dev_alloc(c, &c->sc.stats, accept_stats_doubles() * 8, true)) ||
@@ -1335,9 +1335,9 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         (rc = dev_alloc(c, &c->sc.hist, accept_hist_words() * 8, true)) ||
         (rc = dev_alloc(c, &c->sc.counters, ACCEPT_COUNTER_WORDS * 4, true)) ||
         (rc = dev_alloc(c, &c->sc.tmass, (size_t)32 * 65536 * 8, true)) ||
-        (rc = dev_alloc(c, &c->sc.tcount, (size_t)32 * 65536 * 4, true)) ||
-        (rc = dev_alloc(c, &c->sc.result, sizeof(AcceptResult), true)))
+        (rc = dev_alloc(c, &c->sc.tcount, (size_t)32 * 65536 * 4, true)))
         return fail(rc);
+    c->sc.result = &c->up_dev->res;
     if (c->route_forced && hipMemsetAsync(c->route_forced, 0xFF, (size_t)c->n_layers * 16 * 8 * 4, c->stream) != hipSuccess)
         return fail(TSV_ERR_DEVICE);  // every entry -1: rows route freely until tsv_force_route says otherwise
     for (hipEvent_t& e : c->ring.ev)
@@ -1347,7 +1347,7 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         }
     if (hipHostMalloc((void**)&c->ring.host, sizeof(VerifyParams) * tsv_ctx::ParamRing::SLOTS * tsv_ctx::ParamRing::PER_SLOT) != hipSuccess ||
         hipHostMalloc((void**)&c->vp_host, sizeof(VerifyParams)) != hipSuccess ||
-        hipHostMalloc((void**)&c->ap_host, sizeof(AcceptParams)) != hipSuccess ||
+        hipHostMalloc((void**)&c->up_host, sizeof(AcceptUpload)) != hipSuccess ||
         hipHostMalloc((void**)&c->res_host, sizeof(AcceptResult)) != hipSuccess ||
         hipHostMalloc((void**)&c->tok_host, 64 * 4) != hipSuccess) {
         set_error("open: pinned host allocation failed");
@@ -1355,13 +1355,9 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
     }
     if (share) {
         tsv_ctx::Mtp& h = c->mtp;
-        if ((rc = dev_alloc(c, &h.xf_cat, xfrag_bytes(2 * c->hidden), true)) || (rc = dev_alloc(c, &h.chain, 32 * 4, true)) ||
-            (rc = dev_alloc(c, &h.vp_block, TSV_MAX_ROWS * sizeof(VerifyParams), true)) ||
-            (rc = dev_alloc(c, &h.draw_dev, TSV_MAX_ROWS * sizeof(AcceptParams), true)))
+        if ((rc = dev_alloc(c, &h.xf_cat, xfrag_bytes(2 * c->hidden), true)) || (rc = dev_alloc(c, &h.block, sizeof *h.block, true)))
             return fail(rc);
-        if (hipHostMalloc((void**)&h.chain_host, 32 * 4) != hipSuccess ||
-            hipHostMalloc((void**)&h.draw_host, TSV_MAX_ROWS * sizeof(AcceptParams)) != hipSuccess ||
-            hipHostMalloc((void**)&h.vp_block_host, TSV_MAX_ROWS * sizeof(VerifyParams)) != hipSuccess) {
+        if (hipHostMalloc((void**)&h.chain_host, 32 * 4) != hipSuccess || hipHostMalloc((void**)&h.block_host, sizeof *h.block_host) != hipSuccess) {
             set_error("mtp_open: pinned host allocation failed");
             return fail(TSV_ERR_DEVICE);
         }
@@ -1404,12 +1400,12 @@ extern "C" void tsv_close(tsv_ctx* c) {
     if (c->ring.host) (void)hipHostFree(c->ring.host);
     for (hipEvent_t e : c->ring.ev)
         if (e) (void)hipEventDestroy(e);
-    if (c->ap_host) (void)hipHostFree(c->ap_host);
+    if (c->up_host) (void)hipHostFree(c->up_host);
+    if (c->hist_host) (void)hipHostFree(c->hist_host);
     if (c->res_host) (void)hipHostFree(c->res_host);
     if (c->tok_host) (void)hipHostFree(c->tok_host);
     if (c->mtp.chain_host) (void)hipHostFree(c->mtp.chain_host);
-    if (c->mtp.draw_host) (void)hipHostFree(c->mtp.draw_host);
-    if (c->mtp.vp_block_host) (void)hipHostFree(c->mtp.vp_block_host);
+    if (c->mtp.block_host) (void)hipHostFree(c->mtp.block_host);
     if (c->mtp.on && c->mtp.target && c->mtp.target->mtp_head == c) c->mtp.target->mtp_head = nullptr;
     for (auto& graphs : c->pass_graph)
         for (hipGraphExec_t g : graphs)
@@ -1763,6 +1759,18 @@ extern "C" int32_t tsv_compact_tree(tsv_ctx* c, int64_t base, const uint32_t* pa
 
 namespace tsv {
 
+int upload_begin(tsv_ctx* c) {
+    if (c->uploading) TSV_HIP(hipStreamSynchronize(c->stream));
+    c->uploading = true;
+    return TSV_OK;
+}
+
+int upload_end(tsv_ctx* c) {
+    TSV_HIP(hipStreamSynchronize(c->stream));
+    c->uploading = false;
+    return TSV_OK;
+}
+
 void fill_truncation(AcceptParams* ap, const tsv_shaping& sh) {
     ap->top_k = (int32_t)sh.top_k;
     ap->has_top_p = sh.has_top_p != 0;
@@ -1810,17 +1818,21 @@ int setup_penalties(tsv_ctx* c, const tsv_shaping& sh, const int32_t* history, i
     }
     if ((size_t)n > c->hist_cap) {
         if (c->hist_dev) TSV_HIP(hipFree(c->hist_dev));
-        c->hist_dev = nullptr;
+        if (c->hist_host) TSV_HIP(hipHostFree(c->hist_host));
+        c->hist_dev = c->hist_host = nullptr;
         c->hist_cap = 0;
         const size_t cap = ((size_t)n + 4095) & ~(size_t)4095;
         TSV_HIP(hipMalloc((void**)&c->hist_dev, cap * 4));
+        TSV_HIP(hipHostMalloc((void**)&c->hist_host, cap * 4));
         c->hist_cap = cap;
     }
-    if (n > 0) TSV_HIP(hipMemcpyAsync(c->hist_dev, history, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
+    if (n > 0) {  // by way of pinned memory: the caller's buffer is free again without a wait for the pass that is under way
+        std::memcpy(c->hist_host, history, (size_t)n * 4);
+        TSV_HIP(hipMemcpyAsync(c->hist_dev, c->hist_host, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
+    }
     const int64_t suffix = (int64_t)std::min<uint64_t>(generated, (uint64_t)n);
     int rc = launch_pen_counts(c->stream, c->hist_dev, (long)n, (long)(n - suffix), c->vocab, c->pen_cnt);
     if (rc) return rc;
-    if (n > 0) TSV_HIP(hipStreamSynchronize(c->stream));  // the caller's history buffer is free again
     ap->pen = 1;
     ap->pen_has_rep = sh.repetition_penalty != 1.0;
     // penalty.rs:20-25: the f64 setting as an f32 kept inside the normal range
@@ -1889,19 +1901,22 @@ int accept_impl(tsv_ctx* c, const tsv_round* r, tsv_round_result* out) {
         }
         if ((rc = stage_draft(c, r->draft_logits, r->parent ? r->m : r->m - 1, &draft))) return rc;
     }
-    TSV_HIP(hipStreamSynchronize(c->stream));  // pinned parameter block is about to be rewritten
-    if ((rc = fill_accept(c, r, c->ap_host))) return rc;
-    if ((rc = setup_penalties(c, r->shaping, r->history, r->n_history, r->generated, c->ap_host))) return rc;
-    TSV_HIP(hipMemcpyAsync(c->ap_dev, c->ap_host, sizeof(AcceptParams), hipMemcpyHostToDevice, c->stream));
+    // (no wait for the pass: its launches and these are one queue, with the host ahead of the device throughout)
+    if ((rc = upload_begin(c))) return rc;
+    AcceptParams* ap = &c->up_host->ap;
+    if ((rc = fill_accept(c, r, ap))) return rc;
+    if ((rc = setup_penalties(c, r->shaping, r->history, r->n_history, r->generated, ap))) return rc;
+    c->up_host->clear_result();
+    TSV_HIP(hipMemcpyAsync(c->up_dev, c->up_host, sizeof(AcceptUpload), hipMemcpyHostToDevice, c->stream));
     {
         PROF(PC_ACCEPT);
-        rc = launch_accept(c->stream, c->logits, draft, c->ap_dev, *c->ap_host, c->sc);
+        rc = launch_accept(c->stream, c->logits, draft, &c->up_dev->ap, *ap, c->sc);
     }
     if (rc) return rc;
     TSV_HIP(hipMemcpyAsync(c->res_host, c->sc.result, sizeof(AcceptResult), hipMemcpyDeviceToHost, c->stream));
     if (r->logits_out)
         TSV_HIP(hipMemcpyAsync(r->logits_out, c->logits, (size_t)r->m * c->vocab * 2, hipMemcpyDeviceToHost, c->stream));
-    TSV_HIP(hipStreamSynchronize(c->stream));
+    if ((rc = upload_end(c))) return rc;
     const AcceptResult& a = *c->res_host;
     if (a.error) {
         set_error(std::string("accept: ") + accept_error_text(a.error));
@@ -1962,8 +1977,8 @@ extern "C" int32_t tsv_draft_chain(tsv_ctx* c, const uint16_t* draft_logits, int
     if (rc) return rc;
     const uint16_t* draft = nullptr;
     if ((rc = stage_draft(c, draft_logits, k, &draft))) return rc;
-    TSV_HIP(hipStreamSynchronize(c->stream));
-    AcceptParams* ap = c->ap_host;
+    if ((rc = upload_begin(c))) return rc;
+    AcceptParams* ap = &c->up_host->ap;
     std::memset(ap, 0, sizeof *ap);
     ap->m = 0;
     ap->k = k;
@@ -1974,11 +1989,12 @@ extern "C" int32_t tsv_draft_chain(tsv_ctx* c, const uint16_t* draft_logits, int
     fill_truncation(ap, *sh);
     ap->draw_step = *draw_step;
     if ((rc = setup_penalties(c, *sh, history, n_history, generated, ap))) return rc;
-    TSV_HIP(hipMemcpyAsync(c->ap_dev, ap, sizeof *ap, hipMemcpyHostToDevice, c->stream));
-    if ((rc = launch_draft_chain(c->stream, draft, c->ap_dev, *ap, c->sc, c->tok_dev))) return rc;
+    c->up_host->clear_result();
+    TSV_HIP(hipMemcpyAsync(c->up_dev, c->up_host, sizeof(AcceptUpload), hipMemcpyHostToDevice, c->stream));
+    if ((rc = launch_draft_chain(c->stream, draft, &c->up_dev->ap, *ap, c->sc, c->tok_dev))) return rc;
     TSV_HIP(hipMemcpyAsync(c->tok_host, c->tok_dev, (size_t)k * 4, hipMemcpyDeviceToHost, c->stream));
     TSV_HIP(hipMemcpyAsync(c->res_host, c->sc.result, sizeof(AcceptResult), hipMemcpyDeviceToHost, c->stream));
-    TSV_HIP(hipStreamSynchronize(c->stream));
+    if ((rc = upload_end(c))) return rc;
     if (c->res_host->error) {
         set_error(std::string("draft_chain: ") + accept_error_text(c->res_host->error));
         return (c->res_host->error & 1) ? TSV_ERR_INVALID : TSV_ERR_UNSUPPORTED;

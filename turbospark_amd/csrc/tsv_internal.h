@@ -509,6 +509,16 @@ struct AcceptResult {
     int32_t path_len;
     double min_margin;
     int32_t error;  // 1: non-finite logit
+    int32_t flag;   // the same while the round runs
+};
+// A round's parameters and the result it starts from, which go to the device in one copy: nothing is left to clear there
+struct AcceptUpload {
+    AcceptParams ap;
+    AcceptResult res;
+    void clear_result() {
+        res = AcceptResult{};
+        res.min_margin = 1.0;
+    }
 };
 struct AcceptScratch {
     double* stats;       // accept_stats_doubles() doubles: row statistics, partials, decisions
@@ -518,7 +528,7 @@ struct AcceptScratch {
     uint32_t* counters;  // ACCEPT_COUNTER_WORDS words: error flag, tree path, greedy arg-max partials
     uint64_t* tmass;     // [32 rows][65536] fixed-point softmax mass per rank bin (top-p cut)
     uint32_t* tcount;    // [32 rows][65536] candidates per rank bin (top-k / top-p cut)
-    AcceptResult* result;  // device
+    AcceptResult* result;  // device; the caller uploads it cleared with a round's parameters
 };
 constexpr int ACCEPT_COUNTER_WORDS = 1024;
 size_t accept_stats_doubles(), accept_hist_words();
