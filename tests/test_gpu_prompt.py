@@ -270,6 +270,24 @@ def test_routed_prompts_give_every_row_its_experts(name, n):
         assert far.sum() <= max(1, n // 50), np.flatnonzero(far)
 
 
+# the most experts and the most pairs of a pass, every expert chosen by every row (runs without a padded block, no block past the
+# last), few pairs for many experts (most blocks lie past the last run); an odd count for the last block's filling
+@pytest.mark.parametrize("experts,top_k,n", [(256, 8, 2048), (8, 8, 2048), (256, 8, 97), (3, 1, 81), (1, 1, 96)])
+def test_routed_prompts_at_the_limits_of_the_sort(experts, top_k, n):
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS["moe_small"], max_context=n + 32, n_experts=experts, top_k=top_k)
+    w = synth.make_weights(cfg, seed=5)
+    fast, slow = gc.engine(cfg, w, "prompt"), gc.engine(cfg, w, "16")
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
+    for eng in (fast, slow):
+        eng.prefill(prompt, 0, want_logits=False)
+    assert gc.took(fast, "prompt") and gc.took(slow, "16")
+    for got, want in zip(fast.read_kv(1, 0, n), slow.read_kv(1, 0, n)):
+        got, want = got.astype(np.float32).reshape(n, -1), want.astype(np.float32).reshape(n, -1)
+        far = np.abs(got - want).max(1) > 8 * 2.0 ** -11 * np.abs(want).max(1)   # as above
+        assert far.sum() <= max(1, n // 50), np.flatnonzero(far)
+
+
 # experts in every storage type: with sums (Q4_K, Q5_K: of the gathered rows, and of what gate / up leave), without, and mixed;
 # 16 experts of which four are chosen, 21 to 94 members an expert (tiles of 64 rows) and 188 (128)
 @pytest.mark.parametrize("expert,down", [(12, 12), (13, 14), (14, 13), (8, 8), (30, 30), (12, 8), (39, 12)])

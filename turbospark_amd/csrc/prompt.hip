@@ -770,71 +770,86 @@ __global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
 
 // ---- routed experts: pairs sorted by expert -------------------------------------------------------------------------------
 // One workgroup: counts, runs and tiles of all experts, then every pair's place.  (Where a pair lands inside its expert's run
-// depends on the order of the atomics; no value does: a row of a product does not see its neighbours.)
+// depends on the order of the atomics; no value does: a row of a product does not see its neighbours.)  Bound by round trips, not
+// by bytes: a thread's choices are read once, all in flight, and the count's own atomic says where in the run each goes; the
+// sums over the experts cross lanes, not barriers.  GROUPS_FIGURES
 constexpr int MAX_EXPERTS = 256;
+constexpr int GROUP_SLOTS = PROMPT_ROWS * 8 / 1024;  // of a thread
 __global__ __launch_bounds__(1024) void k_prompt_groups(const int32_t* __restrict__ selected, int n, int top_k, int ne, int bm, PromptRoutes r) {
-    __shared__ int cnt[MAX_EXPERTS], at[MAX_EXPERTS], scan[2][MAX_EXPERTS];
-    const int tid = threadIdx.x;
+    __shared__ int cnt[MAX_EXPERTS], first[MAX_EXPERTS], part[MAX_EXPERTS / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int expert[GROUP_SLOTS], place[GROUP_SLOTS];
+#pragma unroll
+    for (int i = 0; i < GROUP_SLOTS; i++) {
+        const int q = tid + i * 1024;  // row * 8 + slot
+        expert[i] = q < n * 8 && (q & 7) < top_k ? min(max(selected[q], 0), ne - 1) : -1;
+    }
     if (tid < MAX_EXPERTS) cnt[tid] = 0;
     __syncthreads();
-    const int np = n * top_k;
-    for (int p = tid; p < np; p += 1024) {
-        const int row = p / top_k, e = min(max(selected[row * 8 + p - row * top_k], 0), ne - 1);
-        atomicAdd(&cnt[e], 1);
-    }
+#pragma unroll
+    for (int i = 0; i < GROUP_SLOTS; i++)
+        if (expert[i] >= 0) place[i] = atomicAdd(&cnt[expert[i]], 1);
     __syncthreads();
-    // exclusive sums over the experts: rows of the padded runs, then tiles
-    int padded = 0, tiles = 0;
+    // sums over the experts: rows of the padded runs (16 bits: 8 of 2048 rows, 31 more for each of 256 experts), tiles above them
+    static_assert(PROMPT_ROWS * 8 + MAX_EXPERTS * 31 < 1 << 16, "packed sums");
+    uint32_t mine = 0, upto = 0;
     if (tid < MAX_EXPERTS) {
-        padded = (cnt[tid] + 31) & ~31;
-        tiles = (cnt[tid] + bm - 1) / bm;
-        scan[0][tid] = padded;
-        scan[1][tid] = tiles;
+        mine = (uint32_t)(((cnt[tid] + 31) & ~31) | (cnt[tid] + bm - 1) / bm << 16);
+        upto = mine;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t below = __shfl_up(upto, o);
+            if (lane >= o) upto += below;
+        }
+        if (lane == 63) part[wave] = (int)upto;
     }
     __syncthreads();
-    for (int o = 1; o < MAX_EXPERTS; o <<= 1) {
-        int a = 0, b = 0;
-        if (tid >= o && tid < MAX_EXPERTS) {
-            a = scan[0][tid - o];
-            b = scan[1][tid - o];
-        }
-        __syncthreads();
-        if (tid < MAX_EXPERTS) {
-            scan[0][tid] += a;
-            scan[1][tid] += b;
-        }
-        __syncthreads();
+    uint32_t all = 0;
+#pragma unroll
+    for (int w = 0; w < MAX_EXPERTS / 64; w++) {
+        if (w < wave) upto += (uint32_t)part[w];
+        all += (uint32_t)part[w];
     }
     if (tid < ne) {
-        const int first = scan[0][tid] - padded, t0 = scan[1][tid] - tiles;
-        at[tid] = first;
-        for (int t = 0; t < tiles; t++) r.tiles[t0 + t] = PromptTile{tid, first + t * bm, min(bm, cnt[tid] - t * bm), 0};
-        if (tid == ne - 1) *r.n_tiles = scan[1][tid];
-        for (int q = cnt[tid]; q < padded; q++) r.pair[first + q] = -1;
+        const int at = (int)((upto - mine) & 0xFFFF), t0 = (int)((upto - mine) >> 16), tiles = (int)(mine >> 16);
+        first[tid] = at;
+        for (int t = 0; t < tiles; t++) r.tiles[t0 + t] = PromptTile{tid, at + t * bm, min(bm, cnt[tid] - t * bm), 0};
     }
-    if (tid == 0)
-        for (int q = scan[0][ne - 1]; q < prompt_sorted_rows(n, top_k, ne); q += 32) r.pair[q] = -2;  // a block past the last run
+    if (tid == 0) *r.n_tiles = (int)(all >> 16);
+    for (int q = (int)(all & 0xFFFF) + tid * 32; q < prompt_sorted_rows(n, top_k, ne); q += 32 * 1024) r.pair[q] = -2;  // a block past the last run
     __syncthreads();
-    for (int p = tid; p < np; p += 1024) {
-        const int row = p / top_k, slot = p - row * top_k, e = min(max(selected[row * 8 + slot], 0), ne - 1);
-        r.pair[atomicAdd(&at[e], 1)] = row * 8 + slot;
-    }
+    const int e = tid >> 2;  // four threads fill an expert's last block
+    if (e < ne)
+        for (int q = cnt[e] + (tid & 3); q < ((cnt[e] + 31) & ~31); q += 4) r.pair[first[e] + q] = -1;
+#pragma unroll
+    for (int i = 0; i < GROUP_SLOTS; i++)
+        if (expert[i] >= 0) r.pair[first[expert[i]] + place[i]] = tid + i * 1024;
 }
 
-// One workgroup per 32 sorted pairs: lane = pair, so the stores are whole lines of the operand layout; the sixteen-byte loads of
-// a row's line come from the eight half waves side by side
+// 32 sorted pairs to a workgroup, of a part of K: lane = pair, so the stores are whole lines of the operand layout; the
+// sixteen-byte loads of a row's line come from the eight half waves side by side, four of a thread in flight.
+// Bound by round trips: 374 workgroups of whole rows (8000 x 2048) took 16.0 us, in three parts of K 13.6; 312 (6000 x 2880) 21.5,
+// in four 14.6.
 __global__ __launch_bounds__(256) void k_prompt_gather(const uint16_t* __restrict__ rows, const uint8_t* __restrict__ row_sums, int k16,
                                                        const int32_t* __restrict__ pair, int n_sorted, uint8_t* __restrict__ a, uint8_t* __restrict__ asum) {
-    const int p = blockIdx.x * 32 + (threadIdx.x & 31);
+    const int p = blockIdx.x * 32 + (threadIdx.x & 31), half = threadIdx.x >> 5;
     if (pair[blockIdx.x * 32] == -2 || p >= n_sorted) return;
     const int pr = pair[p];
     if (pr < 0) return;
     const u32x4* src = (const u32x4*)(rows + (size_t)(pr >> 3) * (k16 * 16));
     u32x4* dst = (u32x4*)(a + (size_t)blockIdx.x * k16 * 1024) + (threadIdx.x & 31);
-    for (int k8 = threadIdx.x >> 5; k8 < 2 * k16; k8 += 8) dst[k8 * 32] = src[k8];
+    const int end = 2 * k16;
+    for (int k8 = blockIdx.y * 32 + half; k8 < end; k8 += gridDim.y * 32) {
+        u32x4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (k8 + 8 * j < end) v[j] = src[k8 + 8 * j];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (k8 + 8 * j < end) dst[(k8 + 8 * j) * 32] = v[j];
+    }
     if (!asum) return;
     const int row = pr >> 3, kc = k16 >> 4;
-    for (int c = threadIdx.x >> 5; c < 2 * kc; c += 8)  // (both halves of the sums of every 256 K)
+    for (int c = blockIdx.y * 8 + half; c < 2 * kc; c += gridDim.y * 8)  // (both halves of the sums of every 256 K)
         *(u32x4*)(asum + ((size_t)blockIdx.x * 2 * kc + c) * 512 + (threadIdx.x & 31) * 16) =
             *(const u32x4*)(row_sums + ((size_t)(row >> 5) * 2 * kc + c) * 512 + (row & 31) * 16);
 }
@@ -895,8 +910,8 @@ int launch_prompt_norm(hipStream_t s, const PromptNormArgs& a) {
 }
 
 int launch_prompt_groups(hipStream_t s, const int32_t* selected, int n, int top_k, int n_experts, int bm, const PromptRoutes& r) {
-    if (n < 1 || n_experts < 1 || n_experts > MAX_EXPERTS || top_k < 1 || top_k > 8) {
-        set_error("moe: at most 256 experts and top-k 8 in a prompt pass");
+    if (n < 1 || n > PROMPT_ROWS || n_experts < 1 || n_experts > MAX_EXPERTS || top_k < 1 || top_k > 8) {
+        set_error("moe: at most 2048 rows, 256 experts and top-k 8 in a prompt pass");
         return TSV_ERR_UNSUPPORTED;
     }
     hipLaunchKernelGGL(k_prompt_groups, dim3(1), dim3(1024), 0, s, selected, n, top_k, n_experts, bm, r);
@@ -907,7 +922,9 @@ int launch_prompt_groups(hipStream_t s, const int32_t* selected, int n, int top_
 int launch_prompt_gather(hipStream_t s, const uint16_t* rows, const uint8_t* row_sums, int k, const PromptRoutes& r, int n, int top_k, int n_experts,
                          uint8_t* a, uint8_t* asum) {
     const int sorted = prompt_sorted_rows(n, top_k, n_experts);
-    hipLaunchKernelGGL(k_prompt_gather, dim3((sorted + 31) / 32), dim3(256), 0, s, rows, row_sums, prompt_k16(k), r.pair, sorted, a, asum);
+    // parts of K: four workgroups to a compute unit, as long as every thread keeps four loads
+    const int blocks = (sorted + 31) / 32, parts = std::max(1, std::min((1024 + blocks - 1) / blocks, prompt_k16(k) / 16));
+    hipLaunchKernelGGL(k_prompt_gather, dim3(blocks, parts), dim3(256), 0, s, rows, row_sums, prompt_k16(k), r.pair, sorted, a, asum);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }
