@@ -711,15 +711,19 @@ __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
 // rows, 128 experts, top 8, 768 x 2048: 144 each, 114 + 93, 93 + 96.  Of the 357, 298 are left with the weights in the cache, 331
 // with the activations in the L1 and 334 without the unpack: no one thing bounds it, a workgroup's start and end are the rest.
 // Rings of 3 and 4 (1 and 2 units more ahead) are 2 and 4 % slower.
+// So what a start or an end waits for is asked for ahead: the tile beside the count, the row factors behind nothing but the first
+// weights, pairs and biases before the sums meet.  In whole prompts down 98 -> 90 us (1000 rows) and 233 -> 226 (1500), gate/up
+// 96.6 -> 95.9 and 374 -> 373.
 constexpr int NARROW_ROWS = 64, NARROW_RING2 = 2, NARROW_RING1 = 4;
 template <int RB, int RING>
 __device__ __forceinline__ void narrow_products(__amdgpu_buffer_rsrc_t w0, __amdgpu_buffer_rsrc_t w1, __amdgpu_buffer_rsrc_t a, uint32_t rbs, int units,
-                                                int unit0, const int (&shift)[2], int lane, float16v (&acc)[2][2][2]) {
+                                                int unit0, const float (&rs)[2], int lane, float16v (&acc)[2][2][2]) {
     struct Piece {
         u32x4 q[2], a[2][RB];
         uint32_t e[2];
     } r[RING];
     const int last = unit0 + units - 1;
+    int shift[2];
     auto load = [&](Piece& p, int u) {
         u = min(u, last);
         const uint32_t t = (u >> 3) * PromptMx::TILE_BYTES, qa = t + (u & 7) * 1024, ea = t + 8192 + (u & 7);
@@ -761,6 +765,8 @@ __device__ __forceinline__ void narrow_products(__amdgpu_buffer_rsrc_t w0, __amd
     };
 #pragma unroll
     for (int i = 0; i < RING - 1; i++) load(r[i], unit0 + i);
+#pragma unroll
+    for (int c = 0; c < 2; c++) shift[c] = (int)(__float_as_uint(rs[c]) >> 23) - 127;  // (behind the first loads: the factors are under way too)
     for (int u = unit0; u <= last; u += RING) {
 #pragma unroll
         for (int i = 0; i < RING; i++) {
@@ -777,18 +783,15 @@ __global__ __launch_bounds__(256, 2) void k_prompt_experts_narrow(PromptGemmArgs
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // XCD x takes the row tiles x, x + 8, ..., all columns of one before the next
     const int slot = blockIdx.x >> 3, mb = slot / g.nt * 8 + (blockIdx.x & 7), nb0 = slot % g.nt * 2;
+    // (asked for together: what lies behind the count is in the buffer, and not used)
+    const PromptTile t = uniform_tile(g.tiles[min(mb, g.mt - 1)]);
     if (mb >= *g.tile_count) return;
-    const PromptTile t = uniform_tile(g.tiles[mb]);
     const int columns = min(2, g.n_tiles - nb0);  // (an odd count: the last workgroup's second half repeats the last tile, and leaves nothing)
-    int shift[2];
+    float rs[2];
     const size_t tile_bytes = (size_t)g.kchunks * PromptMx::TILE_BYTES;
     const uint8_t* const w = g.w + ((size_t)t.expert * g.n_tiles + nb0) * tile_bytes;
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-        const float rs = g.rs[(t.expert * g.n_tiles + nb0 + min(c, columns - 1)) * 64 + lane];
-        if (wave == 0) factor[c * 64 + lane] = 1.0f / rs;
-        shift[c] = (int)(__float_as_uint(rs) >> 23) - 127;
-    }
+    for (int c = 0; c < 2; c++) rs[c] = g.rs[(t.expert * g.n_tiles + nb0 + min(c, columns - 1)) * 64 + lane];
     float16v acc[2][2][2];
 #pragma unroll
     for (int c = 0; c < 2; c++)
@@ -802,8 +805,27 @@ __global__ __launch_bounds__(256, 2) void k_prompt_experts_narrow(PromptGemmArgs
     const __amdgpu_buffer_rsrc_t w0 = buffer_of(w, tile_bytes), w1 = buffer_of(w + (columns - 1) * tile_bytes, tile_bytes),
                                  a = buffer_of(g.a + (size_t)(t.first >> 5) * rbs, (t.cnt > 32 ? 2 : 1) * rbs);
     const int units = 2 * g.kchunks;
-    if (t.cnt > 32) narrow_products<2, NARROW_RING2>(w0, w1, a, rbs, units, wave * units, shift, lane, acc);
-    else narrow_products<1, NARROW_RING1>(w0, w1, a, rbs, units, wave * units, shift, lane, acc);
+    if (t.cnt > 32) narrow_products<2, NARROW_RING2>(w0, w1, a, rbs, units, wave * units, rs, lane, acc);
+    else narrow_products<1, NARROW_RING1>(w0, w1, a, rbs, units, wave * units, rs, lane, acc);
+    if (wave == 0) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) factor[c * 64 + lane] = 1.0f / rs[c];
+    }
+    // where this lane's sums go and what is added to them, asked for ahead of the barriers
+    int pair[8];
+    float bias[2][2];
+    if (EPI == EPI_PARTIAL) {
+#pragma unroll
+        for (int v = 0; v < 8; v++) pair[v] = g.pair[t.first + min(32 * (v >> 2) + 8 * wave + 4 * (lane >> 5) + (v & 3), t.cnt - 1)];
+    }
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float* const b = EPI == EPI_PARTIAL || !j ? g.bias : g.bias2;
+            const int col = (EPI == EPI_PARTIAL ? (nb0 + c) * 64 + 32 * j : (nb0 + c) * 32) + (lane & 31);
+            bias[c][j] = b && col < g.n_valid ? b[(size_t)t.expert * g.n_valid + col] : 0.f;
+        }
 #pragma unroll
     for (int c = 0; c < 2; c++) {
         const int nb = nb0 + c;
@@ -840,15 +862,14 @@ __global__ __launch_bounds__(256, 2) void k_prompt_experts_narrow(PromptGemmArgs
             for (int j = 0; j < 2; j++) {
                 const int col = nb * 64 + 32 * j + (lane & 31);
                 if (col >= g.n_valid) continue;
-                const float bias = g.bias ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
 #pragma unroll
                 for (int b = 0; b < 2; b++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         const int local = 32 * b + 8 * wave + 4 * (lane >> 5) + i;
                         if (local >= t.cnt) continue;
-                        const int pr = g.pair[t.first + local], row = pr >> 3;
-                        out[((size_t)(row >> 4) * 128 + (pr & 7) * 16 + (row & 15)) * g.ldo + col] = sum[b * 8 + j * 4 + i] + bias;
+                        const int pr = pair[b * 4 + i], row = pr >> 3;
+                        out[((size_t)(row >> 4) * 128 + (pr & 7) * 16 + (row & 15)) * g.ldo + col] = sum[b * 8 + j * 4 + i] + bias[c][j];
                     }
             }
             continue;
@@ -856,16 +877,14 @@ __global__ __launch_bounds__(256, 2) void k_prompt_experts_narrow(PromptGemmArgs
         // 32 gate columns and the matching up columns; the products go through LDS into the order of the next matmul's activations
         __syncthreads();
         _Float16* const act = (_Float16*)meet;
-        const int cc = lane & 31, col = nb * 32 + cc;
-        const float bg = g.bias && col < g.n_valid ? g.bias[(size_t)t.expert * g.n_valid + col] : 0.f;
-        const float bu = g.bias2 && col < g.n_valid ? g.bias2[(size_t)t.expert * g.n_valid + col] : 0.f;
+        const int cc = lane & 31;
 #pragma unroll
         for (int b = 0; b < 2; b++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = 8 * wave + 4 * (lane >> 5) + i;
                 act[(((b * 2 + (cc >> 4)) * 2 + ((cc >> 3) & 1)) * 32 + row) * 8 + (cc & 4) + (((cc & 1) << 1) | ((cc >> 1) & 1))] =
-                    (_Float16)gated(sum[b * 8 + i] + bg, sum[b * 8 + 4 + i] + bu, g.alpha, g.limit);
+                    (_Float16)gated(sum[b * 8 + i] + bias[c][0], sum[b * 8 + 4 + i] + bias[c][1], g.alpha, g.limit);
             }
         __syncthreads();
         const int p = threadIdx.x, b = p >> 7, k16 = nb * 2 + ((p >> 6) & 1);
