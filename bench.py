@@ -83,7 +83,16 @@ def algorithmic_bytes(cfg, ctx, m, union=None, kv_bits=None):
     return dict(per_layer=per_layer, head=head, weights=weights, kv=kv, total=weights + kv + small)
 
 
-def trace_summary(path, first="k_clear_result"):
+# the kernels an acceptance begins with: a sampled round's, a greedy one's, and what traces of earlier builds hold ahead of either
+ACCEPTANCE = ("k_row_max", "k_argmax_part", "k_clear_result")
+
+
+def _first_dispatch(rows, first):
+    """(index, kernel) of the first dispatch of `first`, or of an acceptance kernel where that is None."""
+    return next((i, k) for i, r in enumerate(rows) for k in ((first,) if first else ACCEPTANCE) if k in r["Kernel_Name"])
+
+
+def trace_summary(path, first=None):
     """Per-kernel statistics of the verify STEPS in a `rocprofv3 --kernel-trace --output-format csv`
     trace of this script: only dispatches from the first acceptance kernel on are counted,
     which leaves out weight re-tiling and the prompt passes that build the KV cache (--trace-from
@@ -92,7 +101,7 @@ def trace_summary(path, first="k_clear_result"):
     import csv
     rows = list(csv.DictReader(open(path)))
     rows.sort(key=lambda r: int(r["Start_Timestamp"]))
-    start = next(i for i, r in enumerate(rows) if first in r["Kernel_Name"])
+    start, _ = _first_dispatch(rows, first)
     stats = {}
     for r in rows[start:]:
         name = r["Kernel_Name"].replace("tsv::", "").replace("(anonymous namespace)::", "")
@@ -109,7 +118,7 @@ def trace_summary(path, first="k_clear_result"):
     for (name, wgs, lds), v in sorted(stats.items(), key=lambda kv: -kv[1][1]):
         print(f"{name[:44]:44s} {wgs:6d} {lds:7d} {v[0]:7d} {v[1] / v[0] / 1e3:9.2f} {v[2] / 1e3:9.2f} {v[3] / 1e3:9.2f} "
               f"{100.0 * v[1] / total:6.2f}%")
-    what = "verify steps" if first == "k_clear_result" else f"dispatches from the first {first} on"
+    what = "verify steps" if first is None else f"dispatches from the first {first} on"
     print(f"total kernel time in {what}: {total / 1e6:.3f} ms over the traced steps")
 
 
@@ -267,7 +276,7 @@ def traffic_summary(fetch_csv, write_csv, which):
     print(json.dumps(out, indent=1))
 
 
-def step_traffic(fetch_csv, write_csv, first="k_clear_result"):
+def step_traffic(fetch_csv, write_csv, first=None):
     """HBM bytes per launch of every kernel of the verify passes, from two `rocprofv3 --pmc` collections (FETCH_SIZE,
     then WRITE_SIZE) of `bench.py --copy-probe ...`: dispatches from the first acceptance kernel on, keyed by kernel
     name and grid like --trace-summary, each counter scaled by what it reads for the copy kernel of known size that
@@ -280,7 +289,7 @@ def step_traffic(fetch_csv, write_csv, first="k_clear_result"):
         rows.sort(key=lambda r: int(r["Dispatch_Id"]))
         copies = [float(r["Counter_Value"]) for r in rows if "k_copy_probe" in r["Kernel_Name"]]
         factor = COPY_BYTES / (sum(copies) / len(copies))
-        start = next(i for i, r in enumerate(rows) if first in r["Kernel_Name"])
+        start, begin = _first_dispatch(rows, first)
         passes = sum("k_embed" in r["Kernel_Name"] for r in rows[start:])
         for r in rows[start:]:
             name = r["Kernel_Name"].replace("tsv::", "").replace("(anonymous namespace)::", "").split("(")[0].replace("void ", "")
@@ -296,7 +305,7 @@ def step_traffic(fetch_csv, write_csv, first="k_clear_result"):
         tot[0] += rd[1]
         tot[1] += wr[1]
         print(f"{name[:44]:44s} {wgs:6d} {rd[0]:7d} {rd[1] / max(rd[0], 1):14.0f} {wr[1] / max(wr[0], 1):17.0f}")
-    print(f"all dispatches from the first {first} on: {tot[0] / passes:.0f} B read + {tot[1] / passes:.0f} B written per pass "
+    print(f"all dispatches from the first {begin} on: {tot[0] / passes:.0f} B read + {tot[1] / passes:.0f} B written per pass "
           f"({passes} passes)")
 
 
@@ -326,7 +335,7 @@ def main():
                          "counters) and leave out the per-kernel timing, whose passes launch one kernel class twice")
     ap.add_argument("--probe", default="gate_up", choices=sorted(PROBES),
                     help="which kernel --traffic-probe runs and the two summaries read")
-    ap.add_argument("--trace-from", default="k_clear_result", metavar="KERNEL",
+    ap.add_argument("--trace-from", default=None, metavar="KERNEL",
                     help="--trace-summary counts dispatches from the first one of this kernel on")
     ap.add_argument("--prefill-bench", type=int, default=0, metavar="TOKENS",
                     help="time tsv_prefill over a prompt of this many tokens (after one untimed run of the same), print one "

@@ -7,6 +7,8 @@ import os
 import subprocess
 import sys
 
+import pytest
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -67,6 +69,17 @@ def test_trace_summary_counts_from_the_first_acceptance_kernel(tmp_path, capsys)
     assert any(l.startswith("k_gemm<1, 2>") and " 96 " in l and "6.00" in l for l in out)
     assert "k_embed" not in "\n".join(out)
     assert out[-1].startswith("total kernel time in verify steps: 0.041 ms")
+
+
+@pytest.mark.parametrize("kernel", ["void tsv::k_row_max<false>(int)", "tsv::k_argmax_part(int)"])
+def test_trace_summary_finds_where_a_round_s_acceptance_begins(kernel, tmp_path, capsys):
+    b = _bench()
+    head = ["Kernel_Name", "Start_Timestamp", "End_Timestamp", "Grid_Size_X", "Workgroup_Size_X", "LDS_Block_Size"]
+    p = tmp_path / "t.csv"
+    _write(p, head, [("tsv::k_embed(int)", 0, 5000, 256, 256, 0), (kernel, 10000, 11000, 64, 64, 0)])
+    b.trace_summary(str(p))
+    out = capsys.readouterr().out
+    assert "k_embed" not in out and "total kernel time in verify steps: 0.001 ms" in out
 
 
 def _counter_rows(counter, copy_reading, kernel_name, kernel_readings, grid=448 * 64, first=None):
