@@ -108,6 +108,30 @@ def test_tree_attention_with_a_window():
         assert np.abs(got - want).max() <= 5e-3 * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (64, 8, 64), (32, 4, 128)])
+@pytest.mark.parametrize("m,base,window", [(1, 130, 0), (5, 250, 0), (16, 370, 0), (1, 500, 0), (5, 480, 0), (16, 496, 0), (5, 3000, 128),
+                                           (16, 200, 128)])
+def test_rows_of_a_short_context_are_the_nearest_fp16(nq, nkv, hd, m, base, window):
+    """Against 64 bits: what a row is off by comes from its last rounding.  The scores are fp32 sums of 128 exact products (2^-24 of
+    their norm each, scores of up to 12 in units of log 2: 3e-6 of a weight at most), weights two fp16 terms (2^-22), so a value is off by
+    less than 4e-6 before it is rounded, and the nearest fp16 (a step is 5e-4 of a value or more) is missed where the exact value
+    lies that close to the middle of two: 2 * 4e-6 / 5e-4, less than one in fifty.  Weights rounded to fp16 (2e-4) miss two in five."""
+    from turbospark_amd import ffi
+    q, k, v = _rand(m, nq, nkv, hd, base, 77 + m + base)
+    q *= 2
+    got = ffi.attention(q, k, v, base, window=window)
+    want = np.empty((m, nq, hd))
+    for i in range(m):
+        lo = max(0, base + i + 1 - window) if window else 0
+        kk, vv = (np.repeat(a[lo:base + i + 1].astype(np.float64), nq // nkv, axis=1) for a in (k, v))
+        s = np.einsum("hd,phd->hp", q[i].astype(np.float64), kk) / hd ** 0.5
+        w = np.exp(s - s.max(1, keepdims=True))
+        want[i] = np.einsum("hp,phd->hd", w / w.sum(1, keepdims=True), vv)
+    big = np.abs(want) > 2.0 ** -6 * np.sqrt((want ** 2).mean())   # (a sum that cancels has fewer bits of its own)
+    missed = np.mean(got.astype(np.float16)[big] != want.astype(np.float16)[big])
+    assert missed <= 0.02, missed
+
+
 @pytest.mark.parametrize("seed", range(64))
 def test_random_attention_shapes_and_long_contexts(seed):
     """Seeded sweep: head width, GQA group 1..8, 1..16 rows, chain or random tree, contexts up to 20000

@@ -66,6 +66,13 @@ __global__ __launch_bounds__(64 * TG * attn_phases(TG)) void k_attn_partial_grou
     attn_partial_body<HD, RT, STAGES, false, TG>(a, G, R, blockIdx.x, blockIdx.y, 0, xch);
 }
 
+// A short context (launch_hd): one workgroup per KV head and row group, which finishes its rows
+template <int HD, int RT, int STAGES>
+__global__ __launch_bounds__(512) void k_attn_direct(AttnArgs a, int G, int R) {
+    extern __shared__ float xch[];
+    attn_partial_body<HD, RT, STAGES, false, 1, true>(a, G, R, 0, blockIdx.y, blockIdx.z * RT, xch);
+}
+
 // The same pass over a layer that keeps quantized rows (attn_tq_core.h)
 template <int HD, int RT, int KB, int VB>
 __global__ __launch_bounds__(512) void k_attn_partial_tq(AttnArgs a, int G, int R) {
@@ -185,6 +192,20 @@ static int launch_partial(hipStream_t s, const AttnArgs& a, int G, int R, int gr
     return TSV_OK;
 }
 
+template <int HD, int RT, int STAGES>
+static int launch_direct(hipStream_t s, const AttnArgs& a, int G, int R, int groups) {
+    constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT;
+    constexpr size_t lds = (size_t)8 * 64 * PER_LANE * 4;
+    static bool raised = false;
+    if (lds > 65536 && !raised) {
+        TSV_HIP(hipFuncSetAttribute((const void*)k_attn_direct<HD, RT, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        raised = true;
+    }
+    hipLaunchKernelGGL((k_attn_direct<HD, RT, STAGES>), dim3(1, a.nkv, groups), dim3(512), lds, s, a, G, R);
+    TSV_HIP(hipGetLastError());
+    return TSV_OK;
+}
+
 template <int HD, int RT, int STAGES, int TG>
 static int launch_partial_groups(hipStream_t s, const AttnArgs& a, int G, int R) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT, NW = attn_phases(TG);
@@ -246,10 +267,9 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
     // phases here, so that a row's sums run in one order whatever shares its pass.
     const bool few = attn_short(a.kv_end) || (a.window > 0 && (a.window + TSV_MAX_ROWS + 14) / 16 + 1 <= ATTN_DIRECT_BLOCKS);
     if (a.kv_end > 0 && a.blocks <= 1 && !a.tq.k_bits && !a.frag16 && few) {
-        a.direct = a.nch = 1;
-        a.xcd_groups = 0;
-        return trt <= 1 ? launch_partial<HD, 1, 3>(s, a, G, R, 1)
-                        : launch_partial<HD, 2, (HD == 128 ? TSV_ATTN_STAGES2_HD128 : TSV_ATTN_STAGES2_HD64)>(s, a, G, R, groups);
+        a.nch = 1;
+        return trt <= 1 ? launch_direct<HD, 1, 3>(s, a, G, R, 1)
+                        : launch_direct<HD, 2, (HD == 128 ? TSV_ATTN_STAGES2_HD128 : TSV_ATTN_STAGES2_HD64)>(s, a, G, R, groups);
     }
     a.nch = std::max(std::min(a0.nch, 8), std::min(a0.nch, 256 / (a0.nkv * groups * std::max(a0.blocks, 1))));
     // Several row groups of a verify pass read the same K / V: they are placed on one die.  A workgroup fills a

@@ -40,7 +40,7 @@ __device__ __forceinline__ void store_state(const float (&mrun)[RT], const float
 // work, where folding the states into one wave's, four to a barrier, ended with that wave going through 64 values of each alone
 // (8B shape, a layer's pass at 60 positions, attention in one chunk: 68.9 -> 65.4 us with five rows, 82.7 -> 78.7 with sixteen).
 // (BASE2: the maxima are kept in units of log 2, the weights are powers of two.)  grp: the group's slots, from this lane's column on.
-template <int HD, int RT, int NW, bool BASE2>
+template <int HD, int RT, int NW, bool BASE2, bool DIRECT = false>
 __device__ __forceinline__ void attn_finish(const AttnArgs& a, int G, int R, int chunk, int h, int rt0, int wave, int lane, float* grp,
                                             const float (&mrun)[RT], const float (&lrun)[RT], const float4v (&O)[RT][HD / 16]) {
     constexpr int VT = HD / 16, PER_LANE = RT * VT * 4 + 2 * RT;
@@ -72,7 +72,7 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int G, int R, int
             }
         l += __shfl_xor(l, 16);
         l += __shfl_xor(l, 32);
-        if (!a.direct) {
+        if (!DIRECT) {
             if (r >= R) continue;
             const long slot = ((long)h * a.nch + chunk) * R + r;
             if (kg == 0 && u == 0) {
@@ -131,10 +131,16 @@ __device__ __forceinline__ float max_over_position_groups(float v) {
 // once for all (row, q head) pairs of the pass.  (Legacy callers pass TG = 1 and their own rt0: eight waves, one group.)
 // COH: the query rows and the K / V blocks are read device-coherently (sc1), for a caller whose
 // other compute units wrote them earlier in the same kernel.
+// DIRECT: the only chunk of a short context (attn.hip, launch_hd), whose rows are finished here.  The weights go into the value product as
+// two fp16 terms, through the matrix instruction of twice the depth, which takes the value operand twice and no longer than the other.
+// Rounded to fp16, only the weight that the reference was taken from is exact: in chunks that is one of each block's while a wave has
+// one block, here it would be one of several blocks'.  Distance of the finished rows from 64 bits, scores of two standard deviations,
+// 300 / 700 positions (their own rounding to fp16 is 2.07e-4): in chunks 2.15e-4 / 2.12e-4, in one chunk with rounded weights 2.6e-4 /
+// 2.9e-4, with two terms 2.07e-4.
 // xch: [TG][NW slots][PER_LANE values][64 lanes] floats of LDS.
 __host__ __device__ constexpr int attn_phases(int tg) { return tg == 1 ? 8 : tg == 2 ? 4 : 2; }
 
-template <int HD, int RT, int STAGES, bool COH, int TG = 1>
+template <int HD, int RT, int STAGES, bool COH, int TG = 1, bool DIRECT = false>
 __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int R, int chunk, int h, int rt_first, float* xch) {
     constexpr int NW = attn_phases(TG);
     constexpr int KS = HD / 32;  // K steps of the score MFMA
@@ -240,7 +246,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
         // Three phases over the row tiles -- all score products, then the softmax steps, then all value products --
         // so that the matrix pipe works through one tile's chain while the vector ALU is busy with another's.
         float4v Sx[RT];
-        half4 Px[RT];
+        half4 Px[RT], Lx[RT];  // (DIRECT: and what the rounding left)
 #pragma unroll
         for (int t = 0; t < RT; t++) Sx[t] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -290,24 +296,32 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
                 mrun[t] = mnew;
             }
             const float nref = -fmaxf(mrun[t], -3.0e38f);
-            half4 P;
+            half4 P, left = {};
             float ps = 0.f;
 #pragma unroll
             for (int i4 = 0; i4 < 4; i4++) {
                 const float p = __builtin_amdgcn_exp2f(fmaf(sc[i4], c2, nref));
                 ps += p;
                 P[i4] = (_Float16)p;
+                if (DIRECT) left[i4] = (_Float16)(p - (float)P[i4]);
             }
             lrun[t] += ps;
             Px[t] = P;
+            Lx[t] = left;
         }
 #pragma unroll
         for (int d = 0; d < VT; d++) {
             const u32x4 v2 = st.vf[d >> 1];
             const u32x2 vd = (d & 1) ? u32x2{v2.z, v2.w} : u32x2{v2.x, v2.y};
 #pragma unroll
-            for (int t = 0; t < RT; t++)
-                O[t][d] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(half4, vd), Px[t], O[t][d], 0, 0, 0);
+            for (int t = 0; t < RT; t++) {
+                if constexpr (DIRECT)
+                    O[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        __builtin_bit_cast(half8, u32x4{vd.x, vd.y, vd.x, vd.y}),
+                        half8{Px[t][0], Px[t][1], Px[t][2], Px[t][3], Lx[t][0], Lx[t][1], Lx[t][2], Lx[t][3]}, O[t][d], 0, 0, 0);
+                else
+                    O[t][d] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(half4, vd), Px[t], O[t][d], 0, 0, 0);
+            }
         }
     };
     // Short runs are straight-line code (every load issued before the first wait, no load the run
@@ -348,7 +362,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
             if (i + s < nb) consume(st[s], i + s);
     }
 
-    attn_finish<HD, RT, NW, true>(a, G, R, chunk, h, rt0, wave, lane, xch + tg * NW * 64 * PER_LANE + lane, mrun, lrun, O);
+    attn_finish<HD, RT, NW, true, DIRECT>(a, G, R, chunk, h, rt0, wave, lane, xch + tg * NW * 64 * PER_LANE + lane, mrun, lrun, O);
 }
 
 }  // namespace tsv

@@ -377,7 +377,6 @@ struct AttnArgs {
     float* part_ml;  // [nkv][nch][rows][2]
     uint4* xfrag;    // output, K index = qh*hd + d
     int nq, nkv, hd, max_ctx, nch;  // max_ctx: positions the layer's cache holds
-    int direct;          // set by the launcher: nch is 1 and the partial kernel writes the fragments itself, no merge follows
     int ring;            // non-zero: the cache is a ring, position p in slot p % max_ctx (a windowed layer)
     float scale;
     int window;          // 0: full; else a row sees the last `window` positions of its sequence
