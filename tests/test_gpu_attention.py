@@ -132,6 +132,20 @@ def test_rows_of_a_short_context_are_the_nearest_fp16(nq, nkv, hd, m, base, wind
     assert missed <= 0.02, missed
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (64, 8, 64)])
+@pytest.mark.parametrize("m", [1, 5, 16])
+@pytest.mark.parametrize("end,window", [(511, 0), (512, 0), (513, 0), (900, 481), (900, 482), (900, 483)])
+def test_both_sides_of_the_line_of_short_contexts(nq, nkv, hd, m, end, window):
+    """Contexts and windows around the longest that one workgroup takes whole."""
+    from turbospark_amd import ffi
+    base = end - m
+    q, k, v = _rand(m, nq, nkv, hd, base, 31 * end + m)
+    sinks = np.random.default_rng(m).standard_normal(nq).astype(np.float32) if window else None
+    got = ffi.attention(q, k, v, base, window=window, sinks=sinks)
+    want = _oracle(q, k, v, base, None, window=window, sinks=sinks)
+    assert np.abs(got - want).max() <= 5e-3 * max(1.0, np.abs(want).max())
+
+
 @pytest.mark.parametrize("seed", range(64))
 def test_random_attention_shapes_and_long_contexts(seed):
     """Seeded sweep: head width, GQA group 1..8, 1..16 rows, chain or random tree, contexts up to 20000

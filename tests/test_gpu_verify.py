@@ -171,6 +171,31 @@ def test_graph_replay_of_the_pass_equals_plain_launches():
     assert np.array_equal(plain.verify_tree(feed, parent, base), graph.verify_tree(feed, parent, base))
 
 
+@pytest.mark.parametrize("name", ["small_q4_k", "xcd_q4_k", "gptoss_small"])
+def test_graph_replays_across_the_line_of_short_contexts(name, monkeypatch):
+    """A captured pass is kept for each side of the line (512 positions): rounds of the same rows that cross it forwards and, by
+    rollbacks, backwards, against plain launches by bits.  Each side is captured and replayed."""
+    import turbospark_amd as ts
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS[name], max_context=640)
+    w = synth.make_weights(cfg, seed=21)
+    plain = ts.HipVerifier(cfg, w)
+    monkeypatch.setenv("TSV_GRAPH", "1")
+    graph = ts.HipVerifier(cfg, w)
+    prompt = _prompt(560, cfg["vocab"], 4)
+    for eng in (plain, graph):
+        eng.prefill(prompt, 0, want_logits=False)
+    rng = np.random.default_rng(3)
+    for base in (500, 507, 508, 540, 506, 509, 507, 555, 490, 512):      # five rows: an end of 512 is the last on the short side
+        for m in (5, 1):
+            for eng in (plain, graph):
+                eng.rollback(ts.ffi.Point(base))
+            feed = rng.integers(0, cfg["vocab"], m).astype(np.int32)
+            assert np.array_equal(plain.verify(feed, base), graph.verify(feed, base)), (base, m)
+        for eng in (plain, graph):               # the positions behind are there again for the next base
+            eng.prefill(prompt[eng.position:560], eng.position, want_logits=False)
+
+
 @pytest.mark.parametrize("name,layer,over", [("small_q4_k_m", 0, {}), ("small_q5_k_m", 1, {}), ("small_q4_k_m", 0, dict(head_dim=64, n_q_heads=8, n_kv_heads=2)),
                                              ("small_q4_k_m", 0, dict(hidden=2304, n_q_heads=6, n_kv_heads=2))])
 @pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])

@@ -260,11 +260,14 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
     // (fewer, longer chunks also mean fewer partial results for the merge to read)
     AttnArgs a = a0;
     // A short context in one workgroup per KV head and row group, up to ATTN_DIRECT_BLOCKS / 8 blocks a wave, which finishes its rows
-    // itself.  What that takes off a layer against chunks and a merge (8B shape, 1 / 5 / 16 rows, us): 2.0 / 1.5 / 4.9 at 250 positions,
-    // -0.1 / -0.6 / 2.0 at 700, and beyond the line, with the limit raised, -0.4 / -0.1 / 3.3 at 1000, -1.2 / -2.5 / 0.9 at 1500: a wave then
-    // walks too many blocks alone, and only sixteen rows, whose merge is the longest, would still gain.
-    // Layers of a short window always do (a window's blocks: its own, the pass's, one cut).  All row groups take the form of eight
-    // phases here, so that a row's sums run in one order whatever shares its pass.
+    // itself.  What that takes off a layer against chunks and a merge (8B shape, 1 / 5 / 16 rows, us): 2.5 / 2.9 / 5.3 at 250 positions,
+    // 0.7 / 0.6 / 3.5 at 490, and with the line further out 0.0 / -0.6 / 2.4 at 620, -0.4 / -1.2 / 1.8 at 730; four KV heads with groups
+    // of eight, five rows: 2.6 at 250, 0.2 at 490, -0.8 at 620.
+    // A wave walks more blocks alone the longer the context is; the line lies where the first form of all, one group of two row tiles,
+    // begins to lose.  The others would still gain behind it (sixteen rows), but a line by rows would make a row's bits depend
+    // on its pass over a range of positions.  As it is they do where the passes' ends lie on two sides of the line, which is one of the
+    // 16-position boundaries at which the chunks change.  Layers of a short window always go this way (a window's blocks: its own, the
+    // pass's, one cut).  All row groups take the form of eight phases here, so that a row's sums do not depend on how many share its pass.
     const bool few = attn_short(a.kv_end) || (a.window > 0 && (a.window + TSV_MAX_ROWS + 14) / 16 + 1 <= ATTN_DIRECT_BLOCKS);
     if (a.kv_end > 0 && a.blocks <= 1 && !a.tq.k_bits && !a.frag16 && few) {
         a.nch = 1;

@@ -1541,8 +1541,9 @@ extern "C" int32_t tsv_produce(tsv_ctx* c, int32_t token, int64_t position, uint
 // (mtp_prime_rows_batched, families/qwen/mtp.rs:146-400); next_token: the token after ids[n - 1], or -1.
 int tsv::prefill_passes(tsv_ctx* c, const int32_t* ids, int64_t n, int64_t pos0, uint16_t* logits, tsv_ctx* head, int32_t next_token) {
     const int wide_rows = 16 * WIDE_B;
-    // A call of fewer than 64 tokens keeps verify-sized passes, whose rows have the bits of one-row passes whatever their
-    // number: what a caller gets by feeding a few tokens one by one and at once is the same.
+    // A call of fewer than 64 tokens keeps verify-sized passes: what a caller gets by feeding a few tokens one by one and at once is
+    // the same, by bits as long as the passes end in the same block of sixteen positions and have at most 32 pairs of row and q head of
+    // a group (beyond, and across the line of short contexts, attention adds its chunks up in another order: launch_hd in attn.hip).
     const bool by_prompt_pass = c->prompt.ok && c->prompt.most && !c->profile && !c->route_forced_set && prompt_pays(c, n, pos0, logits || head);
     for (int64_t i = 0; i < n;) {
         if (by_prompt_pass) {

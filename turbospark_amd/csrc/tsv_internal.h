@@ -469,7 +469,7 @@ size_t tq_vq_bytes(int nkv, int cap, int hd, int v_bits);
 int launch_attention_merge(hipStream_t s, const AttnArgs& a, int m);
 int attn_chunks(int nkv);
 // whether a pass that ends at position `kv_end` attends in one workgroup per KV head and row group (attn.hip)
-constexpr int ATTN_DIRECT_BLOCKS = 48;
+constexpr int ATTN_DIRECT_BLOCKS = 32;
 inline bool attn_short(int64_t kv_end) { return kv_end <= 16 * ATTN_DIRECT_BLOCKS; }
 
 int launch_kv_gather(hipStream_t s, uint16_t* const* caches_dev, const int32_t* caps_dev, int n_layers, int nkv, int hd,
