@@ -128,6 +128,10 @@ int32_t tsv_limit_prompt_buffers(tsv_ctx* ctx, int64_t bytes);
 /* Rows of the longest prompt pass the handle takes (0: none), the bytes its buffers hold, and how many prompt passes
  * (passes[0]) and 64-row passes (passes[1]) it has run so far. */
 int32_t tsv_prompt_buffers(const tsv_ctx* ctx, int32_t* rows, int64_t* bytes, int64_t* passes);
+/* Host arithmetic only: how far the prompt matmul's loads reach where a tile of `rows` rows (1..256) works on part `part` of
+ * `splits` of a K of `k`: reach[0] is one past the last byte it asks for of a 64-row weight tile of reach[1] bytes, reach[2] one past
+ * the last of a 32-row block of activations of reach[3]. */
+int32_t tsv_prompt_walk_reach(int32_t dtype, int64_t k, int32_t splits, int32_t part, int32_t rows, int64_t* reach);
 
 #ifdef __cplusplus
 }

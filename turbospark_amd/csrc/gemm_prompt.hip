@@ -58,7 +58,8 @@ __device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast
 __device__ __forceinline__ half2v pair_of(float v) { return half2v{(_Float16)v, (_Float16)v}; }
 
 // Loads through a buffer descriptor: lane offset in a register, the walk's offset in a scalar one, so that no vector instruction
-// goes into addresses (a third of the loop's in the forms of few rows).  Past the end they return zeros.
+// goes into addresses (a third of the loop's in the forms of few rows).  The descriptor's end bounds the lane offset alone: the scalar
+// one has to stay inside by itself (Walk).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (uint32_t)bytes, 0x00027000);
 }
@@ -359,6 +360,25 @@ constexpr int lds_bytes() {
     return (2 * stage_bytes<F>() < 65536 ? 65536 : 2 * stage_bytes<F>()) + 2 * CHUNK_BYTES;
 }
 
+// What a tile's walk over K asks for ahead: the weights of two stages further on, activations RING - 1 steps of 16 K.  Past the end of
+// its part these are the last ones again, which nobody uses (the matrix may end there, and its allocation).
+template <class F, int WN>
+struct Walk {
+    static constexpr int NT = 4 / WN, KS = F::STAGE_K / 16, STEPS = F::SPC * KS;  // 16-K steps of a stage, of a chunk
+    static constexpr int WANT = 16 / NT, RING = STEPS < WANT ? STEPS : WANT;      // activations: steps in registers
+    static __host__ __device__ __forceinline__ int chunk(int stage, int c1) { return stage / F::SPC < c1 ? stage / F::SPC : c1 - 1; }
+    static __host__ __device__ __forceinline__ int step(int at, int c1) { return at < c1 * STEPS ? at : c1 * STEPS - 1; }
+    // the furthest chunk and step asked for in part [c0, c1), as prompt_tile asks
+    static void reach(int c0, int c1, int* far_chunk, int* far_step) {
+        *far_chunk = std::max(chunk(c0 * F::SPC, c1), chunk(c0 * F::SPC + 1, c1));
+        *far_step = step(c0 * STEPS + RING - 2, c1);
+        for (int s = c0 * F::SPC; s < c1 * F::SPC; s++) {
+            *far_chunk = std::max(*far_chunk, chunk(s + 2, c1));
+            for (int i = 0; i < KS; i++) *far_step = std::max(*far_step, step(s * KS + i + RING - 1, c1));
+        }
+    }
+};
+
 // The order of a slot's instructions: what others wait for first (activations, operands), then a share of the vector instructions
 // behind every product, which keeps the matrix pipe for 32 cycles and the issue port for four.
 template <int NT, bool STORED>
@@ -386,8 +406,8 @@ __device__ __forceinline__ void slot_order(bool rescaled) {
 // One tile: BM = 64 * 4 / WN rows from row0 on, of which `rows` exist.
 template <class F, int WN, int EPI>
 __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* lds, int split, int nb, int row0, int rows, int expert) {
-    constexpr int NT = 4 / WN, BM = 64 * (4 / WN), KS = F::STAGE_K / 16, SLOTS = KS * F::TERMS, STAGE = stage_bytes<F>();
-    constexpr int STEPS = F::SPC * KS, WANT = 16 / NT, RING = STEPS < WANT ? STEPS : WANT;  // activations: steps of 16 K in registers
+    using K = Walk<F, WN>;
+    constexpr int NT = K::NT, BM = 64 * NT, KS = K::KS, SLOTS = KS * F::TERMS, STAGE = stage_bytes<F>(), STEPS = K::STEPS, RING = K::RING;
     constexpr int AHEAD = NT == 4 ? 1 : NT == 2 ? 2 : 3, BARRIER = SLOTS - AHEAD, SETS = NT == 4 ? 1 : 4;  // operands: slots ahead of their products
     static_assert(STEPS % RING == 0 && (SETS == 1 || SLOTS % SETS == 0), "the place of a step's registers is known at compile time");
     uint8_t* const side = lds + lds_bytes<F>() - 2 * CHUNK_BYTES;  // [chunk % 2][min operands, coefficients]
@@ -421,11 +441,12 @@ __device__ __forceinline__ void prompt_tile(const PromptGemmArgs& g, uint8_t* ld
     u32x4 a[RING][2], b[SETS][NT], sm[2], mn[NT];
     float into[NT];
     auto load_w = [&](int what, int s, int sub) {
-        F::load(w, what, wsrc, s / F::SPC * F::TILE_BYTES, sub, part, lane);
+        F::load(w, what, wsrc, K::chunk(s, c1) * F::TILE_BYTES, sub, part, lane);
     };
     auto load_a = [&](int place, int step) {
+        const int at = K::step(step, c1) * 1024;
 #pragma unroll
-        for (int t = 0; t < 2; t++) a[place][t] = load16(asrc, a_at[t], step * 1024);
+        for (int t = 0; t < 2; t++) a[place][t] = load16(asrc, a_at[t], at);
     };
     // operand j of a stage's slot: 16-K step slot / TERMS, term slot % TERMS
     auto load_b = [&](u32x4& to, const uint8_t* stage, int slot, int j) {
@@ -1000,6 +1021,21 @@ int row_block(const TiledW& w, int m, int splits) {
 }
 
 }  // namespace
+
+void prompt_walk_reach(int fmt, int rows, int c0, int c1, int* far_chunk, int* far_step) {
+    auto of = [&](auto f) {
+        using F = decltype(f);
+        if (rows > 128) Walk<F, 1>::reach(c0, c1, far_chunk, far_step);
+        else if (rows > 64) Walk<F, 2>::reach(c0, c1, far_chunk, far_step);
+        else Walk<F, 4>::reach(c0, c1, far_chunk, far_step);
+    };
+    if (fmt == FMT_Q4K) of(PromptQ45<false>{});
+    else if (fmt == FMT_Q5K) of(PromptQ45<true>{});
+    else if (fmt == FMT_Q6K) of(PromptQ6{});
+    else if (fmt == FMT_Q80) of(PromptQ8{});
+    else if (fmt == FMT_MX4) of(PromptMx{});
+    else of(PromptBf{});
+}
 
 bool prompt_fmt_has_sums(int fmt) { return fmt == FMT_Q4K || fmt == FMT_Q5K; }
 

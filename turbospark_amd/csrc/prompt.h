@@ -102,6 +102,8 @@ int launch_prompt_experts(hipStream_t s, const TiledW& w, const void* a, const v
 // than one) at most PROMPT_PARTIALS sums in all
 constexpr int64_t PROMPT_PARTIALS = (int64_t)512 * 256 * 128;
 int prompt_splits(const TiledW& w, int m, const TiledW* beside = nullptr);
+// Host arithmetic: the furthest chunk of weights and 16-K step of activations that a tile of `rows` rows asks for in chunks [c0, c1)
+void prompt_walk_reach(int fmt, int rows, int c0, int c1, int* far_chunk, int* far_step);
 // Q8_0, bf16, MXFP4: fills w.row_scale (prompt_row_scales floats), the power-of-two factors of the matrix's rows, and w.rows_unfit;
 // waits for the stream
 inline size_t prompt_row_scales(const TiledW& w) { return (size_t)w.n_tiles * TILE_ROWS + 1; }

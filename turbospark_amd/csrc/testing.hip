@@ -143,6 +143,27 @@ extern "C" int32_t tsv_limit_prompt_buffers(tsv_ctx* c, int64_t bytes) {
     return TSV_OK;
 }
 
+extern "C" int32_t tsv_prompt_walk_reach(int32_t dtype, int64_t k, int32_t splits, int32_t part, int32_t rows, int64_t* reach) {
+    const int fmt = dtype_fmt(dtype), unit = fmt < 0 ? 1 : fmt == FMT_MX4 ? 32 : fmt_chunk_elems(fmt);
+    if (fmt < 0 || k < 1 || k > 1 << 20 || k % unit || splits < 1 || part < 0 || part >= splits || rows < 1 || rows > 256 || !reach) {
+        set_error("prompt_walk_reach: bad argument");
+        return TSV_ERR_INVALID;
+    }
+    const int elems = fmt_chunk_elems(fmt), chunks = (int)((k + elems - 1) / elems), per = (chunks + splits - 1) / splits;
+    const int c0 = part * per, c1 = std::min(c0 + per, chunks);
+    if (c0 >= c1) {
+        set_error("prompt_walk_reach: an empty part of K");
+        return TSV_ERR_INVALID;
+    }
+    int chunk, step;
+    prompt_walk_reach(fmt, rows, c0, c1, &chunk, &step);
+    reach[0] = (int64_t)(chunk + 1) * fmt_tile_bytes(fmt);
+    reach[1] = (int64_t)chunks * fmt_tile_bytes(fmt);
+    reach[2] = (int64_t)(step + 1) * 1024;
+    reach[3] = (int64_t)prompt_k16((int)k) * 1024;
+    return TSV_OK;
+}
+
 extern "C" int32_t tsv_prompt_buffers(const tsv_ctx* c, int32_t* rows, int64_t* bytes, int64_t* passes) {
     TSV_NEED(c && rows && bytes && passes, "prompt_buffers: null argument");
     *rows = c->prompt.most;
