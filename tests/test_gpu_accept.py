@@ -447,3 +447,34 @@ def test_draft_draws_of_any_vocabulary_match_the_oracle(vocab, k, temperature, k
         got = gpu.draft_chain(draft, ts.shaping(temperature, seed=seed, **kw), seed)
         want = ob.draft_chain(draft, ob.shaping(temperature, seed=seed, **kw), [1, 2, 3], 0, seed)
         assert list(got[0]) == list(want[0]) and got[1] == want[1], seed
+
+
+def test_a_refused_call_leaves_no_copy_of_the_caller_s_rows_under_way():
+    """Rows in pinned memory are copied asynchronously: a call that refuses its arguments returns with the stream idle, so that the rows
+    may be freed or rewritten."""
+    import ctypes as C
+    import turbospark_amd as ts
+    from turbospark_amd import hip, synth
+    cfg = dict(synth.CONFIGS["tiny_q8_0"], vocab=200000, n_layers=1, max_context=64)
+    gpu = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=3))
+    pinned = C.c_void_p()
+    hip.check(hip.rt().hipHostMalloc(C.byref(pinned), C.c_size_t(15 * cfg["vocab"] * 2), C.c_uint(0)), "pinned rows")
+    draft = np.ctypeslib.as_array(C.cast(pinned, C.POINTER(C.c_uint16)), (15, cfg["vocab"]))
+    draft[:] = 0
+    feed = list(range(16))
+    idle = lambda: hip.rt().hipStreamQuery(C.c_void_p(gpu.stream)) == 0
+    gpu.verify(feed, 0)
+    with pytest.raises(ts.ffi.TsvError, match="16 stop tokens"):
+        gpu.accept(feed, 0, ts.shaping(0.8, seed=1), draft_logits=draft, stop_tokens=range(17))
+    assert idle()
+    r, keep = gpu._round(feed, 0, ts.shaping(0.8, seed=1, repetition_penalty=1.1), None, draft, 0, None, 0, 0, False)
+    r.n_history = 5                                      # a history that is not there
+    out = ts.ffi.RoundResultC()
+    assert ts.ffi.lib().tsv_accept(gpu._h, C.byref(r), C.byref(out)) != 0
+    assert idle()
+    sh, at, props = ts.shaping(0.8, seed=1, repetition_penalty=1.1), C.c_uint64(0), (C.c_int32 * 16)()
+    assert ts.ffi.lib().tsv_draft_chain(gpu._h, draft.ctypes.data, 15, C.byref(sh), C.byref(at), props, None, C.c_int64(5), C.c_uint64(0)) != 0
+    assert idle()
+    gpu.accept(feed, 0, ts.shaping(0.8, seed=1), draft_logits=draft)      # and takes the same rows when they are right
+    del draft
+    hip.check(hip.rt().hipHostFree(pinned), "free")

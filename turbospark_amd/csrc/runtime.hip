@@ -1787,10 +1787,6 @@ int fill_accept(tsv_ctx* c, const tsv_round* r, AcceptParams* ap) {
     ap->vocab = c->vocab;
     ap->tree = r->parent != nullptr;
     ap->sampled = r->shaping.temperature != 0.0;
-    if (r->n_stop < 0 || r->n_stop > 16) {
-        set_error("accept: at most 16 stop tokens");
-        return TSV_ERR_INVALID;
-    }
     ap->n_stop = r->n_stop;
     for (int i = 0; i < r->m; i++) {
         ap->feed[i] = r->feed[i];
@@ -1806,6 +1802,14 @@ int fill_accept(tsv_ctx* c, const tsv_round* r, AcceptParams* ap) {
     return TSV_OK;
 }
 
+int check_history(const tsv_shaping& sh, const int32_t* history, int64_t n) {
+    if (has_penalties(sh) && (n < 0 || (n > 0 && !history))) {
+        set_error("penalties: the round carries no token history");
+        return TSV_ERR_INVALID;
+    }
+    return TSV_OK;
+}
+
 // Penalised sampled rounds (choose.rs:138-154): uploads the history, counts its tokens on the device
 // and fills the penalty fields of the parameter block.  `generated` is the sink's count of reported
 // tokens: the last min(generated, n) tokens of the history are the generated suffix.
@@ -1813,10 +1817,7 @@ int setup_penalties(tsv_ctx* c, const tsv_shaping& sh, const int32_t* history, i
                     AcceptParams* ap) {
     ap->pen = 0;
     if (!has_penalties(sh)) return TSV_OK;
-    if (n < 0 || (n > 0 && !history)) {
-        set_error("penalties: the round carries no token history");
-        return TSV_ERR_INVALID;
-    }
+    if (int rc = check_history(sh, history, n)) return rc;
     if ((size_t)n > c->hist_cap) {
         if (c->hist_dev) TSV_HIP(hipFree(c->hist_dev));
         if (c->hist_host) TSV_HIP(hipHostFree(c->hist_host));
@@ -1867,6 +1868,16 @@ int check_round(const tsv_round* r) {
     return TSV_OK;
 }
 
+// The caller's rows are on their way (asynchronously where they lie in pinned memory): a call that fails from here on waits, so that the
+// buffer is the caller's again
+struct RowsUnderWay {
+    tsv_ctx* c;
+    bool done = false;
+    ~RowsUnderWay() {
+        if (!done) (void)hipStreamSynchronize(c->stream);
+    }
+};
+
 int accept_impl(tsv_ctx* c, const tsv_round* r, tsv_round_result* out) {
     int rc = check_round(r);
     if (rc) return rc;
@@ -1900,8 +1911,15 @@ int accept_impl(tsv_ctx* c, const tsv_round* r, tsv_round_result* out) {
             set_error("accept: sampled acceptance over a tree takes no stop tokens or budget");
             return TSV_ERR_UNSUPPORTED;
         }
-        if ((rc = stage_draft(c, r->draft_logits, r->parent ? r->m : r->m - 1, &draft))) return rc;
     }
+    if (r->n_stop < 0 || r->n_stop > 16) {
+        set_error("accept: at most 16 stop tokens");
+        return TSV_ERR_INVALID;
+    }
+    if ((rc = check_history(r->shaping, r->history, r->n_history))) return rc;
+    // (everything that a round's arguments are refused for is behind us: from here on the caller's memory is being read)
+    RowsUnderWay rows{c, !sampled};
+    if (sampled && (rc = stage_draft(c, r->draft_logits, r->parent ? r->m : r->m - 1, &draft))) return rc;
     // (no wait for the pass: its launches and these are one queue, with the host ahead of the device throughout)
     if ((rc = upload_begin(c))) return rc;
     AcceptParams* ap = &c->up_host->ap;
@@ -1918,6 +1936,7 @@ int accept_impl(tsv_ctx* c, const tsv_round* r, tsv_round_result* out) {
     if (r->logits_out)
         TSV_HIP(hipMemcpyAsync(r->logits_out, c->logits, (size_t)r->m * c->vocab * 2, hipMemcpyDeviceToHost, c->stream));
     if ((rc = upload_end(c))) return rc;
+    rows.done = true;
     const AcceptResult& a = *c->res_host;
     if (a.error) {
         set_error(std::string("accept: ") + accept_error_text(a.error));
@@ -1975,8 +1994,9 @@ extern "C" int32_t tsv_draft_chain(tsv_ctx* c, const uint16_t* draft_logits, int
         return TSV_ERR_INVALID;
     }
     int rc = check_shaping(*sh, true);
-    if (rc) return rc;
+    if (rc || (rc = check_history(*sh, history, n_history))) return rc;
     const uint16_t* draft = nullptr;
+    RowsUnderWay rows{c};
     if ((rc = stage_draft(c, draft_logits, k, &draft))) return rc;
     if ((rc = upload_begin(c))) return rc;
     AcceptParams* ap = &c->up_host->ap;
@@ -1996,6 +2016,7 @@ extern "C" int32_t tsv_draft_chain(tsv_ctx* c, const uint16_t* draft_logits, int
     TSV_HIP(hipMemcpyAsync(c->tok_host, c->tok_dev, (size_t)k * 4, hipMemcpyDeviceToHost, c->stream));
     TSV_HIP(hipMemcpyAsync(c->res_host, c->sc.result, sizeof(AcceptResult), hipMemcpyDeviceToHost, c->stream));
     if ((rc = upload_end(c))) return rc;
+    rows.done = true;
     if (c->res_host->error) {
         set_error(std::string("draft_chain: ") + accept_error_text(c->res_host->error));
         return (c->res_host->error & 1) ? TSV_ERR_INVALID : TSV_ERR_UNSUPPORTED;
