@@ -181,11 +181,8 @@ template <int HD, int RT, int STAGES>
 static int launch_partial(hipStream_t s, const AttnArgs& a, int G, int R, int groups) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT;
     constexpr size_t lds = (size_t)8 * 64 * PER_LANE * 4;
-    static bool raised = false;  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
-    if (lds > 65536 && !raised) {
-        TSV_HIP(hipFuncSetAttribute((const void*)k_attn_partial<HD, RT, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        raised = true;
-    }
+    static OncePerDevice allowed;
+    if (int rc = allow_lds((const void*)k_attn_partial<HD, RT, STAGES>, lds, allowed)) return rc;
     const dim3 grid = a.xcd_groups ? dim3(attn_grid_size(a.nch * a.nkv, groups)) : dim3(a.nch, a.nkv, groups * std::max(a.blocks, 1));
     hipLaunchKernelGGL((k_attn_partial<HD, RT, STAGES>), grid, dim3(512), lds, s, a, G, R);
     TSV_HIP(hipGetLastError());
@@ -196,11 +193,8 @@ template <int HD, int RT, int STAGES>
 static int launch_direct(hipStream_t s, const AttnArgs& a, int G, int R, int groups) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT;
     constexpr size_t lds = (size_t)8 * 64 * PER_LANE * 4;
-    static bool raised = false;
-    if (lds > 65536 && !raised) {
-        TSV_HIP(hipFuncSetAttribute((const void*)k_attn_direct<HD, RT, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        raised = true;
-    }
+    static OncePerDevice allowed;
+    if (int rc = allow_lds((const void*)k_attn_direct<HD, RT, STAGES>, lds, allowed)) return rc;
     hipLaunchKernelGGL((k_attn_direct<HD, RT, STAGES>), dim3(1, a.nkv, groups), dim3(512), lds, s, a, G, R);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
@@ -210,12 +204,8 @@ template <int HD, int RT, int STAGES, int TG>
 static int launch_partial_groups(hipStream_t s, const AttnArgs& a, int G, int R) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT, NW = attn_phases(TG);
     const size_t lds = (size_t)TG * NW * 64 * PER_LANE * 4;
-    static bool raised = false;  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
-    if (lds > 65536 && !raised) {
-        TSV_HIP(hipFuncSetAttribute((const void*)k_attn_partial_groups<HD, RT, STAGES, TG>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        raised = true;
-    }
+    static OncePerDevice allowed;
+    if (int rc = allow_lds((const void*)k_attn_partial_groups<HD, RT, STAGES, TG>, lds, allowed)) return rc;
     hipLaunchKernelGGL((k_attn_partial_groups<HD, RT, STAGES, TG>), dim3(a.nch, a.nkv, std::max(a.blocks, 1)), dim3(64 * TG * NW),
                        lds, s, a, G, R);
     TSV_HIP(hipGetLastError());
@@ -229,12 +219,8 @@ template <int HD, int RT, int KB, int VB>
 static int launch_partial_tq(hipStream_t s, const AttnArgs& a, int G, int R, int groups) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT;
     const size_t lds = (size_t)8 * 64 * PER_LANE * 4;
-    static bool raised = false;
-    if (lds > 60000 && !raised) {  // with the pair tables beside it the exchange area passes 64 KiB
-        TSV_HIP(hipFuncSetAttribute((const void*)k_attn_partial_tq<HD, RT, KB, VB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds));
-        raised = true;
-    }
+    static OncePerDevice allowed;  // (36, 68, 72 or 136 KiB: the pair tables, 2 KiB of static LDS at most, take none of them over the line)
+    if (int rc = allow_lds((const void*)k_attn_partial_tq<HD, RT, KB, VB>, lds, allowed)) return rc;
     const dim3 grid = a.xcd_groups ? dim3(attn_grid_size(a.nch * a.nkv, groups)) : dim3(a.nch, a.nkv, groups * std::max(a.blocks, 1));
     hipLaunchKernelGGL((k_attn_partial_tq<HD, RT, KB, VB>), grid, dim3(512), lds, s, a, G, R);
     TSV_HIP(hipGetLastError());

@@ -1321,11 +1321,8 @@ int gemm_wide_rows() { return 16 * WIDE_BLOCKS; }
 template <class P, int EPI>
 static int launch_wide_pe(hipStream_t s, const GemmWideArgs& wa) {
     const size_t lds = 2 * (size_t)P::BUF_BYTES + WIDE_BLOCKS * 32 * sizeof(float);
-    static bool attr_set = false;  // more than 64 KiB of dynamic LDS has to be asked for once per kernel
-    if (!attr_set && lds > 65536) {
-        TSV_HIP(hipFuncSetAttribute((const void*)k_gemm_wide<P, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
+    static OncePerDevice allowed;
+    if (int rc = allow_lds((const void*)k_gemm_wide<P, EPI>, lds, allowed)) return rc;
     hipLaunchKernelGGL((k_gemm_wide<P, EPI>), dim3(wa.g.n_tiles * wa.g.splits), dim3(64 * WIDE_BLOCKS), lds, s, wa);
     TSV_HIP(hipGetLastError());
     return TSV_OK;

@@ -35,7 +35,6 @@
 // Workgroups are numbered so that an XCD works on every eighth block of columns with all row blocks side by side: the
 // weights of a block come into that XCD's L2 once, and the activations are shared by the blocks in flight.
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 #include "prompt.h"
@@ -971,15 +970,8 @@ __global__ __launch_bounds__(64) void k_row_scale(const uint8_t* __restrict__ ti
 
 template <class F, int EPI>
 int launch_p(hipStream_t s, const PromptGemmArgs& g) {
-    // more than 64 KiB of dynamic LDS has to be allowed once per kernel and device
-    static std::atomic<uint64_t> allowed{0};
-    int dev = 0;
-    TSV_HIP(hipGetDevice(&dev));
-    const uint64_t bit = 1ull << (dev & 63);
-    if (!(allowed.load(std::memory_order_acquire) & bit)) {
-        TSV_HIP(hipFuncSetAttribute((const void*)k_prompt_gemm<F, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<F>()));
-        allowed.fetch_or(bit, std::memory_order_release);
-    }
+    static OncePerDevice allowed;
+    if (int rc = allow_lds((const void*)k_prompt_gemm<F, EPI>, lds_bytes<F>(), allowed)) return rc;
     const int blocks = (g.nt + 7) / 8 * 8 * g.mt * g.splits;
     hipLaunchKernelGGL((k_prompt_gemm<F, EPI>), dim3(blocks), dim3(256), lds_bytes<F>(), s, g);
     TSV_HIP(hipGetLastError());

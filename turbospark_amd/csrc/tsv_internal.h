@@ -8,6 +8,7 @@
 
 #include "../../include/tsverify.h"
 #include "../../include/tsverify_testing.h"
+#include "per_device.h"
 
 namespace tsv {
 
@@ -23,6 +24,17 @@ const std::string& get_error();
             return TSV_ERR_DEVICE;                                                          \
         }                                                                                   \
     } while (0)
+
+// More than 64 KiB of dynamic LDS has to be allowed once per kernel and device.  once: the kernel's own.
+inline int allow_lds(const void* kernel, size_t bytes, tsv::OncePerDevice& once) {
+    if (bytes <= 65536) return TSV_OK;
+    int device = 0;
+    TSV_HIP(hipGetDevice(&device));
+    if (!once.needed(device)) return TSV_OK;
+    TSV_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    once.note(device);
+    return TSV_OK;
+}
 
 #define TSV_NEED(cond, msg)          \
     do {                             \
