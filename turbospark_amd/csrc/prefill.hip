@@ -124,9 +124,11 @@ int prompt_open(tsv_ctx* c) {
 //   where routed experts have fewer than three rows on average, so that each is read for next to nothing whatever reads it
 //   (gpt-oss layers, 65 / 80 rows: 1151 / 1482 us against 1403 / 1524; the 128-expert shape of eight chosen at 65 rows, four each:
 //   788 against 743);
-//   with quantized KV rows below PROMPT_MIN_ROWS_TQ: callers that count a handle's passes expect up to 150 rows of such a handle in 64-row
-//   passes, as ever, so the line lies behind them and not where a prompt pass begins to win (8B shape, eight layers, 160 rows: 3520 us in
-//   smaller passes, 1733 in one; 130 rows stay at 2650);
+//   with quantized KV rows below PROMPT_MIN_ROWS_TQ: not the faster side, a prompt pass is from 65 rows on (8B shape, 4-bit rows, eight
+//   layers, 64-row passes against a prompt pass: 65 / 96 / 128 / 159 rows at position 0 1612 / 2395 / 3615 / 3438 us against 1359 / 1425 /
+//   1478 / 1741, behind 4000 positions 1741 / 2588 / 3886 / 3758 against 1678 / 1707 / 1745 / 2107; 64-wide heads, 2-bit rows, 65 / 159: 1026 /
+//   2166 against 820 / 942).  The line keeps prompts of up to 150 rows of such a handle in the 64-row passes that they are known by, which
+//   are held to the oracle's quantized rows at these lengths;
 //   far into a context: a prompt pass's attention takes its blocks in whole 128-pair workgroups.  Q4_K, 8B shape, 65 rows: 715
 //   against 695 us at 0, 750 / 765 at 4000, 780 / 846 at 8000; 80 rows: 799 / 701, 831 / 769, 861 / 856, and 564 / 588 (two
 //   layers) at 32 000.

@@ -54,7 +54,10 @@ __host__ __device__ inline int prompt_sorted_rows(int n, int top_k, int n_expert
 //                                    128:  716    862   1156   1470   1879
 //                                    256:  734    872   1151   1523   1984
 // 256 is as far as a pass of 2048 rows gets with eight of 64 experts; beyond, and for other formats beyond 192, tiles of 256 save
-// unpacking.
+// unpacking.  The average decides, also where the rows crowd: with one expert in every row's choice, or the same experts in all rows', 32
+// tiles of 64 rows unpack a crowded expert's weights each and are still the faster ones (MXFP4, narrow against 128 / 256 rows):
+//   even / one / all       32 of 2880 x 2880, four chosen, n = 256: 1922 / 1895 / 1767 against 2181 / 2166 / 1938;  n = 187: 1482 / 1522 /
+//   1360 against 1628 / 1710 / 1447;  128 of 768 x 2048, eight chosen, n = 128: 1486 / 1473 / 1344 against 1599 / 1566 / 1404
 inline int prompt_expert_rows(int n, int top_k, int n_experts, bool narrow) {
     const int avg = n * top_k / n_experts;
     return narrow && avg <= 256 ? 64 : !narrow && avg <= 192 ? 128 : 256;
