@@ -133,10 +133,10 @@ __device__ __forceinline__ float max_over_position_groups(float v) {
 // other compute units wrote them earlier in the same kernel.
 // DIRECT: the only chunk of a short context (attn.hip, launch_hd), whose rows are finished here.  The weights go into the value product as
 // two fp16 terms, through the matrix instruction of twice the depth, which takes the value operand twice and no longer than the other.
-// Rounded to fp16, only the weight that the reference was taken from is exact: in chunks that is one of each block's while a wave has
-// one block, here it would be one of several blocks'.  Distance of the finished rows from 64 bits, scores of two standard deviations,
-// 300 / 700 positions (their own rounding to fp16 is 2.07e-4): in chunks 2.15e-4 / 2.12e-4, in one chunk with rounded weights 2.6e-4 /
-// 2.9e-4, with two terms 2.07e-4.
+// Rounded to fp16, only the weight that the reference was taken from is exact: one of each block's while every wave has one block, as in
+// chunks and here up to 128 positions, where one term it stays (2.15e-4 both ways at 60 positions, 0.2 us a layer less); one of several
+// blocks' beyond.  Distance of the finished rows from 64 bits, scores of two standard deviations, 300 / 700 positions (their own rounding
+// to fp16 is 2.07e-4): in chunks 2.15e-4 / 2.12e-4, in one chunk with rounded weights 2.6e-4 / 2.9e-4, with two terms 2.07e-4.
 // xch: [TG][NW slots][PER_LANE values][64 lanes] floats of LDS.
 __host__ __device__ constexpr int attn_phases(int tg) { return tg == 1 ? 8 : tg == 2 ? 4 : 2; }
 
@@ -240,13 +240,14 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
     // the variant without the visibility words (a wave-uniform choice; a visible position gets the same operations
     // in the same order in both, so its bits do not depend on which variant its block took).
     const float c2 = scale * 1.44269504088896340736f;
-    auto consume = [&](const Blk& st, int i) {
+    auto consume_as = [&](const Blk& st, int i, auto two) {
+        constexpr bool TWO = decltype(two)::value;  // the weights as two terms
         const int p0 = (b0 + wave + NW * i) << 4;
         const bool tail = p0 + 16 > base;
         // Three phases over the row tiles -- all score products, then the softmax steps, then all value products --
         // so that the matrix pipe works through one tile's chain while the vector ALU is busy with another's.
         float4v Sx[RT];
-        half4 Px[RT], Lx[RT];  // (DIRECT: and what the rounding left)
+        half4 Px[RT], Lx[RT];  // (TWO: and what the rounding left)
 #pragma unroll
         for (int t = 0; t < RT; t++) Sx[t] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -303,7 +304,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
                 const float p = __builtin_amdgcn_exp2f(fmaf(sc[i4], c2, nref));
                 ps += p;
                 P[i4] = (_Float16)p;
-                if (DIRECT) left[i4] = (_Float16)(p - (float)P[i4]);
+                if (TWO) left[i4] = (_Float16)(p - (float)P[i4]);
             }
             lrun[t] += ps;
             Px[t] = P;
@@ -315,7 +316,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
             const u32x2 vd = (d & 1) ? u32x2{v2.z, v2.w} : u32x2{v2.x, v2.y};
 #pragma unroll
             for (int t = 0; t < RT; t++) {
-                if constexpr (DIRECT)
+                if constexpr (TWO)
                     O[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                         __builtin_bit_cast(half8, u32x4{vd.x, vd.y, vd.x, vd.y}),
                         half8{Px[t][0], Px[t][1], Px[t][2], Px[t][3], Lx[t][0], Lx[t][1], Lx[t][2], Lx[t][3]}, O[t][d], 0, 0, 0);
@@ -324,13 +325,15 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
             }
         }
     };
+    auto consume = [&](const Blk& st, int i) { consume_as(st, i, std::integral_constant<bool, DIRECT>{}); };
     // Short runs are straight-line code (every load issued before the first wait, no load the run
     // does not need); longer ones keep STAGES blocks in flight, with unconditional loads in the
     // steady state so the compiler waits on the oldest block only.
     if (nb == 1) {
         Blk st;
         fetch(st, 0);
-        consume(st, 0);
+        if (DIRECT && b1 - b0 <= NW) consume_as(st, 0, std::false_type{});  // (every wave has one block)
+        else consume(st, 0);
     } else if (nb == 2) {
         Blk s0, s1;
         fetch(s0, 0);
