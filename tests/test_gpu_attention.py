@@ -134,9 +134,10 @@ def test_rows_of_a_short_context_are_the_nearest_fp16(nq, nkv, hd, m, base, wind
 
 @pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (64, 8, 64)])
 @pytest.mark.parametrize("m", [1, 5, 16])
-@pytest.mark.parametrize("end,window", [(511, 0), (512, 0), (513, 0), (900, 481), (900, 482), (900, 483)])
+@pytest.mark.parametrize("end,window", [(17, 0), (127, 0), (128, 0), (129, 0), (900, 97), (900, 113), (900, 129),
+                                        (511, 0), (512, 0), (513, 0), (900, 481), (900, 482), (900, 483)])
 def test_both_sides_of_the_line_of_short_contexts(nq, nkv, hd, m, end, window):
-    """Contexts and windows around the longest that one workgroup takes whole."""
+    """Contexts and windows around the longest that one workgroup takes whole, and around the longest of one block to each of its waves."""
     from turbospark_amd import ffi
     base = end - m
     q, k, v = _rand(m, nq, nkv, hd, base, 31 * end + m)
