@@ -122,6 +122,10 @@ int32_t tsv_route_selected(tsv_ctx* ctx, int32_t* out, int32_t n_layers);
  * 16-row passes (the larger ones route freely). */
 int32_t tsv_force_route(tsv_ctx* ctx, const int32_t* sel, int32_t n_layers);
 
+/* The order of a prompt matmul's workgroups, nt column blocks in `splits` parts of K and mt row tiles: place[0] workgroups in all, and of workgroup
+   `block` place[1] whether it has a tile, [2] its part of K, [3] column block, [4] row tile.  Host arithmetic. */
+int32_t tsv_prompt_grid(int32_t nt, int32_t splits, int32_t mt, int32_t last_is_short, int32_t block, int32_t* place);
+
 /* Prompt passes take at most the rows whose buffers fit in `bytes`, as on a device that had no more room when the
  * handle was opened (0: the prompt goes in 64-row passes); a larger value gives the rows back. */
 int32_t tsv_limit_prompt_buffers(tsv_ctx* ctx, int64_t bytes);

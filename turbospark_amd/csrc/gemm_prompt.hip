@@ -32,8 +32,9 @@
 // and 256 74.  With a stage unpacked ahead of its products, flat addresses for every load and the last registers of a load under
 // way given to something else (which then waits for it) these were 564, 62 and 90, 299 rows 119 (now 109; Q5_K 131 and 115).
 //
-// Workgroups are numbered so that an XCD works on every eighth block of columns with all row blocks side by side: the
-// weights of a block come into that XCD's L2 once, and the activations are shared by the blocks in flight.
+// Workgroups are numbered so that an XCD works on every eighth (block of columns, part of K) with all row blocks side by side: its
+// weights come into that XCD's L2 once, and the activations are shared by the blocks in flight.  (Numbered by the column block alone a
+// router of 128 experts, one block in eight parts, had all of its work on one XCD: 1000 rows of 2048 24.8 us a launch, 11.8 spread.)
 #include <algorithm>
 #include <type_traits>
 
@@ -692,20 +693,21 @@ __device__ __forceinline__ PromptTile uniform_tile(PromptTile t) {
 template <class F, int EPI>
 __global__ __launch_bounds__(256, 2) void k_prompt_gemm(PromptGemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    // which tile: XCD x takes the column blocks x, x + 8, ..., all full row blocks of one before the next; then the short ones
-    const int nt8 = (g.nt + 7) / 8 * 8, full = g.tiles || g.mt == 1 || g.m % g.bm == 0 ? g.mt : g.mt - 1, first_short = nt8 * full * g.splits;
-    const bool is_short = (int)blockIdx.x >= first_short;
-    const int across = is_short ? 1 : full, at = is_short ? blockIdx.x - first_short : blockIdx.x;
-    const int split = at / (nt8 * across), id = at - split * nt8 * across;
-    const int slot = id >> 3, nb = slot / across * 8 + (id & 7), mb = is_short ? full : slot % across;
-    if (nb >= g.nt) return;
+    const PromptGrid& q = g.grid;
+    asm volatile("" ::"s"(q.units), "s"(q.first_short), "s"(q.full), "s"(q.by_full.magic), "s"(q.nt), "s"(q.by_nt.magic), "s"(g.w), "s"(g.a), "s"(g.asum),
+                 "s"(g.rs), "s"(g.m), "s"(g.n_tiles), "s"(g.kchunks), "s"(g.chunks_per_split), "s"(g.bm), "s"(g.a_k16), "s"(g.tiles), "s"(g.tile_count), "s"(g.mt));
+    int split, nb, mb;
+    if (!q.place(blockIdx.x, split, nb, mb)) return;
     int row0 = mb * g.bm, rows = min(g.m - row0, g.bm), expert = 0;  // the tile's first row and how many of its rows exist
     if (g.tiles) {
-        if (mb >= *g.tile_count) return;
-        const PromptTile t = uniform_tile(g.tiles[mb]);
-        row0 = t.first;
-        rows = t.cnt;
-        expert = t.expert;
+        // (asked for together: what lies behind the count is in the buffer, and not used)
+        const auto* const t = uniform_memory(g.tiles) + min(mb, g.mt - 1);
+        const int count = *uniform_memory(g.tile_count);
+        row0 = t->first;
+        rows = t->cnt;
+        expert = t->expert;
+        asm volatile("" ::"s"(row0), "s"(rows), "s"(expert), "s"(count));
+        if (mb >= count) return;
     }
     if constexpr (std::is_same<F, PromptBfEither>::value) {
         const float* const rs = g.rs + (size_t)expert * g.n_tiles * 64 + (threadIdx.x & 63);
@@ -974,11 +976,11 @@ __global__ __launch_bounds__(64) void k_row_scale(const uint8_t* __restrict__ ti
 }
 
 template <class F, int EPI>
-int launch_p(hipStream_t s, const PromptGemmArgs& g) {
+int launch_p(hipStream_t s, PromptGemmArgs& g) {
     static OncePerDevice allowed;
     if (int rc = allow_lds((const void*)k_prompt_gemm<F, EPI>, lds_bytes<F>(), allowed)) return rc;
-    const int blocks = (g.nt + 7) / 8 * 8 * g.mt * g.splits;
-    hipLaunchKernelGGL((k_prompt_gemm<F, EPI>), dim3(blocks), dim3(256), lds_bytes<F>(), s, g);
+    g.grid = PromptGrid::of(g.nt, g.splits, g.mt, !g.tiles && g.m % g.bm != 0);
+    hipLaunchKernelGGL((k_prompt_gemm<F, EPI>), dim3(g.grid.blocks(g.mt)), dim3(256), lds_bytes<F>(), s, g);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }

@@ -70,7 +70,29 @@ int launch_prompt_groups(hipStream_t s, const int32_t* selected, int n, int top_
 int launch_prompt_gather(hipStream_t s, const uint16_t* rows, const uint8_t* row_sums, int k, const PromptRoutes& r, int n, int top_k, int n_experts,
                          uint8_t* a, uint8_t* asum);
 
+// The order of k_prompt_gemm's workgroups: XCD x takes the units (a part of K of a column block: what shares no weights) x, x + 8, ..., all full
+// row tiles of one before the next; the short tiles (a last row tile that does not fill up) come after all full ones.
+struct PromptGrid {
+    int units, first_short, full, nt;  // nt column blocks x parts of K; the first workgroup of the short tiles; full row tiles
+    UniformDivisor by_full, by_nt;
+    int blocks(int mt) const { return (units + 7) / 8 * 8 * mt; }
+    static PromptGrid of(int nt, int splits, int mt, bool last_is_short) {
+        const int full = last_is_short && mt > 1 ? mt - 1 : mt;
+        return PromptGrid{nt * splits, (nt * splits + 7) / 8 * 8 * full, full, nt, UniformDivisor(full), UniformDivisor(nt)};
+    }
+    __host__ __device__ __forceinline__ bool place(int block, int& split, int& nb, int& mb) const {
+        const bool is_short = block >= first_short;
+        const int at = is_short ? block - first_short : block, slot = at >> 3;
+        const int rank = is_short ? slot : by_full.quotient(slot), unit = rank * 8 + (at & 7);
+        mb = is_short ? full : slot - rank * full;
+        split = by_nt.quotient(unit);
+        nb = unit - split * nt;
+        return unit < units;
+    }
+};
+
 struct PromptGemmArgs {
+    PromptGrid grid;
     const uint8_t* w;     // row tiles (TiledW)
     const uint8_t* a;     // activations
     const uint8_t* asum;  // their sums (formats with a min term)

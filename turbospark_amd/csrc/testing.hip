@@ -143,6 +143,17 @@ extern "C" int32_t tsv_limit_prompt_buffers(tsv_ctx* c, int64_t bytes) {
     return TSV_OK;
 }
 
+extern "C" int32_t tsv_prompt_grid(int32_t nt, int32_t splits, int32_t mt, int32_t last_is_short, int32_t block, int32_t* place) {
+    if (nt < 1 || splits < 1 || mt < 1 || block < 0 || !place) {
+        set_error("prompt_grid: bad argument");
+        return TSV_ERR_INVALID;
+    }
+    const PromptGrid g = PromptGrid::of(nt, splits, mt, last_is_short != 0);
+    place[0] = g.blocks(mt);
+    place[1] = g.place(block, place[2], place[3], place[4]);
+    return TSV_OK;
+}
+
 extern "C" int32_t tsv_prompt_walk_reach(int32_t dtype, int64_t k, int32_t splits, int32_t part, int32_t rows, int64_t* reach) {
     const int fmt = dtype_fmt(dtype), unit = fmt < 0 ? 1 : fmt == FMT_MX4 ? 32 : fmt_chunk_elems(fmt);
     if (fmt < 0 || k < 1 || k > 1 << 20 || k % unit || splits < 1 || part < 0 || part >= splits || rows < 1 || rows > 256 || !reach) {

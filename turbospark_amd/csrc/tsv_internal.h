@@ -147,6 +147,26 @@ __host__ __device__ inline long vcache_index(int h, int pos, int d, int hd, int 
            ((((po >> 2) * 16 + (d & 15)) * 2 + ((d >> 4) & 1)) << 2) + (po & 3);
 }
 
+// Where a kernel's start is a chain of round trips its launch is longer by them, and every launch starts on cold caches.  The arguments sit in
+// memory and are read by scalar loads that the compiler puts where a value is first needed: behind a branch or behind another load's wait
+// that is a round trip of its own, 0.2 us each.  So kernels name theirs in one empty asm statement at the start (as inputs only: a
+// pointer that came out of an asm would be a flat one), which has all of them asked for together.
+//
+// Memory that is the same for a whole launch and every lane, as a pointer that scalar loads go through
+template <class T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T* uniform_memory(const T* p) {
+    return (const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
+
+// n / d in one scalar multiplication (a division of scalars goes through the vector unit and its float reciprocal, some forty dependent
+// instructions).  magic = ceil(2^32 / d) is up to d / 2^32 of itself too large, so that n / d comes out exactly as long as n d < 2^32.
+struct UniformDivisor {
+    uint32_t magic = 0;  // 0: d = 1
+    UniformDivisor() = default;
+    explicit UniformDivisor(int d) : magic(d == 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1) / d)) {}
+    __host__ __device__ __forceinline__ int quotient(int n) const { return magic ? (int)(((uint64_t)(uint32_t)n * magic) >> 32) : n; }
+};
+
 // Per-call parameters every kernel of a verify pass reads from device memory, so a captured
 // launch sequence can be replayed at another base position.
 struct VerifyParams {
