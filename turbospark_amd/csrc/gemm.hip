@@ -245,11 +245,30 @@ int launch_repack(hipStream_t s, int fmt, const uint8_t* raw, int n_rows, int k,
     return TSV_OK;
 }
 
+// The sum over the waves' accumulators of one row group, in wave order: all read before the first addition (at most eight waves)
+__device__ __forceinline__ float4v fold_waves(const float4v* red, int stride, int kparts) {
+    float4v p[8];
+#pragma unroll
+    for (int w = 0; w < 8; w++) p[w] = red[(w < kparts ? w : 0) * stride];
+    float4v v = p[0];
+#pragma unroll
+    for (int w = 1; w < 8; w++)
+        if (w < kparts) v += p[w];
+    return v;
+}
+
+template <int EPI>
+__device__ __forceinline__ RopePre ask_rope(const GemmArgs& a, int tile, int g, int lane) {
+    if constexpr (EPI == EPI_ROPE) return RopePre::ask(a.rope, tile, g, lane);
+    else return RopePre{};
+}
+
 // Stores one row group's finished sums.  v[i] is output column n of activation row 4g+i.
 template <int EPI>
-__device__ __forceinline__ void epilogue(const GemmArgs& a, int tile, int split, int g, float4v v, int lane, int M) {
+__device__ __forceinline__ void epilogue(const GemmArgs& a, int tile, int split, int g, float4v v, int lane, const PassRows& pass, const RopePre& rope) {
+    const int M = pass.m;
     if (EPI == EPI_ROPE) {
-        rope_epilogue(a.rope, a.vp, tile, g, v, lane, M);
+        rope_epilogue(a.rope, pass, rope, tile, g, v, lane);
         return;
     }
     if (EPI == EPI_SILU) {
@@ -259,18 +278,21 @@ __device__ __forceinline__ void epilogue(const GemmArgs& a, int tile, int split,
         const int col = tile * 32 + (lane & 31);  // K index of the down projection
         _Float16* out = (_Float16*)a.out;
         float* sums = (float*)((char*)a.out + xfrag_sum_offset(a.n_valid));
+        _Float16 h[4];
+        float sum[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const float other = __shfl_xor(v[i], 32);
-            const float gate = lane < 32 ? v[i] : other, up = lane < 32 ? other : v[i];
-            const _Float16 h = pinned_half((_Float16)(silu_f(gate) * up));
-            float sum = (float)h;
+            const float2 gu = lanes_by_32(v[i]);
+            h[i] = pinned_half((_Float16)(silu_f(gu.x) * gu.y));
+            sum[i] = sum_of_32((float)h[i]);
+        }
+        if (lane < 32) {
 #pragma unroll
-            for (int o = 1; o < 32; o <<= 1) sum += __shfl_xor(sum, o);
-            const int b = 4 * g + i;
-            if (b < M && lane < 32) {
-                out[frag_index(col, b)] = h;
-                if (lane == 0) sums[xsum_index(col >> 5, b)] = sum;
+            for (int i = 0; i < 4; i++) {
+                const int b = 4 * g + i;
+                if (b >= M) continue;
+                out[frag_index(col, b)] = h[i];
+                if (lane == 0) sums[xsum_index(col >> 5, b)] = sum[i];
             }
         }
         return;
@@ -301,7 +323,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& a, int tile, int split,
 template <class F, int EPI, int NG>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split, int out_tile, float4v* red) {
     constexpr int STAGES = TSV_GEMM_STAGES;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // this wave's run of chunks inside the workgroup's K slice
     const int s0 = split * a.kslice, s1 = min(s0 + a.kslice, a.kchunks);
     const int c0 = min(s0 + wave * a.per, s1);
@@ -316,7 +338,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
     float4v acc[NG];
 #pragma unroll
     for (int g = 0; g < NG; g++) acc[g] = float4v{0.f, 0.f, 0.f, 0.f};
-    const int M = a.vp->m;  // asked for before the K loop, needed after it
+    RopePre rope;
+    const PassRows pass = PassRows::ask(a.vp);
 
     // Software pipeline over the K chunks, STAGES tiles in flight per wave.  Every load in the
     // steady state is unconditional (straight-line code), so the compiler can wait on the oldest
@@ -328,6 +351,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
         auto fetch = [&](Stage<F, NG>& sg, int c) { load_stage(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
 #pragma unroll
         for (int s = 0; s < STAGES; s++) fetch(st[s], min(c0 + s, last));
+        pass.asked();
         int c = 0;
         for (; c + 2 * STAGES <= nc; c += STAGES) {
 #pragma unroll
@@ -336,6 +360,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
                 fetch(st[s], c0 + c + s + STAGES);
             }
         }
+        rope = ask_rope<EPI>(a, out_tile, min(wave, NG - 1), lane);  // (of the row group that the wave finishes first)
         // last group that still has tiles to fetch (fewer than STAGES of them)
 #pragma unroll
         for (int s = 0; s < STAGES; s++) {
@@ -348,11 +373,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
 #pragma unroll
         for (int s = 0; s < STAGES; s++)
             if (c + s < nc) compute(st[s], k, acc);
-    }
+    } else rope = ask_rope<EPI>(a, out_tile, min(wave, NG - 1), lane);
 
     if (a.kparts == 1) {
 #pragma unroll
-        for (int g = 0; g < NG; g++) epilogue<EPI>(a, out_tile, split, g, acc[g], lane, M);
+        for (int g = 0; g < NG; g++) epilogue<EPI>(a, out_tile, split, g, acc[g], lane, pass, ask_rope<EPI>(a, out_tile, g, lane));
         return;
     }
     // fold the waves' accumulators in wave order; wave w finishes row groups w, w + kparts, ...
@@ -360,16 +385,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
     for (int g = 0; g < NG; g++) red[(wave * NG + g) * 64 + lane] = acc[g];
     __syncthreads();
     for (int g = wave; g < NG; g += a.kparts) {
-        float4v v = red[g * 64 + lane];
-        for (int w = 1; w < a.kparts; w++) v += red[(w * NG + g) * 64 + lane];
-        epilogue<EPI>(a, out_tile, split, g, v, lane, M);
+        if (g != wave) rope = ask_rope<EPI>(a, out_tile, g, lane);
+        epilogue<EPI>(a, out_tile, split, g, fold_waves(red + g * 64 + lane, NG * 64, a.kparts), lane, pass, rope);
     }
 }
 
 template <class F, int EPI, int NG>
 __global__ __launch_bounds__(512) void k_gemm(GemmArgs a) {
     extern __shared__ float4v red[];
-    const int split = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
+    ask_for_arguments<EPI>(a);
+    const int tile = a.by_splits.quotient(blockIdx.x), split = blockIdx.x - tile * a.splits;
     gemm_tile<F, EPI, NG>(a, tile, split, tile, red);
 }
 
@@ -463,8 +488,8 @@ __device__ __forceinline__ void compute16(const Stage16& st, const Consts& k, fl
 // the tile); register i is activation row 4 kg + i.
 template <int EPI>
 __device__ __forceinline__ void epilogue16(const GemmArgs& a, int tile, int split, int pr, float4v v0, float4v v1,
-                                           int lane, int M, float* ssum) {
-    const int r = lane & 15, kg = lane >> 4;
+                                           int lane, const PassRows& pass, float* ssum) {
+    const int r = lane & 15, kg = lane >> 4, M = pass.m;
     if (EPI == EPI_SILU) {
         // gate rows are the tile's first 32 rows, up rows the other 32: a lane holds both of a column
         const int col = tile * 32 + 16 * pr + r;  // K index of the down projection
@@ -472,9 +497,7 @@ __device__ __forceinline__ void epilogue16(const GemmArgs& a, int tile, int spli
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const _Float16 h = pinned_half((_Float16)(silu_f(v0[i]) * v1[i]));
-            float sum = (float)h;
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) sum += __shfl_xor(sum, o);
+            const float sum = sum_of_16((float)h);
             const int b = 4 * kg + i;
             if (b < M) out[a.out16 ? frag16_index(col, b) : frag_index(col, b)] = h;
             if (r == 0) ssum[pr * 16 + b] = sum;  // this half of the sub-block's sum
@@ -492,7 +515,7 @@ __device__ __forceinline__ void epilogue16(const GemmArgs& a, int tile, int spli
         const int d0 = kind == 2 ? t * 64 + 16 * pr + r : idim, d1 = kind == 2 ? d0 + 32 : idim + half;
         const int sec = (kind == 0 ? 0 : kind == 1 ? e.nq * hd : (e.nq + e.nkv) * hd) + head * hd;
         const float b0 = e.bias ? e.bias[sec + d0] : 0.f, b1 = e.bias ? e.bias[sec + d1] : 0.f;
-        const int base = a.vp->base;
+        const int base = pass.base;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int b = 4 * kg + i;
@@ -541,7 +564,7 @@ __device__ __forceinline__ void epilogue16(const GemmArgs& a, int tile, int spli
 
 template <int EPI>
 __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, int tile, int split, float4v* red) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int s0 = split * a.kslice, s1 = min(s0 + a.kslice, a.kchunks);
     const int c0 = min(s0 + wave * a.per, s1);
     const int nc = min(a.per, s1 - c0);
@@ -554,10 +577,11 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, int tile, int spl
     float4v acc[4];
 #pragma unroll
     for (int rb = 0; rb < 4; rb++) acc[rb] = float4v{0.f, 0.f, 0.f, 0.f};
-    const int M = a.vp->m;
+    const PassRows pass = PassRows::ask(a.vp);
     if (nc > 0) {
         Stage16 st;
         load_stage16(st, a, wt + (size_t)c0 * Q4K::TILE_BYTES, c0, lane);
+        pass.asked();
         for (int c = 1; c < nc; c++) {
             compute16(st, k, acc, lane >> 4);
             load_stage16(st, a, wt + (size_t)(c0 + c) * Q4K::TILE_BYTES, c0 + c, lane);
@@ -570,17 +594,13 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, int tile, int spl
     __syncthreads();
     float* ssum = (float*)(red + a.kparts * 256);
     for (int pr = wave; pr < 2; pr += a.kparts) {
-        float4v v0 = red[pr * 64 + lane], v1 = red[(pr + 2) * 64 + lane];
-        for (int w = 1; w < a.kparts; w++) {
-            v0 += red[(w * 4 + pr) * 64 + lane];
-            v1 += red[(w * 4 + pr + 2) * 64 + lane];
-        }
-        epilogue16<EPI>(a, tile, split, pr, v0, v1, lane, M, ssum);
+        const float4v v0 = fold_waves(red + pr * 64 + lane, 256, a.kparts), v1 = fold_waves(red + (pr + 2) * 64 + lane, 256, a.kparts);
+        epilogue16<EPI>(a, tile, split, pr, v0, v1, lane, pass, ssum);
     }
     if (EPI == EPI_SILU) {
         // a sub-block of the down projection is this tile's 32 columns: both halves' sums, then one store
         __syncthreads();
-        if (threadIdx.x < 16 && (int)threadIdx.x < M) {
+        if (threadIdx.x < 16 && (int)threadIdx.x < pass.m) {
             float* sums = (float*)((char*)a.out + xfrag_sum_offset(a.n_valid));
             sums[xsum_index(tile, threadIdx.x)] = ssum[threadIdx.x] + ssum[16 + threadIdx.x];
         }
@@ -590,7 +610,9 @@ __device__ __forceinline__ void gemm16_tile(const GemmArgs& a, int tile, int spl
 template <int EPI>
 __global__ __launch_bounds__(512) void k_gemm16(GemmArgs a) {
     extern __shared__ float4v red[];
-    gemm16_tile<EPI>(a, blockIdx.x / a.splits, blockIdx.x % a.splits, red);
+    ask_for_arguments<EPI>(a);
+    const int tile = a.by_splits.quotient(blockIdx.x);
+    gemm16_tile<EPI>(a, tile, blockIdx.x - tile * a.splits, red);
 }
 
 // The rotating q/k/v projection of files that keep the value projection in Q6_K (the *_K_M mixes): the workgroups behind those of the
@@ -603,6 +625,8 @@ template <class F, int NG>
 __global__ __launch_bounds__(512) void k_gemm_qk_v(GemmArgs a, GemmArgs v) {
     extern __shared__ float4v red[];
     const int tile = blockIdx.x;
+    asm volatile("" ::"s"(a.n_tiles), "s"(v.w), "s"(v.kchunks), "s"(v.kslice), "s"(v.per), "s"(v.kparts));
+    ask_for_arguments<EPI_ROPE>(a);
     if (tile >= a.n_tiles) gemm_tile<Q6K, EPI_ROPE, NG ? NG : 4>(v, tile - a.n_tiles, 0, tile, red);
     else if constexpr (NG == 0) gemm16_tile<EPI_ROPE>(a, tile, 0, red);
     else gemm_tile<F, EPI_ROPE, NG>(a, tile, 0, tile, red);
@@ -1083,7 +1107,8 @@ struct WideQ6 {
 template <class P, int EPI>
 __global__ __launch_bounds__(64 * WIDE_BLOCKS) void k_gemm_wide(GemmWideArgs wa) {
     extern __shared__ __attribute__((aligned(16))) uint8_t wide_lds[];  // two unit buffers, then the blocks' sub-block sums
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;  // wave = this wave's block = the row block it unpacks
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave = this wave's block = the row block it unpacks
+    ask_for_arguments<EPI>(wa.g);
     GemmArgs a = wa.g;
     a.xfrag = (const uint2*)((const uint8_t*)a.xfrag + (size_t)wave * wa.x_stride);
     a.xsum = (const float*)((const uint8_t*)a.xsum + (size_t)wave * wa.x_stride);
@@ -1093,7 +1118,7 @@ __global__ __launch_bounds__(64 * WIDE_BLOCKS) void k_gemm_wide(GemmWideArgs wa)
         a.rope.cs += (size_t)wave * 16 * (a.rope.hd >> 1);
         a.rope.q16 += (size_t)wave * 16 * a.rope.nq * a.rope.hd;
     }
-    const int split = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
+    const int tile = a.by_splits.quotient(blockIdx.x), split = blockIdx.x - tile * a.splits;
     const int s0 = split * a.kslice, s1 = min(s0 + a.kslice, a.kchunks);
     const uint8_t* wt = a.w + (size_t)tile * a.kchunks * P::TILE_BYTES;
     Consts k;
@@ -1104,7 +1129,7 @@ __global__ __launch_bounds__(64 * WIDE_BLOCKS) void k_gemm_wide(GemmWideArgs wa)
     float4v acc[4];
 #pragma unroll
     for (int rb = 0; rb < 4; rb++) acc[rb] = float4v{0.f, 0.f, 0.f, 0.f};
-    const int M = a.vp->m;
+    const PassRows pass = PassRows::ask(a.vp);
     // unit u: unpack into buffer u & 1 -> ask for what comes next -> barrier -> multiply unit u.  The
     // barrier of unit u also separates the reads of unit u - 1 from the unpacking of unit u + 1,
     // which goes to the same buffer.  The codes are asked for two units ahead, the activations (which
@@ -1123,6 +1148,7 @@ __global__ __launch_bounds__(64 * WIDE_BLOCKS) void k_gemm_wide(GemmWideArgs wa)
     load_w(w[0], u0);
     P::load_x(x[0], a, u0, lane);
     load_w(w[1], u0 + 1);
+    pass.asked();
     int c = u0;
     for (; c + 2 <= u1; c += 2) {
         P::unpack(w[0], k, buf0, wave, lane);
@@ -1144,10 +1170,10 @@ __global__ __launch_bounds__(64 * WIDE_BLOCKS) void k_gemm_wide(GemmWideArgs wa)
     __syncthreads();  // every wave is done with the unit buffers before the epilogue's sums go to LDS behind them
     float* ssum = (float*)(wide_lds + 2 * P::BUF_BYTES) + wave * 32;
 #pragma unroll
-    for (int pr = 0; pr < 2; pr++) epilogue16<EPI>(a, tile, split, pr, acc[pr], acc[pr + 2], lane, M, ssum);
+    for (int pr = 0; pr < 2; pr++) epilogue16<EPI>(a, tile, split, pr, acc[pr], acc[pr + 2], lane, pass, ssum);
     if (EPI == EPI_SILU) {
         __syncthreads();
-        if (lane < 16 && lane < M) {
+        if (lane < 16 && lane < pass.m) {
             float* sums = (float*)((char*)a.out + xfrag_sum_offset(a.n_valid));
             sums[xsum_index(tile, lane)] = ssum[lane] + ssum[16 + lane];
         }
@@ -1233,6 +1259,7 @@ static int fill_gemm_args(GemmArgs& a, const TiledW& w, const uint4* xfrag, void
     a.kchunks = w.kchunks;
     a.kslice = (w.kchunks + splits - 1) / splits;
     a.splits = (w.kchunks + a.kslice - 1) / a.kslice;
+    a.by_splits = UniformDivisor(a.splits);
     if (epi == EPI_PARTIAL && a.splits != splits) {
         set_error("matmul: split count leaves an empty K slice");
         return TSV_ERR_INVALID;

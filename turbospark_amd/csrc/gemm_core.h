@@ -79,6 +79,14 @@ __device__ __forceinline__ uint32_t lds_after(uint32_t lds, float loaded) {
     return lds;
 }
 
+// A tile's units are asked for in the order in which they are multiplied: loads come back in order, so the first products do not wait for
+// the last unit.  (Left to itself the scheduler puts those that share an address register together.)
+template <class T>
+__device__ __forceinline__ void load_in_order(T& to, const T* p) {
+    to = __builtin_nontemporal_load(p);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // ------------------------------------------------------------------------------- formats
 struct Q4K {
     static constexpr int NSUB = 8, NPAIR = 4, TILE_BYTES = 9216;
@@ -90,7 +98,7 @@ struct Q4K {
     static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int lane) {
         const u32x4* p = (const u32x4*)tile + lane;
 #pragma unroll
-        for (int u = 0; u < 8; u++) r.q[u] = __builtin_nontemporal_load(p + u * 64);
+        for (int u = 0; u < 8; u++) load_in_order(r.q[u], p + u * 64);
         r.s = __builtin_nontemporal_load(p + 512);
     }
     // the same tile copied byte for byte into LDS by the memory pipeline (no registers involved);
@@ -99,9 +107,10 @@ struct Q4K {
 #pragma unroll
         for (int u = 0; u < 9; u++) dma_to_lds_b128(tile + u * 1024 + lane * 16, lds + u * 1024);
     }
-    // float index of this lane's sub-block sums of chunk c, before the row's own offset
+    // float index of the sub-block sums of chunk c, and this lane's place in them before the row's own offset
     // (ActLoader::sumoff) is added: lane (b, i) reads sub-block b
-    static __device__ __forceinline__ int xs_base(int c, int lane) { return c * 128 + ((lane >> 2) & 7) * 4; }
+    static __device__ __forceinline__ int xs_base(int c) { return c * 128; }
+    static __device__ __forceinline__ int xs_lane(int lane) { return ((lane >> 2) & 7) * 4; }
 };
 
 // Q5_K (crates/compute/src/quant_gguf/q5_k.rs:47-96): the Q4_K tile followed by the fifth bits,
@@ -117,12 +126,13 @@ struct Q5K {
     static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int lane) {
         const u32x4* p = (const u32x4*)tile + lane;
 #pragma unroll
-        for (int u = 0; u < 8; u++) r.q[u] = __builtin_nontemporal_load(p + u * 64);
+        for (int u = 0; u < 8; u++) load_in_order(r.q[u], p + u * 64);
         r.s = __builtin_nontemporal_load(p + 512);
         r.h[0] = __builtin_nontemporal_load(p + 576);
         r.h[1] = __builtin_nontemporal_load(p + 640);
     }
-    static __device__ __forceinline__ int xs_base(int c, int lane) { return c * 128 + ((lane >> 2) & 7) * 4; }
+    static __device__ __forceinline__ int xs_base(int c) { return c * 128; }
+    static __device__ __forceinline__ int xs_lane(int lane) { return ((lane >> 2) & 7) * 4; }
 };
 
 struct Q80 {
@@ -135,7 +145,7 @@ struct Q80 {
     static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int lane) {
         const u32x4* p = (const u32x4*)tile + lane;
 #pragma unroll
-        for (int u = 0; u < 8; u++) r.q[u] = __builtin_nontemporal_load(p + u * 64);
+        for (int u = 0; u < 8; u++) load_in_order(r.q[u], p + u * 64);
         r.s = __builtin_nontemporal_load((const u32x2*)(tile + 8192) + lane);
     }
     static __device__ __forceinline__ void load_to_lds(uint32_t lds, const uint8_t* tile, int lane) {
@@ -146,9 +156,8 @@ struct Q80 {
         for (int h = 0; h < 2; h++) dma_to_lds_b32(tile + 8192 + h * 256 + lane * 4, lds + 8192 + h * 256);
     }
     // a 128-element chunk is half of a 256-element sum group: its four sub-blocks go to blocks 0..3
-    static __device__ __forceinline__ int xs_base(int c, int lane) {
-        return (c >> 1) * 128 + (c & 1) * 16 + ((lane >> 2) & 3) * 4;
-    }
+    static __device__ __forceinline__ int xs_base(int c) { return (c >> 1) * 128 + (c & 1) * 16; }
+    static __device__ __forceinline__ int xs_lane(int lane) { return ((lane >> 2) & 3) * 4; }
 };
 
 // activation registers of one K chunk
@@ -167,7 +176,8 @@ struct MX4 {
     static __device__ __forceinline__ void load_to_lds(uint32_t lds, const uint8_t* tile, int lane) {
         Q80::load_to_lds(lds, tile, lane);
     }
-    static __device__ __forceinline__ int xs_base(int c, int lane) { return Q4K::xs_base(c, lane); }
+    static __device__ __forceinline__ int xs_base(int c) { return Q4K::xs_base(c); }
+    static __device__ __forceinline__ int xs_lane(int lane) { return Q4K::xs_lane(lane); }
 };
 
 // bf16 matrices (crates/compute/src/quant.rs:14-39: a bf16 is the upper half of the fp32 bits).
@@ -184,9 +194,10 @@ struct BF16W {
     static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int lane) {
         const u32x4* p = (const u32x4*)tile + lane;
 #pragma unroll
-        for (int u = 0; u < 8; u++) r.q[u] = __builtin_nontemporal_load(p + u * 64);
+        for (int u = 0; u < 8; u++) load_in_order(r.q[u], p + u * 64);
     }
-    static __device__ __forceinline__ int xs_base(int, int) { return 0; }
+    static __device__ __forceinline__ int xs_base(int) { return 0; }
+    static __device__ __forceinline__ int xs_lane(int) { return 0; }
 };
 
 // Q6_K (crates/compute/src/quant_gguf/q6_k.rs:44-88): value = d * sc_j * (level - 32), level = 4 low
@@ -204,11 +215,12 @@ struct Q6K {
     static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int lane) {
         const u32x4* p = (const u32x4*)tile + lane;
 #pragma unroll
-        for (int u = 0; u < 12; u++) r.q[u] = __builtin_nontemporal_load(p + u * 64);
+        for (int u = 0; u < 12; u++) load_in_order(r.q[u], p + u * 64);
         r.s = __builtin_nontemporal_load(p + 12 * 64);
         r.d = __builtin_nontemporal_load((const uint32_t*)(tile + 13312) + lane);
     }
-    static __device__ __forceinline__ int xs_base(int, int) { return 0; }
+    static __device__ __forceinline__ int xs_base(int) { return 0; }
+    static __device__ __forceinline__ int xs_lane(int) { return 0; }
 };
 
 template <int STEP>
@@ -283,13 +295,14 @@ struct ActLoader {
             sums = __builtin_amdgcn_make_buffer_rsrc((void*)xsum, 0, 0x7FFFFFFF, 0x00027000);
         }
     }
-    __device__ __forceinline__ u32x2 frag_at(int idx) const {  // idx in 8-byte units
-        if (COHERENT) return __builtin_amdgcn_raw_buffer_load_b64(frag, idx * 8, 0, 16);
-        return fragp[idx];
+    // fragment `lane_at` (in 8-byte units) behind unit `at`, which is the same for a wave: its share of the address stays on the scalar unit
+    __device__ __forceinline__ u32x2 frag_at(int at, int lane_at) const {
+        if (COHERENT) return __builtin_amdgcn_raw_buffer_load_b64(frag, (at + lane_at) * 8, 0, 16);
+        return *(const u32x2*)((const char*)(fragp + at) + (uint32_t)(lane_at * 8));
     }
-    __device__ __forceinline__ float sum_at(int idx) const {
-        if (COHERENT) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, idx * 4, 0, 16));
-        return sump[idx];
+    __device__ __forceinline__ float sum_at(int at, int lane_at) const {
+        if (COHERENT) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, (at + lane_at) * 4, 0, 16));
+        return *(const float*)((const char*)(sump + at) + (uint32_t)(lane_at * 4));
     }
 };
 
@@ -299,10 +312,10 @@ __device__ __forceinline__ void load_x(XRegs<F, NG>& xr, const ActLoader<COH>& x
 #pragma unroll
     for (int p = 0; p < F::NPAIR; p++)
 #pragma unroll
-        for (int g = 0; g < NG; g++) xr.xa[p][g] = x.frag_at((c * F::NPAIR + p) * 256 + x.rowoff[g] + (lane >> 2) * 4);
+        for (int g = 0; g < NG; g++) xr.xa[p][g] = x.frag_at((c * F::NPAIR + p) * 256, x.rowoff[g] + (lane >> 2) * 4);
     if (F::SUMS) {
 #pragma unroll
-        for (int g = 0; g < NG; g++) xr.xs[g] = x.sum_at(F::xs_base(c, lane) + x.sumoff[g]);
+        for (int g = 0; g < NG; g++) xr.xs[g] = x.sum_at(F::xs_base(c), F::xs_lane(lane) + x.sumoff[g]);
     }
 }
 
@@ -313,6 +326,7 @@ __device__ __forceinline__ void load_stage(Stage<F, NG>& st, const ActLoader<COH
                                            int lane) {
     __builtin_amdgcn_sched_barrier(0);
     load_x(st.x, x, c, lane);
+    __builtin_amdgcn_sched_barrier(0);
     F::load(st.w, tile_chunk, lane);
     __builtin_amdgcn_sched_barrier(0);
 }
@@ -613,45 +627,82 @@ __device__ __forceinline__ void compute(const Stage<F, NG>& st, const Consts& k,
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)); }
 
+// How many rows a pass has and where they begin: asked for before a matmul's K loop, through scalar loads that its end waits for.
+// (A plain load of such a value went through the vector unit, and the compiler waited for it where it stood: the first weights were asked for
+// one round trip to memory later.  With the arguments in one batch, the divisions gone and the ends' sums on the vector ALU, five rows through 32 layers of
+// the 8B shape in Q4_K, 128 launches, 2127 -> 2052 us; twelve routed layers' 37 launches 1153 -> 1131; one row through a Q4_K_M mix 1.9 %.)
+struct PassRows {
+    int m, base;
+    static __device__ __forceinline__ PassRows ask(const VerifyParams* vp) { return {uniform_memory(vp)->m, uniform_memory(vp)->base}; }
+    // keeps the loads where they were asked for, ahead of what stands before this
+    __device__ __forceinline__ void asked() const { asm volatile("" ::"s"(m), "s"(base)); }
+};
+
+// All that a matmul reads of its arguments, asked for together (uniform_memory)
+template <int EPI>
+__device__ __forceinline__ void ask_for_arguments(const GemmArgs& a) {
+    if (EPI == EPI_ROPE)
+        asm volatile("" ::"s"(a.w), "s"(a.xfrag), "s"(a.xsum), "s"(a.vp), "s"(a.kchunks), "s"(a.kslice), "s"(a.splits), "s"(a.by_splits.magic), "s"(a.kparts),
+                     "s"(a.per), "s"(a.rope.cs), "s"(a.rope.bias), "s"(a.rope.q16), "s"(a.rope.kc), "s"(a.rope.vc), "s"(a.rope.nq), "s"(a.rope.nkv),
+                     "s"(a.rope.hd), "s"(a.rope.max_ctx));
+    else
+        asm volatile("" ::"s"(a.w), "s"(a.xfrag), "s"(a.xsum), "s"(a.out), "s"(a.vp), "s"(a.kchunks), "s"(a.kslice), "s"(a.splits), "s"(a.by_splits.magic),
+                     "s"(a.kparts), "s"(a.per), "s"(a.ldo), "s"(a.n_valid), "s"(a.out16));
+}
+
 // The fused q/k/v projection finishing its own rows (no split-K: the sums are complete here).
 // A tile of the rotated sections holds dims i (lanes 0..31) and i + hd/2 (lanes 32..63) of one
 // head: the NeoX pair of a lane is lane ^ 32 (crates/compute/src/rope.rs:208-256).  Bias first,
 // then the rotation (families/gptoss/attn.rs:88-118); q goes to the fp16 q buffer, K and V
 // straight into the cache slot of the row (families/qwen/batched_layers.rs:84-113).
-__device__ __forceinline__ void rope_epilogue(const RopeEpi& e, const VerifyParams* vp, int tile, int g, float4v v, int lane, int M) {
-    const int hd = e.hd, half = hd >> 1, tph = hd >> 6;  // tiles per head
-    const int tq = e.nq * tph, tk = e.nkv * tph;
-    const int kind = tile < tq ? 0 : tile < tq + tk ? 1 : 2;
-    const int st = kind == 0 ? tile : kind == 1 ? tile - tq : tile - tq - tk;
-    const int head = st / tph, t = st - head * tph;
-    const bool hi = lane >= 32;
-    const int idim = (tph == 2 ? 32 * t : 0) + (lane & 31);     // rotation pair index, 0 .. hd/2
-    const int d = kind == 2 ? t * 64 + lane : (hi ? idim + half : idim);  // this lane's head dimension
-    const int col = (kind == 0 ? 0 : kind == 1 ? e.nq * hd : (e.nq + e.nkv) * hd) + head * hd + d;
-    const float bias = e.bias ? e.bias[col] : 0.f;
-    const int base = vp->base;
+struct RopeTile {  // what a tile holds for this lane
+    int kind, head, d, idim;  // 0: q, 1: k, 2: v; the dimension; the rotation pair
+    __device__ __forceinline__ RopeTile(const RopeEpi& e, int tile, int lane) {
+        const int hd = e.hd, half = hd >> 1, sh = hd == 128 ? 1 : 0;  // tiles per head: 1 << sh
+        const int tq = e.nq << sh, tk = e.nkv << sh;
+        kind = tile < tq ? 0 : tile < tq + tk ? 1 : 2;
+        const int st = kind == 0 ? tile : kind == 1 ? tile - tq : tile - tq - tk;
+        head = st >> sh;
+        const int t = st - (head << sh);
+        idim = (sh ? 32 * t : 0) + (lane & 31);  // 0 .. hd/2
+        d = kind == 2 ? t * 64 + lane : (lane >= 32 ? idim + half : idim);
+    }
+};
+// ... and what its rows 4 g .. 4 g + 3 need from memory.  (Rows that do not exist: the table has sixteen.)
+struct RopePre {
     float2 cs[4];
+    float bias;
+    static __device__ __forceinline__ RopePre ask(const RopeEpi& e, int tile, int g, int lane) {
+        const RopeTile at(e, tile, lane);
+        const int half = e.hd >> 1, col = (at.kind == 0 ? 0 : at.kind == 1 ? e.nq * e.hd : (e.nq + e.nkv) * e.hd) + at.head * e.hd + at.d;
+        RopePre p;
+        const float b = *(e.bias ? e.bias + col : (const float*)e.cs);  // (no branch around a load)
+        p.bias = e.bias ? b : 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) cs[i] = kind != 2 && 4 * g + i < M ? e.cs[(4 * g + i) * half + idim] : float2{1.f, 0.f};
+        for (int i = 0; i < 4; i++) p.cs[i] = e.cs[(4 * g + i) * half + at.idim];
+        return p;
+    }
+};
+__device__ __forceinline__ void rope_epilogue(const RopeEpi& e, const PassRows& pass, const RopePre& pre, int tile, int g, float4v v, int lane) {
+    const RopeTile at(e, tile, lane);
+    const int hd = e.hd, first = pass.base % e.max_ctx;
+    const bool hi = lane >= 32;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int b = 4 * g + i;
-        float x = v[i] + bias;
-        const float other = __shfl_xor(x, 32);
-        if (b >= M) continue;
-        if (kind != 2) {
-            const float x0 = hi ? other : x, x1 = hi ? x : other;
-            x = hi ? x0 * cs[i].y + x1 * cs[i].x : x0 * cs[i].x - x1 * cs[i].y;
-        }
+        float x = v[i] + pre.bias;
+        const float2 pair = lanes_by_32(x);
+        if (b >= pass.m) continue;
+        if (at.kind != 2) x = hi ? pair.x * pre.cs[i].y + pair.y * pre.cs[i].x : pair.x * pre.cs[i].x - pair.y * pre.cs[i].y;
         const _Float16 h = (_Float16)x;
-        if (kind == 0) {
-            ((_Float16*)e.q16)[((long)b * e.nq + head) * hd + d] = h;
+        if (at.kind == 0) {
+            ((_Float16*)e.q16)[((long)b * e.nq + at.head) * hd + at.d] = h;
         } else {
-            const int pos = (base + b) % e.max_ctx;  // the cache slot of row b (a ring layer wraps at its capacity)
-            if (kind == 1)
-                ((_Float16*)e.kc)[kcache_index(head, pos, d, hd, e.max_ctx)] = h;
+            const int pos = first + b - (first + b >= e.max_ctx ? e.max_ctx : 0);  // the cache slot of row b (a ring layer wraps at its capacity)
+            if (at.kind == 1)
+                ((_Float16*)e.kc)[kcache_index(at.head, pos, at.d, hd, e.max_ctx)] = h;
             else
-                ((_Float16*)e.vc)[vcache_index(head, pos, d, hd, e.max_ctx)] = h;
+                ((_Float16*)e.vc)[vcache_index(at.head, pos, at.d, hd, e.max_ctx)] = h;
         }
     }
 }

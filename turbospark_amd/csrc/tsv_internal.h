@@ -158,6 +158,50 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* uniform_me
     return (const __attribute__((address_space(4))) T*)(uintptr_t)p;
 }
 
+// Sums over neighbouring lanes on the vector ALU: the same pairs, in the same order and so to the same bits, as v += __shfl_xor(v, o), which goes
+// through the LDS and waits some 120 cycles for each.  All lanes of the wave take part.
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+// The two rows of sixteen lanes, or the two halves of the wave, in both: {the lower one's value, the upper one's}.  (The second operand is
+// hidden from the compiler, which takes the two results of equal operands for one.)
+__device__ __forceinline__ float2 lanes_by_16(float v) {
+    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
+    asm("" : "+v"(b));
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    return float2{__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+}
+__device__ __forceinline__ float2 lanes_by_32(float v) {
+    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
+    asm("" : "+v"(b));
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return float2{__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+}
+// over 16 lanes in the order 1, 2, 4, 8 (lanes whose sums agree already stand in for each other: the mirrors)
+__device__ __forceinline__ float sum_of_16(float v) {
+    v += dpp_f32<0xB1>(v);   // l ^ 1
+    v += dpp_f32<0x4E>(v);   // l ^ 2
+    v += dpp_f32<0x141>(v);  // 7 - l
+    v += dpp_f32<0x140>(v);  // 15 - l
+    return v;
+}
+__device__ __forceinline__ float sum_of_32(float v) {
+    const float2 r = lanes_by_16(sum_of_16(v));
+    return r.x + r.y;
+}
+// over the wave in the order 32, 16, 8, 4, 2, 1
+__device__ __forceinline__ float sum_of_wave(float v) {
+    const float2 h = lanes_by_32(v);
+    const float2 r = lanes_by_16(h.x + h.y);
+    v = r.x + r.y;
+    v += dpp_f32<0x128>(v);  // l + 8 of 16
+    v += dpp_f32<0x124>(v);  // l + 4: the two eights agree
+    v += dpp_f32<0x4E>(v);
+    v += dpp_f32<0xB1>(v);
+    return v;
+}
+
 // n / d in one scalar multiplication (a division of scalars goes through the vector unit and its float reciprocal, some forty dependent
 // instructions).  magic = ceil(2^32 / d) is up to d / 2^32 of itself too large, so that n / d comes out exactly as long as n d < 2^32.
 struct UniformDivisor {
@@ -199,6 +243,7 @@ struct GemmArgs {
                          // next matmul; EPI_LOGITS: half [m][ldo]
     const VerifyParams* vp;
     int n_tiles, kchunks, kslice, splits, kparts, per, ldo, n_valid;
+    UniformDivisor by_splits;
     int out16;     // EPI_SILU: write the fragments in the prompt kernel's layout (frag16_index)
     RopeEpi rope;  // EPI_ROPE only
 };
