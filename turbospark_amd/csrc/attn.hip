@@ -34,23 +34,15 @@ int attn_chunks(int nkv) {
 #define TSV_ATTN_STAGES2_HD64 3
 #endif
 
-// Eight waves per workgroup share a chunk of the context (attn_core.h).
+// Eight waves per workgroup share a chunk of the context (attn_core.h).  Grid (chunks, kv heads, 16-row blocks of a prompt pass).
+// What a launch costs beside its bytes is the round trips before the first K and V are asked for: the arguments come in one batch, and nothing
+// is divided on the way.
 template <int HD, int RT, int STAGES>
 __global__ __launch_bounds__(512) void k_attn_partial(AttnArgs a, int G, int R) {
     extern __shared__ float xch[];  // [8 slots][PER_LANE values][64 lanes]
-    if (a.xcd_groups) {  // several row groups of a verify pass: placed by die
-        int chunk, kvh, grp;
-        if (attn_grid_place(a, blockIdx.x, chunk, kvh, grp)) attn_partial_body<HD, RT, STAGES, false>(a, G, R, chunk, kvh, grp * RT, xch);
-        return;
-    }
-    // grid z: row groups of the pass, times the 16-row blocks of a prompt pass
-    const int groups = gridDim.z / max(a.blocks, 1), blk = blockIdx.z / groups, grp = blockIdx.z - blk * groups;
-    if (a.blocks > 1) {
-        const AttnArgs v = attn_block_view(a, blk);
-        attn_partial_body<HD, RT, STAGES, false>(v, G, R, blockIdx.x, blockIdx.y, grp * RT, xch);
-        return;
-    }
-    attn_partial_body<HD, RT, STAGES, false>(a, G, R, blockIdx.x, blockIdx.y, grp * RT, xch);
+    ask_for_arguments(a, G, R);
+    const AttnArgs v = a.blocks > 1 ? attn_block_view(a, blockIdx.z) : a;
+    attn_partial_body<HD, RT, STAGES, false>(v, G, R, blockIdx.x, blockIdx.y, 0, xch);
 }
 
 // A pass of more than two row tiles: TG tile groups side by side in one workgroup (attn_core.h), one read of the
@@ -58,18 +50,16 @@ __global__ __launch_bounds__(512) void k_attn_partial(AttnArgs a, int G, int R) 
 template <int HD, int RT, int STAGES, int TG>
 __global__ __launch_bounds__(64 * TG * attn_phases(TG)) void k_attn_partial_groups(AttnArgs a, int G, int R) {
     extern __shared__ float xch[];
-    if (a.blocks > 1) {
-        const AttnArgs v = attn_block_view(a, blockIdx.z);
-        attn_partial_body<HD, RT, STAGES, false, TG>(v, G, R, blockIdx.x, blockIdx.y, 0, xch);
-        return;
-    }
-    attn_partial_body<HD, RT, STAGES, false, TG>(a, G, R, blockIdx.x, blockIdx.y, 0, xch);
+    ask_for_arguments(a, G, R);
+    const AttnArgs v = a.blocks > 1 ? attn_block_view(a, blockIdx.z) : a;
+    attn_partial_body<HD, RT, STAGES, false, TG>(v, G, R, blockIdx.x, blockIdx.y, 0, xch);
 }
 
 // A short context (launch_hd): one workgroup per KV head and row group, which finishes its rows
 template <int HD, int RT, int STAGES>
 __global__ __launch_bounds__(512) void k_attn_direct(AttnArgs a, int G, int R) {
     extern __shared__ float xch[];
+    ask_for_arguments(a, G, R);
     attn_partial_body<HD, RT, STAGES, false, 1, true>(a, G, R, 0, blockIdx.y, blockIdx.z * RT, xch);
 }
 
@@ -78,113 +68,114 @@ template <int HD, int RT, int KB, int VB>
 __global__ __launch_bounds__(512) void k_attn_partial_tq(AttnArgs a, int G, int R) {
     extern __shared__ float xch[];
     __shared__ uint32_t s_kpair[1 << (2 * KB)], s_vpair[1 << (2 * VB)];
-    tq_fill_pairs(s_kpair, a.tq.k_cb, KB, threadIdx.x, 512);
-    tq_fill_pairs(s_vpair, a.tq.v_cb, VB, threadIdx.x, 512);
-    __syncthreads();
+    asm volatile("" ::"s"(a.tq.kq), "s"(a.tq.kn), "s"(a.tq.vq), "s"(a.tq.vn), "s"(a.tq.k_cb), "s"(a.tq.v_cb), "s"(a.by_xcd_groups.magic), "s"(a.nkv),
+                 "s"(a.q16), "s"(a.part_o), "s"(a.part_ml), "s"(a.nq), "s"(a.max_ctx), "s"(a.nch), "s"(a.scale), "s"(a.vp), "s"(a.m_hint), "s"(a.base_hint),
+                 "s"(a.blocks), "s"(a.xcd_groups), "s"(a.by_group.magic), "s"(a.by_chunks.magic), "s"(G), "s"(R));
+    TqPairs<KB> kp(a.tq.k_cb, threadIdx.x);
+    TqPairs<VB> vp(a.tq.v_cb, threadIdx.x);
+    // the tables are filled behind the first loads of the stores, one barrier for every wave
+    auto tables = [&] {
+        kp.put(s_kpair, threadIdx.x);
+        vp.put(s_vpair, threadIdx.x);
+        __syncthreads();
+    };
     // blocks in flight: three, two where the three-bit fields' extra words would push the registers past 256
     constexpr int STAGES = (HD == 128 && RT == 2 && KB == 3 && VB == 3) ? 2 : 3;
+    // several row groups of a verify pass are placed by die; else grid z: row groups of the pass, times the 16-row blocks of a prompt pass
+    int chunk = blockIdx.x, kvh = blockIdx.y, grp = blockIdx.z, blk = 0;
     if (a.xcd_groups) {
-        int chunk, kvh, grp;
-        if (attn_grid_place(a, blockIdx.x, chunk, kvh, grp))
-            attn_partial_body_tq<HD, RT, STAGES, KB, VB>(a, G, R, chunk, kvh, grp * RT, xch, s_kpair, s_vpair);
-        return;
+        if (!attn_grid_place(a, blockIdx.x, chunk, kvh, grp)) return;
+    } else if (a.blocks > 1) {
+        const int groups = gridDim.z / a.blocks;
+        blk = blockIdx.z / groups;
+        grp = blockIdx.z - blk * groups;
     }
-    // grid z: row groups of the pass, times the 16-row blocks of a prompt pass
-    const int groups = gridDim.z / max(a.blocks, 1), blk = blockIdx.z / groups, grp = blockIdx.z - blk * groups;
-    if (a.blocks > 1) {
-        const AttnArgs v = attn_block_view(a, blk);
-        attn_partial_body_tq<HD, RT, STAGES, KB, VB>(v, G, R, blockIdx.x, blockIdx.y, grp * RT, xch, s_kpair, s_vpair);
-        return;
-    }
-    attn_partial_body_tq<HD, RT, STAGES, KB, VB>(a, G, R, blockIdx.x, blockIdx.y, grp * RT, xch, s_kpair, s_vpair);
+    const AttnArgs v = a.blocks > 1 ? attn_block_view(a, blk) : a;
+    attn_partial_body_tq<HD, RT, STAGES, KB, VB>(v, G, R, chunk, kvh, grp * RT, xch, s_kpair, s_vpair, tables);
 }
 
 // Merge the chunk partials (crates/gpu/src/shaders/attention.metal:122-140 semantics:
 // m* = max m_c, D = sum l_c e^{m_c-m*}, O = sum O_c e^{m_c-m*}, out = O / D) and store the row
 // as fp16 activation fragments (and sub-block sums) of the output projection (K index =
-// q_head*hd + d).  The first
-// wave turns the (m_c, l_c) pairs into per-chunk weights once; every thread then sums its
-// output element over the chunks with independent loads.
+// q_head*hd + d).  Every wave turns the (m_c, l_c) pairs into per-chunk weights, lane c chunk c's, and hands them to all of its
+// lanes through scalar registers: no LDS and no barrier (with them, arguments fetched where they were needed and lane sums through the LDS the merge
+// of 32 chunks took 3.4 us in the 8B step).
 // NCH > 0: the chunk count as a compile-time constant -- every thread then asks for its output
 // element of all chunks before the (m, l) pairs are looked at (the two groups of loads do not
 // depend on each other), and the kernel is one memory latency instead of two.  NCH == 0: any count.
 template <int NCH, bool UNROT>
-__global__ void k_attn_combine(AttnArgs a0, int G, int R) {
+__global__ __launch_bounds__(128) void k_attn_combine(AttnArgs a0, int G, int R) {
+    asm volatile("" ::"s"(a0.part_o), "s"(a0.part_ml), "s"(a0.xfrag), "s"(a0.nq), "s"(a0.hd), "s"(a0.nch), "s"(a0.sinks), "s"(a0.frag16), "s"(a0.unrot),
+                 "s"(a0.blocks), "s"(a0.by_group.magic), "s"(G), "s"(R));
     const AttnArgs a = a0.blocks > 1 ? attn_block_view(a0, blockIdx.z) : a0;
-    __shared__ float wgt[64];
-    __shared__ float s_den;
-    const int m = blockIdx.x, qh = blockIdx.y, d = threadIdx.x;
-    const int hd = a.hd, nch = NCH > 0 ? NCH : a.nch;
-    const int h = qh / G, g = qh - h * G, r = m * G + g;
-    const float* po = a.part_o + ((long)h * nch * R + r) * hd + min(d, hd - 1);
+    const int m = blockIdx.x, qh = blockIdx.y, t = threadIdx.x, lane = t & 63;
+    const int hd = a.hd, nch = NCH > 0 ? NCH : a.nch;  // (the workgroup has hd threads, 64 or 128)
+    const int h = a.by_group.quotient(qh), g = qh - h * G, r = m * G + g;
+    const long slot0 = (long)h * nch * R + r;
+    const float* const po = a.part_o + slot0 * hd;
     const long stride = (long)R * hd;
+    auto element = [&](int c) { return *(const float*)((const char*)(po + c * stride) + (uint32_t)(t * 4)); };
+    // (a lane past the last chunk: the last chunk's pair, not used)
+    const float2 ml = *(const float2*)(a.part_ml + (slot0 + (long)min(lane, nch - 1) * R) * 2);
     float pre[NCH > 0 ? NCH : 1];
-    if (NCH > 0) {
 #pragma unroll
-        for (int c = 0; c < NCH; c++) pre[c] = po[c * stride];
-    }
-    if (d < 64) {
-        float mc = -INFINITY, lc = 0.f;
-        if (d < nch) {
-            const long slot = ((long)h * nch + d) * R + r;
-            mc = a.part_ml[slot * 2];
-            lc = a.part_ml[slot * 2 + 1];
-        }
-        float mx = mc;
-        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        // the sink joins the maximum and the denominator, never the numerator
-        // (crates/compute/src/attention.rs:94-105)
-        const float sink = a.sinks ? a.sinks[qh] : -INFINITY;
-        mx = fmaxf(mx, sink);
-        const float w = mc > -INFINITY ? __expf(mc - mx) : 0.f;
-        float den = lc * w;
-        for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o);
-        if (a.sinks) den += __expf(sink - mx);
-        wgt[d] = w;
-        if (d == 0) s_den = den;
-    }
-    __syncthreads();
-    if (d >= hd) return;
+    for (int c = 0; c < NCH; c++) pre[c] = element(c);
+    const float sink = a.sinks ? uniform_memory(a.sinks)[qh] : -INFINITY;
+    const float sign = UNROT ? a.unrot[t] : 1.0f;
+    const bool live = lane < nch;
+    const float mc = live ? ml.x : -INFINITY, lc = live ? ml.y : 0.f;
+    // the sink joins the maximum and the denominator, never the numerator
+    // (crates/compute/src/attention.rs:94-105)
+    const float mx = fmaxf(max_of_wave(mc), sink);
+    const float w = mc > -INFINITY ? __expf(mc - mx) : 0.f;
+    float den = sum_of_wave(lc * w);
+    if (a.sinks) den += __expf(sink - mx);
+    auto weight = [&](int c) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), c)); };
     float num = 0.f;
     if (NCH > 0) {
 #pragma unroll
-        for (int c = 0; c < NCH; c++) num = fmaf(wgt[c], pre[c], num);
+        for (int c = 0; c < NCH; c++) num = fmaf(weight(c), pre[c], num);
     } else {
 #pragma unroll 8
-        for (int c = 0; c < nch; c++) num = fmaf(wgt[c], po[c * stride], num);
+        for (int c = 0; c < nch; c++) num = fmaf(weight(c), element(c), num);
     }
-    float res = num / s_den;
+    float res = num / den;
     if (UNROT) {
         // the sum was taken over rotated value rows: back through the normalized Hadamard transform
         // (crates/compute/src/wht.rs:15-29, stage h pairs d with d + h) and the value signs
         __shared__ float s_h[128];
         const float c = 0.70710678118654752440f;
-        for (int st = 1; st < hd; st <<= 1) {
-            s_h[d] = res;
+        auto stage = [&](float other, bool upper) { res = (upper ? other - res : res + other) * c; };
+        stage(lane_xor<1>(res), lane & 1);
+        stage(lane_xor<2>(res), lane & 2);
+        stage(lane_xor<4>(res), lane & 4);
+        stage(lane_xor<8>(res), lane & 8);
+        const float2 p = lanes_by_16(res);
+        stage(lane & 16 ? p.x : p.y, lane & 16);
+        const float2 q = lanes_by_32(res);
+        stage(lane & 32 ? q.x : q.y, lane & 32);
+        if (hd == 128) {  // the two waves' halves
+            s_h[t] = res;
             __syncthreads();
-            const float other = s_h[d ^ st];
-            __syncthreads();
-            res = ((d & st) ? other - res : res + other) * c;
+            stage(s_h[t ^ 64], t & 64);
         }
-        res *= a.unrot[d];
+        res *= sign;
     }
-    const _Float16 o16 = (_Float16)res;
-    const int kk = qh * hd + d;
+    const _Float16 o16 = pinned_half((_Float16)res);
+    const int kk = qh * hd + t;
     ((_Float16*)a.xfrag)[a.frag16 ? frag16_index(kk, m) : frag_index(kk, m)] = o16;
     // sum of each 32-element sub-block of the output projection's input (32 neighbouring threads)
-    float sum = (float)o16;
-    for (int o = 1; o < 32; o <<= 1) sum += __shfl_xor(sum, o);
-    if ((d & 31) == 0) ((float*)((char*)a.xfrag + xfrag_sum_offset(a.nq * hd)))[xsum_index(kk >> 5, m)] = sum;
+    const float sum = sum_of_32((float)o16);
+    if ((t & 31) == 0) ((float*)((char*)a.xfrag + xfrag_sum_offset(a.nq * hd)))[xsum_index(kk >> 5, m)] = sum;
 }
 
 template <int HD, int RT, int STAGES>
-static int launch_partial(hipStream_t s, const AttnArgs& a, int G, int R, int groups) {
+static int launch_partial(hipStream_t s, const AttnArgs& a, int G, int R) {
     constexpr int PER_LANE = RT * (HD / 16) * 4 + 2 * RT;
     constexpr size_t lds = (size_t)8 * 64 * PER_LANE * 4;
     static OncePerDevice allowed;
     if (int rc = allow_lds((const void*)k_attn_partial<HD, RT, STAGES>, lds, allowed)) return rc;
-    const dim3 grid = a.xcd_groups ? dim3(attn_grid_size(a.nch * a.nkv, groups)) : dim3(a.nch, a.nkv, groups * std::max(a.blocks, 1));
-    hipLaunchKernelGGL((k_attn_partial<HD, RT, STAGES>), grid, dim3(512), lds, s, a, G, R);
+    hipLaunchKernelGGL((k_attn_partial<HD, RT, STAGES>), dim3(a.nch, a.nkv, std::max(a.blocks, 1)), dim3(512), lds, s, a, G, R);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }
@@ -245,6 +236,7 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
     // about one workgroup per compute unit: the chunk count shrinks as the row groups multiply
     // (fewer, longer chunks also mean fewer partial results for the merge to read)
     AttnArgs a = a0;
+    a.by_group = UniformDivisor(G);
     // A short context in one workgroup per KV head and row group, up to ATTN_DIRECT_BLOCKS / 8 blocks a wave, which finishes its rows
     // itself.  What that takes off a layer against chunks and a merge (8B shape, 1 / 5 / 16 rows, us): 2.5 / 2.9 / 5.3 at 250 positions,
     // 0.7 / 0.6 / 3.5 at 490, and with the line further out 0.0 / -0.6 / 2.4 at 620, -0.4 / -1.2 / 1.8 at 730; four KV heads with groups
@@ -257,6 +249,7 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
     const bool few = attn_short(a.kv_end) || (a.window > 0 && (a.window + TSV_MAX_ROWS + 14) / 16 + 1 <= ATTN_DIRECT_BLOCKS);
     if (a.kv_end > 0 && a.blocks <= 1 && !a.tq.k_bits && !a.frag16 && few) {
         a.nch = 1;
+        a.by_chunks = UniformDivisor(1);
         return trt <= 1 ? launch_direct<HD, 1, 3>(s, a, G, R, 1)
                         : launch_direct<HD, 2, (HD == 128 ? TSV_ATTN_STAGES2_HD128 : TSV_ATTN_STAGES2_HD64)>(s, a, G, R, groups);
     }
@@ -266,6 +259,8 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
     // workgroups, or its last one waits for a whole workgroup to end (26 against 18 us at 21 chunks x 4 heads x 3)
     a.xcd_groups = (groups > 1 && a0.blocks <= 1) ? groups : 0;
     if (a.xcd_groups) a.nch = std::max(std::min(a0.nch, 8), std::min(a0.nch, 8 * (32 / groups) / a0.nkv));
+    a.by_chunks = UniformDivisor(a.nch);
+    if (a.xcd_groups) a.by_xcd_groups = UniformDivisor(a.xcd_groups);
     int rc;
     if (a.tq.k_bits) {
         if (a.window || a.ring || !a.unrot) {
@@ -274,9 +269,9 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
         }
         rc = trt <= 1 ? launch_partial_tq_widths<HD, 1>(s, a, G, R, 1) : launch_partial_tq_widths<HD, 2>(s, a, G, R, groups);
     } else if (trt <= 1)
-        rc = launch_partial<HD, 1, 3>(s, a, G, R, 1);
+        rc = launch_partial<HD, 1, 3>(s, a, G, R);
     else if (trt <= 2)
-        rc = launch_partial<HD, 2, (HD == 128 ? TSV_ATTN_STAGES2_HD128 : TSV_ATTN_STAGES2_HD64)>(s, a, G, R, 1);
+        rc = launch_partial<HD, 2, (HD == 128 ? TSV_ATTN_STAGES2_HD128 : TSV_ATTN_STAGES2_HD64)>(s, a, G, R);
     else {
         // more row tiles than a wave holds: tile groups inside one workgroup, about one workgroup per compute unit
         a.xcd_groups = 0;
@@ -284,6 +279,7 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
         // (64 chunks at four KV heads would fill the chip, but what the partial pass wins the merge loses reading
         // twice the partial results: 10.9 + 6.0 us against 12.9 + 4.1 us at the Qwen3-30B-A3B shape)
         if (a.nch > 32) a.nch = 32;
+        a.by_chunks = UniformDivisor(a.nch);
         constexpr int ST = HD == 128 ? TSV_ATTN_STAGES2_HD128 : TSV_ATTN_STAGES2_HD64;
         if (HD == 64 && trt >= 7)
             rc = launch_partial_groups<HD, (HD == 64 ? 4 : 2), 2, 2>(s, a, G, R);
@@ -302,7 +298,8 @@ static int launch_hd(hipStream_t s, const AttnArgs& a0, int m, int G, int R) {
 
 template <int HD>
 static int launch_combine(hipStream_t s, const AttnArgs& a, int m, int G, int R) {
-    const dim3 cgrid(m, a.nq, std::max(a.blocks, 1)), cblock(HD < 64 ? 64 : HD);
+    static_assert(HD == 64 || HD == 128, "whole waves, one thread to a dimension");
+    const dim3 cgrid(m, a.nq, std::max(a.blocks, 1)), cblock(HD);
     // the chunk count as a compile-time constant puts every partial's load in flight before the
     // first add (a counted loop waits on each in turn); the sum runs in the same order either way
     // UNROT: the variant that rotates each head's result back (quantized KV rows); the other one is unchanged code
@@ -332,8 +329,10 @@ static int launch_combine(hipStream_t s, const AttnArgs& a, int m, int G, int R)
 }
 
 // the merge alone, over partials some other kernel left (a.nch chunks)
-int launch_attention_merge(hipStream_t s, const AttnArgs& a, int m) {
+int launch_attention_merge(hipStream_t s, const AttnArgs& a0, int m) {
+    AttnArgs a = a0;
     const int G = a.nq / a.nkv, R = m * G;
+    a.by_group = UniformDivisor(G);
     return a.hd == 128 ? launch_combine<128>(s, a, m, G, R) : launch_combine<64>(s, a, m, G, R);
 }
 

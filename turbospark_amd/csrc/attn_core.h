@@ -70,8 +70,7 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int G, int R, int
 #pragma unroll
                 for (int k = 0; k < NW; k++) o[e][i] = fmaf(grp[(k * PER_LANE + 2 * RT + (t * VT + 2 * u + e) * 4 + i) * 64], wgt[k], o[e][i]);
             }
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
+        l = sum_of_rows(l);
         if (!DIRECT) {
             if (r >= R) continue;
             const long slot = ((long)h * a.nch + chunk) * R + r;
@@ -84,7 +83,7 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int G, int R, int
             continue;
         }
         // the only chunk: what the merge would make of it (attn.hip)
-        const int m = min(r, R - 1) / G, qh = h * G + min(r, R - 1) % G;
+        const int rr = min(r, R - 1), m = a.by_group.quotient(rr), qh = h * G + rr - m * G;
         const float mx = BASE2 ? ref * 0.69314718055994530942f : ref, sink = a.sinks ? a.sinks[qh] : -INFINITY, over = fmaxf(mx, sink);
         const float w = __expf(mx - over);
         const float den = a.sinks ? fmaf(l, w, __expf(sink - over)) : l * w;
@@ -99,10 +98,16 @@ __device__ __forceinline__ void attn_finish(const AttnArgs& a, int G, int R, int
             if (r < R) *(half4*)((_Float16*)a.xfrag + frag_index(kk, m)) = half4{h0, h2, h1, h3};
             sum += ((float)h0 + (float)h1) + ((float)h2 + (float)h3);
         }
-        sum += __shfl_xor(sum, 16);
-        sum += __shfl_xor(sum, 32);
+        sum = sum_of_rows(sum);
         if (r < R && kg == 0) ((float*)((char*)a.xfrag + xfrag_sum_offset(a.nq * HD)))[xsum_index((qh * HD >> 5) + u, m)] = sum;
     }
+}
+
+// All that the attention of a chunk reads of its arguments, asked for together (uniform_memory)
+__device__ __forceinline__ void ask_for_arguments(const AttnArgs& a, int G, int R) {
+    asm volatile("" ::"s"(a.q16), "s"(a.kc), "s"(a.vc), "s"(a.part_o), "s"(a.part_ml), "s"(a.xfrag), "s"(a.nq), "s"(a.max_ctx), "s"(a.nch), "s"(a.ring),
+                 "s"(a.scale), "s"(a.window), "s"(a.sinks), "s"(a.vp), "s"(a.m_hint), "s"(a.base_hint), "s"(a.blocks), "s"(a.xcd_groups),
+                 "s"(a.by_group.magic), "s"(a.by_chunks.magic), "s"(G), "s"(R));
 }
 
 // max over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (the four position groups of one (row, q head) pair), in every
@@ -155,7 +160,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
     const int rt0 = rt_first + tg * RT;
     const int j = lane & 15, kg = lane >> 4;
     const VerifyParams* vp = a.vp;
-    const int M = a.base_hint >= 0 ? a.m_hint : vp->m, base = a.base_hint >= 0 ? a.base_hint : vp->base, kvlen = base + M;
+    const int M = a.base_hint >= 0 ? a.m_hint : uniform_memory(vp)->m, base = a.base_hint >= 0 ? a.base_hint : uniform_memory(vp)->base, kvlen = base + M;
     const int nblk = (kvlen + 15) >> 4;
     // sliding window (families/gptoss/attn.rs:120-137): a row at sequence length n sees positions
     // n - window .. n - 1.  The window exceeds the pass width, so every row keeps its whole drafted
@@ -163,7 +168,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
     // read at all, the few blocks where the rows' cuts differ are masked per row.
     const int window = a.window;
     const int bfirst = window > 0 ? max(base + 1 - window, 0) >> 4 : 0;
-    const int bpc = (nblk - bfirst + a.nch - 1) / a.nch;
+    const int bpc = a.by_chunks.quotient(nblk - bfirst + a.nch - 1);
     const int b0 = bfirst + chunk * bpc, b1 = min(b0 + bpc, nblk);
     const int cut_end = window > 0 ? base + M - window : 0;  // positions from here on are inside every row's window
     const float scale = a.scale;
@@ -180,7 +185,7 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
     for (int t = 0; t < RT; t++) {
         const int r = (rt0 + t) * 16 + j;
         const int rr = r < R ? r : 0;
-        const int mrow = rr / G, g = rr - mrow * G;
+        const int mrow = a.by_group.quotient(rr), g = rr - mrow * G;
         const uint32_t anc_row = vp->anc[mrow];
         const int pos_row = vp->pos[mrow];
         const _Float16* q = (const _Float16*)a.q16 + ((long)mrow * a.nq + h * G + g) * HD + 8 * kg;

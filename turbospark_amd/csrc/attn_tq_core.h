@@ -35,10 +35,22 @@ __device__ __forceinline__ void tq_fill_pairs(uint32_t* table, const float* cb, 
     }
 }
 
-// xch: [8 slots][PER_LANE values][64 lanes] floats of LDS; kpair / vpair: the two pair tables
-template <int HD, int RT, int STAGES, int KB, int VB>
+// ... by 512 threads, in two steps: the levels asked for, the table written
+template <int BITS>
+struct TqPairs {
+    static_assert(1 << (2 * BITS) <= 512, "an entry to a thread");
+    float lo, hi;
+    __device__ __forceinline__ TqPairs(const float* cb, int tid) : lo(cb[tid & ((1 << BITS) - 1)]), hi(cb[(tid >> BITS) & ((1 << BITS) - 1)]) {}
+    __device__ __forceinline__ void put(uint32_t* table, int tid) const {
+        if (tid < 1 << (2 * BITS))
+            table[tid] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
+    }
+};
+
+// xch: [8 slots][PER_LANE values][64 lanes] floats of LDS; kpair / vpair: the two pair tables; tables(): fills them, called once by every wave
+template <int HD, int RT, int STAGES, int KB, int VB, class Tables>
 __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, int R, int chunk, int h, int rt0, float* xch,
-                                                     const uint32_t* kpair, const uint32_t* vpair) {
+                                                     const uint32_t* kpair, const uint32_t* vpair, Tables&& tables) {
     constexpr int NW = 8;
     constexpr int KS = HD / 32;  // K steps of the score MFMA
     constexpr int VT = HD / 16;  // output tiles along head_dim
@@ -48,12 +60,12 @@ __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, i
     constexpr int VG = tq_v_group_words(VB);    // words of a V group
     constexpr int VL = VB == 3 ? 2 : 1;         // words of it a lane loads
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, kg = lane >> 4;
     const VerifyParams* vp = a.vp;
-    const int M = a.base_hint >= 0 ? a.m_hint : vp->m, base = a.base_hint >= 0 ? a.base_hint : vp->base, kvlen = base + M;
+    const int M = a.base_hint >= 0 ? a.m_hint : uniform_memory(vp)->m, base = a.base_hint >= 0 ? a.base_hint : uniform_memory(vp)->base, kvlen = base + M;
     const int nblk = (kvlen + 15) >> 4;
-    const int bpc = (nblk + a.nch - 1) / a.nch;
+    const int bpc = a.by_chunks.quotient(nblk + a.nch - 1);
     const int b0 = chunk * bpc, b1 = min(b0 + bpc, nblk);
     const float scale = a.scale;
     const uint32_t mmask = (1u << M) - 1u;  // slots that exist in this pass
@@ -66,7 +78,7 @@ __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, i
     for (int t = 0; t < RT; t++) {
         const int r = (rt0 + t) * 16 + j;
         const int rr = r < R ? r : 0;
-        const int mrow = rr / G, g = rr - mrow * G;
+        const int mrow = a.by_group.quotient(rr), g = rr - mrow * G;
         const uint32_t anc_row = vp->anc[mrow];
         const _Float16* q = (const _Float16*)a.q16 + ((long)mrow * a.nq + h * G + g) * HD + 8 * kg;
 #pragma unroll
@@ -161,8 +173,7 @@ __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, i
             for (int i4 = 0; i4 < 4; i4++)
                 sc[i4] = ((vis4 >> i4) & 1u) ? (S[i4] * __uint_as_float(knb[i4])) * scale : -INFINITY;
             float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-            mb = fmaxf(mb, __shfl_xor(mb, 16));
-            mb = fmaxf(mb, __shfl_xor(mb, 32));
+            mb = max_over_position_groups(mb);
             const float mnew = fmaxf(mrun[t], mb);
             float alpha = 1.f;
             half4 P = {0, 0, 0, 0};
@@ -193,17 +204,20 @@ __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, i
     if (nb == 1) {
         Blk st;
         fetch(st, 0);
+        tables();
         consume(st, 0);
     } else if (nb == 2) {
         Blk s0, s1;
         fetch(s0, 0);
         fetch(s1, 1);
+        tables();
         consume(s0, 0);
         consume(s1, 1);
     } else if (nb >= STAGES) {
         Blk st[STAGES];
 #pragma unroll
         for (int s = 0; s < STAGES; s++) fetch(st[s], s);
+        tables();
         int i = 0;
         for (; i + 2 * STAGES <= nb; i += STAGES) {
 #pragma unroll
@@ -223,7 +237,7 @@ __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, i
 #pragma unroll
         for (int s = 0; s < STAGES; s++)
             if (i + s < nb) consume(st[s], i + s);
-    }
+    } else tables();
 
     attn_finish<HD, RT, 8, false>(a, G, R, chunk, h, rt0, wave, lane, xch + lane, mrun, lrun, O);
 }

@@ -630,7 +630,7 @@ __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)
 // How many rows a pass has and where they begin: asked for before a matmul's K loop, through scalar loads that its end waits for.
 // (A plain load of such a value went through the vector unit, and the compiler waited for it where it stood: the first weights were asked for
 // one round trip to memory later.  With the arguments in one batch, the divisions gone and the ends' sums on the vector ALU, five rows through 32 layers of
-// the 8B shape in Q4_K, 128 launches, 2127 -> 2052 us; twelve routed layers' 37 launches 1153 -> 1131; one row through a Q4_K_M mix 1.9 %.)
+// the 8B shape in Q4_K, 128 launches, 2127 -> 2052 us; twelve routed layers 1153 -> 1131; one row through a Q4_K_M mix 1.9 %.)
 struct PassRows {
     int m, base;
     static __device__ __forceinline__ PassRows ask(const VerifyParams* vp) { return {uniform_memory(vp)->m, uniform_memory(vp)->base}; }

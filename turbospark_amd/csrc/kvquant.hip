@@ -153,13 +153,16 @@ __device__ void commit_row(const TqArgs& a, bool value, int pos, int head, int l
     const TqSide& t = value ? a.v : a.k;
     const _Float16* stage = (const _Float16*)(value ? a.vc : a.kc);
     const int slot = pos % a.stage_cap;
-    float x[EPL];
+    const TqMidpoints mid(t);  // (asked for with the row, as the signs)
+    float x[EPL], sign[EPL];
 #pragma unroll
     for (int j = 0; j < EPL; j++) {
         const int d = lane + 64 * j;
         x[j] = (float)stage[value ? v_at(a.stage_cap, HD, head, slot, d) : k_at(a.stage_cap, HD, head, slot, d)];
-        s_row[d] = x[j];
+        sign[j] = t.signs[d];
     }
+#pragma unroll
+    for (int j = 0; j < EPL; j++) s_row[lane + 64 * j] = x[j];
     if (!value && lane < t.words + 1) s_words[lane] = 0;
     lds_order();
     // every lane adds the squares in index order (the reference's sum); the row comes out of LDS sixteen
@@ -182,9 +185,8 @@ __device__ void commit_row(const TqArgs& a, bool value, int pos, int head, int l
     const float inv = 1.0f / fmaxf(norm, 1e-6f);
     float e[EPL];
 #pragma unroll
-    for (int j = 0; j < EPL; j++) e[j] = __fmul_rn(__fmul_rn(x[j], inv), t.signs[lane + 64 * j]);
+    for (int j = 0; j < EPL; j++) e[j] = __fmul_rn(__fmul_rn(x[j], inv), sign[j]);
     wht<EPL>(e, lane, a.inv_sqrt2);
-    const TqMidpoints mid(t);
     if (lane == 0) (value ? a.store.vn : a.store.kn)[(long)head * a.cap + pos] = norm;
     if (!value) {
         // a K row: packed LSB first (kv_quant.rs:289-312), assembled in LDS
@@ -225,17 +227,20 @@ template <int HD>
 __global__ __launch_bounds__(256) void k_tq_prepare(TqArgs a) {
     __shared__ __attribute__((aligned(16))) float s_row[4][HD];
     __shared__ uint32_t s_words[4][HD / 2 + 1];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m = a.m_hint, base = a.base_hint >= 0 ? a.base_hint : a.vp->base;
-    const int n_q = m * a.nq, n_rows = m * a.nkv, total = n_q + 2 * n_rows;
-    for (int u = blockIdx.x * 4 + wave; u < total; u += gridDim.x * 4) {
-        if (u < n_q) {
-            rotate_q<HD>(a, u / a.nq, u % a.nq, lane);
-        } else {
-            const bool value = u - n_q >= n_rows;
-            const int r = u - n_q - (value ? n_rows : 0);
-            commit_row<HD>(a, value, base + r / a.nkv, r % a.nkv, lane, s_row[wave], s_words[wave]);
-        }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    asm volatile("" ::"s"(a.q16), "s"(a.kc), "s"(a.vc), "s"(a.stage_cap), "s"(a.store.kq), "s"(a.store.kn), "s"(a.store.vq), "s"(a.store.vn), "s"(a.k.signs),
+                 "s"(a.k.mid), "s"(a.k.bits), "s"(a.k.words), "s"(a.v.signs), "s"(a.v.mid), "s"(a.v.bits), "s"(a.nq), "s"(a.nkv), "s"(a.cap), "s"(a.vp),
+                 "s"(a.m_hint), "s"(a.base_hint), "s"(a.inv_sqrt2), "s"(a.by_q.magic), "s"(a.by_kv.magic));
+    const int m = a.m_hint, base = a.base_hint >= 0 ? a.base_hint : uniform_memory(a.vp)->base;
+    const int n_q = m * a.nq, n_rows = m * a.nkv, u = blockIdx.x * 4 + wave;  // (the launch has a wave for every unit)
+    if (u >= n_q + 2 * n_rows) return;
+    if (u < n_q) {
+        const int b = a.by_q.quotient(u);
+        rotate_q<HD>(a, b, u - b * a.nq, lane);
+    } else {
+        const bool value = u - n_q >= n_rows;
+        const int r = u - n_q - (value ? n_rows : 0), b = a.by_kv.quotient(r);
+        commit_row<HD>(a, value, base + b, r - b * a.nkv, lane, s_row[wave], s_words[wave]);
     }
 }
 
@@ -244,6 +249,8 @@ __global__ __launch_bounds__(256) void k_tq_prepare(TqArgs a) {
 int launch_tq_prepare(hipStream_t s, const TqArgs& a0) {
     TqArgs a = a0;
     a.inv_sqrt2 = 1.0f / std::sqrt(2.0f);
+    a.by_q = UniformDivisor(std::max(1, a.nq));
+    a.by_kv = UniformDivisor(std::max(1, a.nkv));
     if ((a.hd != 64 && a.hd != 128) || a.cap % 16 || a.stage_cap % 16 || a.m_hint > a.stage_cap || a.k.bits < 2 || a.k.bits > 4 ||
         a.v.bits < 2 || a.v.bits > 4) {
         set_error("quantized KV: head_dim must be 64 or 128 and the widths 2..4 bits");

@@ -42,14 +42,23 @@ int launch_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float
 }
 
 // ---------------------------------------------------------------- residual add + RMSNorm
+// The sum over a workgroup of 1024 threads: within each wave on the vector ALU, then the sixteen waves' in order.  `red`: 16 floats that nothing
+// else uses until the next barrier.
 __device__ __forceinline__ float block_sum(float v, float* red) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    if ((threadIdx.x & 63) == 0) red[wave] = v;
+    v = sum_of_wave(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
+    float4 r[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = ((const float4*)red)[i];
     float t = 0.f;
-    for (int i = 0; i < nw; i++) t += red[i];
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        t += r[i].x;
+        t += r[i].y;
+        t += r[i].z;
+        t += r[i].w;
+    }
     return t;
 }
 
@@ -58,94 +67,101 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // matmul's fp16 activation fragments plus the sums of the rounded values over every 32-element
 // sub-block (eight neighbouring threads).  One workgroup per row, four consecutive elements per
 // thread so every load of a row is issued before the first one is waited on.
-__global__ __launch_bounds__(1024) void k_addnorm(float* __restrict__ x, const float* __restrict__ partial,
-                                                  int splits, int ldp, const float* __restrict__ w,
-                                                  float eps, int hidden, _Float16* __restrict__ xfrag,
-                                                  const float* __restrict__ weights,
-                                                  const float* __restrict__ bias, X8 x8, int x8_terms, NormBlocks nb) {
-    __shared__ float red[16];
-    const int m = blockIdx.x;
+// What bounds it is one round trip behind the other: the arguments, the row, the sum over the workgroup.  So the partial sums' count and
+// whether they are weighted are known at compile time (chosen by a branch in the kernel, nine bodies had to be jumped over, in an instruction
+// cache that the launches before have filled), the bias is asked for with the row, and the sums stay out of the LDS's permutes.
+struct AddNormArgs {
+    float* x;
+    const float* partial;
+    const float* w;
+    _Float16* xfrag;
+    const float* weights;  // WEIGHTED: [16][8] factors
+    const float* bias;     // nullable; else
+    int ldp, hidden, x8_terms;
+    float eps;
+    NormBlocks nb;
+    X8 x8;
+};
+template <int NS, bool WEIGHTED>
+__global__ __launch_bounds__(1024) void k_addnorm(AddNormArgs a) {
+    __shared__ __attribute__((aligned(16))) float red[16];
+    asm volatile("" ::"s"(a.x), "s"(a.partial), "s"(a.w), "s"(a.xfrag), "s"(a.weights), "s"(a.bias), "s"(a.ldp), "s"(a.hidden), "s"(a.x8_terms), "s"(a.eps),
+                 "s"(a.nb.x), "s"(a.nb.partial), "s"(a.nb.frag), "s"(a.nb.frag16), "s"(a.nb.frag2));
+    const int m = blockIdx.x, blk = blockIdx.y, hidden = a.hidden, n4 = hidden >> 2;
     // a prompt pass of several 16-row blocks: block blockIdx.y has its own rows, partial sums and fragments
-    x += (long)blockIdx.y * nb.x;
-    partial += (long)blockIdx.y * nb.partial;
-    xfrag = (_Float16*)((char*)xfrag + (long)blockIdx.y * nb.frag);
-    float4* xr = (float4*)(x + (long)m * hidden);
-    const float4* wr = (const float4*)w;
-    const int n4 = hidden >> 2;
-    // the norm weights of a thread's first group are asked for now: they come from HBM (nothing
-    // else reads them in a step) and would otherwise be waited for after the reduction
-    const float4 g_first = (int)threadIdx.x < n4 ? wr[threadIdx.x] : float4{0.f, 0.f, 0.f, 0.f};
-    float4 v_first = {0.f, 0.f, 0.f, 0.f};
-    float ss = 0.f;
-    // The partial sums of a group are loaded with a compile-time count (one of nine straight-line
-    // variants, chosen by a uniform branch): all loads are in flight before the first add, where a
-    // counted loop would wait for each in turn.
-    auto run = [&](auto S) {
-        constexpr int NS = decltype(S)::value;
-        for (int i = threadIdx.x; i < n4; i += 1024) {
-            float4 v = xr[i];
-            float4 p[NS > 0 ? NS : 1];
+    float4* const xr = (float4*)(a.x + (long)blk * a.nb.x + (long)m * hidden);
+    const float* const partial = a.partial + (long)blk * a.nb.partial + (long)m * a.ldp;
+    _Float16* const xfrag = (_Float16*)((char*)a.xfrag + (long)blk * a.nb.frag);
+    const float4* const wr = (const float4*)a.w;
+    float ws[NS > 0 ? NS : 1];
+    if (WEIGHTED) {  // (block b's factors follow block b - 1's)
 #pragma unroll
-            for (int s = 0; s < NS; s++) p[s] = *(const float4*)(partial + ((long)s * 16 + m) * ldp + 4 * i);
-            if (weights) {
-                // routed experts (families/llama/moe.rs:193-198): the slot outputs are weighted and summed
-                // in rank order starting from zero, then added to the stream; product and sum rounded apart
-                float4 r = {0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < NS; s++) ws[s] = uniform_memory(a.weights)[(blk * 16 + m) * 8 + s];
+    }
+    auto add = [&](int i) {
+        float4 v = xr[i];
+        float4 p[NS > 0 ? NS : 1];
 #pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    const float ws = weights[(blockIdx.y * 16 + m) * 8 + s];  // (block b's factors follow block b - 1's)
-                    r.x = __fadd_rn(r.x, __fmul_rn(ws, p[s].x));
-                    r.y = __fadd_rn(r.y, __fmul_rn(ws, p[s].y));
-                    r.z = __fadd_rn(r.z, __fmul_rn(ws, p[s].z));
-                    r.w = __fadd_rn(r.w, __fmul_rn(ws, p[s].w));
-                }
-                v.x = __fadd_rn(v.x, r.x);
-                v.y = __fadd_rn(v.y, r.y);
-                v.z = __fadd_rn(v.z, r.z);
-                v.w = __fadd_rn(v.w, r.w);
-            } else {
+        for (int s = 0; s < NS; s++) p[s] = *(const float4*)(partial + (long)s * 16 * a.ldp + 4 * i);
+        if (WEIGHTED) {
+            // routed experts (families/llama/moe.rs:193-198): the slot outputs are weighted and summed
+            // in rank order starting from zero, then added to the stream; product and sum rounded apart
+            float4 r = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    v.x = __fadd_rn(v.x, p[s].x);
-                    v.y = __fadd_rn(v.y, p[s].y);
-                    v.z = __fadd_rn(v.z, p[s].z);
-                    v.w = __fadd_rn(v.w, p[s].w);
-                }
-                if (bias) {  // the output projection's bias (families/gptoss/mod.rs:16)
-                    const float4 b = *(const float4*)(bias + 4 * i);
-                    v.x += b.x;
-                    v.y += b.y;
-                    v.z += b.z;
-                    v.w += b.w;
-                }
+            for (int s = 0; s < NS; s++) {
+                r.x = __fadd_rn(r.x, __fmul_rn(ws[s], p[s].x));
+                r.y = __fadd_rn(r.y, __fmul_rn(ws[s], p[s].y));
+                r.z = __fadd_rn(r.z, __fmul_rn(ws[s], p[s].z));
+                r.w = __fadd_rn(r.w, __fmul_rn(ws[s], p[s].w));
             }
-            xr[i] = v;
-            if (i == (int)threadIdx.x) v_first = v;
-            ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+            v.x = __fadd_rn(v.x, r.x);
+            v.y = __fadd_rn(v.y, r.y);
+            v.z = __fadd_rn(v.z, r.z);
+            v.w = __fadd_rn(v.w, r.w);
+        } else {
+            float4 b = {0.f, 0.f, 0.f, 0.f};
+            if (a.bias) b = *(const float4*)(a.bias + 4 * i);  // the output projection's (families/gptoss/mod.rs:16)
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                v.x = __fadd_rn(v.x, p[s].x);
+                v.y = __fadd_rn(v.y, p[s].y);
+                v.z = __fadd_rn(v.z, p[s].z);
+                v.w = __fadd_rn(v.w, p[s].w);
+            }
+            if (a.bias) {
+                v.x += b.x;
+                v.y += b.y;
+                v.z += b.z;
+                v.w += b.w;
+            }
         }
+        xr[i] = v;
+        return v;
     };
-    switch (splits) {
-        case 0: run(std::integral_constant<int, 0>{}); break;
-        case 1: run(std::integral_constant<int, 1>{}); break;
-        case 2: run(std::integral_constant<int, 2>{}); break;
-        case 3: run(std::integral_constant<int, 3>{}); break;
-        case 4: run(std::integral_constant<int, 4>{}); break;
-        case 5: run(std::integral_constant<int, 5>{}); break;
-        case 6: run(std::integral_constant<int, 6>{}); break;
-        case 7: run(std::integral_constant<int, 7>{}); break;
-        default: run(std::integral_constant<int, 8>{}); break;
+    auto squares = [](const float4& v) { return v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; };
+    const int mine = threadIdx.x;
+    float4 v_first = {0.f, 0.f, 0.f, 0.f}, g_first = v_first;
+    float ss = 0.f;
+    if (mine < n4) {
+        // the norm weights are asked for now: they come from HBM (nothing else reads them in a step)
+        // and would otherwise be waited for after the reduction
+        g_first = wr[mine];
+        v_first = add(mine);
+        ss += squares(v_first);
+        for (int i = mine + 1024; i < n4; i += 1024) ss += squares(add(i));
     }
     ss = block_sum(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float)hidden + eps);
+    const float inv = 1.0f / sqrtf(ss / (float)hidden + a.eps);
     float* sums = (float*)((char*)xfrag + xfrag_sum_offset(hidden));
-    for (int i = threadIdx.x; i < n4; i += 1024) {
-        const bool first = i == (int)threadIdx.x;
-        const float4 v = first ? v_first : xr[i], g = first ? g_first : wr[i];
+    auto finish = [&](int i, const float4& v, const float4& g) {
         // elements 4i..4i+3 are one K step of the fragment layout, stored in the order (0, 2, 1, 3)
         typedef _Float16 half4 __attribute__((ext_vector_type(4)));
         typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-        half4 h = {(_Float16)(v.x * g.x * inv), (_Float16)(v.z * g.z * inv), (_Float16)(v.y * g.y * inv),
-                   (_Float16)(v.w * g.w * inv)};
+        // (the products as floats first: a product converted in the instruction that makes it is rounded once, and which ones that happens to
+        // would differ from one count of partial sums to the next)
+        float e[4] = {v.x * g.x * inv, v.z * g.z * inv, v.y * g.y * inv, v.w * g.w * inv};
+        asm volatile("" : "+v"(e[0]), "+v"(e[1]), "+v"(e[2]), "+v"(e[3]));
+        half4 h = {(_Float16)e[0], (_Float16)e[1], (_Float16)e[2], (_Float16)e[3]};
         // The sums must be those of the stored bits: the matmuls multiply them by the weights' code offsets
         // (up to 1024), so one value rounded differently on the way to the sum than on the way to the store
         // is an error a thousand times its size.  The compiler is free to convert the same product twice, by
@@ -153,33 +169,36 @@ __global__ __launch_bounds__(1024) void k_addnorm(float* __restrict__ x, const f
         u32x2_t hb = __builtin_bit_cast(u32x2_t, h);
         asm volatile("" : "+v"(hb.x), "+v"(hb.y));
         h = __builtin_bit_cast(half4, hb);
-        *(half4*)(xfrag + (nb.frag16 ? frag16_index(4 * i, m) : frag_index(4 * i, m))) = h;
+        *(half4*)(xfrag + (a.nb.frag16 ? frag16_index(4 * i, m) : frag_index(4 * i, m))) = h;
         float sum = ((float)h.x + (float)h.y) + ((float)h.z + (float)h.w);
-        sum += __shfl_xor(sum, 1);
-        sum += __shfl_xor(sum, 2);
-        sum += __shfl_xor(sum, 4);
+        sum += dpp_f32<0xB1>(sum);   // over eight lanes: l ^ 1, l ^ 2, l ^ 4
+        sum += dpp_f32<0x4E>(sum);
+        sum += dpp_f32<0x141>(sum);
         if ((i & 7) == 0) sums[xsum_index(i >> 3, m)] = sum;
-        if (nb.frag2) {  // the same fragments once more, in the other of the two layouts (sums included)
-            _Float16* x2 = (_Float16*)((char*)nb.frag2 + (long)blockIdx.y * nb.frag);
-            *(half4*)(x2 + (nb.frag16 ? frag_index(4 * i, m) : frag16_index(4 * i, m))) = h;
+        if (a.nb.frag2) {  // the same fragments once more, in the other of the two layouts (sums included)
+            _Float16* x2 = (_Float16*)((char*)a.nb.frag2 + (long)blk * a.nb.frag);
+            *(half4*)(x2 + (a.nb.frag16 ? frag_index(4 * i, m) : frag16_index(4 * i, m))) = h;
             if ((i & 7) == 0) ((float*)((char*)x2 + xfrag_sum_offset(hidden)))[xsum_index(i >> 3, m)] = sum;
         }
-        if (x8_terms) {
+        if (a.x8_terms) {
             // the same row as block-scaled fp8 terms, from the unrounded values; the eight threads of a
             // 32-element block are neighbours in one wave (hidden is a multiple of 32)
             float r[4] = {v.x * g.x * inv, v.z * g.z * inv, v.y * g.y * inv, v.w * g.w * inv};
-            for (int t = 0; t < x8_terms; t++) {
+            for (int t = 0; t < a.x8_terms; t++) {
                 float amax = x8_amax4(r);
                 amax = fmaxf(amax, __shfl_xor(amax, 1));
                 amax = fmaxf(amax, __shfl_xor(amax, 2));
                 amax = fmaxf(amax, __shfl_xor(amax, 4));
                 const int byte = x8_scale_byte(amax);
                 const uint32_t word = x8_term4(r, byte);
-                *(uint32_t*)(x8.q + ((size_t)t * 16 + m) * x8.kpad + 4 * i) = word;
-                if ((i & 7) == 0) x8.s[((size_t)t * 16 + m) * (x8.kpad >> 5) + (i >> 3)] = (uint8_t)byte;
+                *(uint32_t*)(a.x8.q + ((size_t)t * 16 + m) * a.x8.kpad + 4 * i) = word;
+                if ((i & 7) == 0) a.x8.s[((size_t)t * 16 + m) * (a.x8.kpad >> 5) + (i >> 3)] = (uint8_t)byte;
             }
         }
-    }
+    };
+    if (mine >= n4) return;
+    finish(mine, v_first, g_first);
+    for (int i = mine + 1024; i < n4; i += 1024) finish(i, xr[i], wr[i]);
 }
 
 int launch_addnorm(hipStream_t s, float* x, const float* partial, int splits, int ldp, const float* w,
@@ -189,8 +208,18 @@ int launch_addnorm(hipStream_t s, float* x, const float* partial, int splits, in
         set_error("residual add: at most eight partial sums");
         return TSV_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(k_addnorm, dim3(m, blocks), dim3(1024), 0, s, x, partial, splits, ldp, w, eps, hidden,
-                       (_Float16*)xfrag, weights, bias, x8 ? *x8 : X8{}, x8 ? x8_terms : 0, nb ? *nb : NormBlocks{});
+    const AddNormArgs a{x,     partial, w,      (_Float16*)xfrag,          weights, bias, ldp,
+                        hidden, x8 ? x8_terms : 0, eps, nb ? *nb : NormBlocks{}, x8 ? *x8 : X8{}};
+    const dim3 grid(m, blocks);
+#define TSV_ADDNORM(N)                                                                               \
+    case N:                                                                                          \
+        if (weights) hipLaunchKernelGGL((k_addnorm<N, true>), grid, dim3(1024), 0, s, a);            \
+        else hipLaunchKernelGGL((k_addnorm<N, false>), grid, dim3(1024), 0, s, a);                   \
+        break;
+    switch (splits) {
+        TSV_ADDNORM(0) TSV_ADDNORM(1) TSV_ADDNORM(2) TSV_ADDNORM(3) TSV_ADDNORM(4) TSV_ADDNORM(5) TSV_ADDNORM(6) TSV_ADDNORM(7) TSV_ADDNORM(8)
+    }
+#undef TSV_ADDNORM
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }
@@ -211,7 +240,7 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
                                                     _Float16* __restrict__ xfrag, float* x_zero,
                                                     const float* __restrict__ freqs, float mscale, int half,
                                                     float2* __restrict__ cs) {
-    __shared__ float red[16];
+    __shared__ __attribute__((aligned(16))) float red[3][16];
     const int m = blockIdx.x;
     if (m >= vp->m) return;
     // The row and the norms' weights are asked for before the token is waited for, and the angles come last: one workgroup is all
@@ -244,8 +273,8 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
         se += ev[j] * ev[j];
         sh += hv[j] * hv[j];
     }
-    se = block_sum(se, red);
-    sh = block_sum(sh, red);
+    se = block_sum(se, red[0]);
+    sh = block_sum(sh, red[1]);
     const float inv_e = 1.0f / sqrtf(se / (float)hidden + eps), inv_h = 1.0f / sqrtf(sh / (float)hidden + eps);
     float st = 0.f;
 #pragma unroll
@@ -254,7 +283,7 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
         hv[j] = i < hidden ? hv[j] * gt[j] * inv_h : 0.f;
         st += hv[j] * hv[j];
     }
-    st = block_sum(st, red);
+    st = block_sum(st, red[2]);
     const float inv_t = 1.0f / sqrtf(st / (float)hidden + eps);
     float* sums = (float*)((char*)xfrag + xfrag_sum_offset(2 * hidden));
 #pragma unroll
@@ -265,11 +294,7 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
         const _Float16 hh = pinned_half((_Float16)(hv[j] * gh[j] * inv_t));
         xfrag[frag_index(i, m)] = he;
         xfrag[frag_index(hidden + i, m)] = hh;
-        float s0 = (float)he, s1 = (float)hh;
-        for (int o = 1; o < 32; o <<= 1) {
-            s0 += __shfl_xor(s0, o);
-            s1 += __shfl_xor(s1, o);
-        }
+        const float s0 = sum_of_32((float)he), s1 = sum_of_32((float)hh);
         if ((i & 31) == 0) {
             sums[xsum_index(i >> 5, m)] = s0;
             sums[xsum_index((hidden + i) >> 5, m)] = s1;
@@ -328,7 +353,9 @@ __global__ __launch_bounds__(64) void k_rope_kv(RopeKvArgs a) {
     a.qkv += (long)blockIdx.z * a.qkv_block_stride;
     a.q16 += (long)blockIdx.z * 16 * a.nq * a.hd;
     // everything the kernel needs from the parameter block is asked for at once
-    const int rows = vp->m, rot_pos = vp->pos[m], base = vp->base;
+    const int rows = uniform_memory(vp)->m, rot_pos = uniform_memory(vp)->pos[m], base = uniform_memory(vp)->base;
+    asm volatile("" ::"s"(rows), "s"(rot_pos), "s"(base), "s"(a.qkv), "s"(a.freqs), "s"(a.bias), "s"(a.q_norm), "s"(a.k_norm), "s"(a.q16), "s"(a.kc), "s"(a.vc),
+                 "s"(a.splits), "s"(a.ldq), "s"(a.mscale), "s"(a.eps), "s"(a.nq), "s"(a.nkv), "s"(a.hd), "s"(a.max_ctx), "s"(a.paired));
     if (m >= rows) return;
     const int hd = a.hd, half = hd >> 1, i = threadIdx.x;
     const int kind = head < a.nq ? 0 : head < a.nq + a.nkv ? 1 : 2;
@@ -340,6 +367,14 @@ __global__ __launch_bounds__(64) void k_rope_kv(RopeKvArgs a) {
     // their partners in its high half
     const bool paired = a.paired && kind != 2;
     const int c0 = paired ? (i >> 5) * 64 + (i & 31) : i, c1 = paired ? c0 + 32 : i + half;
+    // (the head's norm weights and the pair's frequency are asked for with the partial sums)
+    const float* nw = kind == 0 ? a.q_norm : kind == 1 ? a.k_norm : nullptr;
+    float nw0 = 0.f, nw1 = 0.f;
+    const float freq = a.freqs[min(i, half - 1)];
+    if (nw) {
+        nw0 = nw[min(i, half - 1)];
+        nw1 = nw[min(i, half - 1) + half];
+    }
     if (i < half) {
         // compile-time split count (a uniform branch picks the variant): every partial is in flight
         // before the first add
@@ -373,19 +408,17 @@ __global__ __launch_bounds__(64) void k_rope_kv(RopeKvArgs a) {
             x1 += a.bias[col + i + half];
         }
     }
-    const float* nw = kind == 0 ? a.q_norm : kind == 1 ? a.k_norm : nullptr;
     if (nw) {
-        float ss = i < half ? x0 * x0 + x1 * x1 : 0.f;
-        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        const float ss = sum_of_wave(i < half ? x0 * x0 + x1 * x1 : 0.f);
         const float inv = 1.0f / sqrtf(ss / (float)hd + a.eps);
         if (i < half) {
-            x0 = x0 * nw[i] * inv;
-            x1 = x1 * nw[i + half] * inv;
+            x0 = x0 * nw0 * inv;
+            x1 = x1 * nw1 * inv;
         }
     }
     if (i >= half) return;
     if (kind != 2) {
-        const float angle = (float)rot_pos * a.freqs[i];
+        const float angle = (float)rot_pos * freq;
         float sn, cs;
         sincosf(angle, &sn, &cs);
         sn *= a.mscale;

@@ -10,12 +10,16 @@ namespace tsv {
 template <int EPL>
 __device__ __forceinline__ void wht(float (&e)[EPL], int lane, float c) {
 #pragma unroll
-    for (int h = 1; h < 64; h <<= 1) {
-#pragma unroll
-        for (int j = 0; j < EPL; j++) {
-            const float other = __shfl_xor(e[j], h);
-            e[j] = __fmul_rn((lane & h) ? __fsub_rn(other, e[j]) : __fadd_rn(e[j], other), c);
-        }
+    for (int j = 0; j < EPL; j++) {  // the partner on the vector ALU: __shfl_xor goes through the LDS, six times one behind the other
+        auto stage = [&](float other, bool upper) { e[j] = __fmul_rn(upper ? __fsub_rn(other, e[j]) : __fadd_rn(e[j], other), c); };
+        stage(lane_xor<1>(e[j]), lane & 1);
+        stage(lane_xor<2>(e[j]), lane & 2);
+        stage(lane_xor<4>(e[j]), lane & 4);
+        stage(lane_xor<8>(e[j]), lane & 8);
+        const float2 r = lanes_by_16(e[j]);
+        stage(lane & 16 ? r.x : r.y, lane & 16);
+        const float2 h = lanes_by_32(e[j]);
+        stage(lane & 32 ? h.x : h.y, lane & 32);
     }
     if (EPL == 2) {
         const float lo = e[0], hi = e[EPL - 1];
@@ -31,7 +35,7 @@ struct TqMidpoints {
         const int n = (1 << t.bits) - 1;
 #pragma unroll
         for (int i = 0; i < 15; i++) {
-            const float v = t.mid[i];  // the table holds sixteen slots
+            const float v = uniform_memory(t.mid)[i];  // the table holds sixteen slots
             at[i] = i < n ? v : INFINITY;
         }
     }

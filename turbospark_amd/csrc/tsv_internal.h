@@ -178,6 +178,24 @@ __device__ __forceinline__ float2 lanes_by_32(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
     return float2{__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
 }
+// the value of lane l ^ H of the same row of sixteen
+template <int H>
+__device__ __forceinline__ float lane_xor(float v) {
+    static_assert(H == 1 || H == 2 || H == 4 || H == 8, "inside a row of sixteen lanes");
+    if (H == 1) return dpp_f32<0xB1>(v);
+    if (H == 2) return dpp_f32<0x4E>(v);
+    if (H == 4) return dpp_f32<0x1B>(dpp_f32<0x141>(v));  // 7 - l, then 3 - l of four
+    return dpp_f32<0x128>(v);                             // l + 8 of 16
+}
+__device__ __forceinline__ float max_of_wave(float v) {
+    const float2 h = lanes_by_32(v);
+    const float2 r = lanes_by_16(fmaxf(h.x, h.y));
+    v = fmaxf(r.x, r.y);
+    v = fmaxf(v, dpp_f32<0x128>(v));
+    v = fmaxf(v, dpp_f32<0x124>(v));
+    v = fmaxf(v, dpp_f32<0x4E>(v));
+    return fmaxf(v, dpp_f32<0xB1>(v));
+}
 // over 16 lanes in the order 1, 2, 4, 8 (lanes whose sums agree already stand in for each other: the mirrors)
 __device__ __forceinline__ float sum_of_16(float v) {
     v += dpp_f32<0xB1>(v);   // l ^ 1
@@ -189,6 +207,12 @@ __device__ __forceinline__ float sum_of_16(float v) {
 __device__ __forceinline__ float sum_of_32(float v) {
     const float2 r = lanes_by_16(sum_of_16(v));
     return r.x + r.y;
+}
+// over lanes l, l ^ 16, l ^ 32, l ^ 48, in the order 16, 32
+__device__ __forceinline__ float sum_of_rows(float v) {
+    const float2 r = lanes_by_16(v);
+    const float2 h = lanes_by_32(r.x + r.y);
+    return h.x + h.y;
 }
 // over the wave in the order 32, 16, 8, 4, 2, 1
 __device__ __forceinline__ float sum_of_wave(float v) {
@@ -478,6 +502,7 @@ struct AttnArgs {
     // set by the launcher.  Non-zero: a one-dimensional grid in which the row groups of one (chunk, kv head) pair
     // take neighbouring slots of ONE of the eight dies (attn_grid_place), this many groups per pair
     int xcd_groups;
+    UniformDivisor by_group, by_chunks, by_xcd_groups;  // set by the launcher: q heads to a kv head, nch, xcd_groups
     size_t q_stride, part_o_stride, part_ml_stride;  // elements
     size_t frag_stride;                              // bytes
 };
@@ -488,10 +513,10 @@ struct AttnArgs {
 // last pair, nothing to do.
 __device__ inline bool attn_grid_place(const AttnArgs& a, int index, int& chunk, int& kvh, int& grp) {
     const int die = index & 7, slot = index >> 3;
-    grp = slot % a.xcd_groups;
-    const int pair = (slot / a.xcd_groups) * 8 + die;
-    chunk = pair % a.nch;
-    kvh = pair / a.nch;
+    const int turn = a.by_xcd_groups.quotient(slot), pair = turn * 8 + die;
+    grp = slot - turn * a.xcd_groups;
+    kvh = a.by_chunks.quotient(pair);
+    chunk = pair - kvh * a.nch;
     return pair < a.nch * a.nkv;
 }
 inline int attn_grid_size(int pairs, int groups) { return 8 * groups * ((pairs + 7) / 8); }
@@ -528,6 +553,7 @@ struct TqArgs {
     const VerifyParams* vp;
     int m_hint, base_hint;  // rows of the pass; position of its first row (< 0: read vp->base)
     float inv_sqrt2;        // set by the launcher
+    UniformDivisor by_q, by_kv;  // set by the launcher: nq, nkv
 };
 // words of a V group: the sixteen positions' indices of one dimension, 32 bits at two bits per index, else 64
 __host__ __device__ constexpr int tq_v_group_words(int vb) { return vb == 2 ? 1 : 2; }
