@@ -215,3 +215,33 @@ def test_parity_on_unfiltered_inputs_with_the_oracles_routing_forced_onto_the_de
     gpu.force_route(None)
     print(f"{name}: {rounds} unfiltered passes under the oracle's routing, worst logit error / range {worst:.2e}; "
           f"the device's own ranking differed somewhere in {flips} of them")
+
+
+@pytest.mark.parametrize("name", ["moe_small", "gptoss_small"])
+@pytest.mark.parametrize("pattern", ["one set", "apart", "overlapping"])
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 13, 16])
+def test_rows_of_an_expert_in_units_of_four(name, pattern, m):
+    """An expert's rows are multiplied four at a time (k_route_rank lists them): every row count at an edge of four, with all rows on the same
+    experts, on experts of their own and in between.  A row's logits are those of the row by itself, by bits."""
+    import turbospark_amd as ts
+    from turbospark_amd import synth
+    cfg = dict(synth.CONFIGS[name], max_context=64)
+    gpu = ts.HipVerifier(cfg, synth.make_weights(cfg, seed=41, n_layers=cfg["n_layers"]))
+    L, E, K = cfg["n_layers"], cfg["n_experts"], cfg["top_k"]
+    step = dict(zip(["one set", "apart", "overlapping"], [0, K, max(1, K // 2)]))[pattern]
+    sel = np.full((L, 16, 8), -1, np.int32)
+    for l in range(L):
+        for r in range(16):
+            sel[l, r, :K] = (l + r * step + np.arange(K)) % E
+    feed = _prompt(m, cfg["vocab"], 90 + m)
+    gpu.prefill(_prompt(20, cfg["vocab"], 6), 0, want_logits=False)
+    point = gpu.checkpoint()
+    gpu.force_route(sel)
+    batch = gpu.verify(feed, 20)
+    assert np.array_equal(gpu.route_selected()[:, :m, :K], sel[:, :m, :K])
+    gpu.rollback(point)
+    for i, t in enumerate(feed):
+        one = np.full_like(sel, -1)
+        one[:, 0] = sel[:, i]
+        gpu.force_route(one)
+        assert np.array_equal(gpu.produce(int(t), 20 + i), batch[i]), i

@@ -65,7 +65,7 @@ __device__ __forceinline__ float key_value(uint32_t key) {
 // weights and selections.
 // `forced_first` / `forced_mine`: a.forced[m * 8] and a.forced[m * 8 + lane] (lane < k), asked for by the caller before its
 // matmul so that they are not one more memory round trip here.
-__device__ __forceinline__ void route_row(const MoeRouteArgs& a, int m, uint32_t (&key)[4], int lane, int forced_first,
+__device__ __forceinline__ int route_row(const MoeRouteArgs& a, int m, uint32_t (&key)[4], int lane, int forced_first,
                                           int forced_mine) {
     const int ne = a.n_experts, k = a.top_k;
     float top = 0.f, sum = 0.f, my_ex = 0.f;
@@ -114,23 +114,75 @@ __device__ __forceinline__ void route_row(const MoeRouteArgs& a, int m, uint32_t
         a.weights[m * 8 + lane] = my_ex / sum;
         a.selected[m * 8 + lane] = my_sel;
     }
+    return my_sel;  // lane r: slot r's expert
+}
+
+// The units of a pass (MoeUnit), by the waves that ranked its rows: wave m looks for the other pairs that chose its slots' experts (a ballot over
+// all pairs a slot), pairs that name an expert first say how many units it takes, and every pair then finds its own place.
+// `sel`, `need`: LDS, 128 entries each.
+__device__ __forceinline__ void list_units(const MoeRouteArgs& a, int m, int lane, int my_sel, int32_t* sel, int32_t* need) {
+    const int k = a.top_k, np = a.m * k;
+    if (lane < k) sel[m * k + lane] = my_sel;
+    __syncthreads();
+    const int e0 = lane < np ? sel[lane] : -1, e1 = lane + 64 < np ? sel[lane + 64] : -1;
+    auto below = [](uint64_t lo, uint64_t hi, int p) {  // how many of the bits are of pairs before p (0 .. 127)
+        const uint64_t ml = p >= 64 ? ~0ull : (1ull << p) - 1ull, mh = p >= 64 ? (1ull << (p - 64)) - 1ull : 0ull;
+        return __popcll(lo & ml) + __popcll(hi & mh);
+    };
+    int cnt = 0, rank = 0, first = 0;  // of slot `lane`
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        if (j >= k) break;
+        const int e = __builtin_amdgcn_readlane(my_sel, j);
+        const uint64_t b0 = __builtin_amdgcn_ballot_w64(e0 == e), b1 = __builtin_amdgcn_ballot_w64(e1 == e);
+        const int c = __popcll(b0) + __popcll(b1), r = below(b0, b1, m * k + j), f = b0 ? __ffsll((long long)b0) - 1 : 63 + __ffsll((long long)b1);
+        if (lane == j) {
+            cnt = min(c, TSV_MAX_ROWS);  // a row chooses an expert once: never more members than rows
+            rank = r;
+            first = f;
+        }
+    }
+    if (lane < k) need[m * k + lane] = rank == 0 ? (cnt + 3) >> 2 : 0;
+    __syncthreads();
+    const int u0 = lane < np ? need[lane] : 0, u1 = lane + 64 < np ? need[lane + 64] : 0;
+    int base = 0, total = 0;
+#pragma unroll
+    for (int j = 1; j <= 4; j++) {
+        const uint64_t b0 = __builtin_amdgcn_ballot_w64(u0 >= j), b1 = __builtin_amdgcn_ballot_w64(u1 >= j);
+        base += below(b0, b1, first);
+        total += __popcll(b0) + __popcll(b1);
+    }
+    if (m == 0 && lane == 0) *a.n_units = total;
+    if (lane >= k || rank >= cnt) return;
+    MoeUnit* const u = a.units + base + (rank >> 2);
+    const int at = rank & 3;
+    if (at == 0) {
+        u->expert = my_sel;
+        u->cnt = min(cnt - rank, 4);
+    }
+    for (int q = at; q < (rank == cnt - 1 ? 4 : at + 1); q++) {
+        u->rows[q] = m;
+        u->slots[q] = lane;
+    }
 }
 
 // The ranking of every row of a pass: one workgroup, wave m ranks row m.  The router matmul before it is the dense
 // one (split-K partial sums, a workgroup per tile and K slice): its sums are added here in split order.  The
-// groups of rows that share an expert are not built here: every expert matmul workgroup derives its own from
-// the selections (moe_derive_group), which takes a wave a few dozen instructions.
+// units of rows that share an expert are listed behind it (list_units).
 // (One launch for matmul and ranking -- a workgroup of sixteen waves per four rows walking the whole router --
 // measured 12.3 us against 4.8 + 4.2 at 128 x 2048 Q8_0 and 19.5 against 4.6 + 4.3 at 128 x 2880 bf16: a
 // workgroup's 32 or 90 tile chunks are issue-bound on its one compute unit.)
 __global__ __launch_bounds__(1024) void k_route_rank(MoeRouteArgs a) {
-    const int lane = threadIdx.x & 63, m = threadIdx.x >> 6;
-    if (m >= a.m) return;
+    __shared__ int32_t sel[TSV_MAX_ROWS * 8], need[TSV_MAX_ROWS * 8];
+    asm volatile("" ::"s"(a.logits), "s"(a.splits), "s"(a.ld), "s"(a.n_experts), "s"(a.top_k), "s"(a.m), "s"(a.weights), "s"(a.selected), "s"(a.bias),
+                 "s"(a.forced), "s"(a.blocks), "s"(a.logits_block_stride), "s"(a.units), "s"(a.n_units));
+    const int lane = threadIdx.x & 63, m = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // (m waves)
     if (a.blocks > 1) {  // a prompt pass: this workgroup's block of sixteen rows
         a.logits += (long)blockIdx.x * a.logits_block_stride;
         a.weights += blockIdx.x * 16 * 8;
         a.selected += blockIdx.x * 16 * 8;
         a.forced = nullptr;
+        a.units = nullptr;
     }
     const int ne = a.n_experts;
     // everything the row needs is asked for before the first add: the loads have no branch between them (a lane
@@ -155,25 +207,33 @@ __global__ __launch_bounds__(1024) void k_route_rank(MoeRouteArgs a) {
         if (a.bias) sum += bias[j];
         if (j < nj && lane + 64 * j < ne) key[j] = order_key(sum);
     }
-    route_row(a, m, key, lane, forced_first, forced_mine);
+    const int my_sel = route_row(a, m, key, lane, forced_first, forced_mine);
+    if (a.units) list_units(a, m, lane, my_sel, sel, need);
 }
 
 // ---- grouped expert matmul --------------------------------------------------------------------
 
-__device__ __forceinline__ float silu_moe(float x) { return x / (1.0f + __expf(-x)); }
+// silu(gate) * up, or with alpha > 0 the clamped form (moe_gguf.metal:528-556)
+__device__ __forceinline__ float gated_moe(float gate, float up, float alpha, float limit) {
+    if (alpha > 0.0f) {
+        const float x = fminf(gate, limit), y = fminf(fmaxf(up, -limit), limit);
+        return (x / (1.0f + __expf(-alpha * x))) * (y + 1.0f);
+    }
+    return silu_f(gate) * up;
+}
 
 // One 64-row weight tile of expert `e` against up to four of the group's rows (r0 .. r0 + 3).
 // STAGES: tiles in flight per wave.  Two when a wave has at most two K chunks to walk (both are then
 // requested at once); one otherwise (90-100 VGPRs instead of 150-230, so twice the resident waves,
 // which is worth more over a longer walk): the 120B-shaped step 5.86 -> 5.24 ms, the 30B-shaped one
 // 4.43 ms either way.
-// WIDE: the group is an expert's members among the 64 rows of a prompt pass (MoeGroupW): rows and members are
+// The group is an expert's members among the 64 rows of a prompt pass (MoeGroupW): rows and members are
 // addressed through their 16-row blocks, and every wave stays to the end so that the caller can go on to the
-// group's next four members.
-// NG: row groups of four walked side by side (the 64-row passes take four where an expert has many members: the
-// tile is then unpacked once per sixteen rows instead of once per four).
-template <class F, int EPI, int STAGES, bool WIDE = false, class G = MoeGroup, int NG = 1>
-__device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const G& grp, int gi, int r0, float4v* red) {
+// group's next members.
+// NG: row groups of four walked side by side (two where an expert has many members: the
+// tile is then unpacked once per eight rows instead of once per four).
+template <class F, int EPI, int STAGES, int NG = 1>
+__device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const MoeGroupW& grp, int gi, int r0, float4v* red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int tile = blockIdx.x, e = grp.expert, cnt = grp.cnt;
     const int per = (a.kchunks + nw - 1) / nw;
@@ -192,12 +252,8 @@ __device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const G& grp, 
 #pragma unroll
     for (int g = 0; g < NG; g++) {
         const int mine = min(r0 + 4 * g + (lane & 3), cnt - 1);
-        if (WIDE) {
-            if (EPI == EPI_SILU) x.set_row_blocked(g, grp.rows[mine], a.x_block_stride);
-            else x.set_row_blocked(g, mine, a.sub_stride);
-        } else {
-            x.set_row(g, EPI == EPI_SILU ? grp.rows[mine] : mine);
-        }
+        if (EPI == EPI_SILU) x.set_row_blocked(g, grp.rows[mine], a.x_block_stride);
+        else x.set_row_blocked(g, mine, a.sub_stride);
     }
 
     float4v acc[NG];
@@ -235,7 +291,7 @@ __device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const G& grp, 
 #pragma unroll
     for (int g = 0; g < NG; g++) red[(wave * NG + g) * 64 + lane] = acc[g];
     __syncthreads();
-    if (wave != 0) return;  // (WIDE: the caller's barrier is the next thing every wave meets)
+    if (wave != 0) return;  // (the caller's barrier is the next thing every wave meets)
 #pragma unroll
     for (int g = 0; g < NG; g++) {
     const int rg = r0 + 4 * g;
@@ -246,36 +302,22 @@ __device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const G& grp, 
         // lanes 0..31: gate rows, lanes 32..63: up rows of the same 32 columns of this expert
         const int col = tile * 32 + (lane & 31);
         _Float16* out = (_Float16*)((uint8_t*)a.out + (size_t)gi * a.out_stride);
-        float* sums = (float*)((uint8_t*)out + xfrag_sum_offset(a.n_out));
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const float other = __shfl_xor(v[i], 32);
-            float gate = lane < 32 ? v[i] : other, up = lane < 32 ? other : v[i];
+            const float2 gu = lanes_by_32(v[i]);
+            float gate = gu.x, up = gu.y;
             if (a.bias) {  // before the activation, where the clamp reads it too (moe_gguf.metal:585-600)
                 gate += a.bias[(size_t)e * a.n_out + col];
                 up += a.bias2[(size_t)e * a.n_out + col];
             }
-            float act;
-            if (a.alpha > 0.0f) {
-                const float x = fminf(gate, a.limit), y = fminf(fmaxf(up, -a.limit), a.limit);
-                act = (x / (1.0f + __expf(-a.alpha * x))) * (y + 1.0f);
-            } else {
-                act = silu_moe(gate) * up;
-            }
+            const float act = gated_moe(gate, up, a.alpha, a.limit);
             const _Float16 h = pinned_half((_Float16)act);
-            float sum = (float)h;
-#pragma unroll
-            for (int o = 1; o < 32; o <<= 1) sum += __shfl_xor(sum, o);
+            const float sum = sum_of_32((float)h);
             const int b = rg + i;  // the group's own row order
             if (b < cnt && lane < 32) {
-                if (WIDE) {
-                    _Float16* ow = (_Float16*)((uint8_t*)out + (size_t)(b >> 4) * a.sub_stride);
-                    ow[frag_index(col, b & 15)] = h;
-                    if (lane == 0) ((float*)((uint8_t*)ow + xfrag_sum_offset(a.n_out)))[xsum_index(col >> 5, b & 15)] = sum;
-                } else {
-                    out[frag_index(col, b)] = h;
-                    if (lane == 0) sums[xsum_index(col >> 5, b)] = sum;
-                }
+                _Float16* ow = (_Float16*)((uint8_t*)out + (size_t)(b >> 4) * a.sub_stride);
+                ow[frag_index(col, b & 15)] = h;
+                if (lane == 0) ((float*)((uint8_t*)ow + xfrag_sum_offset(a.n_out)))[xsum_index(col >> 5, b & 15)] = sum;
             }
         }
     } else {
@@ -286,8 +328,7 @@ __device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const G& grp, 
                 const int b = rg + i;
                 if (b < cnt) {
                     const int row = grp.rows[b];
-                    const size_t at = WIDE ? (size_t)(row >> 4) * a.out_block_stride + ((size_t)grp.slots[b] * 16 + (row & 15)) * a.n_out
-                                           : ((size_t)grp.slots[b] * 16 + row) * a.n_out;
+                    const size_t at = (size_t)(row >> 4) * a.out_block_stride + ((size_t)grp.slots[b] * 16 + (row & 15)) * a.n_out;
                     ((float*)a.out)[at + n] = a.bias ? v[i] + a.bias[(size_t)e * a.n_out + n] : v[i];
                 }
             }
@@ -296,20 +337,117 @@ __device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const G& grp, 
     }
 }
 
-// grid: (tiles per expert, rows x top_k groups, sweeps).  Groups that repeat an earlier expert leave
-// at once.  A workgroup multiplies its tile by four of the group's rows, 4 z .. 4 z + 3: an expert
-// chosen by more than four rows is covered by several workgroups side by side, and those past the
-// group's count leave at once.  With tiles x groups a multiple of eight the workgroups of one tile
-// run on the same XCD, so the tile comes from HBM once and from that XCD's L2 after.
+// One weight tile of a unit's expert against the unit's rows.  Grid (tiles of an expert, rounded up to a multiple of eight; as many units as there can be):
+// the workgroups of a tile run on the same XCD, so where an expert has several units its tile comes from HBM once and from that XCD's L2 after.
+// What the units are for is the start: a workgroup that worked its group out of all selections had its weights' addresses after a vector load, two
+// ballots and a trip through LDS, and every pair had workgroups, most of which found that another pair led their expert or that it had no
+// fifth or ninth row.  Nine rows through 12 layers of 128 experts, top 8, 768 x 2048 each: 1108 -> 1061 us; four layers top 4, 2880 x 2880: 810 -> 799.
 template <class F, int EPI, int STAGES>
 __global__ __launch_bounds__(512) void k_moe_gemm(MoeGemmArgs a) {
     extern __shared__ float4v red[];
-    __shared__ MoeGroup grp;
-    const int gi = blockIdx.y, r0 = 4 * blockIdx.z;
-    if (threadIdx.x < 64) moe_derive_group(&grp, a.selected, a.rows, a.top_k, gi, threadIdx.x);
+    asm volatile("" ::"s"(a.w), "s"(a.tiles_per_expert), "s"(a.kchunks), "s"(a.k), "s"(a.xfrag), "s"(a.x_stride), "s"(a.out), "s"(a.out_stride), "s"(a.n_out),
+                 "s"(a.units), "s"(a.n_units), "s"(a.waves), "s"(a.per), "s"(a.bias), "s"(a.bias2), "s"(a.alpha), "s"(a.limit));
+    const int tile = blockIdx.x, unit = blockIdx.y;
+    if (tile >= a.tiles_per_expert) return;
+    // (asked for together: a place past the last unit holds an older one)
+    const auto* const u = uniform_memory(a.units) + unit;
+    const int count = *uniform_memory(a.n_units);
+    const int e = u->expert, cnt = u->cnt, row[4] = {u->rows[0], u->rows[1], u->rows[2], u->rows[3]},
+              slot[4] = {u->slots[0], u->slots[1], u->slots[2], u->slots[3]};
+    asm volatile("" ::"s"(count), "s"(e), "s"(cnt), "s"(row[0]), "s"(row[1]), "s"(row[2]), "s"(row[3]), "s"(slot[0]), "s"(slot[1]), "s"(slot[2]), "s"(slot[3]));
+    if (unit >= count) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c0 = min(wave * a.per, a.kchunks), nc = min(a.per, a.kchunks - c0);
+    const uint8_t* wt = a.w + ((size_t)e * a.tiles_per_expert + tile) * a.kchunks * F::TILE_BYTES;
+    Consts k;
+    k.k6400 = 0x64006400u;
+    k.k5400 = 0x54005400u;
+    k.k64 = 0x64646464u;
+    asm volatile("" : "+v"(k.k6400), "+v"(k.k5400), "+v"(k.k64));
+    // activation operand: gate/up gathers the pass's rows, down reads the unit's own buffer
+    const uint8_t* xbase = (const uint8_t*)a.xfrag + (EPI == EPI_SLOT ? (size_t)unit * a.x_stride : 0);
+    ActLoader<false> x(xbase, xbase + xfrag_sum_offset(a.k), lane);
+    const int i4 = lane & 3;
+    x.set_row(0, EPI == EPI_SLOT ? min(i4, cnt - 1) : i4 < 2 ? (i4 ? row[1] : row[0]) : (i4 == 2 ? row[2] : row[3]));
+
+    float4v acc[1] = {float4v{0.f, 0.f, 0.f, 0.f}};
+    const int col = EPI == EPI_SILU ? tile * 32 + (lane & 31) : tile * 64 + lane;
+    float b0 = 0.f, b1 = 0.f;  // the end's biases, asked for behind the first weights
+    auto ask_biases = [&] {
+        if (!a.bias) return;
+        const size_t at = (size_t)e * a.n_out + min(col, a.n_out - 1);
+        b0 = a.bias[at];
+        if (EPI == EPI_SILU) b1 = a.bias2[at];
+    };
+    if (nc > 0) {
+        Stage<F, 1> st[STAGES];
+        const int last = c0 + nc - 1;
+        auto fetch = [&](Stage<F, 1>& sg, int c) { load_stage(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
+#pragma unroll
+        for (int s = 0; s < STAGES; s++) fetch(st[s], min(c0 + s, last));
+        int c = 0;
+        for (; c + 2 * STAGES <= nc; c += STAGES) {
+#pragma unroll
+            for (int s = 0; s < STAGES; s++) {
+                compute(st[s], k, acc);
+                fetch(st[s], c0 + c + s + STAGES);
+            }
+        }
+        if (wave == 0) ask_biases();
+#pragma unroll
+        for (int s = 0; s < STAGES; s++) {
+            if (c + s < nc) {
+                compute(st[s], k, acc);
+                if (c + s + STAGES < nc) fetch(st[s], c0 + c + s + STAGES);
+            }
+        }
+        c += STAGES;
+#pragma unroll
+        for (int s = 0; s < STAGES; s++)
+            if (c + s < nc) compute(st[s], k, acc);
+    }
+    // fold the waves in wave order; wave 0 (which has chunks: the first) finishes
+    if (wave != 0) red[wave * 64 + lane] = acc[0];
     __syncthreads();
-    if (r0 >= grp.cnt) return;
-    expert_tile<F, EPI, STAGES>(a, grp, gi, r0, red);
+    if (wave != 0) return;
+    float4v v = acc[0], p[7];
+#pragma unroll
+    for (int w = 1; w < 8; w++) p[w - 1] = red[(w < a.waves ? w : a.waves - 1) * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 8; w++)
+        if (w < a.waves) v += p[w - 1];
+    if (EPI == EPI_SILU) {
+        // lanes 0..31: gate rows, lanes 32..63: up rows of the same 32 columns of this expert
+        _Float16* out = (_Float16*)((uint8_t*)a.out + (size_t)unit * a.out_stride);
+        float* sums = (float*)((uint8_t*)out + xfrag_sum_offset(a.n_out));
+        _Float16 h[4];
+        float sum[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float2 gu = lanes_by_32(v[i]);
+            float gate = gu.x, up = gu.y;
+            if (a.bias) {  // before the activation, where the clamp reads it too (moe_gguf.metal:585-600)
+                gate += b0;
+                up += b1;
+            }
+            h[i] = pinned_half((_Float16)gated_moe(gate, up, a.alpha, a.limit));
+            sum[i] = sum_of_32((float)h[i]);
+        }
+        if (lane >= 32) return;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (i >= cnt) break;
+            out[frag_index(col, i)] = h[i];
+            if (lane == 0) sums[xsum_index(col >> 5, i)] = sum[i];
+        }
+        return;
+    }
+    if (col >= a.n_out) return;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if (i >= cnt) break;
+        ((float*)a.out)[((size_t)slot[i] * 16 + row[i]) * a.n_out + col] = a.bias ? v[i] + b0 : v[i];
+    }
 }
 
 // ---- the 64 rows of a prompt pass ---------------------------------------------------------------
@@ -368,13 +506,13 @@ __global__ __launch_bounds__(512) void k_moe_gemm_wide(MoeGemmArgs a) {
         // many members: eight per walk of the tile, one stage in flight (sixteen per walk costs 209 registers where this
         // costs 119-164, and the experts with few members, who share the kernel, lose their resident waves)
         for (int r0 = 8 * blockIdx.z; r0 < cnt; r0 += 8 * gridDim.z) {
-            expert_tile<F, EPI, 1, true, MoeGroupW, 2>(a, grp, e, r0, red);
+            expert_tile<F, EPI, 1, 2>(a, grp, e, r0, red);
             __syncthreads();
         }
         return;
     }
     for (int r0 = 4 * blockIdx.z; r0 < cnt; r0 += 4 * gridDim.z) {
-        expert_tile<F, EPI, STAGES, true, MoeGroupW, 1>(a, grp, e, r0, red);
+        expert_tile<F, EPI, STAGES>(a, grp, e, r0, red);
         __syncthreads();
     }
 }
@@ -408,7 +546,12 @@ int launch_moe_wide_f(hipStream_t s, int fmt, const MoeGemmArgs& a) {
 }
 
 template <class F, int EPI>
-int launch_moe_t(hipStream_t s, const MoeGemmArgs& a, int n_groups) {
+int launch_moe_t(hipStream_t s, const MoeGemmArgs& a0, int n_groups) {
+    MoeGemmArgs a = a0;
+    if (!a.units || !a.n_units) {
+        set_error("moe: the pass's units are listed first");
+        return TSV_ERR_INVALID;
+    }
     // waves per workgroup: about four, each with at least two K chunks of the tile to walk (measured on
     // the two routed configurations: 12 chunks -> 4 waves x 3, 8 chunks -> 4 x 2, 3 chunks -> 2 waves)
     static const int forced = [] {
@@ -417,8 +560,10 @@ int launch_moe_t(hipStream_t s, const MoeGemmArgs& a, int n_groups) {
     }();
     const int cpw = forced ? forced : std::max(2, (a.kchunks + 3) / 4);
     const int nw = std::min(8, std::max(1, (a.kchunks + cpw - 1) / cpw));
+    a.waves = nw;
+    a.per = (a.kchunks + nw - 1) / nw;
     const size_t lds = (size_t)nw * 1024;
-    const dim3 grid(a.tiles_per_expert, n_groups, (std::max(1, a.rows) + 3) / 4);  // no group has more members than the pass has rows
+    const dim3 grid((a.tiles_per_expert + 7) / 8 * 8, n_groups);  // (a unit has at least one pair)
     if ((a.kchunks + nw - 1) / nw <= 2)
         hipLaunchKernelGGL((k_moe_gemm<F, EPI, 2>), grid, dim3(64 * nw), lds, s, a);
     else

@@ -494,6 +494,10 @@ int launch_pass(tsv_ctx* c, int m) {
             ra2.selected = c->route_sel + (size_t)l * 16 * 8;  // kept per layer: tsv_route_selected reads them back
             ra2.bias = L.router_bias;
             ra2.forced = c->route_forced + (size_t)l * 16 * 8;
+            if (!c->moe_fp4_terms) {
+                ra2.units = c->moe_units;
+                ra2.n_units = c->moe_n_units;
+            }
             MoeGemmArgs g1{}, g2{};
             g1.w = L.gate_up.tiles;
             g1.tiles_per_expert = c->ffn / 32;
@@ -507,6 +511,8 @@ int launch_pass(tsv_ctx* c, int m) {
             g1.n_out = c->ffn;
             g1.selected = ra2.selected;
             g1.top_k = L.top_k;
+            g1.units = c->moe_units;
+            g1.n_units = c->moe_n_units;
             g1.bias = L.be_gate;
             g1.bias2 = L.be_up;
             g1.alpha = c->act_alpha;
@@ -1313,7 +1319,8 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         (rc = dev_alloc(c, &c->xf_b, xfb, true)) || (rc = dev_alloc(c, &c->xf_c, xfb, true)) ||
         (rc = dev_alloc(c, &c->partial, pneed * 4, true)) ||
         (c->max_experts &&
-         ((rc = dev_alloc(c, &c->route_w, 16 * 8 * 4, true)) || (rc = dev_alloc(c, &c->route_sel, (size_t)c->n_layers * 16 * 8 * 4, true)) ||
+         ((rc = dev_alloc(c, &c->route_w, 16 * 8 * 4, true)) || (rc = dev_alloc(c, &c->moe_units, (size_t)TSV_MAX_ROWS * 8 * sizeof(MoeUnit), true)) ||
+          (rc = dev_alloc(c, &c->moe_n_units, 64, true)) || (rc = dev_alloc(c, &c->route_sel, (size_t)c->n_layers * 16 * 8 * 4, true)) ||
           (rc = dev_alloc(c, &c->route_forced, (size_t)c->n_layers * 16 * 8 * 4)) ||
           (rc = dev_alloc(c, &c->frag_e, (size_t)TSV_MAX_ROWS * 8 * (c->frag_e_stride = (xfrag_bytes(c->ffn) + 255) & ~(size_t)255), true)) ||
           (rc = dev_alloc(c, &c->moe_out, (size_t)8 * 16 * c->hidden * 4, true)) ||

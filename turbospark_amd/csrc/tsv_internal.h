@@ -297,6 +297,14 @@ struct MoeGroup {
     int32_t expert, cnt;
     int32_t rows[16], slots[16];
 };
+// What one workgroup of a verify pass's expert matmuls multiplies a weight tile by: up to four of the rows that chose an expert (k_route_rank lists
+// them, in the order of the pairs that name an expert first; unused entries repeat the last member).  Unit u's rows are rows 0 .. cnt - 1 of
+// fragment buffer u between gate/up and down.
+struct MoeUnit {
+    int32_t expert, cnt;
+    int32_t rows[4], slots[4];
+    int32_t unused[6];  // (64 bytes: one line)
+};
 // Prompt passes of 64 rows: the members of every expert, listed once per layer (k_moe_groups) -- the rows that chose
 // it in pair order (row-major, then slot) and the slot it has in each.
 constexpr int MOE_WIDE_ROWS = 64;
@@ -320,6 +328,9 @@ struct MoeRouteArgs {
     // selections of block b follow those of block b - 1; no forced routing
     int blocks;
     long logits_block_stride;
+    // nullable: the pass's units, and behind their m * top_k places how many there are
+    MoeUnit* units;
+    int32_t* n_units;
 };
 // The group of pair gi (row gi / k, slot gi % k) from the rows' selections, by one whole wave (lane = threadIdx.x
 // < 64) into *g: the expert, the rows that chose it in pair order with the slot it has in each, and cnt != 0 only
@@ -391,6 +402,9 @@ struct MoeGemmArgs {
     int n_out;             // gate/up: expert FFN width; down: hidden
     const int32_t* selected;  // [rows][8] expert ids the rows chose (k_route_rank): the groups are derived from them
     int top_k;
+    const MoeUnit* units;     // a verify pass's units (fp16 activations)
+    const int32_t* n_units;
+    int waves, per;           // set by the launcher: waves of a workgroup, chunks of each
     // nullable per-expert biases, [n_experts][n_out]: gate/up use bias (gate) and bias2 (up), added
     // before the activation; down uses bias, added before the slot is weighted
     const float* bias;
