@@ -352,11 +352,10 @@ __global__ __launch_bounds__(64) void k_rope_kv(RopeKvArgs a) {
     const VerifyParams* vp = a.vp + blockIdx.z;
     a.qkv += (long)blockIdx.z * a.qkv_block_stride;
     a.q16 += (long)blockIdx.z * 16 * a.nq * a.hd;
-    // everything the kernel needs from the parameter block is asked for at once
-    const int rows = uniform_memory(vp)->m, rot_pos = uniform_memory(vp)->pos[m], base = uniform_memory(vp)->base;
-    asm volatile("" ::"s"(rows), "s"(rot_pos), "s"(base), "s"(a.qkv), "s"(a.freqs), "s"(a.bias), "s"(a.q_norm), "s"(a.k_norm), "s"(a.q16), "s"(a.kc), "s"(a.vc),
-                 "s"(a.splits), "s"(a.ldq), "s"(a.mscale), "s"(a.eps), "s"(a.nq), "s"(a.nkv), "s"(a.hd), "s"(a.max_ctx), "s"(a.paired));
-    if (m >= rows) return;
+    asm volatile("" ::"s"(a.qkv), "s"(a.cs), "s"(a.bias), "s"(a.q_norm), "s"(a.k_norm), "s"(a.q16), "s"(a.kc), "s"(a.vc), "s"(a.vp), "s"(a.splits), "s"(a.ldq),
+                 "s"(a.eps), "s"(a.nq), "s"(a.nkv), "s"(a.hd), "s"(a.max_ctx), "s"(a.paired), "s"(a.blocks), "s"(a.qkv_block_stride));
+    // (how many rows the pass has and where they go: waited for at the end)
+    const int rows = uniform_memory(vp)->m, base = uniform_memory(vp)->base;
     const int hd = a.hd, half = hd >> 1, i = threadIdx.x;
     const int kind = head < a.nq ? 0 : head < a.nq + a.nkv ? 1 : 2;
     const int h = kind == 0 ? head : kind == 1 ? head - a.nq : head - a.nq - a.nkv;
@@ -367,10 +366,10 @@ __global__ __launch_bounds__(64) void k_rope_kv(RopeKvArgs a) {
     // their partners in its high half
     const bool paired = a.paired && kind != 2;
     const int c0 = paired ? (i >> 5) * 64 + (i & 31) : i, c1 = paired ? c0 + 32 : i + half;
-    // (the head's norm weights and the pair's frequency are asked for with the partial sums)
+    // (the head's norm weights and the pair's rotation are asked for with the partial sums)
     const float* nw = kind == 0 ? a.q_norm : kind == 1 ? a.k_norm : nullptr;
     float nw0 = 0.f, nw1 = 0.f;
-    const float freq = a.freqs[min(i, half - 1)];
+    const float2 cs = a.cs[((long)blockIdx.z * 16 + m) * half + min(i, half - 1)];
     if (nw) {
         nw0 = nw[min(i, half - 1)];
         nw1 = nw[min(i, half - 1) + half];
@@ -416,15 +415,10 @@ __global__ __launch_bounds__(64) void k_rope_kv(RopeKvArgs a) {
             x1 = x1 * nw1 * inv;
         }
     }
-    if (i >= half) return;
+    if (i >= half || m >= rows) return;
     if (kind != 2) {
-        const float angle = (float)rot_pos * freq;
-        float sn, cs;
-        sincosf(angle, &sn, &cs);
-        sn *= a.mscale;
-        cs *= a.mscale;
-        const float r0 = x0 * cs - x1 * sn;
-        const float r1 = x0 * sn + x1 * cs;
+        const float r0 = x0 * cs.x - x1 * cs.y;
+        const float r1 = x0 * cs.y + x1 * cs.x;
         x0 = r0;
         x1 = r1;
     }

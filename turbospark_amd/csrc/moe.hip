@@ -68,48 +68,45 @@ __device__ __forceinline__ float key_value(uint32_t key) {
 __device__ __forceinline__ int route_row(const MoeRouteArgs& a, int m, uint32_t (&key)[4], int lane, int forced_first,
                                           int forced_mine) {
     const int ne = a.n_experts, k = a.top_k;
-    float top = 0.f, sum = 0.f, my_ex = 0.f;
+    float top = 0.f, my_val = 0.f;  // the largest logit; lane r: slot r's
     int my_sel = 0;
-    const bool forced = forced_first >= 0;  // the same for the whole wave
-    if (forced) {
+    if (forced_first >= 0) {  // the same for the whole wave
         // lane r < k takes slot r's expert as given and fetches that expert's logit from the lane that holds it
         const int e = min(max(lane < k ? forced_mine : 0, 0), ne - 1);
-        float l = 0.f;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const float v = __shfl(key_value(key[j]), e & 63);
-            if ((e >> 6) == j) l = v;
+            if ((e >> 6) == j) my_val = v;
         }
-        top = key_value(wave_umax(lane < k ? order_key(l) : 0u));
-        my_ex = expf(l - top);
+        top = key_value(wave_umax(lane < k ? order_key(my_val) : 0u));
         my_sel = e;
+    } else {
+        // (a loop: what runs once is fetched once, and a launch of one workgroup waits for its instructions)
+#pragma unroll 1
+        for (int r = 0; r < k; r++) {
+            const uint32_t kbest = wave_umax(max(max(key[0], key[1]), max(key[2], key[3])));
+            int bi = ne - 1;  // the lowest index that holds it: ascending j is ascending index
 #pragma unroll
-        for (int r = 0; r < 8; r++)
-            if (r < k) sum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_ex), r));
-    }
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-        if (r < k && !forced) {
-            const uint32_t mine = max(max(key[0], key[1]), max(key[2], key[3]));
-            const uint32_t kbest = wave_umax(mine);
-            uint32_t idx = 0xFFFFFFFFu;  // ascending j is ascending index: the first maximum wins
-#pragma unroll
-            for (int j = 3; j >= 0; j--)
-                if (key[j] == kbest) idx = (uint32_t)(lane + 64 * j);
-            const int bi = (int)min(wave_umin(idx), (uint32_t)(ne - 1));
-            const float best = key_value(kbest);
-            if (r == 0) top = best;
-            const float ex = expf(best - top);
-            sum += ex;  // sequential in rank order, as `exps.iter().sum()`
-            if (lane == r) {  // lane r keeps slot r
-                my_ex = ex;
+            for (int j = 3; j >= 0; j--) {
+                const uint64_t holds = __builtin_amdgcn_ballot_w64(key[j] == kbest);
+                if (holds) bi = 64 * j + __builtin_ctzll(holds);
+            }
+            bi = min(bi, ne - 1);
+            if (lane == r) {
+                my_val = key_value(kbest);
                 my_sel = bi;
             }
 #pragma unroll
             for (int j = 0; j < 4; j++)
                 if (lane + 64 * j == bi) key[j] = 0;
         }
+        top = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_val), 0));
     }
+    const float my_ex = expf(my_val - top);
+    float sum = 0.f;  // sequential in rank order, as `exps.iter().sum()`
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+        if (r < k) sum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_ex), r));
     if (lane < k) {
         a.weights[m * 8 + lane] = my_ex / sum;
         a.selected[m * 8 + lane] = my_sel;
@@ -130,9 +127,8 @@ __device__ __forceinline__ void list_units(const MoeRouteArgs& a, int m, int lan
         return __popcll(lo & ml) + __popcll(hi & mh);
     };
     int cnt = 0, rank = 0, first = 0;  // of slot `lane`
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        if (j >= k) break;
+#pragma unroll 1
+    for (int j = 0; j < k; j++) {
         const int e = __builtin_amdgcn_readlane(my_sel, j);
         const uint64_t b0 = __builtin_amdgcn_ballot_w64(e0 == e), b1 = __builtin_amdgcn_ballot_w64(e1 == e);
         const int c = __popcll(b0) + __popcll(b1), r = below(b0, b1, m * k + j), f = b0 ? __ffsll((long long)b0) - 1 : 63 + __ffsll((long long)b1);
@@ -146,7 +142,7 @@ __device__ __forceinline__ void list_units(const MoeRouteArgs& a, int m, int lan
     __syncthreads();
     const int u0 = lane < np ? need[lane] : 0, u1 = lane + 64 < np ? need[lane + 64] : 0;
     int base = 0, total = 0;
-#pragma unroll
+#pragma unroll 1
     for (int j = 1; j <= 4; j++) {
         const uint64_t b0 = __builtin_amdgcn_ballot_w64(u0 >= j), b1 = __builtin_amdgcn_ballot_w64(u1 >= j);
         base += below(b0, b1, first);
@@ -154,16 +150,17 @@ __device__ __forceinline__ void list_units(const MoeRouteArgs& a, int m, int lan
     }
     if (m == 0 && lane == 0) *a.n_units = total;
     if (lane >= k || rank >= cnt) return;
+    // (every member writes what all of them agree on; the last one the unused entries too)
     MoeUnit* const u = a.units + base + (rank >> 2);
-    const int at = rank & 3;
-    if (at == 0) {
-        u->expert = my_sel;
-        u->cnt = min(cnt - rank, 4);
-    }
-    for (int q = at; q < (rank == cnt - 1 ? 4 : at + 1); q++) {
-        u->rows[q] = m;
-        u->slots[q] = lane;
-    }
+    const int at = rank & 3, from = rank == cnt - 1 ? 3 : at;
+    u->expert = my_sel;
+    u->cnt = min(cnt - (rank & ~3), 4);
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        if (q >= at && q <= from) {
+            u->rows[q] = m;
+            u->slots[q] = lane;
+        }
 }
 
 // The ranking of every row of a pass: one workgroup, wave m ranks row m.  The router matmul before it is the dense

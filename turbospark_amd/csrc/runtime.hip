@@ -393,8 +393,7 @@ int launch_pass(tsv_ctx* c, int m) {
         ra.qkv = c->partial;
         ra.splits = sp;
         ra.ldq = qkv_n;
-        ra.freqs = c->freqs;
-        ra.mscale = c->rope_mscale;
+        ra.cs = c->rope_cs;
         ra.bias = L.bqkv;
         ra.q_norm = L.q_norm;
         ra.k_norm = L.k_norm;
@@ -721,8 +720,7 @@ int launch_wide_pass(tsv_ctx* c, int64_t base) {
             ra.paired = L.rope_fused && c->hd == 128;
             ra.splits = spq;
             ra.ldq = qkv_n;
-            ra.freqs = c->freqs;
-            ra.mscale = c->rope_mscale;
+            ra.cs = w.rope_cs + (size_t)b0 * 16 * half;
             ra.bias = L.bqkv;
             ra.q_norm = L.q_norm;
             ra.k_norm = L.k_norm;

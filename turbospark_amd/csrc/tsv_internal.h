@@ -454,8 +454,7 @@ int launch_mtp_input(hipStream_t s, const uint8_t* raw, int dtype, const VerifyP
 struct RopeKvArgs {
     const float* qkv;  // [splits][16][ldq]
     int splits, ldq;
-    const float* freqs;   // head_dim/2
-    float mscale;         // multiplies cos and sin
+    const float2* cs;     // [blocks * 16][head_dim / 2] (cos, sin) of the rows' rotation angles, scaled
     const float* bias;    // nullable: [ldq] projection biases in the fused q, k, v row order
     const float* q_norm;  // nullable, head_dim
     const float* k_norm;
