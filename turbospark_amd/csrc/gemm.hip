@@ -30,6 +30,7 @@
 //    bits whether it is verified alone or in a block.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "gemm_core.h"
 
@@ -312,17 +313,19 @@ __device__ __forceinline__ void epilogue(const GemmArgs& a, int tile, int split,
 
 // Tiles in flight per wave.  One: up to eight activation rows then fit 128 VGPRs, so four waves
 // per SIMD are resident instead of two, and inside a verify step (cold L2 and TLB at every launch)
-// that hides more latency than a second register stage does -- the 8B step went from 2.31 to
-// 2.23 ms on the same box, the 16-row tree step from 3.62 to 3.51 ms (there the kernel stays at two
-// waves per SIMD either way), although an isolated launch on warm caches times the same.
-#ifndef TSV_GEMM_STAGES
-#define TSV_GEMM_STAGES 1
-#endif
+// that hides more latency than a second register stage does -- the 8B step with two 2137 us for 2019, one row at a time 3950 for
+// 3882, nine rows through routed layers 1073 for 1044.  Two where they fit 128 VGPRs as well (108 to 118): Q8_0 with up to four rows,
+// eight 8B layers 657 and 671 -> 643 and 662 us with four, 2722 and 2783 -> 2656 and 2695 for four rows one by one.  (bf16, 86 to 112 with up to eight rows,
+// times the same both ways.)
+template <class F, int NG>
+constexpr int gemm_stages() {
+    return std::is_same<F, Q80>::value && NG == 1 ? 2 : 1;
+}
 
 // out_tile: the tile's number in the output (a matrix whose rows follow another's)
 template <class F, int EPI, int NG>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split, int out_tile, float4v* red) {
-    constexpr int STAGES = TSV_GEMM_STAGES;
+    constexpr int STAGES = gemm_stages<F, NG>();
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // this wave's run of chunks inside the workgroup's K slice
     const int s0 = split * a.kslice, s1 = min(s0 + a.kslice, a.kchunks);
