@@ -178,3 +178,39 @@ def test_adversarial_tree_rounds(vocab):
         compared += 1
     print(f"vocab {vocab}: {compared} tree rounds compared, {skipped} too close to call or refused by name")
     assert compared >= 30
+
+
+@pytest.mark.parametrize("vocab", [40, 1000, 4096])
+@pytest.mark.parametrize("penalty", [None, 1.25])
+def test_truncation_cuts_at_the_edges_of_a_group_of_rank_bins(vocab, penalty):
+    """The cuts are found in two levels, groups of 64 rank bins and the bins of one: candidates in the last bin of a group, the first of the next
+    one and the last bin but one group, five each (some of them reweighted by a penalty), and cuts that fall before, on and behind each
+    edge, by count, by mass, and by both in one group or in two."""
+    import turbospark_amd as ts
+    cfg, w, gpu, cpu = gc.build_pair("tiny_q8_0", max_context=64, vocab=vocab)
+    edge = np.array([0x4840, 0x4800, 0x47FF], np.uint16)          # 8.5, 8.0: key % 64 == 63; the value below 8.0: key % 64 == 0
+    assert [int((0xFFFF - (int(b) | 0x8000)) % 64) for b in edge] == [63, 63, 0]
+    bits = np.full(vocab, np.float16(-3.0).view(np.uint16), np.uint16)
+    at = np.random.default_rng(5).permutation(vocab)[:15]
+    bits[at] = np.repeat(edge, 5)
+    target = bits.view(np.float16)[None]
+    e = np.exp(target[0].astype(np.float64) - 8.5)
+    share = np.cumsum(np.sort(e / e.sum())[::-1])
+    history = [int(t) for t in at[::4]] if penalty else []
+    kws = [dict(top_k=k) for k in (1, 4, 5, 6, 9, 10, 11, 14, 15, 16)]
+    kws += [dict(top_p=float(0.5 * (share[i] + share[i + 1]))) for i in (0, 3, 4, 5, 8, 9, 10, 13)]
+    kws += [dict(top_k=k, top_p=float(0.5 * (share[i] + share[i + 1]))) for k, i in ((10, 4), (11, 9), (6, 8), (5, 12), (15, 2))]
+    compared = 0
+    for n, kw in enumerate(kws):
+        if penalty:
+            kw = dict(kw, repetition_penalty=penalty)
+        for seed in range(4):
+            gcfg, ocfg = ts.shaping(1.0, seed=10 * n + seed, **kw), ob.shaping(1.0, seed=10 * n + seed, **kw)
+            gpu.write_logits(target, 20)
+            res = gpu.accept([3], 20, gcfg, draft_logits=np.zeros((1, vocab), np.float16), history=history)
+            want = ob.chain_round(target.view(np.uint16), np.zeros((0, vocab), np.uint16), np.zeros(0, np.int32), ocfg, history=history)
+            if res.min_margin < 1e-9:
+                continue
+            assert (res.next, res.draw_step) == (want["next"], want["draw_step"]), (kw, seed)
+            compared += 1
+    assert compared >= 3 * len(kws)

@@ -231,7 +231,7 @@ template <bool PEN>
 __global__ __launch_bounds__(256) void k_row_max(const uint16_t* target, const uint16_t* draft, int m,
                                                  int vocab, double* scratch, int32_t* err,
                                                  unsigned long long* hist, int jobs,
-                                                 const AcceptParams* app) {
+                                                 const AcceptParams* app, unsigned long long* tmass, uint32_t* tcount) {
     __shared__ double red[4];
     const int row = blockIdx.y, seg = blockIdx.x;
     {
@@ -243,6 +243,11 @@ __global__ __launch_bounds__(256) void k_row_max(const uint16_t* target, const u
         };
         clear(hist, jobs * 2 * 65536);
         clear(rank_groups(hist), jobs * 2 * RANK_GROUPS);
+        // and so do the row's truncation histograms, where there will be a cut
+        if (tmass) {
+            const int i = seg * 256 + threadIdx.x;
+            if (i < TRUNC_WORDS) tmass[row * TRUNC_WORDS + i] = 0, tcount[row * TRUNC_WORDS + i] = 0;
+        }
     }
     const uint16_t* p = row_ptr(target, draft, m, vocab, row);
     const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
@@ -573,52 +578,149 @@ __device__ __forceinline__ void scan_chunk(const uint16_t* lp, int v0, int v1, u
 // by ascending index; top-k keeps the first k, top-p the shortest prefix whose cumulative
 // `e / sum` reaches top_p, min-p those with e >= min_p * e_top.  All three keep a PREFIX of the
 // rank order, so the surviving set is described by its last member (rank bin, index); it is found
-// from per-row histograms over the 65536 rank bins (candidates per bin, fixed-point mass per
-// bin) instead of a sort, and the one bin the cut falls into is resolved in index order.
-__global__ __launch_bounds__(256) void k_trunc_clear(unsigned long long* tmass, uint32_t* tcount, int rows) {
-    const size_t n = (size_t)rows * 65536;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        tmass[i] = 0;
-        tcount[i] = 0;
-    }
-}
+// from per-row histograms (candidates, fixed-point mass) instead of a sort, and the one bin the cut falls into is resolved in index
+// order.  The histograms have two levels: every group of 64 consecutive rank bins, then the bins of the groups that hold
+// a cut.  A group's sums come together in LDS, and few entries fall into the second level, where a histogram of all 65536 bins was
+// two atomics on memory for every entry, and 5 MB to clear and to read again (seven rows of 128 256 entries: cleared, filled and cut in 5.3 + 52.5 +
+// 45.5 us; a penalised round of four rows with top-k and top-p 892 -> 838).  The sums are of integers: their order does not matter.
+__device__ __forceinline__ unsigned long long mass_of(float w, double mx, double sum) { return (unsigned long long)((exp((double)w - mx) / sum) * FIX); }
 
 template <bool PEN>
-__global__ __launch_bounds__(256) void k_trunc_hist(const uint16_t* target, const uint16_t* draft, int m, int vocab,
-                                                    double* scratch, unsigned long long* tmass, uint32_t* tcount,
-                                                    int want_mass, const AcceptParams* app) {
+__global__ __launch_bounds__(256) void k_trunc_groups(const uint16_t* target, const uint16_t* draft, int m, int vocab,
+                                                      double* scratch, unsigned long long* tmass, uint32_t* tcount,
+                                                      int want_mass, const AcceptParams* app) {
+    __shared__ unsigned long long mass_sum[RANK_GROUPS];
+    __shared__ uint32_t count[RANK_GROUPS];
     const int row = blockIdx.y, seg = blockIdx.x, lane = threadIdx.x & 63;
     Layout L = layout(scratch);
     const double mx = wave_max_f64(L.pmax[row * NSEG + lane]);
     const double sum = fold_row(L.psum, row);
     const uint16_t* p = row_ptr(target, draft, m, vocab, row);
     const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
-    unsigned long long* hm = tmass + (size_t)row * 65536;
-    uint32_t* hc = tcount + (size_t)row * 65536;
+    for (int i = threadIdx.x; i < RANK_GROUPS; i += 256) mass_sum[i] = 0, count[i] = 0;
+    __syncthreads();
     for (int v = v0 + threadIdx.x; v < v1; v += 256) {
         const uint16_t b = p[v];
-        float w;
-        if constexpr (PEN)
-            w = score_of<true>(*app, row, v, b);
-        else
-            w = h2f(b);
-        const uint32_t key = bin_addr(key_of<PEN>(w, b));
-        unsigned long long mass = 0;
-        if (want_mass) mass = (unsigned long long)((exp((double)w - mx) / sum) * FIX);
+        const float w = score_of<PEN>(*app, row, v, b);
+        const uint32_t key = key_of<PEN>(w, b), group = key >> 6;
+        const unsigned long long mass = want_mass ? mass_of(w, mx, sum) : 0;
         // a run of equal logits (a flat row) would serialise on one address: one lane adds for all
         const uint32_t first = __builtin_amdgcn_readfirstlane(key);
         const unsigned long long active = __ballot(1);
         if (!PEN && __ballot(key == first) == active) {  // (equal keys are equal masses only without penalties)
             if (lane == (int)__builtin_ctzll(active)) {
                 const int n = __builtin_popcountll(active);
-                atomicAdd(hc + key, (uint32_t)n);
-                if (want_mass) atomicAdd(hm + key, mass * (unsigned long long)n);
+                atomicAdd(count + group, (uint32_t)n);
+                if (want_mass) atomicAdd(mass_sum + group, mass * (unsigned long long)n);
             }
         } else {
-            atomicAdd(hc + key, 1u);
-            if (want_mass && mass) atomicAdd(hm + key, mass);
+            atomicAdd(count + group, 1u);
+            if (want_mass && mass) atomicAdd(mass_sum + group, mass);
         }
     }
+    __syncthreads();
+    for (int i = threadIdx.x; i < RANK_GROUPS; i += 256) {
+        if (count[i]) atomicAdd(tcount + (size_t)row * TRUNC_WORDS + i, count[i]);
+        if (mass_sum[i]) atomicAdd(tmass + (size_t)row * TRUNC_WORDS + i, mass_sum[i]);
+    }
+}
+
+// Exclusive prefix of a 64-bit value over the 64 NW threads of a workgroup; *total gets the sum.
+template <int NW>
+__device__ unsigned long long block_scan_u64(unsigned long long loc, unsigned long long* wsum,
+                                             unsigned long long* total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long inc = loc;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t lo = __shfl_up((uint32_t)inc, o), hi = __shfl_up((uint32_t)(inc >> 32), o);
+        const unsigned long long up = ((unsigned long long)hi << 32) | lo;
+        if (lane >= o) inc += up;
+    }
+    __syncthreads();
+    if (lane == 63) wsum[wave] = inc;
+    __syncthreads();
+    unsigned long long wbase = 0, t = 0;
+    for (int i = 0; i < NW; i++) {
+        if (i < wave) wbase += wsum[i];
+        t += wsum[i];
+    }
+    *total = t;
+    return wbase + inc - loc;
+}
+
+// The group in which a running sum over the groups reaches `target` (sum before < target <= sum with it), found by 64 NW threads; -1 where the sums
+// end below it.  Thread t brings the sums of groups t * PER ..; *before: the sum before the group, *all: over every group.
+// `wsum`, `found`, `at`: LDS.
+template <int NW, int PER>
+__device__ __forceinline__ int group_reaching(const unsigned long long (&v)[PER], unsigned long long target, unsigned long long* wsum, int* found,
+                                              unsigned long long* at, unsigned long long* before, unsigned long long* all) {
+    unsigned long long loc = 0;
+#pragma unroll
+    for (int i = 0; i < PER; i++) loc += v[i];
+    if (threadIdx.x == 0) *found = -1;
+    unsigned long long c = block_scan_u64<NW>(loc, wsum, all);
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        if (c < target && target <= c + v[i]) {
+            *found = threadIdx.x * PER + i;
+            *at = c;
+        }
+        c += v[i];
+    }
+    __syncthreads();
+    *before = *at;
+    return *found;
+}
+
+// The second level: candidates and mass of the bins of the groups that hold the cuts, which every workgroup looks for again.
+template <bool PEN>
+__global__ __launch_bounds__(256) void k_trunc_bins(const uint16_t* target, const uint16_t* draft, int m, int vocab, double* scratch,
+                                                    unsigned long long* tmass, uint32_t* tcount, const AcceptParams* app) {
+    __shared__ unsigned long long wsum[4], at, mass_sum[64];
+    __shared__ uint32_t count[2][64];
+    __shared__ int found;
+    const AcceptParams& ap = *app;
+    const int row = blockIdx.y, seg = blockIdx.x, lane = threadIdx.x & 63, tid = threadIdx.x;
+    Layout L = layout(scratch);
+    unsigned long long* const gm = tmass + (size_t)row * TRUNC_WORDS;
+    uint32_t* const gc = tcount + (size_t)row * TRUNC_WORDS;
+    const double mx = wave_max_f64(L.pmax[row * NSEG + lane]);
+    const double sum = fold_row(L.psum, row);
+    if (tid < 64) mass_sum[tid] = 0, count[0][tid] = count[1][tid] = 0;
+    static_assert(RANK_GROUPS == 4 * 256, "four groups to a thread");
+    unsigned long long v[4], before, all;
+    int group_k = -1, group_p = -1;
+    if (ap.top_k > 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = gc[4 * tid + i];
+        group_k = group_reaching<4, 4>(v, (unsigned long long)ap.top_k, wsum, &found, &at, &before, &all);
+        __syncthreads();
+    }
+    if (ap.has_top_p) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = gm[4 * tid + i];
+        group_p = group_reaching<4, 4>(v, (unsigned long long)(ap.top_p * FIX), wsum, &found, &at, &before, &all);
+    }
+    if (group_k < 0 && group_p < 0) return;
+    __syncthreads();
+    const uint16_t* p = row_ptr(target, draft, m, vocab, row);
+    const int per = (vocab + NSEG - 1) / NSEG, v0 = seg * per, v1 = min(v0 + per, vocab);
+    for (int i = v0 + tid; i < v1; i += 256) {
+        const uint16_t b = p[i];
+        const float w = score_of<PEN>(ap, row, i, b);
+        const uint32_t key = key_of<PEN>(w, b);
+        const int group = (int)(key >> 6), bin = (int)(key & 63u);
+        if (group == group_k) atomicAdd(&count[0][bin], 1u);
+        if (group == group_p) {
+            atomicAdd(&count[1][bin], 1u);
+            atomicAdd(&mass_sum[bin], mass_of(w, mx, sum));
+        }
+    }
+    __syncthreads();
+    if (tid >= 64) return;
+    if (count[0][tid]) atomicAdd(gc + RANK_GROUPS + tid, count[0][tid]);
+    if (count[1][tid]) atomicAdd(gc + RANK_GROUPS + 64 + tid, count[1][tid]);
+    if (mass_sum[tid]) atomicAdd(gm + RANK_GROUPS + 64 + tid, mass_sum[tid]);
 }
 
 // fp16 bits whose rank key is `key` (inverse of rank_key; the zero bin maps to +0)
@@ -647,7 +749,7 @@ __device__ __forceinline__ void on_path_tokens(const AcceptParams& ap, int row, 
 // then walks the bits of its own contiguous chunk of `groups` bytes, in the index order the sums are defined in.
 // Penalised: an entry that no penalty touches is found by its fp16 bits like any other; the few touched ones are noted in
 // registers and scored afterwards, each lane its own (scoring inside the sweep would have every wave do it for every group).
-// 128 256 entries, 2000 tokens of history: k_pick 192 -> 43 us; k_trunc_cut, seven rows, 281 -> 46 us (with sum_bins): they read
+// 128 256 entries, 2000 tokens of history: k_pick 192 -> 43 us; k_trunc_cut, seven rows, 281 -> 46 us: they read
 // entry by entry and walked the root path for each.
 constexpr int PICK_MASK_GROUPS = 32;  // groups of eight entries per thread the match mask holds: vocabularies to 262 144
 __device__ __forceinline__ int mask_groups(int vocab) { return ((vocab + 1023) / 1024 + 7) >> 3; }
@@ -815,67 +917,23 @@ __device__ __forceinline__ int collect_side(const AcceptParams& ap, int row, con
     return n;
 }
 
-// Exclusive prefix of a 64-bit value over the 1024 threads of a workgroup; *total gets the sum.
-__device__ unsigned long long block_scan_u64(unsigned long long loc, unsigned long long* wsum,
-                                             unsigned long long* total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned long long inc = loc;
+// The bin of a group, by one whole wave: the first of its 64 bins at which the running sum from `c` on reaches `target`, in every lane (-1: none); *before: the
+// sum before it.
+__device__ __forceinline__ int bin_reaching(unsigned long long v, unsigned long long c, unsigned long long target, unsigned long long* before) {
+    const int lane = threadIdx.x & 63;
+    unsigned long long inc = v;
     for (int o = 1; o < 64; o <<= 1) {
         const uint32_t lo = __shfl_up((uint32_t)inc, o), hi = __shfl_up((uint32_t)(inc >> 32), o);
         const unsigned long long up = ((unsigned long long)hi << 32) | lo;
         if (lane >= o) inc += up;
     }
-    __syncthreads();
-    if (lane == 63) wsum[wave] = inc;
-    __syncthreads();
-    unsigned long long wbase = 0, t = 0;
-    for (int i = 0; i < 16; i++) {
-        if (i < wave) wbase += wsum[i];
-        t += wsum[i];
-    }
-    *total = t;
-    return wbase + inc - loc;
-}
-
-// The 64 rank bins of one thread (64 words apart, see bin_addr): their sum, in four runs of sixteen, and the first bin at which
-// the running sum from *c on reaches `target` (c < target <= c + sum); *c becomes the sum before it.  Only the run that holds it
-// is fetched again, all of it at once: a loop that stops at the hit waits out one memory round trip per bin.
-template <class T>
-__device__ __forceinline__ unsigned long long sum_bins(const T* mine, unsigned long long (&quarter)[4]) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        T v[16];
-#pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = mine[(q * 16 + i) * 64];
-        quarter[q] = 0;
-#pragma unroll
-        for (int i = 0; i < 16; i++) quarter[q] += v[i];
-    }
-    return quarter[0] + quarter[1] + quarter[2] + quarter[3];
-}
-template <class T>
-__device__ __forceinline__ int bin_reaching(const T* mine, const unsigned long long (&quarter)[4], unsigned long long target, unsigned long long* c) {
-    int b = 0;
-#pragma unroll
-    for (int q = 0; q < 3; q++)
-        if (b == q && *c + quarter[q] < target) {
-            *c += quarter[q];
-            b = q + 1;
-        }
-    T v[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) v[i] = mine[(b * 16 + i) * 64];
-    unsigned long long at = *c;
-    int hit = -1;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        if (hit < 0 && target <= at + v[i]) {
-            hit = b * 16 + i;
-            *c = at;
-        }
-        at += v[i];
-    }
-    return hit;
+    const unsigned long long excl = c + inc - v;
+    const unsigned long long hit = __ballot(excl < target && target <= excl + v);
+    if (!hit) return -1;
+    const int at = __builtin_ctzll(hit);
+    const uint32_t lo = __shfl((uint32_t)excl, at), hi = __shfl((uint32_t)(excl >> 32), at);
+    *before = ((unsigned long long)hi << 32) | lo;
+    return at;
 }
 
 // One workgroup per distribution row.
@@ -888,8 +946,8 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
     __shared__ uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // build_mask
     __shared__ int s_nside;
     __shared__ unsigned long long wsum[16];
-    __shared__ unsigned long long s_before_p;
-    __shared__ int s_bin_k, s_j_k, s_bin_p, s_cnt_p, s_minp_key, s_bin, s_j, s_idx;
+    __shared__ unsigned long long s_before_p, s_at;
+    __shared__ int s_bin_k, s_j_k, s_bin_p, s_cnt_p, s_minp_key, s_bin, s_j, s_idx, s_found, s_held_k, s_held_p;
     __shared__ double s_margin;
     const AcceptParams& ap = *app;
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
@@ -897,39 +955,44 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
     Layout L = layout(scratch);
     const double mx = wave_max_f64(L.pmax[row * NSEG + lane]);
     const double sum = fold_row(L.psum, row);
-    const uint32_t* cmine = tcount + (size_t)row * 65536 + (tid >> 6) * 4096 + (tid & 63);
-    const unsigned long long* mmine = tmass + (size_t)row * 65536 + (tid >> 6) * 4096 + (tid & 63);
+    const uint32_t* const gc = tcount + (size_t)row * TRUNC_WORDS;
+    const unsigned long long* const gm = tmass + (size_t)row * TRUNC_WORDS;
+    static_assert(RANK_GROUPS == 1024, "a group to a thread");
     if (tid == 0) {
         s_bin_k = s_bin_p = s_minp_key = s_bin = -1;
         s_idx = 0x7FFFFFFF;
         s_margin = 1.0;
     }
     __syncthreads();
-    unsigned long long total, total_p = 0;
+    unsigned long long total, total_p = 0, before;
     if (ap.top_k > 0) {
-        unsigned long long quarter[4];
-        const unsigned long long loc = sum_bins(cmine, quarter);
-        const unsigned long long excl = block_scan_u64(loc, wsum, &total);
-        const unsigned long long K = (unsigned long long)ap.top_k;
-        if (excl < K && K <= excl + loc) {
-            unsigned long long c = excl;
-            const int i = bin_reaching(cmine, quarter, K, &c);
-            s_bin_k = tid * 64 + i;
-            s_j_k = (int)(K - c);
+        const unsigned long long mine[1] = {gc[tid]}, K = (unsigned long long)ap.top_k;
+        const int group = group_reaching<16, 1>(mine, K, wsum, &s_found, &s_at, &before, &total);
+        if (group >= 0 && tid < 64) {
+            const uint32_t held = gc[RANK_GROUPS + lane];
+            unsigned long long c = 0;
+            const int i = bin_reaching(held, before, K, &c);
+            if (lane == i) {
+                s_bin_k = group * 64 + i;
+                s_j_k = (int)(K - c);
+                s_held_k = (int)held;
+            }
         }
+        __syncthreads();
     }
     if (ap.has_top_p) {
-        unsigned long long quarter[4];
-        const unsigned long long loc = sum_bins(mmine, quarter);
-        const unsigned long long excl = block_scan_u64(loc, wsum, &total);
+        const unsigned long long mine[1] = {gm[tid]}, tgt = (unsigned long long)(ap.top_p * FIX);
+        const int group = group_reaching<16, 1>(mine, tgt, wsum, &s_found, &s_at, &before, &total);
         total_p = total;
-        const unsigned long long tgt = (unsigned long long)(ap.top_p * FIX);
-        if (excl < tgt && tgt <= excl + loc) {
-            unsigned long long c = excl;
-            const int i = bin_reaching(mmine, quarter, tgt, &c);
-            s_bin_p = tid * 64 + i;
-            s_before_p = c;
-            s_cnt_p = (int)cmine[i * 64];
+        if (group >= 0 && tid < 64) {
+            const int held = (int)gc[RANK_GROUPS + 64 + lane];
+            unsigned long long c = 0;
+            const int i = bin_reaching(gm[RANK_GROUPS + 64 + lane], before, tgt, &c);
+            if (lane == i) {
+                s_bin_p = group * 64 + i;
+                s_before_p = c;
+                s_cnt_p = s_held_p = held;
+            }
         }
     }
     if (!PEN && ap.has_min_p) {  // (penalised rounds test e >= min_p per candidate instead)
@@ -1002,7 +1065,7 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
     const int bin = s_bin;
     int j = s_j;
     float cut_w = bin >= 0 ? h2f((uint16_t)key_bits(bin)) : 0.f;
-    if (bin >= 0 && j < (int)tcount[(size_t)row * 65536 + bin_addr(bin)]) {
+    if (bin >= 0 && j < (bin == s_bin_k ? s_held_k : s_held_p)) {
         bool on_value = true;
         if constexpr (PEN) {
             // the bin's candidates above its own value come first in rank order
@@ -1026,7 +1089,7 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
             };
             int n = 0;
             for_matches([&](int) { n++; });
-            const unsigned long long excl = block_scan_u64((unsigned long long)n, wsum, &total);
+            const unsigned long long excl = block_scan_u64<16>((unsigned long long)n, wsum, &total);
             if ((int)excl < j && j <= (int)excl + n) {
                 int c = (int)excl;
                 for_matches([&](int v) {
@@ -1624,9 +1687,9 @@ static void launch_trunc(hipStream_t s, const uint16_t* target, const uint16_t* 
     }
     unsigned long long* tm = (unsigned long long*)sc.tmass;
     if (ap.top_k != 0 || ap.has_top_p) {
-        hipLaunchKernelGGL(k_trunc_clear, dim3(64 * rows), dim3(256), 0, s, tm, sc.tcount, rows);
-        hipLaunchKernelGGL(k_trunc_hist<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, tm,
+        hipLaunchKernelGGL(k_trunc_groups<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, tm,
                            sc.tcount, ap.has_top_p, ap_dev);
+        hipLaunchKernelGGL(k_trunc_bins<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, tm, sc.tcount, ap_dev);
     }
     hipLaunchKernelGGL(k_trunc_cut<PEN>, dim3(rows), dim3(1024), 0, s, target, draft, ap_dev, m, sc.stats, tm, sc.tcount,
                        sc.result, &sc.result->flag);
@@ -1643,7 +1706,7 @@ static void launch_stats(hipStream_t s, const uint16_t* target, const uint16_t* 
     int32_t* err = &sc.result->flag;
     const double inv_t = 1.0 / ap.temperature;
     hipLaunchKernelGGL(k_row_max<PEN>, dim3(NSEG, rows), dim3(256), 0, s, target, draft, m, ap.vocab, sc.stats, err,
-                       (unsigned long long*)sc.hist, jobs, ap_dev);
+                       (unsigned long long*)sc.hist, jobs, ap_dev, ap.top_k != 0 || ap.has_top_p ? (unsigned long long*)sc.tmass : nullptr, sc.tcount);
     const dim3 grid(NSEG, rows, rows <= SPLIT_ROWS ? 4 : 1), block(256);
     if (grid.z > 1) hipLaunchKernelGGL((k_row_sum<PEN, true>), grid, block, 0, s, target, draft, m, ap.vocab, sc.stats, ap_dev);
     else hipLaunchKernelGGL((k_row_sum<PEN, false>), grid, block, 0, s, target, draft, m, ap.vocab, sc.stats, ap_dev);

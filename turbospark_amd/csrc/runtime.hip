@@ -1339,8 +1339,8 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         (rc = dev_alloc(c, &c->sc.work, (size_t)accept_work_rows() * c->vocab * 8, true)) ||
         (rc = dev_alloc(c, &c->sc.hist, accept_hist_words() * 8, true)) ||
         (rc = dev_alloc(c, &c->sc.counters, ACCEPT_COUNTER_WORDS * 4, true)) ||
-        (rc = dev_alloc(c, &c->sc.tmass, (size_t)32 * 65536 * 8, true)) ||
-        (rc = dev_alloc(c, &c->sc.tcount, (size_t)32 * 65536 * 4, true)))
+        (rc = dev_alloc(c, &c->sc.tmass, (size_t)32 * TRUNC_WORDS * 8, true)) ||
+        (rc = dev_alloc(c, &c->sc.tcount, (size_t)32 * TRUNC_WORDS * 4, true)))
         return fail(rc);
     c->sc.result = &c->up_dev->res;
     if (c->route_forced && hipMemsetAsync(c->route_forced, 0xFF, (size_t)c->n_layers * 16 * 8 * 4, c->stream) != hipSuccess)

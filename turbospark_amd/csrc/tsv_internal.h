@@ -635,14 +635,17 @@ struct AcceptUpload {
         res.min_margin = 1.0;
     }
 };
+constexpr int TRUNC_WORDS = 65536 / 64 + 2 * 64;
 struct AcceptScratch {
     double* stats;       // accept_stats_doubles() doubles: row statistics, partials, decisions
     double* work;        // accept_work_rows() rows of vocab: a draw's candidate masses (p, residual), the distributions' reweighted
                          // values, a tree's residuals
     uint64_t* hist;      // accept_hist_words(): fixed-point mass per rank bin and per 64 of them; a round clears what it uses first
     uint32_t* counters;  // ACCEPT_COUNTER_WORDS words: error flag, tree path, greedy arg-max partials
-    uint64_t* tmass;     // [32 rows][65536] fixed-point softmax mass per rank bin (top-p cut)
-    uint32_t* tcount;    // [32 rows][65536] candidates per rank bin (top-k / top-p cut)
+    // truncation cuts, [32 rows][TRUNC_WORDS]: fixed-point softmax mass and candidates per group of 64 rank bins, then per bin of the group
+    // that holds the top-k cut and of the one that holds the top-p cut
+    uint64_t* tmass;
+    uint32_t* tcount;
     AcceptResult* result;  // device; the caller uploads it cleared with a round's parameters
 };
 constexpr int ACCEPT_COUNTER_WORDS = 1024;
