@@ -199,6 +199,8 @@ struct PromptAttnArgs {
     uint8_t *a, *asum;      // the output projection's activations (K index = head * hd + d) and sums
     float *part_o, *part_ml;  // nch > 1: [nch][nkv][n * G][hd] and [nch][nkv][n * G][2]
     int nch;
+    int group;                      // set by the launcher: q heads to a kv head, and its and n's reciprocals
+    UniformDivisor by_n, by_group;
 };
 int prompt_attn_chunks(int n, int base, int nq, int nkv, int window);
 int launch_prompt_attention(hipStream_t s, const PromptAttnArgs& a);

@@ -214,16 +214,20 @@ __device__ __forceinline__ float sum_of_rows(float v) {
     const float2 h = lanes_by_32(r.x + r.y);
     return h.x + h.y;
 }
-// over the wave in the order 32, 16, 8, 4, 2, 1
-__device__ __forceinline__ float sum_of_wave(float v) {
-    const float2 h = lanes_by_32(v);
-    const float2 r = lanes_by_16(h.x + h.y);
+// over 32 lanes in the order 16, 8, 4, 2, 1 (where the other order's bits are not the ones wanted)
+__device__ __forceinline__ float sum_of_32_down(float v) {
+    const float2 r = lanes_by_16(v);
     v = r.x + r.y;
     v += dpp_f32<0x128>(v);  // l + 8 of 16
     v += dpp_f32<0x124>(v);  // l + 4: the two eights agree
     v += dpp_f32<0x4E>(v);
     v += dpp_f32<0xB1>(v);
     return v;
+}
+// over the wave in the order 32, 16, 8, 4, 2, 1
+__device__ __forceinline__ float sum_of_wave(float v) {
+    const float2 h = lanes_by_32(v);
+    return sum_of_32_down(h.x + h.y);
 }
 
 // n / d in one scalar multiplication (a division of scalars goes through the vector unit and its float reciprocal, some forty dependent
