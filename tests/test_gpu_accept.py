@@ -478,3 +478,32 @@ def test_a_refused_call_leaves_no_copy_of_the_caller_s_rows_under_way():
     gpu.accept(feed, 0, ts.shaping(0.8, seed=1), draft_logits=draft)      # and takes the same rows when they are right
     del draft
     hip.check(hip.rt().hipHostFree(pinned), "free")
+
+
+@pytest.mark.parametrize("kw,temperature,rows", [({}, 0.0, 1), ({}, 0.0, 16), ({}, 0.8, 5), (dict(top_k=40, top_p=0.9), 0.7, 4),
+                                                 (dict(repetition_penalty=1.3, frequency_penalty=0.1), 1.0, 6), ({}, 1.0, 16)])
+def test_a_round_in_one_call_is_the_pass_and_the_acceptance_apart(kw, temperature, rows):
+    """In one call the acceptance's parameters go to the device with the pass's; the results are those of the two calls, round after round (what a
+    round leaves behind does not reach the next), and a round that the acceptance refuses is refused as it is apart, the pass done."""
+    import turbospark_amd as ts
+    cfg, gpu, prompt = _setup()
+    V, base = cfg["vocab"], len(prompt)
+    rng = np.random.default_rng(31)
+    point = gpu.checkpoint()
+    history = [int(t) for t in prompt]
+    for rnd in range(4):
+        feed = rng.integers(0, V, rows).astype(np.int32)
+        draft = rng.standard_normal((max(rows - 1, 1), V)).astype(np.float16)
+        shaping = ts.shaping(temperature, seed=rnd, **(kw if temperature else {}))
+        more = dict(draft_logits=draft if temperature else None, history=history)
+        one = gpu.verify_accept(feed, base, shaping, **more)
+        gpu.rollback(point)
+        gpu.verify(feed, base, want_logits=False)
+        two = gpu.accept(feed, base, shaping, **more)
+        gpu.rollback(point)
+        assert one == two, (rnd, one, two)
+    with pytest.raises(Exception, match="at most 16 stop tokens"):
+        gpu.verify_accept(feed, base, shaping, stop_tokens=list(range(17)), **more)
+    assert gpu.position == base + rows
+    gpu.rollback(point)
+    assert gpu.verify_accept(feed, base, shaping, **more) == one

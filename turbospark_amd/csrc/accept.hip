@@ -1118,7 +1118,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
                                                const AcceptParams* app, double* scratch, const double* work,
                                                unsigned long long* hist, const Decision* dec_in,
                                                AcceptResult* res, int32_t* tokens_out, int32_t* err,
-                                               int kind) {
+                                               int kind, AcceptResult* host) {
     __shared__ SideEnt s_raw[PEN ? SIDE_CAP : 1], s_sorted[PEN ? SIDE_CAP : 1];
     __shared__ uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // one bit per vocabulary entry: on the bin's value
     __shared__ int s_nside, s_side_last;
@@ -1328,15 +1328,24 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
             // margins of the k draws are folded on the host side from res->min_margin
             atomicMin((unsigned long long*)&res->min_margin, __builtin_bit_cast(unsigned long long, margin));
         } else {
-            res->accepted = dec.accepted;
-            res->committed = dec.committed;
-            res->stopped = dec.stopped;
-            res->next = dec.stopped ? -1 : token;
-            res->draw_step = dec.draw_step;
-            res->path_len = dec.accepted + 1;
-            for (int i = 0; i <= dec.accepted; i++) res->path[i] = kind == 2 ? tokens_out[i] : i;
-            atomicMin((unsigned long long*)&res->min_margin, __builtin_bit_cast(unsigned long long, margin));
-            res->error = *err;
+            const unsigned long long mine = __builtin_bit_cast(unsigned long long, margin);
+            const double least = __builtin_bit_cast(double, min(atomicMin((unsigned long long*)&res->min_margin, mine), mine));
+            auto put = [&](AcceptResult* to) {
+                to->accepted = dec.accepted;
+                to->committed = dec.committed;
+                to->stopped = dec.stopped;
+                to->next = dec.stopped ? -1 : token;
+                to->draw_step = dec.draw_step;
+                to->path_len = dec.accepted + 1;
+                for (int i = 0; i <= dec.accepted; i++) to->path[i] = kind == 2 ? tokens_out[i] : i;
+                to->error = *err;
+            };
+            put(res);
+            if (host) {
+                put(host);
+                host->min_margin = least;
+                __threadfence_system();
+            }
         }
     }
 }
@@ -1639,22 +1648,29 @@ __device__ GreedyWalk walk_greedy(const AcceptParams& ap, const int32_t* amax) {
 }
 
 __global__ void k_walk_greedy(const AcceptParams* app, const float* pv, const int32_t* pi, AcceptResult* res,
-                              const int32_t* err) {
+                              const int32_t* err, AcceptResult* host) {
     __shared__ int32_t amax[TSV_MAX_ROWS];
     const AcceptParams& ap = *app;
     if ((int)threadIdx.x < ap.m) amax[threadIdx.x] = fold_argmax(pv, pi, threadIdx.x);
     __syncthreads();
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     const GreedyWalk g = walk_greedy(ap, amax);
-    for (int i = 0; i < g.path_len; i++) res->path[i] = g.path[i];
-    res->accepted = g.accepted;
-    res->committed = g.committed;
-    res->stopped = g.stopped;
-    res->next = g.next;
-    res->draw_step = ap.draw_step;
-    res->path_len = g.path_len;
-    res->min_margin = 1.0;
-    res->error = *err;
+    auto put = [&](AcceptResult* to) {
+        for (int i = 0; i < g.path_len; i++) to->path[i] = g.path[i];
+        to->accepted = g.accepted;
+        to->committed = g.committed;
+        to->stopped = g.stopped;
+        to->next = g.next;
+        to->draw_step = ap.draw_step;
+        to->path_len = g.path_len;
+        to->min_margin = 1.0;
+        to->error = *err;
+    };
+    put(res);
+    if (host) {
+        put(host);
+        __threadfence_system();
+    }
 }
 
 __global__ void k_clear_result(AcceptResult* res, int32_t* err) {
@@ -1725,7 +1741,7 @@ static void launch_chain_sampled(hipStream_t s, const uint16_t* target, const ui
     hipLaunchKernelGGL(k_mass_hist<PEN>, dim3(NSEG, 1, NSUB), dim3(256), 0, s, target, draft, ap_dev, sc.stats, sc.work,
                        (unsigned long long*)sc.hist, decisions(sc), 0);
     hipLaunchKernelGGL(k_pick<PEN>, dim3(1), dim3(1024), 0, s, target, draft, ap_dev, sc.stats, sc.work,
-                       (unsigned long long*)sc.hist, decisions(sc), sc.result, (int32_t*)nullptr, err, 0);
+                       (unsigned long long*)sc.hist, decisions(sc), sc.result, (int32_t*)nullptr, err, 0, sc.host_result);
 }
 
 // The most child tests a walk can take before it stops.  At a node with children c_1 < ... < c_n (tested in slot
@@ -1761,7 +1777,7 @@ static void launch_tree_sampled(hipStream_t s, const uint16_t* target, const uin
     hipLaunchKernelGGL(k_tree_finish<PEN>, dim3(TREE_WGS), dim3(256), 0, s, target, ap_dev, sc.stats, sc.work,
                        (unsigned long long*)sc.hist, decisions(sc), path, steps);
     hipLaunchKernelGGL(k_pick<PEN>, dim3(1), dim3(1024), 0, s, target, draft, ap_dev, sc.stats, sc.work,
-                       (unsigned long long*)sc.hist, decisions(sc), sc.result, path, err, 2);
+                       (unsigned long long*)sc.hist, decisions(sc), sc.result, path, err, 2, sc.host_result);
 }
 
 template <bool PEN>
@@ -1772,7 +1788,7 @@ static void launch_draft_sampled(hipStream_t s, const uint16_t* draft, const Acc
     hipLaunchKernelGGL(k_mass_hist<PEN>, dim3(NSEG, ap.k, NSUB), dim3(256), 0, s, draft, draft, ap_dev, sc.stats, sc.work,
                        (unsigned long long*)sc.hist, decisions(sc), 1);
     hipLaunchKernelGGL(k_pick<PEN>, dim3(ap.k), dim3(1024), 0, s, draft, draft, ap_dev, sc.stats, sc.work,
-                       (unsigned long long*)sc.hist, decisions(sc), sc.result, proposals_dev, err, 1);
+                       (unsigned long long*)sc.hist, decisions(sc), sc.result, proposals_dev, err, 1, (AcceptResult*)nullptr);
 }
 
 int launch_accept(hipStream_t s, const uint16_t* target, const uint16_t* draft, const AcceptParams* ap_dev,
@@ -1782,7 +1798,7 @@ int launch_accept(hipStream_t s, const uint16_t* target, const uint16_t* draft, 
     int32_t* pi = (int32_t*)sc.counters + 64 + TSV_MAX_ROWS * ARGMAX_SEG;
     if (!ap.sampled) {  // (the arg-max ignores penalties and truncation: choose.rs:84-88)
         hipLaunchKernelGGL(k_argmax_part, dim3(ARGMAX_SEG, ap.m), dim3(256), 0, s, target, ap.vocab, pv, pi, err);
-        hipLaunchKernelGGL(k_walk_greedy, dim3(1), dim3(64), 0, s, ap_dev, pv, pi, sc.result, err);
+        hipLaunchKernelGGL(k_walk_greedy, dim3(1), dim3(64), 0, s, ap_dev, pv, pi, sc.result, err, sc.host_result);
         TSV_HIP(hipGetLastError());
         return TSV_OK;
     }

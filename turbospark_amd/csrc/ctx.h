@@ -146,6 +146,8 @@ struct tsv_ctx {
         int next = 0;
     } ring;
     AcceptUpload *up_dev = nullptr, *up_host = nullptr;
+    // during a call that passes and accepts at once: the acceptance's parameters, which go to up_dev with the pass's
+    const AcceptUpload* with_pass = nullptr;
     // the stream may still be reading the pinned blocks that calls upload from (a call that failed between its copy and its wait)
     bool uploading = false;
     uint16_t** kv_ptrs = nullptr;  // device: [2 * layer] = K buffer, [2 * layer + 1] = V buffer (tree compaction)

@@ -13,13 +13,11 @@ namespace tsv {
 // arithmetic of dequantize_q4_k / dequantize_q8_0.
 // The last workgroup of a row (when `cs` is given) fills the row's rotation table instead:
 // (cos, sin) of pos * freq, scaled, for every pair index - the same for all layers of the step.
-__global__ void k_embed(const uint8_t* __restrict__ raw, int dtype, int hidden, float* __restrict__ x,
-                        const VerifyParams* __restrict__ vp, const float* __restrict__ freqs, float mscale,
-                        int half, float2* __restrict__ cs, int nblk) {
+__device__ __forceinline__ void embed_rows(const uint8_t* raw, int dtype, int hidden, float* x, long tok, int rot_pos, const float* freqs, float mscale,
+                                           int half, float2* cs, int nblk) {
     const int m = blockIdx.x;
-    if (m >= vp->m) return;
     if ((int)blockIdx.y == nblk) {
-        const float pos = (float)vp->pos[m];
+        const float pos = (float)rot_pos;
         for (int i = threadIdx.x; i < half; i += blockDim.x) {
             float sn, c;
             sincosf(pos * freqs[i], &sn, &c);
@@ -27,16 +25,50 @@ __global__ void k_embed(const uint8_t* __restrict__ raw, int dtype, int hidden, 
         }
         return;
     }
-    const long tok = vp->feed[m];
     for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < hidden; e += blockDim.x * nblk)
         x[(long)m * hidden + e] = embed_elem(raw, dtype, hidden, tok, e);
 }
+__global__ void k_embed(const uint8_t* __restrict__ raw, int dtype, int hidden, float* __restrict__ x,
+                        const VerifyParams* __restrict__ vp, const float* __restrict__ freqs, float mscale,
+                        int half, float2* __restrict__ cs, int nblk) {
+    const int m = blockIdx.x;
+    if (m >= vp->m) return;
+    embed_rows(raw, dtype, hidden, x, vp->feed[m], vp->pos[m], freqs, mscale, half, cs, nblk);
+}
+// ... with the pass's parameters by value, and an acceptance's, which the first workgroup leaves in device memory
+struct EmbedCall {
+    VerifyParams vp;
+    AcceptUpload accept;
+    VerifyParams* vp_dev;
+    AcceptUpload* accept_dev;  // nullable
+};
+__global__ void k_embed_call(const uint8_t* __restrict__ raw, int dtype, int hidden, float* __restrict__ x, EmbedCall now, const float* __restrict__ freqs,
+                             float mscale, int half, float2* __restrict__ cs, int nblk) {
+    static_assert(sizeof(VerifyParams) % 4 == 0 && sizeof(AcceptUpload) % 4 == 0, "copied by words");
+    if (blockIdx.x == 0 && blockIdx.y == 0) {
+        for (int i = threadIdx.x; i < (int)(sizeof(VerifyParams) / 4); i += blockDim.x) ((uint32_t*)now.vp_dev)[i] = ((const uint32_t*)&now.vp)[i];
+        if (now.accept_dev)
+            for (int i = threadIdx.x; i < (int)(sizeof(AcceptUpload) / 4); i += blockDim.x) ((uint32_t*)now.accept_dev)[i] = ((const uint32_t*)&now.accept)[i];
+    }
+    embed_rows(raw, dtype, hidden, x, now.vp.feed[blockIdx.x], now.vp.pos[blockIdx.x], freqs, mscale, half, cs, nblk);
+}
 
 int launch_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float* x,
-                 const VerifyParams* vp, int m, const float* freqs, float mscale, int half, float2* cs) {
+                 const VerifyParams* vp, int m, const float* freqs, float mscale, int half, float2* cs, const PassUpload* now) {
     const int nblk = (hidden + 511) / 512;  // two elements per thread
-    hipLaunchKernelGGL(k_embed, dim3(m, nblk + (cs ? 1 : 0)), dim3(256), 0, s, raw, dtype, hidden, x, vp, freqs, mscale,
-                       half, cs, nblk);
+    const dim3 grid(m, nblk + (cs ? 1 : 0));
+    if (now) {
+        EmbedCall call{};
+        call.vp = *now->vp;
+        call.vp_dev = now->vp_dev;
+        if (now->accept) {
+            call.accept = *now->accept;
+            call.accept_dev = now->accept_dev;
+        }
+        hipLaunchKernelGGL(k_embed_call, grid, dim3(256), 0, s, raw, dtype, hidden, x, call, freqs, mscale, half, cs, nblk);
+    } else {
+        hipLaunchKernelGGL(k_embed, grid, dim3(256), 0, s, raw, dtype, hidden, x, vp, freqs, mscale, half, cs, nblk);
+    }
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }

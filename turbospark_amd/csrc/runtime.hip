@@ -251,6 +251,9 @@ int fill_params(VerifyParams& vp, const int32_t* feed, const int32_t* parent, in
 
 int run_pass(tsv_ctx* c, int m);
 
+// A pass's parameters go with its first launch (launch_embed), except where that is replayed or is a drafter head's
+bool params_by_value(const tsv_ctx* c) { return !c->use_graph && !c->mtp.on; }
+
 // n parameter blocks to `dev` through the next pinned staging slot, on the handle's stream.
 int stage_params(tsv_ctx* c, const VerifyParams* vp, int n, VerifyParams* dev) {
     auto& r = c->ring;
@@ -290,7 +293,7 @@ int enqueue_verify(tsv_ctx* c, const int32_t* feed, const int32_t* parent, int m
     if (prc) return prc;
     *c->vp_host = vp;  // the host's own copy of the pass in flight
     // (a block draft has put the parameter blocks of all its steps on the device in one copy: vp_dev names this step's)
-    if (!c->mtp.params_staged)
+    if (!c->mtp.params_staged && !params_by_value(c))
         if (int prc2 = stage_params(c, &vp, 1, c->vp_dev)) return prc2;
     int rc = run_pass(c, m);
     if (rc) return rc;
@@ -337,8 +340,9 @@ int launch_pass(tsv_ctx* c, int m) {
         rc = launch_gemm(s, h.fc, h.xf_cat, c->partial, c->vp_dev, m, prev_splits, EPI_PARTIAL, c->hidden, c->hidden);
     } else {
         PROF(PC_EMBED);
+        const PassUpload now{c->vp_host, c->vp_dev, c->with_pass, c->up_dev};
         rc = launch_embed(s, c->embed_raw, c->embed_dtype, c->hidden, c->x, c->vp_dev, m, c->freqs, c->rope_mscale,
-                          c->hd / 2, c->rope_cs);
+                          c->hd / 2, c->rope_cs, params_by_value(c) ? &now : nullptr);
     }
     if (rc) return rc;
     const float* prev_partial = c->partial;
@@ -1815,6 +1819,19 @@ int check_history(const tsv_shaping& sh, const int32_t* history, int64_t n) {
     return TSV_OK;
 }
 
+// The penalty fields of a round's parameters: its settings, and where the history's counts will be
+void fill_penalties(tsv_ctx* c, const tsv_shaping& sh, AcceptParams* ap) {
+    ap->pen = has_penalties(sh);
+    if (!ap->pen) return;
+    ap->pen_has_rep = sh.repetition_penalty != 1.0;
+    // penalty.rs:20-25: the f64 setting as an f32 kept inside the normal range
+    ap->pen_rep = std::min(std::max((float)sh.repetition_penalty, 1.17549435e-38f), 3.40282347e+38f);
+    ap->pen_has_pf = sh.presence_penalty != 0.0 || sh.frequency_penalty != 0.0;
+    ap->pen_presence = sh.presence_penalty;
+    ap->pen_frequency = sh.frequency_penalty;
+    ap->pen_cnt = c->pen_cnt;
+}
+
 // Penalised sampled rounds (choose.rs:138-154): uploads the history, counts its tokens on the device
 // and fills the penalty fields of the parameter block.  `generated` is the sink's count of reported
 // tokens: the last min(generated, n) tokens of the history are the generated suffix.
@@ -1840,14 +1857,7 @@ int setup_penalties(tsv_ctx* c, const tsv_shaping& sh, const int32_t* history, i
     const int64_t suffix = (int64_t)std::min<uint64_t>(generated, (uint64_t)n);
     int rc = launch_pen_counts(c->stream, c->hist_dev, (long)n, (long)(n - suffix), c->vocab, c->pen_cnt);
     if (rc) return rc;
-    ap->pen = 1;
-    ap->pen_has_rep = sh.repetition_penalty != 1.0;
-    // penalty.rs:20-25: the f64 setting as an f32 kept inside the normal range
-    ap->pen_rep = std::min(std::max((float)sh.repetition_penalty, 1.17549435e-38f), 3.40282347e+38f);
-    ap->pen_has_pf = sh.presence_penalty != 0.0 || sh.frequency_penalty != 0.0;
-    ap->pen_presence = sh.presence_penalty;
-    ap->pen_frequency = sh.frequency_penalty;
-    ap->pen_cnt = c->pen_cnt;
+    fill_penalties(c, sh, ap);
     return TSV_OK;
 }
 
@@ -1883,7 +1893,8 @@ struct RowsUnderWay {
     }
 };
 
-int accept_impl(tsv_ctx* c, const tsv_round* r, tsv_round_result* out) {
+// staged: the round's parameters went to the device with the pass
+int accept_impl(tsv_ctx* c, const tsv_round* r, tsv_round_result* out, bool staged) {
     int rc = check_round(r);
     if (rc) return rc;
     if (r->m != c->last_m || r->base != c->last_base) {
@@ -1930,14 +1941,17 @@ int accept_impl(tsv_ctx* c, const tsv_round* r, tsv_round_result* out) {
     AcceptParams* ap = &c->up_host->ap;
     if ((rc = fill_accept(c, r, ap))) return rc;
     if ((rc = setup_penalties(c, r->shaping, r->history, r->n_history, r->generated, ap))) return rc;
-    c->up_host->clear_result();
-    TSV_HIP(hipMemcpyAsync(c->up_dev, c->up_host, sizeof(AcceptUpload), hipMemcpyHostToDevice, c->stream));
+    if (!staged) {
+        c->up_host->clear_result();
+        TSV_HIP(hipMemcpyAsync(c->up_dev, c->up_host, sizeof(AcceptUpload), hipMemcpyHostToDevice, c->stream));
+    }
+    AcceptScratch sc = c->sc;
+    sc.host_result = c->res_host;  // (the last kernel leaves it there: no copy)
     {
         PROF(PC_ACCEPT);
-        rc = launch_accept(c->stream, c->logits, draft, &c->up_dev->ap, *ap, c->sc);
+        rc = launch_accept(c->stream, c->logits, draft, &c->up_dev->ap, *ap, sc);
     }
     if (rc) return rc;
-    TSV_HIP(hipMemcpyAsync(c->res_host, c->sc.result, sizeof(AcceptResult), hipMemcpyDeviceToHost, c->stream));
     if (r->logits_out)
         TSV_HIP(hipMemcpyAsync(r->logits_out, c->logits, (size_t)r->m * c->vocab * 2, hipMemcpyDeviceToHost, c->stream));
     if ((rc = upload_end(c))) return rc;
@@ -1977,7 +1991,7 @@ extern "C" int32_t tsv_accept(tsv_ctx* c, const tsv_round* r, tsv_round_result* 
         set_error("accept: null argument");
         return TSV_ERR_INVALID;
     }
-    return accept_impl(c, r, out);
+    return accept_impl(c, r, out, false);
 }
 
 extern "C" int32_t tsv_verify_accept(tsv_ctx* c, const tsv_round* r, tsv_round_result* out) {
@@ -1987,8 +2001,19 @@ extern "C" int32_t tsv_verify_accept(tsv_ctx* c, const tsv_round* r, tsv_round_r
     }
     int rc = check_round(r);
     if (rc) return rc;
-    if ((rc = enqueue_verify(c, r->feed, r->parent, r->m, r->base))) return rc;
-    return accept_impl(c, r, out);
+    // the acceptance's parameters go with the pass, where accept_impl will not refuse the round
+    AcceptUpload upload;
+    const bool staged = params_by_value(c) && r->m >= 1 && r->m <= TSV_MAX_ROWS && r->n_stop >= 0 && r->n_stop <= 16 && (!r->n_stop || r->stop_tokens);
+    if (staged) {
+        fill_accept(c, r, &upload.ap);
+        fill_penalties(c, r->shaping, &upload.ap);
+        upload.clear_result();
+        c->with_pass = &upload;
+    }
+    rc = enqueue_verify(c, r->feed, r->parent, r->m, r->base);
+    c->with_pass = nullptr;
+    if (rc) return rc;
+    return accept_impl(c, r, out, staged);
 }
 
 extern "C" int32_t tsv_draft_chain(tsv_ctx* c, const uint16_t* draft_logits, int32_t k, const tsv_shaping* sh,

@@ -434,9 +434,17 @@ int launch_moe_wide_down(hipStream_t s, int fmt, const MoeGemmArgs& a);
 int launch_moe_fp4_gate_up(hipStream_t s, const MoeGemmArgs& a, int n_groups);
 int launch_moe_fp4_down(hipStream_t s, const MoeGemmArgs& a, int n_groups);
 
+// `now`: what the kernels of the pass (and the acceptance behind it) read of the call, by value: the first kernel leaves it in device memory, where
+// a copy would be a launch of its own, 4 us of the queue's time.  Without it the parameters are at vp already.
+struct AcceptUpload;
+struct PassUpload {
+    const VerifyParams* vp;
+    VerifyParams* vp_dev;
+    const AcceptUpload* accept;  // nullable
+    AcceptUpload* accept_dev;
+};
 int launch_embed(hipStream_t s, const uint8_t* raw, int dtype, int hidden, float* x,
-                 const VerifyParams* vp, int m, const float* freqs = nullptr, float mscale = 1.0f, int half = 0,
-                 float2* cs = nullptr);
+                 const VerifyParams* vp, int m, const float* freqs, float mscale, int half, float2* cs, const PassUpload* now = nullptr);
 // Strides between the 16-row blocks of a prompt pass: rows and partial sums in floats, fragments in bytes.
 struct NormBlocks {
     long x, partial, frag;
@@ -651,6 +659,7 @@ struct AcceptScratch {
     uint64_t* tmass;
     uint32_t* tcount;
     AcceptResult* result;  // device; the caller uploads it cleared with a round's parameters
+    AcceptResult* host_result = nullptr;  // nullable: pinned memory that a round's last kernel leaves the result in as well
 };
 constexpr int ACCEPT_COUNTER_WORDS = 1024;
 size_t accept_stats_doubles(), accept_hist_words();
