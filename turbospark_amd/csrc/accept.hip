@@ -753,24 +753,37 @@ __device__ __forceinline__ void on_path_tokens(const AcceptParams& ap, int row, 
 // entry by entry and walked the root path for each.
 constexpr int PICK_MASK_GROUPS = 32;  // groups of eight entries per thread the match mask holds: vocabularies to 262 144
 __device__ __forceinline__ int mask_groups(int vocab) { return ((vocab + 1023) / 1024 + 7) >> 3; }
+// `ahead`: the first of a lane's groups, asked for before the bin was known (row_ahead).
+constexpr int MASK_AHEAD = 16;
+struct RowAhead {
+    uint4 q[MASK_AHEAD];
+};
+__device__ __forceinline__ RowAhead row_ahead(const uint16_t* lp, int vocab) {
+    RowAhead a;
+    const int groups = mask_groups(vocab), whole = vocab >> 3;
+#pragma unroll
+    for (int j = 0; j < MASK_AHEAD; j++) {
+        const int g = j * 1024 + threadIdx.x;
+        a.q[j] = *(const uint4*)(lp + (j < groups && g < whole ? (long)g * 8 : 0));
+    }
+    return a;
+}
 template <bool PEN>
-__device__ __forceinline__ void build_mask(const AcceptParams& ap, int row, const uint16_t* lp, int bin, uint8_t* mask8) {
+__device__ __forceinline__ void build_mask(const AcceptParams& ap, int row, const uint16_t* lp, int bin, uint8_t* mask8, const RowAhead& ahead) {
     const int tid = threadIdx.x, vocab = ap.vocab, groups = mask_groups(vocab);
     const uint32_t want = key_bits(bin);
     const bool zero_bin = want == 0;
     const float g16 = h2f((uint16_t)want);
     const int whole = vocab >> 3;  // groups of eight entries that lie wholly inside the row
-    constexpr int B = PEN ? 8 : 16;  // loads of the row in flight per lane; a group past the last whole one reads group 0 and is discarded
-    for (int g0 = 0; g0 < groups; g0 += B) {
-        uint4 q[B], c[PEN ? 2 * B : 1];
+    constexpr int B = MASK_AHEAD;  // loads of the row in flight per lane; a group past the last whole one reads group 0 and is discarded
+    const uint8_t* const seen = PEN ? (const uint8_t*)pen_seen(ap.pen_cnt, vocab) : nullptr;  // a group's eight bits
+    auto take = [&](int g0, const uint4 (&q)[B]) {
+        uint32_t pen[PEN ? B : 1];
+        if constexpr (PEN) {
 #pragma unroll
-        for (int j = 0; j < B; j++) {
-            const int g = (g0 + j) * 1024 + tid;
-            const long at = g0 + j < groups && g < whole ? (long)g * 8 : 0;
-            q[j] = *(const uint4*)(lp + at);
-            if constexpr (PEN) {
-                c[2 * j] = *(const uint4*)(ap.pen_cnt + at);
-                c[2 * j + 1] = *(const uint4*)(ap.pen_cnt + at + 4);
+            for (int j = 0; j < B; j++) {
+                const int g = (g0 + j) * 1024 + tid;
+                pen[j] = seen[g0 + j < groups && g < whole ? g : 0];
             }
         }
         uint32_t touched[PEN ? B / 4 : 1] = {};
@@ -785,13 +798,8 @@ __device__ __forceinline__ void build_mask(const AcceptParams& ap, int row, cons
                 m |= (uint32_t)(bits == want || (zero_bin && bits == 0x8000u)) << h;
             }
             if constexpr (PEN) {
-                const uint4 a = c[2 * j], b = c[2 * j + 1];
-                const uint32_t cc[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-                uint32_t pen = 0;
-#pragma unroll
-                for (int h = 0; h < 8; h++) pen |= (uint32_t)(cc[h] != 0) << h;
-                m &= ~pen;
-                if (g0 + j < groups && g < whole) touched[j >> 2] |= pen << (8 * (j & 3));
+                m &= ~pen[j];
+                if (g0 + j < groups && g < whole) touched[j >> 2] |= pen[j] << (8 * (j & 3));
             }
             if (g0 + j < groups) mask8[g] = g < whole ? (uint8_t)m : (uint8_t)0;
         }
@@ -804,6 +812,16 @@ __device__ __forceinline__ void build_mask(const AcceptParams& ap, int row, cons
                     if (penalised(ap, h2f(lp[v]), (cnt >> 31) != 0, cnt & 0x7FFFFFFFu) == g16) mask8[g] |= (uint8_t)(1u << (at & 7));
                 }
         }
+    };
+    take(0, ahead.q);
+    for (int g0 = B; g0 < groups; g0 += B) {
+        uint4 q[B];
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const int g = (g0 + j) * 1024 + tid;
+            q[j] = *(const uint4*)(lp + (g0 + j < groups && g < whole ? (long)g * 8 : 0));
+        }
+        take(g0, q);
     }
     if ((vocab & 7) && whole < groups * 1024 && tid == (whole & 1023)) {  // the row's last, partial group
         uint32_t m = 0;
@@ -829,7 +847,19 @@ __device__ __forceinline__ void build_mask(const AcceptParams& ap, int row, cons
 template <class Fn>
 __device__ __forceinline__ void walk_mask(const uint8_t* mask8, int groups, Fn&& on_match) {
     const uint8_t* mine = mask8 + threadIdx.x * groups;
-    for (int k = 0; k < groups; k++)
+    int k = 0;
+    if ((groups & 15) == 0) {  // sixteen bytes at a time, nearly all of them zero
+        for (; k < groups; k += 16) {
+            const uint4 q = *(const uint4*)(mine + k);
+            if (!(q.x | q.y | q.z | q.w)) continue;
+            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                for (uint32_t m = w[i]; m; m &= m - 1) on_match((threadIdx.x * groups + k) * 8 + 32 * i + (__ffs(m) - 1));
+        }
+        return;
+    }
+    for (; k < groups; k++)
         for (uint32_t m = mine[k]; m; m &= m - 1) on_match((threadIdx.x * groups + k) * 8 + (__ffs(m) - 1));
 }
 
@@ -869,8 +899,7 @@ __device__ __forceinline__ int collect_side(const AcceptParams& ap, int row, con
             if (i < SIDE_CAP) raw[i] = SideEnt{w, v};
         }
     };
-    // the history's table in fours, eight loads in flight; the touched entries are scored afterwards, each lane its own, and
-    // the tokens of the row's path once more by themselves
+    // the tokens of the history, out of its bits, each lane its own, and the tokens of the row's path once more by themselves
     auto on_path = [&](int v) {
         for (int s = row < ap.m ? row : 0; s > 0; s = ap.parent[s])
             if (ap.feed[s] == v) return true;
@@ -881,25 +910,18 @@ __device__ __forceinline__ int collect_side(const AcceptParams& ap, int row, con
         const float w = penalised(ap, h2f(lp[v]), (c >> 31) != 0, c & 0x7FFFFFFFu);
         if (!on_path(v)) look(v, w);
     };
-    const int fours = ap.vocab >> 2;
-    for (int g0 = 0; g0 < fours; g0 += 8 * 1024) {
-        uint4 c[8];
+    const uint32_t* const seen = pen_seen(ap.pen_cnt, ap.vocab);
+    const int words = (ap.vocab + 31) >> 5;
+    for (int w0 = 0; w0 < words; w0 += 4 * 1024) {
+        uint32_t bits[4];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int f = g0 + j * 1024 + tid;
-            c[j] = *(const uint4*)(ap.pen_cnt + (f < fours ? (long)f * 4 : 0));
-        }
-        uint32_t touched = 0;
+        for (int j = 0; j < 4; j++) bits[j] = seen[min(w0 + j * 1024 + tid, words - 1)];
 #pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (g0 + j * 1024 + tid < fours)
-                touched |= ((uint32_t)(c[j].x != 0) | (uint32_t)(c[j].y != 0) << 1 | (uint32_t)(c[j].z != 0) << 2 | (uint32_t)(c[j].w != 0) << 3) << (4 * j);
-        for (; touched; touched &= touched - 1) {
-            const int at = __ffs(touched) - 1;
-            from_table((g0 + (at >> 2) * 1024 + tid) * 4 + (at & 3));
+        for (int j = 0; j < 4; j++) {
+            const int w = w0 + j * 1024 + tid;
+            for (uint32_t left = w < words ? bits[j] : 0u; left; left &= left - 1) from_table(w * 32 + __ffs(left) - 1);
         }
     }
-    if (tid < (ap.vocab & 3) && ap.pen_cnt[fours * 4 + tid] != 0) from_table(fours * 4 + tid);
     on_path_tokens(ap, row, [&](int v) { look(v, score_of<true>(ap, row, v, lp[v])); });
     __syncthreads();
     int n = *counter;
@@ -943,7 +965,7 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
                                                     const unsigned long long* tmass, const uint32_t* tcount,
                                                     AcceptResult* res, int32_t* err) {
     __shared__ SideEnt s_raw[PEN ? SIDE_CAP : 1], s_sorted[PEN ? SIDE_CAP : 1];
-    __shared__ uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // build_mask
+    __shared__ __attribute__((aligned(16))) uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // build_mask
     __shared__ int s_nside;
     __shared__ unsigned long long wsum[16];
     __shared__ unsigned long long s_before_p, s_at;
@@ -955,6 +977,7 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
     Layout L = layout(scratch);
     const double mx = wave_max_f64(L.pmax[row * NSEG + lane]);
     const double sum = fold_row(L.psum, row);
+    const uint16_t* lp = row_ptr(target, draft, m, vocab, row);
     const uint32_t* const gc = tcount + (size_t)row * TRUNC_WORDS;
     const unsigned long long* const gm = tmass + (size_t)row * TRUNC_WORDS;
     static_assert(RANK_GROUPS == 1024, "a group to a thread");
@@ -1006,7 +1029,6 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
         if (best >= 0) atomicMax(&s_minp_key, best);
     }
     __syncthreads();
-    const uint16_t* lp = row_ptr(target, draft, m, vocab, row);
     int ns_p = 0;  // penalised rounds: the top-p bin's candidates above the bin's own value
     if constexpr (PEN) {
         if (s_bin_p >= 0) ns_p = collect_side(ap, row, lp, s_bin_p, s_raw, s_sorted, &s_nside, err);
@@ -1082,7 +1104,7 @@ __global__ __launch_bounds__(1024) void k_trunc_cut(const uint16_t* target, cons
             // the j-th candidate on the bin's value in index order
             const int groups = mask_groups(vocab), v0 = min(tid * groups * 8, vocab), v1 = min(v0 + groups * 8, vocab);
             const bool vec = ((uintptr_t)lp & 15) == 0, masked = vec && groups <= PICK_MASK_GROUPS;
-            if (masked) build_mask<PEN>(ap, row, lp, bin, (uint8_t*)s_mask);
+            if (masked) build_mask<PEN>(ap, row, lp, bin, (uint8_t*)s_mask, row_ahead(lp, vocab));
             auto for_matches = [&](auto&& on_match) {
                 if (masked) walk_mask((const uint8_t*)s_mask, groups, on_match);
                 else scan_on<PEN>(ap, row, lp, v0, v1, bin, vec, on_match);
@@ -1120,7 +1142,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
                                                AcceptResult* res, int32_t* tokens_out, int32_t* err,
                                                int kind, AcceptResult* host) {
     __shared__ SideEnt s_raw[PEN ? SIDE_CAP : 1], s_sorted[PEN ? SIDE_CAP : 1];
-    __shared__ uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // one bit per vocabulary entry: on the bin's value
+    __shared__ __attribute__((aligned(16))) uint32_t s_mask[1024 * PICK_MASK_GROUPS / 4];  // one bit per vocabulary entry: on the bin's value
     __shared__ int s_nside, s_side_last;
     __shared__ double s_side_sum;
     __shared__ unsigned long long wsum[16];
@@ -1130,8 +1152,14 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
     __shared__ double s_cum_before, s_cum_at;
     const AcceptParams& ap = *app;
     const int jobi = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const Decision dec = dec_in[jobi];
+    // What one workgroup costs is the round trips one behind the other: the sums of both modes and the residual's pieces are asked for with the
+    // decision that says which are wanted
     Layout L = layout(scratch);
+    static_assert(NSEG * NSUB == 256, "four waves fold the pieces");
+    const unsigned long long* const sums = rank_groups(hist) + (size_t)jobi * 2 * RANK_GROUPS + tid;
+    const unsigned long long loc_p = sums[0], loc_r = sums[RANK_GROUPS];
+    const double piece = L.segtot[jobi * NSEG * NSUB + (tid & 255)];
+    const Decision dec = dec_in[jobi];
     const int vocab = ap.vocab;
     int token = -1;
     double margin = dec.margin;
@@ -1141,9 +1169,8 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
         double R = 1.0;
         if (mode == 2) {
             // residual mass: the pieces' partial sums folded in a fixed order
-            static_assert(NSEG * NSUB == 256, "four waves fold the pieces");
             if (tid < 256) {
-                const double part = wave_sum_f64(L.segtot[jobi * NSEG * NSUB + tid]);
+                const double part = wave_sum_f64(piece);
                 if (lane == 0) dsum[wave] = part;
             }
             __syncthreads();
@@ -1155,11 +1182,14 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
         unsigned long long* hsel = mode == 2 ? hp + 65536 : hp;
         const double* w = kind == 2 ? work + (long)dec.pad * vocab : work + (long)jobi * 2 * vocab + (mode == 2 ? vocab : 0);
         const uint16_t* lp = row_ptr(target, draft, ap.m, vocab, dec.job.row_p);
+        const int groups = mask_groups(vocab), v0 = min(tid * groups * 8, vocab), v1 = min(v0 + groups * 8, vocab);
+        const bool vec = ((uintptr_t)lp & 15) == 0, masked = vec && groups <= PICK_MASK_GROUPS;
+        RowAhead ahead;  // (the row is on its way while the bin is looked for)
+        if (masked) ahead = row_ahead(lp, vocab);
 
         // 64 consecutive rank bins per thread (see bin_addr), whose sum is there already; integer sums are exact and order
         // independent
-        const unsigned long long* hmine = hsel + (tid >> 6) * 4096 + (tid & 63);
-        const unsigned long long loc = rank_groups(hist)[(jobi * 2 + (mode == 2)) * RANK_GROUPS + tid];
+        const unsigned long long loc = mode == 2 ? loc_r : loc_p;
         unsigned long long inc = loc;
         for (int o = 1; o < 64; o <<= 1) {
             const uint32_t lo = __shfl_up((uint32_t)inc, o), hi = __shfl_up((uint32_t)(inc >> 32), o);
@@ -1184,29 +1214,28 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
         const unsigned long long tgt = (unsigned long long)(dec.job.u * (double)total);
         if (loc > 0) atomicMax(&s_last_bin, tid * 64 + 63);
         if (excl <= tgt && tgt < excl + loc) {
-            // the one thread whose 64 bins hold the target: first bin at which the running sum passes it, out of two rounds of
-            // 32 loads in flight (a loop that stops at the hit waits out one L2 round trip per bin)
-            unsigned long long c = excl, before = excl;
-            int hit = -1;
-#pragma unroll
-            for (int half = 0; half < 2; half++) {
-                unsigned long long hv[32];
-#pragma unroll
-                for (int i = 0; i < 32; i++) hv[i] = hmine[(half * 32 + i) * 64];
-#pragma unroll
-                for (int i = 0; i < 32; i++) {
-                    if (hit < 0 && tgt < c + hv[i]) {
-                        hit = half * 32 + i;
-                        before = c;
-                    }
-                    c += hv[i];
-                }
-            }
-            s_bin = tid * 64 + hit;
-            s_before = before;
+            s_bin = tid;  // the group that holds the target, for now
+            s_before = excl;
         }
         if (tid == 0) s_total = total;
         __syncthreads();
+        if (s_bin >= 0) {
+            // its first bin at which the running sum passes the target: a lane to a bin, every wave for itself
+            const int g = s_bin;
+            const unsigned long long mine = hsel[(g >> 6) * 4096 + (g & 63) + lane * 64], from = s_before;
+            unsigned long long upto = mine;
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t lo = __shfl_up((uint32_t)upto, o), hi = __shfl_up((uint32_t)(upto >> 32), o);
+                if (lane >= o) upto += ((unsigned long long)hi << 32) | lo;
+            }
+            const int hit = __builtin_ctzll(__ballot(tgt < from + upto));  // (the group's sum passes it)
+            __syncthreads();
+            if (tid == hit) {
+                s_bin = g * 64 + hit;
+                s_before = from + upto - mine;
+            }
+            __syncthreads();
+        }
         int bin = s_bin;
         if (bin < 0) {
             // rounding at the tail: the reference falls back to the LAST surviving candidate
@@ -1253,9 +1282,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
             side_sum = s_side_sum;
         }
         // walk the bin in index order: contiguous index chunk per thread
-        const int groups = mask_groups(vocab), v0 = min(tid * groups * 8, vocab), v1 = min(v0 + groups * 8, vocab);
-        const bool vec = ((uintptr_t)lp & 15) == 0, masked = vec && groups <= PICK_MASK_GROUPS;
-        if (masked) build_mask<PEN>(ap, dec.job.row_p, lp, bin, (uint8_t*)s_mask);
+        if (masked) build_mask<PEN>(ap, dec.job.row_p, lp, bin, (uint8_t*)s_mask, ahead);
         // on_match(v) for the candidates of this thread's chunk that sit on the bin's value, ascending
         auto for_matches = [&](auto&& on_match) {
             if (masked) walk_mask((const uint8_t*)s_mask, groups, on_match);
@@ -1858,22 +1885,24 @@ int launch_argmax_rows(hipStream_t s, const uint16_t* logits, int rows, int voca
 // low bits = occurrences in history[suffix_start, n).  Token ids outside [0, vocab) are skipped
 // (penalty.rs:27-33,73-78).
 namespace {
-__global__ void k_pen_clear(uint32_t* cnt, int vocab) {
+__global__ void k_pen_clear(uint32_t* cnt, int words) {
     const int v = blockIdx.x * 256 + threadIdx.x;
-    if (v < vocab) cnt[v] = 0;
+    if (v < words) cnt[v] = 0;
 }
 __global__ void k_pen_count(const int32_t* history, long n, long suffix_start, int vocab, uint32_t* cnt) {
     for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
         const int32_t t = history[i];
         if (t < 0 || t >= vocab) continue;
         atomicOr(cnt + t, 0x80000000u);
+        atomicOr(pen_seen(cnt, vocab) + (t >> 5), 1u << (t & 31));
         if (i >= suffix_start) atomicAdd(cnt + t, 1u);
     }
 }
 }  // namespace
 
 int launch_pen_counts(hipStream_t s, const int32_t* history_dev, long n, long suffix_start, int vocab, uint32_t* cnt) {
-    hipLaunchKernelGGL(k_pen_clear, dim3((vocab + 255) / 256), dim3(256), 0, s, cnt, vocab);
+    const int words = pen_words(vocab);
+    hipLaunchKernelGGL(k_pen_clear, dim3((words + 255) / 256), dim3(256), 0, s, cnt, words);
     if (n > 0) {
         const int blocks = (int)std::min<long>((n + 255) / 256, 256);
         hipLaunchKernelGGL(k_pen_count, dim3(blocks), dim3(256), 0, s, history_dev, n, suffix_start, vocab, cnt);

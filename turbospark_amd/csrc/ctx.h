@@ -153,7 +153,7 @@ struct tsv_ctx {
     uint16_t** kv_ptrs = nullptr;  // device: [2 * layer] = K buffer, [2 * layer + 1] = V buffer (tree compaction)
     int32_t *hist_dev = nullptr, *hist_host = nullptr;  // the token history of a penalised round (grows on demand), and its pinned copy
     size_t hist_cap = 0;
-    uint32_t* pen_cnt = nullptr;  // [vocab] seen flag + generated-suffix count per token
+    uint32_t* pen_cnt = nullptr;  // [vocab] seen flag + generated-suffix count per token, then a bit per token (pen_seen)
     AcceptResult* res_host = nullptr;
     int32_t *tok_dev = nullptr, *tok_host = nullptr;
     AcceptScratch sc{};

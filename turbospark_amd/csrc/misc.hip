@@ -25,8 +25,16 @@ __device__ __forceinline__ void embed_rows(const uint8_t* raw, int dtype, int hi
         }
         return;
     }
-    for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < hidden; e += blockDim.x * nblk)
-        x[(long)m * hidden + e] = embed_elem(raw, dtype, hidden, tok, e);
+    // (workgroups of 256, two values to a thread)
+    embed_types(dtype, [&](auto type) {
+        float v[2];
+        const int e0 = blockIdx.y * 256 + threadIdx.x, step = 256 * nblk;
+#pragma unroll
+        for (int j = 0; j < 2; j++) v[j] = embed_elem<decltype(type)::value>(raw, hidden, tok, min(e0 + j * step, hidden - 1));
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            if (e0 + j * step < hidden) x[(long)m * hidden + e0 + j * step] = v[j];
+    });
 }
 __global__ void k_embed(const uint8_t* __restrict__ raw, int dtype, int hidden, float* __restrict__ x,
                         const VerifyParams* __restrict__ vp, const float* __restrict__ freqs, float mscale,
@@ -265,6 +273,7 @@ int launch_addnorm(hipStream_t s, float* x, const float* partial, int splits, in
 // stream `x_zero` cleared LAST -- it may be the very row h was read from (a chained step), and fc's partial sums
 // are added onto it by the layer's first residual kernel.  Embedding lookup, three norms, the fragment conversion
 // and the token hand-over were four launches and a copy before.
+template <int J>  // values to a thread: hidden <= 1024 J
 __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ raw, int dtype, const VerifyParams* __restrict__ vp,
                                                     const int32_t* __restrict__ token_dev, int vocab, const float* h_rows,
                                                     const float* __restrict__ w_e, const float* __restrict__ w_t,
@@ -274,14 +283,18 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
                                                     float2* __restrict__ cs) {
     __shared__ __attribute__((aligned(16))) float red[3][16];
     const int m = blockIdx.x;
-    if (m >= vp->m) return;
+    asm volatile("" ::"s"(raw), "s"(dtype), "s"(vp), "s"(token_dev), "s"(vocab), "s"(h_rows), "s"(w_e), "s"(w_t), "s"(w_h), "s"(eps), "s"(hidden), "s"(xfrag),
+                 "s"(x_zero), "s"(freqs), "s"(mscale), "s"(half), "s"(cs));
+    const int rows = uniform_memory(vp)->m, fed = uniform_memory(vp)->feed[m], rot = uniform_memory(vp)->pos[m];
+    const int drawn = uniform_memory(token_dev ? token_dev : (const int32_t*)vp)[0];
     // The row and the norms' weights are asked for before the token is waited for, and the angles come last: one workgroup is all
     // there is at a single row, and what it costs is the round trips one behind the other (11.1 -> 10.5 us under a trace; 48 tokens of the loop 16107 -> 15742)
     const float* h = h_rows + (long)m * hidden;
     // at most eight elements per thread (hidden <= 8192): kept in registers across the reductions
-    float ev[8], hv[8], ge[8], gt[8], gh[8];
+    const float freq = freqs[min((int)threadIdx.x, half - 1)];
+    float ev[J], hv[J], ge[J], gt[J], gh[J];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
+    for (int j = 0; j < J; j++) {
         const int i = threadIdx.x + 1024 * j;
         if (i < hidden) {
             hv[j] = h[i];
@@ -292,16 +305,20 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
             hv[j] = ge[j] = gt[j] = gh[j] = 0.f;
         }
     }
-    long tok = vp->feed[m];
-    if (token_dev && m == 0) {
-        const int t = *token_dev;
-        tok = t < 0 ? 0 : t >= vocab ? vocab - 1 : t;
-    }
+    if (m >= rows) return;
+    long tok = fed;
+    if (token_dev && m == 0) tok = drawn < 0 ? 0 : drawn >= vocab ? vocab - 1 : drawn;
+    embed_types(dtype, [&](auto type) {
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const int i = threadIdx.x + 1024 * j;
+            ev[j] = embed_elem<decltype(type)::value>(raw, hidden, tok, min(i, hidden - 1));
+        }
+    });
     float se = 0.f, sh = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int i = threadIdx.x + 1024 * j;
-        ev[j] = i < hidden ? embed_elem(raw, dtype, hidden, tok, i) : 0.f;
+    for (int j = 0; j < J; j++) {
+        if (threadIdx.x + 1024 * j >= hidden) ev[j] = 0.f;
         se += ev[j] * ev[j];
         sh += hv[j] * hv[j];
     }
@@ -310,7 +327,7 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
     const float inv_e = 1.0f / sqrtf(se / (float)hidden + eps), inv_h = 1.0f / sqrtf(sh / (float)hidden + eps);
     float st = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
+    for (int j = 0; j < J; j++) {
         const int i = threadIdx.x + 1024 * j;
         hv[j] = i < hidden ? hv[j] * gt[j] * inv_h : 0.f;
         st += hv[j] * hv[j];
@@ -319,7 +336,7 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
     const float inv_t = 1.0f / sqrtf(st / (float)hidden + eps);
     float* sums = (float*)((char*)xfrag + xfrag_sum_offset(2 * hidden));
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
+    for (int j = 0; j < J; j++) {
         const int i = threadIdx.x + 1024 * j;  // hidden is a multiple of 32: whole sub-blocks stay or leave together
         if (i >= hidden) continue;
         const _Float16 he = pinned_half((_Float16)(ev[j] * ge[j] * inv_e));
@@ -333,11 +350,10 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
         }
         x_zero[(long)m * hidden + i] = 0.f;
     }
-    const float pos = (float)vp->pos[m];
-    for (int i = threadIdx.x; i < half; i += 1024) {
+    if ((int)threadIdx.x < half) {  // (64 pairs at most)
         float sn, c;
-        sincosf(pos * freqs[i], &sn, &c);
-        cs[m * half + i] = float2{c * mscale, sn * mscale};
+        sincosf((float)rot * freq, &sn, &c);
+        cs[m * half + threadIdx.x] = float2{c * mscale, sn * mscale};
     }
 }
 
@@ -348,7 +364,12 @@ int launch_mtp_input(hipStream_t s, const uint8_t* raw, int dtype, const VerifyP
         set_error("drafter head: hidden must be a multiple of 32, at most 8192");
         return TSV_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(k_mtp_input, dim3(m), dim3(1024), 0, s, raw, dtype, vp, token_dev, vocab, h_rows, w_e, w_t, w_h, eps, hidden,
+    if (half > 1024) {
+        set_error("drafter head: at most 1024 rotation pairs");
+        return TSV_ERR_UNSUPPORTED;
+    }
+    const auto kernel = hidden <= 4096 ? k_mtp_input<4> : k_mtp_input<8>;
+    hipLaunchKernelGGL(kernel, dim3(m), dim3(1024), 0, s, raw, dtype, vp, token_dev, vocab, h_rows, w_e, w_t, w_h, eps, hidden,
                        (_Float16*)xfrag, x_zero, freqs, mscale, half, cs);
     TSV_HIP(hipGetLastError());
     return TSV_OK;

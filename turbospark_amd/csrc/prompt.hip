@@ -29,9 +29,16 @@ __global__ __launch_bounds__(256) void k_prompt_embed(const uint8_t* __restrict_
                                                       int half, float2* __restrict__ cs) {
     const int row = blockIdx.x;
     const long tok = ids[row];
-    // (four values to a thread: each is a round trip or two of its own)
-    for (int e = blockIdx.y * 1024 + threadIdx.x; e < min(hidden, (int)blockIdx.y * 1024 + 1024); e += 256)
-        x[(size_t)row * hidden + e] = embed_elem(raw, dtype, hidden, tok, e);
+    // (four values to a thread, in flight together)
+    embed_types(dtype, [&](auto type) {
+        float v[4];
+        const int e0 = blockIdx.y * 1024 + threadIdx.x;
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = embed_elem<decltype(type)::value>(raw, hidden, tok, min(e0 + 256 * j, hidden - 1));
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (e0 + 256 * j < hidden) x[(size_t)row * hidden + e0 + 256 * j] = v[j];
+    });
     if (blockIdx.y) return;
     const float pos = (float)(base + row);
     for (int i = threadIdx.x; i < half; i += 256) {
@@ -104,11 +111,19 @@ __global__ __launch_bounds__(512) void k_prompt_mtp_input(PromptMtpArgs p) {
             hv[i][4 * h] = t.x, hv[i][4 * h + 1] = t.y, hv[i][4 * h + 2] = t.z, hv[i][4 * h + 3] = t.w;
         }
     });
-#pragma unroll 8
-    for (int j = 0; j < NV * 8; j++) {
-        const int e = j * 512 + threadIdx.x;
-        emb[e] = e < p.hidden ? embed_elem(p.raw, p.dtype, p.hidden, tok, e) : 0.f;
-    }
+    embed_types(p.dtype, [&](auto type) {
+#pragma unroll
+        for (int j0 = 0; j0 < NV * 8; j0 += 8) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = embed_elem<decltype(type)::value>(p.raw, p.hidden, tok, min((j0 + j) * 512 + (int)threadIdx.x, p.hidden - 1));
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int e = (j0 + j) * 512 + threadIdx.x;
+                emb[e] = e < p.hidden ? v[j] : 0.f;
+            }
+        }
+    });
     const float pos = (float)(p.base + row);
     for (int i = threadIdx.x; i < p.half; i += 512) {
         float sn, c;

@@ -1337,7 +1337,7 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         (rc = dev_alloc(c, &c->draft_stage, (size_t)16 * c->vocab * 2, true)) ||
         (rc = dev_alloc(c, &c->vp_dev, sizeof(VerifyParams), true)) ||
         (rc = dev_alloc(c, &c->up_dev, sizeof(AcceptUpload), true)) ||
-        (rc = dev_alloc(c, &c->pen_cnt, (size_t)c->vocab * 4, true)) ||
+        (rc = dev_alloc(c, &c->pen_cnt, (size_t)pen_words(c->vocab) * 4, true)) ||
         (rc = dev_alloc(c, &c->tok_dev, 64 * 4, true)) ||
         (rc = dev_alloc(c, &c->sc.stats, accept_stats_doubles() * 8, true)) ||
         (rc = dev_alloc(c, &c->sc.work, (size_t)accept_work_rows() * c->vocab * 8, true)) ||

@@ -608,6 +608,11 @@ int launch_kv_read(hipStream_t s, const uint16_t* kc, const uint16_t* vc, int nk
                    int pos0, int n, uint16_t* k_out, uint16_t* v_out);
 
 // ---- acceptance -------------------------------------------------------------------------
+template <class T>
+__host__ __device__ inline T* pen_seen(T* cnt, int vocab) {
+    return cnt + ((vocab + 3) & ~3);
+}
+inline int pen_words(int vocab) { return ((vocab + 3) & ~3) + (vocab + 31) / 32; }
 struct AcceptParams {
     int32_t m, k;            // rows, proposals (chain: m-1)
     int32_t vocab;
@@ -627,6 +632,7 @@ struct AcceptParams {
     int32_t pen, pen_has_rep, pen_has_pf;
     float pen_rep;  // the repetition penalty as the clamped f32 the reference divides / multiplies by
     double pen_presence, pen_frequency;
+    // Behind the counts one bit a token, whether it is in the history (pen_seen): who looks for the few tokens that are reads 16 KB and not 512.
     const uint32_t* pen_cnt;
 };
 struct AcceptResult {
