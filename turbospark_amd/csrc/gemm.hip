@@ -351,7 +351,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
         Stage<F, NG> st[STAGES];
         const ActLoader<false> x(a.xfrag, a.xsum, lane);
         const int last = c0 + nc - 1;
-        auto fetch = [&](Stage<F, NG>& sg, int c) { load_stage(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
+        auto fetch = [&](Stage<F, NG>& sg, int c) { load_tile(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
 #pragma unroll
         for (int s = 0; s < STAGES; s++) fetch(st[s], min(c0 + s, last));
         pass.asked();
@@ -359,8 +359,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
         for (; c + 2 * STAGES <= nc; c += STAGES) {
 #pragma unroll
             for (int s = 0; s < STAGES; s++) {
-                compute(st[s], k, acc);
-                fetch(st[s], c0 + c + s + STAGES);
+                const int next = c0 + c + s + STAGES;
+                compute_and_load(st[s], k, acc, x, wt + (size_t)next * F::TILE_BYTES, next, lane);
             }
         }
         rope = ask_rope<EPI>(a, out_tile, min(wave, NG - 1), lane);  // (of the row group that the wave finishes first)

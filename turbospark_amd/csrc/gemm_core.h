@@ -2,6 +2,7 @@
 // of the software pipeline, and the per-tile MFMA sequences.  Shared by the stand-alone matmul
 // kernel and the fused per-XCD layer kernels.
 #pragma once
+#include <type_traits>
 #include <utility>
 
 #include "tsv_internal.h"
@@ -88,8 +89,9 @@ __device__ __forceinline__ void load_in_order(T& to, const T* p) {
 }
 
 // ------------------------------------------------------------------------------- formats
+// PARTS: the pieces of a tile (beside its scales) that come free one after the other while it is multiplied; 0: all at the end (load_part)
 struct Q4K {
-    static constexpr int NSUB = 8, NPAIR = 4, TILE_BYTES = 9216;
+    static constexpr int NSUB = 8, NPAIR = 4, TILE_BYTES = 9216, PARTS = 4;
     static constexpr bool SUMS = true;  // the matmul needs the activations' sub-block sums
     struct Regs {
         u32x4 q[8];
@@ -116,7 +118,7 @@ struct Q4K {
 // Q5_K (crates/compute/src/quant_gguf/q5_k.rs:47-96): the Q4_K tile followed by the fifth bits,
 // [2 units][64 lanes][16 B] = the lane's 32 qh bytes.
 struct Q5K {
-    static constexpr int NSUB = 8, NPAIR = 4, TILE_BYTES = 11264;
+    static constexpr int NSUB = 8, NPAIR = 4, TILE_BYTES = 11264, PARTS = 0;
     static constexpr bool SUMS = true;
     struct Regs {
         u32x4 q[8];
@@ -136,7 +138,7 @@ struct Q5K {
 };
 
 struct Q80 {
-    static constexpr int NSUB = 4, NPAIR = 2, TILE_BYTES = 8704;
+    static constexpr int NSUB = 4, NPAIR = 2, TILE_BYTES = 8704, PARTS = 2;
     static constexpr bool SUMS = true;
     struct Regs {
         u32x4 q[8];
@@ -169,7 +171,7 @@ struct Q80 {
 // activations' element order; then the eight scale bytes per lane.  e2m1 values are exact in
 // fp16 and signed, so there is no code offset and no use for the activation sums.
 struct MX4 {
-    static constexpr int NSUB = 8, NPAIR = 4, TILE_BYTES = 8704;
+    static constexpr int NSUB = 8, NPAIR = 4, TILE_BYTES = 8704, PARTS = 4;
     static constexpr bool SUMS = false;
     typedef Q80::Regs Regs;
     static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int lane) { Q80::load(r, tile, lane); }
@@ -186,7 +188,7 @@ struct MX4 {
 // v_mfma_f32_4x4x4_16B_bf16.  The fp16 activations are split exactly into two bf16 terms
 // (upper eight significant bits + remainder), so the products are those of the fp16 values.
 struct BF16W {
-    static constexpr int NSUB = 2, NPAIR = 1, TILE_BYTES = 8192;
+    static constexpr int NSUB = 2, NPAIR = 1, TILE_BYTES = 8192, PARTS = 0;  // (in parts 1 % slower)
     static constexpr bool SUMS = false;
     struct Regs {
         u32x4 q[8];
@@ -205,7 +207,7 @@ struct BF16W {
 // exact fp16 integer level - 32: (low nibble | 0x6400) | (high pair << 4) is 1024 + level, and one
 // packed fp16 add of -1056 removes offset and bias together.
 struct Q6K {
-    static constexpr int NSUB = 16, NPAIR = 4, TILE_BYTES = 13568;
+    static constexpr int NSUB = 16, NPAIR = 4, TILE_BYTES = 13568, PARTS = 4;
     static constexpr bool SUMS = false;
     struct Regs {
         u32x4 q[12];
@@ -343,9 +345,10 @@ __device__ __forceinline__ void fma4(float4v& t, float s, const float4v& d) {
 //   t += sum_j d*sc_j * (X_j . (off_j + q_j))                  64 fp16 MFMAs per group
 // Both parts are summed per tile first so the large code offsets cancel before they reach the
 // running accumulator.
-template <int NG, class Src>
-__device__ __forceinline__ void compute_tile(Q4K, const Src& w, const XRegs<Q4K, NG>& x, const Consts& k,
-                                             float4v (&acc)[NG]) {
+// after(p): called where pair p of the sub-blocks is through (-1: the scales and the sums)
+template <int NG, class Src, class After>
+__device__ __forceinline__ void compute_tile_then(Q4K, const Src& w, const XRegs<Q4K, NG>& x, const Consts& k,
+                                                  float4v (&acc)[NG], After&& after) {
     const u32x4 hs = w.scales();
     const float d = h2f_lo(hs.x), dmin = h2f_hi(hs.x);
     // 6-bit scale / min unpack (q4_k.rs:43-54), four sub-blocks per 32-bit word
@@ -368,6 +371,7 @@ __device__ __forceinline__ void compute_tile(Q4K, const Src& w, const XRegs<Q4K,
 #pragma unroll
         for (int g = 0; g < NG; g++) t[g] = mfma_f32<j>(x.xs[g], cf[j], t[g]);
     });
+    after(-1);
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         const u32x4 qa = w.unit(2 * p), qb = w.unit(2 * p + 1);
@@ -391,11 +395,11 @@ __device__ __forceinline__ void compute_tile(Q4K, const Src& w, const XRegs<Q4K,
             fma4(t[g], sc[2 * p], dlo[g]);
             fma4(t[g], sc[2 * p + 1], dhi[g]);
         }
+        after(p);
     }
 #pragma unroll
     for (int g = 0; g < NG; g++) acc[g] += t[g];
 }
-
 // One Q5_K superblock tile: Q4_K's sequence with the fifth bit of every code OR-ed into the fp16
 // integer before the MFMA (bit 4 of 1024 + q for the low-nibble elements, bit 8 of the 1/16-ulp
 // 64 + q form for the high-nibble ones).  Byte l of the lane's 32 qh bytes serves elements l of all
@@ -462,9 +466,9 @@ __device__ __forceinline__ void compute_tile(Q5K, const Src& w, const XRegs<Q5K,
 
 // One Q8_0 tile (64 rows x 128 K = four 32-element blocks).  Codes go in as 1024 + (q + 128);
 // the 1152 offset comes back out through the activation sums on the fp32 matrix pipe.
-template <int NG, class Src>
-__device__ __forceinline__ void compute_tile(Q80, const Src& w, const XRegs<Q80, NG>& x, const Consts& k,
-                                             float4v (&acc)[NG]) {
+template <int NG, class Src, class After>
+__device__ __forceinline__ void compute_tile_then(Q80, const Src& w, const XRegs<Q80, NG>& x, const Consts& k,
+                                             float4v (&acc)[NG], After&& after) {
     const u32x2 hs = w.scales();
     float dj[4] = {h2f_lo(hs.x), h2f_hi(hs.x), h2f_lo(hs.y), h2f_hi(hs.y)};
     float4v t[NG];
@@ -475,6 +479,7 @@ __device__ __forceinline__ void compute_tile(Q80, const Src& w, const XRegs<Q80,
 #pragma unroll
         for (int g = 0; g < NG; g++) t[g] = mfma_f32<j>(x.xs[g], dj[j] * -1152.0f, t[g]);
     });
+    after(-1);
 #pragma unroll
     for (int p = 0; p < 2; p++) {
         const u32x4 qa0 = w.unit(4 * p), qa1 = w.unit(4 * p + 1), qb0 = w.unit(4 * p + 2), qb1 = w.unit(4 * p + 3);
@@ -499,15 +504,16 @@ __device__ __forceinline__ void compute_tile(Q80, const Src& w, const XRegs<Q80,
             fma4(t[g], dj[2 * p], da[g]);
             fma4(t[g], dj[2 * p + 1], db[g]);
         }
+        after(p);
     }
 #pragma unroll
     for (int g = 0; g < NG; g++) acc[g] += t[g];
 }
 
 // One MXFP4 tile (64 rows x 256 K = eight 32-element blocks): value = e2m1(code) * 2^(e - 127).
-template <int NG, class Src>
-__device__ __forceinline__ void compute_tile(MX4, const Src& w, const XRegs<MX4, NG>& x, const Consts&,
-                                             float4v (&acc)[NG]) {
+template <int NG, class Src, class After>
+__device__ __forceinline__ void compute_tile_then(MX4, const Src& w, const XRegs<MX4, NG>& x, const Consts&,
+                                             float4v (&acc)[NG], After&& after) {
     typedef _Float16 half2v __attribute__((ext_vector_type(2)));
     const u32x2 hs = w.scales();
     float sc[8];
@@ -516,6 +522,7 @@ __device__ __forceinline__ void compute_tile(MX4, const Src& w, const XRegs<MX4,
         const uint32_t e = ((j < 4 ? hs.x : hs.y) >> (8 * (j & 3))) & 0xFFu;
         sc[j] = __uint_as_float(e ? e << 23 : 0x00400000u);  // 2^(e-127); e = 0 is the subnormal 2^-127
     }
+    after(-1);
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         const u32x4 qa = w.unit(2 * p), qb = w.unit(2 * p + 1);
@@ -546,17 +553,19 @@ __device__ __forceinline__ void compute_tile(MX4, const Src& w, const XRegs<MX4,
             fma4(acc[g], sc[2 * p], da[g]);
             fma4(acc[g], sc[2 * p + 1], db[g]);
         }
+        after(p);
     }
 }
 
 // One Q6_K superblock tile (64 rows x 256 K): sixteen 16-element sub-blocks, four K steps each.
-template <int NG, class Src>
-__device__ __forceinline__ void compute_tile(Q6K, const Src& w, const XRegs<Q6K, NG>& x, const Consts& k,
-                                             float4v (&acc)[NG]) {
+template <int NG, class Src, class After>
+__device__ __forceinline__ void compute_tile_then(Q6K, const Src& w, const XRegs<Q6K, NG>& x, const Consts& k,
+                                             float4v (&acc)[NG], After&& after) {
     typedef _Float16 half2v __attribute__((ext_vector_type(2)));
     const u32x4 scw = w.scales();
     const float d = h2f_lo(w.dval());
     const half2v off = {(_Float16)-1056.0f, (_Float16)-1056.0f};
+    after(-1);
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         const u32x4 n0 = w.unit(3 * p), n1 = w.unit(3 * p + 1), hh = w.unit(3 * p + 2);
@@ -587,6 +596,7 @@ __device__ __forceinline__ void compute_tile(Q6K, const Src& w, const XRegs<Q6K,
 #pragma unroll
             for (int g = 0; g < NG; g++) fma4(acc[g], sc, t[g]);
         });
+        after(p);
     }
 }
 
@@ -622,7 +632,59 @@ __device__ __forceinline__ void compute_tile(BF16W, const Src& w, const XRegs<BF
 // a register stage
 template <class F, int NG>
 __device__ __forceinline__ void compute(const Stage<F, NG>& st, const Consts& k, float4v (&acc)[NG]) {
-    compute_tile<NG>(F{}, RegSrc<F>{st.w}, st.x, k, acc);
+    if constexpr (F::PARTS) compute_tile_then<NG>(F{}, RegSrc<F>{st.w}, st.x, k, acc, [](int) {});
+    else compute_tile<NG>(F{}, RegSrc<F>{st.w}, st.x, k, acc);
+}
+
+// Part u of a tile and of its activations: -1 the scales and the sums, else what is multiplied behind them, one after the other.  Loads come
+// back in this order.
+template <class F, int NG, bool COH>
+__device__ __forceinline__ void load_part(Stage<F, NG>& st, const ActLoader<COH>& x, const uint8_t* tile_chunk, int c, int lane, int u) {
+    const u32x4* p = (const u32x4*)tile_chunk + lane;
+    constexpr bool Q6 = std::is_same<F, Q6K>::value, Q4 = std::is_same<F, Q4K>::value;
+    constexpr int UNITS = Q6 ? 3 : std::is_same<F, Q80>::value ? 4 : 2;  // of a part
+    __builtin_amdgcn_sched_barrier(0);
+    if (u < 0) {
+        if constexpr (Q6) {
+            st.w.s = __builtin_nontemporal_load(p + 12 * 64);
+            st.w.d = __builtin_nontemporal_load((const uint32_t*)(tile_chunk + 13312) + lane);
+        } else if constexpr (Q4) {
+            st.w.s = __builtin_nontemporal_load(p + 512);
+        } else {
+            st.w.s = __builtin_nontemporal_load((const u32x2*)(tile_chunk + 8192) + lane);
+        }
+        if (F::SUMS) {
+#pragma unroll
+            for (int g = 0; g < NG; g++) st.x.xs[g] = x.sum_at(F::xs_base(c), F::xs_lane(lane) + x.sumoff[g]);
+        }
+    } else {
+#pragma unroll
+        for (int g = 0; g < NG; g++) st.x.xa[u][g] = x.frag_at((c * F::NPAIR + u) * 256, x.rowoff[g] + (lane >> 2) * 4);
+#pragma unroll
+        for (int i = 0; i < UNITS; i++) st.w.q[UNITS * u + i] = __builtin_nontemporal_load(p + (UNITS * u + i) * 64);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <class F, int NG, bool COH>
+__device__ __forceinline__ void load_tile(Stage<F, NG>& st, const ActLoader<COH>& x, const uint8_t* tile_chunk, int c, int lane) {
+    if constexpr (F::PARTS) {
+#pragma unroll
+        for (int u = -1; u < F::PARTS; u++) load_part(st, x, tile_chunk, c, lane, u);
+    } else load_stage(st, x, tile_chunk, c, lane);
+}
+// Multiplies a tile and asks for the next one, its parts as this one's come free: the first of them are on their way for the rest of the products,
+// in the same registers.  (All of it behind the last product, five rows through 32 layers of the 8B shape in Q4_K took 1938 us for 1900, one row at a time
+// through the Q4_K_M mix 3874 for 3746, six rows of eight Q8_0 layers 687 for 660, nine through routed MXFP4 layers 1018 for 993 and 768 for 752.)
+template <class F, int NG, bool COH>
+__device__ __forceinline__ void compute_and_load(Stage<F, NG>& st, const Consts& k, float4v (&acc)[NG], const ActLoader<COH>& x, const uint8_t* tile_chunk,
+                                                 int c, int lane) {
+    if constexpr (F::PARTS) {
+        const Stage<F, NG> now = st;
+        compute_tile_then<NG>(F{}, RegSrc<F>{now.w}, now.x, k, acc, [&](int u) { load_part(st, x, tile_chunk, c, lane, u); });
+    } else {
+        compute(st, k, acc);
+        load_stage(st, x, tile_chunk, c, lane);
+    }
 }
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)); }

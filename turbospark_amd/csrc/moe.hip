@@ -259,15 +259,15 @@ __device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const MoeGroup
     if (nc > 0) {
         Stage<F, NG> st[STAGES];
         const int last = c0 + nc - 1;
-        auto fetch = [&](Stage<F, NG>& sg, int c) { load_stage(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
+        auto fetch = [&](Stage<F, NG>& sg, int c) { load_tile(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
 #pragma unroll
         for (int s = 0; s < STAGES; s++) fetch(st[s], min(c0 + s, last));
         int c = 0;
         for (; c + 2 * STAGES <= nc; c += STAGES) {
 #pragma unroll
             for (int s = 0; s < STAGES; s++) {
-                compute(st[s], k, acc);
-                fetch(st[s], c0 + c + s + STAGES);
+                const int next = c0 + c + s + STAGES;
+                compute_and_load(st[s], k, acc, x, wt + (size_t)next * F::TILE_BYTES, next, lane);
             }
         }
 #pragma unroll
@@ -379,15 +379,15 @@ __global__ __launch_bounds__(512) void k_moe_gemm(MoeGemmArgs a) {
     if (nc > 0) {
         Stage<F, 1> st[STAGES];
         const int last = c0 + nc - 1;
-        auto fetch = [&](Stage<F, 1>& sg, int c) { load_stage(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
+        auto fetch = [&](Stage<F, 1>& sg, int c) { load_tile(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
 #pragma unroll
         for (int s = 0; s < STAGES; s++) fetch(st[s], min(c0 + s, last));
         int c = 0;
         for (; c + 2 * STAGES <= nc; c += STAGES) {
 #pragma unroll
             for (int s = 0; s < STAGES; s++) {
-                compute(st[s], k, acc);
-                fetch(st[s], c0 + c + s + STAGES);
+                const int next = c0 + c + s + STAGES;
+                compute_and_load(st[s], k, acc, x, wt + (size_t)next * F::TILE_BYTES, next, lane);
             }
         }
         if (wave == 0) ask_biases();
