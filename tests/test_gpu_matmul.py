@@ -60,6 +60,20 @@ def test_split_k_changes_nothing_but_rounding_and_is_deterministic(dtype):
     assert np.abs(a - want[:5]).max() <= np.abs(want).max() * 2e-4 + 1e-5
 
 
+@pytest.mark.parametrize("rows,cols", [(4096, 14336), (4160, 14336), (8192, 8192)])   # whole rounds of 256 workgroups, one tile past, two tiles a unit
+def test_the_chosen_parts_of_k_are_as_near_to_64_bits_as_any(rows, cols):
+    from turbospark_amd import ffi
+    r = np.random.default_rng(5)
+    entry = ffi.quantize(14, r.standard_normal((rows, cols), dtype=np.float32) * np.float32(0.05))
+    x = r.standard_normal((5, cols)).astype(np.float16).astype(np.float32)
+    w = ob.dequantize(14, entry[1], cols).reshape(rows, cols)
+    want = x.astype(np.float64) @ w.T.astype(np.float64)
+    # fp32 sums of K products in any order: at most K 2^-24 of the sum of the magnitudes, and in practice its root's share
+    bound = np.sqrt(cols) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    for splits in (0, 1, 7):
+        assert np.all(np.abs(ffi.matmul(entry, x, splits=splits) - want) <= bound), splits
+
+
 def test_q4k_hand_packed_superblock_through_the_kernel(golden):
     """The reference's literal superblock (quant_gguf.rs:226-267) as a 16-row weight matrix:
     one-hot activations read the decoded weights back out of the kernel."""
