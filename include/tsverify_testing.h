@@ -32,6 +32,8 @@ int32_t tsv_write_logits(tsv_ctx* ctx, const uint16_t* logits, int32_t m, int64_
  * m x rows fp32.  W host tensor in GGUF layout (re-tiled per call).  `splits` <= 0 picks
  * the engine's own split-K factor.  More than TSV_MAX_ROWS rows (2048 at most) go through the prompt passes' kernel. */
 int32_t tsv_matmul(const tsv_tensor* w, const float* x, int32_t m, float* y, int32_t splits);
+/* Host arithmetic only: the parts of K in which the engine's own split-K factor has a matrix of this shape summed. */
+int32_t tsv_matmul_parts(int32_t dtype, int64_t rows, int64_t cols, int32_t* parts);
 
 /* Host arithmetic only: how many launches of the walk kernel a sampled tree round of this shape is given -- the most
  * child tests any walk through the tree can take (children are tested in slot order; a walk rejects all n children of

@@ -1218,12 +1218,6 @@ int gemm_default_splits(const TiledW& w, int) {
     const int cpw = pref_chunks_per_wave(w);
     const int waves = (w.kchunks + cpw - 1) / cpw;
     int splits = std::min(8, (waves + 3) / 4);
-    // Fewer parts, of up to eight waves, where they make exactly a workgroup (or two, ...) for each compute unit: none has one more than another to walk, and
-    // the next kernel adds fewer partial sums.  4096 rows of 14336 in four parts for seven (448 workgroups): a five-row round through 32 layers
-    // 1900 -> 1869 us, sixteen rows through 16 1489 -> 1473.  Where the parts only come near (320 workgroups for 480, 270 for 360) four gpt-oss layers lost 1.7 %.
-    // A wave's own chain of chunks stays as long; six draws of sixteen Q6_K rows against 64 bits: rms 7.38e-7 in both, largest 4.5e-6 -> 4.0e-6.
-    for (int s = 1; s < splits; s++)
-        if (w.n_tiles * s % 256 == 0 && (waves + s - 1) / s <= 8) splits = s;
     const int kslice = (w.kchunks + splits - 1) / splits;
     return (w.kchunks + kslice - 1) / kslice;  // every split non-empty
 }

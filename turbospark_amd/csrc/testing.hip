@@ -313,6 +313,19 @@ static int prompt_matmul(const tsv_tensor* w, const float* x, int32_t m, float* 
     return rc;
 }
 
+extern "C" int32_t tsv_matmul_parts(int32_t dtype, int64_t rows, int64_t cols, int32_t* parts) {
+    const int fmt = dtype_fmt(dtype);
+    if (fmt < 0 || rows < 1 || rows > 1 << 24 || cols < 1 || cols > 1 << 20 || !parts) {
+        set_error("matmul_parts: bad argument");
+        return TSV_ERR_INVALID;
+    }
+    TiledW w;
+    w.n_tiles = (int)((rows + TILE_ROWS - 1) / TILE_ROWS);
+    w.kchunks = (int)((cols + fmt_chunk_elems(fmt) - 1) / fmt_chunk_elems(fmt));
+    *parts = gemm_default_splits(w, 1);
+    return TSV_OK;
+}
+
 extern "C" int32_t tsv_matmul(const tsv_tensor* w, const float* x, int32_t m, float* y, int32_t splits) {
     if (w && x && y && m > TSV_MAX_ROWS && m <= PROMPT_ROWS && splits <= 8) {
         const int rc = check_matrix(*w, w->rows, w->cols, "matmul weight");

@@ -249,7 +249,7 @@ EXPORTS = [
     "tsv_produce", "tsv_prefill", "tsv_checkpoint", "tsv_rollback", "tsv_rollback_retaining",
     "tsv_commit_pending", "tsv_discard_pending", "tsv_verify", "tsv_verify_tree", "tsv_compact_tree",
     "tsv_accept", "tsv_verify_accept", "tsv_accept_greedy_noalloc", "tsv_draft_chain", "tsv_row_bytes", "tsv_quantize_rows",
-    "tsv_synth_tensor", "tsv_read_kv", "tsv_write_kv", "tsv_write_logits", "tsv_matmul", "tsv_attention", "tsv_set_profile", "tsv_get_profile", "tsv_matmul_time", "tsv_copy_time", "tsv_set_repeat",
+    "tsv_synth_tensor", "tsv_read_kv", "tsv_write_kv", "tsv_write_logits", "tsv_matmul", "tsv_matmul_parts", "tsv_attention", "tsv_set_profile", "tsv_get_profile", "tsv_matmul_time", "tsv_copy_time", "tsv_set_repeat",
     "tsv_yarn_frequencies", "tsv_adaptive_init", "tsv_adaptive_depth", "tsv_adaptive_observe", "tsv_adaptive_tile_cap",
     "tsv_run_speculative", "tsv_max_context", "tsv_vocab",
     "tsv_prefix_new", "tsv_prefix_free", "tsv_prefix_clear", "tsv_prefix_taint", "tsv_prefix_record",
@@ -336,6 +336,7 @@ def lib():
         L.tsv_write_kv.argtypes = [C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]
         L.tsv_write_logits.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_int64]
         L.tsv_matmul.argtypes = [C.POINTER(Tensor), C.c_void_p, C.c_int32, C.c_void_p, C.c_int32]
+        L.tsv_matmul_parts.argtypes = [C.c_int32, C.c_int64, C.c_int64, C.POINTER(C.c_int32)]
         L.tsv_attention.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_int32,
                                     C.c_int64, C.c_void_p, C.c_float, C.c_int32, C.c_void_p, C.c_void_p]
         L.tsv_read_kv_quantized.argtypes = [C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]
@@ -443,6 +444,13 @@ def matmul(entry, x, splits=0):
     y = np.empty((m, entry[2]), np.float32)
     check(lib().tsv_matmul(C.byref(t), x.ctypes.data, m, y.ctypes.data, splits))
     return y
+
+
+def matmul_parts(dtype, rows, cols):
+    """The parts of K in which the engine sums a matrix of this shape (matmul's splits = 0)."""
+    n = C.c_int32()
+    check(lib().tsv_matmul_parts(dtype, rows, cols, C.byref(n)))
+    return n.value
 
 
 def attention(q, k, v, base, parent=None, scale=0.0, window=0, sinks=None):
