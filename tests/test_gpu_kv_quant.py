@@ -92,6 +92,32 @@ def test_attention_over_stored_rows_matches_the_rotated_space_oracle(nq, nkv, hd
     assert worst <= 4e-3
 
 
+@pytest.mark.parametrize("hd,nq,m", [(64, 8, 5), (128, 8, 3), (64, 32, 9), (128, 32, 16)])   # one row tile, and several
+@pytest.mark.parametrize("blocks", [1, 7, 8, 32, 33, 256, 257, 288, 289, 545, 801])
+def test_waves_of_a_workgroup_with_unlike_numbers_of_blocks(hd, nq, m, blocks):
+    """Eight KV heads: up to 32 chunks of ceil(blocks / chunks) blocks of sixteen positions, dealt to the eight waves of a workgroup.  No block at all, one
+    for some of the waves, one or two, two or three, three or four, and chunks at the end that are short or empty: every wave comes to the
+    barrier behind which the tables of levels are there, and what a wave does not have is not added."""
+    from oracle import binding as ob
+    from turbospark_amd import ffi
+    nkv, kb, vb = 8, 3 + (blocks & 1), 4
+    base = max(16 * blocks - m - (blocks % 5), 0)
+    rng = np.random.default_rng(blocks * 31 + hd + m)
+    seq = base + m
+    q = rng.standard_normal((m, nq, hd), dtype=np.float32).astype(np.float16)
+    k, v = (rng.standard_normal((seq, nkv, hd), dtype=np.float32).astype(np.float16) for _ in range(2))
+    got, kr, vr = ffi.attention_quantized(q, k, v, base, kb, vb)
+    ks, kc, km, vs, vc, vm = _sides(hd, kb, vb)
+    # The matrix products take the levels as fp16, and so does the reference here: at 64 dimensions and four bits the levels' rounding has a mean of
+    # 8.5e-6, which the inverse transform collects in dimension 0 (8.5e-6 hd = 5.4e-4 of a row's norm, 6e-3 of the largest output where 4000 unlike
+    # rows average out), whatever the waves do.
+    kc, vc = (np.asarray(c, np.float32).astype(np.float16).astype(np.float32) for c in (kc, vc))
+    for i in sorted({0, m - 1}):
+        want = ob.tq_attention(q[i].astype(np.float32), kr[:, :, 1:], kr[:, :, 0].view(np.float32), vr[:, :, 1:],
+                               vr[:, :, 0].view(np.float32), hd, nq, nkv, base + i + 1, kb, ks, kc, vs, vc, v_bits=vb).reshape(nq, hd)
+        assert float(np.abs(got[i] - want).max() / np.abs(want).max()) <= 4e-3, i
+
+
 def _open(name, kv_bits, max_context=96, seed=21, **over):
     import turbospark_amd as ts
     from turbospark_amd import synth

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(512) void k_attn_partial_tq(AttnArgs a, int G, int 
                  "s"(a.blocks), "s"(a.xcd_groups), "s"(a.by_group.magic), "s"(a.by_chunks.magic), "s"(G), "s"(R));
     TqPairs<KB> kp(a.tq.k_cb, threadIdx.x);
     TqPairs<VB> vp(a.tq.v_cb, threadIdx.x);
-    // the tables are filled behind the first loads of the stores, one barrier for every wave
+    // the tables are filled behind the first loads of the stores
     auto tables = [&] {
         kp.put(s_kpair, threadIdx.x);
         vp.put(s_vpair, threadIdx.x);
