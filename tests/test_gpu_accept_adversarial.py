@@ -214,3 +214,48 @@ def test_truncation_cuts_at_the_edges_of_a_group_of_rank_bins(vocab, penalty):
             assert (res.next, res.draw_step) == (want["next"], want["draw_step"]), (kw, seed)
             compared += 1
     assert compared >= 3 * len(kws)
+
+
+def _seed_drawing(bits53, position):
+    """The seed whose uniform at `position` is bits53 2^-53: splitmix64's finaliser (crates/selection/src/derive.rs:19-45) undone step by step."""
+    mask = (1 << 64) - 1
+
+    def unshift(x, n):
+        y = x
+        for _ in range(64 // n + 1):
+            y = x ^ (y >> n)
+        return y
+    x = unshift(bits53 << 11, 31)
+    x = unshift(x * pow(0x94D049BB133111EB, -1, 1 << 64) & mask, 27)
+    x = unshift(x * pow(0xBF58476D1CE4E5B9, -1, 1 << 64) & mask, 30)
+    x = (x - 0x9E3779B97F4A7C15) & mask
+    return x ^ (position * 0x9E3779B97F4A7C15 & mask)
+
+
+@pytest.mark.parametrize("vocab", [37, 1000, 4096])
+@pytest.mark.parametrize("penalty", [None, 1.25])
+def test_draws_at_the_ends_of_the_uniform(vocab, penalty):
+    """The smallest and the largest uniforms there are.  At the largest ones the sums in fixed point and in doubles part by a rounding, no candidate's sum
+    passes the uniform and the draw takes the bin's last: plain draws and draws from a residual, against the oracle.  Rows whose last candidate carries mass enough that
+    rounding cannot decide between it and the one before."""
+    import turbospark_amd as ts
+    cfg, w, gpu, cpu = gc.build_pair("tiny_q8_0", max_context=64, vocab=vocab)
+    r = np.random.default_rng(9)
+    top = (1 << 53) - 1
+    for kind in ("flat", "two", "ties", "normal"):
+        row = _row(r, vocab, kind).astype(np.float16)
+        sure = int(np.argmin(row))                                       # the drafter proposes what the target least wants: refused
+        draft = np.full((1, vocab), -8.0, np.float16)
+        draft[0, sure] = 20.0
+        history = [int(t) for t in r.integers(0, vocab, 30)] if penalty else []
+        kw = dict(repetition_penalty=penalty) if penalty else {}
+        for bits in (0, 1, top - 1, top):
+            for feed, position in (([3], 0), ([3, sure], 1)):
+                seed = _seed_drawing(bits, position)
+                target = np.stack([row] * len(feed))
+                gpu.write_logits(target, 20)
+                res = gpu.accept(feed, 20, ts.shaping(1.0, seed=seed, **kw), draft_logits=draft, history=history)
+                want = ob.chain_round(target.view(np.uint16), draft.view(np.uint16)[:len(feed) - 1], np.asarray(feed[1:], np.int32),
+                                      ob.shaping(1.0, seed=seed, **kw), history=history)
+                assert (res.accepted, res.draw_step) == (want["accepted"], want["draw_step"])
+                assert res.next == want["next"], (kind, bits, feed)

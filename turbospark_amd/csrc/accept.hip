@@ -1338,6 +1338,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
             // the f64 walk and the fixed-point bin search disagreed by a rounding: the uniform
             // sits on a bin edge.  Take the bin's first (u below) or last candidate and report
             // a zero margin.
+            __syncthreads();  // (every wave has read that there is none)
             if (lastv >= 0) atomicMax(&s_token, lastv);
             __syncthreads();
             token = s_token;
