@@ -1148,7 +1148,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
     __shared__ unsigned long long wsum[16];
     __shared__ double dsum[16];
     __shared__ unsigned long long s_total, s_before;
-    __shared__ int s_bin, s_last_bin, s_token, s_fallback;
+    __shared__ int s_group, s_bin, s_last_bin, s_token, s_fallback;
     __shared__ double s_cum_before, s_cum_at;
     const AcceptParams& ap = *app;
     const int jobi = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1198,7 +1198,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
         }
         if (lane == 63) wsum[wave] = inc;
         if (tid == 0) {
-            s_bin = -1;
+            s_group = s_bin = -1;
             s_last_bin = -1;
             s_token = -1;
             s_fallback = 0;
@@ -1214,15 +1214,15 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
         const unsigned long long tgt = (unsigned long long)(dec.job.u * (double)total);
         if (loc > 0) atomicMax(&s_last_bin, tid * 64 + 63);
         if (excl <= tgt && tgt < excl + loc) {
-            s_bin = tid;  // the group that holds the target, for now
+            s_group = tid;
             s_before = excl;
         }
         if (tid == 0) s_total = total;
         __syncthreads();
-        if (s_bin >= 0) {
+        const int group = s_group;  // the group that holds the target (not written again: what comes next differs by it)
+        if (group >= 0) {
             // its first bin at which the running sum passes the target: a lane to a bin, every wave for itself
-            const int g = s_bin;
-            const unsigned long long mine = hsel[(g >> 6) * 4096 + (g & 63) + lane * 64], from = s_before;
+            const unsigned long long mine = hsel[(group >> 6) * 4096 + (group & 63) + lane * 64], from = s_before;
             unsigned long long upto = mine;
             for (int o = 1; o < 64; o <<= 1) {
                 const uint32_t lo = __shfl_up((uint32_t)upto, o), hi = __shfl_up((uint32_t)(upto >> 32), o);
@@ -1231,13 +1231,10 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
             const int hit = __builtin_ctzll(__ballot(tgt < from + upto));  // (the group's sum passes it)
             __syncthreads();
             if (tid == hit) {
-                s_bin = g * 64 + hit;
+                s_bin = group * 64 + hit;
                 s_before = from + upto - mine;
             }
-            __syncthreads();
-        }
-        int bin = s_bin;
-        if (bin < 0) {
+        } else {
             // rounding at the tail: the reference falls back to the LAST surviving candidate
             // (choose.rs:333-338).  Last occupied bin, last matching index.
             const int lb = s_last_bin;  // upper end of the last occupied 64-bin group
@@ -1248,9 +1245,9 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
                 s_before = total;
                 s_fallback = 1;
             }
-            __syncthreads();
-            bin = s_bin;
         }
+        __syncthreads();
+        const int bin = s_bin;
         const bool fallback = s_fallback != 0;
         const double norm = (double)s_total;  // fixed-point total <-> 1.0 (p mode) or R (residual)
         const double cum0 = (double)s_before / norm;  // cumulative mass before this bin
