@@ -66,8 +66,8 @@ struct tsv_ctx {
     int max_experts = 0;
     float* route_w = nullptr;
     int32_t* route_sel = nullptr;
-    MoeUnit* moe_units = nullptr;     // of the layer under way: TSV_MAX_ROWS * 8 places, then their count
-    int32_t* moe_n_units = nullptr;
+    MoeUnit* moe_units = nullptr;     // of the layer under way: TSV_MAX_ROWS * 8 places, nothing behind them
+    int32_t* moe_n_units = nullptr;   // how many of the places are taken: a buffer of its own
     int32_t* route_forced = nullptr;  // test hook (tsv_force_route): [n_layers][16][8], negative = route freely
     uint8_t* frag_e = nullptr;
     size_t frag_e_stride = 0;

@@ -290,7 +290,7 @@ __global__ __launch_bounds__(1024) void k_mtp_input(const uint8_t* __restrict__ 
     // The row and the norms' weights are asked for before the token is waited for, and the angles come last: one workgroup is all
     // there is at a single row, and what it costs is the round trips one behind the other (11.1 -> 10.5 us under a trace; 48 tokens of the loop 16107 -> 15742)
     const float* h = h_rows + (long)m * hidden;
-    // at most eight elements per thread (hidden <= 8192): kept in registers across the reductions
+    // J elements per thread, kept in registers across the reductions
     const float freq = freqs[min((int)threadIdx.x, half - 1)];
     float ev[J], hv[J], ge[J], gt[J], gh[J];
 #pragma unroll

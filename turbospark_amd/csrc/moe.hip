@@ -21,11 +21,10 @@ namespace {
 
 // ---- router ---------------------------------------------------------------------------------
 // One workgroup, one wave per row: the row's logits (split-K partials summed in order) sit
-// 'ne / 64' per lane as order-preserving integer keys; k rounds of two wave-wide reductions on the
-// DPP network (the largest key, then the lowest index that holds it: larger logit, then lower
-// index) pick the experts in rank order.  Then one thread per (row, slot) pair finds the first
-// pair that chose its expert -- the group's leader -- and its own place among that group's
-// members, which are listed in pair order.
+// 'ne / 64' per lane as order-preserving integer keys; k rounds of a wave-wide maximum on the
+// DPP network and a ballot of the lanes that hold it, whose lowest index is taken (larger logit, then lower
+// index), pick the experts in rank order (route_row).  Then the waves list the pass's units, four rows of an expert each, in
+// the order of the pairs that name an expert first (list_units); a prompt pass lists its experts' members in a launch of its own.
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ uint32_t dpp_from(uint32_t v) {  // a lane without a source keeps its own value
     return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW_MASK, 0xf, false);

@@ -332,7 +332,7 @@ struct MoeRouteArgs {
     // selections of block b follow those of block b - 1; no forced routing
     int blocks;
     long logits_block_stride;
-    // nullable: the pass's units, and behind their m * top_k places how many there are
+    // nullable: the pass's units (at most m * top_k), and in a buffer of its own how many there are
     MoeUnit* units;
     int32_t* n_units;
 };
