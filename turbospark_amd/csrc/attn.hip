@@ -42,7 +42,7 @@ __global__ __launch_bounds__(512) void k_attn_partial(AttnArgs a, int G, int R) 
     extern __shared__ float xch[];  // [8 slots][PER_LANE values][64 lanes]
     ask_for_arguments(a, G, R);
     const AttnArgs v = a.blocks > 1 ? attn_block_view(a, blockIdx.z) : a;
-    attn_partial_body<HD, RT, STAGES, false>(v, G, R, blockIdx.x, blockIdx.y, 0, xch);
+    attn_partial_body<HD, RT, STAGES>(v, G, R, blockIdx.x, blockIdx.y, 0, xch);
 }
 
 // A pass of more than two row tiles: TG tile groups side by side in one workgroup (attn_core.h), one read of the
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64 * TG * attn_phases(TG)) void k_attn_partial_grou
     extern __shared__ float xch[];
     ask_for_arguments(a, G, R);
     const AttnArgs v = a.blocks > 1 ? attn_block_view(a, blockIdx.z) : a;
-    attn_partial_body<HD, RT, STAGES, false, TG>(v, G, R, blockIdx.x, blockIdx.y, 0, xch);
+    attn_partial_body<HD, RT, STAGES, TG>(v, G, R, blockIdx.x, blockIdx.y, 0, xch);
 }
 
 // A short context (launch_hd): one workgroup per KV head and row group, which finishes its rows
@@ -60,7 +60,7 @@ template <int HD, int RT, int STAGES>
 __global__ __launch_bounds__(512) void k_attn_direct(AttnArgs a, int G, int R) {
     extern __shared__ float xch[];
     ask_for_arguments(a, G, R);
-    attn_partial_body<HD, RT, STAGES, false, 1, true>(a, G, R, 0, blockIdx.y, blockIdx.z * RT, xch);
+    attn_partial_body<HD, RT, STAGES, 1, true>(a, G, R, 0, blockIdx.y, blockIdx.z * RT, xch);
 }
 
 // The same pass over a layer that keeps quantized rows (attn_tq_core.h)

@@ -134,8 +134,6 @@ __device__ __forceinline__ float max_over_position_groups(float v) {
 // chunk, NW = attn_phases(TG), starting at block w / TG, with up to STAGES blocks of K and V in flight.  The waves of
 // different groups that walk the same blocks run side by side on one compute unit, so a block comes out of the L2
 // once for all (row, q head) pairs of the pass.  (Legacy callers pass TG = 1 and their own rt0: eight waves, one group.)
-// COH: the query rows and the K / V blocks are read device-coherently (sc1), for a caller whose
-// other compute units wrote them earlier in the same kernel.
 // DIRECT: the only chunk of a short context (attn.hip, launch_hd), whose rows are finished here.  The weights go into the value product as
 // two fp16 terms, through the matrix instruction of twice the depth, which takes the value operand twice and no longer than the other.
 // Rounded to fp16, only the weight that the reference was taken from is exact: one of each block's while every wave has one block, as in
@@ -145,13 +143,12 @@ __device__ __forceinline__ float max_over_position_groups(float v) {
 // xch: [TG][NW slots][PER_LANE values][64 lanes] floats of LDS.
 __host__ __device__ constexpr int attn_phases(int tg) { return tg == 1 ? 8 : tg == 2 ? 4 : 2; }
 
-template <int HD, int RT, int STAGES, bool COH, int TG = 1, bool DIRECT = false>
+template <int HD, int RT, int STAGES, int TG = 1, bool DIRECT = false>
 __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int R, int chunk, int h, int rt_first, float* xch) {
     constexpr int NW = attn_phases(TG);
     constexpr int KS = HD / 32;  // K steps of the score MFMA
     constexpr int VT = HD / 16;  // output tiles along head_dim
     constexpr int PER_LANE = RT * VT * 4 + 2 * RT;
-    constexpr int POLICY = COH ? 16 : 0;  // buffer-load cache policy: sc1
 
     // (the wave index as a scalar: everything derived from it -- block numbers, the choice of variant -- then stays
     // on the scalar unit)
@@ -189,16 +186,8 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
         const uint32_t anc_row = vp->anc[mrow];
         const int pos_row = vp->pos[mrow];
         const _Float16* q = (const _Float16*)a.q16 + ((long)mrow * a.nq + h * G + g) * HD + 8 * kg;
-        if (COH) {
-            const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc((void*)a.q16, 0, 0x7FFFFFFF, 0x00027000);
-            const uint32_t qo = (uint32_t)((const char*)q - (const char*)a.q16);
 #pragma unroll
-            for (int s = 0; s < KS; s++)
-                qf[t][s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qrs, qo + 64 * s, 0, 16));
-        } else {
-#pragma unroll
-            for (int s = 0; s < KS; s++) qf[t][s] = *(const uint4*)(q + 32 * s);
-        }
+        for (int s = 0; s < KS; s++) qf[t][s] = *(const uint4*)(q + 32 * s);
         // taken as loaded (for a lane past the end: pair 0's), and not touched before the first K / V loads are out
         anc[t] = anc_row;
         lo[t] = pos_row;
@@ -235,9 +224,9 @@ __device__ __forceinline__ void attn_partial_body(const AttnArgs& a, int G, int 
         const uint32_t bo = (uint32_t)(ring ? blk % nbc : blk) * blk_bytes;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < KS; s++) st.kf[s] = __builtin_amdgcn_raw_buffer_load_b128(krs, bo + loff + 1024 * s, 0, POLICY);
+        for (int s = 0; s < KS; s++) st.kf[s] = __builtin_amdgcn_raw_buffer_load_b128(krs, bo + loff + 1024 * s, 0, 0);
 #pragma unroll
-        for (int u = 0; u < VT / 2; u++) st.vf[u] = __builtin_amdgcn_raw_buffer_load_b128(vrs, bo + loff + 1024 * u, 0, POLICY);
+        for (int u = 0; u < VT / 2; u++) st.vf[u] = __builtin_amdgcn_raw_buffer_load_b128(vrs, bo + loff + 1024 * u, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
     // Scores are kept in units of log 2 (one multiply by scale * log2(e), then v_exp_f32 as it is), and a block that

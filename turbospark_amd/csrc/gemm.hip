@@ -349,7 +349,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split
     // outstanding tile only (s_waitcnt vmcnt(n)) instead of draining the queue.
     if (nc > 0) {
         Stage<F, NG> st[STAGES];
-        const ActLoader<false> x(a.xfrag, a.xsum, lane);
+        const ActLoader x(a.xfrag, a.xsum, lane);
         const int last = c0 + nc - 1;
         auto fetch = [&](Stage<F, NG>& sg, int c) { load_tile(sg, x, wt + (size_t)c * F::TILE_BYTES, c, lane); };
 #pragma unroll

@@ -1,6 +1,6 @@
 // Device-side core of the dequant-fused small-M matmul: weight-tile formats, the register stage
-// of the software pipeline, and the per-tile MFMA sequences.  Shared by the stand-alone matmul
-// kernel and the fused per-XCD layer kernels.
+// of the software pipeline, and the per-tile MFMA sequences.  Shared by the dense and the expert
+// matmul kernels.
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -52,34 +52,6 @@ struct Consts {
     uint32_t k6400, k5400, k64;
 };
 
-typedef __attribute__((address_space(3))) void* lds_ptr;
-
-// 32-bit LDS address of a generic pointer into shared memory
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
-}
-
-// One wave-wide global -> LDS transfer, 16 (or 4) bytes per lane to lds + lane * size, done by the
-// memory pipeline without passing through registers; vmcnt counts it like a load.  Written as
-// inline assembly on purpose: the compiler then neither sees an LDS write (it would otherwise
-// drain the whole load queue before the next LDS access) nor counts the transfer, which only
-// makes its own s_waitcnt values wait for a few more, older, operations.  Readers of the
-// buffer order themselves after a later load with lds_after().
-__device__ __forceinline__ void dma_to_lds_b128(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g) : "memory");
-}
-__device__ __forceinline__ void dma_to_lds_b32(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g) : "memory");
-}
-// An LDS address the compiler believes to depend on `loaded`, a register filled by a load that
-// was issued after the transfers into that buffer: loads complete in issue order, so once the
-// compiler has waited for `loaded`, the buffer is complete, and no read through the returned
-// address can be scheduled before that wait.
-__device__ __forceinline__ uint32_t lds_after(uint32_t lds, float loaded) {
-    asm volatile("" : "+v"(lds) : "v"(loaded));
-    return lds;
-}
-
 // A tile's units are asked for in the order in which they are multiplied: loads come back in order, so the first products do not wait for
 // the last unit.  (Left to itself the scheduler puts those that share an address register together.)
 template <class T>
@@ -102,12 +74,6 @@ struct Q4K {
 #pragma unroll
         for (int u = 0; u < 8; u++) load_in_order(r.q[u], p + u * 64);
         r.s = __builtin_nontemporal_load(p + 512);
-    }
-    // the same tile copied byte for byte into LDS by the memory pipeline (no registers involved);
-    // completion is counted by vmcnt like any other load
-    static __device__ __forceinline__ void load_to_lds(uint32_t lds, const uint8_t* tile, int lane) {
-#pragma unroll
-        for (int u = 0; u < 9; u++) dma_to_lds_b128(tile + u * 1024 + lane * 16, lds + u * 1024);
     }
     // float index of the sub-block sums of chunk c, and this lane's place in them before the row's own offset
     // (ActLoader::sumoff) is added: lane (b, i) reads sub-block b
@@ -150,13 +116,6 @@ struct Q80 {
         for (int u = 0; u < 8; u++) load_in_order(r.q[u], p + u * 64);
         r.s = __builtin_nontemporal_load((const u32x2*)(tile + 8192) + lane);
     }
-    static __device__ __forceinline__ void load_to_lds(uint32_t lds, const uint8_t* tile, int lane) {
-#pragma unroll
-        for (int u = 0; u < 8; u++) dma_to_lds_b128(tile + u * 1024 + lane * 16, lds + u * 1024);
-        // the 512-byte scale block: 8 bytes per lane, as two 4-byte transfers of 256 bytes
-#pragma unroll
-        for (int h = 0; h < 2; h++) dma_to_lds_b32(tile + 8192 + h * 256 + lane * 4, lds + 8192 + h * 256);
-    }
     // a 128-element chunk is half of a 256-element sum group: its four sub-blocks go to blocks 0..3
     static __device__ __forceinline__ int xs_base(int c) { return (c >> 1) * 128 + (c & 1) * 16; }
     static __device__ __forceinline__ int xs_lane(int lane) { return ((lane >> 2) & 3) * 4; }
@@ -175,9 +134,6 @@ struct MX4 {
     static constexpr bool SUMS = false;
     typedef Q80::Regs Regs;
     static __device__ __forceinline__ void load(Regs& r, const uint8_t* tile, int lane) { Q80::load(r, tile, lane); }
-    static __device__ __forceinline__ void load_to_lds(uint32_t lds, const uint8_t* tile, int lane) {
-        Q80::load_to_lds(lds, tile, lane);
-    }
     static __device__ __forceinline__ int xs_base(int c) { return Q4K::xs_base(c); }
     static __device__ __forceinline__ int xs_lane(int lane) { return Q4K::xs_lane(lane); }
 };
@@ -244,8 +200,7 @@ struct Stage {
     XRegs<F, NG> x;
 };
 
-// Where a tile's bytes are read from while it is being multiplied: the registers of a stage, or
-// the LDS copy made by load_to_lds (16 bytes per lane and unit, read just before use).
+// Where a tile's bytes are read from while it is being multiplied: the registers of a stage.
 template <class F>
 struct RegSrc {
     const typename F::Regs& r;
@@ -254,26 +209,9 @@ struct RegSrc {
     __device__ __forceinline__ auto dval() const { return r.d; }
     __device__ __forceinline__ u32x4 high(int u) const { return r.h[u]; }
 };
-template <class F>
-struct LdsSrc {
-    uint32_t base;  // LDS address (see lds_after)
-    int lane;
-    typedef decltype(typename F::Regs{}.s) Scales;
-    __device__ __forceinline__ u32x4 unit(int u) const {
-        return *(__attribute__((address_space(3))) const u32x4*)(uintptr_t)(base + (u * 64 + lane) * 16);
-    }
-    __device__ __forceinline__ Scales scales() const {
-        return *(__attribute__((address_space(3))) const Scales*)(uintptr_t)(base + 8192 + lane * sizeof(Scales));
-    }
-};
-
-// Cache policy of the activation loads: plain, or device-coherent (sc1) for activations that
-// another compute unit wrote earlier in the same kernel (they must not come from this CU's L1).
-// Which activation row feeds slot (g, i) of the MFMA A operand is a per-lane offset table: the
+// The activation loads.  Which activation row feeds slot (g, i) of the MFMA A operand is a per-lane offset table: the
 // identity for a dense matmul, a gather for a routed expert that sees only its own rows.
-template <bool COHERENT>
 struct ActLoader {
-    __amdgpu_buffer_rsrc_t frag, sums;
     const u32x2* fragp;
     const float* sump;
     int rowoff[4], sumoff[4];  // offsets of row group g's row for this lane, in 8-byte units / floats
@@ -292,25 +230,19 @@ struct ActLoader {
         sump = (const float*)xsum;
 #pragma unroll
         for (int g = 0; g < 4; g++) set_row(g, 4 * g + (lane & 3));
-        if (COHERENT) {
-            frag = __builtin_amdgcn_make_buffer_rsrc((void*)xfrag, 0, 0x7FFFFFFF, 0x00027000);
-            sums = __builtin_amdgcn_make_buffer_rsrc((void*)xsum, 0, 0x7FFFFFFF, 0x00027000);
-        }
     }
     // fragment `lane_at` (in 8-byte units) behind unit `at`, which is the same for a wave: its share of the address stays on the scalar unit
     __device__ __forceinline__ u32x2 frag_at(int at, int lane_at) const {
-        if (COHERENT) return __builtin_amdgcn_raw_buffer_load_b64(frag, (at + lane_at) * 8, 0, 16);
         return *(const u32x2*)((const char*)(fragp + at) + (uint32_t)(lane_at * 8));
     }
     __device__ __forceinline__ float sum_at(int at, int lane_at) const {
-        if (COHERENT) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sums, (at + lane_at) * 4, 0, 16));
         return *(const float*)((const char*)(sump + at) + (uint32_t)(lane_at * 4));
     }
 };
 
 // activations of K chunk c (chunk index in the activation's own K axis)
-template <class F, int NG, bool COH>
-__device__ __forceinline__ void load_x(XRegs<F, NG>& xr, const ActLoader<COH>& x, int c, int lane) {
+template <class F, int NG>
+__device__ __forceinline__ void load_x(XRegs<F, NG>& xr, const ActLoader& x, int c, int lane) {
 #pragma unroll
     for (int p = 0; p < F::NPAIR; p++)
 #pragma unroll
@@ -323,8 +255,8 @@ __device__ __forceinline__ void load_x(XRegs<F, NG>& xr, const ActLoader<COH>& x
 
 // The loads of one stage stay together and in program order (scheduling fences on both sides),
 // so "stage s has landed" is one s_waitcnt vmcnt(n) with the same n on every path.
-template <class F, int NG, bool COH>
-__device__ __forceinline__ void load_stage(Stage<F, NG>& st, const ActLoader<COH>& x, const uint8_t* tile_chunk, int c,
+template <class F, int NG>
+__device__ __forceinline__ void load_stage(Stage<F, NG>& st, const ActLoader& x, const uint8_t* tile_chunk, int c,
                                            int lane) {
     __builtin_amdgcn_sched_barrier(0);
     load_x(st.x, x, c, lane);
@@ -638,8 +570,8 @@ __device__ __forceinline__ void compute(const Stage<F, NG>& st, const Consts& k,
 
 // Part u of a tile and of its activations: -1 the scales and the sums, else what is multiplied behind them, one after the other.  Loads come
 // back in this order.
-template <class F, int NG, bool COH>
-__device__ __forceinline__ void load_part(Stage<F, NG>& st, const ActLoader<COH>& x, const uint8_t* tile_chunk, int c, int lane, int u) {
+template <class F, int NG>
+__device__ __forceinline__ void load_part(Stage<F, NG>& st, const ActLoader& x, const uint8_t* tile_chunk, int c, int lane, int u) {
     const u32x4* p = (const u32x4*)tile_chunk + lane;
     constexpr bool Q6 = std::is_same<F, Q6K>::value, Q4 = std::is_same<F, Q4K>::value;
     constexpr int UNITS = Q6 ? 3 : std::is_same<F, Q80>::value ? 4 : 2;  // of a part
@@ -665,8 +597,8 @@ __device__ __forceinline__ void load_part(Stage<F, NG>& st, const ActLoader<COH>
     }
     __builtin_amdgcn_sched_barrier(0);
 }
-template <class F, int NG, bool COH>
-__device__ __forceinline__ void load_tile(Stage<F, NG>& st, const ActLoader<COH>& x, const uint8_t* tile_chunk, int c, int lane) {
+template <class F, int NG>
+__device__ __forceinline__ void load_tile(Stage<F, NG>& st, const ActLoader& x, const uint8_t* tile_chunk, int c, int lane) {
     if constexpr (F::PARTS) {
 #pragma unroll
         for (int u = -1; u < F::PARTS; u++) load_part(st, x, tile_chunk, c, lane, u);
@@ -675,8 +607,8 @@ __device__ __forceinline__ void load_tile(Stage<F, NG>& st, const ActLoader<COH>
 // Multiplies a tile and asks for the next one, its parts as this one's come free: the first of them are on their way for the rest of the products,
 // in the same registers.  (All of it behind the last product, five rows through 32 layers of the 8B shape in Q4_K took 1938 us for 1900, one row at a time
 // through the Q4_K_M mix 3874 for 3746, six rows of eight Q8_0 layers 687 for 660, nine through routed MXFP4 layers 1018 for 993 and 768 for 752.)
-template <class F, int NG, bool COH>
-__device__ __forceinline__ void compute_and_load(Stage<F, NG>& st, const Consts& k, float4v (&acc)[NG], const ActLoader<COH>& x, const uint8_t* tile_chunk,
+template <class F, int NG>
+__device__ __forceinline__ void compute_and_load(Stage<F, NG>& st, const Consts& k, float4v (&acc)[NG], const ActLoader& x, const uint8_t* tile_chunk,
                                                  int c, int lane) {
     if constexpr (F::PARTS) {
         const Stage<F, NG> now = st;

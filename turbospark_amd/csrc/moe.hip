@@ -30,7 +30,7 @@ __device__ __forceinline__ uint32_t dpp_from(uint32_t v) {  // a lane without a 
     return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW_MASK, 0xf, false);
 }
 // quad swaps, shifts by four and eight inside a row of sixteen, then the rows' last lanes handed
-// on to the next row(s): lane 63 ends up with the reduction of all 64 (max and min are idempotent,
+// on to the next row(s): lane 63 ends up with the reduction of all 64 (max is idempotent,
 // so lanes that see a value twice do no harm)
 __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
     v = max(v, dpp_from<0xb1, 0xf>(v));
@@ -39,15 +39,6 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
     v = max(v, dpp_from<0x118, 0xf>(v));
     v = max(v, dpp_from<0x142, 0xa>(v));
     v = max(v, dpp_from<0x143, 0xc>(v));
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-__device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
-    v = min(v, dpp_from<0xb1, 0xf>(v));
-    v = min(v, dpp_from<0x4e, 0xf>(v));
-    v = min(v, dpp_from<0x114, 0xf>(v));
-    v = min(v, dpp_from<0x118, 0xf>(v));
-    v = min(v, dpp_from<0x142, 0xa>(v));
-    v = min(v, dpp_from<0x143, 0xc>(v));
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 // float -> unsigned key with the same order (-0 is folded into +0 first, so equal floats have equal
@@ -244,7 +235,7 @@ __device__ __forceinline__ void expert_tile(const MoeGemmArgs& a, const MoeGroup
     // activation operand: gate/up gathers the pass's rows this expert was chosen by; down reads
     // the group's own buffer, whose rows are already in the group's order
     const uint8_t* xbase = (const uint8_t*)a.xfrag + (EPI == EPI_SLOT ? (size_t)gi * a.x_stride : 0);
-    ActLoader<false> x(xbase, xbase + xfrag_sum_offset(a.k), lane);
+    ActLoader x(xbase, xbase + xfrag_sum_offset(a.k), lane);
 #pragma unroll
     for (int g = 0; g < NG; g++) {
         const int mine = min(r0 + 4 * g + (lane & 3), cnt - 1);
@@ -362,7 +353,7 @@ __global__ __launch_bounds__(512) void k_moe_gemm(MoeGemmArgs a) {
     asm volatile("" : "+v"(k.k6400), "+v"(k.k5400), "+v"(k.k64));
     // activation operand: gate/up gathers the pass's rows, down reads the unit's own buffer
     const uint8_t* xbase = (const uint8_t*)a.xfrag + (EPI == EPI_SLOT ? (size_t)unit * a.x_stride : 0);
-    ActLoader<false> x(xbase, xbase + xfrag_sum_offset(a.k), lane);
+    ActLoader x(xbase, xbase + xfrag_sum_offset(a.k), lane);
     const int i4 = lane & 3;
     x.set_row(0, EPI == EPI_SLOT ? min(i4, cnt - 1) : i4 < 2 ? (i4 ? row[1] : row[0]) : (i4 == 2 ? row[2] : row[3]));
 

@@ -95,7 +95,7 @@ inline int fmt_chunk_elems(int fmt) { return fmt == FMT_Q80 ? 128 : fmt == FMT_B
 inline int fmt_tile_bytes(int fmt) {
     return fmt == FMT_Q4K ? 9216 : fmt == FMT_Q5K ? 11264 : fmt == FMT_BF16 ? 8192 : fmt == FMT_Q6K ? 13568 : 8704;
 }
-inline int fmt_nsub(int fmt) { return fmt == FMT_Q80 ? 4 : fmt == FMT_BF16 ? 2 : fmt == FMT_Q6K ? 16 : 8; }
+
 constexpr int TILE_ROWS = 64;
 
 // An fp16 activation on its way to both the fragment store and the sub-block sum.  The matmuls multiply
