@@ -147,6 +147,18 @@ def test_both_sides_of_the_line_of_short_contexts(nq, nkv, hd, m, end, window):
     assert np.abs(got - want).max() <= 5e-3 * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(7, 7, 64), (12, 6, 128), (10, 5, 64), (32, 4, 128), (4, 1, 64)])   # 36, 42, 51 and 64 chunks
+@pytest.mark.parametrize("m,base", [(1, 560), (1, 1031), (2, 510), (2, 2600)])
+def test_merge_of_more_than_thirty_two_chunks(nq, nkv, hd, m, base):
+    """Counts on both sides of a batch of 32 chunks' end, contexts that leave the last chunks without a position, and long ones."""
+    from turbospark_amd import ffi
+    q, k, v = _rand(m, nq, nkv, hd, base, 7 * base + nkv)
+    sinks = np.random.default_rng(nkv).standard_normal(nq).astype(np.float32) if base % 2 else None
+    got = ffi.attention(q, k, v, base, sinks=sinks)
+    want = _oracle(q, k, v, base, None, sinks=sinks)
+    assert np.abs(got - want).max() <= 5e-3 * max(1.0, np.abs(want).max())
+
+
 @pytest.mark.parametrize("seed", range(64))
 def test_random_attention_shapes_and_long_contexts(seed):
     """Seeded sweep: head width, GQA group 1..8, 1..16 rows, chain or random tree, contexts up to 20000

@@ -102,7 +102,9 @@ __global__ __launch_bounds__(512) void k_attn_partial_tq(AttnArgs a, int G, int 
 // of 32 chunks took 3.4 us in the 8B step).
 // NCH > 0: the chunk count as a compile-time constant -- every thread then asks for its output
 // element of all chunks before the (m, l) pairs are looked at (the two groups of loads do not
-// depend on each other), and the kernel is one memory latency instead of two.  NCH == 0: any count.
+// depend on each other), and the kernel is one memory latency instead of two.  NCH == 0: any count, the first 32 chunks that
+// way, then 32 more at a time.  (A loop over chunks is not unrolled here whatever a pragma asks, because it reads lanes: with
+// a round trip for each of 64 chunks the merge of one row of 32 heads took 17.5 us.)
 template <int NCH, bool UNROT>
 __global__ __launch_bounds__(128) void k_attn_combine(AttnArgs a0, int G, int R) {
     asm volatile("" ::"s"(a0.part_o), "s"(a0.part_ml), "s"(a0.xfrag), "s"(a0.nq), "s"(a0.hd), "s"(a0.nch), "s"(a0.sinks), "s"(a0.frag16), "s"(a0.unrot),
@@ -117,9 +119,10 @@ __global__ __launch_bounds__(128) void k_attn_combine(AttnArgs a0, int G, int R)
     auto element = [&](int c) { return *(const float*)((const char*)(po + c * stride) + (uint32_t)(t * 4)); };
     // (a lane past the last chunk: the last chunk's pair, not used)
     const float2 ml = *(const float2*)(a.part_ml + (slot0 + (long)min(lane, nch - 1) * R) * 2);
-    float pre[NCH > 0 ? NCH : 1];
+    constexpr int BATCH = NCH > 0 ? NCH : 32;
+    float pre[BATCH];
 #pragma unroll
-    for (int c = 0; c < NCH; c++) pre[c] = element(c);
+    for (int c = 0; c < BATCH; c++) pre[c] = element(NCH > 0 ? c : min(c, nch - 1));
     const float sink = a.sinks ? uniform_memory(a.sinks)[qh] : -INFINITY;
     const float sign = UNROT ? a.unrot[t] : 1.0f;
     const bool live = lane < nch;
@@ -132,13 +135,17 @@ __global__ __launch_bounds__(128) void k_attn_combine(AttnArgs a0, int G, int R)
     if (a.sinks) den += __expf(sink - mx);
     auto weight = [&](int c) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), c)); };
     float num = 0.f;
-    if (NCH > 0) {
 #pragma unroll
-        for (int c = 0; c < NCH; c++) num = fmaf(weight(c), pre[c], num);
-    } else {
-#pragma unroll 8
-        for (int c = 0; c < nch; c++) num = fmaf(weight(c), element(c), num);
-    }
+    for (int c = 0; c < BATCH; c++)
+        if (NCH > 0 || c < nch) num = fmaf(weight(c), pre[c], num);
+    if (NCH == 0)
+        for (int c0 = BATCH; c0 < nch; c0 += BATCH) {
+#pragma unroll
+            for (int c = 0; c < BATCH; c++) pre[c] = element(min(c0 + c, nch - 1));
+#pragma unroll
+            for (int c = 0; c < BATCH; c++)
+                if (c0 + c < nch) num = fmaf(weight(c0 + c), pre[c], num);
+        }
     float res = num / den;
     if (UNROT) {
         // the sum was taken over rotated value rows: back through the normalized Hadamard transform
