@@ -81,6 +81,18 @@ def test_the_chosen_parts_of_k_are_as_near_to_64_bits_as_any(rows, cols):
     assert rms[0] <= 1.25 * min(rms.values()), rms
 
 
+@pytest.mark.parametrize("rows,cols,splits", [(64, 128, 1), (64, 1024, 1), (200, 1024, 2), (64, 1152, 1), (4096, 3968, 1), (4096, 4096, 4), (4096, 4224, 5)])
+def test_q8_0_rows_keep_their_bits_with_one_tile_or_more_to_a_wave(rows, cols, splits):
+    """One tile to a wave up to 2048 in all, in at most eight waves of a part; two from there on.  Up to four rows a wave of several
+    has two in flight, five rows never: the same sums."""
+    from turbospark_amd import ffi
+    entry, x, x16, want = _case(8, rows, cols, rows + cols)
+    five = ffi.matmul(entry, x[:5], splits=splits)
+    assert np.abs(five - want[:5]).max() <= np.abs(want).max() * 2e-4 + 1e-5
+    for m in (1, 3, 4):
+        assert np.array_equal(ffi.matmul(entry, x[:m], splits=splits), five[:m]), m
+
+
 def test_q4k_hand_packed_superblock_through_the_kernel(golden):
     """The reference's literal superblock (quant_gguf.rs:226-267) as a 16-row weight matrix:
     one-hot activations read the decoded weights back out of the kernel."""

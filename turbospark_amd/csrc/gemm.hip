@@ -316,16 +316,15 @@ __device__ __forceinline__ void epilogue(const GemmArgs& a, int tile, int split,
 // that hides more latency than a second register stage does -- the 8B step with two 2137 us for 2019, one row at a time 3950 for
 // 3882, nine rows through routed layers 1073 for 1044.  Two where they fit 128 VGPRs as well (108 to 118): Q8_0 with up to four rows,
 // eight 8B layers 657 and 671 -> 643 and 662 us with four, 2722 and 2783 -> 2656 and 2695 for four rows one by one.  (bf16, 86 to 112 with up to eight rows,
-// times the same both ways.)
+// times the same both ways.)  A wave with one tile to walk has no second one: two stages ask for the one twice (launch_t).
 template <class F, int NG>
 constexpr int gemm_stages() {
     return std::is_same<F, Q80>::value && NG == 1 ? 2 : 1;
 }
 
 // out_tile: the tile's number in the output (a matrix whose rows follow another's)
-template <class F, int EPI, int NG>
+template <class F, int EPI, int NG, int STAGES = gemm_stages<F, NG>()>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int tile, int split, int out_tile, float4v* red) {
-    constexpr int STAGES = gemm_stages<F, NG>();
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // this wave's run of chunks inside the workgroup's K slice
     const int s0 = split * a.kslice, s1 = min(s0 + a.kslice, a.kchunks);
@@ -399,6 +398,14 @@ __global__ __launch_bounds__(512) void k_gemm(GemmArgs a) {
     ask_for_arguments<EPI>(a);
     const int tile = a.by_splits.quotient(blockIdx.x), split = blockIdx.x - tile * a.splits;
     gemm_tile<F, EPI, NG>(a, tile, split, tile, red);
+}
+// ... where a wave has one tile to walk and k_gemm would have two in flight
+template <class F, int EPI, int NG>
+__global__ __launch_bounds__(512) void k_gemm_one(GemmArgs a) {
+    extern __shared__ float4v red[];
+    ask_for_arguments<EPI>(a);
+    const int tile = a.by_splits.quotient(blockIdx.x), split = blockIdx.x - tile * a.splits;
+    gemm_tile<F, EPI, NG, 1>(a, tile, split, tile, red);
 }
 
 // ------------------------------------------------------------------------------- nine to sixteen rows
@@ -1225,7 +1232,15 @@ int gemm_default_splits(const TiledW& w, int) {
 template <class F, int EPI, int NG>
 static int launch_t(hipStream_t s, const GemmArgs& a) {
     const size_t lds = a.kparts > 1 ? (size_t)a.kparts * NG * 1024 : 0;
-    hipLaunchKernelGGL((k_gemm<F, EPI, NG>), dim3(a.n_tiles * a.splits), dim3(64 * a.kparts), lds, s, a);
+    const dim3 grid(a.n_tiles * a.splits), block(64 * a.kparts);
+    if constexpr (gemm_stages<F, NG>() > 1) {
+        if (a.per == 1) {
+            hipLaunchKernelGGL((k_gemm_one<F, EPI, NG>), grid, block, lds, s, a);
+            TSV_HIP(hipGetLastError());
+            return TSV_OK;
+        }
+    }
+    hipLaunchKernelGGL((k_gemm<F, EPI, NG>), grid, block, lds, s, a);
     TSV_HIP(hipGetLastError());
     return TSV_OK;
 }
