@@ -96,8 +96,8 @@ def test_attention_over_stored_rows_matches_the_rotated_space_oracle(nq, nkv, hd
 @pytest.mark.parametrize("blocks", [1, 7, 8, 32, 33, 256, 257, 288, 289, 545, 801])
 def test_waves_of_a_workgroup_with_unlike_numbers_of_blocks(hd, nq, m, blocks):
     """Eight KV heads: up to 32 chunks of ceil(blocks / chunks) blocks of sixteen positions, dealt to the eight waves of a workgroup.  No block at all, one
-    for some of the waves, one or two, two or three, three or four, and chunks at the end that are short or empty: every wave comes to the
-    barrier behind which the tables of levels are there, and what a wave does not have is not added."""
+    for some of the waves, one or two, two or three, three or four, and chunks at the end that are short or empty: each number of blocks has a walk of its
+    own, behind the one barrier at which the tables of levels are there, and what a wave does not have is not added."""
     from oracle import binding as ob
     from turbospark_amd import ffi
     nkv, kb, vb = 8, 3 + (blocks & 1), 4

@@ -73,12 +73,12 @@ __global__ __launch_bounds__(512) void k_attn_partial_tq(AttnArgs a, int G, int 
                  "s"(a.blocks), "s"(a.xcd_groups), "s"(a.by_group.magic), "s"(a.by_chunks.magic), "s"(G), "s"(R));
     TqPairs<KB> kp(a.tq.k_cb, threadIdx.x);
     TqPairs<VB> vp(a.tq.v_cb, threadIdx.x);
-    // the tables are filled behind the first loads of the stores
-    auto tables = [&] {
-        kp.put(s_kpair, threadIdx.x);
-        vp.put(s_vpair, threadIdx.x);
-        __syncthreads();
-    };
+    // The tables are filled ahead of everything that differs between the waves: how many blocks a wave has chooses its walk, and no barrier may stand in one.
+    // (Behind the first blocks' loads all waves had to share one walk, whose loads stood under tail conditions: one, four and sixteen rows over 6001
+    // positions 7.9, 8.9 and 16.2 us for 6.8, 7.7 and 14.1; 3-bit and 2-bit keys, four rows over 12000, 13.1 and 11.5 for 11.4 and 9.9.)
+    kp.put(s_kpair, threadIdx.x);
+    vp.put(s_vpair, threadIdx.x);
+    __syncthreads();
     // blocks in flight: three, two where the three-bit fields' extra words would push the registers past 256
     constexpr int STAGES = (HD == 128 && RT == 2 && KB == 3 && VB == 3) ? 2 : 3;
     // several row groups of a verify pass are placed by die; else grid z: row groups of the pass, times the 16-row blocks of a prompt pass
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(512) void k_attn_partial_tq(AttnArgs a, int G, int 
         grp = blockIdx.z - blk * groups;
     }
     const AttnArgs v = a.blocks > 1 ? attn_block_view(a, blk) : a;
-    attn_partial_body_tq<HD, RT, STAGES, KB, VB>(v, G, R, chunk, kvh, grp * RT, xch, s_kpair, s_vpair, tables);
+    attn_partial_body_tq<HD, RT, STAGES, KB, VB>(v, G, R, chunk, kvh, grp * RT, xch, s_kpair, s_vpair);
 }
 
 // Merge the chunk partials (crates/gpu/src/shaders/attention.metal:122-140 semantics:

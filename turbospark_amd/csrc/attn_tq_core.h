@@ -35,7 +35,7 @@ __device__ __forceinline__ void tq_fill_pairs(uint32_t* table, const float* cb, 
     }
 }
 
-// ... by 512 threads, in two steps: the levels asked for, the table written
+// ... by 512 threads, in two steps: the levels asked for (ahead of the arguments' wait), the table written
 template <int BITS>
 struct TqPairs {
     static_assert(1 << (2 * BITS) <= 512, "an entry to a thread");
@@ -47,10 +47,10 @@ struct TqPairs {
     }
 };
 
-// xch: [8 slots][PER_LANE values][64 lanes] floats of LDS; kpair / vpair: the two pair tables; tables(): fills them and waits for the workgroup's other waves
-template <int HD, int RT, int STAGES, int KB, int VB, class Tables>
+// xch: [8 slots][PER_LANE values][64 lanes] floats of LDS; kpair / vpair: the two pair tables, filled
+template <int HD, int RT, int STAGES, int KB, int VB>
 __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, int R, int chunk, int h, int rt0, float* xch,
-                                                     const uint32_t* kpair, const uint32_t* vpair, Tables&& tables) {
+                                                     const uint32_t* kpair, const uint32_t* vpair) {
     constexpr int NW = 8;
     constexpr int KS = HD / 32;  // K steps of the score MFMA
     constexpr int VT = HD / 16;  // output tiles along head_dim
@@ -201,33 +201,40 @@ __device__ __forceinline__ void attn_partial_body_tq(const AttnArgs& a, int G, i
             }
         }
     };
-    // The first blocks of every wave are asked for, then the tables are filled at the one place that all waves of the workgroup reach: how many blocks a
-    // wave has differs inside a workgroup, so no branch on that may hold the barrier.  Blocks that a wave does not have are not asked for: as loads past the
-    // buffers' ends, which bring zeros, they cost a layer 1 us (one row at 2500 positions, eight layers: 500 us for 492).
-    Blk st[STAGES];
+    if (nb == 1) {
+        Blk st;
+        fetch(st, 0);
+        consume(st, 0);
+    } else if (nb == 2) {
+        Blk s0, s1;
+        fetch(s0, 0);
+        fetch(s1, 1);
+        consume(s0, 0);
+        consume(s1, 1);
+    } else if (nb >= STAGES) {
+        Blk st[STAGES];
 #pragma unroll
-    for (int s = 0; s < STAGES; s++)
-        if (s < nb) fetch(st[s], s);
-    tables();
-    int i = 0;
-    for (; i + 2 * STAGES <= nb; i += STAGES) {
+        for (int s = 0; s < STAGES; s++) fetch(st[s], s);
+        int i = 0;
+        for (; i + 2 * STAGES <= nb; i += STAGES) {
+#pragma unroll
+            for (int s = 0; s < STAGES; s++) {
+                consume(st[s], i + s);
+                fetch(st[s], i + s + STAGES);
+            }
+        }
 #pragma unroll
         for (int s = 0; s < STAGES; s++) {
-            consume(st[s], i + s);
-            fetch(st[s], i + s + STAGES);
+            if (i + s < nb) {
+                consume(st[s], i + s);
+                if (i + s + STAGES < nb) fetch(st[s], i + s + STAGES);
+            }
         }
-    }
+        i += STAGES;
 #pragma unroll
-    for (int s = 0; s < STAGES; s++) {
-        if (i + s < nb) {
-            consume(st[s], i + s);
-            if (i + s + STAGES < nb) fetch(st[s], i + s + STAGES);
-        }
+        for (int s = 0; s < STAGES; s++)
+            if (i + s < nb) consume(st[s], i + s);
     }
-    i += STAGES;
-#pragma unroll
-    for (int s = 0; s < STAGES; s++)
-        if (i + s < nb) consume(st[s], i + s);
 
     attn_finish<HD, RT, 8, false>(a, G, R, chunk, h, rt0, wave, lane, xch + lane, mrun, lrun, O);
 }
