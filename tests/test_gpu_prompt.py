@@ -197,6 +197,21 @@ def test_prompt_attention_matches_the_oracle(nq, nkv, hd, m, base, window, sinks
         assert np.abs(got[i] - want).max() <= 5e-3 * max(1.0, np.abs(want).max()), i   # the bound of the verify passes' test
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(8, 8, 64), (16, 4, 128)])
+@pytest.mark.parametrize("end", [991, 992, 1503, 1504, 8200])   # one chunk of the context, two, two, three, sixteen
+def test_prompt_attention_at_the_lines_of_its_chunks(nq, nkv, hd, end):
+    from turbospark_amd import ffi
+    m = 40
+    rng = np.random.default_rng(end)
+    r16 = lambda *s: rng.standard_normal(s).astype(np.float16).astype(np.float32)
+    q, k, v = r16(m, nq, hd), r16(end, nkv, hd), r16(end, nkv, hd)
+    sk = rng.standard_normal(nq).astype(np.float32) if end % 2 else None
+    got = ffi.attention(q, k, v, end - m, sinks=sk)
+    for i in (0, 17, m - 1):
+        want = ob.causal_attention(q[i], k, v, hd, nq, nkv, end - m + i + 1, 0, 0.0, sk).reshape(nq, hd)
+        assert np.abs(got[i] - want).max() <= 5e-3 * max(1.0, np.abs(want).max()), i
+
+
 @pytest.mark.parametrize("nq,nkv,hd", [(8, 2, 128), (4, 2, 64)])
 @pytest.mark.parametrize("m,base,spread", [(320, 0, 1.0), (320, 0, 2.5), (96, 2000, 1.0), (96, 2000, 2.5)])
 def test_prompt_attention_is_the_exact_result_rounded(nq, nkv, hd, m, base, spread):

@@ -791,10 +791,13 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attn(PromptAttnArgs p) {
 }
 
 // The chunks' partial results of one (row, q head) merged, one thread per eight dims; HD / 8 threads to a pair
-template <int HD, bool TQ>
+// MOST: chunks there are at most (prompt_attn_chunks), or 2: just two, as passes of many rows have.  With room for sixteen those held registers that
+// their many workgroups' occupancy was worth more than (1000 rows 9.6 us for 8.2, 4-bit rows 10.5 for 8.9); fewer rows have more chunks to wait for.
+template <int HD, bool TQ, int MOST>
 __global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
     constexpr int TPP = HD / 8;
-    constexpr int MOST = 16, BATCH = 4;  // chunks (prompt_attn_chunks); of the values, in flight together
+    constexpr int BATCH = MOST < 4 ? MOST : 4;  // of the values, in flight together
+    auto have = [&](int ch) { return MOST == 2 || ch < p.nch; };
     const int G = p.group, cols = p.n * G;
     const int id = blockIdx.x * 256 + threadIdx.x, pair = id / TPP, d = id % TPP * 8;
     // consecutive threads: dims, then rows of one head, so that the pieces written side by side are neighbours
@@ -806,25 +809,25 @@ __global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
     float2 ml[MOST];
 #pragma unroll
     for (int ch = 0; ch < MOST; ch++)
-        if (ch < p.nch) ml[ch] = *(const float2*)(p.part_ml + (at0 + ch * step) * 2);
+        if (have(ch)) ml[ch] = *(const float2*)(p.part_ml + (at0 + ch * step) * 2);
     float m = sink;
 #pragma unroll
     for (int ch = 0; ch < MOST; ch++)
-        if (ch < p.nch) m = fmaxf(m, ml[ch].x);
+        if (have(ch)) m = fmaxf(m, ml[ch].x);
     float l = p.sinks ? __builtin_amdgcn_exp2f(sink - m) : 0.f, o[8] = {};
 #pragma unroll
     for (int c0 = 0; c0 < MOST; c0 += BATCH) {
-        if (c0 >= p.nch) break;
+        if (!have(c0)) break;
         float4 a[BATCH], b[BATCH];
 #pragma unroll
         for (int j = 0; j < BATCH; j++)
-            if (c0 + j < p.nch) {
+            if (have(c0 + j)) {
                 a[j] = *(const float4*)(p.part_o + (at0 + (c0 + j) * step) * HD + d);
                 b[j] = *(const float4*)(p.part_o + (at0 + (c0 + j) * step) * HD + d + 4);
             }
 #pragma unroll
         for (int j = 0; j < BATCH; j++)
-            if (c0 + j < p.nch) {
+            if (have(c0 + j)) {
                 const float w = __builtin_amdgcn_exp2f(ml[c0 + j].x - m);
                 l = __builtin_fmaf(ml[c0 + j].y, w, l);
                 const float f[8] = {a[j].x, a[j].y, a[j].z, a[j].w, b[j].x, b[j].y, b[j].z, b[j].w};
@@ -833,8 +836,12 @@ __global__ __launch_bounds__(256) void k_prompt_attn_merge(PromptAttnArgs p) {
             }
     }
     const float inv = 1.0f / l;
+    // (the products as floats first: converted in the instruction that makes it a value is rounded once, and which ones are would differ from variant to variant)
 #pragma unroll
-    for (int e = 0; e < 8; e++) o[e] *= inv;
+    for (int e = 0; e < 8; e++) {
+        o[e] *= inv;
+        asm volatile("" : "+v"(o[e]));
+    }
     if (TQ) {  // back out of the rotated space: three stages inside a thread, the others over the TPP lanes of the pair
         const float c = 0.70710678118654752440f;
 #pragma unroll
@@ -1067,7 +1074,9 @@ static int launch_attn(hipStream_t s, const PromptAttnArgs& a0) {
     const dim3 grid((cols + 127) / 128 * a.nkv, 1, a.nch);
     if (a.nch > 1) {
         hipLaunchKernelGGL((k_prompt_attn<HD, true, TQ>), grid, dim3(256), 0, s, a);
-        hipLaunchKernelGGL((k_prompt_attn_merge<HD, TQ>), dim3(((size_t)a.n * a.nq * (HD / 8) + 255) / 256), dim3(256), 0, s, a);
+        const dim3 mgrid(((size_t)a.n * a.nq * (HD / 8) + 255) / 256);
+        if (a.nch == 2) hipLaunchKernelGGL((k_prompt_attn_merge<HD, TQ, 2>), mgrid, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((k_prompt_attn_merge<HD, TQ, 16>), mgrid, dim3(256), 0, s, a);
     } else {
         hipLaunchKernelGGL((k_prompt_attn<HD, false, TQ>), grid, dim3(256), 0, s, a);
     }
