@@ -259,3 +259,22 @@ def test_draws_at_the_ends_of_the_uniform(vocab, penalty):
                                       ob.shaping(1.0, seed=seed, **kw), history=history)
                 assert (res.accepted, res.draw_step) == (want["accepted"], want["draw_step"])
                 assert res.next == want["next"], (kind, bits, feed)
+
+
+@pytest.mark.parametrize("flat", [(0,), (1,), (7,), (14,), (3, 14)])
+def test_a_draw_that_is_refused_is_refused_whichever_row_it_is_of(flat):
+    """Rows of which 1500 penalised candidates share a score between two fp16 values, more than a draw can put in order, among rows that draw without any."""
+    import turbospark_amd as ts
+    vocab, k = 4096, 15
+    cfg, w, gpu, cpu = gc.build_pair("tiny_q8_0", max_context=64, vocab=vocab)
+    hist = list(range(1500))
+    r = np.random.default_rng(5)
+    rows = (r.standard_normal((k, vocab)) * 0.5).astype(np.float16)
+    rows[:, 2000] = 20.0                                             # sure of a token that no penalty touches
+    for seed in range(3):
+        draft = rows.copy()
+        gpu.draft_chain(draft, ts.shaping(1.0, seed=seed, repetition_penalty=1.1), 0, history=hist)
+        draft[list(flat)] = -40.0
+        draft[list(flat), :1500] = 3.0
+        with pytest.raises(Exception, match="not built"):
+            gpu.draft_chain(draft, ts.shaping(1.0, seed=seed, repetition_penalty=1.1), 0, history=hist)

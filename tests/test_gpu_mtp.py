@@ -262,3 +262,32 @@ def test_refusals_by_name():
     res.tokens, res.capacity = toks.ctypes.data_as(C.POINTER(C.c_int32)), 8
     rc = ffi.lib().tsv_run_speculative(gpu._h, C.byref(d), prompt.ctypes.data, prompt.size, C.byref(g), C.byref(res))
     assert rc != 0 and "step and prime, or draft_block and prefill_chunk" in ffi.last_error()
+
+
+def test_a_draw_that_is_refused_ends_the_block_whichever_step_it_is_of():
+    """A head whose first step gives every token one score: 1500 penalised candidates between two fp16 values, more than a draw can put in order.
+    The steps behind it are sure of their token and need no order, so nothing but the first draw has anything to refuse."""
+    V, start, sure, fork = 1600, 1500, 1501, 1502      # tokens below 1500 are the history; `fork` is followed by `start`, that by anything, anything by `sure`
+    cfg = dict(synth.CONFIGS["tiny_q8_0"], max_context=1700, vocab=V, weak_layers=0.0)
+    w = synth.make_weights(cfg, seed=1)
+    hcfg, hw = synth.make_mtp_weights(cfg, w, seed=2, norm_jitter=0.0)
+    H = cfg["hidden"]
+    e, head = np.zeros((V, H), np.float32), np.zeros((V, H), np.float32)
+    e[:, 1], e[start], e[fork] = 1.0, np.eye(H)[0], np.eye(H)[2]
+    head[:, 0] = 3.0 / H ** 0.5
+    head[sure, 1] = head[start, 2] = 25.0 / H ** 0.5
+    w["embed"] = hw["embed"] = ffi.quantize(ffi.BF16, e)
+    w["lm_head"] = hw["lm_head"] = ffi.quantize(ffi.BF16, head)
+    hw["fc"] = ffi.quantize(ffi.BF16, np.concatenate([np.eye(H), np.zeros((H, H))], axis=1).astype(np.float32))
+    gpu = ts.HipVerifier(cfg, w)
+    mtp = ts.MtpHead(gpu, hcfg, hw)
+    prompt = np.concatenate([np.arange(1500), [fork]]).astype(np.int32)
+    refused = 0
+    for seed in range(8):
+        try:
+            gpu.run_speculative(prompt, mtp, ts.shaping(1.0, seed=seed, repetition_penalty=1.1), 6, 4)
+        except Exception as err:
+            assert "mtp_draft_block" in str(err) and "not built" in str(err), err
+            refused += 1
+        gpu.reset()
+    assert refused >= 4     # the draw falls among the 1500 with 92 %

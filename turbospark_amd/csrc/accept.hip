@@ -1349,7 +1349,7 @@ __global__ __launch_bounds__(1024) void k_pick(const uint16_t* target, const uin
     if (tid == 0) {
         if (kind == 1) {
             tokens_out[jobi] = token;
-            if (jobi == 0) res->error = *err;
+            if (const int32_t seen = *err) atomicOr(&res->error, seen);  // (each draw's own: what another refuses may come after this one's end)
             // margins of the k draws are folded on the host side from res->min_margin
             atomicMin((unsigned long long*)&res->min_margin, __builtin_bit_cast(unsigned long long, margin));
         } else {

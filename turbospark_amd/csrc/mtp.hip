@@ -224,11 +224,14 @@ int tsv_mtp_draft_block_sampled(tsv_ctx* c, int32_t anchor, int64_t base, int32_
     }
     h.own_valid = false;
     TSV_HIP(hipMemcpyAsync(h.chain_host, h.block->chain + 1, (size_t)block * 4, hipMemcpyDeviceToHost, c->stream));
-    TSV_HIP(hipMemcpyAsync(c->res_host, &h.block->draw[block - 1].res, sizeof(AcceptResult), hipMemcpyDeviceToHost, c->stream));
+    // every draw has a result of its own
+    TSV_HIP(hipMemcpyAsync(h.block_host->draw, h.block->draw, block * sizeof(AcceptUpload), hipMemcpyDeviceToHost, c->stream));
     if ((rc = upload_end(c))) return rc;
-    if (c->res_host->error) {  // (every draw has a result of its own: this is the last step's)
-        set_error(std::string("mtp_draft_block: ") + accept_error_text(c->res_host->error));
-        return (c->res_host->error & 1) ? TSV_ERR_INVALID : TSV_ERR_UNSUPPORTED;
+    int error = 0;
+    for (int d = 0; d < block; d++) error |= h.block_host->draw[d].res.error;
+    if (error) {
+        set_error(std::string("mtp_draft_block: ") + accept_error_text(error));
+        return (error & 1) ? TSV_ERR_INVALID : TSV_ERR_UNSUPPORTED;
     }
     for (int i = 0; i < block; i++) proposals[i] = h.chain_host[i];
     return TSV_OK;
