@@ -1052,8 +1052,9 @@ int tsv::open_impl(const tsv_model_desc* d, tsv_ctx* share, const tsv_mtp_desc* 
         // One launch that projects, rotates and stores (no split-K partials, no separate rotation
         // kernel) where the head needs no per-head norm in between and q/k/v share a storage type.
         // The fused launch has one workgroup per 64-row tile and no K split, and one compute unit draws only so much:
-        // it is taken while a tile's weights stay under 256 KiB (8B Q4_K: 147 KB per tile, a tie with the two
-        // launches; gpt-oss-120B bf16: 369 KB, 15.3 us fused against 7.9 + 3.1 us apart).
+        // it is taken while a tile's weights stay under 256 KiB (eight 8B layers over 4096 positions, 1 / 5 / 16 rows, us a round, fused and as two
+        // launches, runs of one side within 3 %: Q4_K, 147 KB per tile, 462 / 516 / 670 and 470 / 513 / 662; Q4_K_M 524 / 581 / 736 and 529 / 578 / 734;
+        // Q5_K_M 603 / 662 / 820 and 604 / 664 / 819; gpt-oss-120B bf16: 369 KB, 15.3 us fused against 7.9 + 3.1 us apart).
         const bool light_tiles = 64 * row_bytes(s.wq.dtype, s.wq.cols) <= 256 * 1024;
         // (a Q6_K value projection beside Q4_K or Q5_K ones goes in the same launch: 215 KB a tile at 4096 columns)
         const bool one_launch = s.wv.dtype == s.wq.dtype || ((s.wq.dtype == TSV_Q4_K || s.wq.dtype == TSV_Q5_K) && s.wv.dtype == TSV_Q6_K &&
